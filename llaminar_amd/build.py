@@ -97,7 +97,8 @@ class InFlightRegisterError(RuntimeError):
 
 
 _VREG = re.compile(r"\bv(\d+)\b|\bv\[(\d+):(\d+)\]")
-_ASM_LOAD = re.compile(r"^\s*(global_load_\w+|buffer_load_\w+)\s+(v\d+|v\[\d+:\d+\])\s*,")
+# (a load into LDS has no destination register: what it names first is its address)
+_ASM_LOAD = re.compile(r"^\s*(global_load_(?!lds_)\w+|buffer_load_\w+)\s+(v\d+|v\[\d+:\d+\])\s*,")
 _VMEM = re.compile(r"^\s*(global_|buffer_|flat_|scratch_)(load|store|atomic)")
 _VMCNT = re.compile(r"vmcnt\((\d+)\)")
 

@@ -26,6 +26,7 @@ namespace llamql
         const int *group_offset;
         const int *row_source;
         int source_div;
+        int groups, group_rows; // groups, and rows of all of them
     };
 
     constexpr int SMALL_M = 16;         // most rows of the row-at-a-time kernel: one operand of the matrix unit

@@ -4,7 +4,7 @@
 // k-steps among themselves and summing through LDS; each weight byte is read once, a contiguous
 // kilobyte per load instruction, several in flight per wavefront.  The rows of A are the second
 // matrix operand (16 columns, those past M ignored).  HBM-bound.
-// More rows (prompts): 128x128 or 64x64 tiles, both operands staged through LDS, double buffered.
+// More rows (prompts): linear_tiled.hip.
 #include "linear.h"
 
 namespace llamql
@@ -198,198 +198,6 @@ namespace llamql
     bool linear_small(const char *fn, const LinearArgs &a, int batch, int dtype, hipStream_t st)
     {
         return dtype == LLAM_SEQ_F32 ? small_dispatch<float>(fn, a, batch, st) : small_dispatch<bf16>(fn, a, batch, st);
-    }
-
-    // ---- more rows ------------------------------------------------------------------------------
-    // Workgroup tile BM rows of A x BN rows of W, four wavefronts in 2 x 2, 64 columns of K per turn.
-    // W is the first operand, so a lane ends with four neighbouring output columns of one row.
-    // LDS: W tiles as they lie in memory (a lane's piece at lane * 16: no bank conflicts), A rows
-    // with their 16-byte pieces permuted by the row (xor), so that 16 rows read 16 bank groups.
-    constexpr int GEMM_BK = 64;
-    constexpr int GEMM_THREADS = 256;
-
-    template <typename T, int BM, int BN>
-    __global__ void __launch_bounds__(GEMM_THREADS)
-        linear_tiled_kernel(LinearArgs p, int m_tiles, int n_tiles)
-    {
-        using O = Operand<T>;
-        using V = typename O::V;
-        constexpr int APIECES = GEMM_BK * sizeof(T) / 16; // 16-byte pieces of a row
-        constexpr int ALOADS = BM * APIECES / GEMM_THREADS;
-        constexpr int WLOADS = BN * (GEMM_BK * 2 / 16) / GEMM_THREADS;
-        constexpr int ABYTES = BM * GEMM_BK * sizeof(T), WBYTES = BN * GEMM_BK * 2;
-        constexpr int TM = BM / 32, TN = BN / 32; // 16-row tiles of a wavefront
-        extern __shared__ __attribute__((aligned(16))) char smem[];
-        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-        const int c = lane & 15, g = lane >> 4;
-        const int wm = wave & 1, wn = wave >> 1;
-
-        // neighbouring tiles (all rows of A for one stretch of W) go to one die: blocks are dealt
-        // round robin over the eight dies
-        const int total = m_tiles * n_tiles;
-        int id = blockIdx.x;
-        const int per = total / 8;
-        if (id < per * 8)
-            id = (id & 7) * per + (id >> 3);
-        const int nt = id / m_tiles, mt = id - nt * m_tiles;
-        const int z = blockIdx.y;
-        int row0 = 0, rows = p.M;
-        if (p.group_offset)
-        {
-            row0 = p.group_offset[z];
-            rows = p.group_offset[z + 1] - row0;
-        }
-        if (mt * BM >= rows)
-            return;
-        const T *abase = static_cast<const T *>(p.a) + (size_t)z * p.a_stride;
-        const bf16 *wbase = static_cast<const bf16 *>(p.w) + (size_t)z * p.w_stride;
-        const int ksteps = p.K >> 5, w_tiles = p.N >> 4;
-
-        const u32x4 *asrc[ALOADS];
-        int adst[ALOADS];
-#pragma unroll
-        for (int i = 0; i < ALOADS; ++i)
-        {
-            const int q = threadIdx.x + i * GEMM_THREADS, r = q / APIECES, piece = q % APIECES;
-            int m = mt * BM + r;
-            m = row0 + (m < rows ? m : rows - 1);
-            if (p.row_source)
-                m = p.row_source[m] / p.source_div;
-            asrc[i] = reinterpret_cast<const u32x4 *>(abase + (size_t)m * p.lda) + piece;
-            adst[i] = r * APIECES + (piece ^ (r & (APIECES - 1)));
-        }
-        const u32x4 *wsrc[WLOADS];
-#pragma unroll
-        for (int i = 0; i < WLOADS; ++i)
-        {
-            const int q = threadIdx.x + i * GEMM_THREADS, t = q >> 7; // a tile's two k-steps: 128 pieces
-            int tile = nt * (BN / 16) + t;
-            tile = tile < w_tiles ? tile : w_tiles - 1;
-            wsrc[i] = reinterpret_cast<const u32x4 *>(wbase) + (size_t)tile * ksteps * 64 + (q & 127);
-        }
-        u32x4 areg[ALOADS], wreg[WLOADS];
-        auto fetch = [&](int kt) __attribute__((always_inline)) {
-#pragma unroll
-            for (int i = 0; i < ALOADS; ++i)
-                areg[i] = asrc[i][(size_t)kt * APIECES];
-#pragma unroll
-            for (int i = 0; i < WLOADS; ++i)
-                wreg[i] = wsrc[i][(size_t)kt * 128];
-        };
-        auto put = [&](int buf) __attribute__((always_inline)) {
-            u32x4 *sa = reinterpret_cast<u32x4 *>(smem + buf * (ABYTES + WBYTES));
-            u32x4 *sw = reinterpret_cast<u32x4 *>(smem + buf * (ABYTES + WBYTES) + ABYTES);
-#pragma unroll
-            for (int i = 0; i < ALOADS; ++i)
-                sa[adst[i]] = areg[i];
-#pragma unroll
-            for (int i = 0; i < WLOADS; ++i)
-                sw[threadIdx.x + i * GEMM_THREADS] = wreg[i];
-        };
-        f32x4 acc[TN][TM];
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-            for (int i = 0; i < TM; ++i)
-                acc[j][i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-
-        const int turns = p.K / GEMM_BK;
-        fetch(0);
-        put(0);
-        __syncthreads();
-        for (int kt = 0; kt < turns; ++kt)
-        {
-            if (kt + 1 < turns)
-                fetch(kt + 1);
-            const u32x4 *sa = reinterpret_cast<const u32x4 *>(smem + (kt & 1) * (ABYTES + WBYTES));
-            const u32x4 *sw = reinterpret_cast<const u32x4 *>(smem + (kt & 1) * (ABYTES + WBYTES) + ABYTES);
-#pragma unroll
-            for (int ks = 0; ks < 2; ++ks)
-            {
-                V a[TM];
-#pragma unroll
-                for (int i = 0; i < TM; ++i)
-                {
-                    const int r = wm * (BM / 2) + i * 16 + c;
-                    if constexpr (sizeof(T) == 2)
-                        a[i] = __builtin_bit_cast(bf16x8, sa[r * APIECES + ((ks * 4 + g) ^ (r & (APIECES - 1)))]);
-                    else
-                    {
-                        const f32x4 lo = __builtin_bit_cast(f32x4, sa[r * APIECES + ((ks * 8 + 2 * g) ^ (r & (APIECES - 1)))]);
-                        const f32x4 hi = __builtin_bit_cast(f32x4, sa[r * APIECES + ((ks * 8 + 2 * g + 1) ^ (r & (APIECES - 1)))]);
-                        a[i] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-                    }
-                }
-#pragma unroll
-                for (int j = 0; j < TN; ++j)
-                {
-                    const V w = O::from_weights(sw[(wn * TN + j) * 128 + ks * 64 + lane]);
-#pragma unroll
-                    for (int i = 0; i < TM; ++i)
-                        acc[j][i] = O::mma(w, a[i], acc[j][i]);
-                }
-            }
-            if (kt + 1 < turns)
-                put((kt + 1) & 1);
-            __syncthreads();
-        }
-
-        const size_t elem = p.out == LLAM_SEQ_OUT_F32 || p.out == LLAM_SEQ_OUT_ADD ? 4 : sizeof(T);
-        char *y = static_cast<char *>(p.y) + (size_t)z * p.y_stride * elem;
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-        {
-            const int m = mt * BM + wm * (BM / 2) + i * 16 + c;
-            if (m >= rows)
-                continue;
-            if (is_gated(p.out))
-            {
-#pragma unroll
-                for (int j = 0; j < TN; j += 2)
-                {
-                    const int tile = nt * (BN / 16) + wn * TN + j;
-                    if (tile < w_tiles)
-                        store4<T>(p, y, row0 + m, tile * 8 + 4 * g, gated4(p, acc[j][i], acc[j + 1][i]));
-                }
-            }
-            else
-            {
-#pragma unroll
-                for (int j = 0; j < TN; ++j)
-                {
-                    const int tile = nt * (BN / 16) + wn * TN + j;
-                    if (tile < w_tiles)
-                        store4<T>(p, y, row0 + m, tile * 16 + 4 * g, acc[j][i]);
-                }
-            }
-        }
-    }
-
-    namespace
-    {
-        template <typename T, int BM, int BN>
-        bool tiled_launch(const char *fn, const LinearArgs &a, int batch, hipStream_t st)
-        {
-            static LdsGrant grant;
-            constexpr size_t lds = 2 * (BM * GEMM_BK * sizeof(T) + BN * GEMM_BK * 2);
-            if (lds > 64 * 1024 && allow_lds(grant, reinterpret_cast<const void *>(&linear_tiled_kernel<T, BM, BN>), lds) != hipSuccess)
-                return fail(fn, "cannot reserve %zu bytes of LDS", lds);
-            const int mt = ceil_div(a.M, BM), nt = ceil_div(a.N, BN);
-            hipLaunchKernelGGL((linear_tiled_kernel<T, BM, BN>), dim3(mt * nt, batch), dim3(GEMM_THREADS), lds, st, a, mt, nt);
-            return launched(fn);
-        }
-        template <typename T>
-        bool tiled_dispatch(const char *fn, const LinearArgs &a, int batch, hipStream_t st)
-        {
-            // the wide tile wherever it still gives every compute unit a workgroup
-            const long wide = (long)ceil_div(a.M, 128) * ceil_div(a.N, 128) * batch;
-            return wide >= 256 ? tiled_launch<T, 128, 128>(fn, a, batch, st) : tiled_launch<T, 64, 64>(fn, a, batch, st);
-        }
-    } // namespace
-
-    bool linear_tiled(const char *fn, const LinearArgs &a, int batch, int dtype, hipStream_t st)
-    {
-        return dtype == LLAM_SEQ_F32 ? tiled_dispatch<float>(fn, a, batch, st) : tiled_dispatch<bf16>(fn, a, batch, st);
     }
 } // namespace llamql
 

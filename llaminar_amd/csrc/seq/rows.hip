@@ -429,7 +429,7 @@ namespace llamql
             // the gated tokens of each expert: every expert may get all M
             l.a = p.h, l.lda = p.K, l.w = p.up, l.w_stride = p.up_stride, l.y = act, l.ldy = p.ff;
             l.M = M, l.N = p.ff, l.K = p.K, l.out = LLAM_SEQ_OUT_RELU2;
-            l.group_offset = offset, l.row_source = order, l.source_div = p.top;
+            l.group_offset = offset, l.row_source = order, l.source_div = p.top, l.groups = p.experts, l.group_rows = M * p.top;
             if (!linear_tiled(fn, l, p.experts, dtype, st))
                 return false;
             l.a = act, l.lda = p.ff, l.w = p.down, l.w_stride = p.down_stride, l.y = pair_out, l.ldy = p.N;

@@ -1,0 +1,126 @@
+"""Linear layers of many rows against sums in 64 bits: every tile of the rule at its edges, strides, batches, outputs."""
+import ctypes
+
+import pytest
+
+from llaminar_amd import sequence as sq
+
+pytestmark = pytest.mark.gpu
+
+F32, BF16 = sq.F32, sq.BF16
+
+
+def tiles(w):
+    n, k = w.shape
+    return w.reshape(n // 16, 16, k // 32, 4, 8).permute(0, 2, 3, 1, 4).contiguous()
+
+
+def run(torch, a, w, y, dtype, out=sq.OUT_F32, N=None, K=None, batch=1, strides=(0, 0, 0), bias=None):
+    M = y.shape[-2] if y.dim() == 3 else y.shape[0]
+    args = sq.LinearArgs(d_a=a.data_ptr(), d_w=w.data_ptr(), d_y=y.data_ptr(), M=M, N=N, K=K, lda=a.stride(-2), ldy=y.stride(-2), out=out,
+                         batch=batch, a_stride=strides[0], w_stride=strides[1], y_stride=strides[2], limit=7.0)
+    if bias is not None:
+        args.d_bias = bias.data_ptr()
+    ok = sq.load().llam_seq_linear(ctypes.byref(args), dtype, 0, torch.cuda.current_stream().cuda_stream)
+    assert ok, sq.load().llam_ql_last_error()
+    torch.cuda.synchronize()
+
+
+def close(torch, y, a, w, K, extra=0.0):
+    """Sums of K products in 32 bits, in any order: each addition is off by 2^-23 of a partial sum at most."""
+    a, w = a.double(), w.double()
+    bound = (K + 1) * 2.0 ** -23 * (a.abs() @ w.abs().T)
+    want = a @ w.T
+    assert ((y.double() - want).abs() <= bound + extra * want.abs()).all()
+    return want
+
+
+# rows x columns x K: a single row more than the row-at-a-time kernel takes, edges of every tile, K of one and of an
+# odd number of turns, sizes at which each tile is chosen
+SHAPES = [(17, 16, 64), (31, 48, 192), (33, 80, 320), (64, 64, 128), (65, 272, 704), (100, 6160, 2048), (127, 144, 64),
+          (129, 256, 2048), (255, 528, 192), (257, 1040, 128), (300, 6160, 512), (522, 2048, 2112), (300, 16384, 192),
+          (1000, 8208, 64), (2048, 2048, 192), (2048, 4112, 128), (2048, 15440, 64)]
+
+
+@pytest.mark.parametrize("dtype", [BF16, F32])
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_sums(dev, M, N, K, dtype):
+    import torch
+
+    torch.manual_seed(M + N)
+    a = torch.randn(M, K + 64, device=dev)[:, :K]
+    a = a if dtype == F32 else torch.nn.functional.pad(a.bfloat16(), (0, 64))[:, :K]
+    w = torch.randn(N, K, device=dev).bfloat16()
+    y = torch.full((M + 1, N + 4), 5.0, device=dev)
+    run(torch, a, tiles(w), y[:M, :N], dtype, N=N, K=K)
+    close(torch, y[:M, :N], a, w, K)
+    assert (y[M:] == 5.0).all() and (y[:, N:] == 5.0).all(), "written past the output"
+
+
+@pytest.mark.parametrize("dtype", [BF16, F32])
+@pytest.mark.parametrize("out", [sq.OUT_ADD, sq.OUT_ELEM, sq.OUT_GATED, sq.OUT_RELU2, sq.OUT_GATED_CLAMP])
+@pytest.mark.parametrize("M,N,K", [(40, 96, 192), (300, 2080, 128), (2048, 4128, 64)])
+def test_outputs(dev, M, N, K, out, dtype):
+    import torch
+
+    torch.manual_seed(out)
+    a, w = torch.randn(M, K, device=dev), (torch.randn(N, K, device=dev) * K ** -0.5).bfloat16()
+    a = a if dtype == F32 else a.bfloat16()
+    gated = out in (sq.OUT_GATED, sq.OUT_GATED_CLAMP)
+    kind = torch.float32 if dtype == F32 or out == sq.OUT_ADD else torch.bfloat16
+    y = torch.randn(M, N // 2 if gated else N, device=dev).to(kind)
+    before = y.double()
+    run(torch, a, tiles(w), y, dtype, out, N, K)
+    z = a.double() @ w.double().T
+    if gated:
+        pair = z.reshape(M, N // 32, 2, 16)
+        gate, up = pair[:, :, 0].reshape(M, -1), pair[:, :, 1].reshape(M, -1)
+        if out == sq.OUT_GATED:
+            want = torch.nn.functional.gelu(gate, approximate="tanh") * up
+        else:
+            g, u = gate.clamp(max=7.0), up.clamp(-7.0, 7.0)
+            want = g * torch.sigmoid(1.702 * g) * (u + 1.0)
+    else:
+        want = {sq.OUT_ADD: before + z, sq.OUT_ELEM: z, sq.OUT_RELU2: torch.relu(z) ** 2}[out]
+    # rounding of the result, and sums of unit size (error below 2^-23 K) through an activation of slope below 20
+    off = (y.double() - want).abs()
+    assert (off <= (2.0 ** -8 if kind == torch.bfloat16 else 2.0 ** -20) * want.abs() + 20 * K * 2.0 ** -23).all()
+
+
+@pytest.mark.parametrize("dtype", [BF16, F32])
+def test_batches_and_strides(dev, dtype):
+    import torch
+
+    B, M, N, K = 5, 70, 48, 128
+    a = torch.randn(M, B, K, device=dev)
+    a = a if dtype == F32 else a.bfloat16()
+    w = torch.randn(B, N, K, device=dev).bfloat16()
+    y = torch.zeros(M, B, N, device=dev)
+    t = torch.stack([tiles(w[b]) for b in range(B)])
+    run(torch, a.permute(1, 0, 2), t, y.permute(1, 0, 2), dtype, N=N, K=K, batch=B, strides=(K, N * K, N))
+    for b in range(B):
+        close(torch, y[:, b], a[:, b], w[b], K)
+
+
+@pytest.mark.parametrize("M", [20, 300, 2048])
+def test_values_at_the_ends_of_the_range(dev, M):
+    """32-bit rows are multiplied in three pieces: infinities, numbers that are none and the largest and the small
+    ones come out as a product of the whole value gives them."""
+    import torch
+
+    N, K = 2048 if M == 2048 else 64, 256
+    torch.manual_seed(1)
+    a = torch.randn(M, K, device=dev)
+    a[3, 5], a[M - 1, 255], a[9, 100], a[11, 0], a[11, 1] = float("inf"), float("-inf"), float("nan"), 3.4e38, -3.4e38
+    a[12] *= 1e-30
+    a[13] = 0.0
+    w = torch.randn(N, K, device=dev).bfloat16()
+    y = torch.zeros(M, N, device=dev)
+    run(torch, a, tiles(w), y, F32, N=N, K=K)
+    want = (a.double() @ w.double().T).float()
+    rows = [m for m in range(M) if m != 11]   # (whose sums overflow or not by the order)
+    for kind in (torch.isnan, torch.isposinf, torch.isneginf):
+        assert torch.equal(kind(y[rows]), kind(want[rows]))
+    plain = [m for m in range(M) if m not in (3, 9, 11, M - 1)]
+    close(torch, y[plain], a[plain], w, K)
+    assert (y[13] == 0.0).all()
