@@ -413,7 +413,7 @@ namespace llamql
 
         float expected(const Tile &t, const LinearArgs &a, int batch)
         {
-            const float rows = a.group_offset ? (float)a.group_rows / t.rows + 0.5f * batch : (float)ceil_div(a.M, t.rows) * batch;
+            const float rows = (float)ceil_div(a.M, t.rows) * batch;
             const float tiles = rows * ceil_div(a.N, t.columns), slots = (float)UNITS * t.resident;
             const float fill = tiles < slots ? tiles / slots : 1.0f;
             const float turn = t.alone + (t.full - t.alone) * fill;
@@ -425,6 +425,14 @@ namespace llamql
     {
         const Tile *tiles = dtype == LLAM_SEQ_F32 ? TILES_F32 : TILES_BF16, *best = tiles;
         const size_t n = dtype == LLAM_SEQ_F32 ? sizeof TILES_F32 / sizeof(Tile) : sizeof TILES_BF16 / sizeof(Tile);
+        if (a.group_offset && dtype == LLAM_SEQ_BF16)
+        {
+            // the weights of many small groups come from memory, and a workgroup's start is long: two per compute unit,
+            // and large tiles from a third of their rows on (64 groups of 1408 x 2048 and back, the two tiles: 3.8 rows each
+            // 149 / 176 us, 12 rows 166 / 177, 48 rows 242 / 205, 192 rows 490 / 376)
+            best = &tiles[(long)a.group_rows < 24l * batch ? 6 : 2];
+            return best->launch(fn, a, batch, st);
+        }
         for (size_t i = 1; i < n; ++i)
             if (expected(tiles[i], a, batch) < expected(*best, a, batch))
                 best = &tiles[i];
