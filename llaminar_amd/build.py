@@ -183,6 +183,62 @@ def check_inflight_registers(asm: str, src_name: str) -> int:
     return followed
 
 
+class ScalarHazardError(RuntimeError):
+    """A hand-issued load reads a scalar register too soon after a vector instruction has written it."""
+
+
+_SREG = re.compile(r"\bs(\d+)\b|\bs\[(\d+):(\d+)\]")
+_VALU_TO_SREG = re.compile(r"^v_\w+\s+(s\d+|s\[\d+:\d+\])\s*,")
+SCALAR_WAIT_STATES = 5
+
+
+def _sregs(text: str) -> set[int]:
+    regs: set[int] = set()
+    for m in _SREG.finditer(text):
+        regs.update([int(m.group(1))] if m.group(1) is not None else range(int(m.group(2)), int(m.group(3)) + 1))
+    return regs
+
+
+def check_scalar_hazards(asm: str, src_name: str) -> int:
+    """Scan the device assembly for vector memory instructions inside inline assembly that read a scalar register
+    less than five wait states after a vector instruction (v_readfirstlane, v_cmp) wrote it.
+
+    The hardware does not wait by itself, and the compiler inserts the wait states for its own instructions only: such
+    a load takes a stale value, half of another pointer, for its base.  An instruction counts as one wait state,
+    s_nop N as N + 1.  Straight-line bookkeeping like check_inflight_registers, carried across labels.  Returns the
+    number of loads and stores looked at.
+    """
+    findings: list[str] = []
+    looked, func, in_asm = 0, "?", False
+    written: dict[int, int] = {}   # scalar register -> wait states since a vector instruction wrote it
+    for raw_line in asm.splitlines():
+        text = raw_line.strip()
+        if text.startswith(";;#ASMSTART") or text.startswith(";;#ASMEND"):
+            in_asm = text.startswith(";;#ASMSTART")
+            continue
+        m = re.match(r"^([A-Za-z_][\w$.]*):", raw_line)
+        if m and not raw_line.startswith(".L"):
+            func, written = m.group(1), {}
+            continue
+        text = text.split(";")[0].strip()
+        if not text or text.startswith(".") or text.endswith(":"):
+            continue
+        if in_asm and _VMEM.match(text):
+            looked += 1
+            hit = sorted(r for r in _sregs(text) if r in written)
+            if hit:
+                findings.append(f"{func}: '{text}' reads s{hit[0]} {written[hit[0]]} wait states after a vector instruction wrote it")
+        passed = int(text.split()[1], 0) + 1 if text.startswith("s_nop") else 1
+        written = {r: n + passed for r, n in written.items() if n + passed < SCALAR_WAIT_STATES}
+        m = _VALU_TO_SREG.match(text)
+        if m:
+            written.update(dict.fromkeys(_sregs(m.group(1)), 0))
+    if findings:
+        shown = "\n  ".join(findings[:12]) + ("" if len(findings) <= 12 else f"\n  ... and {len(findings) - 12} more")
+        raise ScalarHazardError(f"{src_name}: hand-issued loads take a stale scalar register (see check_scalar_hazards):\n  {shown}")
+    return looked
+
+
 def hipcc() -> str:
     exe = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
     if not Path(exe).exists():
@@ -256,7 +312,9 @@ def _compile(src: Path, force: bool = True) -> Path:
     if proc.returncode == 0:
         check_kernel_resources(proc.stderr, src.name)
         for asm_file in OBJDIR.glob(f"{src.stem}-hip-amdgcn-*.s"):
-            check_inflight_registers(asm_file.read_text(), src.name)
+            asm = asm_file.read_text()
+            check_inflight_registers(asm, src.name)
+            check_scalar_hazards(asm, src.name)
     err = "\n".join(_drop_resource_remarks(lines))
     if proc.returncode != 0:
         raise RuntimeError(f"hipcc failed on {src.name}:\n{err}")

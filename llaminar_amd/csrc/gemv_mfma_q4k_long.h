@@ -117,20 +117,14 @@ namespace llamql
             const uint32_t pgrp = (uint32_t)(prow >> 2) * (uint32_t)nsb;
             const uint32_t poff_w = pgrp * 512u + (uint32_t)(prow & 3) * 32u + 16u * (uint32_t)lh;
             const uint32_t poff_h = pgrp * 64u + (uint32_t)(prow & 3) * 16u;
-            auto uniform = [](const uint8_t *p) {
-                const uint64_t b = (uint64_t)p;
-                const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)b);
-                const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(b >> 32));
-                return reinterpret_cast<const uint8_t *>(((uint64_t)hi << 32) | lo);
-            };
             // loads are never predicated: past its last step a lane re-reads that step
             auto issue = [&](Raw &r, int step) {
                 const int sb = sb0 + (nsteps > 0 ? slice + (step < last_step ? step : last_step) * a.slices : 0);
                 if constexpr (PLANE)
-                    mfma_plane_load(r, uniform(a.plane + (size_t)sb * 512),
-                                    uniform(a.plane + q4k_plane_heads_offset(a.N, nsb) + (size_t)sb * 64), poff_w, poff_h);
+                    mfma_plane_load(r, uniform_base(a.plane + (size_t)sb * 512),
+                                    uniform_base(a.plane + q4k_plane_heads_offset(a.N, nsb) + (size_t)sb * 64), poff_w, poff_h);
                 else
-                    mfma_load(r, uniform(tile_base + (size_t)sb * 144), off);
+                    mfma_load(r, uniform_base(tile_base + (size_t)sb * 144), off);
             };
             Raw bufA, bufB;
             issue(bufA, 0);

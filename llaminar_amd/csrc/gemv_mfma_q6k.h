@@ -232,16 +232,10 @@ namespace llamql
             // loads are never predicated: past its last step a lane re-reads that step
             auto issue = [&](Mfma6Raw &r, int step) {
                 const uint32_t sb = nsteps > 0 ? (uint32_t)(slice + (step < last_step ? step : last_step) * a.slices) : 0u;
-                auto uniform = [](const uint8_t *p) {
-                    const uint64_t b = (uint64_t)p;
-                    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)b);
-                    const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(b >> 32));
-                    return reinterpret_cast<const uint8_t *>(((uint64_t)hi << 32) | lo);
-                };
                 Mfma6Ptr pl;
-                pl.ql = uniform(a.w + (size_t)sb * 128);
-                pl.qh = uniform(a.w + T * 128 + (size_t)sb * 64);
-                pl.fc = uniform(a.w + q6k_factors_offset(T) + (size_t)sb * 32);
+                pl.ql = uniform_base(a.w + (size_t)sb * 128);
+                pl.qh = uniform_base(a.w + T * 128 + (size_t)sb * 64);
+                pl.fc = uniform_base(a.w + q6k_factors_offset(T) + (size_t)sb * 32);
                 mfma6_load(r, pl, off);
             };
             Mfma6Raw bufA, bufB;
@@ -489,13 +483,7 @@ namespace llamql
             // loads are never predicated: past its last step a lane re-reads that step
             auto issue = [&](Mfma6PlaneRaw &r, int step) {
                 const uint32_t sb = (uint32_t)sb0 + (nsteps > 0 ? (uint32_t)(slice + (step < last_step ? step : last_step) * a.slices) : 0u);
-                auto uniform = [](const uint8_t *p) {
-                    const uint64_t b = (uint64_t)p;
-                    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)b);
-                    const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(b >> 32));
-                    return reinterpret_cast<const uint8_t *>(((uint64_t)hi << 32) | lo);
-                };
-                mfma6_plane_load(r, uniform(a.plane + (size_t)sb * 1024), uniform(scales + (size_t)sb * 64), off_w, off_s);
+                mfma6_plane_load(r, uniform_base(a.plane + (size_t)sb * 1024), uniform_base(scales + (size_t)sb * 64), off_w, off_s);
             };
             Mfma6PlaneRaw bufA, bufB;
             issue(bufA, 0);

@@ -179,15 +179,6 @@ namespace llamql
         int rows_per_wave, gshift, accumulate;
     };
 
-    // A pointer every lane holds, moved to scalar registers (the weight loads take their base there).
-    __device__ __forceinline__ const void *uniform_ptr(const void *p)
-    {
-        const uint64_t v = (uint64_t)p;
-        const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
-        const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-        return reinterpret_cast<const void *>(((uint64_t)hi << 32) | lo);
-    }
-
     // grid: (workgroups per matrix, n_tokens*top_k, 2 = gate|up)
     template <class F>
     __global__ void __launch_bounds__(GEMV_WAVES *WAVE) moe_gate_up_kernel(const MoEArgs m)
@@ -272,7 +263,7 @@ namespace llamql
         a.w = blockIdx.z == 0 ? m.experts[e].d_gate : m.experts[e].d_up;
         if (!a.w)
             return; // an expert whose matrices live elsewhere: skipped like a bad id (uniform)
-        a.w = uniform_ptr(a.w);
+        a.w = uniform_base(a.w);
         a.N = m.inter;
         a.SB = nsb;
         float *y = (blockIdx.z == 0 ? m.out0 : m.out1) + (size_t)slot * m.inter;
@@ -416,10 +407,7 @@ namespace llamql
         int ld_step = 0, ld_k = 0;
         // loads are never predicated: past the end a lane re-reads its first super-block of the slot
         auto issue = [&](typename Q::Raw &buf) {
-            const uint64_t wp = (uint64_t)live[ld_k].w;
-            const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)wp);
-            const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(wp >> 32));
-            a.w = reinterpret_cast<const void *>(((uint64_t)hi << 32) | lo);
+            a.w = uniform_base(live[ld_k].w);
             const int st = ld_step < nsteps ? ld_step : 0;
             const size_t ti = (size_t)min((step0 + st) * QUAD_STEP_SB + grp, total - 1);
             const typename Q::Cursor wc = Q::cursor(a, ti, ti, lc);
@@ -536,7 +524,7 @@ namespace llamql
             GemvArgs a; // weight addressing only
             a.N = m.hidden;
             a.SB = nsb;
-            a.w = uniform_ptr(w);
+            a.w = uniform_base(w);
             // every step's loads go out at once; never predicated: past the end a lane re-reads an earlier super-block
 #pragma unroll
             for (int i = 0; i < NS; ++i)
@@ -692,8 +680,8 @@ namespace llamql
         const void *wg = m.experts[e].d_gate, *wu = m.experts[e].d_up;
         if (!wg || !wu)
             return; // an expert whose matrices live elsewhere: skipped like a bad id (uniform)
-        wg = uniform_ptr(wg);
-        wu = uniform_ptr(wu);
+        wg = uniform_base(wg);
+        wu = uniform_base(wu);
         const int lane = threadIdx.x & (WAVE - 1);
         const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
         const int l = lane & 3, grp = lane >> 2;
@@ -709,7 +697,7 @@ namespace llamql
         auto issue = [&](typename Q::Raw &buf, int i) {
             const int s = min(s0 + i, 2 * per_mat - 1); // past the end: the last step again, never predicated
             const int mat = s >= per_mat ? 1 : 0;
-            a.w = uniform_ptr(mat ? wu : wg);
+            a.w = uniform_base(mat ? wu : wg);
             const size_t ti = (size_t)blockIdx.x * 32 * nsb + (size_t)(s - mat * per_mat) * QUAD_STEP_SB + grp;
             const typename Q::Cursor wc = Q::cursor(a, ti, ti, lc);
             Q::load(buf, wc, lc, true);
@@ -1278,7 +1266,7 @@ namespace llamql
         const int K = DOWN ? m.inter : m.hidden, N = DOWN ? m.hidden : m.inter;
         const int nsb_log2 = m.gshift, nsb = 1 << nsb_log2;
         GemvArgs a; // weight addressing only
-        a.w = uniform_ptr(w);
+        a.w = uniform_base(w);
         a.N = N;
         a.SB = nsb;
 

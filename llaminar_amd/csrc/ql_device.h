@@ -14,6 +14,22 @@ namespace llamql
 
     constexpr int WAVE = 64;
 
+    // A pointer every lane holds, in scalar registers, for hand-issued loads to take their base from.  A vector memory
+    // instruction may not read a scalar register before five wait states have passed since a vector instruction
+    // (v_readfirstlane here) wrote it; the compiler sees to that for its own instructions but not for those inside
+    // inline assembly, so the wait is part of making the pointer.  Without it a load now and then took half of
+    // another pointer for its base (moe_down_quad_kernel in Q4_K, whose loads followed after three instructions).
+    template <class T>
+    __device__ __forceinline__ const T *uniform_base(const T *p)
+    {
+        const uint64_t v = (uint64_t)p;
+        const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
+        const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+        uint64_t u = ((uint64_t)hi << 32) | lo;
+        asm volatile("s_nop 4" : "+s"(u));
+        return reinterpret_cast<const T *>(u);
+    }
+
     // ---- binary16 helpers ---------------------------------------------------
 
     __device__ __forceinline__ float h2f(uint16_t bits)

@@ -183,3 +183,34 @@ def test_inflight_check_counts_other_memory_operations_and_resets_at_jumps():
 \ts_waitcnt vmcnt(0)
 """)
     assert check_inflight_registers(asm, "demo.hip") == 2
+
+
+# ---- scalar registers that a vector instruction has just written ---------------------------------
+
+SCALAR = """\
+_Z6kernelv:
+\tv_readfirstlane_b32 s7, v3
+{between}
+\t;;#ASMSTART
+\tglobal_load_dwordx4 v[18:21], v2, s[6:7] offset:16
+\t;;#ASMEND
+\ts_endpgm
+"""
+
+
+@pytest.mark.parametrize("between", ["", "\ts_nop 3", "\tv_mov_b32_e32 v1, v2\n\ts_nop 2", "\tv_mul_u32_u24_e32 v3, 0x90, v4\n.LBB0_1:\n\ts_nop 0"])
+def test_a_load_too_soon_after_its_base_was_made_fails_the_build(between):
+    with pytest.raises(b.ScalarHazardError, match="s7"):
+        b.check_scalar_hazards(SCALAR.format(between=between), "moe.hip")
+
+
+@pytest.mark.parametrize("between", ["\ts_nop 4", "\tv_mov_b32_e32 v1, v2\n\ts_nop 3", "\n".join(["\tv_mov_b32_e32 v1, v2"] * 5)])
+def test_a_load_after_five_wait_states_passes(between):
+    assert b.check_scalar_hazards(SCALAR.format(between=between), "moe.hip") == 1
+
+
+def test_scalar_instructions_and_the_compilers_own_loads_need_no_wait():
+    asm = SCALAR.format(between="").replace("v_readfirstlane_b32 s7, v3", "s_mov_b32 s7, s3")
+    assert b.check_scalar_hazards(asm, "moe.hip") == 1
+    own = SCALAR.format(between="").replace("\t;;#ASMSTART\n", "").replace("\t;;#ASMEND\n", "")
+    assert b.check_scalar_hazards(own, "moe.hip") == 0
