@@ -1075,35 +1075,68 @@ namespace llamql
         return Int3{base.a + inc.a - v.a, base.b + inc.b - v.b, base.c + inc.c - v.c};
     }
 
+    // One workgroup.  Every wavefront takes a stretch of the pairs, 64 at a time: lanes that hold the same expert find
+    // each other by the bits of its id, so a lane's place among them is a count of mask bits and the first of them moves
+    // the wavefront's counter of the expert on.  Stable, without atomics; 2997 pairs of 257 experts 100 -> 14.5 us
+    // (every pair used to count the earlier pairs of its expert).
     __global__ void __launch_bounds__(MOE_GROUP_THREADS)
-        moe_group_kernel(const int32_t *__restrict__ ids, int P, int n_experts, void *ws)
+        moe_group_kernel(const int32_t *__restrict__ ids, int P, int n_experts, int bits, void *ws)
     {
-        extern __shared__ int32_t grp_se[]; // expert of every pair (INT_MAX: left out), padded to a multiple of 4
+        constexpr int WAVES = MOE_GROUP_THREADS / WAVE;
+        extern __shared__ uint16_t grp_count[]; // [wavefront][expert]: its pairs, later those before its next one
         __shared__ int hist[MOE_GROUP_MAX_EXPERTS];
-        __shared__ int wave_sums[MOE_GROUP_THREADS / WAVE][3];
+        __shared__ int wave_sums[WAVES][3];
         const MoEGroupView g = moe_group_view(ws, P);
-        const int tid = threadIdx.x;
-        for (int e = tid; e < MOE_GROUP_MAX_EXPERTS; e += blockDim.x)
-            hist[e] = 0;
+        const int tid = threadIdx.x, lane = tid & (WAVE - 1), wave = tid >> 6;
+        for (int i = tid; i < WAVES * n_experts; i += MOE_GROUP_THREADS)
+            grp_count[i] = 0;
         __syncthreads();
-        const int P4 = (P + 3) & ~3;
-        for (int p = tid; p < P4; p += blockDim.x)
-        {
-            const int e = p < P ? ids[p] : -1;
+        volatile uint16_t *own = grp_count + wave * n_experts;
+        const int stretch = (P + WAVES * WAVE - 1) / (WAVES * WAVE) * WAVE;
+        const int first = wave * stretch, last = first + stretch < P ? first + stretch : P;
+        // pair p's expert (-1: left out), its place among the lanes with the same one, and how many they are
+        auto meet = [&](int p, int &place, int &count) {
+            const int e = p < last ? ids[p] : -1;
             const bool ok = e >= 0 && e < n_experts;
-            grp_se[p] = ok ? e : 0x7FFFFFFF;
-            if (ok)
-                atomicAdd(&hist[e], 1); // integer: the counts do not depend on the order
+            unsigned long long same = __ballot(ok);
+            for (int b = 0; b < bits; ++b)
+            {
+                const unsigned long long set = __ballot((e >> b) & 1);
+                same &= (e >> b) & 1 ? set : ~set;
+            }
+            place = __popcll(same & ((1ull << lane) - 1));
+            count = __popcll(same);
+            return ok ? e : -1;
+        };
+        for (int p0 = first; p0 < last; p0 += WAVE)
+        {
+            int place, count;
+            const int e = meet(p0 + lane, place, count);
+            if (e >= 0 && place == 0)
+                own[e] = (uint16_t)(own[e] + count);
         }
         __syncthreads();
         // thread i owns experts 2i and 2i+1: pairs, non-empty experts and chunks before them
-        const int c0 = hist[2 * tid], c1 = hist[2 * tid + 1];
+        int c01[2];
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+        {
+            const int e = 2 * tid + k;
+            int total = 0;
+            for (int w = 0; w < WAVES && e < n_experts; ++w)
+            {
+                const int n = grp_count[w * n_experts + e];
+                grp_count[w * n_experts + e] = (uint16_t)total;
+                total += n;
+            }
+            c01[k] = total;
+        }
+        const int c0 = c01[0], c1 = c01[1];
         const int MOE_CHUNK = moe_chunk_size(P);
         const int k0 = (c0 + MOE_CHUNK - 1) / MOE_CHUNK, k1 = (c1 + MOE_CHUNK - 1) / MOE_CHUNK;
         Int3 total;
         const Int3 ex = block_exclusive_scan3(Int3{c0 + c1, (c0 > 0) + (c1 > 0), k0 + k1}, total, wave_sums);
-        __syncthreads(); // everybody has read its counts: hist becomes the experts' offsets
-        hist[2 * tid] = ex.a;
+        hist[2 * tid] = ex.a; // the experts' offsets
         hist[2 * tid + 1] = ex.a + c0;
         auto emit = [&](int e, int cnt, int seg, int begin, int chunk) {
             g.seg_expert[seg] = e;
@@ -1128,23 +1161,17 @@ namespace llamql
             g.seg_begin[total.b] = total.a;
         }
         __syncthreads();
-        // stable place of every pair: its expert's offset plus the earlier pairs of that expert
-        for (int p = tid; p < P; p += blockDim.x)
+        for (int p0 = first; p0 < last; p0 += WAVE)
         {
-            const int e = grp_se[p];
-            if (e == 0x7FFFFFFF)
-                continue;
-            int same = 0;
-            const int4 *v = reinterpret_cast<const int4 *>(grp_se);
-            const int full = p >> 2;
-            for (int q = 0; q < full; ++q)
-            {
-                const int4 x = v[q];
-                same += (x.x == e) + (x.y == e) + (x.z == e) + (x.w == e);
-            }
-            for (int q = full * 4; q < p; ++q)
-                same += grp_se[q] == e;
-            g.pair_sorted[hist[e] + same] = p;
+            int place, count;
+            const int e = meet(p0 + lane, place, count);
+            const int before = e >= 0 ? own[e] : 0;
+            __builtin_amdgcn_wave_barrier();
+            if (e >= 0)
+                g.pair_sorted[hist[e] + before + place] = p0 + lane;
+            if (e >= 0 && place == 0)
+                own[e] = (uint16_t)(before + count);
+            __builtin_amdgcn_wave_barrier();
         }
     }
 
@@ -1241,6 +1268,12 @@ namespace llamql
         moe_chunk_body<F, MAXM>(a, g, chunk, lds);
     }
 
+} // namespace llamql
+
+#include "moe_grouped_mfma.h"
+
+namespace llamql
+{
     // The grouped launches on the quad-lane decoder (expert rows of 2, 4, 8 or 16 super-blocks): a workgroup
     // row takes one chunk -- an expert and 1..MAXM of its (token, slot) pairs -- decodes every step of the
     // expert's matrix ONCE and multiplies it with each pair's activation row: per pair the decode, the dots
@@ -2060,8 +2093,16 @@ extern "C" bool llam_ql_moe_group(const int32_t *d_ids, int n_tokens, int slot_s
         return false;
     if (n_experts > MOE_GROUP_MAX_EXPERTS)
         return fail(fn, "n_experts=%d: at most %d experts are grouped", n_experts, MOE_GROUP_MAX_EXPERTS);
-    hipLaunchKernelGGL(moe_group_kernel, dim3(1), dim3(MOE_GROUP_THREADS), (size_t)((P + 3) & ~3L) * 4,
-                       as_stream(stream), d_ids, (int)P, n_experts, d_group);
+    static LdsGrant grant;
+    const size_t lds = (size_t)(MOE_GROUP_THREADS / WAVE) * n_experts * sizeof(uint16_t);
+    if (lds > 48 * 1024 && allow_lds(grant, reinterpret_cast<const void *>(&moe_group_kernel),
+                                     (size_t)(MOE_GROUP_THREADS / WAVE) * MOE_GROUP_MAX_EXPERTS * sizeof(uint16_t)) != hipSuccess)
+        return fail(fn, "cannot reserve %zu bytes of LDS", lds);
+    int bits = 0;
+    while ((1 << bits) < n_experts)
+        ++bits;
+    hipLaunchKernelGGL(moe_group_kernel, dim3(1), dim3(MOE_GROUP_THREADS), lds, as_stream(stream), d_ids, (int)P, n_experts,
+                       bits, d_group);
     return launched(fn);
 }
 
@@ -2078,11 +2119,55 @@ namespace llamql
                 hipLaunchKernelGGL((moe_grouped_quad_kernel<Q, 2, DOWN>), grid, dim3(MOE_QUAD_WAVES * WAVE), lds, st, m, ws, P);
         }
 
+        // Batches with this many (token, slot) pairs and so many per expert take the matrix unit.  Below, one decode for
+        // four pairs costs no more and the fewer instructions per pair count: 256 experts of 2048 x 512, IQ3_S, the
+        // whole feed-forward, four pairs a decode / matrix unit: 64 tokens (2.2 pairs an expert) 152 / 163 us, 96 (3.4)
+        // 185 / 187, 128 (4.5) 216 / 201.
+        constexpr int MOE_MFMA_MIN_PAIRS = 432;
+        constexpr int MOE_MFMA_MIN_MEAN = 4;
+
+        template <class F, int MT>
+        bool moe_mfma_launch(const char *fn, bool down, MoEArgs m, void *ws, int P, int device_id, hipStream_t st)
+        {
+            static LdsGrant grants[2];
+            const int rows = down ? m.hidden : m.inter, nsb = (down ? m.inter : m.hidden) / 256;
+            const size_t lds = moe_mfma_lds<F::HAS_MIN>(MT, nsb);
+            const void *kernel = down ? reinterpret_cast<const void *>(&moe_grouped_mfma_kernel<F, MT, true>)
+                                      : reinterpret_cast<const void *>(&moe_grouped_mfma_kernel<F, MT, false>);
+            if (lds > 48 * 1024 && allow_lds(grants[down], kernel, MOE_MFMA_LDS) != hipSuccess)
+                return fail(fn, "cannot reserve %zu bytes of LDS", lds);
+            // tiles of pairs: every expert may have one that is not full
+            const int experts = m.n_experts < P ? m.n_experts : P, tiles = P / (MT * 16) + experts;
+            // row tiles of a wavefront: as many as leave every compute unit six workgroups or so
+            const long all = (long)(rows / 16) * tiles * (down ? 1 : 2);
+            int each = 1;
+            while (each < 8 && all / ((long)MOE_MFMA_WAVES * each * 2) >= 6l * cu_count(device_id))
+                each *= 2;
+            m.rows_per_wave = each;
+            const unsigned gx = (unsigned)((rows / 16 + MOE_MFMA_WAVES * each - 1) / (MOE_MFMA_WAVES * each));
+            if (down)
+                hipLaunchKernelGGL((moe_grouped_mfma_kernel<F, MT, true>), dim3(gx, tiles), dim3(MOE_MFMA_WAVES * WAVE), lds, st, m, ws, P);
+            else
+                hipLaunchKernelGGL((moe_grouped_mfma_kernel<F, MT, false>), dim3(gx, tiles, 2), dim3(MOE_MFMA_WAVES * WAVE), lds, st, m, ws, P);
+            return launched(fn);
+        }
+
         template <class F>
         bool moe_grouped_launch(const char *fn, bool down, const MoEArgs &m_in, void *ws, int P, dim3 grid, int device_id,
                                 hipStream_t st)
         {
             const MoEArgs &m = m_in;
+            {
+                const int rows = down ? m.hidden : m.inter, nsb = (down ? m.inter : m.hidden) / 256;
+                if (P >= MOE_MFMA_MIN_PAIRS && P >= (long)MOE_MFMA_MIN_MEAN * m.n_experts && nsb <= MOE_MFMA_MAX_SB && F::Quad::addressable(rows, nsb))
+                {
+                    // pairs of a tile: about what an expert has, as far as the LDS holds them
+                    const int mean = P / m.n_experts;
+                    if (mean > 12 && moe_mfma_lds<F::HAS_MIN>(2, nsb) <= MOE_MFMA_LDS)
+                        return moe_mfma_launch<F, 2>(fn, down, m, ws, P, device_id, st);
+                    return moe_mfma_launch<F, 1>(fn, down, m, ws, P, device_id, st);
+                }
+            }
             {
                 // expert rows of 2, 4, 8 or 16 super-blocks: the quad-lane decoder, every step decoded once per chunk
                 const int rows = down ? m.hidden : m.inter, nsbq = (down ? m.inter : m.hidden) / 256;
