@@ -418,6 +418,238 @@ namespace llamql
         }
     }
 
+    // ---- activations as they lie, a tile's K steps dealt to the wavefronts ------------------------
+    // Tile of 32 MT tokens x 32 RN weight rows, KS x RN wavefronts: wavefront (rn, ks) multiplies super-blocks ks, ks + KS,
+    // .. of rows 32 rn .. by all tokens of the tile, and the KS partial sums are added through LDS in their order.  The
+    // weights never pass through LDS: lane (r, h) decodes what quad lanes h and h + 2 of row r decode, four whole blocks of
+    // a super-block, and a swap of half registers between the lanes (r, 0) and (r, 1) makes both lanes' blocks into
+    // matrix operands.  The Q8_1 blocks of KS super-blocks of the tokens go from memory into LDS, a step ahead, two buffers,
+    // one barrier a step: the quants as 16-byte pieces, [super-block][token][16], piece p of token m at p ^ (m & 15) (so that
+    // reads of 16 tokens' pieces meet no bank twice), the heads {d, sum} as [super-block][block][token].
+    // Bound by the vector unit: a conversion and a multiply-add per product of a block, and the decoding, which 64 tokens
+    // share; one workgroup of eight wavefronts fits a compute unit (up to 210 registers a lane; 128, for two of them, spill).
+    // 130 tokens x 5000 rows of 5120, Q4_K 54 -> 33 us, Q6_K 60 -> 38; 40 x 8192 x 5120 of IQ3_S 39.6 -> 23.0.
+    // The sums are kept in 2 to 8 parts: their error against 64 bits is 0.5 to 0.9 times gemm_kernel's.
+    template <int MT, int RN, int KS>
+    struct GemmSplit
+    {
+        static constexpr int BM = MT * 32, WAVES = RN * KS;
+        static constexpr int QUANTS = KS * BM * 256, HEADS = KS * BM * 32; // bytes of a step
+        static constexpr int QLOADS = QUANTS / 1024 / WAVES, HLOADS = HEADS / 256 / WAVES; // per wavefront
+        static constexpr int QROWS = 4 * WAVES;                  // tokens x super-blocks that one load of every wavefront covers
+        static constexpr int QM = BM > QROWS ? BM / QROWS : 1;   // tokens a lane loads pieces of
+        static constexpr int HSB = WAVES * 8 / BM;               // super-blocks that one load of every wavefront covers (heads)
+        static_assert(QLOADS * WAVES * 1024 == QUANTS && HLOADS * WAVES * 256 == HEADS, "whole loads");
+        static_assert(QROWS % 16 == 0 && (BM % QROWS == 0 || QROWS % BM == 0), "a lane's piece and tokens stay the same");
+        static_assert(HSB >= 1 && HSB * BM == WAVES * 8, "a lane's block and token stay the same");
+        static constexpr size_t STAGE = QUANTS + HEADS;
+        static constexpr size_t SUMS = (size_t)(KS - 1) * RN * MT * 16 * WAVE * sizeof(float);
+        static constexpr size_t LDS = 2 * STAGE > SUMS ? 2 * STAGE : SUMS;
+    };
+
+    template <class F, int MT, int RN, int KS, bool DUMP>
+    __global__ void __launch_bounds__(RN *KS *WAVE) gemm_split_kernel(const GemmArgs g)
+    {
+        typedef typename F::Quad Q;
+        typedef GemmSplit<MT, RN, KS> G;
+        typedef int v2i_dword __attribute__((ext_vector_type(2), aligned(4)));
+        constexpr int BM = G::BM;
+        extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+        void *tab = format_tables_lds<F>();
+        if (F::TABLE_BYTES > 0)
+            F::stage_tables(tab);
+
+        const int tid = threadIdx.x, lane = tid & 63;
+        const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+        const int rn = wave % RN, ks = wave / RN;
+        const int l32 = lane & 31, lh = lane >> 5;
+        const long n0 = ((long)blockIdx.x * RN + rn) * 32 + (long)g.tile0 * GEMM_BN, m0 = (long)blockIdx.y * BM;
+        const int SB = g.w.SB, KB = SB * 8;
+
+        long n = n0 + l32;
+        if (n >= g.w.N)
+            n = g.w.N - 1; // tail rows: decode a valid row, never stored
+        const typename Q::Lane lane_of[2] = {Q::lane_consts(lh), Q::lane_consts(lh + 2)};
+        const typename Q::Cursor wc = Q::cursor(g.w, (size_t)n * SB, (size_t)n * SB, lane_of[0]);
+        typename Q::Raw raw[2];
+        auto issue_weights = [&](int sb) { // (past the end: the last super-block again)
+            const int at = sb < SB ? sb : SB - 1;
+            Q::load_at(raw[0], wc, lane_of[0], at);
+            Q::load_at(raw[1], wc, lane_of[1], at);
+        };
+        // bytes from the tile's first token to what this lane loads of super-block 0 (past the last token: the last one)
+        const uint8_t *abase = reinterpret_cast<const uint8_t *>(g.q8 + (size_t)m0 * KB * 9);
+        auto token = [&](int m) { return (uint32_t)(m0 + m < g.M ? m : g.M - 1 - m0) * (uint32_t)(KB * 36); };
+        uint32_t qfrom[G::QM], hfrom;
+        {
+            const int row = wave * 4 + (lane >> 4), p = (lane & 15) ^ (row & 15);
+#pragma unroll
+            for (int i = 0; i < G::QM; ++i)
+                qfrom[i] = token((row + i * G::QROWS) % BM) + (uint32_t)((p >> 1) * 36 + 4 + (p & 1) * 16);
+            const int idx = wave * 64 + lane;
+            hfrom = token(idx % BM) + (uint32_t)((idx / BM) & 7) * 36;
+        }
+        const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)smem;
+        auto super_block = [&](int sb) { return abase + (size_t)(sb < SB ? sb : SB - 1) * 288; }; // (past the end: the last one)
+        auto issue_acts = [&](int sb0, int buf) {
+            const uint32_t to = lds0 + (uint32_t)(buf * (int)G::STAGE + wave * 1024);
+#pragma unroll
+            for (int i = 0; i < G::QLOADS; ++i)
+                asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to + (uint32_t)(i * G::WAVES * 1024)),
+                             "v"(qfrom[i % G::QM]), "s"(super_block(sb0 + (wave * 4 + i * G::QROWS) / BM))
+                             : "memory");
+            const uint32_t toh = lds0 + (uint32_t)(buf * (int)G::STAGE + G::QUANTS + wave * 256);
+#pragma unroll
+            for (int i = 0; i < G::HLOADS; ++i)
+                asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(toh + (uint32_t)(i * G::WAVES * 256)),
+                             "v"(hfrom), "s"(super_block(sb0 + (wave * 64 / BM + i * (G::WAVES * 64 / BM)) / 8))
+                             : "memory");
+        };
+        v16f acc[MT];
+#pragma unroll
+        for (int t = 0; t < MT; ++t)
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                acc[t][r] = 0.0f;
+        v16i zero;
+        v32f zero2f;
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+            zero[r] = 0;
+#pragma unroll
+        for (int r = 0; r < 32; ++r)
+            zero2f[r] = 0.0f;
+
+        issue_acts(0, 0);
+        issue_weights(ks);
+        int buf = 0;
+        for (int sb0 = 0; sb0 < SB; sb0 += KS, buf ^= 1)
+        {
+            const int sb = sb0 + ks;
+            // this step's weights and activations have arrived, everybody is done with the other buffer
+            Q::template wait<0>(raw[0]);
+            Q::template wait<0>(raw[1]);
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            v4i w[2][4];
+            typename Q::Scale S[2];
+#pragma unroll
+            for (int c = 0; c < 2; ++c)
+                Q::decode(raw[c], lane_of[c], w[c], S[c]);
+            // decoded here, before the registers are asked for again: sunk below, the decoding would have the compiler copy
+            // the raw words, and copies made ahead of the wait hold what the loads have not brought yet
+#pragma unroll
+            for (int c = 0; c < 2; ++c)
+            {
+                v2i_dword two = __builtin_bit_cast(v2i_dword, S[c]);
+                asm volatile("" : "+v"(w[c][0]), "+v"(w[c][1]), "+v"(w[c][2]), "+v"(w[c][3]), "+v"(two));
+                S[c] = __builtin_bit_cast(typename Q::Scale, two);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            if (sb0 + KS < SB)
+                issue_acts(sb0 + KS, buf ^ 1);
+            issue_weights(sb + KS);
+            __builtin_amdgcn_sched_barrier(0);
+            if (sb < SB) // uniform in the wavefront
+            {
+                const uint8_t *rows = smem + buf * G::STAGE + (size_t)(ks * BM + l32) * 256;
+                const uint32_t *heads = reinterpret_cast<const uint32_t *>(smem + buf * G::STAGE + G::QUANTS) + ks * 8 * BM + l32;
+#pragma unroll
+                for (int c = 0; c < 2; ++c)
+#pragma unroll
+                    for (int i = 0; i < 2; ++i)
+                    {
+                        // block x of quad lane 2c, block y of quad lane 2c + 1: elements 0 .. 15 with lanes (r, 0), 16 .. 31 with (r, 1)
+                        v4i x = w[c][2 * i], y = w[c][2 * i + 1];
+#pragma unroll
+                        for (int d = 0; d < 4; ++d)
+                        {
+                            typedef uint32_t v2u __attribute__((ext_vector_type(2)));
+                            const v2u s = __builtin_bit_cast(v2u, __builtin_amdgcn_permlane32_swap((uint32_t)x[d], (uint32_t)y[d], false, false));
+                            x[d] = (int)s[0], y[d] = (int)s[1];
+                        }
+                        const int kx = Q::block_of(2 * c, i), ky = Q::block_of(2 * c + 1, i);
+                        const float bs = Q::scale_f32(S[c], i);
+#pragma unroll
+                        for (int t = 0; t < MT; ++t)
+                        {
+                            auto quants = [&](int k) {
+                                return *reinterpret_cast<const v4i *>(rows + t * 32 * 256 + (((2 * k + lh) ^ (l32 & 15)) << 4));
+                            };
+                            const uint32_t head = heads[(lh ? ky : kx) * BM + t * 32];
+                            const float ad = h2f((uint16_t)(head & 0xFFFFu));
+                            // the scale products of both blocks, a rank-1 matrix each (exact: both factors are fp16 values)
+                            const v32f cs = __builtin_amdgcn_mfma_f32_32x32x1f32(ad, bs, zero2f, 0, 0, 0);
+                            const v16i dx = __builtin_amdgcn_mfma_i32_32x32x32_i8(quants(kx), x, zero, 0, 0, 0);
+                            const v16i dy = __builtin_amdgcn_mfma_i32_32x32x32_i8(quants(ky), y, zero, 0, 0, 0);
+                            if constexpr (DUMP)
+                            {
+                                const long nn = n0 + l32 - g.row0;
+                                if (n0 + l32 < g.w.N && nn >= 0 && nn < g.nrows)
+                                {
+#pragma unroll
+                                    for (int r = 0; r < 16; ++r)
+                                    {
+                                        const long m = m0 + t * 32 + 8 * (r >> 2) + 4 * lh + (r & 3);
+                                        int32_t *to = g.sums + ((size_t)m * g.nrows + (size_t)nn) * (size_t)KB + (size_t)sb * 8;
+                                        if (m < g.M)
+                                            to[kx] = dx[r], to[ky] = dy[r];
+                                    }
+                                }
+                            }
+#pragma unroll
+                            for (int r = 0; r < 16; ++r)
+                                acc[t][r] = fmaf((float)dx[r], cs[r], acc[t][r]);
+#pragma unroll
+                            for (int r = 0; r < 16; ++r)
+                                acc[t][r] = fmaf((float)dy[r], cs[16 + r], acc[t][r]);
+                            if (F::HAS_MIN)
+                                acc[t] = __builtin_amdgcn_mfma_f32_32x32x2f32((float)(int16_t)(head >> 16) * ad, Q::min_f32(S[c], i), acc[t], 0, 0, 0);
+                        }
+                    }
+            }
+        }
+        Q::template wait<0>(raw[0]);
+        Q::template wait<0>(raw[1]);
+        if (DUMP)
+            return;
+
+        if constexpr (KS > 1)
+        {
+            __syncthreads(); // everybody is done with the activations
+            float *red = reinterpret_cast<float *>(smem) + rn * MT * 16 * WAVE + lane;
+            if (ks > 0)
+            {
+#pragma unroll
+                for (int t = 0; t < MT; ++t)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r)
+                        red[((ks - 1) * RN * MT * 16 + t * 16 + r) * WAVE] = acc[t][r];
+            }
+            __syncthreads();
+            if (ks > 0)
+                return;
+#pragma unroll
+            for (int k = 0; k < KS - 1; ++k)
+#pragma unroll
+                for (int t = 0; t < MT; ++t)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r)
+                        acc[t][r] += red[(k * RN * MT * 16 + t * 16 + r) * WAVE];
+        }
+        if (n0 + l32 < g.w.N)
+        {
+#pragma unroll
+            for (int t = 0; t < MT; ++t)
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                {
+                    const long m = m0 + t * 32 + 8 * (r >> 2) + 4 * lh + (r & 3);
+                    if (m < g.M)
+                        g.y[(size_t)m * g.ldy + n0 + l32] = acc[t][r];
+                }
+        }
+    }
+
     __global__ void __launch_bounds__(256)
         epilogue_kernel(float *__restrict__ c, const float *__restrict__ t, const float *__restrict__ bias,
                         long M, int N, int ldc, float alpha, float beta)
@@ -449,6 +681,68 @@ namespace llamql
         return launched(fn);
     }
 
+    template <class F, bool DUMP, int MT, int RN, int KS>
+    bool gemm_split_launch(const char *fn, const GemmArgs &g, int rows, int M, hipStream_t st)
+    {
+        constexpr size_t lds = GemmSplit<MT, RN, KS>::LDS;
+        static_assert(lds + 6 * 1024 <= 160 * 1024, "LDS, with the decoders' tables");
+        static LdsGrant grant;
+        const auto kernel = &gemm_split_kernel<F, MT, RN, KS, DUMP>;
+        const hipError_t e = allow_lds(grant, reinterpret_cast<const void *>(kernel), lds);
+        if (e != hipSuccess)
+            return fail(fn, "cannot reserve %zu bytes of LDS: %s", lds, hipGetErrorString(e));
+        hipLaunchKernelGGL(kernel, dim3((unsigned)((rows + 32 * RN - 1) / (32 * RN)), (unsigned)((M + 32 * MT - 1) / (32 * MT))),
+                           dim3(RN * KS * WAVE), lds, st, g);
+        return launched(fn);
+    }
+
+    // Which kernel a shape takes: -1 for gemm_kernel, or an entry of SPLIT.  gemm_kernel's workgroup walks the whole of K
+    // alone, so where its tiles do not fill the chip (two workgroups a compute unit) the time is that walk, however little
+    // there is to multiply; gemm_split_kernel gives the walk to 2, 4 or 8 wavefronts.  Where the tiles do fill it,
+    // gemm_kernel's larger ones decode and rescale less per product.  The expected times in microseconds are fitted to
+    // measurements of the three formats:
+    //   tokens x rows x K          gemm_kernel   split (entry)
+    //   40 x 8192 x 5120, IQ3_S       39.6          23.0 (1)
+    //   130 x 5000 x 5120, Q4_K       54            33 (3)
+    //   130 x 5000 x 5120, Q6_K       60            38 (3)
+    //   12 x 1500 x 20480, Q4_K       72            35 (0)
+    //   300 x 2000 x 2048, Q4_K       22            14.6 (2)
+    //   40 x 12000 x 8192, Q6_K       71            55 (3)
+    //   199 x 5120 x 25600, Q6_K      298           270 (4)
+    //   256 x 8192 x 8192, Q4_K       84            78 (4)
+    //   20 x 25600 x 5120, Q4_K       33            34 (2)
+    //   1000 x 4096 x 4096, Q4_K      69            82 (4)
+    //   512 x 25600 x 5120, Q4_K      288           346 (4)
+    struct SplitTile
+    {
+        int mt, rn, ks;
+        double step, fixed; // microseconds: KS super-blocks, and a workgroup's start and end
+    };
+    constexpr SplitTile SPLIT[] = {{1, 1, 8, 4.6, 4.0}, {1, 2, 4, 3.8, 4.0}, {1, 4, 2, 3.4, 4.0}, {2, 2, 4, 5.9, 5.0}, {2, 4, 2, 4.9, 4.0}};
+    constexpr int CHIP_CUS = 256;
+
+    inline int gemm_split_choice(int M, int N, int K)
+    {
+        if (K > 1 << 24) // 32-bit offsets from a tile's first token
+            return -1;
+        const auto over = [](long a, long b) { return (a + b - 1) / b; };
+        const int SB = K / 256;
+        // gemm_kernel: microseconds per super-block of one workgroup alone on a compute unit, and of two sharing it
+        const double alone = M <= 32 ? 0.9 : M <= 64 ? 2.0 : 2.75, two = M <= 32 ? 1.7 : M <= 64 ? 2.75 : 4.5;
+        const long tiles = over(N, GEMM_BN) * over(M, M <= 32 ? 32 : M <= 64 ? 64 : GEMM_BM);
+        const long rest = tiles % (2 * CHIP_CUS);
+        double best = 0.95 * SB * ((double)(tiles / (2 * CHIP_CUS)) * two + (rest == 0 ? 0.0 : rest <= CHIP_CUS ? alone : two));
+        int choice = -1;
+        for (int i = 0; i < (int)(sizeof(SPLIT) / sizeof(SPLIT[0])); ++i)
+        {
+            const SplitTile &t = SPLIT[i];
+            const double us = (double)over(over(N, 32 * t.rn) * over(M, 32 * t.mt), CHIP_CUS) * ((double)over(SB, t.ks) * t.step + t.fixed);
+            if (us < best && over(M, 32 * t.mt) <= 65535) // (the grid's second extent)
+                best = us, choice = i;
+        }
+        return choice;
+    }
+
     // d_sums: the block-sum variant over weight rows [row0, row0+nrows); only the workgroups
     // whose 64-row tile meets the window are launched.
     template <class F, bool DUMP = false>
@@ -475,6 +769,16 @@ namespace llamql
                 return fail(fn, "matrix too large for the kernel's 32-bit offsets (N=%d K=%d)", N, K);
         }
         const int tile_end = DUMP ? (row0 + nrows + GEMM_BN - 1) / GEMM_BN : (N + GEMM_BN - 1) / GEMM_BN;
+        const int rows_end = DUMP ? row0 + nrows : N, rows = rows_end - g.tile0 * GEMM_BN;
+        switch (gemm_split_choice(M, N, K))
+        {
+        case 0: return gemm_split_launch<F, DUMP, 1, 1, 8>(fn, g, rows, M, st);
+        case 1: return gemm_split_launch<F, DUMP, 1, 2, 4>(fn, g, rows, M, st);
+        case 2: return gemm_split_launch<F, DUMP, 1, 4, 2>(fn, g, rows, M, st);
+        case 3: return gemm_split_launch<F, DUMP, 2, 2, 4>(fn, g, rows, M, st);
+        case 4: return gemm_split_launch<F, DUMP, 2, 4, 2>(fn, g, rows, M, st);
+        default: break;
+        }
         // few tokens: one smaller tile of tokens (a 128-token tile would rescale 128 rows for them)
         if (M <= 32)
             return gemm_launch_bm<F, DUMP, 32>(fn, g, tile_end - g.tile0, M, st);

@@ -76,6 +76,39 @@ def test_block_sums_of_the_gemm_kernel(capi, dev, oracle, fmt, M, N, K, r0, nr):
 
 
 @pytest.mark.parametrize("fmt", list(FMTS.values()), ids=list(FMTS))
+@pytest.mark.parametrize("M,N,K", [
+    (12, 97, 8960), (33, 31, 2304),    # to 8: 35 and 9 super-blocks, rows short of a tile
+    (65, 97, 768), (40, 8161, 5120),   # to 4, 32 tokens: less than a step; the last row tile of one row
+    (129, 3999, 1536),                 # to 2, 32 tokens: the last token tile of one token
+    (129, 3999, 2816),                 # to 4, 64 tokens: 11 super-blocks
+    (190, 9985, 1280),                 # to 2, 64 tokens: half a step left over, the last row tile of one row
+])
+def test_a_walk_dealt_to_wavefronts(capi, dev, oracle, fmt, M, N, K):
+    """Tiles whose super-blocks are dealt to several wavefronts: rows, tokens and super-blocks left over.  Every element
+    written and near the oracle's, the block sums of a window that starts inside a tile bit for bit, and the same bits
+    again.  The tolerance is the one of the undivided walk: the parts are sums of the same products."""
+    import torch
+
+    W = synth.weights_numpy(fmt, N, K, 11 + M + N)
+    q8 = oracle.quantize(synth.activations_numpy(M, K, 13 + K))
+    wd = upload_weights(capi, dev, fmt, W)
+    qd = upload_q8(dev, q8)
+    y, again = (torch.full((M, N), float("nan"), device=dev) for _ in range(2))
+    capi.gemm(fmt, wd, qd, M, N, K, out=y)
+    capi.gemm(fmt, wd, qd, M, N, K, out=again)
+    r0 = max(0, N - 75)
+    s = capi.gemm_block_sums(fmt, wd, qd, M, N, K, r0, N - r0)
+    sync()
+    assert torch.equal(y, again)
+    got = y.cpu().numpy()
+    C = oracle.gemm(fmt, W, K, q8)
+    assert rel_err(got, C) <= TOL[fmt] * 1e-2
+    assert np.abs(got - C).max() <= 1e-4 * np.abs(C).max()
+    _, sums = oracle.gemm(fmt, W, K, q8, n0=r0, n1=N, want_sums=True)
+    assert np.array_equal(s.cpu().numpy(), sums)
+
+
+@pytest.mark.parametrize("fmt", list(FMTS.values()), ids=list(FMTS))
 def test_more_tiles_than_the_chip_holds(capi, dev, oracle, fmt):
     """More tiles than the chip holds at once, with a sparsely filled last round of workgroups
     (580 tiles of 128 x 64 on 512 workgroup slots), ragged in both directions (130 tokens: the
