@@ -1,6 +1,6 @@
 // Linear layers with bf16 weights in matrix-unit tiles, for gfx950.
 //
-// Up to 16 rows (decoding): one workgroup per 16-row tile of W, its wavefronts dealing the
+// Up to 16 rows (decoding): one workgroup per 16-row tile of W (or half of one), its wavefronts dealing the
 // k-steps among themselves and summing through LDS; each weight byte is read once, a contiguous
 // kilobyte per load instruction, several in flight per wavefront.  The rows of A are the second
 // matrix operand (16 columns, those past M ignored).  HBM-bound.
@@ -10,28 +10,105 @@
 namespace llamql
 {
     // ---- up to 16 rows ------------------------------------------------------------------------
-    // RT tiles of W per workgroup (2 for a gate tile beside its up tile, or to share the rows), NW wavefronts, U k-steps
+    // fp32 rows into LDS (and h_out, from the first workgroup), normed, as T.  R rows at a time are asked for and summed,
+    // and all rows share one barrier: a row at a time, eight rows of 768 values took 6 us of a 9 us launch.
+    template <typename T, int NW, int R>
+    __device__ __forceinline__ void norm_rows(const LinearArgs &p, T *h, int ldh, bool record)
+    {
+        typedef T t4 __attribute__((ext_vector_type(4)));
+        __shared__ float s_sum[SMALL_M][NW];
+        static_assert(SMALL_M % R == 0, "sums of whole groups");
+        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+        const auto row = [&](int m) { return reinterpret_cast<const f32x4 *>(static_cast<const float *>(p.a) + (size_t)(m < p.M ? m : p.M - 1) * p.lda); };
+        for (int m0 = 0; m0 < p.M; m0 += R)
+        {
+            float sum[R] = {};
+            for (int i = threadIdx.x; i < p.K / 4; i += NW * 64)
+            {
+                f32x4 v[R];
+#pragma unroll
+                for (int k = 0; k < R; ++k)
+                    v[k] = row(m0 + k)[i];
+#pragma unroll
+                for (int k = 0; k < R; ++k)
+                    sum[k] += v[k][0] * v[k][0] + v[k][1] * v[k][1] + v[k][2] * v[k][2] + v[k][3] * v[k][3];
+            }
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1)
+#pragma unroll
+                for (int k = 0; k < R; ++k)
+                    sum[k] += __shfl_xor(sum[k], off, 64);
+            if (lane == 0)
+            {
+#pragma unroll
+                for (int k = 0; k < R; ++k)
+                    s_sum[m0 + k][wave] = sum[k];
+            }
+        }
+        __syncthreads();
+        for (int m0 = 0; m0 < p.M; m0 += R)
+        {
+            float inv[R];
+#pragma unroll
+            for (int k = 0; k < R; ++k)
+            {
+                float total = 0.0f;
+#pragma unroll
+                for (int w = 0; w < NW; ++w)
+                    total += s_sum[m0 + k][w];
+                inv[k] = 1.0f / sqrtf(total / (float)p.k_real + p.eps);
+            }
+            for (int i = threadIdx.x; i < p.K / 4; i += NW * 64)
+            {
+                f32x4 v[R];
+                const f32x4 scale = reinterpret_cast<const f32x4 *>(p.norm)[i];
+#pragma unroll
+                for (int k = 0; k < R; ++k)
+                    v[k] = row(m0 + k)[i];
+#pragma unroll
+                for (int k = 0; k < R; ++k)
+                    if (m0 + k < p.M)
+                    {
+                        const t4 o = __builtin_convertvector(v[k] * inv[k] * scale, t4);
+                        *reinterpret_cast<t4 *>(h + (size_t)(m0 + k) * ldh + 4 * i) = o;
+                        if (record)
+                            *reinterpret_cast<t4 *>(static_cast<T *>(p.h_out) + (size_t)(m0 + k) * p.K + 4 * i) = o;
+                    }
+            }
+        }
+        __syncthreads();
+    }
+
+    // RT tiles of W per workgroup (2 for a gate tile beside its up tile, or to share the rows), NW wavefronts, U steps
     // in flight per wavefront.  NORM: A is fp32, normed by the workgroup into LDS (as T) while the
     // first weights are on their way.
-    template <typename T, int NW, int RT, bool NORM>
+    // HALF: up to 8 rows of A, and a workgroup for 8 rows of W, half a tile: a step is two k-steps, W's rows of the second
+    // beside those of the first as the matrix unit's other 8 rows, A's likewise as its other 8 columns, and of the product
+    // the two blocks that match are kept.  Twice the workgroups, for layers of fewer tiles than the chip has compute units.
+    template <typename T, int NW, int RT, bool NORM, bool HALF = false>
     __device__ __forceinline__ void linear_small_tile(const LinearArgs &p, int block)
     {
         using O = Operand<T>;
         using V = typename O::V;
+        static_assert(!HALF || RT == 1, "half a tile");
         constexpr int U = RT == 1 ? 8 : 4;
+        constexpr int STEP = HALF ? 2 : 1;   // k-steps (their number is even)
         constexpr int LPAD = 16 / sizeof(T); // between LDS rows: the rows start in different banks
         extern __shared__ __attribute__((aligned(16))) char smem[];
         __shared__ __attribute__((aligned(16))) float s_red[NW][RT][64][4];
-        __shared__ float s_sum[NW];
         const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
         const int n = lane & 15, g = lane >> 4;
         const int z = blockIdx.y;
-        const int ksteps = p.K >> 5;
+        const int ksteps = p.K >> 5, steps = ksteps / STEP;
+        const int second = HALF ? n >> 3 : 0;                                 // which k-step of a step is this lane's
+        const int piece = HALF ? g * 16 + (block & 1) * 8 + (n & 7) : lane;   // of a k-step of W
+        const int tile = HALF ? block >> 1 : block * RT;
+        const int row = HALF ? n & 7 : n;                                     // of A
 
         const u32x4 *w[RT];
 #pragma unroll
         for (int t = 0; t < RT; ++t)
-            w[t] = weight_tile(static_cast<const bf16 *>(p.w) + (size_t)z * p.w_stride - (t && (block * RT + t) * 16 >= p.N ? (size_t)ksteps * 512 : 0), (size_t)block * RT + t, ksteps, lane);
+            w[t] = weight_tile(static_cast<const bf16 *>(p.w) + (size_t)z * p.w_stride - (t && (tile + t) * 16 >= p.N ? (size_t)ksteps * 512 : 0), (size_t)tile + t, ksteps, piece) + second * 64;
         u32x4 next[RT][U];
         auto fetch = [&](int s0) __attribute__((always_inline)) {
 #pragma unroll
@@ -40,48 +117,32 @@ namespace llamql
                 const int s = s0 + u * NW;
 #pragma unroll
                 for (int t = 0; t < RT; ++t)
-                    next[t][u] = w[t][(size_t)(s < ksteps ? s : wave < ksteps ? wave : 0) * 64];
+                    next[t][u] = w[t][(size_t)(s < steps ? s : wave < steps ? wave : 0) * (64 * STEP)];
             }
         };
         fetch(wave);
 
         const T *arow;
-        if (NORM)
+        if constexpr (NORM)
         {
             T *h = reinterpret_cast<T *>(smem);
             const int ldh = p.K + LPAD;
-            for (int m = 0; m < p.M; ++m)
-            {
-                const f32x4 *x = reinterpret_cast<const f32x4 *>(static_cast<const float *>(p.a) + (size_t)m * p.lda);
-                float sum = 0.0f;
-                for (int i = threadIdx.x; i < p.K / 4; i += NW * 64)
-                {
-                    const f32x4 v = x[i];
-                    sum += v[0] * v[0] + v[1] * v[1] + v[2] * v[2] + v[3] * v[3];
-                }
-                sum = block_sum<NW * 64>(sum, s_sum);
-                const float inv = 1.0f / sqrtf(sum / (float)p.k_real + p.eps);
-                typedef T t4 __attribute__((ext_vector_type(4)));
-                for (int i = threadIdx.x; i < p.K / 4; i += NW * 64)
-                {
-                    const f32x4 v = x[i] * inv * reinterpret_cast<const f32x4 *>(p.norm)[i];
-                    const t4 o = __builtin_convertvector(v, t4);
-                    *reinterpret_cast<t4 *>(h + (size_t)m * ldh + 4 * i) = o;
-                    if (p.h_out && block == 0)
-                        *reinterpret_cast<t4 *>(static_cast<T *>(p.h_out) + (size_t)m * p.K + 4 * i) = o;
-                }
-            }
-            __syncthreads();
-            arow = h + (size_t)(n < p.M ? n : 0) * ldh + 8 * g;
+            const bool record = p.h_out && block == 0;
+            if (p.M == 1)
+                norm_rows<T, NW, 1>(p, h, ldh, record);
+            else
+                norm_rows<T, NW, 4>(p, h, ldh, record);
+            arow = h + (size_t)(row < p.M ? row : 0) * ldh + 8 * g;
         }
         else
-            arow = static_cast<const T *>(p.a) + (size_t)z * p.a_stride + (size_t)(n < p.M ? n : 0) * p.lda + 8 * g;
+            arow = static_cast<const T *>(p.a) + (size_t)z * p.a_stride + (size_t)(row < p.M ? row : 0) * p.lda + 8 * g;
+        arow += second * 32;
 
         f32x4 acc[RT];
 #pragma unroll
         for (int t = 0; t < RT; ++t)
             acc[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-        for (int s0 = wave; s0 < ksteps; s0 += NW * U)
+        for (int s0 = wave; s0 < steps; s0 += NW * U)
         {
             u32x4 cur[RT][U];
 #pragma unroll
@@ -89,26 +150,34 @@ namespace llamql
 #pragma unroll
                 for (int t = 0; t < RT; ++t)
                     cur[t][u] = next[t][u];
-            if (s0 + NW * U < ksteps)
+            if (s0 + NW * U < steps)
                 fetch(s0 + NW * U);
+            // rows of bf16 are asked for ahead of the products (2048 x 8192 and one row: 11.0 -> 9.2 us); rows of fp32 would
+            // take the registers of a second workgroup (32768 x 2048 and one row: 43 -> 52 us)
+            constexpr bool AHEAD = sizeof(T) == 2;
+            V b[AHEAD ? U : 1];
+            if constexpr (AHEAD)
+            {
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+                    b[u] = O::load(arow + (s0 + u * NW < steps ? s0 + u * NW : s0) * (32 * STEP));
+            }
 #pragma unroll
             for (int u = 0; u < U; ++u)
-            {
-                const int s = s0 + u * NW;
-                if (s < ksteps)
+                if (s0 + u * NW < steps)
                 {
-                    const V b = O::load(arow + s * 32);
+                    if constexpr (!AHEAD)
+                        b[0] = O::load(arow + (s0 + u * NW) * (32 * STEP));
 #pragma unroll
                     for (int t = 0; t < RT; ++t)
-                        acc[t] = O::mma(O::from_weights(cur[t][u]), b, acc[t]);
+                        acc[t] = O::mma(O::from_weights(cur[t][u]), b[AHEAD ? u : 0], acc[t]);
                 }
-            }
         }
 #pragma unroll
         for (int t = 0; t < RT; ++t)
             *reinterpret_cast<f32x4 *>(s_red[wave][t][lane]) = acc[t];
         __syncthreads();
-        if (threadIdx.x < 64 && n < p.M)
+        if (threadIdx.x < 64 && n < p.M && (!HALF || (n < 8 && g < 2)))
         {
             f32x4 sum[RT];
 #pragma unroll
@@ -118,11 +187,19 @@ namespace llamql
 #pragma unroll
                 for (int v = 1; v < NW; ++v)
                     sum[t] = sum[t] + *reinterpret_cast<const f32x4 *>(s_red[v][t][lane]);
+                if (HALF)
+                {
+#pragma unroll
+                    for (int v = 0; v < NW; ++v) // rows and columns 8 ..
+                        sum[t] = sum[t] + *reinterpret_cast<const f32x4 *>(s_red[v][t][lane + 40]);
+                }
             }
             const size_t elem = p.out == LLAM_SEQ_OUT_F32 || p.out == LLAM_SEQ_OUT_ADD ? 4 : sizeof(T);
             char *y = static_cast<char *>(p.y) + (size_t)z * p.y_stride * elem;
             if (RT == 2 && is_gated(p.out))
                 store4<T>(p, y, n, block * 16 + 4 * g, gated4(p, sum[0], sum[RT - 1]));
+            else if (HALF)
+                store4<T>(p, y, n, block * 8 + 4 * g, sum[0]);
             else
             {
                 // (the last tile of an odd number of them is a copy)
@@ -134,11 +211,11 @@ namespace llamql
         }
     }
 
-    template <typename T, int NW, int RT, bool NORM>
+    template <typename T, int NW, int RT, bool NORM, bool HALF>
     __global__ void __launch_bounds__(NW * 64)
         linear_small_kernel(LinearArgs p)
     {
-        linear_small_tile<T, NW, RT, NORM>(p, blockIdx.x);
+        linear_small_tile<T, NW, RT, NORM, HALF>(p, blockIdx.x);
     }
 
     // Two layers over the same rows: the first `blocks` workgroups belong to p.
@@ -152,15 +229,30 @@ namespace llamql
 
     namespace
     {
-        template <typename T, int NW, int RT, bool NORM>
+        template <typename T, int NW, int RT, bool NORM, bool HALF = false>
         bool small_launch(const char *fn, const LinearArgs &a, int batch, hipStream_t st)
         {
             static LdsGrant grant;
             const size_t lds = NORM ? (size_t)a.M * (a.K + 16 / sizeof(T)) * sizeof(T) : 0;
-            if (lds > 32 * 1024 && allow_lds(grant, reinterpret_cast<const void *>(&linear_small_kernel<T, NW, RT, NORM>), 64 * 1024) != hipSuccess)
+            const auto kernel = &linear_small_kernel<T, NW, RT, NORM, HALF>;
+            if (lds > 32 * 1024 && allow_lds(grant, reinterpret_cast<const void *>(kernel), 64 * 1024) != hipSuccess)
                 return fail(fn, "cannot reserve %zu bytes of LDS", lds);
-            hipLaunchKernelGGL((linear_small_kernel<T, NW, RT, NORM>), dim3(a.N / 16 / RT, batch), dim3(NW * 64), lds, st, a);
+            hipLaunchKernelGGL(kernel, dim3(a.N / (HALF ? 8 : 16 * RT), batch), dim3(NW * 64), lds, st, a);
             return launched(fn);
+        }
+        template <typename T, int NW, bool NORM>
+        bool small_tiles(const char *fn, const LinearArgs &a, int batch, hipStream_t st)
+        {
+            // Half tiles where whole ones leave compute units without a workgroup and a workgroup has much to do
+            // (M x N x K, us, whole and half tiles, A ahead of neither):
+            //   8 x 2048 x 8192   bf16 16.4, 11.7  fp32 24.3, 16.2     3 x 2048 x 10240  bf16 19.9, 14.5  fp32 29.6, 19.2
+            //   8 x 2048 x 2048   bf16  4.6,  4.7  fp32  6.8,  5.8     8 x 768 x 2048    bf16  4.1,  4.0  fp32  6.1,  5.1
+            //   8 x 3072 x 2048   bf16  5.7,  6.8  fp32  8.0,  8.9     8 x 6160 x 2048   bf16  8.6, 11.2  fp32 12.2, 15.4
+            // (fp32: the products take as long as the weights, so a workgroup's share counts from fewer k-steps on)
+            constexpr int CUS = 256;
+            const long tiles = (long)a.N / 16 * batch;
+            const bool half = a.M <= 8 && tiles < CUS && (a.K >= 4096 || (sizeof(T) == 4 && tiles <= CUS / 2));
+            return half ? small_launch<T, NW, 1, NORM, true>(fn, a, batch, st) : small_launch<T, NW, 1, NORM>(fn, a, batch, st);
         }
         template <typename T>
         bool small_dispatch(const char *fn, const LinearArgs &a, int batch, hipStream_t st)
@@ -168,10 +260,10 @@ namespace llamql
             const bool gated = is_gated(a.out);
             const bool wide = a.K >= 1024;
             if (a.norm)
-                return gated ? small_launch<T, 8, 2, true>(fn, a, batch, st) : small_launch<T, 8, 1, true>(fn, a, batch, st);
+                return gated ? small_launch<T, 8, 2, true>(fn, a, batch, st) : small_tiles<T, 8, true>(fn, a, batch, st);
             if (gated)
                 return small_launch<T, 8, 2, false>(fn, a, batch, st);
-            return wide ? small_launch<T, 8, 1, false>(fn, a, batch, st) : small_launch<T, 4, 1, false>(fn, a, batch, st);
+            return wide ? small_tiles<T, 8, false>(fn, a, batch, st) : small_tiles<T, 4, false>(fn, a, batch, st);
         }
     } // namespace
 

@@ -1,0 +1,51 @@
+"""Linear layers of up to 16 rows against sums in 64 bits: half and whole tiles at the edges of their rule, the fused norm."""
+import ctypes
+
+import pytest
+
+from llaminar_amd import sequence as sq
+from tests.test_gpu_linear_tiled import tiles
+
+pytestmark = pytest.mark.gpu
+
+F32, BF16 = sq.F32, sq.BF16
+
+# half tiles: one to eight rows, one tile, the most tiles (128 and 255), K of one step, of fewer steps than wavefronts, of
+# an odd number of steps a wavefront; whole tiles on the other side: nine rows, 129 and 256 tiles, K below 4096
+SHAPES = [(1, 16, 64), (8, 16, 4096), (8, 2048, 128), (7, 2064, 1088), (3, 2048, 10304), (8, 4080, 4160), (9, 2048, 4096),
+          (8, 4096, 4096), (5, 4096, 4032), (16, 48, 8256)]
+
+
+@pytest.mark.parametrize("dtype", [BF16, F32])
+@pytest.mark.parametrize("norm", [False, True])
+@pytest.mark.parametrize("M,N,K", SHAPES + [(1, 32, 8192), (2, 80, 4096), (3, 32, 2688), (4, 2048, 2048), (5, 16, 1600), (16, 32, 512)])
+def test_few_rows(dev, M, N, K, norm, dtype):
+    import torch
+
+    if norm and M * K > 8192:
+        pytest.skip("a fused norm takes up to 8192 values")
+    torch.manual_seed(M + N + K)
+    a = torch.randn(M, K + 64, device=dev)[:, :K]
+    w = torch.randn(N, K, device=dev).bfloat16()
+    scale, real = torch.rand(K, device=dev) + 0.5, K - 3
+    y = torch.full((M + 1, N + 4), 5.0, device=dev)
+    h = torch.zeros(M, K, device=dev, dtype=torch.float32 if dtype == F32 else torch.bfloat16)
+    given = a if norm or dtype == F32 else torch.nn.functional.pad(a.bfloat16(), (0, 64))[:, :K]
+    laid = tiles(w)
+    args = sq.LinearArgs(d_a=given.data_ptr(), d_w=laid.data_ptr(), d_y=y.data_ptr(), M=M, N=N, K=K, lda=K + 64, ldy=N + 4, out=sq.OUT_F32, batch=1)
+    if norm:
+        args.d_norm, args.d_h_out, args.k_real, args.eps = scale.data_ptr(), h.data_ptr(), real, 1e-5
+    assert sq.load().llam_seq_linear(ctypes.byref(args), dtype, 0, torch.cuda.current_stream().cuda_stream), sq.load().llam_ql_last_error()
+    torch.cuda.synchronize()
+    x = given.double()
+    if norm:
+        x = x / torch.sqrt((x * x).sum(1, keepdim=True) / real + 1e-5) * scale.double()
+        # the sum of squares: off by K 2^-24 of itself at most, its root by half of that; then three products and a rounding to T
+        # (bf16: 8 significant bits, so half a unit of the last is 2^-8 of the value at most)
+        relative = K * 2.0 ** -25 + 6 * 2.0 ** -24 + (2.0 ** -8 if dtype == BF16 else 0.0)
+        assert ((h.double() - x).abs() <= relative * x.abs()).all()
+        x = h.double()
+    # K products in 32 bits, in any order: each addition is off by 2^-23 of a partial sum at most
+    bound = (K + 1) * 2.0 ** -23 * (x.abs() @ w.double().abs().T)
+    assert ((y[:M, :N].double() - x @ w.double().T).abs() <= bound).all()
+    assert (y[M:] == 5.0).all() and (y[:, N:] == 5.0).all(), "written past the output"
