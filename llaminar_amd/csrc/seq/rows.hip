@@ -138,33 +138,53 @@ namespace llamql
             p.weights[m * (p.top + 1) + p.top] = sigmoidf(z[p.experts]);
     }
 
-    // Few rows.  Workgroup = 16 outputs of one expert of one token.  With a single row all workgroups
-    // choose the token's experts for themselves from the logits, and the first records the choice for
-    // the down projections; with more, a launch before has chosen.
+    // Few rows.  Workgroup = 16 outputs of one expert, for every token that chose it: the tokens are the columns of the
+    // matrix unit's second operand, so an expert's weights are read once however many chose it (the shared one: all).  Of
+    // the workgroups of a (token, choice) pair those of the first token to choose the expert work, the others end.
+    // With a single row all workgroups choose the token's experts for themselves from the logits, and the first records
+    // the choice for the down projections; with more, a launch before has chosen.
+    // Bound by the weights: 8 tokens, 6 of 64 experts of 1408 x 2048 each and a shared one of 2816, 56 us when each token
+    // read its own and 44 now (about 200 MB of distinct weights).  The bits are the same: columns do not meet.
     constexpr int EXPERT_WAVES = 8;
     template <typename T>
     __global__ void __launch_bounds__(EXPERT_WAVES * 64)
-        expert_up_small_kernel(ExpertArgs p)
+        expert_up_small_kernel(ExpertArgs p, int M)
     {
         using O = Operand<T>;
         typedef T t4 __attribute__((ext_vector_type(4)));
         __shared__ __attribute__((aligned(16))) float s_red[EXPERT_WAVES][64][4];
-        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = lane >> 4;
+        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n = lane & 15, g = lane >> 4;
         const int job = blockIdx.y, m = blockIdx.z; // jobs 0 .. top - 1: chosen experts; top: the shared one
         const bool shared = job == p.top;
         const int tile = blockIdx.x;
         const float *z = p.logits + (size_t)m * p.ldz;
-        int id = 0;
-        float weight = 0.0f;
-        if (!shared)
+        int expert = 0;
+        unsigned long long mine = n < M ? 1 : 0; // which of token n's choices the expert is (several: logits that are not numbers)
+        if (shared)
         {
-            if (tile * 16 >= p.ff)
+            if (m > 0 || tile * 16 >= p.shared_ff)
                 return;
-            if (p.routed)
-                id = p.ids[m * p.top + job];
-            else
-                route_wave(z, p.experts, p.top, lane, id, weight);
-            if (!p.routed && tile == 0 && job == 0 && wave == 0)
+        }
+        else if (tile * 16 >= p.ff)
+            return;
+        else if (p.routed)
+        {
+            expert = p.ids[m * p.top + job];
+            mine = 0;
+            for (int j = g; j < p.top; j += 4)
+                if (n < M && p.ids[n * p.top + j] == expert)
+                    mine |= 1ull << j;
+            mine |= __shfl_xor(mine, 16, 64);
+            mine |= __shfl_xor(mine, 32, 64);
+            if ((__ballot(mine != 0) & ((1ull << m) - 1)) != 0)
+                return; // an earlier token's workgroup
+        }
+        else
+        {
+            int id;
+            float weight;
+            route_wave(z, p.experts, p.top, lane, id, weight);
+            if (tile == 0 && job == 0 && wave == 0)
             {
                 if (lane < p.top)
                 {
@@ -174,13 +194,12 @@ namespace llamql
                 if (lane == 0 && p.shared_ff)
                     p.weights[m * (p.top + 1) + p.top] = sigmoidf(z[p.experts]);
             }
+            expert = __shfl(id, job, 64);
+            mine <<= job;
         }
-        else if (tile * 16 >= p.shared_ff)
-            return;
-        const int expert = __shfl(id, shared ? 0 : job, 64);
         const int ksteps = p.K >> 5;
         const u32x4 *w = weight_tile(shared ? p.shared_up : p.up + (size_t)expert * p.up_stride, tile, ksteps, lane);
-        const T *h = static_cast<const T *>(p.h) + (size_t)m * p.K + 8 * g;
+        const T *h = static_cast<const T *>(p.h) + (size_t)(mine != 0 ? n : m) * p.K + 8 * g; // (other columns: m's, unused)
         f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
         constexpr int U = 8;
         for (int s0 = wave; s0 < ksteps; s0 += EXPERT_WAVES * U)
@@ -202,7 +221,7 @@ namespace llamql
         }
         *reinterpret_cast<f32x4 *>(s_red[wave][lane]) = acc;
         __syncthreads();
-        if (threadIdx.x < 64 && (lane & 15) == 0)
+        if (threadIdx.x < 64 && mine != 0)
         {
             f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
@@ -214,8 +233,13 @@ namespace llamql
                 const float y = fmaxf(v[r], 0.0f);
                 v[r] = y * y;
             }
-            T *act = static_cast<T *>(p.act) + (size_t)m * (p.top * p.ff + p.shared_ff) + (size_t)job * p.ff;
-            *reinterpret_cast<t4 *>(act + tile * 16 + 4 * g) = __builtin_convertvector(v, t4);
+            T *act = static_cast<T *>(p.act) + (size_t)n * (p.top * p.ff + p.shared_ff) + tile * 16 + 4 * g;
+            do
+            {
+                const int at = shared ? p.top : __builtin_ctzll(mine);
+                *reinterpret_cast<t4 *>(act + (size_t)at * p.ff) = __builtin_convertvector(v, t4);
+                mine &= mine - 1;
+            } while (mine != 0);
         }
     }
 
@@ -409,7 +433,7 @@ namespace llamql
             {
                 const int widest = p.shared_ff > p.ff ? p.shared_ff : p.ff;
                 hipLaunchKernelGGL(expert_up_small_kernel<T>, dim3(widest / 16, p.top + (p.shared_ff ? 1 : 0), M),
-                                   dim3(EXPERT_WAVES * 64), 0, st, p);
+                                   dim3(EXPERT_WAVES * 64), 0, st, p, M);
                 if (!launched(fn))
                     return false;
                 hipLaunchKernelGGL(expert_down_small_kernel<T>, dim3(p.N / 16, M), dim3(EXPERT_WAVES * 64), 0, st, p);
