@@ -7,13 +7,26 @@
 // More rows (prompts): linear_tiled.hip.
 #include "linear.h"
 
+#include <type_traits>
+
 namespace llamql
 {
     // ---- up to 16 rows ------------------------------------------------------------------------
-    // fp32 rows into LDS (and h_out, from the first workgroup), normed, as T.  R rows at a time are asked for and summed,
+    constexpr int NORM_PAD = 8; // between normed rows in LDS: they start in different banks
+
+    template <typename T>
+    size_t norm_lds(const LinearArgs &a)
+    {
+        return (size_t)(sizeof(T) == 4 ? 3 : 1) * a.M * (a.K + NORM_PAD) * sizeof(bf16);
+    }
+
+    // fp32 rows normed, into h_out as T (from the first workgroup) and into LDS: as bf16, or, for T fp32, in three bf16
+    // pieces that add up to the value (8 + 8 + 8 significant bits, cut off; infinities in the first alone), the pieces
+    // p.M * ldh apart.  Three products of bf16 take 48 cycles of the matrix unit a k-step, one of fp32 256 (3 x 32768 x
+    // 2048: 45 -> 36.6 us; the error against 64 bits falls from 3.0e-7 to 2.0e-7).  R rows at a time are asked for and summed,
     // and all rows share one barrier: a row at a time, eight rows of 768 values took 6 us of a 9 us launch.
     template <typename T, int NW, int R>
-    __device__ __forceinline__ void norm_rows(const LinearArgs &p, T *h, int ldh, bool record)
+    __device__ __forceinline__ void norm_rows(const LinearArgs &p, bf16 *h, int ldh, bool record)
     {
         typedef T t4 __attribute__((ext_vector_type(4)));
         __shared__ float s_sum[SMALL_M][NW];
@@ -70,7 +83,26 @@ namespace llamql
                     if (m0 + k < p.M)
                     {
                         const t4 o = __builtin_convertvector(v[k] * inv[k] * scale, t4);
-                        *reinterpret_cast<t4 *>(h + (size_t)(m0 + k) * ldh + 4 * i) = o;
+                        bf16 *to = h + (size_t)(m0 + k) * ldh + 4 * i;
+                        if constexpr (sizeof(T) == 2)
+                            *reinterpret_cast<t4 *>(to) = o;
+                        else
+                        {
+                            f32x4 rest = o;
+#pragma unroll
+                            for (int piece = 0; piece < 3; ++piece, to += p.M * ldh)
+                            {
+                                u32x4 cut = __builtin_bit_cast(u32x4, rest);
+                                typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+                                *reinterpret_cast<u32x2 *>(to) = u32x2{__builtin_amdgcn_perm(cut[1], cut[0], 0x07060302u),
+                                                                       __builtin_amdgcn_perm(cut[3], cut[2], 0x07060302u)}; // upper halves
+                                cut &= 0xffff0000u;
+                                const f32x4 less = rest - __builtin_bit_cast(f32x4, cut);
+#pragma unroll
+                                for (int e = 0; e < 4; ++e)
+                                    rest[e] = fabsf(rest[e]) == INFINITY ? 0.0f : less[e];
+                            }
+                        }
                         if (record)
                             *reinterpret_cast<t4 *>(static_cast<T *>(p.h_out) + (size_t)(m0 + k) * p.K + 4 * i) = o;
                     }
@@ -93,7 +125,7 @@ namespace llamql
         static_assert(!HALF || RT == 1, "half a tile");
         constexpr int U = RT == 1 ? 8 : 4;
         constexpr int STEP = HALF ? 2 : 1;   // k-steps (their number is even)
-        constexpr int LPAD = 16 / sizeof(T); // between LDS rows: the rows start in different banks
+        constexpr bool CUT = NORM && sizeof(T) == 4; // rows in three bf16 pieces
         extern __shared__ __attribute__((aligned(16))) char smem[];
         __shared__ __attribute__((aligned(16))) float s_red[NW][RT][64][4];
         const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -122,11 +154,12 @@ namespace llamql
         };
         fetch(wave);
 
-        const T *arow;
+        using A = std::conditional_t<NORM, bf16, T>;
+        const int ldh = p.K + NORM_PAD;
+        const A *arow;
         if constexpr (NORM)
         {
-            T *h = reinterpret_cast<T *>(smem);
-            const int ldh = p.K + LPAD;
+            bf16 *h = reinterpret_cast<bf16 *>(smem);
             const bool record = p.h_out && block == 0;
             if (p.M == 1)
                 norm_rows<T, NW, 1>(p, h, ldh, record);
@@ -154,7 +187,7 @@ namespace llamql
                 fetch(s0 + NW * U);
             // rows of bf16 are asked for ahead of the products (2048 x 8192 and one row: 11.0 -> 9.2 us); rows of fp32 would
             // take the registers of a second workgroup (32768 x 2048 and one row: 43 -> 52 us)
-            constexpr bool AHEAD = sizeof(T) == 2;
+            constexpr bool AHEAD = sizeof(T) == 2, LATE = !AHEAD && !CUT;
             V b[AHEAD ? U : 1];
             if constexpr (AHEAD)
             {
@@ -166,7 +199,19 @@ namespace llamql
             for (int u = 0; u < U; ++u)
                 if (s0 + u * NW < steps)
                 {
-                    if constexpr (!AHEAD)
+                    if constexpr (CUT)
+                    {
+#pragma unroll
+                        for (int piece = 2; piece >= 0; --piece)
+                        {
+                            const bf16x8 part = Operand<bf16>::load(arow + piece * p.M * ldh + (s0 + u * NW) * (32 * STEP));
+#pragma unroll
+                            for (int t = 0; t < RT; ++t)
+                                acc[t] = Operand<bf16>::mma(Operand<bf16>::from_weights(cur[t][u]), part, acc[t]);
+                        }
+                        continue;
+                    }
+                    if constexpr (LATE)
                         b[0] = O::load(arow + (s0 + u * NW) * (32 * STEP));
 #pragma unroll
                     for (int t = 0; t < RT; ++t)
@@ -233,7 +278,7 @@ namespace llamql
         bool small_launch(const char *fn, const LinearArgs &a, int batch, hipStream_t st)
         {
             static LdsGrant grant;
-            const size_t lds = NORM ? (size_t)a.M * (a.K + 16 / sizeof(T)) * sizeof(T) : 0;
+            const size_t lds = NORM ? norm_lds<T>(a) : 0;
             const auto kernel = &linear_small_kernel<T, NW, RT, NORM, HALF>;
             if (lds > 32 * 1024 && allow_lds(grant, reinterpret_cast<const void *>(kernel), 64 * 1024) != hipSuccess)
                 return fail(fn, "cannot reserve %zu bytes of LDS", lds);
@@ -273,7 +318,7 @@ namespace llamql
         bool small_pair_launch(const char *fn, const LinearArgs &a, const LinearArgs &b, hipStream_t st)
         {
             static LdsGrant grant;
-            const size_t lds = NORM ? (size_t)a.M * (a.K + 16 / sizeof(T)) * sizeof(T) : 0;
+            const size_t lds = NORM ? norm_lds<T>(a) : 0;
             if (lds > 32 * 1024 && allow_lds(grant, reinterpret_cast<const void *>(&linear_small_pair_kernel<T, 8, NORM>), 64 * 1024) != hipSuccess)
                 return fail(fn, "cannot reserve %zu bytes of LDS", lds);
             const int blocks = ceil_div(a.N, 32);

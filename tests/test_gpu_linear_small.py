@@ -16,14 +16,15 @@ SHAPES = [(1, 16, 64), (8, 16, 4096), (8, 2048, 128), (7, 2064, 1088), (3, 2048,
           (8, 4096, 4096), (5, 4096, 4032), (16, 48, 8256)]
 
 
+# a fused norm takes up to 8192 values: all of them in one row and in sixteen, half and whole tiles
+NORMED = [(1, 16, 64), (7, 2064, 1088), (1, 32, 8192), (2, 80, 4096), (3, 32, 2688), (4, 2048, 2048), (5, 4112, 1600), (16, 32, 512)]
+
+
 @pytest.mark.parametrize("dtype", [BF16, F32])
-@pytest.mark.parametrize("norm", [False, True])
-@pytest.mark.parametrize("M,N,K", SHAPES + [(1, 32, 8192), (2, 80, 4096), (3, 32, 2688), (4, 2048, 2048), (5, 16, 1600), (16, 32, 512)])
+@pytest.mark.parametrize("M,N,K,norm", [(*s, False) for s in SHAPES] + [(*s, True) for s in NORMED])
 def test_few_rows(dev, M, N, K, norm, dtype):
     import torch
 
-    if norm and M * K > 8192:
-        pytest.skip("a fused norm takes up to 8192 values")
     torch.manual_seed(M + N + K)
     a = torch.randn(M, K + 64, device=dev)[:, :K]
     w = torch.randn(N, K, device=dev).bfloat16()
@@ -49,3 +50,20 @@ def test_few_rows(dev, M, N, K, norm, dtype):
     bound = (K + 1) * 2.0 ** -23 * (x.abs() @ w.double().abs().T)
     assert ((y[:M, :N].double() - x @ w.double().T).abs() <= bound).all()
     assert (y[M:] == 5.0).all() and (y[:, N:] == 5.0).all(), "written past the output"
+
+
+def test_a_normed_value_beyond_32_bits(dev):
+    """An infinite normed value of a row of fp32, which is cut in pieces: infinite sums in that row, none in the other."""
+    import torch
+
+    torch.manual_seed(0)
+    a, w = torch.randn(2, 2048, device=dev), torch.randn(64, 2048, device=dev).bfloat16()
+    scale = torch.ones(2048, device=dev)
+    a[0, 5], a[1, 5], scale[5] = 10.0, 0.0, 3e38
+    y, laid = torch.zeros(2, 64, device=dev), tiles(w)
+    args = sq.LinearArgs(d_a=a.data_ptr(), d_w=laid.data_ptr(), d_y=y.data_ptr(), M=2, N=64, K=2048, lda=2048, ldy=64, out=sq.OUT_F32, batch=1)
+    args.d_norm, args.k_real, args.eps = scale.data_ptr(), 2048, 1e-5
+    assert sq.load().llam_seq_linear(ctypes.byref(args), F32, 0, torch.cuda.current_stream().cuda_stream), sq.load().llam_ql_last_error()
+    torch.cuda.synchronize()
+    assert (w[:, 5] != 0).all()
+    assert torch.equal(y[0], torch.sign(w[:, 5].float()) * float("inf")) and torch.isfinite(y[1]).all()
