@@ -123,7 +123,7 @@ namespace llamql
         using O = Operand<T>;
         using V = typename O::V;
         static_assert(!HALF || RT == 1, "half a tile");
-        constexpr int U = RT == 1 ? 8 : 4;
+        constexpr int U = RT == 1 && (NORM || sizeof(T) == 2) ? 8 : 4;
         constexpr int STEP = HALF ? 2 : 1;   // k-steps (their number is even)
         constexpr bool CUT = NORM && sizeof(T) == 4; // rows in three bf16 pieces
         extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -183,18 +183,20 @@ namespace llamql
 #pragma unroll
                 for (int t = 0; t < RT; ++t)
                     cur[t][u] = next[t][u];
-            if (s0 + NW * U < steps)
-                fetch(s0 + NW * U);
-            // rows of bf16 are asked for ahead of the products (2048 x 8192 and one row: 11.0 -> 9.2 us); rows of fp32 would
-            // take the registers of a second workgroup (32768 x 2048 and one row: 43 -> 52 us)
-            constexpr bool AHEAD = sizeof(T) == 2, LATE = !AHEAD && !CUT;
+            // Rows that come from memory are asked for ahead of the next weights: loads arrive in order, so a product that
+            // waits for a row asked for behind them would wait for all of them (3 x 2048 x 10240 bf16 14.5 -> 11.0 us, fp32
+            // 19.3 -> 14.1; 8 x 5120 x 25600 bf16 75 -> 67 us, fp32 110 -> 86)
+            constexpr bool AHEAD = !NORM && (RT == 1 || sizeof(T) == 2); // (two tiles and fp32 rows: registers of a second workgroup)
             V b[AHEAD ? U : 1];
             if constexpr (AHEAD)
             {
 #pragma unroll
                 for (int u = 0; u < U; ++u)
                     b[u] = O::load(arow + (s0 + u * NW < steps ? s0 + u * NW : s0) * (32 * STEP));
+                __builtin_amdgcn_sched_barrier(0);
             }
+            if (s0 + NW * U < steps)
+                fetch(s0 + NW * U);
 #pragma unroll
             for (int u = 0; u < U; ++u)
                 if (s0 + u * NW < steps)
@@ -209,13 +211,15 @@ namespace llamql
                             for (int t = 0; t < RT; ++t)
                                 acc[t] = Operand<bf16>::mma(Operand<bf16>::from_weights(cur[t][u]), part, acc[t]);
                         }
-                        continue;
                     }
-                    if constexpr (LATE)
-                        b[0] = O::load(arow + (s0 + u * NW) * (32 * STEP));
+                    else
+                    {
+                        if constexpr (!AHEAD)
+                            b[0] = O::load(arow + (s0 + u * NW) * (32 * STEP));
 #pragma unroll
-                    for (int t = 0; t < RT; ++t)
-                        acc[t] = O::mma(O::from_weights(cur[t][u]), b[AHEAD ? u : 0], acc[t]);
+                        for (int t = 0; t < RT; ++t)
+                            acc[t] = O::mma(O::from_weights(cur[t][u]), b[AHEAD ? u : 0], acc[t]);
+                    }
                 }
         }
 #pragma unroll
