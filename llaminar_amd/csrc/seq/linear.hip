@@ -20,16 +20,25 @@ namespace llamql
         return (size_t)(sizeof(T) == 4 ? 3 : 1) * a.M * (a.K + NORM_PAD) * sizeof(bf16);
     }
 
+    template <int NW>
+    __device__ __forceinline__ float inverse_norm(const float *sums, int k_real, float eps)
+    {
+        float total = 0.0f;
+#pragma unroll
+        for (int w = 0; w < NW; ++w)
+            total += sums[w];
+        return 1.0f / sqrtf(total / (float)k_real + eps);
+    }
+
     // fp32 rows normed, into h_out as T (from the first workgroup) and into LDS: as bf16, or, for T fp32, in three bf16
-    // pieces that add up to the value (8 + 8 + 8 significant bits, cut off; infinities in the first alone), the pieces
+    // pieces that add up to the value (8 + 8 + 8 significant bits, cut off), the pieces
     // p.M * ldh apart.  Three products of bf16 take 48 cycles of the matrix unit a k-step, one of fp32 256 (3 x 32768 x
     // 2048: 45 -> 36.6 us; the error against 64 bits falls from 3.0e-7 to 2.0e-7).  R rows at a time are asked for and summed,
     // and all rows share one barrier: a row at a time, eight rows of 768 values took 6 us of a 9 us launch.
     template <typename T, int NW, int R>
-    __device__ __forceinline__ void norm_rows(const LinearArgs &p, bf16 *h, int ldh, bool record)
+    __device__ __forceinline__ void norm_rows(const LinearArgs &p, bf16 *h, int ldh, bool record, float (&s_sum)[SMALL_M][NW])
     {
         typedef T t4 __attribute__((ext_vector_type(4)));
-        __shared__ float s_sum[SMALL_M][NW];
         static_assert(SMALL_M % R == 0, "sums of whole groups");
         const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
         const auto row = [&](int m) { return reinterpret_cast<const f32x4 *>(static_cast<const float *>(p.a) + (size_t)(m < p.M ? m : p.M - 1) * p.lda); };
@@ -64,13 +73,7 @@ namespace llamql
             float inv[R];
 #pragma unroll
             for (int k = 0; k < R; ++k)
-            {
-                float total = 0.0f;
-#pragma unroll
-                for (int w = 0; w < NW; ++w)
-                    total += s_sum[m0 + k][w];
-                inv[k] = 1.0f / sqrtf(total / (float)p.k_real + p.eps);
-            }
+                inv[k] = inverse_norm<NW>(s_sum[m0 + k], p.k_real, p.eps);
             for (int i = threadIdx.x; i < p.K / 4; i += NW * 64)
             {
                 f32x4 v[R];
@@ -97,10 +100,7 @@ namespace llamql
                                 *reinterpret_cast<u32x2 *>(to) = u32x2{__builtin_amdgcn_perm(cut[1], cut[0], 0x07060302u),
                                                                        __builtin_amdgcn_perm(cut[3], cut[2], 0x07060302u)}; // upper halves
                                 cut &= 0xffff0000u;
-                                const f32x4 less = rest - __builtin_bit_cast(f32x4, cut);
-#pragma unroll
-                                for (int e = 0; e < 4; ++e)
-                                    rest[e] = fabsf(rest[e]) == INFINITY ? 0.0f : less[e];
+                                rest -= __builtin_bit_cast(f32x4, cut);
                             }
                         }
                         if (record)
@@ -157,14 +157,15 @@ namespace llamql
         using A = std::conditional_t<NORM, bf16, T>;
         const int ldh = p.K + NORM_PAD;
         const A *arow;
+        __shared__ float s_sum[NORM ? SMALL_M : 1][NW];
         if constexpr (NORM)
         {
             bf16 *h = reinterpret_cast<bf16 *>(smem);
             const bool record = p.h_out && block == 0;
             if (p.M == 1)
-                norm_rows<T, NW, 1>(p, h, ldh, record);
+                norm_rows<T, NW, 1>(p, h, ldh, record, s_sum);
             else
-                norm_rows<T, NW, 4>(p, h, ldh, record);
+                norm_rows<T, NW, 4>(p, h, ldh, record, s_sum);
             arow = h + (size_t)(row < p.M ? row : 0) * ldh + 8 * g;
         }
         else
@@ -243,6 +244,45 @@ namespace llamql
                         sum[t] = sum[t] + *reinterpret_cast<const f32x4 *>(s_red[v][t][lane + 40]);
                 }
             }
+            if constexpr (CUT)
+            {
+                // sums that the pieces do not carry (see pieces_fail), once more as products of the whole values
+                bool fail = false;
+#pragma unroll
+                for (int t = 0; t < RT; ++t)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        fail |= pieces_fail(sum[t][r]);
+                if (__builtin_expect(__ballot(fail) != 0, 0))
+                {
+                    const float inv = inverse_norm<NW>(s_sum[n], p.k_real, p.eps);
+                    const float *x = static_cast<const float *>(p.a) + (size_t)n * p.lda, *scale = p.norm;
+                    const int first = (HALF ? (block & 1) * 8 : 0) + 4 * g; // of the tile's rows
+                    f32x4 whole[RT];
+#pragma unroll
+                    for (int t = 0; t < RT; ++t)
+                        whole[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                    for (int k = 0; k < 32 * ksteps; k += 8)
+                    {
+                        const f32x8 v = Operand<float>::load(x + k) * inv * Operand<float>::load(scale + k);
+#pragma unroll
+                        for (int t = 0; t < RT; ++t)
+#pragma unroll
+                            for (int r = 0; r < 4; ++r)
+                            {
+                                const f32x8 q = Operand<float>::from_weights(w[t][(k >> 5) * 64 + ((k >> 3) & 3) * 16 + first + r - piece - second * 64]);
+#pragma unroll
+                                for (int e = 0; e < 8; ++e)
+                                    whole[t][r] = fmaf(v[e], q[e], whole[t][r]);
+                            }
+                    }
+#pragma unroll
+                    for (int t = 0; t < RT; ++t)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r)
+                            sum[t][r] = pieces_fail(sum[t][r]) ? whole[t][r] : sum[t][r];
+                }
+            }
             const size_t elem = p.out == LLAM_SEQ_OUT_F32 || p.out == LLAM_SEQ_OUT_ADD ? 4 : sizeof(T);
             char *y = static_cast<char *>(p.y) + (size_t)z * p.y_stride * elem;
             if (RT == 2 && is_gated(p.out))
@@ -272,8 +312,11 @@ namespace llamql
     __global__ void __launch_bounds__(NW * 64)
         linear_small_pair_kernel(LinearArgs p, LinearArgs second, int blocks)
     {
-        const bool other = (int)blockIdx.x >= blocks;
-        linear_small_tile<T, NW, 2, NORM>(other ? second : p, other ? (int)blockIdx.x - blocks : (int)blockIdx.x);
+        // (either way its own code: of arguments chosen at run time the compiler keeps a copy in scratch memory)
+        if ((int)blockIdx.x < blocks)
+            linear_small_tile<T, NW, 2, NORM>(p, blockIdx.x);
+        else
+            linear_small_tile<T, NW, 2, NORM>(second, (int)blockIdx.x - blocks);
     }
 
     namespace

@@ -33,23 +33,14 @@ namespace llamql
     }
 
     // A 32-bit value as three bf16 values that add up to it: 8 + 8 + 8 significant bits, cut off and not rounded, so that
-    // none is larger than the value.  Infinities stay in the first alone (what is left of them would not be a number).
+    // none is larger than the value.  Of an infinity the second piece is not a number, nor are the sums then: those are made
+    // again without pieces (see pieces_fail).
     __device__ __forceinline__ void three_pieces(f32x8 x, bf16x8 (&out)[3])
     {
         f32x8 r;
-        float most = 0.0f;
 #pragma unroll
         for (int e = 0; e < 8; ++e)
-        {
             r[e] = x[e] - __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, (float)x[e]) & 0xffff0000u);
-            most = fmaxf(most, fabsf(x[e]));
-        }
-        if (__builtin_expect(__ballot(most == INFINITY) != 0, 0))
-        {
-#pragma unroll
-            for (int e = 0; e < 8; ++e)
-                r[e] = fabsf(x[e]) == INFINITY ? 0.0f : r[e];
-        }
         u32x4 p[3];
 #pragma unroll
         for (int k = 0; k < 4; ++k)
@@ -324,6 +315,72 @@ namespace llamql
                             for (int r = 0; r < 4; ++r)
                                 acc[j][i][4 * q + r] += v[r];
                         }
+        }
+
+        if constexpr (sizeof(T) == 4)
+        {
+            // sums that the pieces do not carry (see pieces_fail), once more as products of the whole values, straight from memory
+            bool fail = false;
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r)
+                        fail |= pieces_fail(acc[j][i][r]);
+            if (__builtin_expect(__ballot(fail) != 0, 0))
+            {
+                const float *rows_of_a[TM];
+                const bf16x8 *rows_of_w[TN];
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+                {
+                    int m = mt * BM + (wm * TM + i) * 32 + c;
+                    m = row0 + (m < rows ? m : rows - 1);
+                    if (p.row_source)
+                        m = p.row_source[m] / p.source_div;
+                    rows_of_a[i] = abase + (size_t)m * p.lda + 8 * h;
+                }
+#pragma unroll
+                for (int j = 0; j < TN; ++j)
+                {
+                    int tile = nt * (BN / 16) + (wn * TN + j) * 2 + (c >> 4);
+                    tile = tile < w_tiles ? tile : w_tiles - 1;
+                    rows_of_w[j] = reinterpret_cast<const bf16x8 *>(wbase) + (size_t)tile * ksteps * 64 + h * 16 + (c & 15);
+                }
+                f32x16 whole[TN][TM];
+#pragma unroll
+                for (int j = 0; j < TN; ++j)
+#pragma unroll
+                    for (int i = 0; i < TM; ++i)
+#pragma unroll
+                        for (int r = 0; r < 16; ++r)
+                            whole[j][i][r] = 0.0f;
+                for (int s = 0; s < 2 * ksteps; ++s) // sixteen columns
+                {
+                    f32x8 x[TM], v[TN];
+#pragma unroll
+                    for (int i = 0; i < TM; ++i)
+                        x[i] = Operand<float>::load(rows_of_a[i] + s * 16);
+#pragma unroll
+                    for (int j = 0; j < TN; ++j)
+                        v[j] = __builtin_convertvector(rows_of_w[j][(s >> 1) * 64 + (s & 1) * 32], f32x8);
+#pragma unroll
+                    for (int e = 0; e < 8; ++e)
+#pragma unroll
+                        for (int j = 0; j < TN; ++j)
+#pragma unroll
+                            for (int i = 0; i < TM; ++i)
+                                whole[j][i] = __builtin_amdgcn_mfma_f32_32x32x2f32(v[j][e], x[i][e], whole[j][i], 0, 0, 0);
+                }
+#pragma unroll
+                for (int j = 0; j < TN; ++j)
+#pragma unroll
+                    for (int i = 0; i < TM; ++i)
+#pragma unroll
+                        for (int r = 0; r < 16; ++r)
+                            acc[j][i][r] = pieces_fail(acc[j][i][r]) ? whole[j][i][r] : acc[j][i][r];
+            }
         }
 
         const size_t elem = p.out == LLAM_SEQ_OUT_F32 || p.out == LLAM_SEQ_OUT_ADD ? 4 : sizeof(T);

@@ -67,3 +67,49 @@ def test_a_normed_value_beyond_32_bits(dev):
     torch.cuda.synchronize()
     assert (w[:, 5] != 0).all()
     assert torch.equal(y[0], torch.sign(w[:, 5].float()) * float("inf")) and torch.isfinite(y[1]).all()
+
+
+@pytest.mark.parametrize("pair", [False, True])
+@pytest.mark.parametrize("M,N,K", [(1, 16, 8192), (3, 2064, 2688), (8, 4112, 1024), (16, 48, 512)])
+def test_normed_values_and_weights_beyond_the_pieces(dev, M, N, K, pair):
+    """Normed rows of fp32 are cut in pieces: infinite weights, and values down to the smallest bf16, are multiplied whole."""
+    import torch
+
+    torch.manual_seed(M)
+    a, w = torch.randn(M, K, device=dev), torch.randn(N, K, device=dev).bfloat16()
+    laid, lib, stream = tiles(w), sq.load(), torch.cuda.current_stream().cuda_stream
+    infinite = w.clone()
+    infinite[3, 5], infinite[N - 1, K - 1], infinite[9, 0], infinite[9, 9] = float("inf"), float("-inf"), float("inf"), float("-inf")
+    a[0, 5], a[:, 0] = 0.0, 1.5
+    laid_infinite = tiles(infinite)
+
+    def run(weights, scale):
+        y, h = torch.zeros(2, M, N, device=dev), torch.zeros(M, K, device=dev)
+        args = [sq.LinearArgs(d_a=a.data_ptr(), d_w=weights.data_ptr(), d_y=y[i].data_ptr(), M=M, N=N, K=K, lda=K, ldy=N, out=sq.OUT_F32, batch=1,
+                              d_norm=scale.data_ptr(), k_real=K, eps=1e-5) for i in range(2)]
+        args[0].d_h_out = h.data_ptr()
+        if pair:
+            assert lib.llam_seq_linear_pair(ctypes.byref(args[0]), ctypes.byref(args[1]), F32, 0, stream), lib.llam_ql_last_error()
+        else:
+            assert lib.llam_seq_linear(ctypes.byref(args[0]), F32, 0, stream), lib.llam_ql_last_error()
+        torch.cuda.synchronize()
+        if pair:
+            assert torch.equal(y[0].view(torch.int32), y[1].view(torch.int32))
+        return y[0], h.double()
+
+    y, h = run(laid_infinite, torch.ones(K, device=dev))
+    want = (h @ infinite.double().T).float()
+    assert torch.isnan(want[0, 3])
+    for kind in (torch.isnan, torch.isposinf, torch.isneginf):
+        assert torch.equal(kind(y), kind(want))
+    plain = [n for n in range(N) if n not in (3, 9, N - 1)]
+    bound = (K + 1) * 2.0 ** -23 * (h.abs() @ w.double().abs().T)
+    assert ((y[:, plain].double() - h @ w[plain].double().T).abs() <= bound[:, plain]).all()
+    for size in (1e-30, 1e-36, 1.2e-39):
+        for kept in (1, K):   # single values and whole rows
+            scale = torch.zeros(K, device=dev)
+            scale[:kept] = size
+            y, h = run(laid, scale)
+            # and each product and sum may be rounded to a multiple of the smallest value, 2^-149
+            bound = (K + 1) * 2.0 ** -23 * (h.abs() @ w.double().abs().T) + K * 2.0 ** -149
+            assert (h != 0).any() and ((y.double() - h @ w.double().T).abs() <= bound).all()

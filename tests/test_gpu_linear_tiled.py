@@ -124,3 +124,46 @@ def test_values_at_the_ends_of_the_range(dev, M):
     plain = [m for m in range(M) if m not in (3, 9, 11, M - 1)]
     close(torch, y[plain], a[plain], w, K)
     assert (y[13] == 0.0).all()
+
+
+# the smallest shapes of each tile of 32-bit rows
+WHOLE = [(20, 64, 256), (300, 6160, 512), (257, 4112, 64), (1000, 6160, 192)]
+
+
+@pytest.mark.parametrize("M,N,K", WHOLE)
+def test_infinite_weights_of_32_bit_rows(dev, M, N, K):
+    """Most pieces of a value are zero, and zero times infinity is not a number: such sums are those of the whole values."""
+    import torch
+
+    torch.manual_seed(M)
+    a, w = torch.randn(M, K, device=dev).bfloat16().float(), torch.randn(N, K, device=dev).bfloat16()
+    w[3, 5], w[N - 1, K - 1], w[N // 2, 0], w[N // 2, 9] = float("inf"), float("-inf"), float("inf"), float("-inf")
+    a[2, 5], a[M - 1, 7] = 0.0, float("inf")
+    y = torch.zeros(M, N, device=dev)
+    run(torch, a, tiles(w), y, F32, N=N, K=K)
+    want = (a.double() @ w.double().T).float()
+    assert torch.isposinf(want[:, 3]).any() and torch.isnan(want[2, 3])
+    for kind in (torch.isnan, torch.isposinf, torch.isneginf):
+        assert torch.equal(kind(y), kind(want))
+    plain = [n for n in range(N) if n not in (3, N // 2, N - 1)]
+    close(torch, y[:M - 1][:, plain], a[:M - 1], w[plain], K)
+
+
+@pytest.mark.parametrize("M,N,K", WHOLE)
+def test_small_values_of_32_bit_rows(dev, M, N, K):
+    """Rows down to values of the size of the smallest bf16, whole ones and single values: no bits lost below it."""
+    import torch
+
+    torch.manual_seed(M)
+    a, w = torch.randn(M, K, device=dev), torch.randn(N, K, device=dev).bfloat16()
+    a[::6], a[3::6] = 0.0, 0.0
+    a[::6, 0], a[3::6, K - 1] = 1.2345678, -1.9876543
+    a = (a.double() * 10.0 ** -(20 + torch.arange(M, device=dev) % 20).double().unsqueeze(1)).float()
+    y = torch.zeros(M, N, device=dev)
+    run(torch, a, tiles(w), y, F32, N=N, K=K)
+    want = a.double() @ w.double().T
+    # as in close(), and each product and sum may be rounded to a multiple of the smallest value, 2^-149
+    bound = (K + 1) * 2.0 ** -23 * (a.double().abs() @ w.double().abs().T) + K * 2.0 ** -149
+    # (a sum that the pieces make zero is taken at its word: of each value less than 2^-133 may be missing)
+    bound[y == 0.0] = K * 2.0 ** -133 * float(w.abs().max())
+    assert ((y.double() - want).abs() <= bound).all() and (y != 0.0).double().mean() > 0.99
