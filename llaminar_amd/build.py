@@ -113,6 +113,51 @@ def _vregs(text: str) -> set[int]:
     return regs
 
 
+def _device_functions(asm: str):
+    """(name, blocks) of every function in the device assembly; a block is a label (None: the function's first) and its
+    operations, in order, as the in-flight check needs them."""
+    name, blocks, in_asm = "?", [(None, [])], False
+    for raw_line in asm.splitlines():
+        text = raw_line.strip()
+        if text.startswith(";;#ASMSTART") or text.startswith(";;#ASMEND"):
+            in_asm = text.startswith(";;#ASMSTART")
+            continue
+        text = text.split(";")[0].strip()
+        m = re.match(r"^([A-Za-z_.][\w$.]*):", text)
+        if m and not m.group(1).startswith(".L"):
+            yield name, blocks
+            name, blocks = m.group(1), [(None, [])]
+            continue
+        if m and m.group(1).startswith(".LBB"):
+            blocks.append((m.group(1), []))
+            continue
+        if not text or text.startswith(".") or text.endswith(":"):
+            continue
+        ops = blocks[-1][1]
+        if text.startswith("s_waitcnt"):
+            w = _VMCNT.search(text)
+            if w:
+                ops.append(("wait", int(w.group(1)), text))
+        elif m := re.match(r"^s_c?branch\w*\s+(\S+)", text):
+            ops.append(("jump" if text.startswith("s_branch") else "branch", m.group(1), text))
+        elif re.match(r"^(s_endpgm|s_setpc_b64)\b", text):
+            ops.append(("end", None, text))
+        else:
+            load = _ASM_LOAD.match(text) if in_asm else None
+            touched = frozenset(_vregs(text))
+            if load:
+                ops.append(("load", (frozenset(_vregs(load.group(2))), touched), text))
+            elif _VMEM.match(text):
+                ops.append(("memory", touched, text))
+            elif touched:
+                ops.append(("use", touched, text))
+    yield name, blocks
+
+
+# states of the queue a block may be entered with before the check gives up (the kernels here need up to about a hundred)
+MAX_QUEUES = 4000
+
+
 def check_inflight_registers(asm: str, src_name: str) -> int:
     """Scan the device assembly for the second way the hand-scheduled loads can break.
 
@@ -121,65 +166,66 @@ def check_inflight_registers(asm: str, src_name: str) -> int:
     registers hold their values from the point of issue, so besides spilling them it may
     COPY them (a phi move at a loop entry, a move into another allocation) or reuse them
     while the data is still on its way: the copy reads stale contents, or the load lands in
-    whatever lives in the register by then.  This pass walks every function in program
-    order, keeps the queue of vector memory operations that vmcnt counts (hand-issued loads
-    with their destination registers, everything else as a placeholder), retires entries at
-    each s_waitcnt vmcnt(N), and reports any instruction that names a register of a
-    hand-issued load still in the queue.  Straight-line bookkeeping: the queue is emptied
-    where control cannot fall through (s_branch, s_endpgm, s_setpc), so the pass can miss a
-    hazard across a jump but does not invent one.  Returns the number of hand-issued loads
-    it followed.
+    whatever lives in the register by then.  This pass keeps the queue of vector memory
+    operations that vmcnt counts (hand-issued loads with their destination registers, everything
+    else as a placeholder), retires entries at each s_waitcnt vmcnt(N), and reports any
+    instruction that names a register of a hand-issued load still in the queue.  It follows every
+    jump both ways, a block once for each queue it can be entered with; a path that no run
+    takes (the same condition tested twice with different outcomes) counts as well.  Returns the number of
+    hand-issued loads it found.
     """
-    findings: list[str] = []
+    findings: dict[str, None] = {}
     followed = 0
-    func = "?"
-    queue: list[set[int] | None] = []  # oldest first; None: an operation whose registers the compiler tracks
-    in_asm = False
-    for raw_line in asm.splitlines():
-        line = raw_line.split(";")[0].rstrip() if not raw_line.lstrip().startswith(";;#") else raw_line.strip()
-        if line.startswith(";;#ASMSTART"):
-            in_asm = True
+    for func, blocks in _device_functions(asm):
+        loads = sum(op[0] == "load" for _, ops in blocks for op in ops)
+        followed += loads
+        if not loads:
             continue
-        if line.startswith(";;#ASMEND"):
-            in_asm = False
-            continue
-        m = re.match(r"^([A-Za-z_][\w$.]*):", line)
-        if m and not line.startswith(".L"):
-            func, queue = m.group(1), []
-            continue
-        text = line.strip()
-        if not text or text.startswith(".") or text.endswith(":"):
-            continue
-        if text.startswith("s_waitcnt"):
-            w = _VMCNT.search(text)
-            if w:
-                keep = int(w.group(1))
-                queue = queue[len(queue) - keep:] if keep and keep < len(queue) else ([] if keep == 0 else queue)
-            continue
-        if re.match(r"^(s_branch|s_endpgm|s_setpc_b64)\b", text):
-            queue = []
-            continue
-        touched = _vregs(text)
-        load = _ASM_LOAD.match(text) if in_asm else None
-        pending = set().union(*[q for q in queue if q]) if queue else set()
-        if load:
-            dst = _vregs(load.group(2))
-            hit = (touched - dst) & pending or (dst & pending)
-            if hit:
-                findings.append(f"{func}: '{text}' uses v{sorted(hit)[0]} while a hand-issued load into it is in flight")
-            queue.append(dst)
-            followed += 1
-            continue
-        hit = touched & pending
-        if hit:
-            findings.append(f"{func}: '{text}' touches v{sorted(hit)[0]} before the wait for the hand-issued load into it")
-        if _VMEM.match(text):
-            queue.append(None)
+        at = {label: i for i, (label, _) in enumerate(blocks)}
+        seen: list[set] = [set() for _ in blocks]
+        work: list[tuple[int, tuple]] = []
+
+        def enter(i, queue):
+            while queue and queue[0] is None:   # finished with the wait for anything newer, and no registers
+                queue = queue[1:]
+            if i is not None and i < len(blocks) and queue not in seen[i]:
+                seen[i].add(queue)
+                if len(seen[i]) > MAX_QUEUES:
+                    raise InFlightRegisterError(f"{src_name}: {func}: too many ways to reach {blocks[i][0]}")
+                work.append((i, queue))
+
+        enter(0, ())
+        while work:
+            i, queue = work.pop()   # oldest first; None: an operation whose registers the compiler tracks
+            pending = frozenset().union(*(q for q in queue if q))
+            for kind, what, text in blocks[i][1]:
+                if kind == "wait":
+                    queue = queue[len(queue) - what:] if 0 < what < len(queue) else (() if what == 0 else queue)
+                    pending = frozenset().union(*(q for q in queue if q))
+                elif kind in ("jump", "branch"):
+                    enter(at.get(what), queue)
+                    if kind == "jump":
+                        break
+                elif kind == "end":
+                    break
+                elif kind == "load":
+                    dst, touched = what
+                    if hit := touched & pending:
+                        findings[f"{func}: '{text}' uses v{min(hit)} while a hand-issued load into it is in flight"] = None
+                    queue, pending = (*queue, dst)[-64:], pending | dst   # (vmcnt counts to 63)
+                else:
+                    if hit := what & pending:
+                        findings[f"{func}: '{text}' touches v{min(hit)} before the wait for the hand-issued load into it"] = None
+                    if kind == "memory" and queue:
+                        queue = (*queue, None)[-64:]
+            else:
+                enter(i + 1, queue)
     if findings:
-        shown = "\n  ".join(findings[:12]) + ("" if len(findings) <= 12 else f"\n  ... and {len(findings) - 12} more")
+        shown = list(findings)[:12]
         raise InFlightRegisterError(
             f"{src_name}: registers of hand-issued loads are touched before their s_waitcnt "
-            f"(the data has not arrived; see check_inflight_registers):\n  {shown}")
+            "(the data has not arrived; see check_inflight_registers):\n  " + "\n  ".join(shown)
+            + ("" if len(findings) <= 12 else f"\n  ... and {len(findings) - 12} more"))
     return followed
 
 

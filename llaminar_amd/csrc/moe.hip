@@ -574,6 +574,9 @@ namespace llamql
                 }
             }
         }
+        // (nothing is on its way any more: the last step has waited for all.  Said once more for a reader who follows both
+        // tests of `mine` both ways, as the build's check of registers in flight does)
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
         // one lane per row: the live slots in ascending order
         for (int r = threadIdx.x; r < rows_wg; r += blockDim.x)

@@ -185,6 +185,47 @@ def test_inflight_check_counts_other_memory_operations_and_resets_at_jumps():
     assert check_inflight_registers(asm, "demo.hip") == 2
 
 
+LOOP = """\
+\t;;#ASMSTART
+\tglobal_load_dwordx4 v[8:11], v[2:3], off
+\t;;#ASMEND
+.LBB0_1:
+\t;;#ASMSTART
+\ts_waitcnt vmcnt(0)
+\t;;#ASMEND
+\tv_and_b32_e32 v4, 0xf0f0f0f, v{read}
+\t;;#ASMSTART
+\tglobal_load_dwordx4 v[{dst}], v[2:3], off
+\t;;#ASMEND
+\t{between}
+\ts_cbranch_scc1 .LBB0_1
+\ts_waitcnt vmcnt(0)
+"""
+
+
+def test_inflight_check_follows_a_loop_edge():
+    from llaminar_amd.build import InFlightRegisterError, check_inflight_registers
+
+    assert check_inflight_registers(_asm(LOOP.format(read=8, dst="8:11", between="s_nop 0")), "demo.hip") == 2
+    # the next turn's load lands in other registers, and a copy that brings them to where the loop begins is taken on the
+    # edge, ahead of the wait behind the label: in program order the copy comes before the load
+    edge = LOOP.format(read=8, dst="12:15", between="s_branch .LBB0_3").replace(
+        ".LBB0_1:", "\ts_branch .LBB0_1\n.LBB0_2:\n\tv_mov_b64_e32 v[8:9], v[12:13]\n.LBB0_1:") + \
+        ".LBB0_3:\n\ts_cbranch_scc1 .LBB0_2\n\ts_waitcnt vmcnt(0)\n"
+    with pytest.raises(InFlightRegisterError, match="v12"):
+        check_inflight_registers(_asm(edge), "demo.hip")
+    with pytest.raises(InFlightRegisterError, match="v8"):   # behind a conditional jump over the wait
+        check_inflight_registers(_asm("""\
+\t;;#ASMSTART
+\tglobal_load_dwordx4 v[8:11], v[2:3], off
+\t;;#ASMEND
+\ts_cbranch_vccz .LBB0_2
+\ts_waitcnt vmcnt(0)
+.LBB0_2:
+\tv_mov_b32_e32 v4, v8
+"""), "demo.hip")
+
+
 # ---- scalar registers that a vector instruction has just written ---------------------------------
 
 SCALAR = """\
