@@ -117,13 +117,14 @@ namespace llamql
     // HALF: up to 8 rows of A, and a workgroup for 8 rows of W, half a tile: a step is two k-steps, W's rows of the second
     // beside those of the first as the matrix unit's other 8 rows, A's likewise as its other 8 columns, and of the product
     // the two blocks that match are kept.  Twice the workgroups, for layers of fewer tiles than the chip has compute units.
-    template <typename T, int NW, int RT, bool NORM, bool HALF = false>
+    // LONG: fp32 rows in rounds of four steps with the rows asked for ahead, and not of eight without (see AHEAD).
+    template <typename T, int NW, int RT, bool NORM, bool HALF = false, bool LONG = true>
     __device__ __forceinline__ void linear_small_tile(const LinearArgs &p, int block)
     {
         using O = Operand<T>;
         using V = typename O::V;
         static_assert(!HALF || RT == 1, "half a tile");
-        constexpr int U = RT == 1 && (NORM || sizeof(T) == 2) ? 8 : 4;
+        constexpr int U = RT == 1 && (NORM || sizeof(T) == 2 || !LONG) ? 8 : 4;
         constexpr int STEP = HALF ? 2 : 1;   // k-steps (their number is even)
         constexpr bool CUT = NORM && sizeof(T) == 4; // rows in three bf16 pieces
         extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -164,6 +165,8 @@ namespace llamql
             const bool record = p.h_out && block == 0;
             if (p.M == 1)
                 norm_rows<T, NW, 1>(p, h, ldh, record, s_sum);
+            else if (p.M == 2) // (not four, two of them in vain: 2 x 5120 x 2048 in bf16 6.4 -> 5.3 us)
+                norm_rows<T, NW, 2>(p, h, ldh, record, s_sum);
             else
                 norm_rows<T, NW, 4>(p, h, ldh, record, s_sum);
             arow = h + (size_t)(row < p.M ? row : 0) * ldh + 8 * g;
@@ -186,15 +189,27 @@ namespace llamql
                     cur[t][u] = next[t][u];
             // Rows that come from memory are asked for ahead of the next weights: loads arrive in order, so a product that
             // waits for a row asked for behind them would wait for all of them (3 x 2048 x 10240 bf16 14.5 -> 11.0 us, fp32
-            // 19.3 -> 14.1; 8 x 5120 x 25600 bf16 75 -> 67 us, fp32 110 -> 86)
-            constexpr bool AHEAD = !NORM && (RT == 1 || sizeof(T) == 2); // (two tiles and fp32 rows: registers of a second workgroup)
-            V b[AHEAD ? U : 1];
-            if constexpr (AHEAD)
+            // 19.3 -> 14.1; 8 x 5120 x 25600 bf16 75 -> 67 us, fp32 110 -> 86).  Not in a last round with fewer than U steps:
+            // there are no next weights, and rows asked for in vain took as long as the others (16 x 5120 x 1024 in
+            // bf16 6.3 -> 4.6).
+            // (Two tiles or eight steps of fp32 rows: registers of a second workgroup.  Walks of one round of eight steps gain
+            // nothing from rows ahead of later weights, and lose with half the weights asked for at first: 16 x 5120 x 2048 11.0 -> 10.6.)
+            constexpr bool AHEAD = !NORM && (sizeof(T) == 2 || (RT == 1 && LONG));
+            if (AHEAD && __builtin_amdgcn_readfirstlane(s0 + (U - 1) * NW < steps))
             {
+                V b[AHEAD ? U : 1];
 #pragma unroll
-                for (int u = 0; u < U; ++u)
-                    b[u] = O::load(arow + (s0 + u * NW < steps ? s0 + u * NW : s0) * (32 * STEP));
+                for (int u = 0; u < (AHEAD ? U : 1); ++u)
+                    b[u] = O::load(reinterpret_cast<const T *>(arow) + (s0 + u * NW) * (32 * STEP));
                 __builtin_amdgcn_sched_barrier(0);
+                if (s0 + NW * U < steps)
+                    fetch(s0 + NW * U);
+#pragma unroll
+                for (int u = 0; u < (AHEAD ? U : 1); ++u)
+#pragma unroll
+                    for (int t = 0; t < RT; ++t)
+                        acc[t] = O::mma(O::from_weights(cur[t][u]), b[u], acc[t]);
+                continue;
             }
             if (s0 + NW * U < steps)
                 fetch(s0 + NW * U);
@@ -215,11 +230,10 @@ namespace llamql
                     }
                     else
                     {
-                        if constexpr (!AHEAD)
-                            b[0] = O::load(arow + (s0 + u * NW) * (32 * STEP));
+                        const V b = O::load(arow + (s0 + u * NW) * (32 * STEP));
 #pragma unroll
                         for (int t = 0; t < RT; ++t)
-                            acc[t] = O::mma(O::from_weights(cur[t][u]), b[AHEAD ? u : 0], acc[t]);
+                            acc[t] = O::mma(O::from_weights(cur[t][u]), b, acc[t]);
                     }
                 }
         }
@@ -300,11 +314,11 @@ namespace llamql
         }
     }
 
-    template <typename T, int NW, int RT, bool NORM, bool HALF>
+    template <typename T, int NW, int RT, bool NORM, bool HALF, bool LONG>
     __global__ void __launch_bounds__(NW * 64)
         linear_small_kernel(LinearArgs p)
     {
-        linear_small_tile<T, NW, RT, NORM, HALF>(p, blockIdx.x);
+        linear_small_tile<T, NW, RT, NORM, HALF, LONG>(p, blockIdx.x);
     }
 
     // Two layers over the same rows: the first `blocks` workgroups belong to p.
@@ -321,12 +335,12 @@ namespace llamql
 
     namespace
     {
-        template <typename T, int NW, int RT, bool NORM, bool HALF = false>
+        template <typename T, int NW, int RT, bool NORM, bool HALF = false, bool LONG = true>
         bool small_launch(const char *fn, const LinearArgs &a, int batch, hipStream_t st)
         {
             static LdsGrant grant;
             const size_t lds = NORM ? norm_lds<T>(a) : 0;
-            const auto kernel = &linear_small_kernel<T, NW, RT, NORM, HALF>;
+            const auto kernel = &linear_small_kernel<T, NW, RT, NORM, HALF, LONG>;
             if (lds > 32 * 1024 && allow_lds(grant, reinterpret_cast<const void *>(kernel), 64 * 1024) != hipSuccess)
                 return fail(fn, "cannot reserve %zu bytes of LDS", lds);
             hipLaunchKernelGGL(kernel, dim3(a.N / (HALF ? 8 : 16 * RT), batch), dim3(NW * 64), lds, st, a);
@@ -344,7 +358,11 @@ namespace llamql
             constexpr int CUS = 256;
             const long tiles = (long)a.N / 16 * batch;
             const bool half = a.M <= 8 && tiles < CUS && (a.K >= 4096 || (sizeof(T) == 4 && tiles <= CUS / 2));
-            return half ? small_launch<T, NW, 1, NORM, true>(fn, a, batch, st) : small_launch<T, NW, 1, NORM>(fn, a, batch, st);
+            if (half)
+                return small_launch<T, NW, 1, NORM, true>(fn, a, batch, st);
+            if (sizeof(T) == 4 && !NORM && a.K <= 8 * NW * 32) // one round of eight steps
+                return small_launch<T, NW, 1, NORM, false, false>(fn, a, batch, st);
+            return small_launch<T, NW, 1, NORM>(fn, a, batch, st);
         }
         template <typename T>
         bool small_dispatch(const char *fn, const LinearArgs &a, int batch, hipStream_t st)
