@@ -349,15 +349,19 @@ namespace llamql
         template <typename T, int NW, bool NORM>
         bool small_tiles(const char *fn, const LinearArgs &a, int batch, hipStream_t st)
         {
-            // Half tiles where whole ones leave compute units without a workgroup and a workgroup has much to do
-            // (M x N x K, us, whole and half tiles, A ahead of neither):
-            //   8 x 2048 x 8192   bf16 16.4, 11.7  fp32 24.3, 16.2     3 x 2048 x 10240  bf16 19.9, 14.5  fp32 29.6, 19.2
-            //   8 x 2048 x 2048   bf16  4.6,  4.7  fp32  6.8,  5.8     8 x 768 x 2048    bf16  4.1,  4.0  fp32  6.1,  5.1
-            //   8 x 3072 x 2048   bf16  5.7,  6.8  fp32  8.0,  8.9     8 x 6160 x 2048   bf16  8.6, 11.2  fp32 12.2, 15.4
-            // (fp32: the products take as long as the weights, so a workgroup's share counts from fewer k-steps on)
+            // Half tiles where they too find a compute unit each and whole ones need more than a round of eight steps for K (fp32
+            // rows from memory: always, their products take as long as the weights).  Not between a quarter and half of the
+            // units with rows of W 8 or 16 KB apart: eight rows of each of so many workgroups meet in the same channels.
+            // M x N x K, us, whole and half tiles:
+            //   8 x 1024 x 3072  bf16  4.6,  3.9  fp32  7.0,  5.7      1 x 2048 x 5120   bf16  4.9,  4.0  normed  5.4,  5.1
+            //   8 x 2048 x 10240 bf16 11.8, 11.1  fp32 19.0, 14.4      8 x 2304 x 10240  bf16 12.2, 16.5  fp32   19.1, 24.4
+            //   8 x 2048 x 2048  bf16  3.4,  3.6  fp32  5.8,  4.5      8 x 512 x 512     bf16  2.6,  2.6  fp32    3.5,  2.8
+            //   1 x 1536 x 8192  bf16  5.5,  5.8  normed 6.5, 8.5      1 x 512 x 8192    bf16  5.4,  3.8  normed  6.2,  5.3
+            //   1 x 1792 x 4096  bf16  3.6,  4.2  normed 4.7, 5.9      8 x 2048 x 16384  bf16 16.8, 14.9  fp32   27.4, 20.1
             constexpr int CUS = 256;
             const long tiles = (long)a.N / 16 * batch;
-            const bool half = a.M <= 8 && tiles < CUS && (a.K >= 4096 || (sizeof(T) == 4 && tiles <= CUS / 2));
+            const bool channels = tiles > CUS / 4 && (a.K == 4096 || a.K == 8192);
+            const bool half = a.M <= 8 && tiles <= CUS / 2 && ((sizeof(T) == 4 && !NORM) || (a.K > 2048 && !channels));
             if (half)
                 return small_launch<T, NW, 1, NORM, true>(fn, a, batch, st);
             if (sizeof(T) == 4 && !NORM && a.K <= 8 * NW * 32) // one round of eight steps

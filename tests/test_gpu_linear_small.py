@@ -10,16 +10,16 @@ pytestmark = pytest.mark.gpu
 
 F32, BF16 = sq.F32, sq.BF16
 
-# half tiles: one to eight rows, one tile, the most tiles (128 and 255), K of one step, of fewer steps than wavefronts, of
-# an odd number of steps a wavefront; whole tiles on the other side: nine rows, 129 and 256 tiles, K below 4096; walks of half a
-# round of steps, of one round and of one and a part
+# half tiles: one to eight rows, one tile, the most tiles (128), K of one step, of fewer steps than wavefronts, of an odd
+# number of steps a wavefront; whole tiles on the other side: nine rows, 65 tiles and K of 4096, 129 and 256 tiles, K of
+# 2048 (bf16); walks of half a round of steps, of one round and of one and a part
 SHAPES = [(1, 16, 64), (8, 16, 4096), (8, 2048, 128), (7, 2064, 1088), (3, 2048, 10304), (8, 4080, 4160), (9, 2048, 4096),
-          (8, 4096, 4096), (5, 4096, 4032), (16, 48, 8256), (12, 4112, 1024), (16, 80, 2048),
+          (8, 4096, 4096), (5, 4096, 4032), (6, 1040, 4096), (8, 2048, 5120), (4, 1024, 2112), (8, 48, 2048), (16, 48, 8256), (12, 4112, 1024), (16, 80, 2048),
           (9, 48, 2112)]
 
 
 # a fused norm takes up to 8192 values: all of them in one row and in sixteen, half and whole tiles
-NORMED = [(1, 16, 64), (7, 2064, 1088), (1, 32, 8192), (2, 80, 4096), (3, 32, 2688), (4, 2048, 2048), (5, 4112, 1600), (16, 32, 512)]
+NORMED = [(1, 16, 64), (1, 2048, 5120), (2, 1040, 4096), (3, 80, 2112), (7, 2064, 1088), (1, 32, 8192), (2, 80, 4096), (3, 32, 2688), (4, 2048, 2048), (5, 4112, 1600), (16, 32, 512)]
 
 
 @pytest.mark.parametrize("dtype", [BF16, F32])
