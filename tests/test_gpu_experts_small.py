@@ -1,4 +1,5 @@
-"""Routed experts of 2 to 16 rows: the rows that share an expert are multiplied together, and each is what it is alone."""
+"""Routed experts.  Of 2 to 16 rows: the rows that share an expert are multiplied together, and each is what it is alone.
+Of more: rows grouped by expert, against sums in 64 bits."""
 import ctypes
 
 import pytest
@@ -40,3 +41,46 @@ def test_rows_together_are_rows_alone(dev, M, experts, top, ff, shared, dtype):
     alone = torch.cat([run([m]) for m in range(M)])
     assert torch.isfinite(together).all() and not torch.equal(together, base)
     assert torch.equal(together, alone)
+
+
+# rows, experts, of a row, width of an expert, of the model, slope of the logits: few rows; more than 64 experts, evenly and
+# mostly the first ones chosen, many without a row; groups of several tiles with a last one of few rows, of all rows
+@pytest.mark.parametrize("dtype", [sq.BF16, sq.F32])
+@pytest.mark.parametrize("M,experts,top,ff,K,slope", [(17, 8, 2, 64, 320, 0.0), (40, 130, 3, 192, 256, 0.0), (300, 150, 4, 192, 128, 0.2),
+                                                      (300, 64, 6, 320, 192, 0.0), (700, 3, 2, 320, 128, 0.5), (260, 5, 1, 64, 64, 9.0),
+                                                      (500, 40, 3, 2048, 64, 0.1), (400, 20, 3, 64, 1088, 0.0)])
+def test_rows_grouped_by_expert(dev, M, experts, top, ff, K, slope, dtype):
+    import torch
+
+    T = torch.float32 if dtype == sq.F32 else torch.bfloat16
+    torch.manual_seed(M + experts)
+    up, down = torch.randn(experts, ff, K, device=dev) * K ** -0.5, torch.randn(experts, K, ff, device=dev) * ff ** -0.5
+    up, down = up.bfloat16(), down.bfloat16()
+    lay = lambda w: w.reshape(experts, w.shape[1] // 16, 16, w.shape[2] // 32, 4, 8).permute(0, 1, 3, 4, 2, 5).contiguous()
+    up_laid, down_laid = lay(up), lay(down)
+    logits = torch.randn(M, experts + 16, device=dev)
+    logits[:, :experts] -= slope * torch.arange(experts, device=dev)
+    h, base = torch.randn(M, K, device=dev).to(T), torch.randn(M, K, device=dev)
+    x, lib = base.clone(), sq.load()
+    size = lib.llam_seq_experts_scratch_bytes(M, experts, top, ff, 0, K)
+    scratch = torch.full((size,), 255, dtype=torch.uint8, device=dev)
+    a = sq.ExpertsArgs(d_logits=logits.data_ptr(), ldz=experts + 16, d_up=up_laid.data_ptr(), d_down=down_laid.data_ptr(), up_stride=ff * K,
+                       down_stride=ff * K, experts=experts, top=top, ff=ff, K=K, N=K, d_h=h.data_ptr(), d_x=x.data_ptr(), ldx=K)
+    assert lib.llam_seq_experts(ctypes.byref(a), M, scratch.data_ptr(), size, dtype, 0, torch.cuda.current_stream().cuda_stream), lib.llam_ql_last_error()
+    torch.cuda.synchronize()
+    chosen, ids = logits[:, :experts].double().topk(top, 1)
+    weights = torch.softmax(chosen, 1)
+    want, bound, unit = base.double(), 2.0 ** -21 * base.double().abs(), 2.0 ** -23
+    for e in range(experts):
+        rows, at = (ids == e).nonzero(as_tuple=True)
+        if not len(rows):
+            continue
+        u, d, r = up[e].double(), down[e].double(), h[rows].double()
+        s = r @ u.T
+        off = (K + 1) * unit * (r.abs() @ u.abs().T)            # sums of K products in 32 bits, in any order
+        act = torch.relu(s) ** 2
+        off = 2 * s.abs() * off + off ** 2 + (2.0 ** -8 if dtype == sq.BF16 else unit) * act   # squared, rounded to T
+        w = weights[rows, at].unsqueeze(1)
+        want.index_add_(0, rows, w * (act @ d.T))
+        bound.index_add_(0, rows, 1.01 * w * ((off + (ff + 16) * unit * act) @ d.abs().T))   # (16: the weight and the sum of choices)
+    assert ((x.double() - want).abs() <= bound).all()
