@@ -99,21 +99,36 @@ namespace llamql
         const int c = lane & 31, h = lane >> 5;
         const int wm = wave % WM, wn = wave / WM;
 
-        // neighbouring tiles go to one die (blocks are dealt round robin over the eight dies), eight tiles of rows side
-        // by side, then the next tile of W: what a die works on at a time is about square
-        auto group_tiles = [&](int g) __attribute__((always_inline)) { return g < p.groups ? (p.group_offset[g + 1] - p.group_offset[g] + BM - 1) / BM : 0; };
+        // groups g0 .. g0 + 63, one a lane: its first row, rows and tiles; returns the tiles up to the lane's
+        int lo = 0, n = 0, tiles = 0;
+        auto look = [&](int g0) __attribute__((always_inline)) {
+            const int e = g0 + lane < p.groups ? g0 + lane : p.groups - 1;
+            lo = p.group_offset[e], n = g0 + lane < p.groups ? p.group_offset[e + 1] - lo : 0;
+            tiles = (n + BM - 1) / BM;
+            int upto = tiles;
+#pragma unroll
+            for (int off = 1; off < 64; off <<= 1)
+            {
+                const int o = __shfl_up(upto, off, 64);
+                upto += lane >= off ? o : 0;
+            }
+            return upto;
+        };
+        int upto = 0;
         if (p.group_offset)
         {
             // the tiles of rows that there are: dealt out by the most there can be, the first dies would get them all (300 rows,
             // 8 of 128 experts of 768 x 2048 each, mostly of the first 40: 182 -> 123 us, of all of them: 210 -> 193)
             int live = 0;
-            for (int g = lane; g < p.groups; g += 64)
-                live += group_tiles(g);
-#pragma unroll
-            for (int off = 32; off > 0; off >>= 1)
-                live += __shfl_xor(live, off, 64);
+            for (int g0 = (p.groups - 1) / 64 * 64; g0 >= 0; g0 -= 64)
+            {
+                upto = look(g0);
+                live += __shfl(upto, 63, 64);
+            }
             m_tiles = __builtin_amdgcn_readfirstlane(live);
         }
+        // neighbouring tiles go to one die (blocks are dealt round robin over the eight dies), eight tiles of rows side
+        // by side, then the next tile of W: what a die works on at a time is about square
         const int total = m_tiles * n_tiles;
         int id = blockIdx.x;
         if (id >= total)
@@ -132,29 +147,26 @@ namespace llamql
             const int want = mt;
             int seen = 0;
             z = -1;
-            for (int g0 = 0; g0 < p.groups && z < 0; g0 += 64)
+            for (int g0 = 0; g0 < p.groups; g0 += 64)
             {
-                const int tiles = group_tiles(g0 + lane);
-                int upto = tiles;
-#pragma unroll
-                for (int off = 1; off < 64; off <<= 1)
-                {
-                    const int o = __shfl_up(upto, off, 64);
-                    upto += lane >= off ? o : 0;
-                }
+                if (g0 > 0) // (the first ones were looked at last)
+                    upto = look(g0);
                 const unsigned long long past = __ballot(seen + upto > want);
                 if (past)
                 {
                     const int who = __builtin_ctzll(past);
                     z = g0 + who;
+                    row0 = __shfl(lo, who, 64);
+                    rows = __shfl(n, who, 64);
                     mt = want - (seen + __shfl(upto - tiles, who, 64));
+                    break;
                 }
                 seen += __shfl(upto, 63, 64);
             }
             if (z < 0)
                 return;
-            z = __builtin_amdgcn_readfirstlane(z), mt = __builtin_amdgcn_readfirstlane(mt);
-            row0 = p.group_offset[z], rows = p.group_offset[z + 1] - row0;
+            z = __builtin_amdgcn_readfirstlane(z), row0 = __builtin_amdgcn_readfirstlane(row0);
+            rows = __builtin_amdgcn_readfirstlane(rows), mt = __builtin_amdgcn_readfirstlane(mt);
         }
         const T *abase = static_cast<const T *>(p.a) + (size_t)z * p.a_stride;
         const char *wbase = reinterpret_cast<const char *>(static_cast<const bf16 *>(p.w) + (size_t)z * p.w_stride);
