@@ -356,11 +356,15 @@ def _compile(src: Path, force: bool = True) -> Path:
     noise = "is not a recognized feature for this target"
     lines = [l for l in proc.stderr.splitlines() if noise not in l]
     if proc.returncode == 0:
-        check_kernel_resources(proc.stderr, src.name)
-        for asm_file in OBJDIR.glob(f"{src.stem}-hip-amdgcn-*.s"):
-            asm = asm_file.read_text()
-            check_inflight_registers(asm, src.name)
-            check_scalar_hazards(asm, src.name)
+        try:
+            check_kernel_resources(proc.stderr, src.name)
+            for asm_file in OBJDIR.glob(f"{src.stem}-hip-amdgcn-*.s"):
+                asm = asm_file.read_text()
+                check_inflight_registers(asm, src.name)
+                check_scalar_hazards(asm, src.name)
+        except Exception:
+            obj.unlink(missing_ok=True)   # (a later build without force would keep it)
+            raise
     err = "\n".join(_drop_resource_remarks(lines))
     if proc.returncode != 0:
         raise RuntimeError(f"hipcc failed on {src.name}:\n{err}")

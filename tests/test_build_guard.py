@@ -76,6 +76,26 @@ def test_compile_command_asks_for_the_remarks():
     assert b.RESOURCE_FLAG == "-Rpass-analysis=kernel-resource-usage"
 
 
+def test_a_refused_object_is_not_kept(tmp_path, monkeypatch):
+    """A build without force keeps objects newer than their sources: one that the checks refused must not be there."""
+    source, stderr = tmp_path / "demo.hip", REMARKS.format(u=4, scratch=4, spill=0)
+    source.write_text("")
+
+    def compiler(cmd, **_):
+        (tmp_path / "demo.o").write_text("object")
+        return b.subprocess.CompletedProcess(cmd, 0, "", stderr)
+
+    monkeypatch.setattr(b, "OBJDIR", tmp_path)
+    monkeypatch.setattr(b, "_headers_mtime", lambda: 0.0)
+    monkeypatch.setattr(b, "hipcc", lambda: "hipcc")
+    monkeypatch.setattr(b.subprocess, "run", compiler)
+    for _ in range(2):
+        with pytest.raises(b.SpillError):
+            b._compile(source, force=False)
+    stderr = REMARKS.format(u=4, scratch=0, spill=0)
+    assert b._compile(source, force=False).exists()
+
+
 # ---- the second check: registers of hand-issued loads touched before their wait ----------
 
 _PROLOGUE = """\
