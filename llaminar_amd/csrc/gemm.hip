@@ -701,18 +701,24 @@ namespace llamql
     // there is to multiply; gemm_split_kernel gives the walk to 2, 4 or 8 wavefronts.  Where the tiles do fill it,
     // gemm_kernel's larger ones decode and rescale less per product.  The expected times in microseconds are fitted to
     // measurements of the three formats:
-    //   tokens x rows x K          gemm_kernel   split (entry)
-    //   40 x 8192 x 5120, IQ3_S       39.6          23.0 (1)
-    //   130 x 5000 x 5120, Q4_K       54            33 (3)
+    //   tokens x rows x K          gemm_kernel   split (its best entry)
+    //   40 x 8192 x 5120, IQ3_S       38            23 (1)
+    //   130 x 5000 x 5120, Q4_K       52            29 (2), 32 (3) is taken
     //   130 x 5000 x 5120, Q6_K       60            38 (3)
-    //   12 x 1500 x 20480, Q4_K       72            35 (0)
-    //   300 x 2000 x 2048, Q4_K       22            14.6 (2)
-    //   40 x 12000 x 8192, Q6_K       71            55 (3)
-    //   199 x 5120 x 25600, Q6_K      298           270 (4)
-    //   256 x 8192 x 8192, Q4_K       84            78 (4)
-    //   20 x 25600 x 5120, Q4_K       33            34 (2)
-    //   1000 x 4096 x 4096, Q4_K      69            82 (4)
-    //   512 x 25600 x 5120, Q4_K      288           346 (4)
+    //   12 x 1500 x 20480, Q4_K       72            34 (0)
+    //   64 x 4096 x 4096, Q4_K        26            12 (0)
+    //   300 x 2000 x 2048, Q4_K       22            15 (2, 3)
+    //   40 x 12000 x 8192, Q6_K       63            51 (3)
+    //   199 x 5120 x 25600, Q6_K      279           261 (4)
+    //   256 x 8192 x 8192, Q4_K       85            79 (4)
+    //   129 x 25600 x 5120, Q4_K      152           116 (2)
+    //   129 x 25600 x 5120, Q6_K      176           166 (4), 170 (2) is taken
+    // and gemm_kernel's shapes:
+    //   20 x 25600 x 5120, Q4_K       30            30 (2)
+    //   1000 x 4096 x 4096, Q4_K      71            83 (4)
+    //   300 x 25600 x 5120, IQ3_S     202           220 (4)
+    //   520 x 14000 x 5120, IQ3_S     197           224 (4)
+    //   512 x 25600 x 5120, Q4_K      275           347 (4)
     struct SplitTile
     {
         int mt, rn, ks;
@@ -731,13 +737,16 @@ namespace llamql
         const double alone = M <= 32 ? 0.9 : M <= 64 ? 2.0 : 2.75, two = M <= 32 ? 1.7 : M <= 64 ? 2.75 : 4.5;
         const long tiles = over(N, GEMM_BN) * over(M, M <= 32 ? 32 : M <= 64 ? 64 : GEMM_BM);
         const long rest = tiles % (2 * CHIP_CUS);
-        double best = 0.95 * SB * ((double)(tiles / (2 * CHIP_CUS)) * two + (rest == 0 ? 0.0 : rest <= CHIP_CUS ? alone : two));
+        const double undivided = SB * ((double)(tiles / (2 * CHIP_CUS)) * two + (rest == 0 ? 0.0 : rest <= CHIP_CUS ? alone : two));
+        double best = undivided;
         int choice = -1;
         for (int i = 0; i < (int)(sizeof(SPLIT) / sizeof(SPLIT[0])); ++i)
         {
             const SplitTile &t = SPLIT[i];
-            const double us = (double)over(over(N, 32 * t.rn) * over(M, 32 * t.mt), CHIP_CUS) * ((double)over(SB, t.ks) * t.step + t.fixed);
-            if (us < best && over(M, 32 * t.mt) <= 65535) // (the grid's second extent)
+            const long rounds = over(over(N, 32 * t.rn) * over(M, 32 * t.mt), CHIP_CUS);
+            const double us = (double)rounds * ((double)over(SB, t.ks) * t.step + t.fixed);
+            // (several rounds: gemm_kernel's overlap, two workgroups a compute unit, and take less than they are counted for)
+            if (us < best && us < (rounds > 1 ? 0.85 : 0.95) * undivided && over(M, 32 * t.mt) <= 65535) // (the grid's second extent)
                 best = us, choice = i;
         }
         return choice;
