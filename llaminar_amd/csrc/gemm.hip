@@ -725,9 +725,8 @@ namespace llamql
         double step, fixed; // microseconds: KS super-blocks, and a workgroup's start and end
     };
     constexpr SplitTile SPLIT[] = {{1, 1, 8, 4.6, 4.0}, {1, 2, 4, 3.8, 4.0}, {1, 4, 2, 3.4, 4.0}, {2, 2, 4, 5.9, 5.0}, {2, 4, 2, 4.9, 4.0}};
-    constexpr int CHIP_CUS = 256;
 
-    inline int gemm_split_choice(int M, int N, int K)
+    inline int gemm_split_choice(int M, int N, int K, int cus)
     {
         if (K > 1 << 24) // 32-bit offsets from a tile's first token
             return -1;
@@ -736,14 +735,14 @@ namespace llamql
         // gemm_kernel: microseconds per super-block of one workgroup alone on a compute unit, and of two sharing it
         const double alone = M <= 32 ? 0.9 : M <= 64 ? 2.0 : 2.75, two = M <= 32 ? 1.7 : M <= 64 ? 2.75 : 4.5;
         const long tiles = over(N, GEMM_BN) * over(M, M <= 32 ? 32 : M <= 64 ? 64 : GEMM_BM);
-        const long rest = tiles % (2 * CHIP_CUS);
-        const double undivided = SB * ((double)(tiles / (2 * CHIP_CUS)) * two + (rest == 0 ? 0.0 : rest <= CHIP_CUS ? alone : two));
+        const long rest = tiles % (2 * cus);
+        const double undivided = SB * ((double)(tiles / (2 * cus)) * two + (rest == 0 ? 0.0 : rest <= cus ? alone : two));
         double best = undivided;
         int choice = -1;
         for (int i = 0; i < (int)(sizeof(SPLIT) / sizeof(SPLIT[0])); ++i)
         {
             const SplitTile &t = SPLIT[i];
-            const long rounds = over(over(N, 32 * t.rn) * over(M, 32 * t.mt), CHIP_CUS);
+            const long rounds = over(over(N, 32 * t.rn) * over(M, 32 * t.mt), cus);
             const double us = (double)rounds * ((double)over(SB, t.ks) * t.step + t.fixed);
             // (several rounds: gemm_kernel's overlap, two workgroups a compute unit, and take less than they are counted for)
             if (us < best && us < (rounds > 1 ? 0.85 : 0.95) * undivided && over(M, 32 * t.mt) <= 65535) // (the grid's second extent)
@@ -756,7 +755,7 @@ namespace llamql
     // whose 64-row tile meets the window are launched.
     template <class F, bool DUMP = false>
     bool gemm_launch(const char *fn, const void *d_w, const void *d_q8, float *d_y, int M, int N, int K, int ldy,
-                     hipStream_t st, int32_t *d_sums = nullptr, int row0 = 0, int nrows = 0)
+                     int device_id, hipStream_t st, int32_t *d_sums = nullptr, int row0 = 0, int nrows = 0)
     {
         GemmArgs g;
         g.w = GemvArgs{};
@@ -779,7 +778,7 @@ namespace llamql
         }
         const int tile_end = DUMP ? (row0 + nrows + GEMM_BN - 1) / GEMM_BN : (N + GEMM_BN - 1) / GEMM_BN;
         const int rows_end = DUMP ? row0 + nrows : N, rows = rows_end - g.tile0 * GEMM_BN;
-        switch (gemm_split_choice(M, N, K))
+        switch (gemm_split_choice(M, N, K, cu_count(device_id)))
         {
         case 0: return gemm_split_launch<F, DUMP, 1, 1, 8>(fn, g, rows, M, st);
         case 1: return gemm_split_launch<F, DUMP, 1, 2, 4>(fn, g, rows, M, st);
@@ -823,9 +822,9 @@ extern "C" bool llam_ql_gemm(uint8_t fmt, const void *d_w, const void *d_q8, flo
     hipStream_t st = as_stream(stream);
     switch (fmt)
     {
-    case LLAM_FMT_Q4_K: return gemm_launch<Q4KTraits>(fn, d_w, d_q8, d_y, M, N, K, ldy, st);
-    case LLAM_FMT_Q6_K: return gemm_launch<Q6KTraits>(fn, d_w, d_q8, d_y, M, N, K, ldy, st);
-    default: return gemm_launch<IQ3STraits>(fn, d_w, d_q8, d_y, M, N, K, ldy, st);
+    case LLAM_FMT_Q4_K: return gemm_launch<Q4KTraits>(fn, d_w, d_q8, d_y, M, N, K, ldy, device_id, st);
+    case LLAM_FMT_Q6_K: return gemm_launch<Q6KTraits>(fn, d_w, d_q8, d_y, M, N, K, ldy, device_id, st);
+    default: return gemm_launch<IQ3STraits>(fn, d_w, d_q8, d_y, M, N, K, ldy, device_id, st);
     }
 }
 
@@ -853,9 +852,9 @@ extern "C" bool llam_ql_gemm_block_sums(uint8_t fmt, const void *d_w, const void
     hipStream_t st = as_stream(stream);
     switch (fmt)
     {
-    case LLAM_FMT_Q4_K: return gemm_launch<Q4KTraits, true>(fn, d_w, d_q8, nullptr, M, N, K, 0, st, d_sums, row0, nrows);
-    case LLAM_FMT_Q6_K: return gemm_launch<Q6KTraits, true>(fn, d_w, d_q8, nullptr, M, N, K, 0, st, d_sums, row0, nrows);
-    default: return gemm_launch<IQ3STraits, true>(fn, d_w, d_q8, nullptr, M, N, K, 0, st, d_sums, row0, nrows);
+    case LLAM_FMT_Q4_K: return gemm_launch<Q4KTraits, true>(fn, d_w, d_q8, nullptr, M, N, K, 0, device_id, st, d_sums, row0, nrows);
+    case LLAM_FMT_Q6_K: return gemm_launch<Q6KTraits, true>(fn, d_w, d_q8, nullptr, M, N, K, 0, device_id, st, d_sums, row0, nrows);
+    default: return gemm_launch<IQ3STraits, true>(fn, d_w, d_q8, nullptr, M, N, K, 0, device_id, st, d_sums, row0, nrows);
     }
 }
 

@@ -33,8 +33,8 @@ namespace llamql
     constexpr int NORM_FUSE_MAX = 8192; // most values (rows x columns) every workgroup norms for itself
 
     __host__ __device__ inline bool is_gated(int out) { return out == LLAM_SEQ_OUT_GATED || out == LLAM_SEQ_OUT_GATED_CLAMP; }
-    bool linear_small(const char *fn, const LinearArgs &a, int batch, int dtype, hipStream_t st);
-    bool linear_tiled(const char *fn, const LinearArgs &a, int batch, int dtype, hipStream_t st);
+    bool linear_small(const char *fn, const LinearArgs &a, int batch, int dtype, int device_id, hipStream_t st);
+    bool linear_tiled(const char *fn, const LinearArgs &a, int batch, int dtype, int device_id, hipStream_t st);
 
     // Whether a sum of products in three bf16 pieces of each 32-bit value may not be that of the whole values, which then
     // are multiplied once more without pieces: the second and third piece of most values are zero, and zero times an infinite

@@ -347,7 +347,7 @@ namespace llamql
             return launched(fn);
         }
         template <typename T, int NW, bool NORM>
-        bool small_tiles(const char *fn, const LinearArgs &a, int batch, hipStream_t st)
+        bool small_tiles(const char *fn, const LinearArgs &a, int batch, int cus, hipStream_t st)
         {
             // Half tiles where they too find a compute unit each and whole ones need more than a round of eight steps for K (fp32
             // rows from memory: always, their products take as long as the weights).  Not between a quarter and half of the
@@ -358,10 +358,9 @@ namespace llamql
             //   8 x 2048 x 2048  bf16  3.4,  3.6  fp32  5.8,  4.5      8 x 512 x 512     bf16  2.6,  2.6  fp32    3.5,  2.8
             //   1 x 1536 x 8192  bf16  5.5,  5.8  normed 6.5, 8.5      1 x 512 x 8192    bf16  5.4,  3.8  normed  6.2,  5.3
             //   1 x 1792 x 4096  bf16  3.6,  4.2  normed 4.7, 5.9      8 x 2048 x 16384  bf16 16.8, 14.9  fp32   27.4, 20.1
-            constexpr int CUS = 256;
             const long tiles = (long)a.N / 16 * batch;
-            const bool channels = tiles > CUS / 4 && (a.K == 4096 || a.K == 8192);
-            const bool half = a.M <= 8 && tiles <= CUS / 2 && ((sizeof(T) == 4 && !NORM) || (a.K > 2048 && !channels));
+            const bool channels = tiles > cus / 4 && (a.K == 4096 || a.K == 8192);
+            const bool half = a.M <= 8 && tiles <= cus / 2 && ((sizeof(T) == 4 && !NORM) || (a.K > 2048 && !channels));
             if (half)
                 return small_launch<T, NW, 1, NORM, true>(fn, a, batch, st);
             if (sizeof(T) == 4 && !NORM && a.K <= 8 * NW * 32) // one round of eight steps
@@ -369,15 +368,15 @@ namespace llamql
             return small_launch<T, NW, 1, NORM>(fn, a, batch, st);
         }
         template <typename T>
-        bool small_dispatch(const char *fn, const LinearArgs &a, int batch, hipStream_t st)
+        bool small_dispatch(const char *fn, const LinearArgs &a, int batch, int cus, hipStream_t st)
         {
             const bool gated = is_gated(a.out);
             const bool wide = a.K >= 1024;
             if (a.norm)
-                return gated ? small_launch<T, 8, 2, true>(fn, a, batch, st) : small_tiles<T, 8, true>(fn, a, batch, st);
+                return gated ? small_launch<T, 8, 2, true>(fn, a, batch, st) : small_tiles<T, 8, true>(fn, a, batch, cus, st);
             if (gated)
                 return small_launch<T, 8, 2, false>(fn, a, batch, st);
-            return wide ? small_tiles<T, 8, false>(fn, a, batch, st) : small_tiles<T, 4, false>(fn, a, batch, st);
+            return wide ? small_tiles<T, 8, false>(fn, a, batch, cus, st) : small_tiles<T, 4, false>(fn, a, batch, cus, st);
         }
     } // namespace
 
@@ -401,9 +400,10 @@ namespace llamql
         }
     } // namespace
 
-    bool linear_small(const char *fn, const LinearArgs &a, int batch, int dtype, hipStream_t st)
+    bool linear_small(const char *fn, const LinearArgs &a, int batch, int dtype, int device_id, hipStream_t st)
     {
-        return dtype == LLAM_SEQ_F32 ? small_dispatch<float>(fn, a, batch, st) : small_dispatch<bf16>(fn, a, batch, st);
+        const int cus = cu_count(device_id);
+        return dtype == LLAM_SEQ_F32 ? small_dispatch<float>(fn, a, batch, cus, st) : small_dispatch<bf16>(fn, a, batch, cus, st);
     }
 } // namespace llamql
 
@@ -451,8 +451,8 @@ extern "C" bool llam_seq_linear(const llam_seq_linear_args *a, int dtype, int de
         return true;
     if (!set_device(fn, device_id))
         return false;
-    return a->M <= SMALL_M ? linear_small(fn, p, a->batch, dtype, as_stream(stream))
-                           : linear_tiled(fn, p, a->batch, dtype, as_stream(stream));
+    return a->M <= SMALL_M ? linear_small(fn, p, a->batch, dtype, device_id, as_stream(stream))
+                           : linear_tiled(fn, p, a->batch, dtype, device_id, as_stream(stream));
 }
 
 extern "C" bool llam_seq_linear_pair(const llam_seq_linear_args *a, const llam_seq_linear_args *b, int dtype, int device_id, void *stream)
@@ -470,5 +470,5 @@ extern "C" bool llam_seq_linear_pair(const llam_seq_linear_args *a, const llam_s
     hipStream_t st = as_stream(stream);
     if (p.M <= SMALL_M)
         return dtype == LLAM_SEQ_F32 ? small_pair_dispatch<float>(fn, p, q, st) : small_pair_dispatch<bf16>(fn, p, q, st);
-    return linear_tiled(fn, p, 1, dtype, st) && linear_tiled(fn, q, 1, dtype, st);
+    return linear_tiled(fn, p, 1, dtype, device_id, st) && linear_tiled(fn, q, 1, dtype, device_id, st);
 }

@@ -493,9 +493,8 @@ namespace llamql
             {64, 128, 2, 1, 1.45f, 1.75f, 3.0f, wide_launch<float, 64, 128, 2, 2, 2, 2>},
             {64, 64, 2, 1, 1.15f, 1.30f, 3.0f, wide_launch<float, 64, 64, 2, 2, 2, 3>},
         };
-        constexpr int UNITS = 256; // compute units
 
-        float expected(const Tile &t, const LinearArgs &a, int batch)
+        float expected(const Tile &t, const LinearArgs &a, int batch, int cus)
         {
             float rows = (float)ceil_div(a.M, t.rows) * batch;
             if (a.group_offset)
@@ -504,19 +503,20 @@ namespace llamql
                 const float groups = (float)(batch < a.group_rows ? batch : a.group_rows);
                 rows = fmaxf(groups, (float)a.group_rows / t.rows + 0.5f * groups);
             }
-            const float tiles = rows * ceil_div(a.N, t.columns), slots = (float)UNITS * t.resident;
+            const float tiles = rows * ceil_div(a.N, t.columns), slots = (float)cus * t.resident;
             const float fill = tiles < slots ? tiles / slots : 1.0f;
             const float turn = t.alone + (t.full - t.alone) * fill;
             return ceilf(tiles / slots) * (ceil_div(a.K / TILE_K, t.groups) * turn + t.start);
         }
     } // namespace
 
-    bool linear_tiled(const char *fn, const LinearArgs &a, int batch, int dtype, hipStream_t st)
+    bool linear_tiled(const char *fn, const LinearArgs &a, int batch, int dtype, int device_id, hipStream_t st)
     {
+        const int cus = cu_count(device_id);
         const Tile *tiles = dtype == LLAM_SEQ_F32 ? TILES_F32 : TILES_BF16, *best = tiles;
         const size_t n = dtype == LLAM_SEQ_F32 ? sizeof TILES_F32 / sizeof(Tile) : sizeof TILES_BF16 / sizeof(Tile);
         for (size_t i = 1; i < n; ++i)
-            if (expected(tiles[i], a, batch) < expected(*best, a, batch))
+            if (expected(tiles[i], a, batch, cus) < expected(*best, a, batch, cus))
                 best = &tiles[i];
         return best->launch(fn, a, batch, st);
     }

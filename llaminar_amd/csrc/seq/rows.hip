@@ -411,7 +411,7 @@ namespace llamql
         }
 
         template <typename T>
-        bool experts_run(const char *fn, ExpertArgs p, int M, char *scratch, int dtype, hipStream_t st)
+        bool experts_run(const char *fn, ExpertArgs p, int M, char *scratch, int dtype, int device_id, hipStream_t st)
         {
             const ExpertScratch at = expert_scratch(M, p.experts, p.top, p.ff, p.shared_ff, p.N);
             p.ids = reinterpret_cast<int *>(scratch + at.ids);
@@ -449,11 +449,11 @@ namespace llamql
             l.a = p.h, l.lda = p.K, l.w = p.up, l.w_stride = p.up_stride, l.y = act, l.ldy = p.ff;
             l.M = M, l.N = p.ff, l.K = p.K, l.out = LLAM_SEQ_OUT_RELU2;
             l.group_offset = offset, l.row_source = order, l.source_div = p.top, l.groups = p.experts, l.group_rows = M * p.top;
-            if (!linear_tiled(fn, l, p.experts, dtype, st))
+            if (!linear_tiled(fn, l, p.experts, dtype, device_id, st))
                 return false;
             l.a = act, l.lda = p.ff, l.w = p.down, l.w_stride = p.down_stride, l.y = pair_out, l.ldy = p.N;
             l.N = p.N, l.K = p.ff, l.out = LLAM_SEQ_OUT_F32, l.row_source = nullptr, l.source_div = 1;
-            if (!linear_tiled(fn, l, p.experts, dtype, st))
+            if (!linear_tiled(fn, l, p.experts, dtype, device_id, st))
                 return false;
             if (p.shared_ff)
             {
@@ -461,11 +461,11 @@ namespace llamql
                 s.source_div = 1;
                 s.a = p.h, s.lda = p.K, s.w = p.shared_up, s.y = shared_act, s.ldy = p.shared_ff;
                 s.M = M, s.N = p.shared_ff, s.K = p.K, s.out = LLAM_SEQ_OUT_RELU2;
-                if (!linear_tiled(fn, s, 1, dtype, st))
+                if (!linear_tiled(fn, s, 1, dtype, device_id, st))
                     return false;
                 s.a = shared_act, s.lda = p.shared_ff, s.w = p.shared_down, s.y = shared_out, s.ldy = p.N;
                 s.N = p.N, s.K = p.shared_ff, s.out = LLAM_SEQ_OUT_F32;
-                if (!linear_tiled(fn, s, 1, dtype, st))
+                if (!linear_tiled(fn, s, 1, dtype, device_id, st))
                     return false;
             }
             hipLaunchKernelGGL(expert_combine_kernel, dim3(M), dim3(ROW_THREADS), 0, st, p, pair_out, shared_out, place);
@@ -572,8 +572,8 @@ extern "C" bool llam_seq_experts(const llam_seq_experts_args *a, int M, void *d_
     p.up_stride = a->up_stride, p.down_stride = a->down_stride;
     p.experts = a->experts, p.top = a->top, p.ff = a->ff, p.shared_ff = a->shared_ff, p.K = a->K, p.N = a->N;
     p.h = a->d_h, p.x = a->d_x, p.ldx = a->ldx;
-    return dtype == LLAM_SEQ_F32 ? experts_run<float>(fn, p, M, static_cast<char *>(d_scratch), dtype, as_stream(stream))
-                                 : experts_run<bf16>(fn, p, M, static_cast<char *>(d_scratch), dtype, as_stream(stream));
+    return dtype == LLAM_SEQ_F32 ? experts_run<float>(fn, p, M, static_cast<char *>(d_scratch), dtype, device_id, as_stream(stream))
+                                 : experts_run<bf16>(fn, p, M, static_cast<char *>(d_scratch), dtype, device_id, as_stream(stream));
 }
 
 extern "C" bool llam_seq_record(const int32_t *d_ids, int n, int32_t *d_out, int32_t *d_count, int max_count,
