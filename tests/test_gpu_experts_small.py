@@ -44,11 +44,14 @@ def test_rows_together_are_rows_alone(dev, M, experts, top, ff, shared, dtype):
 
 
 # rows, experts, of a row, width of an expert, of the model, slope of the logits: few rows; more than 64 experts, evenly and
-# mostly the first ones chosen, many without a row; groups of several tiles with a last one of few rows, of all rows
+# mostly the first ones chosen, many without a row; groups of several tiles with a last one of few rows, of all rows; each tile
+# (test_launch_rules.py)
 @pytest.mark.parametrize("dtype", [sq.BF16, sq.F32])
 @pytest.mark.parametrize("M,experts,top,ff,K,slope", [(17, 8, 2, 64, 320, 0.0), (40, 130, 3, 192, 256, 0.0), (300, 150, 4, 192, 128, 0.2),
                                                       (300, 64, 6, 320, 192, 0.0), (700, 3, 2, 320, 128, 0.5), (260, 5, 1, 64, 64, 9.0),
-                                                      (500, 40, 3, 2048, 64, 0.1), (400, 20, 3, 64, 1088, 0.0)])
+                                                      (500, 40, 3, 2048, 64, 0.1), (400, 20, 3, 64, 1088, 0.0),
+                                                      (200, 12, 2, 2688, 64, 0.2), (1200, 2, 2, 2368, 64, 0.0), (700, 4, 2, 1024, 1088, 0.5),
+                                                      (1500, 3, 3, 4096, 64, 0.0)])
 def test_rows_grouped_by_expert(dev, M, experts, top, ff, K, slope, dtype):
     import torch
 

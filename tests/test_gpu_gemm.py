@@ -33,7 +33,9 @@ def test_golden_fixture(capi, dev, golden, fmt):
                                    (32, 200, 1024), (33, 130, 5120), (96, 64, 2048), (97, 64, 2048),
                                    # 33 to 64 tokens whose walk one workgroup keeps: a tile of 64, full and not, rows
                                    # of one row tile and of many
-                                   (64, 130, 1024), (40, 130, 512), (33, 20480, 2048), (57, 65, 256)])
+                                   (64, 130, 1024), (40, 130, 512), (33, 20480, 2048), (57, 65, 256),
+                                   # and more, in tiles of 128
+                                   (130, 257, 256), (255, 100, 512)])
 def test_random_shapes(capi, dev, oracle, fmt, M, N, K):
     W = synth.weights_numpy(fmt, N, K, 7 + M + N)
     q8 = oracle.quantize(synth.activations_numpy(M, K, 9 + K))
@@ -63,7 +65,8 @@ def test_gemm_rows_equal_gemv(capi, dev, oracle, fmt):
 @pytest.mark.parametrize("fmt", list(FMTS.values()), ids=list(FMTS))
 @pytest.mark.parametrize("M,N,K,r0,nr", [(1, 128, 256, 0, 128), (17, 100, 512, 37, 63), (130, 257, 768, 190, 67),
                                          (300, 200, 2048, 60, 70), (40, 130, 1280, 60, 70), (96, 70, 512, 0, 70),
-                                         (64, 130, 1024, 60, 70), (40, 130, 512, 1, 129), (57, 65, 256, 64, 1)])
+                                         (64, 130, 1024, 60, 70), (40, 130, 512, 1, 129), (57, 65, 256, 64, 1),
+                                         (130, 257, 256, 190, 67), (255, 100, 512, 37, 63)])
 def test_block_sums_of_the_gemm_kernel(capi, dev, oracle, fmt, M, N, K, r0, nr):
     """The matrix unit's per-block results of llam_ql_gemm's own kernels (block-sum variants, chosen by the same rule) are
     the reference's int32 sums bit for bit: ragged tiles, windows that start and end inside a 64-row tile, token tails,

@@ -36,10 +36,11 @@ def close(torch, y, a, w, K, extra=0.0):
 
 
 # rows x columns x K: a single row more than the row-at-a-time kernel takes, edges of every tile, K of one and of an
-# odd number of turns, sizes at which each tile is chosen
+# odd number of turns, and each tile with rows and columns left over (test_launch_rules.py)
 SHAPES = [(17, 16, 64), (31, 48, 192), (33, 80, 320), (64, 64, 128), (65, 272, 704), (100, 6160, 2048), (127, 144, 64),
           (129, 256, 2048), (255, 528, 192), (257, 1040, 128), (300, 6160, 512), (522, 2048, 2112), (300, 16384, 192),
-          (1000, 8208, 64), (2048, 2048, 192), (2048, 4112, 128), (2048, 15440, 64)]
+          (1000, 8208, 64), (2048, 2048, 192), (2048, 4112, 128), (2048, 15440, 64),
+          (1000, 6160, 192), (2000, 3088, 320), (300, 8208, 192), (2000, 2064, 192), (520, 2064, 2112)]
 
 
 @pytest.mark.parametrize("dtype", [BF16, F32])
@@ -59,7 +60,7 @@ def test_sums(dev, M, N, K, dtype):
 
 @pytest.mark.parametrize("dtype", [BF16, F32])
 @pytest.mark.parametrize("out", [sq.OUT_ADD, sq.OUT_ELEM, sq.OUT_GATED, sq.OUT_RELU2, sq.OUT_GATED_CLAMP])
-@pytest.mark.parametrize("M,N,K", [(40, 96, 192), (300, 2080, 128), (2048, 4128, 64)])
+@pytest.mark.parametrize("M,N,K", [(40, 96, 192), (300, 2080, 128), (2048, 4128, 64), (1000, 6176, 192)])
 def test_outputs(dev, M, N, K, out, dtype):
     import torch
 
