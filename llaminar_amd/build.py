@@ -115,7 +115,7 @@ def _vregs(text: str) -> set[int]:
 
 def _device_functions(asm: str):
     """(name, blocks) of every function in the device assembly; a block is a label (None: the function's first) and its
-    operations, in order, as the in-flight check needs them."""
+    instructions, in order, each with whether it lies inside inline assembly."""
     name, blocks, in_asm = "?", [(None, [])], False
     for raw_line in asm.splitlines():
         text = raw_line.strip()
@@ -131,17 +131,28 @@ def _device_functions(asm: str):
         if m and m.group(1).startswith(".LBB"):
             blocks.append((m.group(1), []))
             continue
-        if not text or text.startswith(".") or text.endswith(":"):
-            continue
-        ops = blocks[-1][1]
+        if text and not text.startswith(".") and not text.endswith(":"):
+            blocks[-1][1].append((text, in_asm))
+    yield name, blocks
+
+
+def _control(text: str):
+    """("jump" or "branch", label) or ("end", None) of an instruction that control may leave its block at, else None."""
+    if m := re.match(r"^s_c?branch\w*\s+(\S+)", text):
+        return "jump" if text.startswith("s_branch") else "branch", m.group(1)
+    return ("end", None) if re.match(r"^(s_endpgm|s_setpc_b64)\b", text) else None
+
+
+def _queue_operations(instructions):
+    """What of a block's instructions matters to the in-flight check: (kind, registers or label or count, text)."""
+    ops = []
+    for text, in_asm in instructions:
         if text.startswith("s_waitcnt"):
             w = _VMCNT.search(text)
             if w:
                 ops.append(("wait", int(w.group(1)), text))
-        elif m := re.match(r"^s_c?branch\w*\s+(\S+)", text):
-            ops.append(("jump" if text.startswith("s_branch") else "branch", m.group(1), text))
-        elif re.match(r"^(s_endpgm|s_setpc_b64)\b", text):
-            ops.append(("end", None, text))
+        elif control := _control(text):
+            ops.append((*control, text))
         else:
             load = _ASM_LOAD.match(text) if in_asm else None
             touched = frozenset(_vregs(text))
@@ -151,7 +162,7 @@ def _device_functions(asm: str):
                 ops.append(("memory", touched, text))
             elif touched:
                 ops.append(("use", touched, text))
-    yield name, blocks
+    return ops
 
 
 # states of the queue a block may be entered with before the check gives up (the kernels here need up to about a hundred)
@@ -177,6 +188,7 @@ def check_inflight_registers(asm: str, src_name: str) -> int:
     findings: dict[str, None] = {}
     followed = 0
     for func, blocks in _device_functions(asm):
+        blocks = [(label, _queue_operations(instructions)) for label, instructions in blocks]
         loads = sum(op[0] == "load" for _, ops in blocks for op in ops)
         followed += loads
         if not loads:
@@ -251,36 +263,55 @@ def check_scalar_hazards(asm: str, src_name: str) -> int:
 
     The hardware does not wait by itself, and the compiler inserts the wait states for its own instructions only: such
     a load takes a stale value, half of another pointer, for its base.  An instruction counts as one wait state,
-    s_nop N as N + 1.  Straight-line bookkeeping like check_inflight_registers, carried across labels.  Returns the
-    number of loads and stores looked at.
+    s_nop N as N + 1.  Every jump is followed both ways; where ways meet, a register counts as written as lately as on any of
+    them.  Returns the number of loads and stores looked at.
     """
-    findings: list[str] = []
-    looked, func, in_asm = 0, "?", False
-    written: dict[int, int] = {}   # scalar register -> wait states since a vector instruction wrote it
-    for raw_line in asm.splitlines():
-        text = raw_line.strip()
-        if text.startswith(";;#ASMSTART") or text.startswith(";;#ASMEND"):
-            in_asm = text.startswith(";;#ASMSTART")
+    findings: dict[str, None] = {}
+    looked = 0
+    for func, blocks in _device_functions(asm):
+        own = sum(in_asm and _VMEM.match(text) is not None for _, instructions in blocks for text, in_asm in instructions)
+        looked += own
+        if not own:
             continue
-        m = re.match(r"^([A-Za-z_][\w$.]*):", raw_line)
-        if m and not raw_line.startswith(".L"):
-            func, written = m.group(1), {}
-            continue
-        text = text.split(";")[0].strip()
-        if not text or text.startswith(".") or text.endswith(":"):
-            continue
-        if in_asm and _VMEM.match(text):
-            looked += 1
-            hit = sorted(r for r in _sregs(text) if r in written)
-            if hit:
-                findings.append(f"{func}: '{text}' reads s{hit[0]} {written[hit[0]]} wait states after a vector instruction wrote it")
-        passed = int(text.split()[1], 0) + 1 if text.startswith("s_nop") else 1
-        written = {r: n + passed for r, n in written.items() if n + passed < SCALAR_WAIT_STATES}
-        m = _VALU_TO_SREG.match(text)
-        if m:
-            written.update(dict.fromkeys(_sregs(m.group(1)), 0))
+        at = {label: i for i, (label, _) in enumerate(blocks)}
+        # scalar register -> fewest wait states since a vector instruction wrote it, where a block begins (None: not reached)
+        begin: list[dict[int, int] | None] = [None] * len(blocks)
+        work: list[int] = []
+
+        def enter(i, written):
+            if i is None or i >= len(blocks):
+                return
+            if begin[i] is None:
+                begin[i] = dict(written)
+            else:
+                less = {r: n for r, n in written.items() if n < begin[i].get(r, SCALAR_WAIT_STATES)}
+                if not less:
+                    return
+                begin[i].update(less)
+            work.append(i)
+
+        enter(0, {})
+        while work:
+            i = work.pop()
+            written = dict(begin[i])
+            for text, in_asm in blocks[i][1]:
+                if in_asm and written and _VMEM.match(text):
+                    hit = sorted(r for r in _sregs(text) if r in written)
+                    if hit:
+                        findings[f"{func}: '{text}' reads s{hit[0]} {written[hit[0]]} wait states after a vector instruction wrote it"] = None
+                if written:
+                    passed = int(text.split()[1], 0) + 1 if text.startswith("s_nop") else 1
+                    written = {r: n + passed for r, n in written.items() if n + passed < SCALAR_WAIT_STATES}
+                if m := _VALU_TO_SREG.match(text):
+                    written.update(dict.fromkeys(_sregs(m.group(1)), 0))
+                if control := _control(text):
+                    enter(at.get(control[1]), written)
+                    if control[0] != "branch":
+                        break
+            else:
+                enter(i + 1, written)
     if findings:
-        shown = "\n  ".join(findings[:12]) + ("" if len(findings) <= 12 else f"\n  ... and {len(findings) - 12} more")
+        shown = "\n  ".join(list(findings)[:12]) + ("" if len(findings) <= 12 else f"\n  ... and {len(findings) - 12} more")
         raise ScalarHazardError(f"{src_name}: hand-issued loads take a stale scalar register (see check_scalar_hazards):\n  {shown}")
     return looked
 

@@ -275,3 +275,25 @@ def test_scalar_instructions_and_the_compilers_own_loads_need_no_wait():
     assert b.check_scalar_hazards(asm, "moe.hip") == 1
     own = SCALAR.format(between="").replace("\t;;#ASMSTART\n", "").replace("\t;;#ASMEND\n", "")
     assert b.check_scalar_hazards(own, "moe.hip") == 0
+
+
+def test_the_wait_for_a_base_is_followed_over_jumps():
+    loop = """\
+_Z6kernelv:
+.LBB0_1:
+\t;;#ASMSTART
+\tglobal_load_dwordx4 v[18:21], v2, s[6:7]
+\t;;#ASMEND
+\tv_readfirstlane_b32 s6, v3
+{between}
+\ts_cbranch_scc1 .LBB0_1
+\ts_endpgm
+"""
+    with pytest.raises(b.ScalarHazardError, match="s6 4 wait states"):
+        b.check_scalar_hazards(loop.format(between="\ts_nop 2"), "moe.hip")
+    assert b.check_scalar_hazards(loop.format(between="\ts_nop 3"), "moe.hip") == 1
+    # ahead of an unconditional jump, and what stands behind it in the text only
+    with pytest.raises(b.ScalarHazardError, match="s6"):
+        b.check_scalar_hazards(loop.format(between="\ts_branch .LBB0_1"), "moe.hip")
+    past = "_Z6kernelv:\n\tv_readfirstlane_b32 s7, v3\n\ts_branch .LBB0_2\n.LBB0_1:\n" + SCALAR.split("{between}\n")[1] + ".LBB0_2:\n\ts_endpgm\n"
+    assert b.check_scalar_hazards(past, "moe.hip") == 1
