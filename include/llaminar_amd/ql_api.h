@@ -290,15 +290,19 @@ bool llam_ql_gemv_describe(uint8_t fmt, int M, int N, int K, int has_plane, int 
  * gemm_native_vnni_preq (CPUNativeVNNIGemv.h:2046-2287); device-side
  * counterpart of launch_native_vnni_gemm
  * (src/v2/kernels/rocm/gemm/ROCmQuantisedGemmKernel_native_VNNI.hip:2580-2632).
- * Token tiles of 32 (M <= 32), 64 (M <= 64) or 128 tokens: the fp32 sum of a row's blocks
- * is formed in an order that depends on the tile, so a row's last bits may differ between
- * calls of different M (the per-block int32 sums never do). */
+ * Two kernels, chosen by their expected times: token tiles of 32 (M <= 32), 64 (M <= 64) or
+ * 128 tokens whose walk along K one workgroup keeps, and, where those would leave the chip
+ * partly idle, tiles of 32 or 64 tokens whose walk is dealt to 2, 4 or 8 wavefronts.  The
+ * fp32 sum of a row's blocks is formed in an order that depends on the kernel and the tile,
+ * so a row's last bits may differ between calls of different M or N (the per-block int32
+ * sums never do).  The same call always gives the same bits. */
 bool llam_ql_gemm(uint8_t fmt, const void *d_w, const void *d_q8, float *d_y,
                   int M, int N, int K, int ldy, int device_id, void *stream);
 
 /* Parity hook of the GEMM: the matrix unit's exact per-block int32 sums of weight rows
  * [row0, row0+nrows) for all M activation rows, d_sums[(m*nrows + r)*(K/32) + kb], from
- * the block-sum variant of llam_ql_gemm's kernel (same tiles, same decode, same MFMA).
+ * the block-sum variant of the kernel that llam_ql_gemm runs for (M, N, K): same tiles, same
+ * decode, same MFMA.
  * Counterpart of the reference's int32 accumulators in gemm_2row_native_chunk /
  * gemm_2row_int8_chunk (CPUNativeVNNIGemv.h:1046-1376). */
 bool llam_ql_gemm_block_sums(uint8_t fmt, const void *d_w, const void *d_q8, int32_t *d_sums,

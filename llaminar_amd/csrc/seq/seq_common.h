@@ -2,11 +2,13 @@
 // reductions, launch-time checks.
 //
 // Every kernel is a template over the operand type T: bf16 (16-bit matrix operands, 32-bit sums)
-// or float (true 32-bit products on v_mfma_f32_16x16x4_f32).  One "k-step" is 32 elements of the
-// inner dimension in both: lane (r = lane & 15, g = lane >> 4) holds elements 8 g .. 8 g + 7 of
-// row (or column) r.  For float the step is eight 16x16x4 products, product j pairing element
-// 8 g + j of both operands, so the two operand layouts are the same.  A 16x16 result leaves lane
-// (c, g) with rows 4 g .. 4 g + 3 of column c.
+// or float (32-bit values and sums).  One "k-step" is 32 elements of the inner dimension in both:
+// lane (r = lane & 15, g = lane >> 4) holds elements 8 g .. 8 g + 7 of row (or column) r.  For
+// float the step is eight products of v_mfma_f32_16x16x4_f32, product j pairing element 8 g + j
+// of both operands, so the two operand layouts are the same.  A 16x16 result leaves lane
+// (c, g) with rows 4 g .. 4 g + 3 of column c.  Linear layers of more than 16 rows, and those
+// that norm their rows, cut a float into three bf16 values that add up to it instead (exact:
+// the weights are bf16; linear_tiled.hip, linear.hip).
 #pragma once
 
 #include <hip/hip_runtime.h>

@@ -16,8 +16,8 @@ def capi(dev):
     return capi
 
 
-# format, hidden, inter, routed experts, tokens, routed slots: tiles of 16, 32 and 64 pairs; experts of one pair and
-# of all tokens; rows of 1, 2, 3, 8 and 16 super-blocks (the longest leave no room for 64 pairs)
+# format, hidden, inter, routed experts, tokens, routed slots: tiles of 16 and 32 pairs; experts of one pair and
+# of all tokens; rows of 1, 2, 3, 4, 8 and 16 super-blocks (of the longest in Q4_K, 32 pairs find no room)
 CASES = [("iq3_s", 2048, 512, 64, 61, 8), ("iq3_s", 768, 256, 40, 73, 5), ("q4_k", 1024, 768, 16, 100, 4),
          ("q6_k", 512, 1024, 8, 150, 2), ("q4_k", 4096, 256, 4, 300, 1), ("iq3_s", 256, 4096, 3, 220, 2),
          ("q6_k", 2048, 512, 100, 64, 8), ("q4_k", 2048, 512, 32, 60, 8), ("q4_k", 256, 256, 1, 431, 1)]
