@@ -350,17 +350,16 @@ namespace llamql
         bool small_tiles(const char *fn, const LinearArgs &a, int batch, int cus, hipStream_t st)
         {
             // Half tiles where they too find a compute unit each and whole ones need more than a round of eight steps for K (fp32
-            // rows from memory: always, their products take as long as the weights).  Not between a quarter and half of the
-            // units with rows of W 8 or 16 KB apart: eight rows of each of so many workgroups meet in the same channels.
-            // M x N x K, us, whole and half tiles:
-            //   8 x 1024 x 3072  bf16  4.6,  3.9  fp32  7.0,  5.7      1 x 2048 x 5120   bf16  4.9,  4.0  normed  5.4,  5.1
-            //   8 x 2048 x 10240 bf16 11.8, 11.1  fp32 19.0, 14.4      8 x 2304 x 10240  bf16 12.2, 16.5  fp32   19.1, 24.4
-            //   8 x 2048 x 2048  bf16  3.4,  3.6  fp32  5.8,  4.5      8 x 512 x 512     bf16  2.6,  2.6  fp32    3.5,  2.8
-            //   1 x 1536 x 8192  bf16  5.5,  5.8  normed 6.5, 8.5      1 x 512 x 8192    bf16  5.4,  3.8  normed  6.2,  5.3
-            //   1 x 1792 x 4096  bf16  3.6,  4.2  normed 4.7, 5.9      8 x 2048 x 16384  bf16 16.8, 14.9  fp32   27.4, 20.1
+            // rows from memory: always, their products take as long as the weights).  M x N x K, us, whole and half tiles, weights
+            // from memory as in a decode step, whose layers do not fit the caches:
+            //   8 x 1024 x 3072  bf16  6.3,  5.3  fp32  8.2,  7.0      1 x 2048 x 5120   bf16  7.8,  7.1  normed  8.4,  8.0
+            //   8 x 2048 x 10240 bf16 14.9, 13.1  fp32 20.7, 16.2      8 x 2304 x 10240  bf16 15.1, 20.4  fp32   20.9, 27.2
+            //   8 x 2048 x 2048  bf16  5.0,  5.0  fp32  7.3,  6.1      8 x 512 x 512     bf16  2.9,  2.8  fp32    3.7,  3.0
+            //   1 x 2048 x 8192  bf16  9.9,  8.3  normed 11.4, 10.9    1 x 4080 x 4096   bf16  8.0,  7.9  normed  9.5,  9.6
+            // (Of weights that the caches hold, as in a loop over one matrix, rows of W 8 or 16 KB apart meet in the same channels, and
+            // 1 x 2048 x 8192 normed takes 7.8 and 9.8, unnormed 6.2 and 6.8.)
             const long tiles = (long)a.N / 16 * batch;
-            const bool channels = tiles > cus / 4 && (a.K == 4096 || a.K == 8192);
-            const bool half = a.M <= 8 && tiles <= cus / 2 && ((sizeof(T) == 4 && !NORM) || (a.K > 2048 && !channels));
+            const bool half = a.M <= 8 && tiles <= cus / 2 && ((sizeof(T) == 4 && !NORM) || a.K > 2048);
             if (half)
                 return small_launch<T, NW, 1, NORM, true>(fn, a, batch, st);
             if (sizeof(T) == 4 && !NORM && a.K <= 8 * NW * 32) // one round of eight steps
