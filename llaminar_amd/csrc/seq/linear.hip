@@ -117,14 +117,13 @@ namespace llamql
     // HALF: up to 8 rows of A, and a workgroup for 8 rows of W, half a tile: a step is two k-steps, W's rows of the second
     // beside those of the first as the matrix unit's other 8 rows, A's likewise as its other 8 columns, and of the product
     // the two blocks that match are kept.  Twice the workgroups, for layers of fewer tiles than the chip has compute units.
-    // LONG: fp32 rows in rounds of four steps with the rows asked for ahead, and not of eight without (see AHEAD).
-    template <typename T, int NW, int RT, bool NORM, bool HALF = false, bool LONG = true>
+    template <typename T, int NW, int RT, bool NORM, bool HALF = false>
     __device__ __forceinline__ void linear_small_tile(const LinearArgs &p, int block)
     {
         using O = Operand<T>;
         using V = typename O::V;
         static_assert(!HALF || RT == 1, "half a tile");
-        constexpr int U = RT == 1 && (NORM || sizeof(T) == 2 || !LONG) ? 8 : 4;
+        constexpr int U = RT == 1 && (NORM || sizeof(T) == 2) ? 8 : 4;
         constexpr int STEP = HALF ? 2 : 1;   // k-steps (their number is even)
         constexpr bool CUT = NORM && sizeof(T) == 4; // rows in three bf16 pieces
         extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -192,9 +191,7 @@ namespace llamql
             // 19.3 -> 14.1; 8 x 5120 x 25600 bf16 75 -> 67 us, fp32 110 -> 86).  Not in a last round with fewer than U steps:
             // there are no next weights, and rows asked for in vain took as long as the others (16 x 5120 x 1024 in
             // bf16 6.3 -> 4.6).
-            // (Two tiles or eight steps of fp32 rows: registers of a second workgroup.  Walks of one round of eight steps gain
-            // nothing from rows ahead of later weights, and lose with half the weights asked for at first: 16 x 5120 x 2048 11.0 -> 10.6.)
-            constexpr bool AHEAD = !NORM && (sizeof(T) == 2 || (RT == 1 && LONG));
+            constexpr bool AHEAD = !NORM && (sizeof(T) == 2 || RT == 1); // (two tiles of fp32 rows: registers of a second workgroup)
             if (AHEAD && __builtin_amdgcn_readfirstlane(s0 + (U - 1) * NW < steps))
             {
                 V b[AHEAD ? U : 1];
@@ -314,11 +311,11 @@ namespace llamql
         }
     }
 
-    template <typename T, int NW, int RT, bool NORM, bool HALF, bool LONG>
+    template <typename T, int NW, int RT, bool NORM, bool HALF>
     __global__ void __launch_bounds__(NW * 64)
         linear_small_kernel(LinearArgs p)
     {
-        linear_small_tile<T, NW, RT, NORM, HALF, LONG>(p, blockIdx.x);
+        linear_small_tile<T, NW, RT, NORM, HALF>(p, blockIdx.x);
     }
 
     // Two layers over the same rows: the first `blocks` workgroups belong to p.
@@ -335,12 +332,12 @@ namespace llamql
 
     namespace
     {
-        template <typename T, int NW, int RT, bool NORM, bool HALF = false, bool LONG = true>
+        template <typename T, int NW, int RT, bool NORM, bool HALF = false>
         bool small_launch(const char *fn, const LinearArgs &a, int batch, hipStream_t st)
         {
             static LdsGrant grant;
             const size_t lds = NORM ? norm_lds<T>(a) : 0;
-            const auto kernel = &linear_small_kernel<T, NW, RT, NORM, HALF, LONG>;
+            const auto kernel = &linear_small_kernel<T, NW, RT, NORM, HALF>;
             if (lds > 32 * 1024 && allow_lds(grant, reinterpret_cast<const void *>(kernel), 64 * 1024) != hipSuccess)
                 return fail(fn, "cannot reserve %zu bytes of LDS", lds);
             hipLaunchKernelGGL(kernel, dim3(a.N / (HALF ? 8 : 16 * RT), batch), dim3(NW * 64), lds, st, a);
@@ -360,11 +357,7 @@ namespace llamql
             // 1 x 2048 x 8192 normed takes 7.8 and 9.8, unnormed 6.2 and 6.8.)
             const long tiles = (long)a.N / 16 * batch;
             const bool half = a.M <= 8 && tiles <= cus / 2 && ((sizeof(T) == 4 && !NORM) || a.K > 2048);
-            if (half)
-                return small_launch<T, NW, 1, NORM, true>(fn, a, batch, st);
-            if (sizeof(T) == 4 && !NORM && a.K <= 8 * NW * 32) // one round of eight steps
-                return small_launch<T, NW, 1, NORM, false, false>(fn, a, batch, st);
-            return small_launch<T, NW, 1, NORM>(fn, a, batch, st);
+            return half ? small_launch<T, NW, 1, NORM, true>(fn, a, batch, st) : small_launch<T, NW, 1, NORM>(fn, a, batch, st);
         }
         template <typename T>
         bool small_dispatch(const char *fn, const LinearArgs &a, int batch, int cus, hipStream_t st)
