@@ -162,12 +162,14 @@ namespace llamql
         {
             bf16 *h = reinterpret_cast<bf16 *>(smem);
             const bool record = p.h_out && block == 0;
-            if (p.M == 1)
-                norm_rows<T, NW, 1>(p, h, ldh, record, s_sum);
-            else if (p.M == 2) // (not four, two of them in vain: 2 x 5120 x 2048 in bf16 6.4 -> 5.3 us)
+            // (two rows not as four, two of them in vain: 2 x 5120 x 2048 in bf16 6.4 -> 5.3 us; the way of many rows first in the
+            // code: behind the others it took 1.3 us more where compute units have several workgroups, 4 x 12288 x 512 10.8 and 9.5)
+            if (__builtin_expect(p.M > 2, 1))
+                norm_rows<T, NW, 4>(p, h, ldh, record, s_sum);
+            else if (p.M == 2)
                 norm_rows<T, NW, 2>(p, h, ldh, record, s_sum);
             else
-                norm_rows<T, NW, 4>(p, h, ldh, record, s_sum);
+                norm_rows<T, NW, 1>(p, h, ldh, record, s_sum);
             arow = h + (size_t)(row < p.M ? row : 0) * ldh + 8 * g;
         }
         else
