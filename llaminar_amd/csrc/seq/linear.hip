@@ -33,7 +33,7 @@ namespace llamql
     // fp32 rows normed, into h_out as T (from the first workgroup) and into LDS: as bf16, or, for T fp32, in three bf16
     // pieces that add up to the value (8 + 8 + 8 significant bits, cut off), the pieces
     // p.M * ldh apart.  Three products of bf16 take 48 cycles of the matrix unit a k-step, one of fp32 256 (3 x 32768 x
-    // 2048: 45 -> 36.6 us; the error against 64 bits falls from 3.0e-7 to 2.0e-7).  R rows at a time are asked for and summed,
+    // 2048: 43.4 -> 34.5 us; the error against 64 bits falls from 3.0e-7 to 2.0e-7).  R rows at a time are asked for and summed,
     // and all rows share one barrier: a row at a time, eight rows of 768 values took 6 us of a 9 us launch.
     template <typename T, int NW, int R>
     __device__ __forceinline__ void norm_rows(const LinearArgs &p, bf16 *h, int ldh, bool record, float (&s_sum)[SMALL_M][NW])
@@ -189,8 +189,8 @@ namespace llamql
                 for (int t = 0; t < RT; ++t)
                     cur[t][u] = next[t][u];
             // Rows that come from memory are asked for ahead of the next weights: loads arrive in order, so a product that
-            // waits for a row asked for behind them would wait for all of them (3 x 2048 x 10240 bf16 14.5 -> 11.0 us, fp32
-            // 19.3 -> 14.1; 8 x 5120 x 25600 bf16 75 -> 67 us, fp32 110 -> 86).  Not in a last round with fewer than U steps:
+            // waits for a row asked for behind them would wait for all of them (3 x 2048 x 10240 bf16 11.8 -> 10.3 us, fp32
+            // 18.7 -> 12.8; 8 x 5120 x 25600 bf16 72 -> 67 us, fp32 108 -> 85).  Not in a last round with fewer than U steps:
             // there are no next weights, and rows asked for in vain took as long as the others (16 x 5120 x 1024 in
             // bf16 6.3 -> 4.6).
             constexpr bool AHEAD = !NORM && (sizeof(T) == 2 || RT == 1); // (two tiles of fp32 rows: registers of a second workgroup)

@@ -9,7 +9,7 @@
 // holds under this load; without any loads of A and W the same loop takes 260 instead of 285 us, LDS conflicts are none.
 // Time before (128 x 128 tiles staged through registers) and now: 390 -> 285 us (830 -> 1140 TFLOP/s), 2048 x 51200 x
 // 5120 1200 -> 940 us, 300 x 2048 x 8192 63 -> 28 us; 32-bit rows (v_mfma_f32_16x16x4 before) 2048 x 51200 x 5120 9490 ->
-// 2610 us, 522 x 2048 x 10240 380 -> 126 us.
+// 2480 us, 522 x 2048 x 10240 380 -> 126 us.
 #include "linear.h"
 
 namespace llamql

@@ -263,7 +263,7 @@ namespace llamql
         f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
         constexpr int U = 8;
         // the wavefront's place in the list: step s is step `in` of expert `job` (scalars: as vector code, with the experts in LDS,
-        // eighty instructions and a wait stood between two loads; a layer of 8 fp32 rows, 6 of 64 experts: 161 -> 153 us)
+        // eighty instructions and a wait stood between two loads; a layer of 8 fp32 rows, 6 of 64 experts: 149 -> 141 us)
         int job = 0, in = wave;
         for (int s0 = wave; s0 < total; s0 += EXPERT_WAVES * U)
         {
