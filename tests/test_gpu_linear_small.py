@@ -11,11 +11,12 @@ pytestmark = pytest.mark.gpu
 F32, BF16 = sq.F32, sq.BF16
 
 # half tiles: one to eight rows, one tile, the most tiles (128), K of one step, of fewer steps than wavefronts, of an odd
-# number of steps a wavefront; whole tiles on the other side: nine rows, 65 tiles and K of 4096, 129 and 256 tiles, K of
-# 2048 (bf16); walks of half a round of steps, of one round and of one and a part
+# number of steps a wavefront, 65 tiles and K of 4096; whole tiles on the other side: nine rows, 129 and 256 tiles, K of
+# 2048 (bf16); walks of half a round of steps, of one round and of one and a part, four wavefronts with rounds of 4, 5, 7
+# and 8 steps
 SHAPES = [(1, 16, 64), (8, 16, 4096), (8, 2048, 128), (7, 2064, 1088), (3, 2048, 10304), (8, 4080, 4160), (9, 2048, 4096),
           (8, 4096, 4096), (5, 4096, 4032), (6, 1040, 4096), (8, 2048, 5120), (4, 1024, 2112), (8, 48, 2048), (16, 48, 8256), (12, 4112, 1024), (16, 80, 2048),
-          (9, 48, 2112)]
+          (9, 48, 2112), (9, 48, 960), (12, 2064, 576)]
 
 
 # a fused norm takes up to 8192 values: all of them in one row and in sixteen, half and whole tiles
