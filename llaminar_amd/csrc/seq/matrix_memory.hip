@@ -42,6 +42,10 @@ namespace llamql
         int splits;     // decoding: workgroups along dim
         void *qk;       // T [2][heads][rows of the portion][dim]: scaled q, then k
         int qk_rows;
+        // long portions: stretches of `stretch` chunks (0: the portion is one), what each adds to the memory and keeps of it
+        int stretch;
+        float *starts; // [stretches][heads][dim][vdim + 16]: the memory before the portion, then what stretch 0 .. adds
+        float *kept;   // [stretches][heads]: what is left of the memory after stretch 0 ..
     };
 
     __device__ __forceinline__ void memory_gates(const MemoryArgs &p, const float *row, int h, float &i, float &f)
@@ -265,7 +269,14 @@ namespace llamql
     // dim is 16 DT exactly, so that no product hangs on a condition.
     // What the next chunk needs from memory (q and k for the LDS, this column's values, the products) is
     // requested before the matrix work of the current one.
-    template <typename T, int LC, int DT, bool FULL>
+    // The walk is a chain, 6 to 7 us a chunk of 64 tokens, and 36 workgroups (4 heads of 256 x 512) leave most of the chip idle.
+    // A long portion is therefore cut into stretches that run side by side (blockIdx.z): the recurrence is linear in S, so a first
+    // launch (SUM) walks each stretch from an empty memory without outputs and leaves what the stretch adds, and the walk
+    // proper starts each stretch from the sum of what those before it added, each scaled by what the ones between keep.
+    // 2048 tokens, 4 heads of 256 x 512: 232 -> 80 us for both launches, seven stretches of five chunks.  Stretches of fewer than
+    // three chunks gain nothing: a chunk without outputs takes half the time of one with them, and is walked twice.
+    // (CUT: portions may be cut.  Of more than 256 rows of S it would take more registers than there are.)
+    template <typename T, int LC, int DT, bool FULL, bool CUT, bool SUM>
     __global__ void __launch_bounds__(256)
         memory_chunk_kernel(MemoryArgs p)
     {
@@ -293,15 +304,63 @@ namespace llamql
         f32x4 S[DT];
         float *state = p.state + ((size_t)slot * p.heads + h) * dim * ldv + (live ? col : 0);
         const bool fresh = p.pos[e] == 0;
+        auto load_state = [&](const float *from) {
+#pragma unroll
+            for (int t = 0; t < DT; ++t)
+                if (t < dtiles)
+                {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        S[t][r] = from[(size_t)(16 * t + 4 * g + r) * ldv];
+                }
+        };
+        auto store_state = [&](float *to) {
+#pragma unroll
+            for (int t = 0; t < DT; ++t)
+                if (t < dtiles)
+                {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        to[(size_t)(16 * t + 4 * g + r) * ldv] = S[t][r];
+                }
+        };
+        const int part = CUT ? blockIdx.z : 0, first = CUT ? part * p.stretch * LC : 0; // this stretch and its first token
+        const bool last = !CUT || part + 1 == (int)gridDim.z;
+        const int stop = last || first + p.stretch * LC > ntok ? ntok : first + p.stretch * LC;
+        const size_t part_floats = (size_t)p.heads * dim * ldv;
+        float *starts = p.starts + (size_t)h * dim * ldv + (live ? col : 0);
 #pragma unroll
         for (int t = 0; t < DT; ++t)
-        {
             S[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-            if (t < dtiles && !fresh && live)
+        if (SUM)
+        {
+            if (last)
             {
+                // the last stretch adds to nobody's start: here the memory before the portion is put aside
+                if (!fresh && live)
+                {
+                    load_state(state);
+                    store_state(starts);
+                }
+                return;
+            }
+        }
+        else if (live)
+        {
+            if (!fresh)
+                load_state(CUT && p.stretch ? starts : state);
+            for (int i = 1; CUT && i <= part; ++i)
+            {
+                const float kept = p.kept[(i - 1) * p.heads + h];
+                const float *add = starts + i * part_floats;
 #pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    S[t][r] = state[(size_t)(16 * t + 4 * g + r) * ldv];
+                for (int t = 0; t < DT; ++t)
+                    if (t < dtiles)
+                    {
+#pragma unroll
+                        for (int r = 0; r < 4; ++r)
+                            S[t][r] = fmaf(S[t][r], kept, add[(size_t)(16 * t + 4 * g + r) * ldv]);
+                    }
             }
         }
 
@@ -324,7 +383,8 @@ namespace llamql
                 for (int i = 0; i < LOADS; ++i)
                 {
                     const int at = sseg + i * TPR < pieces ? i * TPR : 0;
-                    hq[i] = q[at];
+                    if (!SUM)
+                        hq[i] = q[at];
                     hk[i] = k[at];
                 }
             }
@@ -345,14 +405,17 @@ namespace llamql
                                              : p.proj[(size_t)(r0 + (tt < n ? tt : n - 1)) * p.ldp + (size_t)p.heads * 2 * dim + h * p.vdim + col];
                 }
         };
-        request(0);
-        float m0 = p.m0[h];
-        for (int t0 = 0; t0 < ntok; t0 += LC)
+        if (first < ntok)
+            request(first);
+        float m0 = first == 0 ? p.m0[h] : first < ntok ? p.mt[(size_t)(row0 + first - 1) * p.heads + h] : 0.0f;
+        float kept = 1.0f;
+        for (int t0 = first; t0 < stop; t0 += LC)
         {
             const int n = ntok - t0 < LC ? ntok - t0 : LC;
             const int r0 = row0 + t0;
             const float decay = expf((float)(h_end + (double)m0));
             const float m_end = h_mt;
+            kept *= decay;
             __syncthreads();
             if (threadIdx.x < LC)
             {
@@ -368,7 +431,8 @@ namespace llamql
                     for (int i = 0; i < LOADS; ++i)
                         if (sseg + i * TPR < pieces)
                         {
-                            dq[i * TPR] = hq[i];
+                            if (!SUM)
+                                dq[i * TPR] = hq[i];
                             dk[i * TPR] = hk[i];
                         }
                 }
@@ -379,7 +443,8 @@ namespace llamql
 #pragma unroll 4
                     for (int i = 0; sseg + i < pieces; i += TPR)
                     {
-                        dq[i] = q[i];
+                        if (!SUM)
+                            dq[i] = q[i];
                         dk[i] = k[i];
                     }
                 }
@@ -396,9 +461,9 @@ namespace llamql
             for (int i = 0; i < LC / 16; ++i)
 #pragma unroll
                 for (int s = 0; s < LC / 32; ++s)
-                    if (32 * s <= 16 * i + 15)
+                    if (!SUM && 32 * s <= 16 * i + 15)
                         w[i][s] = Operand<float>::load(prod + (16 * i + c) * LC + 32 * s + 8 * g);
-            if (t0 + LC < ntok)
+            if (t0 + LC < stop)
                 request(t0 + LC);
             if (live)
             {
@@ -422,59 +487,62 @@ namespace llamql
                         y[j] = (float)one[0][j] * s_gate[32 * s + 8 * g + j];
                     split_pieces<T, NP>(y, gv[s]);
                 }
-                // carried part: q . S
-                f32x4 out[LC / 16];
-#pragma unroll
-                for (int i = 0; i < LC / 16; ++i)
-                    out[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-                for (int t = 0; t < DT; t += 2)
-                    if (t < dtiles)
-                    {
-                        V b[NP], a[LC / 16];
-                        split_pieces<T, NP>(__builtin_shufflevector(S[t], S[t + 1], 0, 1, 2, 3, 4, 5, 6, 7), b);
-#pragma unroll
-                        for (int i = 0; i < LC / 16; ++i)
-                        {
-                            const T *qr = sq + (16 * i + c) * ld + 16 * t + 4 * g;
-                            const t4 lo = *reinterpret_cast<const t4 *>(qr), hi = *reinterpret_cast<const t4 *>(qr + 16);
-                            a[i] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-                        }
-#pragma unroll
-                        for (int k = 0; k < NP; ++k)
-#pragma unroll
-                            for (int i = 0; i < LC / 16; ++i)
-                                out[i] = O::mma(a[i], b[k], out[i]);
-                    }
-                // plus the chunk's own tokens
-#pragma unroll
-                for (int i = 0; i < LC / 16; ++i)
+                if constexpr (!SUM)
                 {
-#pragma unroll
-                    for (int r = 0; r < 4; ++r)
-                        out[i][r] *= s_carry[16 * i + 4 * g + r];
-                }
-#pragma unroll
-                for (int s = 0; s < LC / 32; ++s)
+                    // carried part: q . S
+                    f32x4 out[LC / 16];
 #pragma unroll
                     for (int i = 0; i < LC / 16; ++i)
-                        if (32 * s <= 16 * i + 15)
+                        out[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                    for (int t = 0; t < DT; t += 2)
+                        if (t < dtiles)
                         {
-                            V q[NP];
-                            split_pieces<T, NP>(w[i][s], q);
+                            V b[NP], a[LC / 16];
+                            split_pieces<T, NP>(__builtin_shufflevector(S[t], S[t + 1], 0, 1, 2, 3, 4, 5, 6, 7), b);
+#pragma unroll
+                            for (int i = 0; i < LC / 16; ++i)
+                            {
+                                const T *qr = sq + (16 * i + c) * ld + 16 * t + 4 * g;
+                                const t4 lo = *reinterpret_cast<const t4 *>(qr), hi = *reinterpret_cast<const t4 *>(qr + 16);
+                                a[i] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+                            }
 #pragma unroll
                             for (int k = 0; k < NP; ++k)
-                                out[i] = O::mma(q[k], v[s], out[i]);
+#pragma unroll
+                                for (int i = 0; i < LC / 16; ++i)
+                                    out[i] = O::mma(a[i], b[k], out[i]);
                         }
+                    // plus the chunk's own tokens
 #pragma unroll
-                for (int i = 0; i < LC / 16; ++i)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r)
+                    for (int i = 0; i < LC / 16; ++i)
                     {
-                        const int t = 16 * i + 4 * g + r;
-                        if (t < n)
-                            p.num[((size_t)(r0 + t) * p.heads + h) * ldv + col] = out[i][r];
+#pragma unroll
+                        for (int r = 0; r < 4; ++r)
+                            out[i][r] *= s_carry[16 * i + 4 * g + r];
                     }
+#pragma unroll
+                    for (int s = 0; s < LC / 32; ++s)
+#pragma unroll
+                        for (int i = 0; i < LC / 16; ++i)
+                            if (32 * s <= 16 * i + 15)
+                            {
+                                V q[NP];
+                                split_pieces<T, NP>(w[i][s], q);
+#pragma unroll
+                                for (int k = 0; k < NP; ++k)
+                                    out[i] = O::mma(q[k], v[s], out[i]);
+                            }
+#pragma unroll
+                    for (int i = 0; i < LC / 16; ++i)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r)
+                        {
+                            const int t = 16 * i + 4 * g + r;
+                            if (t < n)
+                                p.num[((size_t)(r0 + t) * p.heads + h) * ldv + col] = out[i][r];
+                        }
+                }
                 // S of the next chunk
 #pragma unroll
                 for (int t = 0; t < DT; ++t)
@@ -505,17 +573,15 @@ namespace llamql
             }
             m0 = m_end;
         }
-        if (live)
+        if (SUM)
         {
-#pragma unroll
-            for (int t = 0; t < DT; ++t)
-                if (t < dtiles)
-                {
-#pragma unroll
-                    for (int r = 0; r < 4; ++r)
-                        state[(size_t)(16 * t + 4 * g + r) * ldv] = S[t][r];
-                }
+            if (live)
+                store_state(starts + (part + 1) * part_floats);
+            if (blockIdx.x == 0 && threadIdx.x == 0)
+                p.kept[part * p.heads + h] = kept;
         }
+        else if (live && last)
+            store_state(state);
     }
 
     // ---- output: normaliser, head norm, gate ------------------------------------------------------------
@@ -582,12 +648,22 @@ namespace llamql
     namespace
     {
         constexpr int LC16 = 64, LC32 = 32; // chunk lengths of the two number formats
+        constexpr int CUT_TILES = 16;                    // 16-row tiles of S up to which a portion is cut into stretches
+        constexpr int STRETCHES = 8, STRETCH_MIN = 3; // stretches of a portion at most, chunks of one at least
         constexpr int STEP_SPLIT_ENTRIES = 32; // sequences up to which a decoding step splits the rows of S (in at most 8)
 
         struct MemoryScratch
         {
-            size_t ga, a, mt, m0, prod, num, qk, total;
+            size_t ga, a, mt, m0, prod, num, qk, starts, kept, total;
         };
+        // Stretches of a portion that are walked side by side (1: the walk is one).
+        int memory_stretches(int ntok, int dim, int lc)
+        {
+            if (dim > 16 * CUT_TILES)
+                return 1;
+            const int chunks = ceil_div(ntok, lc), n = chunks / STRETCH_MIN;
+            return n < 2 ? 1 : n < STRETCHES ? n : STRETCHES;
+        }
         MemoryScratch memory_scratch(int rows, int heads, int dim, int vdim)
         {
             MemoryScratch s{};
@@ -605,6 +681,9 @@ namespace llamql
             const size_t outs = (size_t)(rows > STEP_SPLIT_ENTRIES * 8 ? rows : STEP_SPLIT_ENTRIES * 8);
             s.num = take(outs * heads * (vdim + 16) * 4);
             s.qk = take((size_t)2 * heads * round_up(rows, LC16) * dim * 4);
+            const int stretches = memory_stretches(rows, dim, LC32); // (the shorter chunks: the most that any portion has)
+            s.starts = take(stretches > 1 ? (size_t)stretches * heads * dim * (vdim + 16) * 4 : 0);
+            s.kept = take((size_t)stretches * heads * 4);
             s.total = at;
             return s;
         }
@@ -646,39 +725,54 @@ namespace llamql
             p.mt = reinterpret_cast<float *>(s + at.mt), p.m0 = reinterpret_cast<float *>(s + at.m0);
             p.prod = reinterpret_cast<float *>(s + at.prod), p.num = reinterpret_cast<float *>(s + at.num);
             p.qk = s + at.qk, p.qk_rows = rows;
+            p.starts = reinterpret_cast<float *>(s + at.starts), p.kept = reinterpret_cast<float *>(s + at.kept);
         }
 
-        template <typename T, int LC, int DT, bool FULL>
-        bool chunk_launch_as(const char *fn, const MemoryArgs &p, hipStream_t st)
+        template <typename T, int LC, int DT, bool FULL, bool CUT, bool SUM>
+        bool chunk_launch_one(const char *fn, const MemoryArgs &p, int stretches, hipStream_t st)
         {
             static LdsGrant grant;
             const size_t lds = (size_t)2 * LC * (p.dim + 16 / sizeof(T)) * sizeof(T);
-            if (lds > 48 * 1024 && allow_lds(grant, reinterpret_cast<const void *>(&memory_chunk_kernel<T, LC, DT, FULL>), 140 * 1024) != hipSuccess)
+            const auto kernel = &memory_chunk_kernel<T, LC, DT, FULL, CUT, SUM>;
+            if (lds > 48 * 1024 && allow_lds(grant, reinterpret_cast<const void *>(kernel), 140 * 1024) != hipSuccess)
                 return fail(fn, "cannot reserve %zu bytes of LDS", lds);
-            hipLaunchKernelGGL((memory_chunk_kernel<T, LC, DT, FULL>), dim3(ceil_div(p.vdim + 16, 64), p.heads), dim3(256), lds, st, p);
+            hipLaunchKernelGGL(kernel, dim3(ceil_div(p.vdim + 16, 64), p.heads, stretches), dim3(256), lds, st, p);
             return launched(fn);
         }
+        template <typename T, int LC, int DT, bool FULL>
+        bool chunk_launch_as(const char *fn, const MemoryArgs &p, int stretches, hipStream_t st)
+        {
+            if constexpr (DT <= CUT_TILES)
+                return (stretches == 1 || chunk_launch_one<T, LC, DT, FULL, true, true>(fn, p, stretches, st)) &&
+                       chunk_launch_one<T, LC, DT, FULL, true, false>(fn, p, stretches, st);
+            else
+                return chunk_launch_one<T, LC, DT, FULL, false, false>(fn, p, 1, st);
+        }
         template <typename T, int LC, int DT>
-        bool chunk_launch(const char *fn, const MemoryArgs &p, hipStream_t st)
+        bool chunk_launch(const char *fn, const MemoryArgs &p, int stretches, hipStream_t st)
         {
             if constexpr (sizeof(T) == 2)
             {
                 if (p.dim == 16 * DT)
-                    return chunk_launch_as<T, LC, DT, true>(fn, p, st);
+                    return chunk_launch_as<T, LC, DT, true>(fn, p, stretches, st);
             }
-            return chunk_launch_as<T, LC, DT, false>(fn, p, st);
+            return chunk_launch_as<T, LC, DT, false>(fn, p, stretches, st);
         }
         template <typename T, int LC>
-        bool prefill_run(const char *fn, const MemoryArgs &p, int ntok, hipStream_t st)
+        bool prefill_run(const char *fn, MemoryArgs p, int ntok, int cus, hipStream_t st)
         {
+            // (a workgroup fills a compute unit: no second round of them)
+            const int most = cus / (ceil_div(p.vdim + 16, 64) * p.heads), can = memory_stretches(ntok, p.dim, LC);
+            const int stretches = most < 2 ? 1 : can < most ? can : most;
+            p.stretch = stretches > 1 ? ceil_div(ceil_div(ntok, LC), stretches) : 0;
             hipLaunchKernelGGL(memory_gates_kernel<LC>, dim3(p.heads), dim3(GATE_WAVES * 64), 0, st, p);
             if (!launched(fn))
                 return false;
             hipLaunchKernelGGL((memory_product_kernel<T, LC>), dim3(ceil_div(ntok, LC), p.heads), dim3(LC * 4), 0, st, p);
             if (!launched(fn))
                 return false;
-            const bool ok = p.dim <= 64 ? chunk_launch<T, LC, 4>(fn, p, st) : p.dim <= 128 ? chunk_launch<T, LC, 8>(fn, p, st)
-                            : p.dim <= 256 ? chunk_launch<T, LC, 16>(fn, p, st) : chunk_launch<T, LC, 32>(fn, p, st);
+            const bool ok = p.dim <= 64 ? chunk_launch<T, LC, 4>(fn, p, stretches, st) : p.dim <= 128 ? chunk_launch<T, LC, 8>(fn, p, stretches, st)
+                            : p.dim <= 256 ? chunk_launch<T, LC, 16>(fn, p, stretches, st) : chunk_launch<T, LC, 32>(fn, p, stretches, st);
             if (!ok)
                 return false;
             hipLaunchKernelGGL((memory_output_kernel<T, false>), dim3(p.heads, ntok), dim3(128), 0, st, p);
@@ -743,6 +837,6 @@ extern "C" bool llam_seq_memory_prefill(const llam_seq_memory_args *a, const lla
     place_scratch(p, d_scratch, scratch_bytes);
     if (!set_device(fn, device_id))
         return false;
-    return dtype == LLAM_SEQ_F32 ? prefill_run<float, LC32>(fn, p, ntok, as_stream(stream))
-                                 : prefill_run<bf16, LC16>(fn, p, ntok, as_stream(stream));
+    return dtype == LLAM_SEQ_F32 ? prefill_run<float, LC32>(fn, p, ntok, cu_count(device_id), as_stream(stream))
+                                 : prefill_run<bf16, LC16>(fn, p, ntok, cu_count(device_id), as_stream(stream));
 }

@@ -229,6 +229,24 @@ def test_memory_keeps_an_early_token_for_long():
     model.close()
 
 
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("heads,dim,vdim", [(2, 40, 24), (1, 128, 200), (1, 200, 64), (66, 16, 16), (1, 300, 24)],
+                         ids=["64 rows", "128 rows", "256 rows", "no room for eight", "too many rows"])
+def test_a_long_portion_is_walked_in_stretches(heads, dim, vdim, dtype):
+    """Portions from one token short of the first that is cut to one with more chunks than eight stretches of three, ends
+    within a chunk and a stretch, from an empty memory and onto one; what they leave behind, read by the next tokens."""
+    cfg = sm.config(sm.mlstm(heads=heads, dim=dim, vdim=vdim), width=64)
+    t = sm.random_weights(cfg, 5, forget_bias=3.0)
+    chunk = 32 if dtype == "float32" else 64
+    tokens = tokens_of(cfg, 26 * chunk + 20)
+    want = so.kogilix(cfg, t.plain(), tokens)
+    model = load(cfg, t, dtype, cap=len(tokens), max_rows=len(tokens))
+    for n in (5 * chunk, 5 * chunk + 1, 7 * chunk + 9, 9 * chunk, 25 * chunk + 7):
+        check(run(model, 0, tokens, [n, 1, 9]), want[:n + 10], dtype, note=f"{n} tokens at once")
+        check(run(model, 1, tokens, [3, n, 7]), want[:n + 10], dtype, note=f"{n} tokens at position 3")
+    model.close()
+
+
 def test_generation_through_the_scheduler(whole, whole_f32):
     """More requests than slots, portions mixed with decoding, bursts on the device: the tokens of a plain loop."""
     t, _, _ = whole
