@@ -419,41 +419,63 @@ namespace llamql
     }
 
     // ---- activations as they lie, a tile's K steps dealt to the wavefronts ------------------------
-    // Tile of 32 MT tokens x 32 RN weight rows, KS x RN wavefronts: wavefront (rn, ks) multiplies super-blocks ks, ks + KS,
-    // .. of rows 32 rn .. by all tokens of the tile, and the KS partial sums are added through LDS in their order.  The
-    // weights never pass through LDS: lane (r, h) decodes what quad lanes h and h + 2 of row r decode, four whole blocks of
-    // a super-block, and a swap of half registers between the lanes (r, 0) and (r, 1) makes both lanes' blocks into
-    // matrix operands.  The Q8_1 blocks of KS super-blocks of the tokens go from memory into LDS, a step ahead, two buffers,
-    // one barrier a step: the quants as 16-byte pieces, [super-block][token][16], piece p of token m at p ^ (m & 15) (so that
-    // reads of 16 tokens' pieces meet no bank twice), the heads {d, sum} as [super-block][block][token].
-    // Bound by the vector unit: a conversion and a multiply-add per product of a block, and the decoding, which 64 tokens
-    // share; one workgroup of eight wavefronts fits a compute unit (up to 210 registers a lane; 128, for two of them, spill).
-    // 130 tokens x 5000 rows of 5120, Q4_K 54 -> 33 us, Q6_K 60 -> 38; 40 x 8192 x 5120 of IQ3_S 39.6 -> 23.0.
+    // Tile of 32 MT tokens x 32 RN weight rows, a step of KS super-blocks, 2 KS RN = 8 wavefronts: wavefront (rn, kw) multiplies
+    // half a super-block, the blocks of quad lanes 2 (kw % 2) and 2 (kw % 2) + 1, of rows 32 rn .. by all tokens of the tile, and
+    // the 2 KS partial sums are added through LDS in their order.  The weights never pass through LDS: lane (r, h) decodes
+    // what quad lane h of the half decodes, two whole blocks, and a swap of half registers between the lanes (r, 0) and (r, 1)
+    // makes both lanes' blocks into matrix operands.  The Q8_1 blocks of the tokens go from memory into LDS a step ahead, two
+    // buffers, one barrier a step: the quants as 16-byte pieces, [super-block][token][16], piece p of token m at p ^ (m & 15)
+    // (so that reads of 16 tokens' pieces meet no bank twice), the heads {d, sum} as [super-block][8 tokens][block][8], block k
+    // of the group of tokens g at k ^ (g & 7): a load of 64 heads reads 8 tokens' whole super-blocks, 24 cache lines, where a
+    // block of 64 tokens would read 64.
+    // What bounds it: the address unit of the loads (5000 of 11000 cycles a step when every lane's head was a line of its own and
+    // all loads were issued together, the wavefronts standing still meanwhile), then the vector unit: rescaling and decoding.  So
+    // the loads are dealt out among the products, a wavefront takes half a super-block of twice the tokens (half the decoding and
+    // half the loads of weights a product), and the matrix unit works on a product while the vector unit rescales the one before.
+    // One workgroup of eight wavefronts fits a compute unit (up to 250 registers a lane).
+    // Against whole super-blocks a wavefront and loads together: 199 x 5120 x 25600 Q6_K 272 -> 207 us, 40 x 8192 x 5120 IQ3_S
+    // 23.3 -> 19.0, 256 x 8192 x 8192 Q4_K 79 -> 65, 63 x 5034 x 18944 Q6_K 93 -> 70.5, 130 x 5000 x 5120 Q4_K 29.2 -> 26.7.
     // The sums are kept in 2 to 8 parts: their error against 64 bits is 0.5 to 0.9 times gemm_kernel's.
     template <int MT, int RN, int KS>
     struct GemmSplit
     {
-        static constexpr int BM = MT * 32, WAVES = RN * KS;
+        static constexpr int BM = MT * 32, KW = 2 * KS, WAVES = RN * KW; // wavefronts along K, and of a workgroup
         static constexpr int QUANTS = KS * BM * 256, HEADS = KS * BM * 32; // bytes of a step
         static constexpr int QLOADS = QUANTS / 1024 / WAVES, HLOADS = HEADS / 256 / WAVES; // per wavefront
         static constexpr int QROWS = 4 * WAVES;                  // tokens x super-blocks that one load of every wavefront covers
         static constexpr int QM = BM > QROWS ? BM / QROWS : 1;   // tokens a lane loads pieces of
-        static constexpr int HSB = WAVES * 8 / BM;               // super-blocks that one load of every wavefront covers (heads)
+        static constexpr int HM = BM > 8 * WAVES ? BM / (8 * WAVES) : 1; // tokens a lane loads heads of
         static_assert(QLOADS * WAVES * 1024 == QUANTS && HLOADS * WAVES * 256 == HEADS, "whole loads");
         static_assert(QROWS % 16 == 0 && (BM % QROWS == 0 || QROWS % BM == 0), "a lane's piece and tokens stay the same");
-        static_assert(HSB >= 1 && HSB * BM == WAVES * 8, "a lane's block and token stay the same");
+        static_assert(BM % (8 * WAVES) == 0 || 8 * WAVES % BM == 0, "a lane's tokens stay the same");
         static constexpr size_t STAGE = QUANTS + HEADS;
-        static constexpr size_t SUMS = (size_t)(KS - 1) * RN * MT * 16 * WAVE * sizeof(float);
+        static constexpr size_t SUMS = (size_t)(KW - 1) * RN * MT * 16 * WAVE * sizeof(float);
         static constexpr size_t LDS = 2 * STAGE > SUMS ? 2 * STAGE : SUMS;
     };
 
+    // Block sums as floats without a conversion: the products start from the bits of 1.5 * 2^23 instead of zero, so that the bits of
+    // their integer result are those of the float 1.5 * 2^23 + sum (sums stay within 32 * 128 * 128 = 2^19, a unit of the last
+    // place is 1), and one subtraction leaves the sum, exactly.  Conversions and matrix instructions hold each other up: two
+    // products with their rescaling take 308 cycles instead of 409, two wavefronts a SIMD unit.
+    constexpr float BIAS = 12582912.0f;
+    __device__ __forceinline__ v16i integer_bias()
+    {
+        v16i b;
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+            b[r] = __builtin_bit_cast(int, BIAS);
+        asm volatile("" : "+v"(b)); // kept in registers: made anew for every product it would cost what it saves
+        return b;
+    }
+    __device__ __forceinline__ float biased_to_float(int sum) { return __builtin_bit_cast(float, sum) - BIAS; }
+
     template <class F, int MT, int RN, int KS, bool DUMP>
-    __global__ void __launch_bounds__(RN *KS *WAVE) gemm_split_kernel(const GemmArgs g)
+    __global__ void __launch_bounds__(RN * 2 * KS * WAVE) gemm_split_kernel(const GemmArgs g)
     {
         typedef typename F::Quad Q;
         typedef GemmSplit<MT, RN, KS> G;
         typedef int v2i_dword __attribute__((ext_vector_type(2), aligned(4)));
-        constexpr int BM = G::BM;
+        constexpr int BM = G::BM, KW = G::KW;
         extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
         void *tab = format_tables_lds<F>();
         if (F::TABLE_BYTES > 0)
@@ -461,7 +483,8 @@ namespace llamql
 
         const int tid = threadIdx.x, lane = tid & 63;
         const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-        const int rn = wave % RN, ks = wave / RN;
+        const int rn = wave % RN, kw = wave / RN;
+        const int own_sb = kw >> 1, half = kw & 1; // of a step; of the super-block
         const int l32 = lane & 31, lh = lane >> 5;
         const long n0 = ((long)blockIdx.x * RN + rn) * 32 + (long)g.tile0 * GEMM_BN, m0 = (long)blockIdx.y * BM;
         const int SB = g.w.SB, KB = SB * 8;
@@ -469,173 +492,202 @@ namespace llamql
         long n = n0 + l32;
         if (n >= g.w.N)
             n = g.w.N - 1; // tail rows: decode a valid row, never stored
-        const typename Q::Lane lane_of[2] = {Q::lane_consts(lh), Q::lane_consts(lh + 2)};
-        const typename Q::Cursor wc = Q::cursor(g.w, (size_t)n * SB, (size_t)n * SB, lane_of[0]);
-        typename Q::Raw raw[2];
-        auto issue_weights = [&](int sb) { // (past the end: the last super-block again)
-            const int at = sb < SB ? sb : SB - 1;
-            Q::load_at(raw[0], wc, lane_of[0], at);
-            Q::load_at(raw[1], wc, lane_of[1], at);
-        };
+        const typename Q::Lane lc = Q::lane_consts(lh + 2 * half);
+        const typename Q::Cursor wc = Q::cursor(g.w, (size_t)n * SB, (size_t)n * SB, lc);
+        typename Q::Raw raw;
+        auto issue_weights = [&](int sb) { Q::load_at(raw, wc, lc, sb < SB ? sb : SB - 1); }; // (past the end: the last super-block again)
         // bytes from the tile's first token to what this lane loads of super-block 0 (past the last token: the last one)
         const uint8_t *abase = reinterpret_cast<const uint8_t *>(g.q8 + (size_t)m0 * KB * 9);
         auto token = [&](int m) { return (uint32_t)(m0 + m < g.M ? m : g.M - 1 - m0) * (uint32_t)(KB * 36); };
-        uint32_t qfrom[G::QM], hfrom;
+        uint32_t qfrom[G::QM], hfrom[G::HM];
         {
             const int row = wave * 4 + (lane >> 4), p = (lane & 15) ^ (row & 15);
 #pragma unroll
             for (int i = 0; i < G::QM; ++i)
                 qfrom[i] = token((row + i * G::QROWS) % BM) + (uint32_t)((p >> 1) * 36 + 4 + (p & 1) * 16);
-            const int idx = wave * 64 + lane;
-            hfrom = token(idx % BM) + (uint32_t)((idx / BM) & 7) * 36;
+#pragma unroll
+            for (int i = 0; i < G::HM; ++i)
+            {
+                const int group = (wave + i * G::WAVES) % (BM / 8);
+                hfrom[i] = token(group * 8 + (lane & 7)) + (uint32_t)((lane >> 3) ^ (group & 7)) * 36;
+            }
         }
         const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)smem;
         auto super_block = [&](int sb) { return abase + (size_t)(sb < SB ? sb : SB - 1) * 288; }; // (past the end: the last one)
-        auto issue_acts = [&](int sb0, int buf) {
-            const uint32_t to = lds0 + (uint32_t)(buf * (int)G::STAGE + wave * 1024);
-#pragma unroll
-            for (int i = 0; i < G::QLOADS; ++i)
-                asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to + (uint32_t)(i * G::WAVES * 1024)),
-                             "v"(qfrom[i % G::QM]), "s"(super_block(sb0 + (wave * 4 + i * G::QROWS) / BM))
-                             : "memory");
-            const uint32_t toh = lds0 + (uint32_t)(buf * (int)G::STAGE + G::QUANTS + wave * 256);
-#pragma unroll
-            for (int i = 0; i < G::HLOADS; ++i)
-                asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(toh + (uint32_t)(i * G::WAVES * 256)),
-                             "v"(hfrom), "s"(super_block(sb0 + (wave * 64 / BM + i * (G::WAVES * 64 / BM)) / 8))
-                             : "memory");
+        // Load i of the step of super-block sb0, where there is one: else no lane takes part (a branch among the products would
+        // have the compiler copy their registers at its ends).
+        constexpr int LOADS = G::QLOADS + G::HLOADS;
+        auto issue_act = [&](int i, int sb0, int buf) {
+            uint64_t all;
+            if (i < G::QLOADS)
+                asm volatile("s_mov_b32 m0, %1\n\ts_mov_b64 %0, exec\n\ts_cmp_lt_i32 %4, %5\n\ts_cselect_b64 exec, -1, 0\n\tglobal_load_lds_dwordx4 %2, %3\n\ts_mov_b64 exec, %0"
+                             : "=&s"(all)
+                             : "s"(lds0 + (uint32_t)(buf * (int)G::STAGE + wave * 1024 + i * G::WAVES * 1024)), "v"(qfrom[i % G::QM]),
+                               "s"(super_block(sb0 + (wave * 4 + i * G::QROWS) / BM)), "s"(sb0), "s"(SB)
+                             : "memory", "scc");
+            else
+            {
+                const int h = i - G::QLOADS;
+                asm volatile("s_mov_b32 m0, %1\n\ts_mov_b64 %0, exec\n\ts_cmp_lt_i32 %4, %5\n\ts_cselect_b64 exec, -1, 0\n\tglobal_load_lds_dword %2, %3\n\ts_mov_b64 exec, %0"
+                             : "=&s"(all)
+                             : "s"(lds0 + (uint32_t)(buf * (int)G::STAGE + G::QUANTS + wave * 256 + h * G::WAVES * 256)), "v"(hfrom[h % G::HM]),
+                               "s"(super_block(sb0 + (wave + h * G::WAVES) / (BM / 8))), "s"(sb0), "s"(SB)
+                             : "memory", "scc");
+            }
         };
+        const v16i bias = integer_bias();
         v16f acc[MT];
 #pragma unroll
         for (int t = 0; t < MT; ++t)
 #pragma unroll
             for (int r = 0; r < 16; ++r)
                 acc[t][r] = 0.0f;
-        v16i zero;
         v32f zero2f;
-#pragma unroll
-        for (int r = 0; r < 16; ++r)
-            zero[r] = 0;
 #pragma unroll
         for (int r = 0; r < 32; ++r)
             zero2f[r] = 0.0f;
 
-        issue_acts(0, 0);
-        issue_weights(ks);
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i)
+            issue_act(i, 0, 0);
+        issue_weights(own_sb);
         int buf = 0;
         for (int sb0 = 0; sb0 < SB; sb0 += KS, buf ^= 1)
         {
-            const int sb = sb0 + ks;
+            const int sb = sb0 + own_sb;
             // this step's weights and activations have arrived, everybody is done with the other buffer
-            Q::template wait<0>(raw[0]);
-            Q::template wait<0>(raw[1]);
+            Q::template wait<0>(raw);
             asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-            v4i w[2][4];
-            typename Q::Scale S[2];
-#pragma unroll
-            for (int c = 0; c < 2; ++c)
-                Q::decode(raw[c], lane_of[c], w[c], S[c]);
+            v4i w[4];
+            typename Q::Scale S;
+            Q::decode(raw, lc, w, S);
             // decoded here, before the registers are asked for again: sunk below, the decoding would have the compiler copy
             // the raw words, and copies made ahead of the wait hold what the loads have not brought yet
-#pragma unroll
-            for (int c = 0; c < 2; ++c)
-            {
-                v2i_dword two = __builtin_bit_cast(v2i_dword, S[c]);
-                asm volatile("" : "+v"(w[c][0]), "+v"(w[c][1]), "+v"(w[c][2]), "+v"(w[c][3]), "+v"(two));
-                S[c] = __builtin_bit_cast(typename Q::Scale, two);
-            }
+            v2i_dword two = __builtin_bit_cast(v2i_dword, S);
+            asm volatile("" : "+v"(w[0]), "+v"(w[1]), "+v"(w[2]), "+v"(w[3]), "+v"(two));
+            S = __builtin_bit_cast(typename Q::Scale, two);
             __builtin_amdgcn_sched_barrier(0);
-            if (sb0 + KS < SB)
-                issue_acts(sb0 + KS, buf ^ 1);
+            // (the weights at once: they come from memory, and dealt out behind the products they were waited for)
             issue_weights(sb + KS);
             __builtin_amdgcn_sched_barrier(0);
             if (sb < SB) // uniform in the wavefront
             {
-                const uint8_t *rows = smem + buf * G::STAGE + (size_t)(ks * BM + l32) * 256;
-                const uint32_t *heads = reinterpret_cast<const uint32_t *>(smem + buf * G::STAGE + G::QUANTS) + ks * 8 * BM + l32;
+                const uint8_t *rows = smem + buf * G::STAGE + (size_t)(own_sb * BM + l32) * 256;
+                const uint32_t *heads = reinterpret_cast<const uint32_t *>(smem + buf * G::STAGE + G::QUANTS) + own_sb * 8 * BM + (l32 >> 3) * 64 + (l32 & 7);
+                // block x of the half's first quad lane, block y of its second: elements 0 .. 15 with lanes (r, 0), 16 .. 31 with (r, 1)
 #pragma unroll
-                for (int c = 0; c < 2; ++c)
+                for (int i = 0; i < 2; ++i)
 #pragma unroll
-                    for (int i = 0; i < 2; ++i)
+                    for (int d = 0; d < 4; ++d)
                     {
-                        // block x of quad lane 2c, block y of quad lane 2c + 1: elements 0 .. 15 with lanes (r, 0), 16 .. 31 with (r, 1)
-                        v4i x = w[c][2 * i], y = w[c][2 * i + 1];
+                        typedef uint32_t v2u __attribute__((ext_vector_type(2)));
+                        const v2u s = __builtin_bit_cast(v2u, __builtin_amdgcn_permlane32_swap((uint32_t)w[2 * i][d], (uint32_t)w[2 * i + 1][d], false, false));
+                        w[2 * i][d] = (int)s[0], w[2 * i + 1][d] = (int)s[1];
+                    }
+                // Product j: pair of blocks j / MT by tokens 32 (j % MT) ...  The matrix unit works on a product while the vector
+                // unit rescales the one before it, and the LDS brings the operands of the next.
+                constexpr int JOBS = 2 * MT, EACH = (LOADS + JOBS - 1) / JOBS;
+                auto fence = []() __attribute__((always_inline)) {
+                    if (MT > 1) // (two products of a step are not enough for it: the compiler's order is 10 % faster)
+                        __builtin_amdgcn_sched_barrier(0);
+                };
+                auto block = [&](int j, int which) { return Q::block_of(2 * half + which, j / MT); };
+                auto quants = [&](int j, int which) {
+                    return *reinterpret_cast<const v4i *>(rows + (j % MT) * 32 * 256 + (((2 * block(j, which) + lh) ^ (l32 & 15)) << 4));
+                };
+                auto head_of = [&](int j) { return heads[(((lh ? block(j, 1) : block(j, 0)) ^ ((j % MT & 1) * 4 + (l32 >> 3))) * 8) + (j % MT) * 256]; };
+                auto scale_of = [](uint32_t head) { return h2f((uint16_t)(head & 0xFFFFu)); };
+                // the scale products of both blocks, a rank-1 matrix each (exact: both factors are fp16 values)
+                auto scales = [&](int j, uint32_t head) { return __builtin_amdgcn_mfma_f32_32x32x1f32(scale_of(head), Q::scale_f32(S, j / MT), zero2f, 0, 0, 0); };
+                auto product = [&](int j, int which, v4i a) { return __builtin_amdgcn_mfma_i32_32x32x32_i8(a, w[2 * (j / MT) + which], bias, 0, 0, 0); };
+                auto dump = [&](int j, int which, const v16i &d) {
+                    const long nn = n0 + l32 - g.row0;
+                    if (n0 + l32 < g.w.N && nn >= 0 && nn < g.nrows)
+                    {
+                        // (less than 2 GiB of sums: offsets of 32 bits, made anew for each, or they would fill the registers)
+                        const uint32_t token = (uint32_t)g.nrows * (uint32_t)KB;
+                        uint32_t at = ((uint32_t)m0 + 4 * lh) * token + (uint32_t)nn * (uint32_t)KB + (uint32_t)(sb * 8 + block(j, which));
 #pragma unroll
-                        for (int d = 0; d < 4; ++d)
+                        for (int r = 0; r < 16; ++r)
                         {
-                            typedef uint32_t v2u __attribute__((ext_vector_type(2)));
-                            const v2u s = __builtin_bit_cast(v2u, __builtin_amdgcn_permlane32_swap((uint32_t)x[d], (uint32_t)y[d], false, false));
-                            x[d] = (int)s[0], y[d] = (int)s[1];
-                        }
-                        const int kx = Q::block_of(2 * c, i), ky = Q::block_of(2 * c + 1, i);
-                        const float bs = Q::scale_f32(S[c], i);
-#pragma unroll
-                        for (int t = 0; t < MT; ++t)
-                        {
-                            auto quants = [&](int k) {
-                                return *reinterpret_cast<const v4i *>(rows + t * 32 * 256 + (((2 * k + lh) ^ (l32 & 15)) << 4));
-                            };
-                            const uint32_t head = heads[(lh ? ky : kx) * BM + t * 32];
-                            const float ad = h2f((uint16_t)(head & 0xFFFFu));
-                            // the scale products of both blocks, a rank-1 matrix each (exact: both factors are fp16 values)
-                            const v32f cs = __builtin_amdgcn_mfma_f32_32x32x1f32(ad, bs, zero2f, 0, 0, 0);
-                            const v16i dx = __builtin_amdgcn_mfma_i32_32x32x32_i8(quants(kx), x, zero, 0, 0, 0);
-                            const v16i dy = __builtin_amdgcn_mfma_i32_32x32x32_i8(quants(ky), y, zero, 0, 0, 0);
-                            if constexpr (DUMP)
-                            {
-                                const long nn = n0 + l32 - g.row0;
-                                if (n0 + l32 < g.w.N && nn >= 0 && nn < g.nrows)
-                                {
-#pragma unroll
-                                    for (int r = 0; r < 16; ++r)
-                                    {
-                                        const long m = m0 + t * 32 + 8 * (r >> 2) + 4 * lh + (r & 3);
-                                        int32_t *to = g.sums + ((size_t)m * g.nrows + (size_t)nn) * (size_t)KB + (size_t)sb * 8;
-                                        if (m < g.M)
-                                            to[kx] = dx[r], to[ky] = dy[r];
-                                    }
-                                }
-                            }
-#pragma unroll
-                            for (int r = 0; r < 16; ++r)
-                                acc[t][r] = fmaf((float)dx[r], cs[r], acc[t][r]);
-#pragma unroll
-                            for (int r = 0; r < 16; ++r)
-                                acc[t][r] = fmaf((float)dy[r], cs[16 + r], acc[t][r]);
-                            if (F::HAS_MIN)
-                                acc[t] = __builtin_amdgcn_mfma_f32_32x32x2f32((float)(int16_t)(head >> 16) * ad, Q::min_f32(S[c], i), acc[t], 0, 0, 0);
+                            const int m = j % MT * 32 + 8 * (r >> 2) + (r & 3);
+                            asm volatile("" : "+v"(at));
+                            if (m0 + 4 * lh + m < g.M)
+                                g.sums[at + (uint32_t)m * token] = (int32_t)biased_to_float(d[r]);
                         }
                     }
+                };
+                uint32_t head[2] = {head_of(0), 0};
+                v32f cs[2];
+                cs[0] = scales(0, head[0]);
+                v16i dx = product(0, 0, quants(0, 0)), dy = product(0, 1, quants(0, 1));
+#pragma unroll
+                for (int j = 0; j < JOBS; ++j)
+                {
+                    const int t = j % MT, now = j & 1, next = now ^ 1;
+                    v4i a;
+                    fence();
+#pragma unroll
+                    for (int i = j * EACH; i < (j + 1) * EACH; ++i)
+                        if (i < LOADS)
+                            issue_act(i, sb0 + KS, buf ^ 1);
+                    fence();
+                    if (j + 1 < JOBS)
+                    {
+                        head[next] = head_of(j + 1);
+                        a = quants(j + 1, 0);
+                    }
+                    if (DUMP)
+                        dump(j, 0, dx);
+#pragma unroll
+                    for (int r = 0; r < 16; ++r)
+                        acc[t][r] = fmaf(biased_to_float(dx[r]), cs[now][r], acc[t][r]);
+                    fence();
+                    if (j + 1 < JOBS)
+                    {
+                        cs[next] = scales(j + 1, head[next]);
+                        dx = product(j + 1, 0, a);
+                        a = quants(j + 1, 1);
+                    }
+                    fence();
+                    if (DUMP)
+                        dump(j, 1, dy);
+#pragma unroll
+                    for (int r = 0; r < 16; ++r)
+                        acc[t][r] = fmaf(biased_to_float(dy[r]), cs[now][16 + r], acc[t][r]);
+                    fence();
+                    if (j + 1 < JOBS)
+                        dy = product(j + 1, 1, a);
+                    if (F::HAS_MIN)
+                        acc[t] = __builtin_amdgcn_mfma_f32_32x32x2f32((float)(int16_t)(head[now] >> 16) * scale_of(head[now]), Q::min_f32(S, j / MT), acc[t], 0, 0, 0);
+                }
             }
         }
-        Q::template wait<0>(raw[0]);
-        Q::template wait<0>(raw[1]);
+        Q::template wait<0>(raw);
         if (DUMP)
             return;
 
-        if constexpr (KS > 1)
+        __syncthreads(); // everybody is done with the activations
+        float *red = reinterpret_cast<float *>(smem) + rn * MT * 16 * WAVE + lane;
+        if (kw > 0)
         {
-            __syncthreads(); // everybody is done with the activations
-            float *red = reinterpret_cast<float *>(smem) + rn * MT * 16 * WAVE + lane;
-            if (ks > 0)
-            {
 #pragma unroll
-                for (int t = 0; t < MT; ++t)
+            for (int t = 0; t < MT; ++t)
 #pragma unroll
-                    for (int r = 0; r < 16; ++r)
-                        red[((ks - 1) * RN * MT * 16 + t * 16 + r) * WAVE] = acc[t][r];
-            }
-            __syncthreads();
-            if (ks > 0)
-                return;
-#pragma unroll
-            for (int k = 0; k < KS - 1; ++k)
-#pragma unroll
-                for (int t = 0; t < MT; ++t)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r)
-                        acc[t][r] += red[(k * RN * MT * 16 + t * 16 + r) * WAVE];
+                for (int r = 0; r < 16; ++r)
+                    red[((kw - 1) * RN * MT * 16 + t * 16 + r) * WAVE] = acc[t][r];
         }
+        __syncthreads();
+        if (kw > 0)
+            return;
+        // (not unrolled: all sums asked for at once would not fit the registers)
+#pragma unroll 1
+        for (int k = 0; k < KW - 1; ++k)
+#pragma unroll
+            for (int t = 0; t < MT; ++t)
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    acc[t][r] += red[(k * RN * MT * 16 + t * 16 + r) * WAVE];
         if (n0 + l32 < g.w.N)
         {
 #pragma unroll
@@ -692,60 +744,73 @@ namespace llamql
         if (e != hipSuccess)
             return fail(fn, "cannot reserve %zu bytes of LDS: %s", lds, hipGetErrorString(e));
         hipLaunchKernelGGL(kernel, dim3((unsigned)((rows + 32 * RN - 1) / (32 * RN)), (unsigned)((M + 32 * MT - 1) / (32 * MT))),
-                           dim3(RN * KS * WAVE), lds, st, g);
+                           dim3(RN * 2 * KS * WAVE), lds, st, g);
         return launched(fn);
     }
 
     // Which kernel a shape takes: -1 for gemm_kernel, or an entry of SPLIT.  gemm_kernel's workgroup walks the whole of K
-    // alone, so where its tiles do not fill the chip (two workgroups a compute unit) the time is that walk, however little
-    // there is to multiply; gemm_split_kernel gives the walk to 2, 4 or 8 wavefronts.  Where the tiles do fill it,
-    // gemm_kernel's larger ones decode and rescale less per product.  The expected times in microseconds are fitted to
-    // measurements of the three formats:
-    //   tokens x rows x K          gemm_kernel   split (its best entry)
-    //   40 x 8192 x 5120, IQ3_S       38            23 (1)
-    //   130 x 5000 x 5120, Q4_K       52            29 (2), 32 (3) is taken
-    //   130 x 5000 x 5120, Q6_K       60            38 (3)
-    //   12 x 1500 x 20480, Q4_K       72            34 (0)
-    //   64 x 4096 x 4096, Q4_K        26            12 (0)
-    //   300 x 2000 x 2048, Q4_K       22            15 (2, 3)
-    //   40 x 12000 x 8192, Q6_K       63            51 (3)
-    //   199 x 5120 x 25600, Q6_K      279           261 (4)
-    //   256 x 8192 x 8192, Q4_K       85            79 (4)
-    //   129 x 25600 x 5120, Q4_K      152           116 (2)
-    //   129 x 25600 x 5120, Q6_K      176           166 (4), 170 (2) is taken
-    // and gemm_kernel's shapes:
-    //   20 x 25600 x 5120, Q4_K       30            30 (2)
-    //   1000 x 4096 x 4096, Q4_K      71            83 (4)
-    //   300 x 25600 x 5120, IQ3_S     202           220 (4)
-    //   520 x 14000 x 5120, IQ3_S     197           224 (4)
-    //   512 x 25600 x 5120, Q4_K      275           347 (4)
+    // alone, two of them on a compute unit; gemm_split_kernel has one there and gives the walk to 2, 4 or 8 pairs of wavefronts.
+    // The expected times in microseconds are fitted to measurements, weights from memory (us, gemm_kernel and the entries):
+    //   tokens x rows x K             gemm_kernel  0: 1,1,4  1: 1,2,2  2: 2,1,4  3: 2,2,2  4: 2,4,1  5: 4,2,2  6: 4,4,1
+    //   10 x 4096 x 4096, Q4_K           16.5         9.8     13.5      13.5      20.5      32.9      32.5      52.6
+    //   64 x 4096 x 4096, IQ3_S          31.3        12.6     18.3      16.7      23.6      38.2      33.7      55.0
+    //   20 x 12000 x 4096, IQ3_S         23.1        21.6     18.5      28.9      24.1      38.2      34.5      55.2
+    //   40 x 8192 x 5120, IQ3_S          38.4        25.2     21.9      19.0      28.7      46.8      40.7      67.7
+    //   63 x 5034 x 18944, Q6_K          162         103      96.0      70.5      114       201       153       279
+    //   130 x 5000 x 5120, Q4_K          52.2        36.7     30.0      33.2      26.7      40.7      40.9      65.6
+    //   64 x 25600 x 5120, Q4_K          53.8        68.1     60.0      68.4      51.9      45.1      82.0      70.5
+    //   80 x 9762 x 3072, Q6_K           37.3        38.1     31.7      39.8      37.8      31.9      29.1      45.3
+    //   199 x 5120 x 25600, Q6_K         298         298      314       230       260       241       207       369
+    //   256 x 8192 x 8192, Q4_K          86.2        122      92.2      97.1      75.8      65.7      64.8      106
+    //   1000 x 4096 x 4096, Q4_K         65.8        122      94.1      110       79.4      66.5      68.1      57.8
+    //   256 x 25600 x 5120, Q4_K         154         228      184       211       167       160       161       140
+    // and gemm_kernel's shapes, tiles of 32 tokens in one round, or three and more rounds of tiles of 128:
+    //   16 x 25600 x 5120, Q6_K          49.9        65.1     57.7      77.0      67.4      59.0      93.0      83.2
+    //   384 x 25600 x 5120, Q4_K         194         339      267       303       236       201       201       208
+    //   512 x 25600 x 5120, Q4_K         266         445      351       401       309       280       282       275
+    //   2048 x 6400 x 5120, IQ3_S        263         518      473       410       350       322       279       272
     struct SplitTile
     {
         int mt, rn, ks;
-        double step, fixed; // microseconds: KS super-blocks, and a workgroup's start and end
+        double step[3]; // microseconds: a step (KS super-blocks) of Q4_K, Q6_K and IQ3_S
     };
-    constexpr SplitTile SPLIT[] = {{1, 1, 8, 4.6, 4.0}, {1, 2, 4, 3.8, 4.0}, {1, 4, 2, 3.4, 4.0}, {2, 2, 4, 5.9, 5.0}, {2, 4, 2, 4.9, 4.0}};
+    constexpr SplitTile SPLIT[] = {
+        {1, 1, 4, {1.6, 2.8, 2.4}}, {1, 2, 2, {1.35, 2.45, 1.9}}, {2, 1, 4, {2.65, 3.5, 3.2}}, {2, 2, 2, {2.35, 3.05, 2.6}},
+        {2, 4, 1, {2.05, 2.9, 2.4}}, {4, 2, 2, {3.83, 4.1, 4.0}}, {4, 4, 1, {3.45, 3.85, 3.6}}};
+    constexpr double SPLIT_START = 3.5, WHOLE_START = 2.0; // a workgroup's start and end
+    // gemm_kernel: microseconds a super-block of a tile of 32, 64 or 128 tokens takes in a round of two workgroups a compute unit
+    // that others follow, in the last round, and in a last round of one
+    struct WholeTile
+    {
+        int tokens;
+        double full[3], last[3], alone[3];
+    };
+    constexpr WholeTile WHOLE[] = {{32, {1.4, 2.2, 1.9}, {1.6, 2.5, 2.2}, {0.9, 1.5, 1.4}},
+                                   {64, {2.4, 3.1, 2.65}, {2.7, 3.6, 3.05}, {1.65, 2.2, 1.9}},
+                                   {GEMM_BM, {3.55, 3.95, 3.55}, {4.2, 4.8, 4.35}, {2.6, 3.0, 2.8}}};
 
-    inline int gemm_split_choice(int M, int N, int K, int cus)
+    inline int gemm_split_choice(int format, int M, int N, int K, int cus)
     {
         if (K > 1 << 24) // 32-bit offsets from a tile's first token
             return -1;
         const auto over = [](long a, long b) { return (a + b - 1) / b; };
         const int SB = K / 256;
-        // gemm_kernel: microseconds per super-block of one workgroup alone on a compute unit, and of two sharing it
-        const double alone = M <= 32 ? 0.9 : M <= 64 ? 2.0 : 2.75, two = M <= 32 ? 1.7 : M <= 64 ? 2.75 : 4.5;
-        const long tiles = over(N, GEMM_BN) * over(M, M <= 32 ? 32 : M <= 64 ? 64 : GEMM_BM);
-        const long rest = tiles % (2 * cus);
-        const double undivided = SB * ((double)(tiles / (2 * cus)) * two + (rest == 0 ? 0.0 : rest <= cus ? alone : two));
-        double best = undivided;
+        const WholeTile &whole = WHOLE[M <= 32 ? 0 : M <= 64 ? 1 : 2];
+        const long tiles = over(N, GEMM_BN) * over(M, whole.tokens), rest = tiles % (2 * cus);
+        const double undivided = WHOLE_START + SB * ((double)(tiles / (2 * cus)) * whole.full[format] +
+                                                     (rest == 0 ? 0.0 : rest <= cus ? whole.alone[format] : whole.last[format]));
+        double best = 0.97 * undivided;
         int choice = -1;
         for (int i = 0; i < (int)(sizeof(SPLIT) / sizeof(SPLIT[0])); ++i)
         {
             const SplitTile &t = SPLIT[i];
-            const long rounds = over(over(N, 32 * t.rn) * over(M, 32 * t.mt), cus);
-            const double us = (double)rounds * ((double)over(SB, t.ks) * t.step + t.fixed);
-            // (several rounds: gemm_kernel's overlap, two workgroups a compute unit, and take less than they are counted for)
-            if (us < best && us < (rounds > 1 ? 0.85 : 0.95) * undivided && over(M, 32 * t.mt) <= 65535) // (the grid's second extent)
+            if (over(M, 32 * t.mt) > 65535) // (the grid's second extent)
+                continue;
+            // (a last round of few workgroups is faster: they have the memory and the clock to themselves)
+            const long groups = over(N, 32 * t.rn) * over(M, 32 * t.mt), left = groups % cus;
+            const double rounds = groups <= cus ? 1.0 : (double)(groups / cus) + (left ? 0.6 + 0.4 * (double)left / cus : 0.0);
+            const double us = rounds * ((double)over(SB, t.ks) * t.step[format] + SPLIT_START);
+            if (us < best)
                 best = us, choice = i;
         }
         return choice;
@@ -778,13 +843,16 @@ namespace llamql
         }
         const int tile_end = DUMP ? (row0 + nrows + GEMM_BN - 1) / GEMM_BN : (N + GEMM_BN - 1) / GEMM_BN;
         const int rows_end = DUMP ? row0 + nrows : N, rows = rows_end - g.tile0 * GEMM_BN;
-        switch (gemm_split_choice(M, N, K, cu_count(device_id)))
+        constexpr int format = F::HAS_MIN ? 0 : F::TABLE_BYTES > 0 ? 2 : 1; // Q4_K, Q6_K, IQ3_S
+        switch (gemm_split_choice(format, M, N, K, cu_count(device_id)))
         {
-        case 0: return gemm_split_launch<F, DUMP, 1, 1, 8>(fn, g, rows, M, st);
-        case 1: return gemm_split_launch<F, DUMP, 1, 2, 4>(fn, g, rows, M, st);
-        case 2: return gemm_split_launch<F, DUMP, 1, 4, 2>(fn, g, rows, M, st);
-        case 3: return gemm_split_launch<F, DUMP, 2, 2, 4>(fn, g, rows, M, st);
-        case 4: return gemm_split_launch<F, DUMP, 2, 4, 2>(fn, g, rows, M, st);
+        case 0: return gemm_split_launch<F, DUMP, 1, 1, 4>(fn, g, rows, M, st);
+        case 1: return gemm_split_launch<F, DUMP, 1, 2, 2>(fn, g, rows, M, st);
+        case 2: return gemm_split_launch<F, DUMP, 2, 1, 4>(fn, g, rows, M, st);
+        case 3: return gemm_split_launch<F, DUMP, 2, 2, 2>(fn, g, rows, M, st);
+        case 4: return gemm_split_launch<F, DUMP, 2, 4, 1>(fn, g, rows, M, st);
+        case 5: return gemm_split_launch<F, DUMP, 4, 2, 2>(fn, g, rows, M, st);
+        case 6: return gemm_split_launch<F, DUMP, 4, 4, 1>(fn, g, rows, M, st);
         default: break;
         }
         // few tokens: one smaller tile of tokens (a 128-token tile would rescale 128 rows for them)

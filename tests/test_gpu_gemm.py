@@ -115,6 +115,61 @@ def test_a_walk_dealt_to_wavefronts(capi, dev, oracle, fmt, M, N, K):
 
 
 @pytest.mark.parametrize("fmt", list(FMTS.values()), ids=list(FMTS))
+@pytest.mark.parametrize("M,N,K", [
+    (9, 33, 1792), (31, 4095, 2304),        # tiles of 32 x 32: super-blocks left over
+    (20, 12001, 4864), (31, 8161, 1280), (33, 4100, 2816),  # 32 x 64
+    (63, 8161, 2048), (33, 8161, 4864),     # 64 x 32
+    (129, 4999, 1536), (129, 4999, 2816),   # 64 x 64: the last token tile of one token, a super-block left over
+    (64, 20001, 1024), (33, 24997, 1280),   # 64 x 128
+    (97, 9799, 4352), (193, 8000, 2560),    # 128 x 64
+    (128, 24997, 1280), (257, 8129, 2304),  # 128 x 128
+])
+def test_tiles_of_dealt_walks(capi, dev, oracle, fmt, M, N, K):
+    """Every tile whose half super-blocks are dealt to wavefronts, with rows, tokens and super-blocks left over: each element
+    written once and the same bits again, near the oracle's on the first and last rows of W, their block sums bit for bit.
+    The tolerance is that of the undivided walk: the parts are sums of the same products."""
+    import torch
+
+    W = synth.weights_numpy(fmt, N, K, 17 + M + N)
+    q8 = oracle.quantize(synth.activations_numpy(M, K, 19 + K))
+    wd = upload_weights(capi, dev, fmt, W)
+    qd = upload_q8(dev, q8)
+    y, again = (torch.full((M, N + 4), float("nan"), device=dev) for _ in range(2))
+    for out in (y, again):
+        capi.gemm(fmt, wd, qd, M, N, K, out=out[:, :N])
+    sync()
+    assert torch.equal(y[:, :N], again[:, :N]) and bool(torch.isnan(y[:, N:]).all())
+    got, n = y.cpu().numpy(), min(N, 96)
+    for r0 in (0, N - n):
+        s = capi.gemm_block_sums(fmt, wd, qd, M, N, K, r0, n)
+        sync()
+        C, sums = oracle.gemm(fmt, W, K, q8, n0=r0, n1=r0 + n, want_sums=True)
+        part = got[:, r0:r0 + n]
+        assert rel_err(part, C) <= TOL[fmt] * 1e-2
+        assert np.abs(part - C).max() <= 1e-4 * np.abs(C).max()
+        assert np.array_equal(s.cpu().numpy(), sums)
+
+
+def test_block_sums_at_their_limits(capi, dev, oracle):
+    """Q6_K rows and activations whose every product is the largest there is, 127 and -128 both ways: sums of 32 of them."""
+    M, N, K, fmt = 33, 4096, 512, FMT_Q6_K
+    W = synth.weights_numpy(fmt, N, K, 5)
+    W.reshape(N, -1, 210)[:, :, :192] = np.where(np.arange(N)[:, None, None] % 2, 255, 0)   # all bits: q = 31; none: -32
+    W.reshape(N, -1, 210)[:, :, 192:208] = 127
+    x = np.where(np.arange(M)[:, None] % 2, 1.0, -1.0) * np.ones((M, K), np.float32)
+    q8 = oracle.quantize(x.astype(np.float32))
+    wd = upload_weights(capi, dev, fmt, W)
+    qd = upload_q8(dev, q8)
+    s = capi.gemm_block_sums(fmt, wd, qd, M, N, K, 0, 64)
+    y = capi.gemm(fmt, wd, qd, M, N, K)
+    sync()
+    C, sums = oracle.gemm(fmt, W, K, q8, n0=0, n1=64, want_sums=True)
+    assert np.abs(sums).max() >= 32 * 120 * 127
+    assert np.array_equal(s.cpu().numpy(), sums)
+    assert rel_err(y.cpu().numpy()[:, :64], C) <= TOL[fmt] * 1e-2
+
+
+@pytest.mark.parametrize("fmt", list(FMTS.values()), ids=list(FMTS))
 def test_more_tiles_than_the_chip_holds(capi, dev, oracle, fmt):
     """More tiles than the chip holds at once, with a sparsely filled last round of workgroups
     (580 tiles of 128 x 64 on 512 workgroup slots), ragged in both directions (130 tokens: the

@@ -65,30 +65,48 @@ def test_every_tile_of_grouped_layers_has_sizes(kind):
 # ---- prompt GEMM (gemm.hip: gemm_split_choice) -----------------------------------------------------------
 
 GEMM = (CSRC / "gemm.hip").read_text()
-SPLIT = [tuple(map(float, t)) for t in
-         re.findall(r"\{(\d), (\d), (\d), ([\d.]+), ([\d.]+)\}", re.search(r"SPLIT\[\] = \{(.*)\};", GEMM).group(1))]
 
 
-def gemm_choice(M, N, K):
-    SB, alone, two = K // 256, 0.9 if M <= 32 else 2.0 if M <= 64 else 2.75, 1.7 if M <= 32 else 2.75 if M <= 64 else 4.5
-    tiles = over(N, 64) * over(M, 32 if M <= 32 else 64 if M <= 64 else 128)
+def triples(text):
+    return [tuple(map(float, t)) for t in re.findall(r"\{([\d.]+), ([\d.]+), ([\d.]+)\}", text)]
+
+
+TABLE = re.search(r"SPLIT\[\] = \{(.*?)\}\};", GEMM, re.S).group(1) + "}"
+SPLIT = list(zip([tuple(map(int, t)) for t in re.findall(r"\{(\d), (\d), (\d), \{", TABLE)], triples(TABLE)))
+START, WHOLE_START = map(float, re.search(r"SPLIT_START = ([\d.]+), WHOLE_START = ([\d.]+)", GEMM).groups())
+WHOLE = triples(re.search(r"WHOLE\[\] = \{(.*?)\}\}\};", GEMM, re.S).group(1) + "}")
+
+
+def gemm_choice(fmt, M, N, K):
+    """fmt: 0, 1, 2 for Q4_K, Q6_K, IQ3_S."""
+    SB, kind = K // 256, 0 if M <= 32 else 1 if M <= 64 else 2
+    full, last, alone = (t[fmt] for t in WHOLE[3 * kind:3 * kind + 3])
+    tiles = over(N, 64) * over(M, (32, 64, 128)[kind])
     rest = tiles % (2 * CUS)
-    undivided = SB * (tiles // (2 * CUS) * two + (0.0 if rest == 0 else alone if rest <= CUS else two))
-    best, choice = undivided, -1
-    for i, (mt, rn, ks, step, fixed) in enumerate(SPLIT):
-        rounds = over(over(N, 32 * int(rn)) * over(M, 32 * int(mt)), CUS)
-        us = rounds * (over(SB, int(ks)) * step + fixed)
-        if us < best and us < (0.85 if rounds > 1 else 0.95) * undivided:
+    best, choice = 0.97 * (WHOLE_START + SB * (tiles // (2 * CUS) * full + (0.0 if rest == 0 else alone if rest <= CUS else last))), -1
+    for i, ((mt, rn, ks), step) in enumerate(SPLIT):
+        groups = over(N, 32 * rn) * over(M, 32 * mt)
+        left = groups % CUS
+        rounds = 1.0 if groups <= CUS else groups // CUS + (0.6 + 0.4 * left / CUS if left else 0.0)
+        us = rounds * (over(SB, ks) * step[fmt] + START)
+        if us < best:
             best, choice = us, i
     return choice
 
 
 def test_every_kernel_of_the_prompt_gemm_has_sizes():
-    assert len(SPLIT) == GEMM.count("case") - GEMM.count("case LLAM") == 5
-    products = sizes(test_gpu_gemm.test_random_shapes) + sizes(test_gpu_gemm.test_a_walk_dealt_to_wavefronts)
-    sums = [s[:3] for s in sizes(test_gpu_gemm.test_block_sums_of_the_gemm_kernel)] + sizes(test_gpu_gemm.test_a_walk_dealt_to_wavefronts)
-    for shapes in (products, sums):
-        assert {gemm_choice(*s) for s in shapes} == {-1, 0, 1, 2, 3, 4}
-        undivided = [M for M, N, K in shapes if gemm_choice(M, N, K) == -1]
-        assert {0 if M <= 32 else 1 if M <= 64 else 2 for M in undivided} == {0, 1, 2}, "a tile of 32, 64 or 128 tokens"
-        assert any(M % 64 for M in undivided if 32 < M <= 64)
+    assert len(SPLIT) == GEMM.count("case") - GEMM.count("case LLAM") == 7 and len(WHOLE) == 9
+    dealt = sizes(test_gpu_gemm.test_a_walk_dealt_to_wavefronts) + sizes(test_gpu_gemm.test_tiles_of_dealt_walks)
+    products = sizes(test_gpu_gemm.test_random_shapes) + dealt
+    sums = [s[:3] for s in sizes(test_gpu_gemm.test_block_sums_of_the_gemm_kernel)] + dealt
+    for fmt in range(3):
+        for shapes in (products, sums):
+            chosen = {s: gemm_choice(fmt, *s) for s in shapes}
+            assert set(chosen.values()) == set(range(-1, len(SPLIT)))
+            for i, ((mt, rn, ks), _) in enumerate(SPLIT):
+                own = [s for s in shapes if chosen[s] == i]
+                assert any(M % (32 * mt) for M, N, K in own) and any(N % (32 * rn) for M, N, K in own), (fmt, SPLIT[i])
+                assert ks == 1 or any(K // 256 % ks for M, N, K in own), (fmt, SPLIT[i])
+            undivided = [M for M, N, K in shapes if chosen[M, N, K] == -1]
+            assert {0 if M <= 32 else 1 if M <= 64 else 2 for M in undivided} == {0, 1, 2}, "a tile of 32, 64 or 128 tokens"
+            assert any(M % 64 for M in undivided if 32 < M <= 64)
