@@ -8,16 +8,23 @@
 // one is the pairs' activations, [block][pair][32] in LDS, so the exact block sums of pairs 4 l .. 4 l + 3 lie with row
 // c's scale; the scales are exchanged with the same swaps.
 //
-// Bound by the decoders (vector instructions and, for IQ3_S, table gathers) and the weights' bytes; the products and
-// the rescale of 16 pairs are a fifth of the instructions.  256 experts of 2048 x 512 and one for all tokens, IQ3_S,
-// 333 tokens of 9 slots: gate and up 279 -> 138 us, down 134 -> 70 us against one decode for four pairs (the weights alone
-// are 45 and 23 us of reads).
+// Bound by the decoders (vector instructions and, for IQ3_S, table gathers: the LDS is busy four fifths of the time), the
+// weights' bytes, and a workgroup's start (a chain of five loads; half as many row tiles a workgroup take 15 % longer, for all that
+// their last round is fuller); the products and the rescale of 16 pairs are a seventh of the instructions.  256 experts of 2048 x 512
+// and one for all tokens, IQ3_S, 333 tokens of 9 slots: gate and up 279 -> 138 us, down 134 -> 70 us against one decode for
+// four pairs (the weights alone are 45 and 23 us of reads).  Scales multiplied on the matrix unit, sums without a conversion
+// and carries by branches are 258 instead of 352 vector instructions a super-block; whole feed-forwards, IQ3_S: 440 tokens, 128 experts of
+// 2048 x 1024 (32 pairs a tile) 324 -> 292 us, the 333 tokens above 228 -> 224; Q4_K 217 -> 207, 440 tokens, 64 of 4096 x 768 516 -> 470.
 #pragma once
+
+#include <type_traits>
 
 namespace llamql
 {
     constexpr int MOE_MFMA_WAVES = 8;
     constexpr int MOE_MFMA_MAX_SB = 16; // super-blocks of a row
+    typedef float v16f_moe __attribute__((ext_vector_type(16)));
+    constexpr float MOE_MFMA_BIAS = 12582912.0f; // 1.5 * 2^23
     constexpr size_t MOE_MFMA_LDS = 150 * 1024; // of the 160 KB, beside the decoders' tables
 
     // bytes of a block's activations in LDS: a pad, so that neighbouring blocks of a pair start in different banks
@@ -44,7 +51,8 @@ namespace llamql
     // grid: (workgroups per matrix, tiles of pairs (upper bound), DOWN ? 1 : 2 = gate|up)
     // m.rows_per_wave: 16-row tiles of a wavefront
     template <class F, int MT, bool DOWN>
-    __global__ void __launch_bounds__(MOE_MFMA_WAVES *WAVE) moe_grouped_mfma_kernel(const MoEArgs m, void *ws, int P)
+    __global__ void __launch_bounds__(MOE_MFMA_WAVES *WAVE) __attribute__((amdgpu_waves_per_eu(F::TABLE_BYTES > 0 ? 4 : 1)))
+        moe_grouped_mfma_kernel(const MoEArgs m, void *ws, int P)
     {
         typedef typename F::Quad Q;
         constexpr int KBS = moe_mfma_block_bytes(MT);
@@ -160,26 +168,50 @@ namespace llamql
                 for (int r = 0; r < 4; ++r)
                     level[t][k][r] = 0.0f;
         int step = 0, sb = 0, row = tile0 * 16 + c;
+        // (branches, which are uniform, and not choices between registers: those were 32 of 350 instructions a super-block)
+        auto carry = [&](auto &self, int t, float (&sum)[4], auto depth) __attribute__((always_inline)) {
+            constexpr int k = decltype(depth)::value;
+            if constexpr (k + 1 < LEVELS)
+            {
+                if ((sb >> k) & 1)
+                {
+                    asm volatile("");
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        sum[r] = level[t][k][r] + sum[r];
+                    self(self, t, sum, std::integral_constant<int, k + 1>());
+                    return;
+                }
+                asm volatile("");
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                level[t][k][r] = sum[r];
+        };
+        v4i bias;
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            bias[r] = __float_as_int(MOE_MFMA_BIAS);
+        asm volatile("" : "+v"(bias));
         const uint8_t *a_lane = moe_mfma_smem + c * 32 + l * 8;
         auto compute = [&](const typename Q::Raw &buf) {
             v4i wq[4];
             typename Q::Scale S;
             Q::decode(buf, lc, wq, S);
-            uint32_t lo[2][4], hi[2][4], scale[2][4], low[2][4];
+            uint32_t lo[2][4], hi[2][4], low[2][4];
 #pragma unroll
             for (int i = 0; i < 2; ++i)
             {
-                const uint32_t s = __float_as_uint(Q::scale_f32(S, i)), mn = __float_as_uint(Q::min_f32(S, i));
+                const uint32_t mn = __float_as_uint(Q::min_f32(S, i));
 #pragma unroll
                 for (int k = 0; k < 4; ++k)
                 {
                     lo[i][k] = (uint32_t)wq[2 * i + (k >> 1)][2 * (k & 1)];
                     hi[i][k] = (uint32_t)wq[2 * i + (k >> 1)][2 * (k & 1) + 1];
-                    scale[i][k] = s, low[i][k] = mn;
+                    low[i][k] = mn;
                 }
                 quarter_exchange(lo[i]);
                 quarter_exchange(hi[i]);
-                quarter_exchange(scale[i]);
                 if (F::HAS_MIN)
                     quarter_exchange(low[i]);
             }
@@ -190,21 +222,27 @@ namespace llamql
                     break; // uniform
                 float sum[4][4];
 #pragma unroll
-                for (int k = 0; k < 4; ++k)
+                for (int i = 0; i < 2; ++i)
+                {
+                    // A lane's own scale times the pairs' of its block: rank-1 matrices of four blocks, in the layout of the block sums
+                    // (exact: both factors are fp16 values)
+                    const v16f_moe none = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+                    const v16f_moe scale = __builtin_amdgcn_mfma_f32_16x16x1f32(ad[(sb * 8 + Q::block_of(l, i)) * MT * 16 + t * 16 + c], Q::scale_f32(S, i), none, 0, 0, 0);
 #pragma unroll
-                    for (int i = 0; i < 2; ++i)
+                    for (int k = 0; k < 4; ++k)
                     {
                         const int kb = sb * 8 + Q::block_of(k, i);
                         const long b = (long)(((uint64_t)hi[i][k] << 32) | lo[i][k]);
-                        const float bs = __uint_as_float(scale[i][k]), bm = __uint_as_float(low[i][k]);
+                        const float bm = __uint_as_float(low[i][k]);
                         const long x = *reinterpret_cast<const long *>(a_lane + (size_t)kb * KBS + t * 512);
-                        const v4i zero = {0, 0, 0, 0};
-                        const v4i d = __builtin_amdgcn_mfma_i32_16x16x32_i8(x, b, zero, 0, 0, 0);
-                        const float4 da = *reinterpret_cast<const float4 *>(ad + kb * MT * 16 + t * 16 + 4 * l);
-                        const float ds[4] = {da.x, da.y, da.z, da.w};
+                        // started from the bits of 1.5 * 2^23, the integer result has those of 1.5 * 2^23 + sum: no conversion
+                        const v4i d = __builtin_amdgcn_mfma_i32_16x16x32_i8(x, b, bias, 0, 0, 0);
 #pragma unroll
                         for (int r = 0; r < 4; ++r)
-                            sum[k][r] = i == 0 ? (float)d[r] * (ds[r] * bs) : fmaf((float)d[r], ds[r] * bs, sum[k][r]);
+                        {
+                            const float f = __int_as_float(d[r]) - MOE_MFMA_BIAS;
+                            sum[k][r] = i == 0 ? f * scale[4 * k + r] : fmaf(f, scale[4 * k + r], sum[k][r]);
+                        }
                         if (F::HAS_MIN)
                         {
                             const float4 sa = *reinterpret_cast<const float4 *>(asd + kb * MT * 16 + t * 16 + 4 * l);
@@ -214,24 +252,11 @@ namespace llamql
                                 sum[k][r] = fmaf(ss[r], bm, sum[k][r]);
                         }
                     }
+                }
 #pragma unroll
                 for (int r = 0; r < 4; ++r)
                     sum[0][r] = (sum[0][r] + sum[1][r]) + (sum[2][r] + sum[3][r]);
-                bool up = true;
-#pragma unroll
-                for (int k = 0; k < LEVELS; ++k)
-                {
-                    const bool set = (sb >> k) & 1; // uniform
-#pragma unroll
-                    for (int r = 0; r < 4; ++r)
-                    {
-                        if (up && set)
-                            sum[0][r] = level[t][k][r] + sum[0][r];
-                        else if (up)
-                            level[t][k][r] = sum[0][r];
-                    }
-                    up = up && set;
-                }
+                carry(carry, t, sum[0], std::integral_constant<int, 0>());
             }
             ++step;
             if (++sb == nsb)
