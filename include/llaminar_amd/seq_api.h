@@ -153,6 +153,10 @@ bool llam_seq_memory_decode(const llam_seq_memory_args *a, const llam_seq_entrie
 /* one entry of ntok tokens, in chunks */
 bool llam_seq_memory_prefill(const llam_seq_memory_args *a, const llam_seq_entries *e, int entry, int ntok,
                              void *d_scratch, size_t scratch_bytes, int dtype, int device_id, void *stream);
+/* The portions of entries first .. first + n - 1, of at most max_ntok tokens each, in one launch a kernel; rows: past the
+ * last of their rows (and no more than the scratch was sized for). */
+bool llam_seq_memory_prefill_many(const llam_seq_memory_args *a, const llam_seq_entries *e, int first, int n, int max_ntok,
+                                  int rows, void *d_scratch, size_t scratch_bytes, int dtype, int device_id, void *stream);
 
 /* Grouped-query attention with rotary positions.  Query head h reads key/value head h / (heads / kv_heads).
  * Caches: elem, k [slots][kv_heads][ring][dim], v [slots][kv_heads][ring][vdim]; position p lies in row
@@ -213,6 +217,9 @@ bool llam_seq_delta_decode(const llam_seq_delta_args *a, const llam_seq_entries 
 /* one entry of ntok tokens, in chunks */
 bool llam_seq_delta_prefill(const llam_seq_delta_args *a, const llam_seq_entries *e, int entry, int ntok, void *d_scratch,
                             size_t scratch_bytes, int dtype, int device_id, void *stream);
+/* As llam_seq_memory_prefill_many. */
+bool llam_seq_delta_prefill_many(const llam_seq_delta_args *a, const llam_seq_entries *e, int first, int n, int max_ntok, int rows,
+                                 void *d_scratch, size_t scratch_bytes, int dtype, int device_id, void *stream);
 
 /* Routed experts.  logits: fp32 [M][ldz], column e < experts of expert e, column `experts` the
  * logit of the shared expert's gate where there is one.  Expert e's matrices: d_up + e *

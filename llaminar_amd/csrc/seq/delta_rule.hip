@@ -23,6 +23,7 @@
 namespace llamql
 {
     constexpr int DC = 64;             // tokens of a chunk
+    constexpr int DELTA_MANY = 16;     // portions of a launch at most
     constexpr int DELTA_DIM_MAX = 256; // a wavefront holds a q or k vector, four values a lane
 
     struct DeltaArgs
@@ -30,12 +31,16 @@ namespace llamql
         llam_seq_delta_args a;
         const int32_t *row0, *ntok, *slot, *pos;
         int entry, rows, channels; // rows: tokens the scratch is laid out for
+        bool many;                 // several portions: a portion's tokens are kept from token (row0 / DC + its place among them) DC on
         float *q, *k, *v;          // [kv_heads][rows][dim] (tiled), the same, [heads][rows][vdim]
         float *beta, *log_decay;   // [heads][rows]
         float *P, *U, *W, *kd;     // per chunk and head: [DC][DC], [DC][vdim], [DC][dim], [dim][DC], tiled but for U
         float *gamma;              // per chunk and head: e^(G_t), [DC], then e^(G_end)
         float *o;                  // [rows][heads][vdim]
     };
+
+    // the first kept token of the call's portion ei
+    __device__ __forceinline__ int first_kept(const DeltaArgs &p, int ei) { return p.many ? (p.row0[p.entry + ei] / DC + ei) * DC : 0; }
 
     // Tiled: what a wavefront reads as a matrix operand lies as its lanes read it, 16 rows x 32 columns as two kilobytes, of which lane
     // (r, g) has 16 bytes each: columns 8 g .. + 3 and 8 g + 4 .. + 7 of row r.  Row by row, sixteen neighbouring lanes read sixteen rows,
@@ -239,7 +244,7 @@ namespace llamql
         delta_inputs_kernel(DeltaArgs p)
     {
         const llam_seq_delta_args &a = p.a;
-        const int e = p.entry, n = p.ntok[e], unit = blockIdx.x, G = a.kv_heads;
+        const int e = p.entry + blockIdx.z, n = p.ntok[e], unit = blockIdx.x, G = a.kv_heads, kept = first_kept(p, blockIdx.z);
         const int slot = p.slot[e], pos0 = p.pos[e];
         const int size = unit < 2 * G ? a.dim : a.vdim, lanes = size <= 64 ? 16 : size <= 128 ? 32 : 64;
         const int lane = threadIdx.x & (lanes - 1);
@@ -256,16 +261,16 @@ namespace llamql
                     y = delta_conv(p, r, pos0 + t, pos0, slot, unit * a.dim + lane * 4);
                 y = y * (delta_unit(y, lanes) * (query ? 1.0f / sqrtf((float)a.dim_real) : 1.0f));
                 if (lane * 4 < a.dim)
-                    *reinterpret_cast<f32x4 *>(query ? p.q + (size_t)unit * p.rows * a.dim + tiled_at(t, lane * 4, a.dim)
-                                                     : p.k + ((size_t)(unit - G) * p.rows + t) * a.dim + lane * 4) = y;
+                    *reinterpret_cast<f32x4 *>(query ? p.q + ((size_t)unit * p.rows + kept) * a.dim + tiled_at(t, lane * 4, a.dim)
+                                                     : p.k + ((size_t)(unit - G) * p.rows + kept + t) * a.dim + lane * 4) = y;
             }
             else
             {
                 const int h = unit - 2 * G;
                 for (int d = lane * 4; d < a.vdim; d += lanes * 4)
-                    *reinterpret_cast<f32x4 *>(p.v + ((size_t)h * p.rows + t) * a.vdim + d) = delta_conv(p, r, pos0 + t, pos0, slot, 2 * G * a.dim + h * a.vdim + d);
+                    *reinterpret_cast<f32x4 *>(p.v + ((size_t)h * p.rows + kept + t) * a.vdim + d) = delta_conv(p, r, pos0 + t, pos0, slot, 2 * G * a.dim + h * a.vdim + d);
                 if (lane == 0)
-                    delta_gates(a, a.d_proj + (size_t)r * a.ldp, h, p.beta[(size_t)h * p.rows + t], p.log_decay[(size_t)h * p.rows + t]);
+                    delta_gates(a, a.d_proj + (size_t)r * a.ldp, h, p.beta[(size_t)h * p.rows + kept + t], p.log_decay[(size_t)h * p.rows + kept + t]);
             }
         }
     }
@@ -274,7 +279,7 @@ namespace llamql
     __global__ void __launch_bounds__(256)
         delta_keep_kernel(DeltaArgs p)
     {
-        const int e = p.entry, n = p.ntok[e], back = blockIdx.y; // back = 0: the last token
+        const int e = p.entry + blockIdx.z, n = p.ntok[e], back = blockIdx.y; // back = 0: the last token
         const int ch = (blockIdx.x * 256 + threadIdx.x) * 4;
         if (back >= n || ch >= p.channels)
             return;
@@ -294,10 +299,11 @@ namespace llamql
         __shared__ float s_beta[DC], s_in[DC], s_out[DC]; // beta_t e^(G_t), e^(G_end - G_t)
         const llam_seq_delta_args &a = p.a;
         const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = lane & 15, g = lane >> 4;
-        const int h = blockIdx.y, chunk = blockIdx.x, t0 = chunk * DC, dim = a.dim;
-        const int n = p.ntok[p.entry] - t0 < DC ? p.ntok[p.entry] - t0 : DC;
+        const int h = blockIdx.y, e = p.entry + blockIdx.z, dim = a.dim, left = p.ntok[e] - (int)blockIdx.x * DC;
+        const int n = left < DC ? left : DC;
         if (n <= 0)
             return;
+        const int t0 = first_kept(p, blockIdx.z) + blockIdx.x * DC, chunk = t0 / DC; // as they are kept
         const int kv = h / (a.heads / a.kv_heads);
         const float *q = p.q + ((size_t)kv * p.rows + t0 + wave * 16) * dim, *k = p.k + ((size_t)kv * p.rows + t0) * dim;
         const float *v = p.v + ((size_t)h * p.rows + t0) * a.vdim;
@@ -429,11 +435,11 @@ namespace llamql
         const int blocks = a.vdim / 16, h = blockIdx.x / (8 * blocks) * 8 + (blockIdx.x & 7);
         if (h >= a.heads)
             return;
-        const int e = p.entry, ntok = p.ntok[e];
+        const int e = p.entry + blockIdx.y, ntok = p.ntok[e], kept = first_kept(p, blockIdx.y);
         const int kv = h / (a.heads / a.kv_heads), col = (blockIdx.x >> 3) % blocks * 16 + c;
         const bool fresh = p.pos[e] == 0;
         float *state = a.d_state + ((size_t)p.slot[e] * a.heads + h) * DP * a.vdim + col;
-        const float *qrows = p.q + (size_t)kv * p.rows * DP;
+        const float *qrows = p.q + ((size_t)kv * p.rows + kept) * DP;
 
         f32x4 S[TS];
 #pragma unroll
@@ -452,7 +458,7 @@ namespace llamql
         f32x8 w[KS], q[KS];
         float u0[4];
         auto request = [&](int t0) __attribute__((always_inline)) {
-            const size_t job = (size_t)(t0 / DC) * a.heads + h;
+            const size_t job = (size_t)((kept + t0) / DC) * a.heads + h;
             const float *wr = p.W + (job * DC + wave * 16) * DP, *qr = qrows + (size_t)(t0 + wave * 16) * DP;
 #pragma unroll
             for (int s = 0; s < KS; ++s)
@@ -468,7 +474,7 @@ namespace llamql
         __syncthreads();
         for (int t0 = 0; t0 < ntok; t0 += DC)
         {
-            const size_t job = (size_t)(t0 / DC) * a.heads + h;
+            const size_t job = (size_t)((kept + t0) / DC) * a.heads + h;
             f32x8 P[DC / 32], kd[TS][DC / 32];
             const float *gamma = p.gamma + job * (DC + 4);
             const f32x4 carried = *reinterpret_cast<const f32x4 *>(gamma + wave * 16 + 4 * g);
@@ -522,7 +528,7 @@ namespace llamql
             {
                 const int t = t0 + wave * 16 + 4 * g + r;
                 if (t < ntok)
-                    p.o[((size_t)t * a.heads + h) * a.vdim + col] = out[r];
+                    p.o[((size_t)(kept + t) * a.heads + h) * a.vdim + col] = out[r];
             }
             __syncthreads();
         }
@@ -541,10 +547,11 @@ namespace llamql
         typedef T t4 __attribute__((ext_vector_type(4)));
         const llam_seq_delta_args &a = p.a;
         const int lane = threadIdx.x & 63, h = blockIdx.x * 4 + (threadIdx.x >> 6), t = blockIdx.y;
-        if (h >= a.heads)
+        const int e = p.entry + blockIdx.z;
+        if (h >= a.heads || t >= p.ntok[e])
             return;
-        const int r = p.row0[p.entry] + t;
-        const float *o = p.o + ((size_t)t * a.heads + h) * a.vdim;
+        const int r = p.row0[e] + t;
+        const float *o = p.o + ((size_t)(first_kept(p, blockIdx.z) + t) * a.heads + h) * a.vdim;
         const float *gate = a.d_proj + (size_t)r * a.ldp + 2 * a.kv_heads * a.dim + (a.heads + h) * a.vdim;
         float sum = 0.0f;
         for (int d = lane * 4; d < a.vdim; d += 256)
@@ -629,9 +636,9 @@ namespace llamql
                    : p.a.dim == 192 ? step_launch<T, 12>(fn, p, n, st) : step_launch<T, 16>(fn, p, n, st);
         }
         template <int DP>
-        bool walk_launch(const char *fn, const DeltaArgs &p, hipStream_t st)
+        bool walk_launch(const char *fn, const DeltaArgs &p, int n, hipStream_t st)
         {
-            hipLaunchKernelGGL(delta_walk_kernel<DP>, dim3(round_up(p.a.heads, 8) * (p.a.vdim / 16)), dim3(256), 0, st, p);
+            hipLaunchKernelGGL(delta_walk_kernel<DP>, dim3(round_up(p.a.heads, 8) * (p.a.vdim / 16), n), dim3(256), 0, st, p);
             return launched(fn);
         }
     } // namespace
@@ -643,7 +650,7 @@ extern "C" size_t llam_seq_delta_scratch_bytes(int max_rows, int heads, int kv_h
 {
     if (max_rows < 1 || heads < 1 || kv_heads < 1 || dim < 1 || vdim < 1)
         return 0;
-    return delta_scratch(max_rows, heads, kv_heads, dim, vdim).total;
+    return delta_scratch(round_up(max_rows, DC) + DELTA_MANY * DC, heads, kv_heads, dim, vdim).total; // (of several portions: whole chunks)
 }
 
 extern "C" bool llam_seq_delta_decode(const llam_seq_delta_args *a, const llam_seq_entries *e, int first, int n, int dtype,
@@ -663,48 +670,69 @@ extern "C" bool llam_seq_delta_decode(const llam_seq_delta_args *a, const llam_s
     return dtype == LLAM_SEQ_F32 ? step_dispatch<float>(fn, p, n, as_stream(stream)) : step_dispatch<bf16>(fn, p, n, as_stream(stream));
 }
 
+namespace
+{
+    bool delta_prefill(const char *fn, const DeltaArgs &p, int n, int ntok, int dtype, hipStream_t st)
+    {
+        const llam_seq_delta_args &a = p.a;
+        hipLaunchKernelGGL(delta_inputs_kernel, dim3(2 * a.kv_heads + a.heads, ceil_div(ntok, INPUT_TOKENS), n), dim3(256), 0, st, p);
+        if (!launched(fn))
+            return false;
+        if (a.taps > 1)
+        {
+            hipLaunchKernelGGL(delta_keep_kernel, dim3(ceil_div(p.channels, 1024), a.taps - 1, n), dim3(256), 0, st, p);
+            if (!launched(fn))
+                return false;
+        }
+        hipLaunchKernelGGL(delta_chunk_kernel, dim3(ceil_div(ntok, DC), a.heads, n), dim3(256), 0, st, p);
+        if (!launched(fn))
+            return false;
+        const bool ok = a.dim == 64 ? walk_launch<64>(fn, p, n, st) : a.dim == 128 ? walk_launch<128>(fn, p, n, st)
+                        : a.dim == 192 ? walk_launch<192>(fn, p, n, st) : walk_launch<256>(fn, p, n, st);
+        if (!ok)
+            return false;
+        const dim3 grid(ceil_div(a.heads, 4), ntok, n);
+        if (dtype == LLAM_SEQ_F32)
+            hipLaunchKernelGGL(delta_output_kernel<float>, grid, dim3(256), 0, st, p);
+        else
+            hipLaunchKernelGGL(delta_output_kernel<bf16>, grid, dim3(256), 0, st, p);
+        return launched(fn);
+    }
+} // namespace
+
 extern "C" bool llam_seq_delta_prefill(const llam_seq_delta_args *a, const llam_seq_entries *e, int entry, int ntok, void *d_scratch,
                                        size_t scratch_bytes, int dtype, int device_id, void *stream)
 {
+    return llam_seq_delta_prefill_many(a, e, entry, 1, ntok, ntok, d_scratch, scratch_bytes, dtype, device_id, stream);
+}
+
+extern "C" bool llam_seq_delta_prefill_many(const llam_seq_delta_args *a, const llam_seq_entries *e, int first, int n, int max_ntok, int rows,
+                                            void *d_scratch, size_t scratch_bytes, int dtype, int device_id, void *stream)
+{
     static const char *fn = "llam_seq_delta_prefill";
     DeltaArgs p;
-    if (ntok < 0 || entry < 0 || ntok > 65535)
-        return fail(fn, "bad size (entry=%d ntok=%d)", entry, ntok);
-    if (ntok == 0)
+    if (n < 0 || max_ntok < 0 || first < 0 || max_ntok > 65535 || rows < max_ntok)
+        return fail(fn, "bad size (first=%d n=%d ntok=%d rows=%d)", first, n, max_ntok, rows);
+    if (n == 0 || max_ntok == 0)
         return true;
     if (!delta_args(fn, a, e, dtype, p))
         return false;
-    const DeltaScratch at = delta_scratch(ntok, a->heads, a->kv_heads, a->dim, a->vdim);
+    p.many = n > 1;
+    p.rows = p.many ? round_up(rows, DC) + DELTA_MANY * DC : round_up(max_ntok, DC);
+    const DeltaScratch at = delta_scratch(p.rows, a->heads, a->kv_heads, a->dim, a->vdim);
     if (!d_scratch || at.total > scratch_bytes)
         return fail(fn, "scratch too small");
-    p.entry = entry, p.rows = round_up(ntok, DC);
     char *s = static_cast<char *>(d_scratch);
     auto place = [s](size_t offset) { return reinterpret_cast<float *>(s + offset); };
     p.q = place(at.q), p.k = place(at.k), p.v = place(at.v), p.beta = place(at.beta), p.log_decay = place(at.log_decay);
     p.P = place(at.P), p.U = place(at.U), p.W = place(at.W), p.kd = place(at.kd), p.gamma = place(at.gamma), p.o = place(at.o);
     if (!set_device(fn, device_id))
         return false;
-    hipStream_t st = as_stream(stream);
-    hipLaunchKernelGGL(delta_inputs_kernel, dim3(2 * a->kv_heads + a->heads, ceil_div(ntok, INPUT_TOKENS)), dim3(256), 0, st, p);
-    if (!launched(fn))
-        return false;
-    if (a->taps > 1)
+    for (int k = 0; k < n; k += DELTA_MANY)
     {
-        hipLaunchKernelGGL(delta_keep_kernel, dim3(ceil_div(p.channels, 1024), a->taps - 1), dim3(256), 0, st, p);
-        if (!launched(fn))
+        p.entry = first + k;
+        if (!delta_prefill(fn, p, n - k < DELTA_MANY ? n - k : DELTA_MANY, max_ntok, dtype, as_stream(stream)))
             return false;
     }
-    hipLaunchKernelGGL(delta_chunk_kernel, dim3(ceil_div(ntok, DC), a->heads), dim3(256), 0, st, p);
-    if (!launched(fn))
-        return false;
-    const bool ok = a->dim == 64 ? walk_launch<64>(fn, p, st) : a->dim == 128 ? walk_launch<128>(fn, p, st)
-                    : a->dim == 192 ? walk_launch<192>(fn, p, st) : walk_launch<256>(fn, p, st);
-    if (!ok)
-        return false;
-    const dim3 grid(ceil_div(a->heads, 4), ntok);
-    if (dtype == LLAM_SEQ_F32)
-        hipLaunchKernelGGL(delta_output_kernel<float>, grid, dim3(256), 0, st, p);
-    else
-        hipLaunchKernelGGL(delta_output_kernel<bf16>, grid, dim3(256), 0, st, p);
-    return launched(fn);
+    return true;
 }

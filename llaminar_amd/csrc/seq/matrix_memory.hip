@@ -18,6 +18,9 @@
 // is read in the same order.  In bf16, S and the gated values enter the products in three pieces,
 // i.e. as 32-bit values; q, k and v are bf16 (the output format of a projection).
 #include "seq_common.h"
+
+#include <algorithm>
+
 #include "llaminar_amd/seq_api.h"
 
 namespace llamql
@@ -34,18 +37,19 @@ namespace llamql
         float q_scale, gate_cap, eps;
         const int32_t *row0, *ntok, *slot, *pos;
         int entry;      // first entry of the call
+        bool many;      // several portions: a portion's chunks are kept from chunk row0 / LC + (its place among them) on
         double *ga, *a; // [rows][heads]: F_t - m_t, a_t
         float *mt;      // [rows][heads]: m_t
-        float *m0;      // [heads]: m before the portion
+        float *m0;      // [portions][heads]: m before the portion
         float *prod;    // [chunks][heads][LC][LC]
         float *num;     // [rows][heads][vdim + 16]; decoding: [entries][heads][splits][vdim + 16]
         int splits;     // decoding: workgroups along dim
         void *qk;       // T [2][heads][rows of the portion][dim]: scaled q, then k
         int qk_rows;
         // long portions: stretches of `stretch` chunks (0: the portion is one), what each adds to the memory and keeps of it
-        int stretch;
-        float *starts; // [stretches][heads][dim][vdim + 16]: the memory before the portion, then what stretch 0 .. adds
-        float *kept;   // [stretches][heads]: what is left of the memory after stretch 0 ..
+        int stretch, parts; // `parts` of them
+        float *starts; // [portions][stretches][heads][dim][vdim + 16]: the memory before the portion, then what stretch 0 .. adds
+        float *kept;   // [portions][stretches][heads]: what is left of the memory after stretch 0 ..
     };
 
     __device__ __forceinline__ void memory_gates(const MemoryArgs &p, const float *row, int h, float &i, float &f)
@@ -138,6 +142,13 @@ namespace llamql
         }
     }
 
+    // where the chunks of the call's portion ei are kept
+    template <int LC>
+    __device__ __forceinline__ int first_chunk(const MemoryArgs &p, int ei)
+    {
+        return p.many ? p.row0[p.entry + ei] / LC + ei : 0;
+    }
+
     // ---- prompts: gates -------------------------------------------------------------------------
     // A wavefront scans a chunk by itself; the running maximum passes from chunk to chunk by the chunks' totals.
     constexpr int GATE_WAVES = 16;
@@ -146,11 +157,11 @@ namespace llamql
         memory_gates_kernel(MemoryArgs p)
     {
         __shared__ double s_total[GATE_WAVES], s_top[GATE_WAVES];
-        const int h = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, e = p.entry;
+        const int h = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, e = p.entry + blockIdx.y;
         const int r0 = p.row0[e], n = p.ntok[e], slot = p.slot[e];
         float m = p.pos[e] == 0 ? 0.0f : p.m[slot * p.heads + h];
         if (threadIdx.x == 0)
-            p.m0[h] = m;
+            p.m0[blockIdx.y * p.heads + h] = m;
         for (int t0 = 0; t0 < n; t0 += GATE_WAVES * LC)
         {
             const int t = t0 + wave * LC + lane;
@@ -214,14 +225,15 @@ namespace llamql
         using O = Operand<T>;
         using V = typename O::V;
         const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = lane & 15, g = lane >> 4;
-        const int h = blockIdx.y, chunk = blockIdx.x, e = p.entry;
+        const int h = blockIdx.y, chunk = blockIdx.x, e = p.entry + blockIdx.z;
         const int n = p.ntok[e] - chunk * LC < LC ? p.ntok[e] - chunk * LC : LC;
         if (n <= 0)
             return;
         const int r0 = p.row0[e] + chunk * LC;
         auto row = [&](int t) { return p.proj + (size_t)(r0 + (t < n ? t : n - 1)) * p.ldp; };
         const float *q = row(wave * 16 + c) + h * p.dim + 8 * g;
-        T *qk = static_cast<T *>(p.qk) + ((size_t)h * p.qk_rows + chunk * LC + wave * 16 + c) * p.dim + 8 * g;
+        const int kept = chunk + first_chunk<LC>(p, blockIdx.z);
+        T *qk = static_cast<T *>(p.qk) + ((size_t)h * p.qk_rows + kept * LC + wave * 16 + c) * p.dim + 8 * g;
         const size_t k_after = (size_t)p.heads * p.qk_rows * p.dim;
         const float *k[LC / 16];
 #pragma unroll
@@ -246,7 +258,7 @@ namespace llamql
                         *reinterpret_cast<V *>(qk + k_after + s) = b[0];
                 }
         }
-        float *out = p.prod + ((size_t)chunk * p.heads + h) * LC * LC;
+        float *out = p.prod + ((size_t)kept * p.heads + h) * LC * LC;
 #pragma unroll
         for (int j = 0; j < LC / 16; ++j)
         {
@@ -291,7 +303,8 @@ namespace llamql
         extern __shared__ __attribute__((aligned(16))) char smem[];
         __shared__ float s_carry[LC], s_gate[LC]; // e^(F_t + m0 - m_t), e^(F_end + a_j - m_end)
         const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = lane & 15, g = lane >> 4;
-        const int h = blockIdx.y, e = p.entry;
+        const int h = blockIdx.y, ei = CUT ? (int)blockIdx.z / p.parts : (int)blockIdx.z, e = p.entry + ei;
+        const int chunk0 = first_chunk<LC>(p, ei);
         const int ntok = p.ntok[e], slot = p.slot[e], row0 = p.row0[e];
         const int dim = FULL ? 16 * DT : p.dim;
         const int ldv = p.vdim + 16, ld = dim + LPAD;
@@ -324,11 +337,12 @@ namespace llamql
                         to[(size_t)(16 * t + 4 * g + r) * ldv] = S[t][r];
                 }
         };
-        const int part = CUT ? blockIdx.z : 0, first = CUT ? part * p.stretch * LC : 0; // this stretch and its first token
-        const bool last = !CUT || part + 1 == (int)gridDim.z;
+        const int part = CUT ? (int)blockIdx.z - ei * p.parts : 0, first = CUT ? part * p.stretch * LC : 0; // this stretch and its first token
+        const bool last = !CUT || part + 1 == p.parts;
         const int stop = last || first + p.stretch * LC > ntok ? ntok : first + p.stretch * LC;
         const size_t part_floats = (size_t)p.heads * dim * ldv;
-        float *starts = p.starts + (size_t)h * dim * ldv + (live ? col : 0);
+        float *starts = p.starts + (size_t)ei * p.parts * part_floats + (size_t)h * dim * ldv + (live ? col : 0);
+        float *part_kept = p.kept + (size_t)ei * p.parts * p.heads + h;
 #pragma unroll
         for (int t = 0; t < DT; ++t)
             S[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
@@ -351,7 +365,7 @@ namespace llamql
                 load_state(CUT && p.stretch ? starts : state);
             for (int i = 1; CUT && i <= part; ++i)
             {
-                const float kept = p.kept[(i - 1) * p.heads + h];
+                const float kept = part_kept[(i - 1) * p.heads];
                 const float *add = starts + i * part_floats;
 #pragma unroll
                 for (int t = 0; t < DT; ++t)
@@ -365,7 +379,7 @@ namespace llamql
         }
 
         const int srow = threadIdx.x / TPR, sseg = threadIdx.x % TPR, pieces = dim * (int)sizeof(T) / 16;
-        const T *qrows = static_cast<const T *>(p.qk) + (size_t)h * p.qk_rows * dim;
+        const T *qrows = static_cast<const T *>(p.qk) + ((size_t)h * p.qk_rows + (size_t)chunk0 * LC) * dim;
         const T *krows = qrows + (size_t)p.heads * p.qk_rows * dim;
         u32x4 hq[AHEAD ? LOADS : 1], hk[AHEAD ? LOADS : 1];
         f32x8 hv[LC / 32];
@@ -407,7 +421,7 @@ namespace llamql
         };
         if (first < ntok)
             request(first);
-        float m0 = first == 0 ? p.m0[h] : first < ntok ? p.mt[(size_t)(row0 + first - 1) * p.heads + h] : 0.0f;
+        float m0 = first == 0 ? p.m0[ei * p.heads + h] : first < ntok ? p.mt[(size_t)(row0 + first - 1) * p.heads + h] : 0.0f;
         float kept = 1.0f;
         for (int t0 = first; t0 < stop; t0 += LC)
         {
@@ -455,7 +469,7 @@ namespace llamql
                 x[s] = hv[s];
             __syncthreads();
             // the chunk's products, 16 rows at a time (a row block needs columns up to its own)
-            const float *prod = p.prod + ((size_t)(t0 / LC) * p.heads + h) * LC * LC;
+            const float *prod = p.prod + ((size_t)(chunk0 + t0 / LC) * p.heads + h) * LC * LC;
             f32x8 w[LC / 16][LC / 32];
 #pragma unroll
             for (int i = 0; i < LC / 16; ++i)
@@ -578,7 +592,7 @@ namespace llamql
             if (live)
                 store_state(starts + (part + 1) * part_floats);
             if (blockIdx.x == 0 && threadIdx.x == 0)
-                p.kept[part * p.heads + h] = kept;
+                part_kept[part * p.heads] = kept;
         }
         else if (live && last)
             store_state(state);
@@ -592,7 +606,9 @@ namespace llamql
     {
         __shared__ float s_sum[2];
         const int h = blockIdx.x;
-        const int e = p.entry + (DECODE ? blockIdx.y : 0);
+        const int e = p.entry + (DECODE ? blockIdx.y : blockIdx.z);
+        if (!DECODE && (int)blockIdx.y >= p.ntok[e])
+            return;
         const int r = DECODE ? p.row0[e] : p.row0[e] + blockIdx.y;
         const float *row = p.proj + (size_t)r * p.ldp;
         const int ldv = p.vdim + 16;
@@ -649,6 +665,7 @@ namespace llamql
     {
         constexpr int LC16 = 64, LC32 = 32; // chunk lengths of the two number formats
         constexpr int CUT_TILES = 16;                    // 16-row tiles of S up to which a portion is cut into stretches
+        constexpr int MANY = 16;                         // portions of a launch at most
         constexpr int STRETCHES = 8, STRETCH_MIN = 3; // stretches of a portion at most, chunks of one at least
         constexpr int STEP_SPLIT_ENTRIES = 32; // sequences up to which a decoding step splits the rows of S (in at most 8)
 
@@ -676,11 +693,12 @@ namespace llamql
             s.ga = take((size_t)rows * heads * 8);
             s.a = take((size_t)rows * heads * 8);
             s.mt = take((size_t)rows * heads * 4);
-            s.m0 = take((size_t)heads * 4);
-            s.prod = take((size_t)round_up(rows, LC16) * heads * LC16 * 4);
+            s.m0 = take((size_t)MANY * heads * 4);
+            const size_t kept = (size_t)round_up(rows, LC16) + MANY * LC16; // rows of whole chunks, of several portions
+            s.prod = take(kept * heads * LC16 * 4);
             const size_t outs = (size_t)(rows > STEP_SPLIT_ENTRIES * 8 ? rows : STEP_SPLIT_ENTRIES * 8);
             s.num = take(outs * heads * (vdim + 16) * 4);
-            s.qk = take((size_t)2 * heads * round_up(rows, LC16) * dim * 4);
+            s.qk = take((size_t)2 * heads * kept * dim * 4);
             const int stretches = memory_stretches(rows, dim, LC32); // (the shorter chunks: the most that any portion has)
             s.starts = take(stretches > 1 ? (size_t)stretches * heads * dim * (vdim + 16) * 4 : 0);
             s.kept = take((size_t)stretches * heads * 4);
@@ -724,58 +742,59 @@ namespace llamql
             p.ga = reinterpret_cast<double *>(s + at.ga), p.a = reinterpret_cast<double *>(s + at.a);
             p.mt = reinterpret_cast<float *>(s + at.mt), p.m0 = reinterpret_cast<float *>(s + at.m0);
             p.prod = reinterpret_cast<float *>(s + at.prod), p.num = reinterpret_cast<float *>(s + at.num);
-            p.qk = s + at.qk, p.qk_rows = rows;
+            p.qk = s + at.qk, p.qk_rows = rows + MANY * LC16;
+            p.parts = memory_stretches(rows, p.dim, LC32); // (as many as there is room for)
             p.starts = reinterpret_cast<float *>(s + at.starts), p.kept = reinterpret_cast<float *>(s + at.kept);
         }
 
         template <typename T, int LC, int DT, bool FULL, bool CUT, bool SUM>
-        bool chunk_launch_one(const char *fn, const MemoryArgs &p, int stretches, hipStream_t st)
+        bool chunk_launch_one(const char *fn, const MemoryArgs &p, int n, hipStream_t st)
         {
             static LdsGrant grant;
             const size_t lds = (size_t)2 * LC * (p.dim + 16 / sizeof(T)) * sizeof(T);
             const auto kernel = &memory_chunk_kernel<T, LC, DT, FULL, CUT, SUM>;
             if (lds > 48 * 1024 && allow_lds(grant, reinterpret_cast<const void *>(kernel), 140 * 1024) != hipSuccess)
                 return fail(fn, "cannot reserve %zu bytes of LDS", lds);
-            hipLaunchKernelGGL(kernel, dim3(ceil_div(p.vdim + 16, 64), p.heads, stretches), dim3(256), lds, st, p);
+            hipLaunchKernelGGL(kernel, dim3(ceil_div(p.vdim + 16, 64), p.heads, p.parts * n), dim3(256), lds, st, p);
             return launched(fn);
         }
         template <typename T, int LC, int DT, bool FULL>
-        bool chunk_launch_as(const char *fn, const MemoryArgs &p, int stretches, hipStream_t st)
+        bool chunk_launch_as(const char *fn, const MemoryArgs &p, int n, hipStream_t st)
         {
             if constexpr (DT <= CUT_TILES)
-                return (stretches == 1 || chunk_launch_one<T, LC, DT, FULL, true, true>(fn, p, stretches, st)) &&
-                       chunk_launch_one<T, LC, DT, FULL, true, false>(fn, p, stretches, st);
+                return (p.parts == 1 || chunk_launch_one<T, LC, DT, FULL, true, true>(fn, p, n, st)) &&
+                       chunk_launch_one<T, LC, DT, FULL, true, false>(fn, p, n, st);
             else
-                return chunk_launch_one<T, LC, DT, FULL, false, false>(fn, p, 1, st);
+                return chunk_launch_one<T, LC, DT, FULL, false, false>(fn, p, n, st);
         }
         template <typename T, int LC, int DT>
-        bool chunk_launch(const char *fn, const MemoryArgs &p, int stretches, hipStream_t st)
+        bool chunk_launch(const char *fn, const MemoryArgs &p, int n, hipStream_t st)
         {
             if constexpr (sizeof(T) == 2)
             {
                 if (p.dim == 16 * DT)
-                    return chunk_launch_as<T, LC, DT, true>(fn, p, stretches, st);
+                    return chunk_launch_as<T, LC, DT, true>(fn, p, n, st);
             }
-            return chunk_launch_as<T, LC, DT, false>(fn, p, stretches, st);
+            return chunk_launch_as<T, LC, DT, false>(fn, p, n, st);
         }
         template <typename T, int LC>
-        bool prefill_run(const char *fn, MemoryArgs p, int ntok, int cus, hipStream_t st)
+        bool prefill_run(const char *fn, MemoryArgs p, int n, int ntok, int cus, hipStream_t st)
         {
-            // (a workgroup fills a compute unit: no second round of them)
-            const int most = cus / (ceil_div(p.vdim + 16, 64) * p.heads), can = memory_stretches(ntok, p.dim, LC);
-            const int stretches = most < 2 ? 1 : can < most ? can : most;
-            p.stretch = stretches > 1 ? ceil_div(ceil_div(ntok, LC), stretches) : 0;
-            hipLaunchKernelGGL(memory_gates_kernel<LC>, dim3(p.heads), dim3(GATE_WAVES * 64), 0, st, p);
+            // (a workgroup fills a compute unit: no second round of them; and as many stretches as the scratch has room for)
+            const int most = std::min(cus / (ceil_div(p.vdim + 16, 64) * p.heads), p.parts) / n, can = memory_stretches(ntok, p.dim, LC);
+            p.parts = std::max(1, std::min(can, most));
+            p.stretch = p.parts > 1 ? ceil_div(ceil_div(ntok, LC), p.parts) : 0;
+            hipLaunchKernelGGL(memory_gates_kernel<LC>, dim3(p.heads, n), dim3(GATE_WAVES * 64), 0, st, p);
             if (!launched(fn))
                 return false;
-            hipLaunchKernelGGL((memory_product_kernel<T, LC>), dim3(ceil_div(ntok, LC), p.heads), dim3(LC * 4), 0, st, p);
+            hipLaunchKernelGGL((memory_product_kernel<T, LC>), dim3(ceil_div(ntok, LC), p.heads, n), dim3(LC * 4), 0, st, p);
             if (!launched(fn))
                 return false;
-            const bool ok = p.dim <= 64 ? chunk_launch<T, LC, 4>(fn, p, stretches, st) : p.dim <= 128 ? chunk_launch<T, LC, 8>(fn, p, stretches, st)
-                            : p.dim <= 256 ? chunk_launch<T, LC, 16>(fn, p, stretches, st) : chunk_launch<T, LC, 32>(fn, p, stretches, st);
+            const bool ok = p.dim <= 64 ? chunk_launch<T, LC, 4>(fn, p, n, st) : p.dim <= 128 ? chunk_launch<T, LC, 8>(fn, p, n, st)
+                            : p.dim <= 256 ? chunk_launch<T, LC, 16>(fn, p, n, st) : chunk_launch<T, LC, 32>(fn, p, n, st);
             if (!ok)
                 return false;
-            hipLaunchKernelGGL((memory_output_kernel<T, false>), dim3(p.heads, ntok), dim3(128), 0, st, p);
+            hipLaunchKernelGGL((memory_output_kernel<T, false>), dim3(p.heads, ntok, n), dim3(128), 0, st, p);
             return launched(fn);
         }
         template <typename T>
@@ -823,20 +842,33 @@ extern "C" bool llam_seq_memory_decode(const llam_seq_memory_args *a, const llam
 extern "C" bool llam_seq_memory_prefill(const llam_seq_memory_args *a, const llam_seq_entries *e, int entry, int ntok,
                                         void *d_scratch, size_t scratch_bytes, int dtype, int device_id, void *stream)
 {
+    return llam_seq_memory_prefill_many(a, e, entry, 1, ntok, ntok, d_scratch, scratch_bytes, dtype, device_id, stream);
+}
+
+extern "C" bool llam_seq_memory_prefill_many(const llam_seq_memory_args *a, const llam_seq_entries *e, int first, int n, int max_ntok,
+                                             int rows, void *d_scratch, size_t scratch_bytes, int dtype, int device_id, void *stream)
+{
     static const char *fn = "llam_seq_memory_prefill";
     MemoryArgs p;
-    if (ntok < 0 || entry < 0 || ntok > 65535)
-        return fail(fn, "bad size (entry=%d ntok=%d)", entry, ntok);
-    if (ntok == 0)
+    if (n < 0 || max_ntok < 0 || first < 0 || max_ntok > 65535 || rows < max_ntok)
+        return fail(fn, "bad size (first=%d n=%d ntok=%d rows=%d)", first, n, max_ntok, rows);
+    if (n == 0 || max_ntok == 0)
         return true;
     if (!memory_args(fn, a, e, d_scratch, dtype, p))
         return false;
-    if (llam_seq_memory_scratch_bytes(ntok, p.heads, p.dim, p.vdim) > scratch_bytes)
+    if (llam_seq_memory_scratch_bytes(rows, p.heads, p.dim, p.vdim) > scratch_bytes)
         return fail(fn, "scratch too small");
-    p.entry = entry;
     place_scratch(p, d_scratch, scratch_bytes);
     if (!set_device(fn, device_id))
         return false;
-    return dtype == LLAM_SEQ_F32 ? prefill_run<float, LC32>(fn, p, ntok, cu_count(device_id), as_stream(stream))
-                                 : prefill_run<bf16, LC16>(fn, p, ntok, cu_count(device_id), as_stream(stream));
+    p.many = n > 1;
+    for (int k = 0; k < n; k += MANY)
+    {
+        const int some = n - k < MANY ? n - k : MANY;
+        p.entry = first + k;
+        if (!(dtype == LLAM_SEQ_F32 ? prefill_run<float, LC32>(fn, p, some, max_ntok, cu_count(device_id), as_stream(stream))
+                                    : prefill_run<bf16, LC16>(fn, p, some, max_ntok, cu_count(device_id), as_stream(stream))))
+            return false;
+    }
+    return true;
 }

@@ -134,12 +134,38 @@ namespace
         llam_seq_entries entries() const { return {entry(0), entry(1), entry(2), entry(3)}; }
     };
 
-    // what a step looks like to the layers: `single` one-token entries first, then the portions
+    // what a step looks like to the layers: `single` one-token entries first, then the portions, in runs
     struct Step
     {
         int M = 0, single = 0;
         int max_len = 1; // bound on the length of the one-token entries' sequences
-        std::vector<std::pair<int, int>> portions; // (tokens, length afterwards) of entries single ..
+        // runs of portions that are launched together: entries first .. first + n - 1, the most tokens and the longest afterwards
+        struct Run
+        {
+            int first, n, ntok, len;
+        };
+        std::vector<Run> runs;
+        long run_rows = 0; // tokens of the last one
+
+        // Another portion.  A launch of several takes as long as its longest, where a launch for each has few workgroups and
+        // pays for the latencies of its chain (eight prompts of 251 tokens and two steps, width 2048: Kogilix 5.0 -> 3.9 ms,
+        // Bosirax 3.55 -> 2.67); a grid is made for the longest, so a portion that would leave two thirds of it empty starts a run of
+        // its own.
+        void add(int entry, int ntok, int len)
+        {
+            if (!runs.empty())
+            {
+                Run &r = runs.back();
+                if ((long)(r.n + 1) * std::max(r.ntok, ntok) <= 3 * (run_rows + ntok))
+                {
+                    ++r.n, run_rows += ntok;
+                    r.ntok = std::max(r.ntok, ntok), r.len = std::max(r.len, len);
+                    return;
+                }
+            }
+            runs.push_back({entry, 1, ntok, len});
+            run_rows = ntok;
+        }
         const int32_t *row_slot = nullptr, *row_pos = nullptr;
     };
 
@@ -220,9 +246,9 @@ namespace
             if (s.single && !forward(fn, llam_seq_attention(&a, md.q, &e, 0, s.single, 1, s.max_len, md.mix, ldm, md.lat_scratch, md.lat_floats,
                                                             c.dtype, c.device_id, st)))
                 return false;
-            for (size_t k = 0; k < s.portions.size(); ++k)
-                if (!forward(fn, llam_seq_attention(&a, md.q, &e, s.single + (int)k, 1, s.portions[k].first, s.portions[k].second, md.mix, ldm,
-                                                    md.lat_scratch, md.lat_floats, c.dtype, c.device_id, st)))
+            for (const Step::Run &r : s.runs)
+                if (!forward(fn, llam_seq_attention(&a, md.q, &e, r.first, r.n, r.ntok, r.len, md.mix, ldm, md.lat_scratch, md.lat_floats,
+                                                    c.dtype, c.device_id, st)))
                     return false;
             return add_output(w, s);
         }
@@ -240,9 +266,9 @@ namespace
             const llam_seq_entries e = md.entries();
             if (s.single && !forward(fn, llam_seq_delta_decode(&a, &e, 0, s.single, c.dtype, c.device_id, st)))
                 return false;
-            for (size_t k = 0; k < s.portions.size(); ++k)
-                if (!forward(fn, llam_seq_delta_prefill(&a, &e, s.single + (int)k, s.portions[k].first, md.scratch, md.scratch_bytes, c.dtype,
-                                                        c.device_id, st)))
+            for (const Step::Run &r : s.runs)
+                if (!forward(fn, llam_seq_delta_prefill_many(&a, &e, r.first, r.n, r.ntok, s.M, md.scratch, md.scratch_bytes, c.dtype,
+                                                             c.device_id, st)))
                     return false;
             return add_output(w, s);
         }
@@ -266,10 +292,9 @@ namespace
             if (s.single && !forward(fn, llam_seq_latent_attention(md.qlat, cache, &e, 0, s.single, 1, s.max_len, H, rp, c.cap, w.scale,
                                                                    md.olat, md.lat_scratch, md.lat_floats, c.dtype, c.device_id, st)))
                 return false;
-            for (size_t k = 0; k < s.portions.size(); ++k)
-                if (!forward(fn, llam_seq_latent_attention(md.qlat, cache, &e, s.single + (int)k, 1, s.portions[k].first,
-                                                           s.portions[k].second, H, rp, c.cap, w.scale, md.olat, md.lat_scratch,
-                                                           md.lat_floats, c.dtype, c.device_id, st)))
+            for (const Step::Run &r : s.runs)
+                if (!forward(fn, llam_seq_latent_attention(md.qlat, cache, &e, r.first, r.n, r.ntok, r.len, H, rp, c.cap, w.scale, md.olat,
+                                                           md.lat_scratch, md.lat_floats, c.dtype, c.device_id, st)))
                     return false;
             return linear(md.olat, H * rp, w.w_uv, vp, rp, md.mix, mix_columns(w), LLAM_SEQ_OUT_ELEM, s.M, nullptr, nullptr, 0, nullptr, H,
                           rp, (long)vp * rp, vp) &&
@@ -290,9 +315,9 @@ namespace
             const llam_seq_entries e = md.entries();
             if (s.single && !forward(fn, llam_seq_memory_decode(&a, &e, 0, s.single, md.scratch, md.scratch_bytes, c.dtype, c.device_id, st)))
                 return false;
-            for (size_t k = 0; k < s.portions.size(); ++k)
-                if (!forward(fn, llam_seq_memory_prefill(&a, &e, s.single + (int)k, s.portions[k].first, md.scratch, md.scratch_bytes,
-                                                         c.dtype, c.device_id, st)))
+            for (const Step::Run &r : s.runs)
+                if (!forward(fn, llam_seq_memory_prefill_many(&a, &e, r.first, r.n, r.ntok, s.M, md.scratch, md.scratch_bytes, c.dtype,
+                                                              c.device_id, st)))
                     return false;
             return add_output(w, s);
         }
@@ -698,8 +723,8 @@ extern "C" bool llam_seqm_forward(void *model, int n, const int32_t *h_slot, con
     for (int e = 0; e < n; ++e)
         if (h_ntok[e] > 1)
         {
+            s.add(placed, h_ntok[e], h_pos[e] + h_ntok[e]);
             place(e);
-            s.portions.emplace_back(h_ntok[e], h_pos[e] + h_ntok[e]);
         }
     s.row_slot = md->row_slot();
     s.row_pos = md->row_pos();

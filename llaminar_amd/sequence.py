@@ -112,6 +112,8 @@ SIGNATURES = {
     "llam_seq_delta_decode": (c_bool, [POINTER(DeltaArgs), POINTER(Entries), c_int, c_int, c_int, c_int, c_void_p]),
     "llam_seq_delta_prefill": (c_bool, [POINTER(DeltaArgs), POINTER(Entries), c_int, c_int, c_void_p, c_size_t, c_int, c_int,
                                         c_void_p]),
+    "llam_seq_delta_prefill_many": (c_bool, [POINTER(DeltaArgs), POINTER(Entries), c_int, c_int, c_int, c_int, c_void_p, c_size_t,
+                                             c_int, c_int, c_void_p]),
     "llam_seq_latent_append": (c_bool, [c_void_p, c_int, c_void_p, c_float, c_int, c_void_p, c_void_p, c_void_p, c_int,
                                         c_int, c_int, c_int, c_int, c_void_p]),
     "llam_seq_latent_scratch_floats": (c_size_t, [c_int, c_int, c_int, c_int, c_int]),
@@ -122,6 +124,8 @@ SIGNATURES = {
                                         c_int, c_void_p]),
     "llam_seq_memory_prefill": (c_bool, [POINTER(MemoryArgs), POINTER(Entries), c_int, c_int, c_void_p, c_size_t, c_int,
                                          c_int, c_void_p]),
+    "llam_seq_memory_prefill_many": (c_bool, [POINTER(MemoryArgs), POINTER(Entries), c_int, c_int, c_int, c_int, c_void_p, c_size_t,
+                                              c_int, c_int, c_void_p]),
     "llam_seq_experts_scratch_bytes": (c_size_t, [c_int, c_int, c_int, c_int, c_int, c_int]),
     "llam_seq_experts": (c_bool, [POINTER(ExpertsArgs), c_int, c_void_p, c_size_t, c_int, c_int, c_void_p]),
     "llam_seq_record": (c_bool, [c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_void_p]),

@@ -150,6 +150,29 @@ def test_unequal_requests_in_one_step(whole, whole_f32):
         check(np.concatenate(got[b]), want[b], "float32", note=f"sequence {b}")
 
 
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_many_portions_in_one_launch(dtype):
+    """Twenty prompts of like lengths in one step (more than a launch takes), longer and shorter ones that start launches of their own,
+    single tokens between them, then second portions onto what the first left: each sequence against itself alone."""
+    cfg = sm.config(sm.mlstm(), sm.latent(), sm.mlstm(heads=2, dim=300, vdim=40))
+    t = sm.random_weights(cfg, 12)
+    lengths = [(33 + 7 * b % 40, 30 + 5 * b % 41) for b in range(20)] + [(400, 210), (2, 3), (70, 260), (1, 66), (300, 1), (1, 1)]
+    seqs = [tokens_of(cfg, sum(n), seed=b) for b, n in enumerate(lengths)]
+    rows = max(sum(n[k] for n in lengths) for k in range(2))
+    model = load(cfg, t, dtype, slots=len(seqs), max_rows=rows)
+    got = [[] for _ in seqs]
+    for k in range(2):
+        entries = [(b, sum(n[:k]), seqs[b][sum(n[:k]):sum(n[:k + 1])]) for b, n in enumerate(lengths)]
+        logits, row = model.forward(entries, range(sum(n[k] for n in lengths))), 0
+        for b, n in enumerate(lengths):
+            got[b].append(logits[row:row + n[k]])
+            row += n[k]
+    plain = t.plain()
+    for b, tokens in enumerate(seqs):
+        check(np.concatenate(got[b]), so.kogilix(cfg, plain, tokens), dtype, note=f"sequence {b}")
+    model.close()
+
+
 def test_a_slot_used_again_starts_afresh(whole, whole_f32):
     t, tokens, want = whole
     other = tokens_of(WHOLE, 200, seed=9)
