@@ -122,6 +122,12 @@ size_t llam_seq_latent_scratch_floats(int max_rows, int slots, int heads, int ra
 bool llam_seq_latent_attention(const void *d_q, const void *d_cache, const llam_seq_entries *e, int first, int n,
                                int max_ntok, int max_len, int heads, int rank, int cap, float scale, void *d_o,
                                float *d_scratch, size_t scratch_floats, int dtype, int device_id, void *stream);
+/* The same for the portions of a step, entries first .. first + n - 1 of ntok[i] tokens whose sequences have len[i] positions
+ * afterwards (host arrays).  Each is cut up as it would be in a call of its own, so that its outputs are the same bits whatever
+ * portions lie beside it; those that can share a launch do. */
+bool llam_seq_latent_portions(const void *d_q, const void *d_cache, const llam_seq_entries *e, int first, int n, const int *ntok,
+                              const int *len, int heads, int rank, int cap, float scale, void *d_o, float *d_scratch,
+                              size_t scratch_floats, int dtype, int device_id, void *stream);
 
 /* Matrix-memory recurrence (per head a dim x vdim memory S, a vector n and a running maximum m):
  *   i = cap tanh(i_raw / cap), f = logsigmoid(cap tanh(f_raw / cap)), m' = max(f + m, i)
@@ -186,6 +192,10 @@ size_t llam_seq_attention_scratch_floats(int vdim);
 bool llam_seq_attention(const llam_seq_attention_args *a, const void *d_q, const llam_seq_entries *e, int first, int n,
                         int max_ntok, int max_len, void *d_o, int ldo, float *d_scratch, size_t scratch_floats, int dtype,
                         int device_id, void *stream);
+/* The portions of a step, as in llam_seq_latent_portions. */
+bool llam_seq_attention_portions(const llam_seq_attention_args *a, const void *d_q, const llam_seq_entries *e, int first, int n,
+                                 const int *ntok, const int *len, void *d_o, int ldo, float *d_scratch, size_t scratch_floats,
+                                 int dtype, int device_id, void *stream);
 
 /* Gated delta rule (per head a dim x vdim state S; heads / kv_heads heads share q and k):
  *   q, k, v pass a causal convolution over `taps` tokens per channel and silu; q and k become unit vectors

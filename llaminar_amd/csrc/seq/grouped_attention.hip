@@ -51,6 +51,13 @@ namespace llamql
         return v;
     }
 
+    // How an entry's positions are cut: positions of a stretch, stretches, and its partial results: rows before them and of a stretch.
+    struct AttentionCut
+    {
+        int stretch, nsplit, first, rows;
+    };
+    constexpr int ATT_MANY = 16; // portions of a launch at most
+
     struct AttentionArgs
     {
         const void *q, *k, *v;
@@ -61,7 +68,13 @@ namespace llamql
         void *o;
         int ldo;
         float *part_o, *part_ml;
+        bool own; // every entry has its own cut; else all have that of the call
+        AttentionCut cut[ATT_MANY];
     };
+    __device__ __forceinline__ AttentionCut attention_cut(const AttentionArgs &p, int ei)
+    {
+        return p.own ? p.cut[ei] : AttentionCut{p.stretch, p.nsplit, ei * p.groups * p.nsplit * p.rcap, p.rcap};
+    }
 
     // first position that position i sees
     __device__ __forceinline__ int att_low(int i, int chunk) { return i / chunk * chunk; }
@@ -99,10 +112,11 @@ namespace llamql
         const int last_row = rb + 16 * RG * WR - 1 < R ? rb + 16 * RG * WR - 1 : R - 1;
         const int pfirst = pos0 + rb / per, kmax = pos0 + last_row / per; // positions of the block's tokens
         const int low0 = att_low(pfirst, p.chunk);
-        const int k0 = low0 + split * p.stretch;
+        const AttentionCut cut = attention_cut(p, ei);
+        const int k0 = low0 + split * cut.stretch;
         if (k0 > kmax)
             return;
-        const int k1 = k0 + p.stretch < kmax + 1 ? k0 + p.stretch : kmax + 1;
+        const int k1 = k0 + cut.stretch < kmax + 1 ? k0 + cut.stretch : kmax + 1;
 
         const size_t head = (size_t)p.slot[e] * p.groups + kv;
         const u32x4 *kcache = static_cast<const u32x4 *>(p.k) + head * p.ring * KP;
@@ -320,7 +334,7 @@ namespace llamql
             const int tok = row / per;
             return static_cast<T *>(p.o) + (size_t)(row0 + tok) * p.ldo + (size_t)(kv * per + row - tok * per) * DV;
         };
-        const size_t part = ((size_t)blockIdx.z * p.nsplit + split) * p.rcap;
+        const size_t part = cut.first + (size_t)(kv * cut.nsplit + split) * cut.rows;
 
         if constexpr (WR == 1)
         {
@@ -352,11 +366,11 @@ namespace llamql
                     f[w] = att_exp(s_ml[w][row][0] - base);
                     L += f[w] * s_ml[w][row][1];
                 }
-                const float inv = p.nsplit == 1 ? 1.0f / L : 1.0f;
+                const float inv = cut.nsplit == 1 ? 1.0f / L : 1.0f;
 #pragma unroll
                 for (int w = 0; w < 4; ++w)
                     s_f[w][row] = f[w] * inv;
-                if (p.nsplit > 1 && rb + row < R)
+                if (cut.nsplit > 1 && rb + row < R)
                 {
                     p.part_ml[(part + rb + row) * 2] = M;
                     p.part_ml[(part + rb + row) * 2 + 1] = L;
@@ -372,7 +386,7 @@ namespace llamql
 #pragma unroll
                 for (int w = 0; w < 4; ++w)
                     y = y + *reinterpret_cast<const f32x4 *>(s_o + (w * 16 + row) * OLD + d) * s_f[w][row];
-                if (p.nsplit == 1)
+                if (cut.nsplit == 1)
                     *reinterpret_cast<t4 *>(result(rb + row) + d) = __builtin_convertvector(y, t4);
                 else
                     *reinterpret_cast<f32x4 *>(p.part_o + (part + rb + row) * DV + d) = y;
@@ -390,12 +404,12 @@ namespace llamql
 #pragma unroll
             for (int t = 0; t < NT; ++t)
             {
-                if (p.nsplit == 1)
+                if (cut.nsplit == 1)
                     *reinterpret_cast<t4 *>(out + 16 * t + 4 * g) = __builtin_convertvector(acc[r][t] * inv, t4);
                 else
                     *reinterpret_cast<f32x4 *>(p.part_o + (part + row) * DV + 16 * t + 4 * g) = acc[r][t];
             }
-            if (p.nsplit > 1 && g == 0)
+            if (cut.nsplit > 1 && g == 0)
             {
                 p.part_ml[(part + row) * 2] = m[r];
                 p.part_ml[(part + row) * 2 + 1] = l[r];
@@ -413,20 +427,21 @@ namespace llamql
         __shared__ __attribute__((aligned(16))) float s_y[TEAMS][DV];
         const int ei = blockIdx.y / p.groups, kv = blockIdx.y - ei * p.groups, e = p.first + ei, row = blockIdx.x;
         const int per = p.heads / p.groups;
-        if (row >= p.ntok[e] * per)
+        const AttentionCut cut = attention_cut(p, ei);
+        if (row >= p.ntok[e] * per || cut.nsplit == 1)
             return;
         const int tok = row / per, pos0 = p.pos[e];
         const int low = att_low(pos0 + row / p.block_rows * p.block_rows / per, p.chunk); // of the row's block
-        int used = (pos0 + tok - low) / p.stretch + 1;
-        used = used < p.nsplit ? used : p.nsplit;
-        const size_t at = (size_t)blockIdx.y * p.nsplit * p.rcap + row;
+        int used = (pos0 + tok - low) / cut.stretch + 1;
+        used = used < cut.nsplit ? used : cut.nsplit;
+        const size_t at = cut.first + (size_t)kv * cut.nsplit * cut.rows + row;
         const int team = threadIdx.x / LANES, d = threadIdx.x % LANES * 4, lane = threadIdx.x & 63;
         // every wavefront works out the factors, a stretch a lane
         float M = -INFINITY, L = 0.0f;
         f32x4 y = {0.0f, 0.0f, 0.0f, 0.0f};
         for (int s0 = 0; s0 < used; s0 += 64)
         {
-            const size_t k = (at + (size_t)(s0 + lane < used ? s0 + lane : s0) * p.rcap) * 2;
+            const size_t k = (at + (size_t)(s0 + lane < used ? s0 + lane : s0) * cut.rows) * 2;
             const float m = s0 + lane < used ? p.part_ml[k] : -INFINITY, l = p.part_ml[k + 1];
             float top = fmaxf(m, M);
 #pragma unroll
@@ -445,7 +460,7 @@ namespace llamql
                     const bool in = s + j * TEAMS < n;
                     const int mine = in ? s + j * TEAMS : 0;
                     const float w = __shfl(f, mine, 64);
-                    const f32x4 o = *reinterpret_cast<const f32x4 *>(p.part_o + (at + (size_t)(s0 + mine) * p.rcap) * DV + d);
+                    const f32x4 o = *reinterpret_cast<const f32x4 *>(p.part_o + (at + (size_t)(s0 + mine) * cut.rows) * DV + d);
                     y = y + o * (in ? w : 0.0f);
                 }
         }
@@ -563,40 +578,104 @@ namespace llamql
             hipLaunchKernelGGL((attention_kernel<T, DK, DV, WR, RG>), dim3(row_blocks, p.nsplit, z), dim3(ATT_THREADS), lds, st, p);
             return launched(fn);
         }
+        // how a call of n entries is cut up
+        struct AttentionPlan
+        {
+            bool narrow; // a block of 16 rows that the wavefronts share
+            int block_rows, row_blocks, stretch, nsplit;
+        };
         template <typename T, int DK, int DV>
-        bool attention_rows(const char *fn, AttentionArgs &p, int n, int max_ntok, int max_len, size_t scratch_floats, hipStream_t st)
+        AttentionPlan attention_plan(const AttentionArgs &p, int n, int max_ntok, int max_len)
         {
             constexpr bool NARROW = sizeof(T) == 2 || DK + DV <= 256; // positions dealt to the wavefronts fit the LDS
             constexpr int RG = sizeof(T) == 2 && DK + DV <= 384 ? 2 : 1; // (registers)
+            AttentionPlan pl{};
             const int per = p.heads / p.groups, R = max_ntok * per;
-            const bool narrow = NARROW && R <= 16;
-            p.block_rows = narrow ? 16 : 64 * RG;
-            p.rcap = R;
-            const int row_blocks = ceil_div(R, p.block_rows), z = n * p.groups;
-            const int pt = narrow ? 128 : 64;
+            pl.narrow = NARROW && R <= 16;
+            pl.block_rows = pl.narrow ? 16 : 64 * RG;
+            pl.row_blocks = ceil_div(R, pl.block_rows);
+            const int pt = pl.narrow ? 128 : 64;
             // positions from the first that a block's first row sees to its last row's own
-            const long reach = (long)p.chunk + p.block_rows / per + 1;
+            const long reach = (long)p.chunk + pl.block_rows / per + 1;
             const int sight = reach < max_len ? (int)reach : max_len;
-            int nsplit = ceil_div(ATT_TARGET, row_blocks * z);
+            int nsplit = ceil_div(ATT_TARGET, pl.row_blocks * n * p.groups);
             const int most = ceil_div(sight, pt);
             nsplit = nsplit < most ? nsplit : most;
-            p.stretch = round_up(ceil_div(sight, nsplit), pt);
-            p.nsplit = ceil_div(sight, p.stretch);
-            const size_t parts = (size_t)z * p.nsplit * p.rcap;
-            if (p.nsplit > 1 && parts * (DV + 2) > scratch_floats)
-                return fail(fn, "scratch too small");
-            if (row_blocks > 65535 || z > 65535 || p.nsplit > 65535)
-                return fail(fn, "too many entries or rows");
+            pl.stretch = round_up(ceil_div(sight, nsplit), pt);
+            pl.nsplit = ceil_div(sight, pl.stretch);
+            return pl;
+        }
+        // p.nsplit, p.rcap: the most of any entry; parts: rows of partial results
+        template <typename T, int DK, int DV>
+        bool attention_run(const char *fn, AttentionArgs &p, const AttentionPlan &pl, int row_blocks, int n, size_t parts, hipStream_t st)
+        {
+            constexpr bool NARROW = sizeof(T) == 2 || DK + DV <= 256;
+            constexpr int RG = sizeof(T) == 2 && DK + DV <= 384 ? 2 : 1;
+            const int z = n * p.groups;
+            p.block_rows = pl.block_rows;
             p.part_ml = p.part_o + parts * DV;
             bool ok;
             if constexpr (NARROW)
-                ok = narrow ? attention_launch<T, DK, DV, 1, 1>(fn, p, row_blocks, z, st) : attention_launch<T, DK, DV, 4, RG>(fn, p, row_blocks, z, st);
+                ok = pl.narrow ? attention_launch<T, DK, DV, 1, 1>(fn, p, row_blocks, z, st) : attention_launch<T, DK, DV, 4, RG>(fn, p, row_blocks, z, st);
             else
                 ok = attention_launch<T, DK, DV, 4, RG>(fn, p, row_blocks, z, st);
             if (!ok || p.nsplit == 1)
                 return ok;
-            hipLaunchKernelGGL((attention_merge_kernel<T, DV>), dim3(R, z), dim3(ATT_THREADS), 0, st, p);
+            hipLaunchKernelGGL((attention_merge_kernel<T, DV>), dim3(p.rcap, z), dim3(ATT_THREADS), 0, st, p);
             return launched(fn);
+        }
+        template <typename T, int DK, int DV>
+        bool attention_rows(const char *fn, AttentionArgs &p, int n, int max_ntok, int max_len, size_t scratch_floats, hipStream_t st)
+        {
+            const AttentionPlan pl = attention_plan<T, DK, DV>(p, n, max_ntok, max_len);
+            const int z = n * p.groups;
+            p.rcap = max_ntok * (p.heads / p.groups), p.stretch = pl.stretch, p.nsplit = pl.nsplit;
+            const size_t parts = (size_t)z * p.nsplit * p.rcap;
+            if (p.nsplit > 1 && parts * (DV + 2) > scratch_floats)
+                return fail(fn, "scratch too small");
+            if (pl.row_blocks > 65535 || z > 65535 || p.nsplit > 65535)
+                return fail(fn, "too many entries or rows");
+            return attention_run<T, DK, DV>(fn, p, pl, pl.row_blocks, n, parts, st);
+        }
+        // Portions share a launch where that is no waste: as many as the scratch holds the partial results of, and none whose
+        // stretches or rows would leave two thirds of the others' grid empty (a short portion far into its sequence has many stretches).
+        template <typename T, int DK, int DV>
+        bool attention_rows(const char *fn, AttentionArgs &p, int n, const int *ntok, const int *len, size_t scratch_floats, hipStream_t st)
+        {
+            const int first = p.first, per = p.heads / p.groups;
+            auto partial = [&](int i, const AttentionPlan &pl) { return pl.nsplit > 1 ? (size_t)p.groups * pl.nsplit * ntok[i] * per : 0; };
+            for (int i = 0; i < n; ++i)
+            {
+                const AttentionPlan pl = attention_plan<T, DK, DV>(p, 1, ntok[i], len[i]);
+                if (partial(i, pl) * (DV + 2) > scratch_floats)
+                    return fail(fn, "scratch too small");
+                if (pl.row_blocks > 65535 || p.groups > 65535 || pl.nsplit > 65535)
+                    return fail(fn, "too many entries or rows");
+            }
+            p.own = true;
+            for (int i = 0, some; i < n; i += some)
+            {
+                AttentionPlan all{};
+                size_t parts = 0;
+                long blocks = 0; // workgroups of a key/value head that have work
+                p.first = first + i, p.nsplit = p.rcap = 0;
+                for (some = 0; some < ATT_MANY && i + some < n; ++some)
+                {
+                    const int R = ntok[i + some] * per;
+                    const AttentionPlan pl = attention_plan<T, DK, DV>(p, 1, ntok[i + some], len[i + some]);
+                    const size_t own = partial(i + some, pl);
+                    const int high = all.row_blocks > pl.row_blocks ? all.row_blocks : pl.row_blocks, wide = p.nsplit > pl.nsplit ? p.nsplit : pl.nsplit;
+                    if (some > 0 && (pl.narrow != all.narrow || (parts + own) * (DV + 2) > scratch_floats || (long)(some + 1) * p.groups > 65535 ||
+                                     (long)(some + 1) * high * wide > 3 * (blocks + (long)pl.row_blocks * pl.nsplit)))
+                        break;
+                    p.cut[some] = {pl.stretch, pl.nsplit, (int)parts, R};
+                    parts += own, blocks += (long)pl.row_blocks * pl.nsplit;
+                    all = pl, all.row_blocks = high, p.nsplit = wide, p.rcap = p.rcap > R ? p.rcap : R;
+                }
+                if (!attention_run<T, DK, DV>(fn, p, all, all.row_blocks, some, parts, st))
+                    return false;
+            }
+            return true;
         }
         template <typename T, int DK, typename... Rest>
         bool attention_values(int vdim, Rest &&...rest)
@@ -646,6 +725,28 @@ extern "C" bool llam_seq_rotary(const llam_seq_attention_args *a, const float *d
     return launched(fn);
 }
 
+namespace
+{
+    bool attention_args(const char *fn, const llam_seq_attention_args *a, const void *d_q, const llam_seq_entries *e, int first, void *d_o, int ldo,
+                        float *d_scratch, AttentionArgs &p)
+    {
+        if (!d_q || !a->d_k || !a->d_v || !e || !e->d_row0 || !e->d_ntok || !e->d_slot || !e->d_pos || !d_o || !d_scratch)
+            return fail(fn, "null pointer");
+        if (!aligned16(d_q) || !aligned16(a->d_k) || !aligned16(a->d_v) || !aligned16(d_o) || !aligned16(d_scratch))
+            return fail(fn, "misaligned rows");
+        p = AttentionArgs{};
+        p.q = d_q, p.k = a->d_k, p.v = a->d_v, p.row0 = e->d_row0, p.ntok = e->d_ntok, p.slot = e->d_slot, p.pos = e->d_pos;
+        p.first = first, p.heads = a->heads, p.groups = a->kv_heads, p.ring = a->ring, p.chunk = a->chunk > 0 ? a->chunk : 0x3fffffff;
+        p.scale = a->scale, p.o = d_o, p.ldo = ldo, p.part_o = d_scratch;
+        return true;
+    }
+    bool attention_in_sight(const char *fn, const llam_seq_attention_args *a, int ntok, int len)
+    {
+        const long sight = a->chunk > 0 && a->chunk - 1 + (long)ntok < len ? a->chunk - 1 + (long)ntok : len;
+        return sight <= a->ring || fail(fn, "%ld positions in sight of an entry, the cache keeps %d", sight, a->ring);
+    }
+} // namespace
+
 extern "C" bool llam_seq_attention(const llam_seq_attention_args *a, const void *d_q, const llam_seq_entries *e, int first, int n,
                                    int max_ntok, int max_len, void *d_o, int ldo, float *d_scratch, size_t scratch_floats,
                                    int dtype, int device_id, void *stream)
@@ -655,23 +756,42 @@ extern "C" bool llam_seq_attention(const llam_seq_attention_args *a, const void 
         return false;
     if (n < 0 || first < 0 || max_ntok < 1 || max_len < 1 || ldo < a->heads * a->vdim || (ldo % 8) != 0)
         return fail(fn, "bad size (n=%d max_ntok=%d max_len=%d ldo=%d)", n, max_ntok, max_len, ldo);
-    const long sight = a->chunk > 0 && a->chunk - 1 + (long)max_ntok < max_len ? a->chunk - 1 + (long)max_ntok : max_len;
-    if (sight > a->ring)
-        return fail(fn, "%ld positions in sight of an entry, the cache keeps %d", sight, a->ring);
+    if (!attention_in_sight(fn, a, max_ntok, max_len))
+        return false;
     if (n == 0)
         return true;
-    if (!d_q || !a->d_k || !a->d_v || !e || !e->d_row0 || !e->d_ntok || !e->d_slot || !e->d_pos || !d_o || !d_scratch)
-        return fail(fn, "null pointer");
-    if (!aligned16(d_q) || !aligned16(a->d_k) || !aligned16(a->d_v) || !aligned16(d_o) || !aligned16(d_scratch))
-        return fail(fn, "misaligned rows");
-    if (!set_device(fn, device_id))
+    AttentionArgs p;
+    if (!attention_args(fn, a, d_q, e, first, d_o, ldo, d_scratch, p) || !set_device(fn, device_id))
         return false;
-    AttentionArgs p{};
-    p.q = d_q, p.k = a->d_k, p.v = a->d_v, p.row0 = e->d_row0, p.ntok = e->d_ntok, p.slot = e->d_slot, p.pos = e->d_pos;
-    p.first = first, p.heads = a->heads, p.groups = a->kv_heads, p.ring = a->ring, p.chunk = a->chunk > 0 ? a->chunk : 0x3fffffff;
-    p.scale = a->scale, p.o = d_o, p.ldo = ldo, p.part_o = d_scratch;
     hipStream_t st = as_stream(stream);
     if (dtype == LLAM_SEQ_F32)
         return attention_keys<float>(a->dim, a->vdim, fn, p, n, max_ntok, max_len, scratch_floats, st);
     return attention_keys<bf16>(a->dim, a->vdim, fn, p, n, max_ntok, max_len, scratch_floats, st);
+}
+
+extern "C" bool llam_seq_attention_portions(const llam_seq_attention_args *a, const void *d_q, const llam_seq_entries *e, int first, int n,
+                                            const int *ntok, const int *len, void *d_o, int ldo, float *d_scratch, size_t scratch_floats,
+                                            int dtype, int device_id, void *stream)
+{
+    static const char *fn = "llam_seq_attention_portions";
+    if (!attention_sizes(fn, a, dtype))
+        return false;
+    if (n < 0 || first < 0 || (n > 0 && (!ntok || !len)) || ldo < a->heads * a->vdim || (ldo % 8) != 0)
+        return fail(fn, "bad size (n=%d ldo=%d)", n, ldo);
+    for (int i = 0; i < n; ++i)
+    {
+        if (ntok[i] < 1 || len[i] < ntok[i])
+            return fail(fn, "bad size (portion %d: ntok=%d len=%d)", i, ntok[i], len[i]);
+        if (!attention_in_sight(fn, a, ntok[i], len[i]))
+            return false;
+    }
+    if (n == 0)
+        return true;
+    AttentionArgs p;
+    if (!attention_args(fn, a, d_q, e, first, d_o, ldo, d_scratch, p) || !set_device(fn, device_id))
+        return false;
+    hipStream_t st = as_stream(stream);
+    if (dtype == LLAM_SEQ_F32)
+        return attention_keys<float>(a->dim, a->vdim, fn, p, n, ntok, len, scratch_floats, st);
+    return attention_keys<bf16>(a->dim, a->vdim, fn, p, n, ntok, len, scratch_floats, st);
 }

@@ -52,6 +52,13 @@ namespace llamql
         return v;
     }
 
+    // How an entry's sequence is cut: positions of a stretch, stretches, and its partial results: rows before them and of a stretch.
+    struct LatentCut
+    {
+        int chunk, nsplit, first, rows;
+    };
+    constexpr int LAT_MANY = 16; // portions of a launch at most
+
     struct LatentArgs
     {
         const void *q;
@@ -61,7 +68,13 @@ namespace llamql
         float scale;
         void *o;
         float *part_o, *part_ml;
+        bool own; // every entry has its own cut; else all have that of the call
+        LatentCut cut[LAT_MANY];
     };
+    __device__ __forceinline__ LatentCut latent_cut(const LatentArgs &p, int ei)
+    {
+        return p.own ? p.cut[ei] : LatentCut{p.chunk, p.nsplit, ei * p.nsplit * p.rcap, p.rcap};
+    }
 
     // NOUT: 16-column output tiles of a row block, half of them per wavefront.  QREG: the query rows stay in
     // registers (rank <= 16 NOUT); otherwise they are read again for every turn and blockIdx.z also counts
@@ -93,10 +106,11 @@ namespace llamql
             return;
         const int last_row = rb + 16 * WR - 1 < R ? rb + 16 * WR - 1 : R - 1;
         const int kmax = pos0 + last_row / p.heads; // newest position any row of the block sees
-        const int k0 = split * p.chunk;
+        const LatentCut cut = latent_cut(p, ei);
+        const int k0 = split * cut.chunk;
         if (k0 > kmax || kmax >= p.cap)
             return;
-        const int k1 = k0 + p.chunk < kmax + 1 ? k0 + p.chunk : kmax + 1;
+        const int k1 = k0 + cut.chunk < kmax + 1 ? k0 + cut.chunk : kmax + 1;
 
         const int rank = FULL ? 16 * NOUT : p.rank;
         const int ksteps = rank >> 5;
@@ -324,13 +338,13 @@ namespace llamql
                     f[w] = fast_exp(s_ml[(w * WR * 16 + row) * 2] - base);
                     L += f[w] * s_ml[(w * WR * 16 + row) * 2 + 1];
                 }
-                const float inv = p.nsplit == 1 ? 1.0f / L : 1.0f;
+                const float inv = cut.nsplit == 1 ? 1.0f / L : 1.0f;
 #pragma unroll
                 for (int w = 0; w < WP; ++w)
                     s_f[w * WR * 16 + row] = f[w] * inv;
-                if (p.nsplit > 1 && slice == 0 && rb + row < R)
+                if (cut.nsplit > 1 && slice == 0 && rb + row < R)
                 {
-                    const size_t at = ((size_t)ei * p.nsplit + split) * p.rcap + rb + row;
+                    const size_t at = cut.first + (size_t)split * cut.rows + rb + row;
                     p.part_ml[at * 2] = M;
                     p.part_ml[at * 2 + 1] = L;
                 }
@@ -346,31 +360,31 @@ namespace llamql
                     for (int w = 0; w < WP; ++w)
                         y = y + *reinterpret_cast<const f32x4 *>(s_o + (w * WR * 16 + row) * OLD + d) * s_f[w * WR * 16 + row];
                     const int col = slice * NOUT * 16 + d;
-                    if (p.nsplit == 1)
+                    if (cut.nsplit == 1)
                         *reinterpret_cast<t4 *>(static_cast<T *>(p.o) + ((size_t)p.row0[e] * p.heads + rb + row) * rank + col) =
                             __builtin_convertvector(y, t4);
                     else
-                        *reinterpret_cast<f32x4 *>(p.part_o + (((size_t)ei * p.nsplit + split) * p.rcap + rb + row) * rank + col) = y;
+                        *reinterpret_cast<f32x4 *>(p.part_o + (cut.first + (size_t)split * cut.rows + rb + row) * rank + col) = y;
                 }
             return;
         }
         const int row = rb + wr * 16 + c;
         if (row >= R)
             return;
-        const size_t at = ((size_t)ei * p.nsplit + split) * p.rcap + row;
+        const size_t at = cut.first + (size_t)split * cut.rows + row;
         const float inv = 1.0f / l;
 #pragma unroll
         for (int t = 0; t < NT; ++t)
             if (t < out_tiles)
             {
                 const int col = (tile0 + t) * 16 + 4 * g;
-                if (p.nsplit == 1)
+                if (cut.nsplit == 1)
                     *reinterpret_cast<t4 *>(static_cast<T *>(p.o) + ((size_t)p.row0[e] * p.heads + row) * rank + col) =
                         __builtin_convertvector(acc[t] * inv, t4);
                 else
                     *reinterpret_cast<f32x4 *>(p.part_o + at * rank + col) = acc[t];
             }
-        if (p.nsplit > 1 && half == 0 && g == 0 && slice == 0)
+        if (cut.nsplit > 1 && half == 0 && g == 0 && slice == 0)
         {
             p.part_ml[at * 2] = m;
             p.part_ml[at * 2 + 1] = l;
@@ -392,14 +406,15 @@ namespace llamql
         if (row >= p.ntok[e] * p.heads)
             return;
         const int limit = p.pos[e] + row / p.heads;
-        if (limit >= p.cap)
+        const LatentCut cut = latent_cut(p, ei);
+        if (limit >= p.cap || cut.nsplit == 1)
             return;
-        const int used = limit / p.chunk + 1;
-        const size_t at = (size_t)ei * p.nsplit * p.rcap + row;
+        const int used = limit / cut.chunk + 1;
+        const size_t at = (size_t)cut.first + row;
         const int group = threadIdx.x >> 5, d = blockIdx.z * LAT_MERGE_COLS + (threadIdx.x & 31) * 4;
         float M = -INFINITY;
         for (int s = threadIdx.x; s < used; s += 256)
-            M = fmaxf(M, p.part_ml[(at + (size_t)s * p.rcap) * 2]);
+            M = fmaxf(M, p.part_ml[(at + (size_t)s * cut.rows) * 2]);
 #pragma unroll
         for (int off = 32; off > 0; off >>= 1)
             M = fmaxf(M, __shfl_xor(M, off, 64));
@@ -410,7 +425,7 @@ namespace llamql
         float L = 0.0f;
         for (int s = threadIdx.x; s < used; s += 256)
         {
-            const size_t k = (at + (size_t)s * p.rcap) * 2;
+            const size_t k = (at + (size_t)s * cut.rows) * 2;
             const float f = expf(p.part_ml[k] - M);
             s_w[s] = f;
             L += f * p.part_ml[k + 1];
@@ -421,7 +436,7 @@ namespace llamql
         {
 #pragma unroll 8
             for (int s = group; s < used; s += 8)
-                y = y + *reinterpret_cast<const f32x4 *>(p.part_o + (at + (size_t)s * p.rcap) * p.rank + d) * s_w[s];
+                y = y + *reinterpret_cast<const f32x4 *>(p.part_o + (at + (size_t)s * cut.rows) * p.rank + d) * s_w[s];
         }
         *reinterpret_cast<f32x4 *>(&s_y[group][(threadIdx.x & 31) * 4]) = y;
         __syncthreads();
@@ -565,6 +580,59 @@ extern "C" size_t llam_seq_latent_scratch_floats(int max_rows, int slots, int he
     return ((size_t)2 * LAT_TARGET + slots) * 64 * ((size_t)rank + 2);
 }
 
+namespace
+{
+    bool latent_args(const char *fn, const void *d_q, const void *d_cache, const llam_seq_entries *e, int heads, int rank, int cap, float scale,
+                     void *d_o, float *d_scratch, int dtype, LatentArgs &p)
+    {
+        if (!d_q || !d_cache || !e || !e->d_row0 || !e->d_ntok || !e->d_slot || !e->d_pos || !d_o || !d_scratch)
+            return fail(fn, "null pointer");
+        if ((rank % PAD) != 0 || !aligned16(d_q) || !aligned16(d_cache) || !aligned16(d_o) || !aligned16(d_scratch))
+            return fail(fn, "rank=%d must be a multiple of %d, rows 16-byte aligned", rank, PAD);
+        if (dtype != LLAM_SEQ_BF16 && dtype != LLAM_SEQ_F32)
+            return fail(fn, "dtype %d", dtype);
+        p = LatentArgs{};
+        p.q = d_q, p.cache = d_cache, p.row0 = e->d_row0, p.ntok = e->d_ntok, p.slot = e->d_slot, p.pos = e->d_pos;
+        p.heads = heads, p.rank = rank, p.cap = cap, p.scale = scale, p.o = d_o, p.slices = 1, p.part_o = d_scratch;
+        return true;
+    }
+
+    // p.nsplit, p.rcap: the most of any entry
+    bool latent_run(const char *fn, LatentArgs &p, int wr, int row_blocks, int n, int dtype, hipStream_t st)
+    {
+        const int rank = p.rank;
+        bool ok;
+        if (dtype == LLAM_SEQ_F32)
+        {
+            if (rank <= 128)
+                ok = latent_rows<float, 8, true>(fn, p, wr, row_blocks, n, st);
+            else
+            {
+                p.slices = ceil_div(rank, 256);
+                ok = latent_rows<float, 16, false>(fn, p, wr, row_blocks, n, st);
+            }
+        }
+        else if (rank <= 128)
+            ok = latent_rows<bf16, 8, true>(fn, p, wr, row_blocks, n, st);
+        else if (rank <= 256)
+            ok = latent_rows<bf16, 16, true>(fn, p, wr, row_blocks, n, st);
+        else if (rank <= 512)
+            ok = latent_rows<bf16, 32, true>(fn, p, wr, row_blocks, n, st);
+        else
+        {
+            p.slices = ceil_div(rank, 256);
+            ok = latent_rows<bf16, 16, false>(fn, p, wr, row_blocks, n, st);
+        }
+        if (!ok || p.nsplit == 1)
+            return ok;
+        if (dtype == LLAM_SEQ_F32)
+            hipLaunchKernelGGL(latent_merge_kernel<float>, dim3(p.rcap, n, ceil_div(rank, LAT_MERGE_COLS)), dim3(256), 0, st, p);
+        else
+            hipLaunchKernelGGL(latent_merge_kernel<bf16>, dim3(p.rcap, n, ceil_div(rank, LAT_MERGE_COLS)), dim3(256), 0, st, p);
+        return launched(fn);
+    }
+} // namespace
+
 extern "C" bool llam_seq_latent_attention(const void *d_q, const void *d_cache, const llam_seq_entries *e, int first,
                                           int n, int max_ntok, int max_len, int heads, int rank, int cap, float scale,
                                           void *d_o, float *d_scratch, size_t scratch_floats, int dtype, int device_id,
@@ -575,54 +643,66 @@ extern "C" bool llam_seq_latent_attention(const void *d_q, const void *d_cache, 
         return fail(fn, "bad size (n=%d heads=%d rank=%d cap=%d max_ntok=%d max_len=%d)", n, heads, rank, cap, max_ntok, max_len);
     if (n == 0)
         return true;
-    if (!d_q || !d_cache || !e || !e->d_row0 || !e->d_ntok || !e->d_slot || !e->d_pos || !d_o || !d_scratch)
-        return fail(fn, "null pointer");
-    if ((rank % PAD) != 0 || !aligned16(d_q) || !aligned16(d_cache) || !aligned16(d_o) || !aligned16(d_scratch))
-        return fail(fn, "rank=%d must be a multiple of %d, rows 16-byte aligned", rank, PAD);
-    if (dtype != LLAM_SEQ_BF16 && dtype != LLAM_SEQ_F32)
-        return fail(fn, "dtype %d", dtype);
+    LatentArgs p;
+    if (!latent_args(fn, d_q, d_cache, e, heads, rank, cap, scale, d_o, d_scratch, dtype, p))
+        return false;
     const LatentPlan pl = latent_plan(n, max_ntok, max_len, heads, rank, dtype == LLAM_SEQ_F32 ? 4 : 2);
-    LatentArgs p{};
-    p.q = d_q, p.cache = d_cache, p.row0 = e->d_row0, p.ntok = e->d_ntok, p.slot = e->d_slot, p.pos = e->d_pos;
-    p.first = first, p.heads = heads, p.rank = rank, p.cap = cap, p.chunk = pl.chunk, p.nsplit = pl.nsplit;
-    p.scale = scale, p.o = d_o, p.slices = 1;
-    p.rcap = max_ntok * heads;
+    p.first = first, p.chunk = pl.chunk, p.nsplit = pl.nsplit, p.rcap = max_ntok * heads;
     const size_t parts = (size_t)n * pl.nsplit * p.rcap;
     if (pl.nsplit > 1 && parts * ((size_t)rank + 2) > scratch_floats)
         return fail(fn, "scratch too small");
-    p.part_o = d_scratch, p.part_ml = d_scratch + parts * rank;
+    p.part_ml = d_scratch + parts * rank;
     if (n > 65535 || pl.nsplit > 65535)
         return fail(fn, "too many entries");
-    if (!set_device(fn, device_id))
+    return set_device(fn, device_id) && latent_run(fn, p, pl.wr, pl.row_blocks, n, dtype, as_stream(stream));
+}
+
+// Portions share a launch where that is no waste: as many as the scratch holds the partial results of, and none whose
+// stretches or rows would leave two thirds of the others' grid empty (a short portion far into its sequence has many stretches).
+extern "C" bool llam_seq_latent_portions(const void *d_q, const void *d_cache, const llam_seq_entries *e, int first, int n, const int *ntok,
+                                         const int *len, int heads, int rank, int cap, float scale, void *d_o, float *d_scratch,
+                                         size_t scratch_floats, int dtype, int device_id, void *stream)
+{
+    static const char *fn = "llam_seq_latent_portions";
+    if (n < 0 || first < 0 || heads < 1 || rank < 1 || cap < 1 || (n > 0 && (!ntok || !len)))
+        return fail(fn, "bad size (n=%d heads=%d rank=%d cap=%d)", n, heads, rank, cap);
+    LatentArgs p;
+    if (n > 0 && !latent_args(fn, d_q, d_cache, e, heads, rank, cap, scale, d_o, d_scratch, dtype, p))
         return false;
-    hipStream_t st = as_stream(stream);
-    bool ok;
-    if (dtype == LLAM_SEQ_F32)
+    const int elem = dtype == LLAM_SEQ_F32 ? 4 : 2;
+    for (int i = 0; i < n; ++i)
     {
-        if (rank <= 128)
-            ok = latent_rows<float, 8, true>(fn, p, pl.wr, pl.row_blocks, n, st);
-        else
+        if (ntok[i] < 1 || len[i] < ntok[i] || len[i] > cap)
+            return fail(fn, "bad size (portion %d: ntok=%d len=%d cap=%d)", i, ntok[i], len[i], cap);
+        const LatentPlan pl = latent_plan(1, ntok[i], len[i], heads, rank, elem);
+        if (pl.nsplit > 65535 || (pl.nsplit > 1 && (size_t)pl.nsplit * ntok[i] * heads * ((size_t)rank + 2) > scratch_floats))
+            return fail(fn, "scratch too small");
+    }
+    if (n > 0 && !set_device(fn, device_id))
+        return false;
+    p.own = true;
+    for (int i = 0, some; i < n; i += some)
+    {
+        size_t rows = 0; // of partial results
+        long blocks = 0; // workgroups that have work
+        int wr = 0, row_blocks = 0;
+        p.first = first + i, p.nsplit = p.rcap = 0;
+        for (some = 0; some < LAT_MANY && i + some < n; ++some)
         {
-            p.slices = ceil_div(rank, 256);
-            ok = latent_rows<float, 16, false>(fn, p, pl.wr, pl.row_blocks, n, st);
+            const int R = ntok[i + some] * heads;
+            const LatentPlan pl = latent_plan(1, ntok[i + some], len[i + some], heads, rank, elem);
+            const size_t own = pl.nsplit > 1 ? (size_t)pl.nsplit * R : 0;
+            const int high = row_blocks > pl.row_blocks ? row_blocks : pl.row_blocks, wide = p.nsplit > pl.nsplit ? p.nsplit : pl.nsplit;
+            if (some > 0 && (pl.wr != wr || (rows + own) * ((size_t)rank + 2) > scratch_floats ||
+                             (long)(some + 1) * high * wide > 3 * (blocks + (long)pl.row_blocks * pl.nsplit)))
+                break;
+            p.cut[some] = {pl.chunk, pl.nsplit, (int)rows, R};
+            rows += own, blocks += (long)pl.row_blocks * pl.nsplit;
+            wr = pl.wr, row_blocks = high, p.nsplit = wide, p.rcap = p.rcap > R ? p.rcap : R;
         }
+        p.part_ml = d_scratch + rows * rank;
+        if (!latent_run(fn, p, wr, row_blocks, some, dtype, as_stream(stream)))
+            return false;
     }
-    else if (rank <= 128)
-        ok = latent_rows<bf16, 8, true>(fn, p, pl.wr, pl.row_blocks, n, st);
-    else if (rank <= 256)
-        ok = latent_rows<bf16, 16, true>(fn, p, pl.wr, pl.row_blocks, n, st);
-    else if (rank <= 512)
-        ok = latent_rows<bf16, 32, true>(fn, p, pl.wr, pl.row_blocks, n, st);
-    else
-    {
-        p.slices = ceil_div(rank, 256);
-        ok = latent_rows<bf16, 16, false>(fn, p, pl.wr, pl.row_blocks, n, st);
-    }
-    if (!ok || pl.nsplit == 1)
-        return ok;
-    if (dtype == LLAM_SEQ_F32)
-        hipLaunchKernelGGL(latent_merge_kernel<float>, dim3(p.rcap, n, ceil_div(rank, LAT_MERGE_COLS)), dim3(256), 0, st, p);
-    else
-        hipLaunchKernelGGL(latent_merge_kernel<bf16>, dim3(p.rcap, n, ceil_div(rank, LAT_MERGE_COLS)), dim3(256), 0, st, p);
-    return launched(fn);
+    return true;
 }

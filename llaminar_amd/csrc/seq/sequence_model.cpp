@@ -139,10 +139,11 @@ namespace
     {
         int M = 0, single = 0;
         int max_len = 1; // bound on the length of the one-token entries' sequences
-        // runs of portions that are launched together: entries first .. first + n - 1, the most tokens and the longest afterwards
+        std::vector<int> ntok, len; // the portions' tokens, and their sequences' lengths afterwards
+        // runs of portions that the recurrent mixers launch together: entries first .. first + n - 1, the most tokens
         struct Run
         {
-            int first, n, ntok, len;
+            int first, n, ntok;
         };
         std::vector<Run> runs;
         long run_rows = 0; // tokens of the last one
@@ -151,21 +152,23 @@ namespace
         // pays for the latencies of its chain (eight prompts of 251 tokens and two steps, width 2048: Kogilix 5.0 -> 3.9 ms,
         // Bosirax 3.55 -> 2.67); a grid is made for the longest, so a portion that would leave two thirds of it empty starts a run of
         // its own.
-        void add(int entry, int ntok, int len)
+        void add(int entry, int tokens, int length)
         {
+            ntok.push_back(tokens), len.push_back(length);
             if (!runs.empty())
             {
                 Run &r = runs.back();
-                if ((long)(r.n + 1) * std::max(r.ntok, ntok) <= 3 * (run_rows + ntok))
+                if ((long)(r.n + 1) * std::max(r.ntok, tokens) <= 3 * (run_rows + tokens))
                 {
-                    ++r.n, run_rows += ntok;
-                    r.ntok = std::max(r.ntok, ntok), r.len = std::max(r.len, len);
+                    ++r.n, run_rows += tokens;
+                    r.ntok = std::max(r.ntok, tokens);
                     return;
                 }
             }
-            runs.push_back({entry, 1, ntok, len});
-            run_rows = ntok;
+            runs.push_back({entry, 1, tokens});
+            run_rows = tokens;
         }
+        int portions() const { return (int)ntok.size(); }
         const int32_t *row_slot = nullptr, *row_pos = nullptr;
     };
 
@@ -246,10 +249,9 @@ namespace
             if (s.single && !forward(fn, llam_seq_attention(&a, md.q, &e, 0, s.single, 1, s.max_len, md.mix, ldm, md.lat_scratch, md.lat_floats,
                                                             c.dtype, c.device_id, st)))
                 return false;
-            for (const Step::Run &r : s.runs)
-                if (!forward(fn, llam_seq_attention(&a, md.q, &e, r.first, r.n, r.ntok, r.len, md.mix, ldm, md.lat_scratch, md.lat_floats,
-                                                    c.dtype, c.device_id, st)))
-                    return false;
+            if (s.portions() && !forward(fn, llam_seq_attention_portions(&a, md.q, &e, s.single, s.portions(), s.ntok.data(), s.len.data(), md.mix, ldm,
+                                                                         md.lat_scratch, md.lat_floats, c.dtype, c.device_id, st)))
+                return false;
             return add_output(w, s);
         }
 
@@ -292,10 +294,9 @@ namespace
             if (s.single && !forward(fn, llam_seq_latent_attention(md.qlat, cache, &e, 0, s.single, 1, s.max_len, H, rp, c.cap, w.scale,
                                                                    md.olat, md.lat_scratch, md.lat_floats, c.dtype, c.device_id, st)))
                 return false;
-            for (const Step::Run &r : s.runs)
-                if (!forward(fn, llam_seq_latent_attention(md.qlat, cache, &e, r.first, r.n, r.ntok, r.len, H, rp, c.cap, w.scale, md.olat,
-                                                           md.lat_scratch, md.lat_floats, c.dtype, c.device_id, st)))
-                    return false;
+            if (s.portions() && !forward(fn, llam_seq_latent_portions(md.qlat, cache, &e, s.single, s.portions(), s.ntok.data(), s.len.data(), H, rp, c.cap,
+                                                                      w.scale, md.olat, md.lat_scratch, md.lat_floats, c.dtype, c.device_id, st)))
+                return false;
             return linear(md.olat, H * rp, w.w_uv, vp, rp, md.mix, mix_columns(w), LLAM_SEQ_OUT_ELEM, s.M, nullptr, nullptr, 0, nullptr, H,
                           rp, (long)vp * rp, vp) &&
                    add_output(w, s);

@@ -273,6 +273,39 @@ def test_many_portions_in_one_launch(dtype):
     model.close()
 
 
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("layer,at,n,others", [
+    (sm.attention(heads=16, kv_heads=16), 300, 64, [[160], [80, 80], [20] * 8, [8, 152], [10] * 16]),
+    (sm.attention(heads=16, kv_heads=8, chunk=250), 300, 64, [[160], [20] * 8, [8, 152]]),
+    (sm.attention(heads=40, kv_heads=20), 600, 3, [[34], [2] * 17, [17, 17]]),
+    (sm.delta(), 100, 150, [[320], [32] * 10, [20, 300], [64] * 5]),
+], ids=["attention", "attention, chunks", "attention, few tokens", "delta rule"])
+def test_a_portion_does_not_depend_on_those_beside_it(layer, at, n, others, dtype):
+    """The same bits beside one portion as beside many, like ones and unlike ones, shorter and longer."""
+    cfg = sm.bosirax(layer)
+    t = sm.random_bosirax(cfg, 5)
+    model = load(cfg, t, dtype, slots=18, cap=at + n + 320, max_rows=max(at, n + sum(others[0])))
+    got = sm.beside(model, cfg, at, n, others)
+    check(got[0], so.bosirax(cfg, t.plain(), tokens_of(cfg, at + n))[at:], dtype)
+    for g, o in zip(got, others):
+        assert np.array_equal(g, got[0]), f"beside {o} as beside {others[0]}"
+    model.close()
+
+
+def test_as_many_portions_as_a_step_may_have():
+    """Portions times key/value heads past 65535, the most that a grid's third extent takes."""
+    cfg = sm.bosirax(sm.attention(heads=17, kv_heads=17, dim=8, vdim=8, rot=8))
+    t = sm.random_bosirax(cfg, 3)
+    slots = 65535 // 17 + 2
+    model = load(cfg, t, "bfloat16", slots=slots, cap=128, max_rows=2 * slots)
+    tokens, plain = [tokens_of(cfg, 2, seed=b % 5) for b in range(slots)], t.plain()
+    last = [0, slots // 2, slots - 1]
+    got = model.forward([(b, 0, tokens[b]) for b in range(slots)], [2 * b + k for b in last for k in range(2)])
+    for i, b in enumerate(last):
+        check(got[2 * i:2 * i + 2], so.bosirax(cfg, plain, tokens[b]), "bfloat16", note=f"portion {b}")
+    model.close()
+
+
 def test_a_slot_used_again_starts_afresh(whole, whole_f32):
     _, tokens, want = whole
     other = tokens_of(WHOLE, 200, seed=9)
