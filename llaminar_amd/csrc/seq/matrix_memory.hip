@@ -46,11 +46,22 @@ namespace llamql
         int splits;     // decoding: workgroups along dim
         void *qk;       // T [2][heads][rows of the portion][dim]: scaled q, then k
         int qk_rows;
-        // long portions: stretches of `stretch` chunks (0: the portion is one), what each adds to the memory and keeps of it
-        int stretch, parts; // `parts` of them
+        // long portions: stretches (a portion's at most, the most of any of the call's), what each adds to the memory and keeps of it
+        int most, parts;
         float *starts; // [portions][stretches][heads][dim][vdim + 16]: the memory before the portion, then what stretch 0 .. adds
         float *kept;   // [portions][stretches][heads]: what is left of the memory after stretch 0 ..
     };
+
+    constexpr int STRETCH_MIN = 3; // chunks of a stretch at least
+    // Stretches of a portion that are walked side by side (1: the walk is one): a portion's own length decides, so that its
+    // sums are the same whatever portions lie beside it, and a long one keeps its stretches beside short ones (a step of 2048, 60
+    // and 60 tokens, Kogilix, width 2048: 2.99 -> 2.94 ms).  Portions that are cut and would fill the chip uncut pay for it:
+    // five of 400 tokens take two launches of each kernel and 118 us a layer instead of 61.
+    __host__ __device__ __forceinline__ int memory_stretches(int chunks, int most)
+    {
+        const int n = chunks / STRETCH_MIN;
+        return n < 2 || most < 2 ? 1 : n < most ? n : most;
+    }
 
     __device__ __forceinline__ void memory_gates(const MemoryArgs &p, const float *row, int h, float &i, float &f)
     {
@@ -337,9 +348,13 @@ namespace llamql
                         to[(size_t)(16 * t + 4 * g + r) * ldv] = S[t][r];
                 }
         };
-        const int part = CUT ? (int)blockIdx.z - ei * p.parts : 0, first = CUT ? part * p.stretch * LC : 0; // this stretch and its first token
-        const bool last = !CUT || part + 1 == p.parts;
-        const int stop = last || first + p.stretch * LC > ntok ? ntok : first + p.stretch * LC;
+        const int chunks = (ntok + LC - 1) / LC, parts = CUT ? memory_stretches(chunks, p.most) : 1;
+        const int part = CUT ? (int)blockIdx.z - ei * p.parts : 0;
+        if (part >= parts || (SUM && parts == 1))
+            return;
+        const int stretch = (chunks + parts - 1) / parts * LC, first = part * stretch; // tokens of a stretch, the first of this one
+        const bool last = part + 1 == parts;
+        const int stop = last || first + stretch > ntok ? ntok : first + stretch;
         const size_t part_floats = (size_t)p.heads * dim * ldv;
         float *starts = p.starts + (size_t)ei * p.parts * part_floats + (size_t)h * dim * ldv + (live ? col : 0);
         float *part_kept = p.kept + (size_t)ei * p.parts * p.heads + h;
@@ -362,7 +377,7 @@ namespace llamql
         else if (live)
         {
             if (!fresh)
-                load_state(CUT && p.stretch ? starts : state);
+                load_state(parts > 1 ? starts : state);
             for (int i = 1; CUT && i <= part; ++i)
             {
                 const float kept = part_kept[(i - 1) * p.heads];
@@ -666,21 +681,15 @@ namespace llamql
         constexpr int LC16 = 64, LC32 = 32; // chunk lengths of the two number formats
         constexpr int CUT_TILES = 16;                    // 16-row tiles of S up to which a portion is cut into stretches
         constexpr int MANY = 16;                         // portions of a launch at most
-        constexpr int STRETCHES = 8, STRETCH_MIN = 3; // stretches of a portion at most, chunks of one at least
+        constexpr int STRETCHES = 8;                     // stretches of a portion at most, and that there is room for
         constexpr int STEP_SPLIT_ENTRIES = 32; // sequences up to which a decoding step splits the rows of S (in at most 8)
 
         struct MemoryScratch
         {
             size_t ga, a, mt, m0, prod, num, qk, starts, kept, total;
         };
-        // Stretches of a portion that are walked side by side (1: the walk is one).
-        int memory_stretches(int ntok, int dim, int lc)
-        {
-            if (dim > 16 * CUT_TILES)
-                return 1;
-            const int chunks = ceil_div(ntok, lc), n = chunks / STRETCH_MIN;
-            return n < 2 ? 1 : n < STRETCHES ? n : STRETCHES;
-        }
+        // Stretches that the scratch of `rows` has room for (the shorter chunks: the most that any portion has).
+        int stretch_room(int rows, int dim) { return dim > 16 * CUT_TILES ? 1 : memory_stretches(ceil_div(rows, LC32), STRETCHES); }
         MemoryScratch memory_scratch(int rows, int heads, int dim, int vdim)
         {
             MemoryScratch s{};
@@ -699,7 +708,7 @@ namespace llamql
             const size_t outs = (size_t)(rows > STEP_SPLIT_ENTRIES * 8 ? rows : STEP_SPLIT_ENTRIES * 8);
             s.num = take(outs * heads * (vdim + 16) * 4);
             s.qk = take((size_t)2 * heads * kept * dim * 4);
-            const int stretches = memory_stretches(rows, dim, LC32); // (the shorter chunks: the most that any portion has)
+            const int stretches = stretch_room(rows, dim);
             s.starts = take(stretches > 1 ? (size_t)stretches * heads * dim * (vdim + 16) * 4 : 0);
             s.kept = take((size_t)stretches * heads * 4);
             s.total = at;
@@ -743,7 +752,7 @@ namespace llamql
             p.mt = reinterpret_cast<float *>(s + at.mt), p.m0 = reinterpret_cast<float *>(s + at.m0);
             p.prod = reinterpret_cast<float *>(s + at.prod), p.num = reinterpret_cast<float *>(s + at.num);
             p.qk = s + at.qk, p.qk_rows = rows + MANY * LC16;
-            p.parts = memory_stretches(rows, p.dim, LC32); // (as many as there is room for)
+            p.parts = stretch_room(rows, p.dim); // (as many as there is room for)
             p.starts = reinterpret_cast<float *>(s + at.starts), p.kept = reinterpret_cast<float *>(s + at.kept);
         }
 
@@ -780,10 +789,22 @@ namespace llamql
         template <typename T, int LC>
         bool prefill_run(const char *fn, MemoryArgs p, int n, int ntok, int cus, hipStream_t st)
         {
-            // (a workgroup fills a compute unit: no second round of them; and as many stretches as the scratch has room for)
-            const int most = std::min(cus / (ceil_div(p.vdim + 16, 64) * p.heads), p.parts) / n, can = memory_stretches(ntok, p.dim, LC);
-            p.parts = std::max(1, std::min(can, most));
-            p.stretch = p.parts > 1 ? ceil_div(ceil_div(ntok, LC), p.parts) : 0;
+            // (a workgroup fills a compute unit: no second round of a portion's)
+            const int room = p.parts;
+            p.most = p.dim > 16 * CUT_TILES ? 1 : std::min(STRETCHES, cus / (ceil_div(p.vdim + 16, 64) * p.heads));
+            p.parts = memory_stretches(ceil_div(ntok, LC), p.most);
+            if (p.parts > 1 && n > room / p.parts) // as many portions at a time as there is room for the stretches of
+            {
+                const int few = room / p.parts, entry = p.entry;
+                p.parts = room;
+                for (int k = 0; k < n; k += few)
+                {
+                    p.entry = entry + k;
+                    if (!prefill_run<T, LC>(fn, p, std::min(few, n - k), ntok, cus, st))
+                        return false;
+                }
+                return true;
+            }
             hipLaunchKernelGGL(memory_gates_kernel<LC>, dim3(p.heads, n), dim3(GATE_WAVES * 64), 0, st, p);
             if (!launched(fn))
                 return false;

@@ -199,14 +199,15 @@ def run(model, slot, tokens, cuts, at=0):
 
 
 def beside(model, cfg, at, n, others):
-    """Logits of a portion of n tokens at position `at`, once per list of portions that lie beside it in the step (slots 1 ..,
-    from position 0): all lists hold as many tokens, so that every row-wise layer sees the same rows."""
+    """Logits of a portion of n tokens at position `at` and of those beside it in the step (slots 1 .., from position 0), once per
+    list of these: all lists hold as many tokens, so that every row-wise layer sees the same rows."""
     assert len({sum(o) for o in others}) == 1
     tokens, got = tokens_of(cfg, at + n), []
     for o in others:
         if at:
             model.forward([(0, 0, tokens[:at])])
-        got.append(model.forward([(0, at, tokens[at:])] + [(1 + i, 0, tokens_of(cfg, k, seed=2 + i)) for i, k in enumerate(o)], range(n)))
+        got.append(model.forward([(0, at, tokens[at:])] + [(1 + i, 0, tokens_of(cfg, k, seed=2 + i)) for i, k in enumerate(o)],
+                                 range(n + sum(o))))
     return got
 
 

@@ -285,10 +285,15 @@ def test_a_portion_does_not_depend_on_those_beside_it(layer, at, n, others, dtyp
     cfg = sm.bosirax(layer)
     t = sm.random_bosirax(cfg, 5)
     model = load(cfg, t, dtype, slots=18, cap=at + n + 320, max_rows=max(at, n + sum(others[0])))
-    got = sm.beside(model, cfg, at, n, others)
-    check(got[0], so.bosirax(cfg, t.plain(), tokens_of(cfg, at + n))[at:], dtype)
+    got, plain = sm.beside(model, cfg, at, n, others), t.plain()
+    check(got[0][:n], so.bosirax(cfg, plain, tokens_of(cfg, at + n))[at:], dtype)
     for g, o in zip(got, others):
-        assert np.array_equal(g, got[0]), f"beside {o} as beside {others[0]}"
+        assert np.array_equal(g[:n], got[0][:n]), f"beside {o} as beside {others[0]}"
+        row = n
+        for i, k in enumerate(o):
+            if i == 0 or i + 1 == len(o):
+                check(g[row:row + k], so.bosirax(cfg, plain, tokens_of(cfg, k, seed=2 + i)), dtype, note=f"{k} of {o}")
+            row += k
     model.close()
 
 

@@ -275,16 +275,22 @@ def test_a_long_portion_is_walked_in_stretches(heads, dim, vdim, dtype):
     (sm.latent(heads=20, dim=12, vdim=4, q_rank=64, kv_rank=64), 300, 64, [[160], [80, 80], [20] * 8, [8, 152], [10] * 16]),
     (sm.latent(heads=20, dim=12, vdim=4, q_rank=64, kv_rank=330), 300, 64, [[160], [20] * 8, [8, 152]]),
     (sm.latent(heads=9, kv_rank=150), 600, 3, [[34], [2] * 17, [17, 17]]),
-], ids=["latent", "latent, wide", "latent, few tokens"])
+    (sm.mlstm(gate_cap=15.0), 70, 810, [[600], [300, 300], [200] * 3, [540, 60], [100] * 6, [450, 150]]),
+], ids=["latent", "latent, wide", "latent, few tokens", "memory"])
 def test_a_portion_does_not_depend_on_those_beside_it(layer, at, n, others, dtype):
     """The same bits beside one portion as beside many, like ones and unlike ones, shorter and longer."""
     cfg = sm.config(layer)
-    t = sm.random_weights(cfg, 5)
+    t = sm.random_weights(cfg, 5, forget_bias=6.0)
     model = load(cfg, t, dtype, slots=18, cap=at + n + 200, max_rows=max(at, n + sum(others[0])))
-    got = sm.beside(model, cfg, at, n, others)
-    check(got[0], so.kogilix(cfg, t.plain(), tokens_of(cfg, at + n))[at:], dtype)
+    got, plain = sm.beside(model, cfg, at, n, others), t.plain()
+    check(got[0][:n], so.kogilix(cfg, plain, tokens_of(cfg, at + n))[at:], dtype)
     for g, o in zip(got, others):
-        assert np.array_equal(g, got[0]), f"beside {o} as beside {others[0]}"
+        assert np.array_equal(g[:n], got[0][:n]), f"beside {o} as beside {others[0]}"
+        row = n
+        for i, k in enumerate(o):
+            if i == 0 or i + 1 == len(o):
+                check(g[row:row + k], so.kogilix(cfg, plain, tokens_of(cfg, k, seed=2 + i)), dtype, note=f"{k} of {o}")
+            row += k
     model.close()
 
 
