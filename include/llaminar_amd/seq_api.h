@@ -153,6 +153,8 @@ typedef struct
     float q_scale, gate_cap, eps;
 } llam_seq_memory_args;
 size_t llam_seq_memory_scratch_bytes(int max_rows, int heads, int dim, int vdim);
+/* where a call never has more than `portions` portions (less: several are kept in whole chunks each) */
+size_t llam_seq_memory_portions_scratch_bytes(int max_rows, int portions, int heads, int dim, int vdim);
 /* one token per entry, entries first .. first + n - 1 */
 bool llam_seq_memory_decode(const llam_seq_memory_args *a, const llam_seq_entries *e, int first, int n,
                             void *d_scratch, size_t scratch_bytes, int dtype, int device_id, void *stream);
@@ -221,6 +223,8 @@ typedef struct
     float eps;
 } llam_seq_delta_args;
 size_t llam_seq_delta_scratch_bytes(int max_rows, int heads, int kv_heads, int dim, int vdim);
+/* As llam_seq_memory_portions_scratch_bytes. */
+size_t llam_seq_delta_portions_scratch_bytes(int max_rows, int portions, int heads, int kv_heads, int dim, int vdim);
 /* one token per entry, entries first .. first + n - 1 */
 bool llam_seq_delta_decode(const llam_seq_delta_args *a, const llam_seq_entries *e, int first, int n, int dtype,
                            int device_id, void *stream);

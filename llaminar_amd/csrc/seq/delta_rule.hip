@@ -635,6 +635,8 @@ namespace llamql
             return p.a.dim == 64 ? step_launch<T, 4>(fn, p, n, st) : p.a.dim == 128 ? step_launch<T, 8>(fn, p, n, st)
                    : p.a.dim == 192 ? step_launch<T, 12>(fn, p, n, st) : step_launch<T, 16>(fn, p, n, st);
         }
+        // tokens of whole chunks; of several portions (as many as share a launch) each has some of its own
+        int kept_tokens(int rows, int portions) { return round_up(rows, DC) + (portions > 1 ? (portions < DELTA_MANY ? portions : DELTA_MANY) * DC : 0); }
         template <int DP>
         bool walk_launch(const char *fn, const DeltaArgs &p, int n, hipStream_t st)
         {
@@ -648,9 +650,14 @@ using namespace llamql;
 
 extern "C" size_t llam_seq_delta_scratch_bytes(int max_rows, int heads, int kv_heads, int dim, int vdim)
 {
-    if (max_rows < 1 || heads < 1 || kv_heads < 1 || dim < 1 || vdim < 1)
+    return llam_seq_delta_portions_scratch_bytes(max_rows, DELTA_MANY, heads, kv_heads, dim, vdim);
+}
+
+extern "C" size_t llam_seq_delta_portions_scratch_bytes(int max_rows, int portions, int heads, int kv_heads, int dim, int vdim)
+{
+    if (max_rows < 1 || portions < 1 || heads < 1 || kv_heads < 1 || dim < 1 || vdim < 1)
         return 0;
-    return delta_scratch(round_up(max_rows, DC) + DELTA_MANY * DC, heads, kv_heads, dim, vdim).total; // (of several portions: whole chunks)
+    return delta_scratch(kept_tokens(max_rows, portions), heads, kv_heads, dim, vdim).total;
 }
 
 extern "C" bool llam_seq_delta_decode(const llam_seq_delta_args *a, const llam_seq_entries *e, int first, int n, int dtype,
@@ -718,7 +725,7 @@ extern "C" bool llam_seq_delta_prefill_many(const llam_seq_delta_args *a, const 
     if (!delta_args(fn, a, e, dtype, p))
         return false;
     p.many = n > 1;
-    p.rows = p.many ? round_up(rows, DC) + DELTA_MANY * DC : round_up(max_ntok, DC);
+    p.rows = kept_tokens(p.many ? rows : max_ntok, n);
     const DeltaScratch at = delta_scratch(p.rows, a->heads, a->kv_heads, a->dim, a->vdim);
     if (!d_scratch || at.total > scratch_bytes)
         return fail(fn, "scratch too small");

@@ -690,7 +690,9 @@ namespace llamql
         };
         // Stretches that the scratch of `rows` has room for (the shorter chunks: the most that any portion has).
         int stretch_room(int rows, int dim) { return dim > 16 * CUT_TILES ? 1 : memory_stretches(ceil_div(rows, LC32), STRETCHES); }
-        MemoryScratch memory_scratch(int rows, int heads, int dim, int vdim)
+        // rows of whole chunks; of several portions each has some of its own
+        int kept_rows(int rows, int portions) { return round_up(rows, LC16) + (portions > 1 ? portions * LC16 : 0); }
+        MemoryScratch memory_scratch(int rows, int portions, int heads, int dim, int vdim)
         {
             MemoryScratch s{};
             size_t at = 0;
@@ -702,8 +704,8 @@ namespace llamql
             s.ga = take((size_t)rows * heads * 8);
             s.a = take((size_t)rows * heads * 8);
             s.mt = take((size_t)rows * heads * 4);
-            s.m0 = take((size_t)MANY * heads * 4);
-            const size_t kept = (size_t)round_up(rows, LC16) + MANY * LC16; // rows of whole chunks, of several portions
+            s.m0 = take((size_t)portions * heads * 4);
+            const size_t kept = kept_rows(rows, portions);
             s.prod = take(kept * heads * LC16 * 4);
             const size_t outs = (size_t)(rows > STEP_SPLIT_ENTRIES * 8 ? rows : STEP_SPLIT_ENTRIES * 8);
             s.num = take(outs * heads * (vdim + 16) * 4);
@@ -739,19 +741,19 @@ namespace llamql
             p.row0 = e->d_row0, p.ntok = e->d_ntok, p.slot = e->d_slot, p.pos = e->d_pos;
             return true;
         }
-        void place_scratch(MemoryArgs &p, void *d_scratch, size_t scratch_bytes)
+        void place_scratch(MemoryArgs &p, void *d_scratch, size_t scratch_bytes, int portions)
         {
             // rows of the step are absolute, so the offsets are those of the whole buffer: the largest
             // row count whose scratch fits
             int rows = 64;
-            while (memory_scratch(rows + 64, p.heads, p.dim, p.vdim).total <= scratch_bytes)
+            while (memory_scratch(rows + 64, portions, p.heads, p.dim, p.vdim).total <= scratch_bytes)
                 rows += 64;
-            const MemoryScratch at = memory_scratch(rows, p.heads, p.dim, p.vdim);
+            const MemoryScratch at = memory_scratch(rows, portions, p.heads, p.dim, p.vdim);
             char *s = static_cast<char *>(d_scratch);
             p.ga = reinterpret_cast<double *>(s + at.ga), p.a = reinterpret_cast<double *>(s + at.a);
             p.mt = reinterpret_cast<float *>(s + at.mt), p.m0 = reinterpret_cast<float *>(s + at.m0);
             p.prod = reinterpret_cast<float *>(s + at.prod), p.num = reinterpret_cast<float *>(s + at.num);
-            p.qk = s + at.qk, p.qk_rows = rows + MANY * LC16;
+            p.qk = s + at.qk, p.qk_rows = kept_rows(rows, portions);
             p.parts = stretch_room(rows, p.dim); // (as many as there is room for)
             p.starts = reinterpret_cast<float *>(s + at.starts), p.kept = reinterpret_cast<float *>(s + at.kept);
         }
@@ -835,9 +837,14 @@ using namespace llamql;
 
 extern "C" size_t llam_seq_memory_scratch_bytes(int max_rows, int heads, int dim, int vdim)
 {
-    if (max_rows < 1 || heads < 1 || dim < 1 || vdim < 1)
+    return llam_seq_memory_portions_scratch_bytes(max_rows, MANY, heads, dim, vdim);
+}
+
+extern "C" size_t llam_seq_memory_portions_scratch_bytes(int max_rows, int portions, int heads, int dim, int vdim)
+{
+    if (max_rows < 1 || portions < 1 || heads < 1 || dim < 1 || vdim < 1)
         return 0;
-    return memory_scratch(round_up(max_rows, LC16), heads, dim, vdim).total;
+    return memory_scratch(round_up(max_rows, LC16), portions < MANY ? portions : MANY, heads, dim, vdim).total;
 }
 
 extern "C" bool llam_seq_memory_decode(const llam_seq_memory_args *a, const llam_seq_entries *e, int first, int n,
@@ -851,10 +858,10 @@ extern "C" bool llam_seq_memory_decode(const llam_seq_memory_args *a, const llam
         return true;
     if (!memory_args(fn, a, e, d_scratch, dtype, p))
         return false;
-    if (llam_seq_memory_scratch_bytes(first + n, p.heads, p.dim, p.vdim) > scratch_bytes)
+    if (llam_seq_memory_portions_scratch_bytes(first + n, 1, p.heads, p.dim, p.vdim) > scratch_bytes)
         return fail(fn, "scratch too small");
     p.entry = first;
-    place_scratch(p, d_scratch, scratch_bytes);
+    place_scratch(p, d_scratch, scratch_bytes, 1);
     if (!set_device(fn, device_id))
         return false;
     return dtype == LLAM_SEQ_F32 ? decode_run<float>(fn, p, n, as_stream(stream)) : decode_run<bf16>(fn, p, n, as_stream(stream));
@@ -877,9 +884,10 @@ extern "C" bool llam_seq_memory_prefill_many(const llam_seq_memory_args *a, cons
         return true;
     if (!memory_args(fn, a, e, d_scratch, dtype, p))
         return false;
-    if (llam_seq_memory_scratch_bytes(rows, p.heads, p.dim, p.vdim) > scratch_bytes)
+    const int portions = n < MANY ? n : MANY;
+    if (llam_seq_memory_portions_scratch_bytes(rows, portions, p.heads, p.dim, p.vdim) > scratch_bytes)
         return fail(fn, "scratch too small");
-    place_scratch(p, d_scratch, scratch_bytes);
+    place_scratch(p, d_scratch, scratch_bytes, portions);
     if (!set_device(fn, device_id))
         return false;
     p.many = n > 1;

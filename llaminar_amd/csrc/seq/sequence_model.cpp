@@ -543,6 +543,7 @@ extern "C" bool llam_seqm_set_globals(void *model, const llam_seqm_globals *g)
     const size_t M = c.max_rows, elem = md->elem;
     bool parallel = false;
     size_t n_in = 0, q = 0, lat = 0, mix = 0, act = 0, z = 16, h = md->wp, latf = 0, scratch = 0;
+    const int portions = std::max(1, std::min(c.slots, c.max_rows / 2)); // (of two tokens at least) in a step
     for (const llam_seqm_layer &w : md->layers)
     {
         const size_t H = w.heads, dp = P(w.dim), vp = P(w.vdim);
@@ -566,12 +567,12 @@ extern "C" bool llam_seqm_set_globals(void *model, const llam_seqm_globals *g)
         else if (w.mixer == LLAM_MIXER_DELTA)
         {
             n_in = std::max(n_in, (size_t)pad((int)(2 * w.kv_heads * dp + 2 * H * vp + 2 * H), 16));
-            scratch = std::max(scratch, llam_seq_delta_scratch_bytes(c.max_rows, w.heads, w.kv_heads, (int)dp, (int)vp));
+            scratch = std::max(scratch, llam_seq_delta_portions_scratch_bytes(c.max_rows, portions, w.heads, w.kv_heads, (int)dp, (int)vp));
         }
         else
         {
             n_in = std::max(n_in, (size_t)pad((int)(2 * H * (dp + vp) + 2 * H), 16));
-            scratch = std::max(scratch, llam_seq_memory_scratch_bytes(std::max(c.max_rows, c.slots), w.heads, (int)dp, (int)vp));
+            scratch = std::max(scratch, llam_seq_memory_portions_scratch_bytes(std::max(c.max_rows, c.slots), portions, w.heads, (int)dp, (int)vp));
         }
         if (gated(w.ffn) && !w.parallel)
             act = std::max(act, (size_t)P(w.ff));

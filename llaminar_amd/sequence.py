@@ -111,6 +111,7 @@ SIGNATURES = {
     "llam_seq_attention_portions": (c_bool, [POINTER(AttentionArgs), c_void_p, POINTER(Entries), c_int, c_int, POINTER(c_int), POINTER(c_int),
                                              c_void_p, c_int, c_void_p, c_size_t, c_int, c_int, c_void_p]),
     "llam_seq_delta_scratch_bytes": (c_size_t, [c_int, c_int, c_int, c_int, c_int]),
+    "llam_seq_delta_portions_scratch_bytes": (c_size_t, [c_int, c_int, c_int, c_int, c_int, c_int]),
     "llam_seq_delta_decode": (c_bool, [POINTER(DeltaArgs), POINTER(Entries), c_int, c_int, c_int, c_int, c_void_p]),
     "llam_seq_delta_prefill": (c_bool, [POINTER(DeltaArgs), POINTER(Entries), c_int, c_int, c_void_p, c_size_t, c_int, c_int,
                                         c_void_p]),
@@ -124,6 +125,7 @@ SIGNATURES = {
     "llam_seq_latent_portions": (c_bool, [c_void_p, c_void_p, POINTER(Entries), c_int, c_int, POINTER(c_int), POINTER(c_int), c_int, c_int,
                                           c_int, c_float, c_void_p, c_void_p, c_size_t, c_int, c_int, c_void_p]),
     "llam_seq_memory_scratch_bytes": (c_size_t, [c_int, c_int, c_int, c_int]),
+    "llam_seq_memory_portions_scratch_bytes": (c_size_t, [c_int, c_int, c_int, c_int, c_int]),
     "llam_seq_memory_decode": (c_bool, [POINTER(MemoryArgs), POINTER(Entries), c_int, c_int, c_void_p, c_size_t, c_int,
                                         c_int, c_void_p]),
     "llam_seq_memory_prefill": (c_bool, [POINTER(MemoryArgs), POINTER(Entries), c_int, c_int, c_void_p, c_size_t, c_int,

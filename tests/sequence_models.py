@@ -211,6 +211,20 @@ def beside(model, cfg, at, n, others):
     return got
 
 
+def check_scratch(load, chunk):
+    """Every portion of a step, up to sixteen, has a chunk's values (`chunk` bytes at least) of its own where there are several: a
+    model of one slot has none for others, nor one whose steps hold a single portion."""
+    def beside_slots(slots, rows):
+        model = load(slots, rows)
+        left = model.device_bytes() - slots * model.slot_bytes()
+        model.close()
+        return left
+
+    of = {s: beside_slots(s, 64) for s in (1, 2, 16, 17)}
+    assert of[2] - of[1] >= 2 * chunk and of[16] - of[2] >= 14 * chunk and of[17] - of[16] < chunk, of
+    assert beside_slots(5, 3) - beside_slots(1, 3) < chunk
+
+
 def tokens_of(cfg, n, seed=0):
     return np.random.default_rng(seed + 1000).integers(0, cfg["vocab"], n).tolist()
 

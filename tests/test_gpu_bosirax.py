@@ -311,6 +311,12 @@ def test_as_many_portions_as_a_step_may_have():
     model.close()
 
 
+def test_scratch_holds_the_portions_that_a_step_can_have():
+    cfg = sm.bosirax(sm.delta())
+    t = sm.random_bosirax(cfg, 1)
+    sm.check_scratch(lambda slots, rows: load(cfg, t, slots=slots, cap=64, max_rows=rows), 64 * (2 * 2 * 64 + 4 * 64) * 4)
+
+
 def test_a_slot_used_again_starts_afresh(whole, whole_f32):
     _, tokens, want = whole
     other = tokens_of(WHOLE, 200, seed=9)

@@ -294,6 +294,12 @@ def test_a_portion_does_not_depend_on_those_beside_it(layer, at, n, others, dtyp
     model.close()
 
 
+def test_scratch_holds_the_portions_that_a_step_can_have():
+    cfg = sm.config(sm.mlstm())
+    t = sm.random_weights(cfg, 1)
+    sm.check_scratch(lambda slots, rows: load(cfg, t, slots=slots, cap=64, max_rows=rows), 64 * 2 * 3 * 64 * 4)
+
+
 def test_generation_through_the_scheduler(whole, whole_f32):
     """More requests than slots, portions mixed with decoding, bursts on the device: the tokens of a plain loop."""
     t, _, _ = whole

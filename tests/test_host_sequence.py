@@ -29,6 +29,16 @@ def test_library_exports_every_declared_symbol():
     assert names | {"llam_ql_last_error"} == set(sequence.SIGNATURES)
 
 
+def test_scratch_by_the_portions_of_a_call():
+    """More for every portion up to the sixteen that share a launch, as much as without a bound from there on."""
+    lib = sequence.load()
+    for of, unbound in ((lambda n, rows=700: lib.llam_seq_delta_portions_scratch_bytes(rows, n, 40, 20, 128, 128), lib.llam_seq_delta_scratch_bytes(700, 40, 20, 128, 128)),
+                        (lambda n, rows=700: lib.llam_seq_memory_portions_scratch_bytes(rows, n, 4, 256, 512), lib.llam_seq_memory_scratch_bytes(700, 4, 256, 512))):
+        sizes = [of(n) for n in range(1, 19)]
+        assert sizes[:16] == sorted(set(sizes)) and sizes[15] == sizes[16] == sizes[17] == unbound
+        assert of(0) == of(1, 0) == 0
+
+
 def test_bad_arguments_are_refused_before_any_launch():
     lib = sequence.load()
     buf = np.zeros(4096, np.uint8)
