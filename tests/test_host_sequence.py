@@ -39,6 +39,30 @@ def test_scratch_by_the_portions_of_a_call():
         assert of(0) == of(1, 0) == 0
 
 
+def test_portions_of_attention_are_refused_before_any_launch():
+    lib = sequence.load()
+    buf = np.zeros(4096, np.uint8)
+    p = buf.ctypes.data + (-buf.ctypes.data % 16)
+    err = lambda: lib.llam_ql_last_error().decode()
+    e, ints = sequence.Entries(p, p, p, p), lambda *v: (ctypes.c_int * len(v))(*v)
+    latent = lambda n, ntok, length, floats=1 << 30, rank=64: lib.llam_seq_latent_portions(
+        p, p, ctypes.byref(e), 0, n, ntok, length, 4, rank, 512, 1.0, p, p, floats, 0, 0, None)
+    assert latent(0, None, None)
+    assert not latent(2, None, ints(3, 3)) and "bad size" in err()
+    assert not latent(2, ints(3, 0), ints(3, 3)) and "portion 1" in err()
+    assert not latent(2, ints(3, 4), ints(3, 3)) and "portion 1" in err()
+    assert not latent(1, ints(3), ints(513)) and "len=513" in err()
+    assert not latent(1, ints(3), ints(512), 1000) and "scratch too small" in err()
+    assert not latent(1, ints(3), ints(3), 1000, 65) and "rank=65" in err()
+    g = sequence.AttentionArgs(4, 2, 64, 64, 128, 100, 1.0, p, p)
+    grouped = lambda n, ntok, length, floats=1 << 30: lib.llam_seq_attention_portions(
+        ctypes.byref(g), p, ctypes.byref(e), 0, n, ntok, length, p, 256, p, floats, 0, 0, None)
+    assert grouped(0, None, None)
+    assert not grouped(2, ints(3, 3), None) and "bad size" in err()
+    assert not grouped(2, ints(3, 4), ints(3, 3)) and "portion 1" in err()
+    assert not grouped(2, ints(3, 40), ints(3, 1000)) and "139 positions" in err()
+
+
 def test_bad_arguments_are_refused_before_any_launch():
     lib = sequence.load()
     buf = np.zeros(4096, np.uint8)
