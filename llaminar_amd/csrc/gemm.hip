@@ -769,6 +769,12 @@ namespace llamql
     //   384 x 25600 x 5120, Q4_K         194         339      267       303       236       201       201       208
     //   512 x 25600 x 5120, Q4_K         266         445      351       401       309       280       282       275
     //   2048 x 6400 x 5120, IQ3_S        263         518      473       410       350       322       279       272
+    // Tiles that fill their last round exactly, one round or several (us, gemm_kernel and the entry that is taken; Q4_K, Q6_K, IQ3_S):
+    //   1024 x 4096 x 4096    67.2, 75.3, 66.8 -> 59.5, 62.6, 59.0 (6)     512 x 16384 x 4096    130, 147, 130 -> 118, 124, 120 (6)
+    //   512 x 8192 x 12800    200, 228, 199 -> 172, 183, 174 (6)           40 x 32768 x 1024     15.4, 18.4, 16.7 -> 14.2, 17.0, 15.8 (4)
+    // and gemm_kernel's (us, gemm_kernel and the entry that would come next):
+    //   512 x 8192 x 768      17.2, 18.4, 17.4 : 18.2, 18.7, 18.4 (6)      16 x 32768 x 8192     49.3, 75.2, 67.7 : 55.5, 75.8, 69.2 (1)
+    //   1000 x 4096 x 512     13.1, 13.9, 13.0 : 13.3, 15.4, 13.2 (6)      256 x 16384 x 1024    21.3, 24.2, 21.4 : 21.7, 24.1, 22.0 (6)
     struct SplitTile
     {
         int mt, rn, ks;
@@ -796,9 +802,12 @@ namespace llamql
         const auto over = [](long a, long b) { return (a + b - 1) / b; };
         const int SB = K / 256;
         const WholeTile &whole = WHOLE[M <= 32 ? 0 : M <= 64 ? 1 : 2];
-        const long tiles = over(N, GEMM_BN) * over(M, whole.tokens), rest = tiles % (2 * cus);
-        const double undivided = WHOLE_START + SB * ((double)(tiles / (2 * cus)) * whole.full[format] +
-                                                     (rest == 0 ? 0.0 : rest <= cus ? whole.alone[format] : whole.last[format]));
+        const long tiles = over(N, GEMM_BN) * over(M, whole.tokens), rounds_before = (tiles - 1) / (2 * cus), rest = tiles - rounds_before * 2 * cus;
+        // (a last round that is exactly full is a last round all the same; but tiles of 32 tokens fare better in it, and the entry of
+        // the largest tiles, which alone rivals full rounds of 128 tokens, starts too slowly for walks of four super-blocks and less)
+        const bool light = rest == 2 * cus && (M <= 32 || (M > 64 && SB <= 4));
+        const double *last = rest <= cus ? whole.alone : light ? whole.full : whole.last;
+        const double undivided = WHOLE_START + SB * ((double)rounds_before * whole.full[format] + last[format]);
         double best = 0.97 * undivided;
         int choice = -1;
         for (int i = 0; i < (int)(sizeof(SPLIT) / sizeof(SPLIT[0])); ++i)

@@ -123,6 +123,7 @@ def test_a_walk_dealt_to_wavefronts(capi, dev, oracle, fmt, M, N, K):
     (64, 20001, 1024), (33, 24997, 1280),   # 64 x 128
     (97, 9799, 4352), (193, 8000, 2560),    # 128 x 64
     (128, 24997, 1280), (257, 8129, 2304),  # 128 x 128
+    (512, 8192, 1280),                      # one whole round of them
 ])
 def test_tiles_of_dealt_walks(capi, dev, oracle, fmt, M, N, K):
     """Every tile whose half super-blocks are dealt to wavefronts, with rows, tokens and super-blocks left over: each element

@@ -82,8 +82,11 @@ def gemm_choice(fmt, M, N, K):
     SB, kind = K // 256, 0 if M <= 32 else 1 if M <= 64 else 2
     full, last, alone = (t[fmt] for t in WHOLE[3 * kind:3 * kind + 3])
     tiles = over(N, 64) * over(M, (32, 64, 128)[kind])
-    rest = tiles % (2 * CUS)
-    best, choice = 0.97 * (WHOLE_START + SB * (tiles // (2 * CUS) * full + (0.0 if rest == 0 else alone if rest <= CUS else last))), -1
+    before = (tiles - 1) // (2 * CUS)
+    rest = tiles - before * 2 * CUS
+    light = rest == 2 * CUS and (M <= 32 or (M > 64 and SB <= 4))
+    end = alone if rest <= CUS else full if light else last
+    best, choice = 0.97 * (WHOLE_START + SB * (before * full + end)), -1
     for i, ((mt, rn, ks), step) in enumerate(SPLIT):
         groups = over(N, 32 * rn) * over(M, 32 * mt)
         left = groups % CUS
@@ -92,6 +95,27 @@ def gemm_choice(fmt, M, N, K):
         if us < best:
             best, choice = us, i
     return choice
+
+
+def test_the_prompt_gemm_takes_the_fastest_kernel_of_each_measured_size():
+    """The tables of measured times beside the rule: within 3 % of the fastest (two sizes of a table are that close)."""
+    names = ["Q4_K", "Q6_K", "IQ3_S"]
+    rows = re.findall(r"//   (\d+) x (\d+) x (\d+), (\w+) +([\d. ]+)\n", GEMM)
+    assert len(rows) == 16
+    for M, N, K, fmt, times in rows:
+        times = [float(t) for t in times.split()]
+        assert len(times) == 8
+        assert times[1 + gemm_choice(names.index(fmt), int(M), int(N), int(K))] <= 1.03 * min(times), (M, N, K, fmt)
+    number = r"([\d.]+), ([\d.]+), ([\d.]+)"
+    full = re.findall(rf"(\d+) x (\d+) x (\d+) +{number} (->|:) {number} \((\d)\)", GEMM)
+    assert len(full) == 8
+    for M, N, K, *rest in full:
+        M, N, K, entry = int(M), int(N), int(K), int(rest[7])
+        assert over(N, 64) * over(M, 32 if M <= 32 else 64 if M <= 64 else 128) % (2 * CUS) == 0
+        whole, other = [float(t) for t in rest[:3]], [float(t) for t in rest[4:7]]
+        for fmt in range(3):
+            assert gemm_choice(fmt, M, N, K) == (entry if rest[3] == "->" else -1)
+            assert (other if rest[3] == "->" else whole)[fmt] <= 1.01 * (whole if rest[3] == "->" else other)[fmt]
 
 
 def test_every_kernel_of_the_prompt_gemm_has_sizes():
