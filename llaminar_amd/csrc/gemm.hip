@@ -749,7 +749,7 @@ namespace llamql
     }
 
     // Which kernel a shape takes: -1 for gemm_kernel, or an entry of SPLIT.  gemm_kernel's workgroup walks the whole of K
-    // alone, two of them on a compute unit; gemm_split_kernel has one there and gives the walk to 2, 4 or 8 pairs of wavefronts.
+    // alone, two of them on a compute unit; gemm_split_kernel has one there and gives the walk to 2, 4 or 8 wavefronts.
     // The expected times in microseconds are fitted to measurements, weights from memory (us, gemm_kernel and the entries):
     //   tokens x rows x K             gemm_kernel  0: 1,1,4  1: 1,2,2  2: 2,1,4  3: 2,2,2  4: 2,4,1  5: 4,2,2  6: 4,4,1
     //   10 x 4096 x 4096, Q4_K           16.5         9.8     13.5      13.5      20.5      32.9      32.5      52.6

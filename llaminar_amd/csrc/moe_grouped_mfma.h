@@ -5,8 +5,9 @@
 // wavefront decodes 16 rows of a super-block at a time and every weight once for all pairs of the tile (the quad-lane
 // kernel below once for four pairs).  v_mfma_i32_16x16x32_i8 wants lane (c, l) to hold elements 8 l .. of one block of
 // row c: the four lanes of a row exchange quarters of their blocks with four lane swaps per pair of registers.  Operand
-// one is the pairs' activations, [block][pair][32] in LDS, so the exact block sums of pairs 4 l .. 4 l + 3 lie with row
-// c's scale; the scales are exchanged with the same swaps.
+// one is the pairs' activations, [block][pair][32] in LDS, so the exact block sums of pairs 4 l .. 4 l + 3 lie with row c.
+// The scales need no exchange: the matrix unit multiplies a lane's own by those of the pairs and leaves the products where the
+// block sums lie.  Minima (Q4_K) are exchanged with the same swaps.
 //
 // Bound by the decoders (vector instructions and, for IQ3_S, table gathers: the LDS is busy four fifths of the time), the
 // weights' bytes, and a workgroup's start (a chain of five loads; half as many row tiles a workgroup take 15 % longer, for all that
@@ -14,7 +15,7 @@
 // and one for all tokens, IQ3_S, 333 tokens of 9 slots: gate and up 279 -> 138 us, down 134 -> 70 us against one decode for
 // four pairs (the weights alone are 45 and 23 us of reads).  Scales multiplied on the matrix unit, sums without a conversion
 // and carries by branches are 258 instead of 352 vector instructions a super-block; whole feed-forwards, IQ3_S: 440 tokens, 128 experts of
-// 2048 x 1024 (32 pairs a tile) 324 -> 292 us, the 333 tokens above 228 -> 224; Q4_K 217 -> 207, 440 tokens, 64 of 4096 x 768 516 -> 470.
+// 2048 x 1024 (32 pairs a tile) 327 -> 292 us, the 333 tokens above 1 to 2 % (the tables); Q4_K 217 -> 208, 440 tokens, 64 of 4096 x 768 519 -> 470.
 #pragma once
 
 #include <type_traits>

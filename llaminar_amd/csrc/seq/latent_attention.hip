@@ -658,7 +658,10 @@ extern "C" bool llam_seq_latent_attention(const void *d_q, const void *d_cache, 
 }
 
 // Portions share a launch where that is no waste: as many as the scratch holds the partial results of, and none whose
-// stretches or rows would leave two thirds of the others' grid empty (a short portion far into its sequence has many stretches).
+// stretches or rows would leave two thirds of the others' grid empty (a short portion far into its sequence has many stretches: 64
+// tokens at position 8000 beside fifteen times 64 at 0, a step of Kogilix, width 2048, 2.33 -> 1.60 ms against one cut for all).
+// Eight portions of 251 tokens, 16 heads, rank 512: two a launch, 27 us and 44 of merging; alone 17.5 and 23 each; with one cut
+// for all 53 us and nothing to merge, but bits that depend on the others.
 extern "C" bool llam_seq_latent_portions(const void *d_q, const void *d_cache, const llam_seq_entries *e, int first, int n, const int *ntok,
                                          const int *len, int heads, int rank, int cap, float scale, void *d_o, float *d_scratch,
                                          size_t scratch_floats, int dtype, int device_id, void *stream)

@@ -149,9 +149,10 @@ namespace
         long run_rows = 0; // tokens of the last one
 
         // Another portion.  A launch of several takes as long as its longest, where a launch for each has few workgroups and
-        // pays for the latencies of its chain (eight prompts of 251 tokens and two steps, width 2048: Kogilix 5.0 -> 3.9 ms,
-        // Bosirax 3.55 -> 2.67); a grid is made for the longest, so a portion that would leave two thirds of it empty starts a run of
-        // its own.
+        // pays for the latencies of its chain (eight prompts of 251 tokens and two steps, width 2048, the attentions' launches shared
+        // as well: Kogilix 5.1 -> 4.3 ms, Bosirax 3.6 -> 2.7); a grid is made for the longest, so a portion that would leave two
+        // thirds of it empty starts a run of its own.  What a portion's outputs are does not depend on its run: every mixer cuts
+        // a portion up by its own length.
         void add(int entry, int tokens, int length)
         {
             ntok.push_back(tokens), len.push_back(length);
