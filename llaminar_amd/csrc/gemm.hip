@@ -30,6 +30,8 @@
 
 #include "llaminar_amd/ql_api.h"
 
+#include <type_traits>
+
 namespace llamql
 {
     typedef float v16f __attribute__((ext_vector_type(16)));
@@ -421,21 +423,24 @@ namespace llamql
     // ---- activations as they lie, a tile's K steps dealt to the wavefronts ------------------------
     // Tile of 32 MT tokens x 32 RN weight rows, a step of KS super-blocks, 2 KS RN = 8 wavefronts: wavefront (rn, kw) multiplies
     // half a super-block, the blocks of quad lanes 2 (kw % 2) and 2 (kw % 2) + 1, of rows 32 rn .. by all tokens of the tile, and
-    // the 2 KS partial sums are added through LDS in their order.  The weights never pass through LDS: lane (r, h) decodes
-    // what quad lane h of the half decodes, two whole blocks, and a swap of half registers between the lanes (r, 0) and (r, 1)
-    // makes both lanes' blocks into matrix operands.  The Q8_1 blocks of the tokens go from memory into LDS a step ahead, two
-    // buffers, one barrier a step: the quants as 16-byte pieces, [super-block][token][16], piece p of token m at p ^ (m & 15)
-    // (so that reads of 16 tokens' pieces meet no bank twice), the heads {d, sum} as [super-block][8 tokens][block][8], block k
-    // of the group of tokens g at k ^ (g & 7): a load of 64 heads reads 8 tokens' whole super-blocks, 24 cache lines, where a
-    // block of 64 tokens would read 64.
-    // What bounds it: the address unit of the loads (5000 of 11000 cycles a step when every lane's head was a line of its own and
-    // all loads were issued together, the wavefronts standing still meanwhile), then the vector unit: rescaling and decoding.  So
-    // the loads are dealt out among the products, a wavefront takes half a super-block of twice the tokens (half the decoding and
-    // half the loads of weights a product), and the matrix unit works on a product while the vector unit rescales the one before.
-    // One workgroup of eight wavefronts fits a compute unit (up to 250 registers a lane).
-    // Against whole super-blocks a wavefront and loads together: 199 x 5120 x 25600 Q6_K 272 -> 207 us, 40 x 8192 x 5120 IQ3_S
-    // 23.3 -> 19.0, 256 x 8192 x 8192 Q4_K 79 -> 65, 63 x 5034 x 18944 Q6_K 93 -> 70.5, 130 x 5000 x 5120 Q4_K 29.2 -> 26.7.
-    // The sums are kept in 2 to 8 parts: their error against 64 bits is 0.5 to 0.9 times gemm_kernel's.
+    // the 2 KS partial sums are added through LDS, always by the same twos.  Lane (r, h) decodes what quad lane h of the half decodes, two
+    // whole blocks, and a swap of half registers between the lanes (r, 0) and (r, 1) makes both lanes' blocks into matrix operands.
+    // The wavefront's raw weights come by way of LDS where it has room (HalfRows).  The Q8_1 blocks of the tokens go from memory
+    // into LDS a step ahead, two buffers, one barrier a step: the quants as 16-byte pieces, [super-block][token][16], piece p of
+    // token m at p ^ (m & 15) (so that reads of 16 tokens' pieces meet no bank twice), the heads {d, sum} as
+    // [super-block][token][8], block k of token m at k ^ (m / 8 & 7).
+    // The weights are the products' first operand, so a lane holds 16 rows' sums of one token: its scale is one register, the rows'
+    // scales, copied into that layout by the matrix unit once for all tokens of the tile, are 16.  A block sum then costs two
+    // multiply-adds (rescale below), where a subtraction, a multiply-add and a 32-bit matrix product for the pairs of scales took 352
+    // cycles for two products, two wavefronts a SIMD unit: now 221 to 239 (products with 32-bit operands hold the vector unit up).
+    // What bounds it: a step's time is the sum of what its two wavefronts a SIMD unit decode and rescale, as far as loads, swaps
+    // and the first products do not add to it (step of 128 x 128, Q6_K: 6350 cycles; decoding 1000 and 16 products 1750 of each of the
+    // two).  The older wavefront of the two is served first and waited at the barrier for a third of the step, so decoding goes
+    // ahead of rescaling, and the younger's rescaling ahead of the older's.  One workgroup of eight wavefronts fits a compute unit.
+    // Against a subtraction, a multiply-add and scales on the 32-bit matrix unit, weights straight into registers: 199 x 5120 x 25600
+    // Q6_K 206 -> 143 us (tiles of 96 x 64; of 128 x 64 that walk is 182), 40 x 8192 x 5120 IQ3_S 21.8 -> 18.2, 512 x 25600 x 5120
+    // Q4_K 270 -> 227 (gemm_kernel before; two launches now), 256 x 25600 x 5120 Q4_K 140 -> 137, 130 x 5000 x 5120 Q4_K 26.5 -> 23.5, 63 x 5034 x 18944 Q6_K 71 -> 62.
+    // Errors against 64 bits: 0.8 to 0.95 times those before (199 x 5120 x 25600 Q6_K 2.57e-7 -> 2.27e-7, 40 x 8192 x 5120 9.9e-8 -> 8.0e-8).
     template <int MT, int RN, int KS>
     struct GemmSplit
     {
@@ -444,13 +449,18 @@ namespace llamql
         static constexpr int QLOADS = QUANTS / 1024 / WAVES, HLOADS = HEADS / 256 / WAVES; // per wavefront
         static constexpr int QROWS = 4 * WAVES;                  // tokens x super-blocks that one load of every wavefront covers
         static constexpr int QM = BM > QROWS ? BM / QROWS : 1;   // tokens a lane loads pieces of
-        static constexpr int HM = BM > 8 * WAVES ? BM / (8 * WAVES) : 1; // tokens a lane loads heads of
+        static constexpr int HM = 8 * WAVES % BM == 0 ? 1 : BM % (8 * WAVES) == 0 ? BM / (8 * WAVES) : HLOADS; // tokens a lane loads heads of
         static_assert(QLOADS * WAVES * 1024 == QUANTS && HLOADS * WAVES * 256 == HEADS, "whole loads");
         static_assert(QROWS % 16 == 0 && (BM % QROWS == 0 || QROWS % BM == 0), "a lane's piece and tokens stay the same");
-        static_assert(BM % (8 * WAVES) == 0 || 8 * WAVES % BM == 0, "a lane's tokens stay the same");
         static constexpr size_t STAGE = QUANTS + HEADS;
-        static constexpr size_t SUMS = (size_t)(KW - 1) * RN * MT * 16 * WAVE * sizeof(float);
-        static constexpr size_t LDS = 2 * STAGE > SUMS ? 2 * STAGE : SUMS;
+        static constexpr size_t SUMS = (size_t)KW * RN * MT * 16 * WAVE * sizeof(float);
+        // with `half` bytes of raw weights a wavefront beside the activations, where there is room for them
+        static constexpr bool raw_lds(size_t half) { return 2 * STAGE + WAVES * half + 6 * 1024 <= 160 * 1024; }
+        static constexpr size_t lds(size_t half)
+        {
+            const size_t walk = 2 * STAGE + (raw_lds(half) ? WAVES * half : 0), end = SUMS + 4 * WAVES;
+            return walk > end ? walk : end;
+        }
     };
 
     // Block sums as floats without a conversion: the products start from the bits of 1.5 * 2^23 instead of zero, so that the bits of
@@ -493,9 +503,29 @@ namespace llamql
         if (n >= g.w.N)
             n = g.w.N - 1; // tail rows: decode a valid row, never stored
         const typename Q::Lane lc = Q::lane_consts(lh + 2 * half);
+        const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)smem;
+        // the weights, by way of LDS or, where the activations leave no room, straight into registers (and three loads for one token
+        // tile: 12 x 1483 x 20992 Q4_K 31.1 -> 29.8 us)
+        constexpr bool RAW_LDS = G::raw_lds(Q::Half::BYTES) && !(MT == 1 && F::HAS_MIN);
         const typename Q::Cursor wc = Q::cursor(g.w, (size_t)n * SB, (size_t)n * SB, lc);
+        typename Q::Half rows_half;
+        if constexpr (RAW_LDS)
+            rows_half.init(g.w, n0, half, lane);
+        const uint32_t raw_at = (uint32_t)(2 * G::STAGE) + (uint32_t)(wave * Q::Half::BYTES);
         typename Q::Raw raw;
-        auto issue_weights = [&](int sb) { Q::load_at(raw, wc, lc, sb < SB ? sb : SB - 1); }; // (past the end: the last super-block again)
+        auto issue_weights = [&](int sb) __attribute__((always_inline)) {
+            const int at = sb < SB ? sb : SB - 1; // (past the end: the last super-block again)
+            if constexpr (RAW_LDS)
+                rows_half.load(lds0 + raw_at, at);
+            else
+                Q::load_at(raw, wc, lc, at);
+        };
+        auto wait_weights = [&]() __attribute__((always_inline)) {
+            if constexpr (RAW_LDS)
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            else
+                Q::template wait<0>(raw);
+        };
         // bytes from the tile's first token to what this lane loads of super-block 0 (past the last token: the last one)
         const uint8_t *abase = reinterpret_cast<const uint8_t *>(g.q8 + (size_t)m0 * KB * 9);
         auto token = [&](int m) { return (uint32_t)(m0 + m < g.M ? m : g.M - 1 - m0) * (uint32_t)(KB * 36); };
@@ -509,57 +539,68 @@ namespace llamql
             for (int i = 0; i < G::HM; ++i)
             {
                 const int group = (wave + i * G::WAVES) % (BM / 8);
-                hfrom[i] = token(group * 8 + (lane & 7)) + (uint32_t)((lane >> 3) ^ (group & 7)) * 36;
+                hfrom[i] = token(group * 8 + (lane >> 3)) + (uint32_t)((lane & 7) ^ (group & 7)) * 36;
             }
         }
-        const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)smem;
-        auto super_block = [&](int sb) { return abase + (size_t)(sb < SB ? sb : SB - 1) * 288; }; // (past the end: the last one)
-        // Load i of the step of super-block sb0, where there is one: else no lane takes part (a branch among the products would
-        // have the compiler copy their registers at its ends).
+        // Load i of the step of super-block sb0 (past the end: the last super-block); `lanes` are none where there is no such step (a
+        // branch among the products would have the compiler copy their registers at its ends).
         constexpr int LOADS = G::QLOADS + G::HLOADS;
-        auto issue_act = [&](int i, int sb0, int buf) {
-            uint64_t all;
-            if (i < G::QLOADS)
-                asm volatile("s_mov_b32 m0, %1\n\ts_mov_b64 %0, exec\n\ts_cmp_lt_i32 %4, %5\n\ts_cselect_b64 exec, -1, 0\n\tglobal_load_lds_dwordx4 %2, %3\n\ts_mov_b64 exec, %0"
-                             : "=&s"(all)
-                             : "s"(lds0 + (uint32_t)(buf * (int)G::STAGE + wave * 1024 + i * G::WAVES * 1024)), "v"(qfrom[i % G::QM]),
-                               "s"(super_block(sb0 + (wave * 4 + i * G::QROWS) / BM)), "s"(sb0), "s"(SB)
-                             : "memory", "scc");
+        auto issue_act = [&](int i, int sb0, int buf, uint64_t lanes) {
+            const bool quants = i < G::QLOADS;
+            const int h = i - G::QLOADS, part = KS == 1 ? 0 : quants ? (wave * 4 + i * G::QROWS) / BM : (wave + h * G::WAVES) / (BM / 8);
+            const uint8_t *from = abase + (size_t)(sb0 + part < SB ? sb0 + part : SB - 1) * 288;
+            const uint32_t to = lds0 + (uint32_t)(buf * (int)G::STAGE + (quants ? wave * 1024 + i * G::WAVES * 1024 : G::QUANTS + wave * 256 + h * G::WAVES * 256));
+            if (quants)
+                asm volatile("s_mov_b32 m0, %0\n\ts_mov_b64 exec, %3\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b64 exec, -1"
+                             :: "s"(to), "v"(qfrom[i % G::QM]), "s"(from), "s"(lanes) : "memory");
             else
-            {
-                const int h = i - G::QLOADS;
-                asm volatile("s_mov_b32 m0, %1\n\ts_mov_b64 %0, exec\n\ts_cmp_lt_i32 %4, %5\n\ts_cselect_b64 exec, -1, 0\n\tglobal_load_lds_dword %2, %3\n\ts_mov_b64 exec, %0"
-                             : "=&s"(all)
-                             : "s"(lds0 + (uint32_t)(buf * (int)G::STAGE + G::QUANTS + wave * 256 + h * G::WAVES * 256)), "v"(hfrom[h % G::HM]),
-                               "s"(super_block(sb0 + (wave + h * G::WAVES) / (BM / 8))), "s"(sb0), "s"(SB)
-                             : "memory", "scc");
-            }
+                asm volatile("s_mov_b32 m0, %0\n\ts_mov_b64 exec, %3\n\tglobal_load_lds_dword %1, %2\n\ts_mov_b64 exec, -1"
+                             :: "s"(to), "v"(hfrom[h % G::HM]), "s"(from), "s"(lanes) : "memory");
         };
         const v16i bias = integer_bias();
-        v16f acc[MT];
+        v16f acc[MT], zero1f;
+        v32f zero2f;
+#pragma unroll
+        for (int r = 0; r < 32; ++r)
+            zero2f[r] = 0.0f;
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+            zero1f[r] = 0.0f;
+
+        // The walk along K.  WHOLE: the sums as such, for tiles that hold something infinite or not a number.
+        auto walk = [&](auto whole) __attribute__((always_inline)) {
+        constexpr bool WHOLE = decltype(whole)::value;
 #pragma unroll
         for (int t = 0; t < MT; ++t)
 #pragma unroll
             for (int r = 0; r < 16; ++r)
                 acc[t][r] = 0.0f;
-        v32f zero2f;
-#pragma unroll
-        for (int r = 0; r < 32; ++r)
-            zero2f[r] = 0.0f;
-
+        int first = 0;
+        asm volatile("" : "+s"(first)); // (addresses of both walks known ahead would fill the scalar registers)
 #pragma unroll
         for (int i = 0; i < LOADS; ++i)
-            issue_act(i, 0, 0);
+            issue_act(i, first, 0, ~0ull);
         issue_weights(own_sb);
         int buf = 0;
         for (int sb0 = 0; sb0 < SB; sb0 += KS, buf ^= 1)
         {
             const int sb = sb0 + own_sb;
+            uint64_t more;
+            asm("s_cmp_lt_i32 %1, %2\n\ts_cselect_b64 %0, -1, 0" : "=s"(more) : "s"(sb0 + KS), "s"(SB) : "scc");
             // this step's weights and activations have arrived, everybody is done with the other buffer
-            Q::template wait<0>(raw);
+            wait_weights();
             asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            __builtin_amdgcn_s_setprio(2);
             v4i w[4];
             typename Q::Scale S;
+            if constexpr (RAW_LDS)
+            {
+                Q::Half::read(raw, smem + raw_at, l32, lh);
+                Q::keep(raw);
+                // (read, before they are asked for again; ahead of the decoding, to leave while it goes on)
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                issue_weights(sb + KS);
+            }
             Q::decode(raw, lc, w, S);
             // decoded here, before the registers are asked for again: sunk below, the decoding would have the compiler copy
             // the raw words, and copies made ahead of the wait hold what the loads have not brought yet
@@ -568,12 +609,13 @@ namespace llamql
             S = __builtin_bit_cast(typename Q::Scale, two);
             __builtin_amdgcn_sched_barrier(0);
             // (the weights at once: they come from memory, and dealt out behind the products they were waited for)
-            issue_weights(sb + KS);
+            if constexpr (!RAW_LDS)
+                issue_weights(sb + KS);
             __builtin_amdgcn_sched_barrier(0);
             if (sb < SB) // uniform in the wavefront
             {
                 const uint8_t *rows = smem + buf * G::STAGE + (size_t)(own_sb * BM + l32) * 256;
-                const uint32_t *heads = reinterpret_cast<const uint32_t *>(smem + buf * G::STAGE + G::QUANTS) + own_sb * 8 * BM + (l32 >> 3) * 64 + (l32 & 7);
+                const uint32_t *heads = reinterpret_cast<const uint32_t *>(smem + buf * G::STAGE + G::QUANTS) + own_sb * 8 * BM + l32 * 8;
                 // block x of the half's first quad lane, block y of its second: elements 0 .. 15 with lanes (r, 0), 16 .. 31 with (r, 1)
 #pragma unroll
                 for (int i = 0; i < 2; ++i)
@@ -584,121 +626,260 @@ namespace llamql
                         const v2u s = __builtin_bit_cast(v2u, __builtin_amdgcn_permlane32_swap((uint32_t)w[2 * i][d], (uint32_t)w[2 * i + 1][d], false, false));
                         w[2 * i][d] = (int)s[0], w[2 * i + 1][d] = (int)s[1];
                     }
-                // Product j: pair of blocks j / MT by tokens 32 (j % MT) ...  The matrix unit works on a product while the vector
+                // Product j: pair of blocks i_of(j) by tokens 32 t_of(j) ...  The matrix unit works on a product while the vector
                 // unit rescales the one before it, and the LDS brings the operands of the next.
                 constexpr int JOBS = 2 * MT, EACH = (LOADS + JOBS - 1) / JOBS;
+                // (tokens by tokens, where the rows' scales of all four blocks fit the registers)
+                constexpr bool APART = KW < 8 && (MT > 1 || !F::HAS_MIN) && (MT < 4 || RAW_LDS), FOURS = APART && (MT == 1 || (MT == 2 && RAW_LDS));
+                auto t_of = [](int j) { return FOURS ? j >> 1 : j % MT; };
+                auto i_of = [](int j) { return FOURS ? j & 1 : j / MT; };
                 auto fence = []() __attribute__((always_inline)) {
                     if (MT > 1) // (two products of a step are not enough for it: the compiler's order is 10 % faster)
                         __builtin_amdgcn_sched_barrier(0);
                 };
-                auto block = [&](int j, int which) { return Q::block_of(2 * half + which, j / MT); };
+                auto block = [&](int j, int which) { return Q::block_of(2 * half + which, i_of(j)); };
                 auto quants = [&](int j, int which) {
-                    return *reinterpret_cast<const v4i *>(rows + (j % MT) * 32 * 256 + (((2 * block(j, which) + lh) ^ (l32 & 15)) << 4));
+                    return *reinterpret_cast<const v4i *>(rows + t_of(j) * 32 * 256 + (((2 * block(j, which) + lh) ^ (l32 & 15)) << 4));
                 };
-                auto head_of = [&](int j) { return heads[(((lh ? block(j, 1) : block(j, 0)) ^ ((j % MT & 1) * 4 + (l32 >> 3))) * 8) + (j % MT) * 256]; };
-                auto scale_of = [](uint32_t head) { return h2f((uint16_t)(head & 0xFFFFu)); };
-                // the scale products of both blocks, a rank-1 matrix each (exact: both factors are fp16 values)
-                auto scales = [&](int j, uint32_t head) { return __builtin_amdgcn_mfma_f32_32x32x1f32(scale_of(head), Q::scale_f32(S, j / MT), zero2f, 0, 0, 0); };
-                auto product = [&](int j, int which, v4i a) { return __builtin_amdgcn_mfma_i32_32x32x32_i8(a, w[2 * (j / MT) + which], bias, 0, 0, 0); };
+                auto head_of = [&](int j, int which) { return heads[(block(j, which) ^ ((t_of(j) & 1) * 4 + (l32 >> 3))) + t_of(j) * 256]; };
+                // a block's scales of the rows that a lane's sums belong to: the matrix unit copies them there (times one: exact)
+                auto scales = [&](int i, int which) {
+                    typedef _Float16 v4h __attribute__((ext_vector_type(4)));
+                    const _Float16 none = (_Float16)0.0f;
+                    const v4h own = {lh == which ? (_Float16)Q::scale_f32(S, i) : none, none, none, none};
+                    const v4h one = {(_Float16)1.0f, none, none, none};
+                    return __builtin_amdgcn_mfma_f32_32x32x8f16(own, one, zero1f, 0, 0, 0);
+                };
+                auto scales_of_both = [&](int i) {
+                    typedef _Float16 v4h __attribute__((ext_vector_type(4)));
+                    const _Float16 none = (_Float16)0.0f;
+                    const v4h own = {(_Float16)Q::scale_f32(S, i), none, none, none}, one = {(_Float16)1.0f, none, none, none};
+                    return __builtin_amdgcn_mfma_f32_32x32x4f16(own, one, zero2f, 0, 0, 0);
+                };
+                auto product = [&](int j, int which, v4i a) { return __builtin_amdgcn_mfma_i32_32x32x32_i8(w[2 * i_of(j) + which], a, bias, 0, 0, 0); };
                 auto dump = [&](int j, int which, const v16i &d) {
-                    const long nn = n0 + l32 - g.row0;
-                    if (n0 + l32 < g.w.N && nn >= 0 && nn < g.nrows)
+                    // (less than 2 GiB of sums: offsets of 32 bits, made anew for each, or they would fill the registers)
+                    const int m = (int)m0 + t_of(j) * 32 + l32, nn = (int)(n0 - g.row0) + 4 * lh;
+                    uint32_t at = ((uint32_t)m * (uint32_t)g.nrows + (uint32_t)nn) * (uint32_t)KB + (uint32_t)(sb * 8 + block(j, which));
+                    if (m < g.M)
                     {
-                        // (less than 2 GiB of sums: offsets of 32 bits, made anew for each, or they would fill the registers)
-                        const uint32_t token = (uint32_t)g.nrows * (uint32_t)KB;
-                        uint32_t at = ((uint32_t)m0 + 4 * lh) * token + (uint32_t)nn * (uint32_t)KB + (uint32_t)(sb * 8 + block(j, which));
 #pragma unroll
                         for (int r = 0; r < 16; ++r)
                         {
-                            const int m = j % MT * 32 + 8 * (r >> 2) + (r & 3);
+                            const int row = 8 * (r >> 2) + (r & 3);
                             asm volatile("" : "+v"(at));
-                            if (m0 + 4 * lh + m < g.M)
-                                g.sums[at + (uint32_t)m * token] = (int32_t)biased_to_float(d[r]);
+                            if (n0 + 4 * lh + row < g.w.N && nn + row >= 0 && nn + row < g.nrows)
+                                g.sums[at + (uint32_t)row * (uint32_t)KB] = (int32_t)biased_to_float(d[r]);
                         }
                     }
                 };
-                uint32_t head[2] = {head_of(0), 0};
-                v32f cs[2];
-                cs[0] = scales(0, head[0]);
+                // Two multiply-adds a sum: biased sum times the token's scale less bias times scale is the sum times the scale, rounded
+                // once, and that times the row's scale.  Four blocks of a token, or two of four, are added up by themselves before they
+                // meet the sum of those before them: the roundings at the size of the whole sum are 1 or 3 instead of 4, which more than
+                // makes up for the one more here, at one addition to eight multiply-adds (eight partial sums need it not; nor do one
+                // token tile's with minima, which gain nothing by it, and 128 x 64, which has no registers for it).
+                v16f apart;
+                auto rescale = [&](int j, int which, const v16i &d, uint32_t head, const v16f &cs) __attribute__((always_inline)) {
+                    typedef float v2f __attribute__((ext_vector_type(2)));
+                    typedef float v8f __attribute__((ext_vector_type(8)));
+                    const int t = t_of(j), n = 2 * i_of(j) + which; // the n-th of a token's four blocks
+                    const bool plain = !APART || (!FOURS && n >= 2), last = n == (FOURS ? 3 : 1);
+                    v2f da; // {scale, offset}
+                    da[0] = h2f((uint16_t)(head & 0xFFFFu));
+                    da[1] = -BIAS * da[0];
+                    if (!WHOLE)
+                        asm("" : "+v"(da)); // (floats from here on: v_fma_mix_f32, which would read the half, takes twice as long)
+#pragma unroll
+                    for (int r = 0; r < 16; r += 8)
+                    {
+                        v8f s; // (that of row r + i in place i ^ 1: an instruction waits for three operands of even, or three of odd registers)
+#pragma unroll
+                        for (int i = 0; i < 8; ++i)
+                            s[i ^ 1] = WHOLE ? biased_to_float(d[r + i]) : fmaf(__int_as_float(d[r + i]), da[0], da[1]);
+                        if (!WHOLE)
+                            asm("" : "+v"(s));
+#pragma unroll
+                        for (int i = 0; i < 8; ++i)
+                        {
+                            const float c = WHOLE ? da[0] * cs[r + i] : cs[r + i];
+                            if (plain)
+                                acc[t][r + i] = fmaf(s[i ^ 1], c, acc[t][r + i]);
+                            else if (n == 0)
+                                apart[r + i] = s[i ^ 1] * c;
+                            else if (!last)
+                                apart[r + i] = fmaf(s[i ^ 1], c, apart[r + i]);
+                            else
+                                acc[t][r + i] += fmaf(s[i ^ 1], c, apart[r + i]);
+                        }
+                    }
+                };
+                // Minima times the tokens' scaled sums.  The matrix unit's 32-bit products hold the vector unit up for all of their 64
+                // cycles; of bf16 it does 16 in 32, so three pieces of a sum that add up to it (24 bits) times the two of a minimum (11).
+                constexpr bool PIECES = !WHOLE && MT > 1; // (of one token tile their making would take longer)
+                v4i low[2];
+                if constexpr (F::HAS_MIN && PIECES)
+#pragma unroll
+                    for (int i = 0; i < 2; ++i)
+                    {
+                        const float m = Q::min_f32(S, i), m1 = __uint_as_float(and_k<0xFFFF0000u>(__float_as_uint(m))), m2 = m - m1;
+                        const uint32_t u1 = __float_as_uint(m1), u2 = __float_as_uint(m2);
+                        low[i] = (v4i){(int)(u1 | u1 >> 16), (int)(u2 | u2 >> 16), (int)u1, (int)u2};
+                    }
+                const uint32_t upper = vector_constant(lh ? ~0u : 0u);
+                auto add_minima = [&](int j, uint32_t x, uint32_t y) __attribute__((always_inline)) {
+                    const uint32_t h = bit_select(y, x, upper);
+                    const float sum = (float)(int16_t)(h >> 16) * h2f((uint16_t)(h & 0xFFFFu));
+                    if constexpr (!PIECES)
+                        acc[t_of(j)] = __builtin_amdgcn_mfma_f32_32x32x2f32(Q::min_f32(S, i_of(j)), sum, acc[t_of(j)], 0, 0, 0);
+                    else
+                    {
+                        typedef __bf16 v8b __attribute__((ext_vector_type(8)));
+                        const float p1 = __uint_as_float(and_k<0xFFFF0000u>(__float_as_uint(sum))), rest = sum - p1;
+                        const float p2 = __uint_as_float(and_k<0xFFFF0000u>(__float_as_uint(rest))), p3 = rest - p2;
+                        const int both = (int)__builtin_amdgcn_perm(__float_as_uint(p2), __float_as_uint(p1), 0x07060302u);
+                        // slots p1 p2 p1 p2 0 p3 0 p3 of the block of either half of the lanes, times m1 m1 m2 m2 0 m1 0 m2
+                        const v4i pieces = {both, both, __float_as_int(p3), __float_as_int(p3)};
+                        acc[t_of(j)] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8b, low[i_of(j)]), __builtin_bit_cast(v8b, pieces), acc[t_of(j)], 0, 0, 0);
+                    }
+                };
+#pragma unroll
+                for (int t = 0; t < MT; ++t)
+                    if (!DUMP)
+                        asm("" : "+v"(acc[t]));
+                v16f cs[4];
+                if constexpr (MT <= 2)
+                {
+#pragma unroll
+                    for (int i = 0; i < 2; ++i)
+                    {
+                        const v32f both = scales_of_both(i);
+                        cs[2 * i] = __builtin_shufflevector(both, both, 0, 1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15);
+                        cs[2 * i + 1] = __builtin_shufflevector(both, both, 16, 17, 18, 19, 20, 21, 22, 23, 24, 25, 26, 27, 28, 29, 30, 31);
+                    }
+                }
+                else
+                    cs[0] = scales(0, 0), cs[1] = scales(0, 1);
+                uint32_t hx = head_of(0, 0), hy = head_of(0, 1);
                 v16i dx = product(0, 0, quants(0, 0)), dy = product(0, 1, quants(0, 1));
+                // (of one and two token tiles, too: 12 x 1483 x 20992 Q6_K 40.4 -> 35.8 us)
+                if (wave >= G::WAVES / 2)
+                    __builtin_amdgcn_s_setprio(1);
+                else
+                    __builtin_amdgcn_s_setprio(0);
 #pragma unroll
                 for (int j = 0; j < JOBS; ++j)
                 {
-                    const int t = j % MT, now = j & 1, next = now ^ 1;
-                    v4i a;
+                    v4i a, b;
+                    uint32_t nx = 0, ny = 0;
+                    fence();
+                    if (j + 1 < JOBS)
+                    {
+                        nx = head_of(j + 1, 0), ny = head_of(j + 1, 1);
+                        a = quants(j + 1, 0), b = quants(j + 1, 1);
+                    }
                     fence();
 #pragma unroll
                     for (int i = j * EACH; i < (j + 1) * EACH; ++i)
                         if (i < LOADS)
-                            issue_act(i, sb0 + KS, buf ^ 1);
+                            issue_act(i, sb0 + KS, buf ^ 1, more);
                     fence();
-                    if (j + 1 < JOBS)
-                    {
-                        head[next] = head_of(j + 1);
-                        a = quants(j + 1, 0);
-                    }
                     if (DUMP)
                         dump(j, 0, dx);
-#pragma unroll
-                    for (int r = 0; r < 16; ++r)
-                        acc[t][r] = fmaf(biased_to_float(dx[r]), cs[now][r], acc[t][r]);
+                    else
+                        rescale(j, 0, dx, hx, cs[2 * i_of(j)]);
                     fence();
                     if (j + 1 < JOBS)
-                    {
-                        cs[next] = scales(j + 1, head[next]);
                         dx = product(j + 1, 0, a);
-                        a = quants(j + 1, 1);
-                    }
+                    if (MT > 2 && j + 1 == MT)
+                        cs[2] = scales(1, 0);
                     fence();
                     if (DUMP)
                         dump(j, 1, dy);
-#pragma unroll
-                    for (int r = 0; r < 16; ++r)
-                        acc[t][r] = fmaf(biased_to_float(dy[r]), cs[now][16 + r], acc[t][r]);
+                    else
+                        rescale(j, 1, dy, hy, cs[2 * i_of(j) + 1]);
                     fence();
                     if (j + 1 < JOBS)
-                        dy = product(j + 1, 1, a);
-                    if (F::HAS_MIN)
-                        acc[t] = __builtin_amdgcn_mfma_f32_32x32x2f32((float)(int16_t)(head[now] >> 16) * scale_of(head[now]), Q::min_f32(S, j / MT), acc[t], 0, 0, 0);
+                        dy = product(j + 1, 1, b);
+                    if (MT > 2 && j + 1 == MT)
+                        cs[3] = scales(1, 1);
+                    if (F::HAS_MIN && !DUMP)
+                        add_minima(j, hx, hy);
+                    hx = nx, hy = ny;
                 }
             }
         }
-        Q::template wait<0>(raw);
+        wait_weights();
+        };
+        walk(std::integral_constant<bool, DUMP>());
         if (DUMP)
             return;
 
-        __syncthreads(); // everybody is done with the activations
+        // The KW partial sums of a place are added by twos, by all wavefronts: wavefront kw adds and stores the kw-th part of
+        // its tile's registers.
+        constexpr int SHARE = MT * 16 / KW, AT_ONCE = SHARE < 4 ? SHARE : 4;
         float *red = reinterpret_cast<float *>(smem) + rn * MT * 16 * WAVE + lane;
-        if (kw > 0)
-        {
-#pragma unroll
-            for (int t = 0; t < MT; ++t)
-#pragma unroll
-                for (int r = 0; r < 16; ++r)
-                    red[((kw - 1) * RN * MT * 16 + t * 16 + r) * WAVE] = acc[t][r];
-        }
-        __syncthreads();
-        if (kw > 0)
-            return;
-        // (not unrolled: all sums asked for at once would not fit the registers)
-#pragma unroll 1
-        for (int k = 0; k < KW - 1; ++k)
-#pragma unroll
-            for (int t = 0; t < MT; ++t)
-#pragma unroll
-                for (int r = 0; r < 16; ++r)
-                    acc[t][r] += red[(k * RN * MT * 16 + t * 16 + r) * WAVE];
-        if (n0 + l32 < g.w.N)
-        {
+        int *odd = reinterpret_cast<int *>(smem + G::SUMS);
+        auto gather = [&]() __attribute__((always_inline)) {
+            float finite = 0.0f;
+            __syncthreads(); // everybody is done with the activations
 #pragma unroll
             for (int t = 0; t < MT; ++t)
 #pragma unroll
                 for (int r = 0; r < 16; ++r)
                 {
-                    const long m = m0 + t * 32 + 8 * (r >> 2) + 4 * lh + (r & 3);
-                    if (m < g.M)
-                        g.y[(size_t)m * g.ldy + n0 + l32] = acc[t][r];
+                    finite = fmaf(acc[t][r], 0.0f, finite);
+                    red[(kw * RN * MT * 16 + t * 16 + r) * WAVE] = acc[t][r];
                 }
+            if (lane == 0)
+                odd[wave] = 0;
+            if (!(finite == 0.0f))
+                odd[wave] = 1;
+            __syncthreads();
+            int any = 0;
+            for (int i = 0; i < G::WAVES; ++i)
+                any |= odd[i];
+            return __builtin_amdgcn_readfirstlane(any) != 0;
+        };
+        if (__builtin_expect(gather(), 0))
+        {
+            __syncthreads();
+            walk(std::true_type());
+            gather();
+        }
+        // a lane holds a token's sums of rows 8 k + 4 lh .. + 3
+        typedef float vf_dword __attribute__((ext_vector_type(AT_ONCE), aligned(4)));
+#pragma unroll
+        for (int q = 0; q < SHARE; q += AT_ONCE)
+        {
+            const int reg = kw * SHARE + q, r = reg & 15; // uniform
+            const long m = m0 + (reg >> 4) * 32 + l32;
+            vf_dword sum;
+#pragma unroll
+            for (int i = 0; i < AT_ONCE; ++i)
+            {
+                float part[KW];
+#pragma unroll
+                for (int k = 0; k < KW; ++k)
+                    part[k] = red[(k * RN * MT * 16 + reg + i) * WAVE];
+#pragma unroll
+                for (int k = 1; k < KW; k *= 2)
+#pragma unroll
+                    for (int l = 0; l < KW; l += 2 * k)
+                        part[l] += part[l + k];
+                sum[i] = part[0];
+            }
+            const long at = n0 + 8 * (r >> 2) + 4 * lh + (r & 3), left = g.w.N - at;
+            if (m < g.M && left > 0)
+            {
+                float *y = g.y + (size_t)m * g.ldy + at;
+                if (left >= AT_ONCE)
+                    *reinterpret_cast<vf_dword *>(y) = sum;
+                else
+#pragma unroll
+                    for (int i = 0; i < AT_ONCE - 1; ++i)
+                        if (i < left)
+                            y[i] = sum[i];
+            }
         }
     }
 
@@ -736,7 +917,7 @@ namespace llamql
     template <class F, bool DUMP, int MT, int RN, int KS>
     bool gemm_split_launch(const char *fn, const GemmArgs &g, int rows, int M, hipStream_t st)
     {
-        constexpr size_t lds = GemmSplit<MT, RN, KS>::LDS;
+        constexpr size_t lds = GemmSplit<MT, RN, KS>::lds(F::Quad::Half::BYTES);
         static_assert(lds + 6 * 1024 <= 160 * 1024, "LDS, with the decoders' tables");
         static LdsGrant grant;
         const auto kernel = &gemm_split_kernel<F, MT, RN, KS, DUMP>;
@@ -751,39 +932,51 @@ namespace llamql
     // Which kernel a shape takes: -1 for gemm_kernel, or an entry of SPLIT.  gemm_kernel's workgroup walks the whole of K
     // alone, two of them on a compute unit; gemm_split_kernel has one there and gives the walk to 2, 4 or 8 wavefronts.
     // The expected times in microseconds are fitted to measurements, weights from memory (us, gemm_kernel and the entries):
-    //   tokens x rows x K             gemm_kernel  0: 1,1,4  1: 1,2,2  2: 2,1,4  3: 2,2,2  4: 2,4,1  5: 4,2,2  6: 4,4,1
-    //   10 x 4096 x 4096, Q4_K           16.5         9.8     13.5      13.5      20.5      32.9      32.5      52.6
-    //   64 x 4096 x 4096, IQ3_S          31.3        12.6     18.3      16.7      23.6      38.2      33.7      55.0
-    //   20 x 12000 x 4096, IQ3_S         23.1        21.6     18.5      28.9      24.1      38.2      34.5      55.2
-    //   40 x 8192 x 5120, IQ3_S          38.4        25.2     21.9      19.0      28.7      46.8      40.7      67.7
-    //   63 x 5034 x 18944, Q6_K          162         103      96.0      70.5      114       201       153       279
-    //   130 x 5000 x 5120, Q4_K          52.2        36.7     30.0      33.2      26.7      40.7      40.9      65.6
-    //   64 x 25600 x 5120, Q4_K          53.8        68.1     60.0      68.4      51.9      45.1      82.0      70.5
-    //   80 x 9762 x 3072, Q6_K           37.3        38.1     31.7      39.8      37.8      31.9      29.1      45.3
-    //   199 x 5120 x 25600, Q6_K         298         298      314       230       260       241       207       369
-    //   256 x 8192 x 8192, Q4_K          86.2        122      92.2      97.1      75.8      65.7      64.8      106
-    //   1000 x 4096 x 4096, Q4_K         65.8        122      94.1      110       79.4      66.5      68.1      57.8
-    //   256 x 25600 x 5120, Q4_K         154         228      184       211       167       160       161       140
-    // and gemm_kernel's shapes, tiles of 32 tokens in one round, or three and more rounds of tiles of 128:
-    //   16 x 25600 x 5120, Q6_K          49.9        65.1     57.7      77.0      67.4      59.0      93.0      83.2
-    //   384 x 25600 x 5120, Q4_K         194         339      267       303       236       201       201       208
-    //   512 x 25600 x 5120, Q4_K         266         445      351       401       309       280       282       275
-    //   2048 x 6400 x 5120, IQ3_S        263         518      473       410       350       322       279       272
+    //   tokens x rows x K             gemm_kernel  0: 1,1,4  1: 1,2,2  2: 2,1,4  3: 2,2,2  4: 2,4,1  5: 3,2,2  6: 4,4,1
+    //   10 x 4096 x 4096, Q4_K            17.0      8.8     12.9     12.3     17.6     28.7     23.2     48.3
+    //   64 x 4096 x 4096, IQ3_S           31.7     11.1     16.2     14.5     19.9     34.1     24.3     48.3
+    //   20 x 12000 x 4096, IQ3_S          25.7     20.0     17.3     27.9     21.0     34.7     25.9     49.0
+    //   40 x 8192 x 5120, IQ3_S           42.0     24.3     20.8     18.2     24.4     42.8     30.6     60.3
+    //   63 x 5034 x 18944, Q6_K            158     78.2     69.9     62.4     87.3      150      104      207
+    //   130 x 5000 x 5120, Q4_K           53.2     39.7     34.6     29.8     23.5     36.2     29.5     61.1
+    //   64 x 25600 x 5120, Q4_K           56.8     73.9     69.6     63.3     46.8     41.7     59.5     65.0
+    //   80 x 9762 x 3072, Q6_K            42.1     35.1     28.0     36.8     32.0     30.4     23.1     40.6
+    //   199 x 5120 x 25600, Q6_K           303      236      241      223      200      204      144      285
+    //   256 x 8192 x 8192, Q4_K           91.9      124      102     93.0     67.2     62.2     87.4     97.3
+    //   1000 x 4096 x 4096, Q4_K          69.3      131      107     97.5     71.0     62.3     72.9     57.6
+    //   256 x 25600 x 5120, Q4_K           156      252      222      194      156      149      157      137
+    //   16 x 25600 x 5120, Q6_K           50.1     51.3     45.4     72.0     54.1     50.0     63.8     66.3
+    //   384 x 25600 x 5120, Q4_K           203      380      322      282      220      195      218      198
+    //   512 x 25600 x 5120, Q4_K           271      500      423      370      286      261      306      264
+    //   2048 x 6400 x 5120, IQ3_S          264      515      465      367      296      291      275      257
     // Tiles that fill their last round exactly, one round or several (us, gemm_kernel and the entry that is taken; Q4_K, Q6_K, IQ3_S):
-    //   1024 x 4096 x 4096    67.2, 75.3, 66.8 -> 59.5, 62.6, 59.0 (6)     512 x 16384 x 4096    130, 147, 130 -> 118, 124, 120 (6)
-    //   512 x 8192 x 12800    200, 228, 199 -> 172, 183, 174 (6)           40 x 32768 x 1024     15.4, 18.4, 16.7 -> 14.2, 17.0, 15.8 (4)
+    //   1024 x 4096 x 4096    67.7, 77.2, 68.1 -> 57.4, 58.3, 56.5 (6)     512 x 16384 x 4096    131, 157, 135 -> 116, 115, 111 (6)
+    //   512 x 8192 x 12800    207, 241, 213 -> 162, 169, 157 (6)           40 x 32768 x 1024     15.3, 19.3, 17.3 -> 13.6, 16.2, 14.3 (4)
+    //   2048 x 4096 x 2048    69.2, 78.3, 71.6 -> 64.1, 64.4, 63.8 (6)     1024 x 8192 x 2048    70.2, 79.5, 70.9 -> 64.4, 64.7, 61.8 (6)
+    //   64 x 32768 x 2048     26.3, 32.8, 29.4 -> 21.1, 26.4, 23.4 (4)
     // and gemm_kernel's (us, gemm_kernel and the entry that would come next):
-    //   512 x 8192 x 768      17.2, 18.4, 17.4 : 18.2, 18.7, 18.4 (6)      16 x 32768 x 8192     49.3, 75.2, 67.7 : 55.5, 75.8, 69.2 (1)
-    //   1000 x 4096 x 512     13.1, 13.9, 13.0 : 13.3, 15.4, 13.2 (6)      256 x 16384 x 1024    21.3, 24.2, 21.4 : 21.7, 24.1, 22.0 (6)
+    //   1000 x 4096 x 512     13.6, 14.3, 13.6 : 14.5, 14.2, 14.3 (6)
     struct SplitTile
     {
         int mt, rn, ks;
         double step[3]; // microseconds: a step (KS super-blocks) of Q4_K, Q6_K and IQ3_S
     };
     constexpr SplitTile SPLIT[] = {
-        {1, 1, 4, {1.6, 2.8, 2.4}}, {1, 2, 2, {1.35, 2.45, 1.9}}, {2, 1, 4, {2.65, 3.5, 3.2}}, {2, 2, 2, {2.35, 3.05, 2.6}},
-        {2, 4, 1, {2.05, 2.9, 2.4}}, {4, 2, 2, {3.83, 4.1, 4.0}}, {4, 4, 1, {3.45, 3.85, 3.6}}};
+        {1, 1, 4, {1.7, 1.85, 1.65}}, {1, 2, 2, {1.45, 1.8, 1.65}}, {2, 1, 4, {2.25, 2.9, 2.7}}, {2, 2, 2, {1.85, 2.2, 1.9}},
+        {2, 4, 1, {1.65, 2.15, 2.0}}, {3, 2, 2, {2.5, 2.6, 2.5}}, {4, 4, 1, {3.2, 3.3, 2.9}}};
     constexpr double SPLIT_START = 3.5, WHOLE_START = 2.0; // a workgroup's start and end
+    // Beside them, for launches that it alone fits in one round or fills evenly: its activations leave the weights no room in LDS.
+    // (us, the best of the others and this one: 256 x 8192 x 8192 Q6_K and IQ3_S 76, 72 -> 69.8, 64.8)
+    constexpr int GEMM_WIDE = 7;
+    constexpr SplitTile WIDE = {4, 2, 2, {3.75, 4.15, 3.85}};
+    inline double split_expected(const SplitTile &t, int format, int M, int N, int K, int cus)
+    {
+        const auto over = [](long a, long b) { return (a + b - 1) / b; };
+        // (a last round of few workgroups is faster: they have the memory and the clock to themselves)
+        const long groups = over(N, 32 * t.rn) * over(M, 32 * t.mt), left = groups % cus;
+        const double rounds = groups <= cus ? 1.0 : (double)(groups / cus) + (left ? 0.6 + 0.4 * (double)left / cus : 0.0);
+        return rounds * ((double)over(K / 256, t.ks) * t.step[format] + SPLIT_START);
+    }
     // gemm_kernel: microseconds a super-block of a tile of 32, 64 or 128 tokens takes in a round of two workgroups a compute unit
     // that others follow, in the last round, and in a last round of one
     struct WholeTile
@@ -791,12 +984,14 @@ namespace llamql
         int tokens;
         double full[3], last[3], alone[3];
     };
-    constexpr WholeTile WHOLE[] = {{32, {1.4, 2.2, 1.9}, {1.6, 2.5, 2.2}, {0.9, 1.5, 1.4}},
+    constexpr WholeTile WHOLE[] = {{32, {1.4, 2.2, 1.9}, {1.6, 2.5, 2.2}, {1.2, 1.5, 1.4}},
                                    {64, {2.4, 3.1, 2.65}, {2.7, 3.6, 3.05}, {1.65, 2.2, 1.9}},
                                    {GEMM_BM, {3.55, 3.95, 3.55}, {4.2, 4.8, 4.35}, {2.6, 3.0, 2.8}}};
 
-    inline int gemm_split_choice(int format, int M, int N, int K, int cus)
+    inline int gemm_split_choice(int format, int M, int N, int K, int cus, double *expected = nullptr)
     {
+        if (expected)
+            *expected = 1e30;
         if (K > 1 << 24) // 32-bit offsets from a tile's first token
             return -1;
         const auto over = [](long a, long b) { return (a + b - 1) / b; };
@@ -815,14 +1010,72 @@ namespace llamql
             const SplitTile &t = SPLIT[i];
             if (over(M, 32 * t.mt) > 65535) // (the grid's second extent)
                 continue;
-            // (a last round of few workgroups is faster: they have the memory and the clock to themselves)
-            const long groups = over(N, 32 * t.rn) * over(M, 32 * t.mt), left = groups % cus;
-            const double rounds = groups <= cus ? 1.0 : (double)(groups / cus) + (left ? 0.6 + 0.4 * (double)left / cus : 0.0);
-            const double us = rounds * ((double)over(SB, t.ks) * t.step[format] + SPLIT_START);
+            const double us = split_expected(t, format, M, N, K, cus);
             if (us < best)
                 best = us, choice = i;
         }
+        if (expected)
+            *expected = choice < 0 ? undivided : best;
         return choice;
+    }
+
+    // A launch whose last round of tiles is sparse does better as two: the rows whose tiles fill whole rounds by themselves, and
+    // the rest, as tiles that fit it.  Rows of the first launch (a multiple of 64; 0: one launch is as good), `choice` that of the
+    // first.  The second waits for the first to end and starts anew: GEMM_SECOND microseconds, and only where a twentieth is gained.
+    // Measured, one launch and two: 512 x 25600 x 5120 Q4_K 260 -> 227 us, Q6_K 263 -> 229, 2048 x 6400 x 5120 Q4_K 262 -> 222, 82 x 19449 x 19968
+    // Q4_K 210 -> 164, 384 x 25600 x 5120 IQ3_S 193 -> 169.
+    constexpr double GEMM_SECOND = 3.0;
+    inline int gemm_rows_first(int format, int M, int N, int K, int cus, int &choice)
+    {
+        double whole;
+        choice = gemm_split_choice(format, M, N, K, cus, &whole);
+        const auto over = [](long a, long b) { return (a + b - 1) / b; };
+        const int SB = K / 256;
+        int rows = 0;
+        if (const double us = split_expected(WIDE, format, M, N, K, cus); us < 0.97 * whole && over(M, 128) <= 65535 && K <= 1 << 24)
+            choice = GEMM_WIDE, whole = us;
+        double best = 0.95 * whole;
+        for (int i = 0; i < (int)(sizeof(SPLIT) / sizeof(SPLIT[0])); ++i)
+        {
+            const SplitTile &t = SPLIT[i];
+            const long across = over(M, 32 * t.mt), rounds = over(N, 32 * t.rn) * across / cus;
+            const int first = (int)(rounds * cus / across * 32 * t.rn) & ~63;
+            if (first < 64 || first >= N || across > 65535 || K > 1 << 24)
+                continue;
+            double rest;
+            gemm_split_choice(format, M, N - first, K, cus, &rest);
+            const double us = (double)rounds * ((double)over(SB, t.ks) * t.step[format] + SPLIT_START) + GEMM_SECOND + rest;
+            if (us < best)
+                best = us, choice = i, rows = first;
+        }
+        return rows;
+    }
+
+
+    // weight rows from 64 g.tile0 up to rows_end, by the kernel of gemm_split_choice's answer
+    template <class F, bool DUMP>
+    bool gemm_launch_rows(const char *fn, const GemmArgs &g, int choice, int rows_end, int M, hipStream_t st)
+    {
+        const int rows = rows_end - g.tile0 * GEMM_BN, tiles = (rows + GEMM_BN - 1) / GEMM_BN;
+        if (choice == GEMM_WIDE)
+            return gemm_split_launch<F, DUMP, 4, 2, 2>(fn, g, rows, M, st);
+        switch (choice)
+        {
+        case 0: return gemm_split_launch<F, DUMP, 1, 1, 4>(fn, g, rows, M, st);
+        case 1: return gemm_split_launch<F, DUMP, 1, 2, 2>(fn, g, rows, M, st);
+        case 2: return gemm_split_launch<F, DUMP, 2, 1, 4>(fn, g, rows, M, st);
+        case 3: return gemm_split_launch<F, DUMP, 2, 2, 2>(fn, g, rows, M, st);
+        case 4: return gemm_split_launch<F, DUMP, 2, 4, 1>(fn, g, rows, M, st);
+        case 5: return gemm_split_launch<F, DUMP, 3, 2, 2>(fn, g, rows, M, st);
+        case 6: return gemm_split_launch<F, DUMP, 4, 4, 1>(fn, g, rows, M, st);
+        default: break;
+        }
+        // few tokens: one smaller tile of tokens (a 128-token tile would rescale 128 rows for them)
+        if (M <= 32)
+            return gemm_launch_bm<F, DUMP, 32>(fn, g, tiles, M, st);
+        if (M <= 64)
+            return gemm_launch_bm<F, DUMP, 64>(fn, g, tiles, M, st);
+        return gemm_launch_bm<F, DUMP, GEMM_BM>(fn, g, tiles, M, st);
     }
 
     // d_sums: the block-sum variant over weight rows [row0, row0+nrows); only the workgroups
@@ -850,26 +1103,20 @@ namespace llamql
             if (!F::Quad::addressable(N, K / 256))
                 return fail(fn, "matrix too large for the kernel's 32-bit offsets (N=%d K=%d)", N, K);
         }
-        const int tile_end = DUMP ? (row0 + nrows + GEMM_BN - 1) / GEMM_BN : (N + GEMM_BN - 1) / GEMM_BN;
-        const int rows_end = DUMP ? row0 + nrows : N, rows = rows_end - g.tile0 * GEMM_BN;
         constexpr int format = F::HAS_MIN ? 0 : F::TABLE_BYTES > 0 ? 2 : 1; // Q4_K, Q6_K, IQ3_S
-        switch (gemm_split_choice(format, M, N, K, cu_count(device_id)))
+        const int cus = cu_count(device_id);
+        if (DUMP)
+            return gemm_launch_rows<F, DUMP>(fn, g, gemm_split_choice(format, M, N, K, cus), row0 + nrows, M, st);
+        int choice;
+        const int first = gemm_rows_first(format, M, N, K, cus, choice);
+        if (first > 0)
         {
-        case 0: return gemm_split_launch<F, DUMP, 1, 1, 4>(fn, g, rows, M, st);
-        case 1: return gemm_split_launch<F, DUMP, 1, 2, 2>(fn, g, rows, M, st);
-        case 2: return gemm_split_launch<F, DUMP, 2, 1, 4>(fn, g, rows, M, st);
-        case 3: return gemm_split_launch<F, DUMP, 2, 2, 2>(fn, g, rows, M, st);
-        case 4: return gemm_split_launch<F, DUMP, 2, 4, 1>(fn, g, rows, M, st);
-        case 5: return gemm_split_launch<F, DUMP, 4, 2, 2>(fn, g, rows, M, st);
-        case 6: return gemm_split_launch<F, DUMP, 4, 4, 1>(fn, g, rows, M, st);
-        default: break;
+            if (!gemm_launch_rows<F, DUMP>(fn, g, choice, first, M, st))
+                return false;
+            g.tile0 = first / GEMM_BN;
+            choice = gemm_split_choice(format, M, N - first, K, cus);
         }
-        // few tokens: one smaller tile of tokens (a 128-token tile would rescale 128 rows for them)
-        if (M <= 32)
-            return gemm_launch_bm<F, DUMP, 32>(fn, g, tile_end - g.tile0, M, st);
-        if (M <= 64)
-            return gemm_launch_bm<F, DUMP, 64>(fn, g, tile_end - g.tile0, M, st);
-        return gemm_launch_bm<F, DUMP, GEMM_BM>(fn, g, tile_end - g.tile0, M, st);
+        return gemm_launch_rows<F, DUMP>(fn, g, choice, N, M, st);
     }
 } // namespace llamql
 

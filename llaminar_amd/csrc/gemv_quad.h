@@ -421,6 +421,50 @@ namespace llamql
     // group l holds blocks 2l (low nibbles) and 2l+1 (high nibbles), element e in byte e
     // (Q4_KTensor.cpp:768-792).  Effective scale f16(d*sc), min f16(-dmin*m) with the
     // packer's fp16 rounding (Q4_KTensor.cpp:794-799, FP16Utils.h:75-118).
+    // 32 rows of one half of a super-block, raw, by way of LDS: what the quad lanes 2 half and 2 half + 1 of every row decode.
+    // A load of 16 bytes a lane reads a row's piece of a plane with neighbouring lanes (four cover 64 bytes), where a lane that
+    // loads for itself meets a cache line of its own: 16 or 32 instead of 64 cycles of the address unit.  A piece lies in LDS where
+    // eight lanes that read eight neighbouring rows meet no bank twice.
+    // PIECES: 16-byte pieces of a row; AT: the place of the first of them
+    template <int PIECES>
+    struct HalfRows
+    {
+        static constexpr int ROWS = 64 / PIECES < 32 ? 64 / PIECES : 32; // of a load
+        static constexpr int LOADS = 32 / ROWS, BYTES = 32 * PIECES * 16;
+        static constexpr uint64_t LANES = ROWS * PIECES == 64 ? ~0ull : (1ull << (ROWS * PIECES)) - 1;
+        __device__ __forceinline__ static int place(int row, int piece)
+        {
+            return PIECES == 4 ? piece ^ ((row >> 1) & 3) : PIECES == 2 ? piece ^ ((row >> 2) & 1) : piece;
+        }
+        // row_of(r): where row r's pieces start, in bytes from the base that the load is given
+        template <class R>
+        __device__ __forceinline__ static void offsets(uint32_t (&from)[LOADS], int lane, R row_of)
+        {
+#pragma unroll
+            for (int i = 0; i < LOADS; ++i)
+            {
+                const int row = (i * ROWS + lane / PIECES) & 31;
+                from[i] = row_of(row) + 16u * (uint32_t)place(row, lane % PIECES);
+            }
+        }
+        // to: LDS address (uniform)
+        __device__ __forceinline__ static void load(uint32_t to, const uint32_t (&from)[LOADS], const uint8_t *base)
+        {
+#pragma unroll
+            for (int i = 0; i < LOADS; ++i)
+                if (LANES == ~0ull)
+                    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to + (uint32_t)(i * 1024)), "v"(from[i]), "s"(base) : "memory");
+                else
+                    asm volatile("s_mov_b32 m0, %0\n\ts_mov_b64 exec, %3\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b64 exec, -1"
+                                 ::"s"(to + (uint32_t)(i * 1024)), "v"(from[i]), "s"(base), "s"(LANES) : "memory");
+        }
+        template <class V>
+        __device__ __forceinline__ static V read(const uint8_t *at, int row, int piece, int byte = 0)
+        {
+            return *reinterpret_cast<const V *>(at + (row * PIECES + place(row, piece)) * 16 + byte);
+        }
+    };
+
     struct Q4KQuad
     {
         static constexpr int SB_BYTES = 144;
@@ -537,6 +581,34 @@ namespace llamql
             asm volatile("global_load_dwordx4 %0, %1, %2" : "=&v"(r.qa) : "v"(ogrp), "s"(c.base));
             asm volatile("global_load_dwordx4 %0, %1, %2 offset:16" : "=&v"(r.qb) : "v"(ogrp), "s"(c.base));
         }
+        // (HalfRows: a row's header, and the 64 bytes of two groups)
+        struct Half
+        {
+            typedef HalfRows<1> Head;
+            typedef HalfRows<4> Group;
+            static constexpr int BYTES = Head::BYTES + Group::BYTES;
+            uint32_t head[Head::LOADS], group[Group::LOADS];
+            const uint8_t *base;
+            __device__ __forceinline__ void init(const GemvArgs &a, long n0, int half, int lane)
+            {
+                base = uniform_base(static_cast<const uint8_t *>(a.w));
+                const auto row = [&](int r) { return (uint32_t)(n0 + r < a.N ? n0 + r : a.N - 1) * (uint32_t)(a.SB * SB_BYTES); };
+                Head::offsets(head, lane, row);
+                Group::offsets(group, lane, [&](int r) { return row(r) + 16u + 64u * (uint32_t)half; });
+            }
+            __device__ __forceinline__ void load(uint32_t to, int sb) const
+            {
+                Head::load(to, head, base + (size_t)sb * SB_BYTES);
+                Group::load(to + Head::BYTES, group, base + (size_t)sb * SB_BYTES);
+            }
+            // what lane (row, l & 1) of them decodes
+            __device__ __forceinline__ static void read(Raw &r, const uint8_t *at, int row, int odd)
+            {
+                r.head = Head::read<v4i>(at, row, 0);
+                r.qa = Group::read<v4i>(at + Head::BYTES, row, 2 * odd);
+                r.qb = Group::read<v4i>(at + Head::BYTES, row, 2 * odd + 1);
+            }
+        };
         // Marks r's registers as in use up to this point (emits nothing).
         __device__ __forceinline__ static void keep(Raw &r)
         {
@@ -744,6 +816,41 @@ namespace llamql
             asm volatile("global_load_dwordx4 %0, %1, %2 offset:16" : "=&v"(r.qhb) : "v"(oqh), "s"(c.qh));
             asm volatile("global_load_dwordx2 %0, %1, %2" : "=&v"(r.fc) : "v"(ofc), "s"(c.fc));
         }
+        // (HalfRows: 64 bytes of low bits, 32 of upper bits, four factor records)
+        struct Half
+        {
+            typedef HalfRows<4> Low;
+            typedef HalfRows<2> Upper;
+            typedef HalfRows<1> Factors;
+            static constexpr int BYTES = Low::BYTES + Upper::BYTES + Factors::BYTES;
+            uint32_t low[Low::LOADS], upper[Upper::LOADS], factors[Factors::LOADS];
+            const uint8_t *ql, *qh, *fc;
+            __device__ __forceinline__ void init(const GemvArgs &a, long n0, int half, int lane)
+            {
+                const size_t T = (size_t)a.N * a.SB;
+                ql = uniform_base(static_cast<const uint8_t *>(a.w));
+                qh = ql + T * 128;
+                fc = ql + q6k_factors_offset(T);
+                const auto row = [&](int r) { return (uint32_t)(n0 + r < a.N ? n0 + r : a.N - 1) * (uint32_t)a.SB; };
+                Low::offsets(low, lane, [&](int r) { return row(r) * 128u + 64u * (uint32_t)half; });
+                Upper::offsets(upper, lane, [&](int r) { return row(r) * 64u + 32u * (uint32_t)half; });
+                Factors::offsets(factors, lane, [&](int r) { return row(r) * 32u + 16u * (uint32_t)half; });
+            }
+            __device__ __forceinline__ void load(uint32_t to, int sb) const
+            {
+                Low::load(to, low, ql + (size_t)sb * 128);
+                Upper::load(to + Low::BYTES, upper, qh + (size_t)sb * 64);
+                Factors::load(to + Low::BYTES + Upper::BYTES, factors, fc + (size_t)sb * 32);
+            }
+            __device__ __forceinline__ static void read(Raw &r, const uint8_t *at, int row, int odd)
+            {
+                r.qla = Low::read<v4i>(at, row, 2 * odd);
+                r.qlb = Low::read<v4i>(at, row, 2 * odd + 1);
+                r.qha = Upper::read<v4i>(at + Low::BYTES, row, 0);
+                r.qhb = Upper::read<v4i>(at + Low::BYTES, row, 1);
+                r.fc = Factors::read<v2i_>(at + Low::BYTES + Upper::BYTES, row, 0, 8 * odd);
+            }
+        };
         __device__ __forceinline__ static void keep(Raw &r)
         {
             asm volatile("" : "+v"(r.qla), "+v"(r.qlb), "+v"(r.qha), "+v"(r.qhb), "+v"(r.fc));

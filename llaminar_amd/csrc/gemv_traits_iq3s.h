@@ -393,6 +393,39 @@ namespace llamql
             asm volatile("global_load_dwordx4 %0, %1, %2" : "=&v"(r.meta) : "v"(om), "s"(c.meta));
             asm volatile("global_load_dwordx2 %0, %1, %2" : "=&v"(r.sg) : "v"(osg), "s"(c.sg));
         }
+        // (HalfRows: 32 bytes of indices, 16 of signs, the super-block's record)
+        struct Half
+        {
+            typedef HalfRows<2> Index;
+            typedef HalfRows<1> Sign;
+            typedef HalfRows<1> Meta;
+            static constexpr int BYTES = Index::BYTES + Sign::BYTES + Meta::BYTES;
+            uint32_t index[Index::LOADS], sign[Sign::LOADS], record[Meta::LOADS];
+            const uint8_t *qs, *sg, *meta;
+            __device__ __forceinline__ void init(const GemvArgs &a, long n0, int half, int lane)
+            {
+                const size_t T = (size_t)a.N * a.SB;
+                qs = uniform_base(static_cast<const uint8_t *>(a.w));
+                sg = qs + T * 64;
+                meta = qs + T * 96;
+                const auto row = [&](int r) { return (uint32_t)(n0 + r < a.N ? n0 + r : a.N - 1) * (uint32_t)a.SB; };
+                Index::offsets(index, lane, [&](int r) { return row(r) * 64u + 32u * (uint32_t)half; });
+                Sign::offsets(sign, lane, [&](int r) { return row(r) * 32u + 16u * (uint32_t)half; });
+                Meta::offsets(record, lane, [&](int r) { return row(r) * 16u; });
+            }
+            __device__ __forceinline__ void load(uint32_t to, int sb) const
+            {
+                Index::load(to, index, qs + (size_t)sb * 64);
+                Sign::load(to + Index::BYTES, sign, sg + (size_t)sb * 32);
+                Meta::load(to + Index::BYTES + Sign::BYTES, record, meta + (size_t)sb * 16);
+            }
+            __device__ __forceinline__ static void read(Raw &r, const uint8_t *at, int row, int odd)
+            {
+                r.qs = Index::read<v4i>(at, row, odd);
+                r.sg = Sign::read<v2i_>(at + Index::BYTES, row, 0, 8 * odd);
+                r.meta = Meta::read<v4i>(at + Index::BYTES + Sign::BYTES, row, 0);
+            }
+        };
         __device__ __forceinline__ static void keep(Raw &r)
         {
             asm volatile("" : "+v"(r.qs), "+v"(r.meta), "+v"(r.sg));

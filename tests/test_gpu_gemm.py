@@ -121,8 +121,9 @@ def test_a_walk_dealt_to_wavefronts(capi, dev, oracle, fmt, M, N, K):
     (63, 8161, 2048), (33, 8161, 4864),     # 64 x 32
     (129, 4999, 1536), (129, 4999, 2816),   # 64 x 64: the last token tile of one token, a super-block left over
     (64, 20001, 1024), (33, 24997, 1280),   # 64 x 128
-    (97, 9799, 4352), (193, 8000, 2560),    # 128 x 64
+    (97, 9799, 4352), (193, 8000, 2560),    # 96 x 64
     (128, 24997, 1280), (257, 8129, 2304),  # 128 x 128
+    (255, 24997, 1280),                     # and short of a tile both ways
     (512, 8192, 1280),                      # one whole round of them
 ])
 def test_tiles_of_dealt_walks(capi, dev, oracle, fmt, M, N, K):
@@ -149,6 +150,65 @@ def test_tiles_of_dealt_walks(capi, dev, oracle, fmt, M, N, K):
         assert rel_err(part, C) <= TOL[fmt] * 1e-2
         assert np.abs(part - C).max() <= 1e-4 * np.abs(C).max()
         assert np.array_equal(s.cpu().numpy(), sums)
+
+
+@pytest.mark.parametrize("fmt", list(FMTS.values()), ids=list(FMTS))
+@pytest.mark.parametrize("M,N,K,first", [(193, 17159, 1024, 16384), (65, 18660, 3840, 16384), (193, 19075, 1536, 16384),
+                                         (250, 8191, 4096, 0)])
+def test_rows_in_two_launches(capi, dev, oracle, fmt, M, N, K, first):
+    """Rows whose tiles fill whole rounds and the rest as a launch of its own (and, without one, the tile of 128 x 64): every element
+    written, those on both sides of the seam and the last ones near the oracle's, the same bits again."""
+    import torch
+
+    W = synth.weights_numpy(fmt, N, K, 31 + M)
+    q8 = oracle.quantize(synth.activations_numpy(M, K, 37 + K))
+    wd, qd = upload_weights(capi, dev, fmt, W), upload_q8(dev, q8)
+    y, again = (torch.full((M, N + 3), float("nan"), device=dev) for _ in range(2))
+    for out in (y, again):
+        capi.gemm(fmt, wd, qd, M, N, K, out=out[:, :N])
+    sync()
+    assert torch.equal(y[:, :N], again[:, :N]) and bool(torch.isnan(y[:, N:]).all()) and not bool(torch.isnan(y[:, :N]).any())
+    got = y.cpu().numpy()
+    for r0 in (max(0, first - 48), N - 96):
+        C = oracle.gemm(fmt, W, K, q8, n0=r0, n1=r0 + 96)
+        assert rel_err(got[:, r0:r0 + 96], C) <= TOL[fmt] * 1e-2
+        assert np.abs(got[:, r0:r0 + 96] - C).max() <= 1e-4 * np.abs(C).max()
+
+
+@pytest.mark.parametrize("fmt", list(FMTS.values()), ids=list(FMTS))
+@pytest.mark.parametrize("M,N,K", [(40, 1000, 2304), (129, 4999, 1536), (97, 9799, 1536), (255, 24997, 512)])
+def test_dealt_walks_at_the_ends_of_the_scales(capi, dev, oracle, fmt, M, N, K):
+    """Scales that are not finite, and scales that are fp16's smallest: an infinite or undefined scale of one Q8_1 block makes
+    exactly that token's outputs what the sums as such are (infinite, or not a number), weights' scales below fp16's normal
+    range and tokens' scales of one unit are multiplied as they are.  The tolerance is that of every walk."""
+    import torch
+
+    W = synth.weights_numpy(fmt, N, K, 23 + M)
+    at = {FMT_Q4_K: 0, FMT_Q6_K: 208}.get(fmt, 0)
+    blocks = W.reshape(N, K // 256, -1)
+    blocks[5::7, :, at:at + 2] = np.frombuffer(np.float16(3e-6).tobytes(), np.uint8)
+    q8 = oracle.quantize(synth.activations_numpy(M, K, 29 + K))
+    heads = q8.reshape(M, K // 32, 36)
+    special = {0: np.float16(np.inf), 7: np.float16(np.nan), M - 1: np.float16(-np.inf), 3: np.float16(6e-8)}
+    for m, d in special.items():
+        heads[m, (5 * m) % (K // 32), :2] = np.frombuffer(d.tobytes(), np.uint8)
+    wd = upload_weights(capi, dev, fmt, W)
+    y = capi.gemm(fmt, wd, upload_q8(dev, q8), M, N, K)
+    sync()
+    got, n = y.cpu().numpy(), min(N, 96)
+    for r0 in (0, N - n):
+        C, sums = oracle.gemm(fmt, W, K, q8, n0=r0, n1=r0 + n, want_sums=True)
+        if fmt != FMT_Q4_K:
+            # (the oracle adds minima of zero times an infinite scale, which these formats do not have)
+            for m in (0, M - 1):
+                with np.errstate(invalid="ignore"):
+                    C[m] = sums[m, :, (5 * m) % (K // 32)] * np.float32(special[m])
+        part = got[:, r0:r0 + n]
+        assert np.array_equal(np.isnan(part), np.isnan(C)) and np.array_equal(np.isposinf(part), np.isposinf(C))
+        assert np.array_equal(np.isneginf(part), np.isneginf(C))
+        whole = np.isfinite(C).all(1)
+        assert rel_err(part[whole], C[whole]) <= TOL[fmt] * 1e-2
+        assert whole.sum() == M - 3
 
 
 def test_block_sums_at_their_limits(capi, dev, oracle):
