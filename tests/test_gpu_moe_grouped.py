@@ -86,3 +86,55 @@ def test_pairs_sorted_by_expert(capi, dev, T, S, E):
     assert np.array_equal(w[4:4 + len(experts)], experts)
     assert np.array_equal(w[4 + P:4 + P + len(experts) + 1], np.append(begins, len(valid)))
     assert np.array_equal(w[5 + 2 * P:5 + 2 * P + len(valid)], order)
+
+
+@pytest.mark.parametrize("T,S,E", [(5, 3, 4), (64, 9, 257), (455, 9, 257), (4096, 1, 2048), (2, 2000, 3), (1023, 4, 1)])
+def test_chunks_of_an_experts_pairs(capi, dev, T, S, E):
+    """The units of work: every expert's run of pairs in stretches of two or four, in order."""
+    import torch
+
+    ids = np.random.default_rng(T).integers(-1, E + 1, size=(T, S)).astype(np.int32)
+    P = T * S
+    g = capi.moe_group(torch.from_numpy(ids).to(dev), E)
+    torch.cuda.synchronize()
+    w = g.cpu().numpy().view(np.int32)
+    size = 4 if P >= 512 else 2
+    counts = np.bincount(ids[(ids >= 0) & (ids < E)], minlength=E)
+    want, begin = [], 0
+    for e, n in enumerate(counts):
+        want += [(e, begin + j, min(size, n - j)) for j in range(0, n, size)]
+        begin += n
+    assert (int(w[2]), int(w[3])) == (len(want), size)
+    at = 5 + 3 * P
+    got = np.stack([w[at + k * P:at + k * P + len(want)] for k in range(3)], 1)
+    assert np.array_equal(got, np.array(want, np.int32).reshape(-1, 3))
+
+
+@pytest.mark.parametrize("S,hidden,accumulate", [(1, 256, False), (10, 1280, False), (11, 256, True), (63, 1024, False), (70, 1280, True)])
+def test_weighted_sums_of_a_tokens_slots(capi, dev, S, hidden, accumulate):
+    """One to many slots, some without an expert (what lies in their rows is not a number), a token without any: the live slots one
+    after the other, products and sums rounded to 32 bits, the same bits."""
+    import torch
+
+    T, E, inter, fmt = 7, 5, 256, capi.FORMATS["q4_k"]
+    mats = [tuple(capi.prepare_weights(fmt, synth.weights_torch(fmt, n, k, 3 * e + j, dev), n, k)
+                  for j, (n, k) in enumerate(((inter, hidden), (inter, hidden), (hidden, inter)))) for e in range(E)]
+    table = capi.expert_table(mats, dev)
+    table.view(torch.int64).view(E, 3)[3] = 0   # expert 3 lives elsewhere
+    rng = np.random.default_rng(S)
+    ids = rng.integers(-1, E + 1, size=(T, S)).astype(np.int32)
+    ids[4] = -1
+    idd, w = torch.from_numpy(ids).to(dev), torch.from_numpy(rng.standard_normal((T, S)).astype(np.float32)).to(dev)
+    act = capi.quantize_q8_1(torch.from_numpy(synth.activations_numpy(T * S, inter, 9)).to(dev))
+    pairs, base = torch.full((T * S, hidden), float("nan"), device=dev), torch.randn(T, hidden, device=dev)
+    out = base.clone()
+    capi.moe_down_grouped(fmt, table, E, capi.moe_group(idd, E), idd, w, act, pairs, out, T, S, hidden, inter, accumulate=accumulate)
+    torch.cuda.synchronize()
+    rows, weights, start = pairs.cpu().numpy().reshape(T, S, hidden), w.cpu().numpy(), base.cpu().numpy()
+    for t in range(T):
+        y = start[t] if accumulate else None
+        for s in range(S):
+            if 0 <= ids[t, s] < E and ids[t, s] != 3:
+                v = weights[t, s] * rows[t, s]
+                y = v if y is None else y + v
+        assert np.array_equal(out[t].cpu().numpy(), np.zeros(hidden, np.float32) if y is None else y), t
