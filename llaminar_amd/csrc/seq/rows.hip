@@ -59,7 +59,11 @@ namespace llamql
         }
     }
 
-    template <typename T>
+    // Workgroup = a row.  A few rows are bound by the chain of waits, so a thread asks for its HOLD pieces of the row and of the
+    // norms at once and keeps them, where it used to read the row again and the norm only after the sum (0: longer rows still do).
+    // The norm of 8 rows of 2048: a step of 33 passes with nine norms each 19.03 -> 18.80 ms; 2048 rows of 2048 columns
+    // 6.3 -> 5.7 us, of 5120 21.9 -> 19.0.
+    template <typename T, int HOLD>
     __global__ void __launch_bounds__(ROW_THREADS)
         seq_rmsnorm_kernel(const float *__restrict__ x, int ldx, const int32_t *__restrict__ rows,
                            const float *__restrict__ norm, float eps, int k_real, T *__restrict__ y, int K,
@@ -69,23 +73,53 @@ namespace llamql
         __shared__ float s_sum[ROW_THREADS / 64];
         const int m = blockIdx.x;
         const f32x4 *row = reinterpret_cast<const f32x4 *>(x + (size_t)(rows ? rows[m] : m) * ldx);
+        const f32x4 *scale = reinterpret_cast<const f32x4 *>(norm), *scale2 = reinterpret_cast<const f32x4 *>(norm2);
+        t4 *out = reinterpret_cast<t4 *>(y + (size_t)m * K), *out2 = reinterpret_cast<t4 *>(y2 + (norm2 ? (size_t)m * K : 0));
+        f32x4 v[HOLD + 1], a[HOLD + 1], b[HOLD + 1];
         float sum = 0.0f;
-        for (int i = threadIdx.x; i < K / 4; i += ROW_THREADS)
+        auto add = [&sum](f32x4 u) { sum += u[0] * u[0] + u[1] * u[1] + u[2] * u[2] + u[3] * u[3]; };
+#pragma unroll
+        for (int j = 0; j < HOLD; ++j)
         {
-            const f32x4 v = row[i];
-            sum += v[0] * v[0] + v[1] * v[1] + v[2] * v[2] + v[3] * v[3];
+            const int i = threadIdx.x + j * ROW_THREADS, at = i < K / 4 ? i : 0;
+            v[j] = row[at], a[j] = scale[at];
+            if (norm2)
+                b[j] = scale2[at];
         }
+        if (HOLD)
+        {
+#pragma unroll
+            for (int j = 0; j < HOLD; ++j)
+                if ((int)threadIdx.x + j * ROW_THREADS < K / 4)
+                    add(v[j]);
+        }
+        else
+            for (int i = threadIdx.x; i < K / 4; i += ROW_THREADS)
+                add(row[i]);
         sum = block_sum<ROW_THREADS>(sum, s_sum);
         const float inv = 1.0f / sqrtf(sum / (float)k_real + eps);
-        for (int i = threadIdx.x; i < K / 4; i += ROW_THREADS)
+        if (HOLD)
         {
-            const f32x4 v = row[i] * inv;
-            *reinterpret_cast<t4 *>(y + (size_t)m * K + 4 * i) =
-                __builtin_convertvector(v * reinterpret_cast<const f32x4 *>(norm)[i], t4);
-            if (norm2)
-                *reinterpret_cast<t4 *>(y2 + (size_t)m * K + 4 * i) =
-                    __builtin_convertvector(v * reinterpret_cast<const f32x4 *>(norm2)[i], t4);
+#pragma unroll
+            for (int j = 0; j < HOLD; ++j)
+            {
+                const int i = threadIdx.x + j * ROW_THREADS;
+                if (i >= K / 4)
+                    break;
+                const f32x4 u = v[j] * inv;
+                out[i] = __builtin_convertvector(u * a[j], t4);
+                if (norm2)
+                    out2[i] = __builtin_convertvector(u * b[j], t4);
+            }
         }
+        else
+            for (int i = threadIdx.x; i < K / 4; i += ROW_THREADS)
+            {
+                const f32x4 u = row[i] * inv;
+                out[i] = __builtin_convertvector(u * scale[i], t4);
+                if (norm2)
+                    out2[i] = __builtin_convertvector(u * scale2[i], t4);
+            }
     }
 
     __global__ void __launch_bounds__(64)
@@ -498,6 +532,17 @@ extern "C" bool llam_seq_embed(const llam_seq_embed_args *a, const int32_t *d_id
 
 namespace
 {
+    // two or six pieces of four columns a thread, or any number
+    template <typename T>
+    void rmsnorm_launch(int M, hipStream_t st, const float *x, int ldx, const int32_t *rows, const float *norm, float eps, int k_real, T *y, int K,
+                        const float *norm2, T *y2)
+    {
+        auto *kernel = K <= 2 * 4 * ROW_THREADS   ? seq_rmsnorm_kernel<T, 2>
+                       : K <= 6 * 4 * ROW_THREADS ? seq_rmsnorm_kernel<T, 6>
+                                                  : seq_rmsnorm_kernel<T, 0>;
+        hipLaunchKernelGGL(kernel, dim3(M), dim3(ROW_THREADS), 0, st, x, ldx, rows, norm, eps, k_real, y, K, norm2, y2);
+    }
+
     bool rmsnorm(const char *fn, const float *d_x, int ldx, const int32_t *d_rows, const float *d_norm, const float *d_norm2, float eps,
                  int k_real, void *d_y, void *d_y2, int M, int K, int dtype, int device_id, void *stream)
     {
@@ -512,11 +557,9 @@ namespace
         if (!set_device(fn, device_id))
             return false;
         if (dtype == LLAM_SEQ_F32)
-            hipLaunchKernelGGL(seq_rmsnorm_kernel<float>, dim3(M), dim3(ROW_THREADS), 0, as_stream(stream), d_x, ldx, d_rows,
-                               d_norm, eps, k_real, static_cast<float *>(d_y), K, d_norm2, static_cast<float *>(d_y2));
+            rmsnorm_launch(M, as_stream(stream), d_x, ldx, d_rows, d_norm, eps, k_real, static_cast<float *>(d_y), K, d_norm2, static_cast<float *>(d_y2));
         else
-            hipLaunchKernelGGL(seq_rmsnorm_kernel<bf16>, dim3(M), dim3(ROW_THREADS), 0, as_stream(stream), d_x, ldx, d_rows,
-                               d_norm, eps, k_real, static_cast<bf16 *>(d_y), K, d_norm2, static_cast<bf16 *>(d_y2));
+            rmsnorm_launch(M, as_stream(stream), d_x, ldx, d_rows, d_norm, eps, k_real, static_cast<bf16 *>(d_y), K, d_norm2, static_cast<bf16 *>(d_y2));
         return launched(fn);
     }
 } // namespace
