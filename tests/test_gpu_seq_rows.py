@@ -1,4 +1,5 @@
 """Row operators of sequence models by themselves: at the edges of what a thread, a workgroup or a wavefront holds."""
+import ctypes
 
 import numpy as np
 import pytest
@@ -42,3 +43,33 @@ def test_norm_of_short_and_long_rows(torch, lib, dev, K, dtype):
         # the sum: 32-bit additions, up to 24 in a thread and 9 above it; root, reciprocal, two products; then the type's rounding
         bound = np.abs(want) * (40 * 2.0 ** -24 + (2.0 ** -8 if dtype != sequence.F32 else 0))
         assert (np.abs(got[n] - want) <= bound + 1e-30).all(), n
+
+
+@pytest.mark.parametrize("M,top,experts", [(17, 1, 3), (500, 2, 7), (1820, 9, 40), (1821, 9, 40), (4000, 9, 40)])
+def test_experts_of_many_tokens(torch, lib, dev, M, top, experts):
+    """(token, choice) pairs by their expert: up to 16384 of them are held at once, more are not."""
+    W = 64
+    rng = np.random.default_rng(M)
+    h, z = rng.standard_normal((M, W)).astype(np.float32), rng.standard_normal((M, experts)).astype(np.float32)
+    up, down = (torch.from_numpy(rng.standard_normal((experts, W, W)).astype(np.float32) / 8).bfloat16() for _ in range(2))
+    tiles = [torch.from_numpy(np.stack([sequence.tiled(m) for m in w.view(torch.uint16).numpy()]).view(np.int16)).to(dev) for w in (up, down)]
+    hd, zd, x = torch.from_numpy(h).to(dev), torch.from_numpy(z).to(dev), torch.zeros((M, W), device=dev)
+    a = sequence.ExpertsArgs()
+    a.d_logits, a.ldz, a.d_up, a.d_down, a.up_stride, a.down_stride = zd.data_ptr(), experts, tiles[0].data_ptr(), tiles[1].data_ptr(), W * W, W * W
+    a.experts, a.top, a.ff, a.shared_ff, a.K, a.N, a.d_h, a.d_x, a.ldx = experts, top, W, 0, W, W, hd.data_ptr(), x.data_ptr(), W
+    size = lib.llam_seq_experts_scratch_bytes(M, experts, top, W, 0, W)
+    scratch = torch.zeros(size, dtype=torch.uint8, device=dev)
+    assert lib.llam_seq_experts(ctypes.byref(a), M, scratch.data_ptr(), size, sequence.F32, 0, None), lib.llam_ql_last_error()
+    torch.cuda.synchronize()
+    chosen = np.argsort(-z, axis=1, kind="stable")[:, :top]
+    w = np.exp(np.take_along_axis(z, chosen, 1).astype(np.float64))
+    w /= w.sum(1, keepdims=True)
+    u, d = up.double().numpy(), down.double().numpy()
+    want, size = np.zeros((M, W)), np.zeros((M, W))
+    for e in range(experts):
+        t, c = np.nonzero(chosen == e)
+        y = np.maximum(h[t].astype(np.float64) @ u[e].T, 0) ** 2
+        want[t] += w[t, c][:, None] * (y @ d[e].T)
+        size[t] += w[t, c][:, None] * ((np.abs(h[t]) @ np.abs(u[e]).T) ** 2 @ np.abs(d[e]).T)
+    # two products of 64 terms, the first squared, and a sum of the choices, all in 32 bits
+    assert (np.abs(x.cpu().numpy() - want) <= size * (3 * 64 + top + 16) * 2.0 ** -24).all()
