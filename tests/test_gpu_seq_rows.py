@@ -73,3 +73,34 @@ def test_experts_of_many_tokens(torch, lib, dev, M, top, experts):
         size[t] += w[t, c][:, None] * ((np.abs(h[t]) @ np.abs(u[e]).T) ** 2 @ np.abs(d[e]).T)
     # two products of 64 terms, the first squared, and a sum of the choices, all in 32 bits
     assert (np.abs(x.cpu().numpy() - want) <= size * (3 * 64 + top + 16) * 2.0 ** -24).all()
+
+
+@pytest.mark.parametrize("dtype", [0, 1])
+@pytest.mark.parametrize("rank,tokens,length", [(64, 1, 129), (64, 1, 1024), (64, 1, 1025), (512, 1, 1024), (512, 70, 100), (128, 40, 511),
+                                                (128, 40, 513), (576, 300, 330), (192, 1, 2000)])
+def test_latent_attention_merged_from_stretches(torch, lib, dev, rank, tokens, length, dtype):
+    """Two to sixteen stretches of a sequence: up to eight are merged by a wavefront a row, more by a workgroup."""
+    heads = 16
+    rng = np.random.default_rng(length)
+    kind = torch.float32 if dtype == sequence.F32 else torch.bfloat16
+    q, cache = (torch.from_numpy(rng.standard_normal(s).astype(np.float32)).to(kind) for s in ((tokens * heads, rank), (2, length, rank)))
+    qd, cd, out = q.to(dev), cache.to(dev), torch.zeros((tokens * heads, rank), dtype=kind, device=dev)
+    where = [torch.tensor([v], dtype=torch.int32, device=dev) for v in (0, tokens, 1, length - tokens)]
+    e = sequence.Entries(*(t.data_ptr() for t in where))
+    floats = lib.llam_seq_latent_scratch_floats(tokens, 2, heads, rank, length)
+    scratch = torch.full((floats,), float("nan"), device=dev)
+    scale = rank ** -0.5
+    assert lib.llam_seq_latent_attention(qd.data_ptr(), cd.data_ptr(), ctypes.byref(e), 0, 1, tokens, length, heads, rank, length, scale,
+                                         out.data_ptr(), scratch.data_ptr(), floats, dtype, 0, None), lib.llam_ql_last_error()
+    torch.cuda.synchronize()
+    k = cache[1].double().numpy()
+    s = q.double().numpy().reshape(tokens, heads, rank) @ k.T * scale
+    hidden = np.arange(length)[None, None] > (length - tokens + np.arange(tokens))[:, None, None]
+    s = np.where(hidden, -np.inf, s)
+    p = np.exp(s - s.max(-1, keepdims=True))
+    want = (p / p.sum(-1, keepdims=True) @ k).reshape(tokens * heads, rank)
+    # scores: `rank` products of size 0.64 scale added in 32 bits, the exponential's argument rounded; a weight's relative error is twice that;
+    # bf16: weights in two pieces of 8 bits, the result rounded
+    wrong = 2 * (0.64 * rank * scale * 32 + 8) * 2.0 ** -24 + (2.0 ** -16 if dtype != sequence.F32 else 0)
+    bound = wrong * np.abs(k).max() + (np.abs(want) * 2.0 ** -8 if dtype != sequence.F32 else 0)
+    assert (np.abs(out.float().cpu().numpy() - want) <= bound).all()
