@@ -451,7 +451,7 @@ namespace llamql
     }
 
     // The same of at most LAT_FEW stretches, the same sums in the same order: a wavefront a row.  A long portion has many rows of few
-    // stretches each, and the kernel above a workgroup for every 128 columns of a row that ends after one load a thread: four portions
+    // stretches each, and the kernel above a workgroup for every 128 columns of a row that ends after one load a thread: two portions
     // of 251 tokens, 16 heads, rank 512 37 -> 9 us, a call of one row an entry as before (4.6).
     constexpr int LAT_FEW = 8;
     template <typename T>
@@ -713,7 +713,7 @@ extern "C" bool llam_seq_latent_attention(const void *d_q, const void *d_cache, 
 // Portions share a launch where that is no waste: as many as the scratch holds the partial results of, and none whose
 // stretches or rows would leave two thirds of the others' grid empty (a short portion far into its sequence has many stretches: 64
 // tokens at position 8000 beside fifteen times 64 at 0, a step of Kogilix, width 2048, 2.33 -> 1.60 ms against one cut for all).
-// Eight portions of 251 tokens, 16 heads, rank 512: two a launch, 27 us and 44 of merging; alone 17.5 and 23 each; with one cut
+// Eight portions of 251 tokens, 16 heads, rank 512: two a launch, 27 us and 9 of merging (a wavefront a row); alone 17.5 and 5 each; with one cut
 // for all 53 us and nothing to merge, but bits that depend on the others.
 extern "C" bool llam_seq_latent_portions(const void *d_q, const void *d_cache, const llam_seq_entries *e, int first, int n, const int *ntok,
                                          const int *len, int heads, int rank, int cap, float scale, void *d_o, float *d_scratch,
