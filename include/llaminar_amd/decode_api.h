@@ -131,6 +131,10 @@ size_t llam_dec_argmax_scratch_bytes(int B, int n);
  * If d_pos is not NULL, d_pos[b] += 1 afterwards (the next token's position). */
 bool llam_dec_argmax(const float *d_logits, int ld, int n, int B, int32_t *d_ids, int32_t *d_pos,
                      void *d_scratch, int device_id, void *stream);
+/* The same, and the tokens of replayed steps in order: *d_count += 1, then d_out[(*d_count - 1) * B + b] = d_ids[b] as long as
+ * *d_count is not above max_count.  (With B = 0 nothing is counted.) */
+bool llam_dec_argmax_record(const float *d_logits, int ld, int n, int B, int32_t *d_ids, int32_t *d_pos, int32_t *d_out,
+                            int32_t *d_count, int max_count, void *d_scratch, int device_id, void *stream);
 
 #ifdef __cplusplus
 }

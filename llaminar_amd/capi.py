@@ -132,6 +132,8 @@ SIGNATURES = {
                                          c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p]),
     "llam_dec_argmax_scratch_bytes": (c_size_t, [c_int, c_int]),
     "llam_dec_argmax": (c_bool, [c_void_p, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p]),
+    "llam_dec_argmax_record": (c_bool, [c_void_p, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p,
+                                        c_int, c_void_p]),
 }
 
 _lib = None

@@ -50,7 +50,7 @@ namespace llamql
 
     __global__ void __launch_bounds__(ARGMAX_THREADS)
         argmax_partial_kernel(const float *__restrict__ logits, int ld, int n, float *__restrict__ pv,
-                              int *__restrict__ pi)
+                              int *__restrict__ pi, int32_t *__restrict__ count)
     {
         __shared__ float s_v[ARGMAX_THREADS / WAVE];
         __shared__ int s_i[ARGMAX_THREADS / WAVE];
@@ -73,12 +73,17 @@ namespace llamql
         {
             pv[(size_t)b * gridDim.x + blockIdx.x] = v;
             pi[(size_t)b * gridDim.x + blockIdx.x] = idx;
+            if (count && b == 0 && blockIdx.x == 0)
+                *count += 1;
         }
     }
 
+    // count: also record the rows' tokens as those of step *count - 1 (the launch before has counted it, so that no row reads the
+    // counter while another moves it; a launch of its own for one word a row took 4 us of a step)
     __global__ void __launch_bounds__(ARGMAX_THREADS)
         argmax_final_kernel(const float *__restrict__ pv, const int *__restrict__ pi, int n_part,
-                            int32_t *__restrict__ ids, int32_t *__restrict__ pos)
+                            int32_t *__restrict__ ids, int32_t *__restrict__ pos, int32_t *__restrict__ out,
+                            const int32_t *__restrict__ count, int max_count)
     {
         __shared__ float s_v[ARGMAX_THREADS / WAVE];
         __shared__ int s_i[ARGMAX_THREADS / WAVE];
@@ -101,6 +106,8 @@ namespace llamql
             ids[b] = idx;
             if (pos)
                 pos[b] += 1;
+            if (count && *count <= max_count)
+                out[(size_t)(*count - 1) * gridDim.x + b] = idx;
         }
     }
 
@@ -120,10 +127,9 @@ extern "C" size_t llam_dec_argmax_scratch_bytes(int B, int n)
     return (size_t)B * argmax_blocks(n) * (sizeof(float) + sizeof(int));
 }
 
-extern "C" bool llam_dec_argmax(const float *d_logits, int ld, int n, int B, int32_t *d_ids, int32_t *d_pos,
-                                void *d_scratch, int device_id, void *stream)
+static bool argmax(const char *fn, const float *d_logits, int ld, int n, int B, int32_t *d_ids, int32_t *d_pos, int32_t *d_out,
+                   int32_t *d_count, int max_count, void *d_scratch, int device_id, void *stream)
 {
-    static const char *fn = "llam_dec_argmax";
     if (B < 0 || n < 1 || ld < n)
         return fail(fn, "bad size (B=%d n=%d ld=%d)", B, n, ld);
     if (B == 0)
@@ -140,10 +146,27 @@ extern "C" bool llam_dec_argmax(const float *d_logits, int ld, int n, int B, int
     float *pv = static_cast<float *>(d_scratch);
     int *pi = reinterpret_cast<int *>(pv + (size_t)B * blocks);
     hipLaunchKernelGGL(argmax_partial_kernel, dim3(blocks, B), dim3(ARGMAX_THREADS), 0, as_stream(stream), d_logits,
-                       ld, n, pv, pi);
+                       ld, n, pv, pi, d_count);
     if (!launched(fn))
         return false;
     hipLaunchKernelGGL(argmax_final_kernel, dim3(B), dim3(ARGMAX_THREADS), 0, as_stream(stream), pv, pi, blocks,
-                       d_ids, d_pos);
+                       d_ids, d_pos, d_out, d_count, max_count);
     return launched(fn);
+}
+
+extern "C" bool llam_dec_argmax(const float *d_logits, int ld, int n, int B, int32_t *d_ids, int32_t *d_pos,
+                                void *d_scratch, int device_id, void *stream)
+{
+    return argmax("llam_dec_argmax", d_logits, ld, n, B, d_ids, d_pos, nullptr, nullptr, 0, d_scratch, device_id, stream);
+}
+
+extern "C" bool llam_dec_argmax_record(const float *d_logits, int ld, int n, int B, int32_t *d_ids, int32_t *d_pos, int32_t *d_out,
+                                       int32_t *d_count, int max_count, void *d_scratch, int device_id, void *stream)
+{
+    static const char *fn = "llam_dec_argmax_record";
+    if (!d_out || !d_count || max_count < 0)
+        return fail(fn, "bad arguments");
+    if (!aligned4(d_out) || !aligned4(d_count))
+        return fail(fn, "misaligned pointer");
+    return argmax(fn, d_logits, ld, n, B, d_ids, d_pos, d_out, d_count, max_count, d_scratch, device_id, stream);
 }

@@ -387,8 +387,8 @@ namespace
             s.row_slot = md.entry(2);
             s.row_pos = md.entry(3);
             return layers(s) && logits(nullptr, n) &&
-                   forward(fn, llam_dec_argmax(md.logits, md.vp, c.vocab, n, md.ids(), md.entry(3), md.arg_scratch, c.device_id, st)) &&
-                   forward(fn, llam_seq_record(md.ids(), n, md.ring, md.count, DECODE_RING / n, c.device_id, st));
+                   forward(fn, llam_dec_argmax_record(md.logits, md.vp, c.vocab, n, md.ids(), md.entry(3), md.ring, md.count, DECODE_RING / n,
+                                                      md.arg_scratch, c.device_id, st));
         }
     };
 

@@ -271,3 +271,21 @@ def test_argmax(capi, dev, oracle):
     assert pos.cpu().tolist() == [6, 7, 8, 9]
     small = torch.tensor([[1.0, 3.0, 3.0, 2.0]], device=dev)
     assert capi.argmax(small, 4).cpu().tolist() == [1]
+
+
+@pytest.mark.parametrize("B,n", [(1, 1), (3, 5000), (16, 40000)])
+def test_argmax_recorded_step_by_step(capi, dev, B, n):
+    """Four steps into room for three: tokens and positions as without the record, and nothing beyond the room."""
+    import torch
+
+    x = torch.randn(4, B, n, device=dev)
+    ids, pos, count = (torch.zeros(k, dtype=torch.int32, device=dev) for k in (B, B, 1))
+    out = torch.full((4, B), -7, dtype=torch.int32, device=dev)
+    scratch = torch.zeros(capi.load().llam_dec_argmax_scratch_bytes(B, n), dtype=torch.uint8, device=dev)
+    for step in range(4):
+        assert capi.load().llam_dec_argmax_record(x[step].data_ptr(), n, n, B, ids.data_ptr(), pos.data_ptr(), out.data_ptr(), count.data_ptr(), 3,
+                                                  scratch.data_ptr(), 0, None)
+        torch.cuda.synchronize()
+        assert np.array_equal(ids.cpu().numpy(), x[step].cpu().numpy().argmax(1))
+    assert np.array_equal(out[:3].cpu().numpy(), x[:3].cpu().numpy().argmax(2)) and (out[3] == -7).all()
+    assert (pos == 4).all() and int(count) == 4
