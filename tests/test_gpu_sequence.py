@@ -420,3 +420,21 @@ def test_the_dense_family_behind_the_same_engine(tmp_path, dev):
                 tokens.append(chosen)
         dec.close()
         assert output == want
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_decoding_for_long_replays_several_steps_at_once(whole, dtype):
+    """A shape's first 128 steps are replayed one by one, then four at a time where so many are left: the same tokens whatever the bursts."""
+    t, tokens, _ = whole
+    model = load(WHOLE, t, dtype, cap=600)
+    runs = []
+    for bursts in ((64, 64, 1, 9, 12), (3, 4, 5, 138), (1, 149)):
+        ids = [int(model.forward([(slot, 0, tokens[slot:slot + 20])], [19], best=True)[0]) for slot in (0, 2)]
+        pos, out = np.array([20, 20]), []
+        for steps in bursts:
+            out.append(model.decode([0, 2], pos, ids, steps))
+            pos, ids = pos + steps, out[-1][-1]
+            model.forward([(1, 0, tokens[:9])], [8])     # eager work between replays
+        runs.append(np.concatenate(out))
+    assert np.array_equal(runs[0], runs[1]) and np.array_equal(runs[0], runs[2])
+    model.close()
