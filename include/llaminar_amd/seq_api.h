@@ -194,6 +194,12 @@ size_t llam_seq_attention_scratch_floats(int vdim);
 bool llam_seq_attention(const llam_seq_attention_args *a, const void *d_q, const llam_seq_entries *e, int first, int n,
                         int max_ntok, int max_len, void *d_o, int ldo, float *d_scratch, size_t scratch_floats, int dtype,
                         int device_id, void *stream);
+/* llam_seq_rotary of n rows and llam_seq_attention of entries 0 .. n - 1, one token each, whose rows (row0), slots and positions
+ * are those of d_row_slot and d_row_pos.  What d_q holds afterwards is not defined. */
+bool llam_seq_attention_decode(const llam_seq_attention_args *a, const float *d_proj, int ldp, bool append, const double *d_turns,
+                               int rot_dims, const llam_seq_entries *e, const int32_t *d_row_slot, const int32_t *d_row_pos, int n,
+                               int max_len, void *d_q, void *d_o, int ldo, float *d_scratch, size_t scratch_floats, int dtype,
+                               int device_id, void *stream);
 /* The portions of a step, as in llam_seq_latent_portions. */
 bool llam_seq_attention_portions(const llam_seq_attention_args *a, const void *d_q, const llam_seq_entries *e, int first, int n,
                                  const int *ntok, const int *len, void *d_o, int ldo, float *d_scratch, size_t scratch_floats,

@@ -250,10 +250,15 @@ namespace
             a.heads = w.heads, a.kv_heads = w.kv_heads, a.dim = A(w.dim), a.vdim = A(w.vdim);
             a.ring = md.cache_rows[from], a.chunk = w.chunk, a.scale = w.scale, a.d_k = md.cache[from], a.d_v = md.values[from];
             const int n_in = w.heads * a.dim + (own ? w.kv_heads * (a.dim + a.vdim) : 0), ldm = mix_columns(w);
-            if (!project(w, n_in, s) ||
-                !forward(fn, llam_seq_rotary(&a, md.in, n_in, own, w.turns, w.rot_dims, s.row_slot, s.row_pos, md.q, s.M, c.dtype, c.device_id, st)))
+            if (!project(w, n_in, s))
                 return false;
             const llam_seq_entries e = md.entries();
+            if (!s.portions())
+                return forward(fn, llam_seq_attention_decode(&a, md.in, n_in, own, w.turns, w.rot_dims, &e, s.row_slot, s.row_pos, s.single, s.max_len,
+                                                             md.q, md.mix, ldm, md.lat_scratch, md.lat_floats, c.dtype, c.device_id, st)) &&
+                       add_output(w, s);
+            if (!forward(fn, llam_seq_rotary(&a, md.in, n_in, own, w.turns, w.rot_dims, s.row_slot, s.row_pos, md.q, s.M, c.dtype, c.device_id, st)))
+                return false;
             if (s.single && !forward(fn, llam_seq_attention(&a, md.q, &e, 0, s.single, 1, s.max_len, md.mix, ldm, md.lat_scratch, md.lat_floats,
                                                             c.dtype, c.device_id, st)))
                 return false;

@@ -108,6 +108,8 @@ SIGNATURES = {
     "llam_seq_attention_scratch_floats": (c_size_t, [c_int]),
     "llam_seq_attention": (c_bool, [POINTER(AttentionArgs), c_void_p, POINTER(Entries), c_int, c_int, c_int, c_int, c_void_p,
                                     c_int, c_void_p, c_size_t, c_int, c_int, c_void_p]),
+    "llam_seq_attention_decode": (c_bool, [POINTER(AttentionArgs), c_void_p, c_int, c_bool, c_void_p, c_int, POINTER(Entries), c_void_p,
+                                           c_void_p, c_int, c_int, c_void_p, c_void_p, c_int, c_void_p, c_size_t, c_int, c_int, c_void_p]),
     "llam_seq_attention_portions": (c_bool, [POINTER(AttentionArgs), c_void_p, POINTER(Entries), c_int, c_int, POINTER(c_int), POINTER(c_int),
                                              c_void_p, c_int, c_void_p, c_size_t, c_int, c_int, c_void_p]),
     "llam_seq_delta_scratch_bytes": (c_size_t, [c_int, c_int, c_int, c_int, c_int]),

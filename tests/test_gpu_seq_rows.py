@@ -104,3 +104,40 @@ def test_latent_attention_merged_from_stretches(torch, lib, dev, rank, tokens, l
     wrong = 2 * (0.64 * rank * scale * 32 + 8) * 2.0 ** -24 + (2.0 ** -16 if dtype != sequence.F32 else 0)
     bound = wrong * np.abs(k).max() + (np.abs(want) * 2.0 ** -8 if dtype != sequence.F32 else 0)
     assert (np.abs(out.float().cpu().numpy() - want) <= bound).all()
+
+
+@pytest.mark.parametrize("dtype", [0, 1])
+@pytest.mark.parametrize("heads,kv,dim,vdim,rot,chunk,append", [(4, 2, 64, 64, 0, 0, True), (16, 1, 128, 128, 128, 0, True), (12, 4, 128, 64, 50, 100, True),
+                                                                (6, 6, 256, 128, 254, 128, True), (34, 2, 64, 128, 64, 0, True),
+                                                                (8, 2, 128, 256, 32, 0, False), (5, 1, 64, 64, 64, 60, False)])
+def test_a_decoded_token_is_turned_by_its_attention(torch, lib, dev, heads, kv, dim, vdim, rot, chunk, append, dtype):
+    """One launch or rotary_kernel before it: outputs and caches the same bits, at the edges of tiles, stretches and the ring."""
+    n, ring = 6, 256
+    positions = [0, 127, 128, 255, 200, 31] if not chunk else [0, 127, 128, 255, 256, 700]
+    kind = torch.float32 if dtype == sequence.F32 else torch.bfloat16
+    columns = heads * dim + kv * (dim + vdim)
+    torch.manual_seed(heads)
+    proj, turns = torch.randn(n, columns + 4, device=dev), torch.rand(max(rot // 2, 1), dtype=torch.float64, device=dev)
+    caches = [torch.randn(n, kv, ring, d, device=dev).to(kind) for d in (dim, vdim)]
+    slot = torch.tensor([3, 0, 5, 1, 2, 4], dtype=torch.int32, device=dev)
+    pos, row, one = (torch.tensor(v, dtype=torch.int32, device=dev) for v in (positions, list(range(n)), [1] * n))
+    e = sequence.Entries(row.data_ptr(), one.data_ptr(), slot.data_ptr(), pos.data_ptr())
+    floats = lib.llam_seq_attention_scratch_floats(vdim)
+    got = []
+    for together in (False, True):
+        k, v = (c.clone() for c in caches)
+        q, o = torch.zeros(n, heads * dim, dtype=kind, device=dev), torch.zeros(n, heads * vdim, dtype=kind, device=dev)
+        scratch = torch.full((floats,), float("nan"), device=dev)
+        a = sequence.AttentionArgs(heads, kv, dim, vdim, ring, chunk, dim ** -0.5, k.data_ptr(), v.data_ptr())
+        end = (max(positions) + 1, o.data_ptr(), heads * vdim, scratch.data_ptr(), floats, dtype, 0, None)
+        if together:
+            assert lib.llam_seq_attention_decode(ctypes.byref(a), proj.data_ptr(), columns + 4, append, turns.data_ptr(), rot, ctypes.byref(e),
+                                                 slot.data_ptr(), pos.data_ptr(), n, end[0], q.data_ptr(), *end[1:]), lib.llam_ql_last_error()
+        else:
+            assert lib.llam_seq_rotary(ctypes.byref(a), proj.data_ptr(), columns + 4, append, turns.data_ptr(), rot, slot.data_ptr(), pos.data_ptr(),
+                                       q.data_ptr(), n, dtype, 0, None)
+            assert lib.llam_seq_attention(ctypes.byref(a), q.data_ptr(), ctypes.byref(e), 0, n, 1, *end), lib.llam_ql_last_error()
+        torch.cuda.synchronize()
+        got.append((o, k, v))
+    assert torch.isfinite(got[0][0].float()).all()
+    assert all(torch.equal(x, y) for x, y in zip(*got))
