@@ -972,10 +972,13 @@ namespace llamql
     inline double split_expected(const SplitTile &t, int format, int M, int N, int K, int cus)
     {
         const auto over = [](long a, long b) { return (a + b - 1) / b; };
-        // (a last round of few workgroups is faster: they have the memory and the clock to themselves)
-        const long groups = over(N, 32 * t.rn) * over(M, 32 * t.mt), left = groups % cus;
-        const double rounds = groups <= cus ? 1.0 : (double)(groups / cus) + (left ? 0.6 + 0.4 * (double)left / cus : 0.0);
-        return rounds * ((double)over(K / 256, t.ks) * t.step[format] + SPLIT_START);
+        // (a last round of few workgroups is faster: they have the memory and the clock to themselves; not one of at most eight steps,
+        // which is over before that shows: us, 1757 x 3121 x 1792 IQ3_S 49.7 by gemm_kernel and 54.3 by
+        // entry 6, 876 x 2630 x 1280 Q4_K 22.0 by entry 6 and 25.2 by 4)
+        const long groups = over(N, 32 * t.rn) * over(M, 32 * t.mt), left = groups % cus, steps = over(K / 256, t.ks);
+        const double last = left == 0 ? 0.0 : steps <= 8 ? 1.0 : 0.6 + 0.4 * (double)left / cus;
+        const double rounds = groups <= cus ? 1.0 : (double)(groups / cus) + last;
+        return rounds * ((double)steps * t.step[format] + SPLIT_START);
     }
     // gemm_kernel: microseconds a super-block of a tile of 32, 64 or 128 tokens takes in a round of two workgroups a compute unit
     // that others follow, in the last round, and in a last round of one
@@ -1021,7 +1024,8 @@ namespace llamql
 
     // A launch whose last round of tiles is sparse does better as two: the rows whose tiles fill whole rounds by themselves, and
     // the rest, as tiles that fit it.  Rows of the first launch (a multiple of 64; 0: one launch is as good), `choice` that of the
-    // first.  The second waits for the first to end and starts anew: GEMM_SECOND microseconds, and only where a twentieth is gained.
+    // first.  The second waits for the first to end and starts anew: GEMM_SECOND microseconds, and only where a twentieth is gained
+    // and the first's walks have more than eight steps (seven: 1757 x 3121 x 1792 Q4_K 52.1 us in one launch, 56.6 in two, with the quantiser).
     // Measured, one launch and two: 512 x 25600 x 5120 Q4_K 260 -> 227 us, Q6_K 263 -> 229, 2048 x 6400 x 5120 Q4_K 262 -> 222, 82 x 19449 x 19968
     // Q4_K 210 -> 164, 384 x 25600 x 5120 IQ3_S 193 -> 169.
     constexpr double GEMM_SECOND = 3.0;
@@ -1040,7 +1044,7 @@ namespace llamql
             const SplitTile &t = SPLIT[i];
             const long across = over(M, 32 * t.mt), rounds = over(N, 32 * t.rn) * across / cus;
             const int first = (int)(rounds * cus / across * 32 * t.rn) & ~63;
-            if (first < 64 || first >= N || across > 65535 || K > 1 << 24)
+            if (first < 64 || first >= N || across > 65535 || K > 1 << 24 || over(SB, t.ks) <= 8)
                 continue;
             double rest;
             gemm_split_choice(format, M, N - first, K, cus, &rest);
