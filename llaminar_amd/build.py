@@ -242,12 +242,17 @@ def check_inflight_registers(asm: str, src_name: str) -> int:
 
 
 class ScalarHazardError(RuntimeError):
-    """A hand-issued load reads a scalar register too soon after a vector instruction has written it."""
+    """A hand-issued load reads a scalar register too soon after it has been written."""
 
 
 _SREG = re.compile(r"\bs(\d+)\b|\bs\[(\d+):(\d+)\]")
 _VALU_TO_SREG = re.compile(r"^v_\w+\s+(s\d+|s\[\d+:\d+\])\s*,")
 SCALAR_WAIT_STATES = 5
+# m0: the address of a load into LDS
+_M0_WRITE = re.compile(r"^[sv]_\w+\s+m0\s*,")
+_LDS_LOAD = re.compile(r"^(global_load_lds_\w+|(buffer|global)_load_\w+\s.*\blds\b)")
+M0_WAIT_STATES = 1
+M0 = -1
 
 
 def _sregs(text: str) -> set[int]:
@@ -263,7 +268,8 @@ def check_scalar_hazards(asm: str, src_name: str) -> int:
 
     The hardware does not wait by itself, and the compiler inserts the wait states for its own instructions only: such
     a load takes a stale value, half of another pointer, for its base.  An instruction counts as one wait state,
-    s_nop N as N + 1.  Every jump is followed both ways; where ways meet, a register counts as written as lately as on any of
+    s_nop N as N + 1.  Likewise a load into LDS whose address was written into m0 less than one wait state before: it may
+    land at the address before.  Every jump is followed both ways; where ways meet, a register counts as written as lately as on any of
     them.  Returns the number of loads and stores looked at.
     """
     findings: dict[str, None] = {}
@@ -274,7 +280,7 @@ def check_scalar_hazards(asm: str, src_name: str) -> int:
         if not own:
             continue
         at = {label: i for i, (label, _) in enumerate(blocks)}
-        # scalar register -> fewest wait states since a vector instruction wrote it, where a block begins (None: not reached)
+        # scalar register -> fewest wait states since a vector instruction (m0: any) wrote it, where a block begins (None: not reached)
         begin: list[dict[int, int] | None] = [None] * len(blocks)
         work: list[int] = []
 
@@ -299,11 +305,15 @@ def check_scalar_hazards(asm: str, src_name: str) -> int:
                     hit = sorted(r for r in _sregs(text) if r in written)
                     if hit:
                         findings[f"{func}: '{text}' reads s{hit[0]} {written[hit[0]]} wait states after a vector instruction wrote it"] = None
+                    if _LDS_LOAD.match(text) and written.get(M0, M0_WAIT_STATES) < M0_WAIT_STATES:
+                        findings[f"{func}: '{text}' reads m0 {written[M0]} wait states after it was written"] = None
                 if written:
                     passed = int(text.split()[1], 0) + 1 if text.startswith("s_nop") else 1
                     written = {r: n + passed for r, n in written.items() if n + passed < SCALAR_WAIT_STATES}
                 if m := _VALU_TO_SREG.match(text):
                     written.update(dict.fromkeys(_sregs(m.group(1)), 0))
+                if _M0_WRITE.match(text):
+                    written[M0] = 0
                 if control := _control(text):
                     enter(at.get(control[1]), written)
                     if control[0] != "branch":

@@ -447,13 +447,13 @@ namespace llamql
                 from[i] = row_of(row) + 16u * (uint32_t)place(row, lane % PIECES);
             }
         }
-        // to: LDS address (uniform)
+        // to: LDS address (uniform).  (m0 is written a wait state before the load that reads it: the compiler inserts none here)
         __device__ __forceinline__ static void load(uint32_t to, const uint32_t (&from)[LOADS], const uint8_t *base)
         {
 #pragma unroll
             for (int i = 0; i < LOADS; ++i)
                 if (LANES == ~0ull)
-                    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to + (uint32_t)(i * 1024)), "v"(from[i]), "s"(base) : "memory");
+                    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to + (uint32_t)(i * 1024)), "v"(from[i]), "s"(base) : "memory");
                 else
                     asm volatile("s_mov_b32 m0, %0\n\ts_mov_b64 exec, %3\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b64 exec, -1"
                                  ::"s"(to + (uint32_t)(i * 1024)), "v"(from[i]), "s"(base), "s"(LANES) : "memory");

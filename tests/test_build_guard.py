@@ -297,3 +297,30 @@ _Z6kernelv:
         b.check_scalar_hazards(loop.format(between="\ts_branch .LBB0_1"), "moe.hip")
     past = "_Z6kernelv:\n\tv_readfirstlane_b32 s7, v3\n\ts_branch .LBB0_2\n.LBB0_1:\n" + SCALAR.split("{between}\n")[1] + ".LBB0_2:\n\ts_endpgm\n"
     assert b.check_scalar_hazards(past, "moe.hip") == 1
+
+
+# ---- m0, just before a load into LDS -----------------------------------------------------------------
+
+TO_LDS = """\
+_Z6kernelv:
+\t;;#ASMSTART
+\ts_mov_b32 m0, s5
+{between}
+\t{load}
+\t;;#ASMEND
+\ts_endpgm
+"""
+LDS_LOADS = ["global_load_lds_dwordx4 v2, s[6:7]", "global_load_lds_dword v[2:3], off", "buffer_load_dword v2, s[8:11], 0 offen lds"]
+
+
+@pytest.mark.parametrize("load", LDS_LOADS)
+def test_a_load_into_lds_right_after_its_address_fails_the_build(load):
+    for between in ("", "\t;;#ASMEND\n.LBB0_1:\n\t;;#ASMSTART"):
+        with pytest.raises(b.ScalarHazardError, match="m0 0 wait states"):
+            b.check_scalar_hazards(TO_LDS.format(between=between, load=load), "gemm.hip")
+    for between in ("\ts_nop 0", "\ts_mov_b64 exec, s[2:3]"):
+        assert b.check_scalar_hazards(TO_LDS.format(between=between, load=load), "gemm.hip") == 1
+
+
+def test_loads_into_registers_need_no_wait_after_m0():
+    assert b.check_scalar_hazards(TO_LDS.format(between="", load="global_load_dwordx4 v[8:11], v2, s[6:7]"), "gemm.hip") == 1
