@@ -440,7 +440,8 @@ namespace llamql
     // Against a subtraction, a multiply-add and scales on the 32-bit matrix unit, weights straight into registers: 199 x 5120 x 25600
     // Q6_K 206 -> 143 us (tiles of 96 x 64; of 128 x 64 that walk is 182), 40 x 8192 x 5120 IQ3_S 21.8 -> 18.2, 512 x 25600 x 5120
     // Q4_K 270 -> 227 (gemm_kernel before; two launches now), 256 x 25600 x 5120 Q4_K 140 -> 137, 130 x 5000 x 5120 Q4_K 26.5 -> 23.5, 63 x 5034 x 18944 Q6_K 71 -> 62.
-    // Errors against 64 bits: 0.8 to 0.95 times those before (199 x 5120 x 25600 Q6_K 2.57e-7 -> 2.27e-7, 40 x 8192 x 5120 9.9e-8 -> 8.0e-8).
+    // Errors against 64 bits: 0.4 to 1.0 times those before (199 x 5120 x 25600 Q6_K 2.57e-7 -> 1.76e-7, 512 x 25600 x 5120 Q4_K 3.20e-7 ->
+    // 1.22e-7, 40 x 8192 x 5120 IQ3_S 9.9e-8 -> 9.8e-8).
     template <int MT, int RN, int KS>
     struct GemmSplit
     {
@@ -629,10 +630,15 @@ namespace llamql
                 // Product j: pair of blocks i_of(j) by tokens 32 t_of(j) ...  The matrix unit works on a product while the vector
                 // unit rescales the one before it, and the LDS brings the operands of the next.
                 constexpr int JOBS = 2 * MT, EACH = (LOADS + JOBS - 1) / JOBS;
-                // (tokens by tokens, where the rows' scales of all four blocks fit the registers)
+                // (tokens by tokens, where the rows' scales of all four blocks fit the registers; else there and back, so that one tile of
+                // tokens has its four blocks in a row)
                 constexpr bool APART = KW < 8 && (MT > 1 || !F::HAS_MIN) && (MT < 4 || RAW_LDS), FOURS = APART && (MT == 1 || (MT == 2 && RAW_LDS));
-                auto t_of = [](int j) { return FOURS ? j >> 1 : j % MT; };
+                auto t_of = [](int j) { return FOURS ? j >> 1 : j < MT ? j : 2 * MT - 1 - j; };
                 auto i_of = [](int j) { return FOURS ? j & 1 : j / MT; };
+                // Sums of a job's two blocks that are added up by themselves (see rescale): with those of the job before, of the job after
+                auto with_before = [](int j) { return APART && (FOURS ? j & 1 : j == MT); };
+                auto with_after = [](int j) { return APART && (FOURS ? !(j & 1) : j == MT - 1); };
+                auto is_apart = [](int j) { return APART || (MT == 4 && j >= 2 * MT - 2); };
                 auto fence = []() __attribute__((always_inline)) {
                     if (MT > 1) // (two products of a step are not enough for it: the compiler's order is 10 % faster)
                         __builtin_amdgcn_sched_barrier(0);
@@ -674,16 +680,19 @@ namespace llamql
                     }
                 };
                 // Two multiply-adds a sum: biased sum times the token's scale less bias times scale is the sum times the scale, rounded
-                // once, and that times the row's scale.  Four blocks of a token, or two of four, are added up by themselves before they
-                // meet the sum of those before them: the roundings at the size of the whole sum are 1 or 3 instead of 4, which more than
-                // makes up for the one more here, at one addition to eight multiply-adds (eight partial sums need it not; nor do one
-                // token tile's with minima, which gain nothing by it, and 128 x 64, which has no registers for it).
+                // once, and that times the row's scale.  Four blocks of a token, or two and two, are added up by themselves, their minima
+                // among them, before they meet the sum of those before: 1 or 2 roundings at the size of the whole sum instead of 4, or 6
+                // with minima.  Two partial sums are then no coarser than four of block after block: 232 x 16587 x 13312 Q6_K
+                // 1.83e-7 from 64 bits (1.88e-7 by four such sums, 2.28e-7 with two blocks of four apart), Q4_K 1.82e-7 (2.58e-7, 3.38e-7),
+                // at an addition to four or eight multiply-adds (tiles of 128 x 128 1 to 2 %, of 96 x 64 up to 2 %).  Eight partial sums need it
+                // not, 128 x 64 has registers for the second pairs of two token tiles, and one token tile's with minima stay as they were (17 x 8370 x
+                // 18944 Q4_K 51.1 us and 2.95e-7, or 53.7 and 1.26e-7).
                 v16f apart;
                 auto rescale = [&](int j, int which, const v16i &d, uint32_t head, const v16f &cs) __attribute__((always_inline)) {
                     typedef float v2f __attribute__((ext_vector_type(2)));
                     typedef float v8f __attribute__((ext_vector_type(8)));
-                    const int t = t_of(j), n = 2 * i_of(j) + which; // the n-th of a token's four blocks
-                    const bool plain = !APART || (!FOURS && n >= 2), last = n == (FOURS ? 3 : 1);
+                    const int t = t_of(j);
+                    const bool start = which == 0 && !with_before(j), last = which == 1 && !with_after(j);
                     v2f da; // {scale, offset}
                     da[0] = h2f((uint16_t)(head & 0xFFFFu));
                     da[1] = -BIAS * da[0];
@@ -702,9 +711,9 @@ namespace llamql
                         for (int i = 0; i < 8; ++i)
                         {
                             const float c = WHOLE ? da[0] * cs[r + i] : cs[r + i];
-                            if (plain)
+                            if (!is_apart(j))
                                 acc[t][r + i] = fmaf(s[i ^ 1], c, acc[t][r + i]);
-                            else if (n == 0)
+                            else if (start)
                                 apart[r + i] = s[i ^ 1] * c;
                             else if (!last)
                                 apart[r + i] = fmaf(s[i ^ 1], c, apart[r + i]);
@@ -738,8 +747,9 @@ namespace llamql
                         const float p2 = __uint_as_float(and_k<0xFFFF0000u>(__float_as_uint(rest))), p3 = rest - p2;
                         const int both = (int)__builtin_amdgcn_perm(__float_as_uint(p2), __float_as_uint(p1), 0x07060302u);
                         // slots p1 p2 p1 p2 0 p3 0 p3 of the block of either half of the lanes, times m1 m1 m2 m2 0 m1 0 m2
+                        v16f &to = is_apart(j) ? apart : acc[t_of(j)];
                         const v4i pieces = {both, both, __float_as_int(p3), __float_as_int(p3)};
-                        acc[t_of(j)] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8b, low[i_of(j)]), __builtin_bit_cast(v8b, pieces), acc[t_of(j)], 0, 0, 0);
+                        to = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8b, low[i_of(j)]), __builtin_bit_cast(v8b, pieces), to, 0, 0, 0);
                     }
                 };
 #pragma unroll
@@ -792,6 +802,8 @@ namespace llamql
                         dx = product(j + 1, 0, a);
                     if (MT > 2 && j + 1 == MT)
                         cs[2] = scales(1, 0);
+                    if (F::HAS_MIN && !DUMP && is_apart(j))
+                        add_minima(j, hx, hy);
                     fence();
                     if (DUMP)
                         dump(j, 1, dy);
@@ -802,7 +814,7 @@ namespace llamql
                         dy = product(j + 1, 1, b);
                     if (MT > 2 && j + 1 == MT)
                         cs[3] = scales(1, 1);
-                    if (F::HAS_MIN && !DUMP)
+                    if (F::HAS_MIN && !DUMP && !is_apart(j))
                         add_minima(j, hx, hy);
                     hx = nx, hy = ny;
                 }

@@ -176,6 +176,34 @@ def test_rows_in_two_launches(capi, dev, oracle, fmt, M, N, K, first):
 
 
 @pytest.mark.parametrize("fmt", list(FMTS.values()), ids=list(FMTS))
+@pytest.mark.parametrize("M,N,K", [(116, 14367, 1536), (992, 4800, 6400), (256, 8192, 8192), (232, 16587, 13312), (252, 4642, 24576)])
+def test_dealt_walks_round_no_coarser_than_four_sums(capi, dev, oracle, fmt, M, N, K):
+    """The distance from 64 bits.  A rounding of a 32-bit number is off by 0.425 x 2^-24 of it in the root mean square (evenly spread
+    over a unit in the last place, significands by their logarithm).  A walk of B blocks in P sums, each block rounded once at the size
+    of the sum by then, is B / 2P roundings at the size of the result; a block's own product and the last additions are few more.
+    So four sums give sqrt(B / 8 + 6) roundings, and a tenth is left for the sample."""
+    W = synth.weights_numpy(fmt, N, K, 41 + M)
+    q8 = oracle.quantize(synth.activations_numpy(M, K, 43 + K))
+    y = capi.gemm(fmt, upload_weights(capi, dev, fmt, W), upload_q8(dev, q8), M, N, K)
+    sync()
+    n0, n, blocks = 64, 48, K // 32
+    _, sums = oracle.gemm(fmt, W, K, q8, n0=n0, n1=n0 + n, want_sums=True)
+    scales, minima = np.empty((n, blocks)), np.empty((n, blocks))
+    for r in range(n):
+        for sb in range(K // 256):
+            _, d, m = oracle.subblocks(fmt, W[n0 + r, sb])
+            scales[r, 8 * sb:8 * sb + 8], minima[r, 8 * sb:8 * sb + 8] = d.view(np.float16), m.view(np.float16)
+    heads = q8.reshape(M, blocks, 36)
+    a = heads[:, :, :2].copy().view(np.float16)[:, :, 0].astype(np.float64)
+    a_sum = heads[:, :, 2:4].copy().view(np.int16)[:, :, 0] * a
+    exact = np.einsum("mnb,nb,mb->mn", sums.astype(np.float64), scales, a, optimize=True)
+    if fmt == FMT_Q4_K:
+        exact += a_sum @ minima.T
+    got = y.cpu().numpy()[:, n0:n0 + n].astype(np.float64)
+    assert np.linalg.norm(got - exact) / np.linalg.norm(exact) <= 1.1 * 0.425 * 2.0 ** -24 * np.sqrt(blocks / 8 + 6)
+
+
+@pytest.mark.parametrize("fmt", list(FMTS.values()), ids=list(FMTS))
 @pytest.mark.parametrize("M,N,K", [(40, 1000, 2304), (129, 4999, 1536), (97, 9799, 1536), (255, 24997, 512)])
 def test_dealt_walks_at_the_ends_of_the_scales(capi, dev, oracle, fmt, M, N, K):
     """Scales that are not finite, and scales that are fp16's smallest: an infinite or undefined scale of one Q8_1 block makes
