@@ -480,7 +480,8 @@ namespace llamql
     }
     __device__ __forceinline__ float biased_to_float(int sum) { return __builtin_bit_cast(float, sum) - BIAS; }
 
-    template <class F, int MT, int RN, int KS, bool DUMP>
+    // BY_LDS: the raw weights come by way of LDS where there is room
+    template <class F, int MT, int RN, int KS, bool DUMP, bool BY_LDS>
     __global__ void __launch_bounds__(RN * 2 * KS * WAVE) gemm_split_kernel(const GemmArgs g)
     {
         typedef typename F::Quad Q;
@@ -505,9 +506,8 @@ namespace llamql
             n = g.w.N - 1; // tail rows: decode a valid row, never stored
         const typename Q::Lane lc = Q::lane_consts(lh + 2 * half);
         const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)smem;
-        // the weights, by way of LDS or, where the activations leave no room, straight into registers (and three loads for one token
-        // tile: 12 x 1483 x 20992 Q4_K 31.1 -> 29.8 us)
-        constexpr bool RAW_LDS = G::raw_lds(Q::Half::BYTES) && !(MT == 1 && F::HAS_MIN);
+        // the weights, by way of LDS or, where the activations leave no room, straight into registers
+        constexpr bool RAW_LDS = BY_LDS && G::raw_lds(Q::Half::BYTES);
         const typename Q::Cursor wc = Q::cursor(g.w, (size_t)n * SB, (size_t)n * SB, lc);
         typename Q::Half rows_half;
         if constexpr (RAW_LDS)
@@ -724,7 +724,7 @@ namespace llamql
                 };
                 // Minima times the tokens' scaled sums.  The matrix unit's 32-bit products hold the vector unit up for all of their 64
                 // cycles; of bf16 it does 16 in 32, so three pieces of a sum that add up to it (24 bits) times the two of a minimum (11).
-                constexpr bool PIECES = !WHOLE && MT > 1; // (of one token tile their making would take longer)
+                constexpr bool PIECES = !WHOLE && (MT > 1 || KW == 8); // (in walks of one token tile and four or fewer sums their making would take longer)
                 v4i low[2];
                 if constexpr (F::HAS_MIN && PIECES)
 #pragma unroll
@@ -757,15 +757,17 @@ namespace llamql
                     if (!DUMP)
                         asm("" : "+v"(acc[t]));
                 v16f cs[4];
+                auto scales_of_pair = [&](int i) {
+                    const v32f both = scales_of_both(i);
+                    cs[2 * i] = __builtin_shufflevector(both, both, 0, 1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15);
+                    cs[2 * i + 1] = __builtin_shufflevector(both, both, 16, 17, 18, 19, 20, 21, 22, 23, 24, 25, 26, 27, 28, 29, 30, 31);
+                };
+                constexpr bool LATER = MT == 1 && KW < 8; // (the second pair's scales beside the first pair's products: 388 x 1157 x 18688 Q4_K 51.8 -> 49.9 us)
                 if constexpr (MT <= 2)
                 {
-#pragma unroll
-                    for (int i = 0; i < 2; ++i)
-                    {
-                        const v32f both = scales_of_both(i);
-                        cs[2 * i] = __builtin_shufflevector(both, both, 0, 1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15);
-                        cs[2 * i + 1] = __builtin_shufflevector(both, both, 16, 17, 18, 19, 20, 21, 22, 23, 24, 25, 26, 27, 28, 29, 30, 31);
-                    }
+                    scales_of_pair(0);
+                    if (!LATER)
+                        scales_of_pair(1);
                 }
                 else
                     cs[0] = scales(0, 0), cs[1] = scales(0, 1);
@@ -800,6 +802,8 @@ namespace llamql
                     fence();
                     if (j + 1 < JOBS)
                         dx = product(j + 1, 0, a);
+                    if (LATER && j == 0)
+                        scales_of_pair(1);
                     if (MT > 2 && j + 1 == MT)
                         cs[2] = scales(1, 0);
                     if (F::HAS_MIN && !DUMP && is_apart(j))
@@ -926,13 +930,13 @@ namespace llamql
         return launched(fn);
     }
 
-    template <class F, bool DUMP, int MT, int RN, int KS>
+    template <class F, bool DUMP, int MT, int RN, int KS, bool BY_LDS = true>
     bool gemm_split_launch(const char *fn, const GemmArgs &g, int rows, int M, hipStream_t st)
     {
         constexpr size_t lds = GemmSplit<MT, RN, KS>::lds(F::Quad::Half::BYTES);
         static_assert(lds + 6 * 1024 <= 160 * 1024, "LDS, with the decoders' tables");
         static LdsGrant grant;
-        const auto kernel = &gemm_split_kernel<F, MT, RN, KS, DUMP>;
+        const auto kernel = &gemm_split_kernel<F, MT, RN, KS, DUMP, BY_LDS>;
         const hipError_t e = allow_lds(grant, reinterpret_cast<const void *>(kernel), lds);
         if (e != hipSuccess)
             return fail(fn, "cannot reserve %zu bytes of LDS: %s", lds, hipGetErrorString(e));
@@ -1078,7 +1082,13 @@ namespace llamql
         switch (choice)
         {
         case 0: return gemm_split_launch<F, DUMP, 1, 1, 4>(fn, g, rows, M, st);
-        case 1: return gemm_split_launch<F, DUMP, 1, 2, 2>(fn, g, rows, M, st);
+        case 1:
+            // Q4_K weights of several token tiles come from the cache but for the first time, and straight into registers is the shorter
+            // way (us, by LDS and straight: 388 x 1157 x 18688 51.7 and 49.9, 138 x 3037 x 11264 32.5 and 32.1; 14 x 12406 x 18432 51.4 and
+            // 59.9, 16 x 16000 x 8192 27.0 and 29.3)
+            if (F::HAS_MIN && M > 32)
+                return gemm_split_launch<F, DUMP, 1, 2, 2, !F::HAS_MIN>(fn, g, rows, M, st);
+            return gemm_split_launch<F, DUMP, 1, 2, 2>(fn, g, rows, M, st);
         case 2: return gemm_split_launch<F, DUMP, 2, 1, 4>(fn, g, rows, M, st);
         case 3: return gemm_split_launch<F, DUMP, 2, 2, 2>(fn, g, rows, M, st);
         case 4: return gemm_split_launch<F, DUMP, 2, 4, 1>(fn, g, rows, M, st);
