@@ -846,56 +846,70 @@ namespace llamql
                     finite = fmaf(acc[t][r], 0.0f, finite);
                     red[(kw * RN * MT * 16 + t * 16 + r) * WAVE] = acc[t][r];
                 }
+            const bool own = __any(!(finite == 0.0f));
             if (lane == 0)
-                odd[wave] = 0;
-            if (!(finite == 0.0f))
-                odd[wave] = 1;
+                odd[wave] = own;
             __syncthreads();
             int any = 0;
             for (int i = 0; i < G::WAVES; ++i)
                 any |= odd[i];
             return __builtin_amdgcn_readfirstlane(any) != 0;
         };
-        if (__builtin_expect(gather(), 0))
+        // a lane holds a token's sums of rows 8 k + 4 lh .. + 3
+        typedef float vf_dword __attribute__((ext_vector_type(AT_ONCE), aligned(4)));
+        // again: after the second walk, whose sums are rounded otherwise.  What was finite stays (nothing else of its token or row was
+        // infinite then), so that no element depends on another one's infinity.
+        auto store = [&](auto again) __attribute__((always_inline)) {
+            int row_base = (int)n0, l = lane;
+            asm volatile("" : "+s"(row_base), "+v"(l)); // (addresses made anew: kept over the second walk they would fill the registers)
+            const float *sums = reinterpret_cast<const float *>(smem) + rn * MT * 16 * WAVE + l;
+#pragma unroll
+            for (int q = 0; q < SHARE; q += AT_ONCE)
+            {
+                const int reg = kw * SHARE + q, r = reg & 15; // uniform
+                const long m = m0 + (reg >> 4) * 32 + (l & 31);
+                vf_dword sum;
+#pragma unroll
+                for (int i = 0; i < AT_ONCE; ++i)
+                {
+                    float part[KW];
+#pragma unroll
+                    for (int k = 0; k < KW; ++k)
+                        part[k] = sums[(k * RN * MT * 16 + reg + i) * WAVE];
+#pragma unroll
+                    for (int k = 1; k < KW; k *= 2)
+#pragma unroll
+                        for (int l = 0; l < KW; l += 2 * k)
+                            part[l] += part[l + k];
+                    sum[i] = part[0];
+                }
+                const long at = row_base + 8 * (r >> 2) + 4 * (l >> 5) + (r & 3), left = g.w.N - at;
+                if (m < g.M && left > 0)
+                {
+                    float *y = g.y + (size_t)m * g.ldy + at;
+                    if (decltype(again)::value)
+#pragma unroll
+                        for (int i = 0; i < AT_ONCE; ++i)
+                            if (i < left && __builtin_isfinite(y[i]))
+                                sum[i] = y[i];
+                    if (left >= AT_ONCE)
+                        *reinterpret_cast<vf_dword *>(y) = sum;
+                    else
+#pragma unroll
+                        for (int i = 0; i < AT_ONCE - 1; ++i)
+                            if (i < left)
+                                y[i] = sum[i];
+                }
+            }
+        };
+        const bool any_odd = gather();
+        store(std::false_type());
+        if (__builtin_expect(any_odd, 0))
         {
             __syncthreads();
             walk(std::true_type());
             gather();
-        }
-        // a lane holds a token's sums of rows 8 k + 4 lh .. + 3
-        typedef float vf_dword __attribute__((ext_vector_type(AT_ONCE), aligned(4)));
-#pragma unroll
-        for (int q = 0; q < SHARE; q += AT_ONCE)
-        {
-            const int reg = kw * SHARE + q, r = reg & 15; // uniform
-            const long m = m0 + (reg >> 4) * 32 + l32;
-            vf_dword sum;
-#pragma unroll
-            for (int i = 0; i < AT_ONCE; ++i)
-            {
-                float part[KW];
-#pragma unroll
-                for (int k = 0; k < KW; ++k)
-                    part[k] = red[(k * RN * MT * 16 + reg + i) * WAVE];
-#pragma unroll
-                for (int k = 1; k < KW; k *= 2)
-#pragma unroll
-                    for (int l = 0; l < KW; l += 2 * k)
-                        part[l] += part[l + k];
-                sum[i] = part[0];
-            }
-            const long at = n0 + 8 * (r >> 2) + 4 * lh + (r & 3), left = g.w.N - at;
-            if (m < g.M && left > 0)
-            {
-                float *y = g.y + (size_t)m * g.ldy + at;
-                if (left >= AT_ONCE)
-                    *reinterpret_cast<vf_dword *>(y) = sum;
-                else
-#pragma unroll
-                    for (int i = 0; i < AT_ONCE - 1; ++i)
-                        if (i < left)
-                            y[i] = sum[i];
-            }
+            store(std::true_type());
         }
     }
 

@@ -239,6 +239,28 @@ def test_dealt_walks_at_the_ends_of_the_scales(capi, dev, oracle, fmt, M, N, K):
         assert whole.sum() == M - 3
 
 
+@pytest.mark.parametrize("fmt", list(FMTS.values()), ids=list(FMTS))
+@pytest.mark.parametrize("M,N,K", [(31, 4095, 2304), (20, 12001, 4864), (40, 1000, 2304), (129, 4999, 1536), (33, 24997, 1280),
+                                   (199, 5120, 1536), (255, 24997, 1280), (256, 8192, 2048)])
+def test_an_infinite_scale_leaves_other_tokens_and_rows_alone(capi, dev, oracle, fmt, M, N, K):
+    """An infinity in one token and one in one row of W: every other element has the bits that it has without them."""
+    import torch
+
+    W = synth.weights_numpy(fmt, N, K, 51 + M)
+    q8 = oracle.quantize(synth.activations_numpy(M, K, 53 + K))
+    plain = capi.gemm(fmt, upload_weights(capi, dev, fmt, W), upload_q8(dev, q8), M, N, K)
+    infinite = np.frombuffer(np.float16(np.inf).tobytes(), np.uint8)
+    token, row, at = M // 2, N // 2, {FMT_Q4_K: 0, FMT_Q6_K: 208}.get(fmt, 0)
+    q8.reshape(M, K // 32, 36)[token, 3, :2] = infinite
+    W.reshape(N, K // 256, -1)[row, 1, at:at + 2] = infinite
+    odd = capi.gemm(fmt, upload_weights(capi, dev, fmt, W), upload_q8(dev, q8), M, N, K)
+    sync()
+    others = torch.ones(M, N, dtype=torch.bool, device=dev)
+    others[token], others[:, row] = False, False
+    assert torch.equal(plain[others], odd[others])
+    assert not bool(torch.isfinite(odd[token]).any()) and not bool(torch.isfinite(odd[:, row]).all())
+
+
 def test_block_sums_at_their_limits(capi, dev, oracle):
     """Q6_K rows and activations whose every product is the largest there is, 127 and -128 both ways: sums of 32 of them."""
     M, N, K, fmt = 33, 4096, 512, FMT_Q6_K
