@@ -56,7 +56,7 @@ namespace llamql
         // sums[(m * nrows + n - row0) * (K/32) + block]
         int32_t *sums;
         int row0, nrows;
-        int tile0; // first 64-row tile of the launch (0 unless DUMP)
+        int tile0; // first 64-row tile of the launch
     };
 
     template <class F, int BM>
@@ -993,12 +993,10 @@ namespace llamql
     };
     constexpr SplitTile SPLIT[] = {
         {1, 1, 4, {1.7, 1.85, 1.65}}, {1, 2, 2, {1.45, 1.8, 1.65}}, {2, 1, 4, {2.25, 2.9, 2.7}}, {2, 2, 2, {1.85, 2.2, 1.9}},
-        {2, 4, 1, {1.65, 2.15, 2.0}}, {3, 2, 2, {2.5, 2.6, 2.5}}, {4, 4, 1, {3.2, 3.3, 2.9}}};
+        {2, 4, 1, {1.65, 2.15, 2.0}}, {3, 2, 2, {2.5, 2.6, 2.5}}, {4, 4, 1, {3.2, 3.3, 2.9}},
+        {4, 2, 2, {3.75, 4.15, 3.85}}}; // (the last one's activations leave the weights no room in LDS)
+    constexpr int SPLITS = (int)(sizeof(SPLIT) / sizeof(SPLIT[0]));
     constexpr double SPLIT_START = 3.5, WHOLE_START = 2.0; // a workgroup's start and end
-    // Beside them, for launches that it alone fits in one round or fills evenly: its activations leave the weights no room in LDS.
-    // (us, the best of the others and this one: 256 x 8192 x 8192 Q6_K and IQ3_S 76, 72 -> 69.8, 64.8)
-    constexpr int GEMM_WIDE = 7;
-    constexpr SplitTile WIDE = {4, 2, 2, {3.75, 4.15, 3.85}};
     inline double split_expected(const SplitTile &t, int format, int M, int N, int K, int cus)
     {
         const auto over = [](long a, long b) { return (a + b - 1) / b; };
@@ -1038,7 +1036,7 @@ namespace llamql
         const double undivided = WHOLE_START + SB * ((double)rounds_before * whole.full[format] + last[format]);
         double best = 0.97 * undivided;
         int choice = -1;
-        for (int i = 0; i < (int)(sizeof(SPLIT) / sizeof(SPLIT[0])); ++i)
+        for (int i = 0; i < SPLITS - 1; ++i)
         {
             const SplitTile &t = SPLIT[i];
             if (over(M, 32 * t.mt) > 65535) // (the grid's second extent)
@@ -1053,46 +1051,49 @@ namespace llamql
     }
 
     // A launch whose last round of tiles is sparse does better as two: the rows whose tiles fill whole rounds by themselves, and
-    // the rest, as tiles that fit it.  Rows of the first launch (a multiple of 64; 0: one launch is as good), `choice` that of the
-    // first.  The second waits for the first to end and starts anew: GEMM_SECOND microseconds, and only where a twentieth is gained
+    // the rest, as tiles that fit it.  The first's rows are a multiple of 64.  The second waits for the first to end and starts anew: GEMM_SECOND microseconds, and only where a twentieth is gained
     // and the first's walks have more than eight steps (seven: 1757 x 3121 x 1792 Q4_K 52.1 us in one launch, 56.6 in two, with the quantiser).
     // Measured, one launch and two: 512 x 25600 x 5120 Q4_K 260 -> 227 us, Q6_K 263 -> 229, 2048 x 6400 x 5120 Q4_K 262 -> 222, 82 x 19449 x 19968
     // Q4_K 210 -> 164, 384 x 25600 x 5120 IQ3_S 193 -> 169.
     constexpr double GEMM_SECOND = 3.0;
-    inline int gemm_rows_first(int format, int M, int N, int K, int cus, int &choice)
+    struct GemmPlan
     {
-        double whole;
-        choice = gemm_split_choice(format, M, N, K, cus, &whole);
+        int choice, first, rest; // weight rows [0, first) by `choice`, the others by `rest`; first = 0: all by `choice`
+    };
+    inline GemmPlan gemm_plan(int format, int M, int N, int K, int cus)
+    {
         const auto over = [](long a, long b) { return (a + b - 1) / b; };
         const int SB = K / 256;
-        int rows = 0;
-        if (const double us = split_expected(WIDE, format, M, N, K, cus); us < 0.97 * whole && over(M, 128) <= 65535 && K <= 1 << 24)
-            choice = GEMM_WIDE, whole = us;
+        double whole;
+        GemmPlan plan = {gemm_split_choice(format, M, N, K, cus, &whole), 0, -1};
+        if (K > 1 << 24)
+            return plan;
+        // (the last entry for launches that it alone fits in one round or fills evenly; us, the best of the others and this one: 256 x
+        // 8192 x 8192 Q6_K and IQ3_S 76, 72 -> 69.8, 64.8)
+        if (const double us = split_expected(SPLIT[SPLITS - 1], format, M, N, K, cus); us < 0.97 * whole && over(M, 128) <= 65535)
+            plan.choice = SPLITS - 1, whole = us;
         double best = 0.95 * whole;
-        for (int i = 0; i < (int)(sizeof(SPLIT) / sizeof(SPLIT[0])); ++i)
+        for (int i = 0; i < SPLITS - 1; ++i)
         {
             const SplitTile &t = SPLIT[i];
             const long across = over(M, 32 * t.mt), rounds = over(N, 32 * t.rn) * across / cus;
             const int first = (int)(rounds * cus / across * 32 * t.rn) & ~63;
-            if (first < 64 || first >= N || across > 65535 || K > 1 << 24 || over(SB, t.ks) <= 8)
+            if (first < 64 || first >= N || across > 65535 || over(SB, t.ks) <= 8)
                 continue;
-            double rest;
-            gemm_split_choice(format, M, N - first, K, cus, &rest);
-            const double us = (double)rounds * ((double)over(SB, t.ks) * t.step[format] + SPLIT_START) + GEMM_SECOND + rest;
+            double after;
+            const int rest = gemm_split_choice(format, M, N - first, K, cus, &after);
+            const double us = (double)rounds * ((double)over(SB, t.ks) * t.step[format] + SPLIT_START) + GEMM_SECOND + after;
             if (us < best)
-                best = us, choice = i, rows = first;
+                best = us, plan = {i, first, rest};
         }
-        return rows;
+        return plan;
     }
 
-
-    // weight rows from 64 g.tile0 up to rows_end, by the kernel of gemm_split_choice's answer
+    // weight rows from 64 g.tile0 up to rows_end, by the kernel of gemm_plan's answer
     template <class F, bool DUMP>
     bool gemm_launch_rows(const char *fn, const GemmArgs &g, int choice, int rows_end, int M, hipStream_t st)
     {
         const int rows = rows_end - g.tile0 * GEMM_BN, tiles = (rows + GEMM_BN - 1) / GEMM_BN;
-        if (choice == GEMM_WIDE)
-            return gemm_split_launch<F, DUMP, 4, 2, 2>(fn, g, rows, M, st);
         switch (choice)
         {
         case 0: return gemm_split_launch<F, DUMP, 1, 1, 4>(fn, g, rows, M, st);
@@ -1108,6 +1109,7 @@ namespace llamql
         case 4: return gemm_split_launch<F, DUMP, 2, 4, 1>(fn, g, rows, M, st);
         case 5: return gemm_split_launch<F, DUMP, 3, 2, 2>(fn, g, rows, M, st);
         case 6: return gemm_split_launch<F, DUMP, 4, 4, 1>(fn, g, rows, M, st);
+        case 7: return gemm_split_launch<F, DUMP, 4, 2, 2>(fn, g, rows, M, st);
         default: break;
         }
         // few tokens: one smaller tile of tokens (a 128-token tile would rescale 128 rows for them)
@@ -1118,8 +1120,8 @@ namespace llamql
         return gemm_launch_bm<F, DUMP, GEMM_BM>(fn, g, tiles, M, st);
     }
 
-    // d_sums: the block-sum variant over weight rows [row0, row0+nrows); only the workgroups
-    // whose 64-row tile meets the window are launched.
+    // d_sums: the block-sum variant of the same launches over weight rows [row0, row0+nrows); only the workgroups
+    // whose rows meet the window are launched.
     template <class F, bool DUMP = false>
     bool gemm_launch(const char *fn, const void *d_w, const void *d_q8, float *d_y, int M, int N, int K, int ldy,
                      int device_id, hipStream_t st, int32_t *d_sums = nullptr, int row0 = 0, int nrows = 0)
@@ -1136,7 +1138,6 @@ namespace llamql
         g.sums = d_sums;
         g.row0 = row0;
         g.nrows = nrows;
-        g.tile0 = DUMP ? row0 / GEMM_BN : 0;
         // (the quad-lane decoders address a matrix through 32-bit offsets)
         if constexpr (F::USE_QUAD)
         {
@@ -1144,19 +1145,17 @@ namespace llamql
                 return fail(fn, "matrix too large for the kernel's 32-bit offsets (N=%d K=%d)", N, K);
         }
         constexpr int format = F::HAS_MIN ? 0 : F::TABLE_BYTES > 0 ? 2 : 1; // Q4_K, Q6_K, IQ3_S
-        const int cus = cu_count(device_id);
-        if (DUMP)
-            return gemm_launch_rows<F, DUMP>(fn, g, gemm_split_choice(format, M, N, K, cus), row0 + nrows, M, st);
-        int choice;
-        const int first = gemm_rows_first(format, M, N, K, cus, choice);
-        if (first > 0)
-        {
-            if (!gemm_launch_rows<F, DUMP>(fn, g, choice, first, M, st))
-                return false;
-            g.tile0 = first / GEMM_BN;
-            choice = gemm_split_choice(format, M, N - first, K, cus);
-        }
-        return gemm_launch_rows<F, DUMP>(fn, g, choice, N, M, st);
+        const GemmPlan plan = gemm_plan(format, M, N, K, cu_count(device_id));
+        // weight rows from `from` to `to`, as far as they are wanted
+        const auto part = [&](int choice, int from, int to) {
+            const int low = DUMP && row0 > from ? row0 : from, high = DUMP && row0 + nrows < to ? row0 + nrows : to;
+            if (low >= high)
+                return true;
+            const int tile = choice < 0 || SPLIT[choice].rn < 2 ? GEMM_BN : 32 * SPLIT[choice].rn;
+            g.tile0 = (from + (low - from) / tile * tile) / GEMM_BN;
+            return gemm_launch_rows<F, DUMP>(fn, g, choice, high, M, st);
+        };
+        return part(plan.choice, 0, plan.first > 0 ? plan.first : N) && (plan.first == 0 || part(plan.rest, plan.first, N));
     }
 } // namespace llamql
 

@@ -121,8 +121,11 @@ def test_a_walk_dealt_to_wavefronts(capi, dev, oracle, fmt, M, N, K):
     (63, 8161, 2048), (33, 8161, 4864),     # 64 x 32
     (129, 4999, 1536), (129, 4999, 2816),   # 64 x 64: the last token tile of one token, a super-block left over
     (64, 20001, 1024), (33, 24997, 1280),   # 64 x 128
-    (97, 9799, 4352), (193, 8000, 2560),    # 96 x 64
-    (128, 24997, 1280), (257, 8129, 2304),  # 128 x 128
+    (66, 4259, 768),                        # 32 x 64, several token tiles
+    (67, 8573, 1280),                       # 96 x 64: the last token tile of three tokens less, rows and a super-block left over
+    (324, 5397, 1792),                      # 128 x 64
+    (97, 9799, 4352), (193, 8000, 2560), (257, 8129, 2304),  # (others by format)
+    (128, 24997, 1280),                     # 128 x 128
     (255, 24997, 1280),                     # and short of a tile both ways
     (512, 8192, 1280),                      # one whole round of them
 ])
@@ -153,11 +156,25 @@ def test_tiles_of_dealt_walks(capi, dev, oracle, fmt, M, N, K):
 
 
 @pytest.mark.parametrize("fmt", list(FMTS.values()), ids=list(FMTS))
-@pytest.mark.parametrize("M,N,K,first", [(193, 17159, 1024, 16384), (65, 18660, 3840, 16384), (193, 19075, 1536, 16384),
-                                         (250, 8191, 4096, 0)])
-def test_rows_in_two_launches(capi, dev, oracle, fmt, M, N, K, first):
-    """Rows whose tiles fill whole rounds and the rest as a launch of its own (and, without one, the tile of 128 x 64): every element
-    written, those on both sides of the seam and the last ones near the oracle's, the same bits again."""
+@pytest.mark.parametrize("M,N,K,seams", [  # seams: where the second launch of Q4_K, Q6_K and IQ3_S begins (0: there is none)
+    (193, 17159, 1024, (0, 0, 0)),
+    (65, 18660, 3840, (16384, 0, 0)),
+    (193, 19075, 1536, (0, 0, 0)),
+    (250, 8191, 4096, (0, 0, 0)),
+    (196, 16697, 2304, (16384, 16384, 16384)),
+    (262, 11930, 2560, (0, 6528, 6528)),
+    (205, 18287, 2304, (16384, 16384, 16384)),
+    (198, 19661, 2304, (16384, 16384, 16384)),
+    (222, 18644, 2304, (16384, 16384, 16384)),
+    (77, 17381, 4864, (16384, 16384, 16384)),
+    (132, 11388, 2816, (10880, 0, 0)),
+    (100, 10226, 8192, (8192, 8192, 8192)),
+    (338, 14686, 2560, (10880, 10880, 10880)),
+])
+def test_rows_in_two_launches(capi, dev, oracle, fmt, M, N, K, seams):
+    """Rows whose tiles fill whole rounds and the rest as a launch of its own (and some sizes that one launch does): every element
+    written, those on both sides of the seam and the last ones near the oracle's, the same bits again, and the block sums of
+    windows that lie on both sides of the seam bit for bit."""
     import torch
 
     W = synth.weights_numpy(fmt, N, K, 31 + M)
@@ -169,10 +186,13 @@ def test_rows_in_two_launches(capi, dev, oracle, fmt, M, N, K, first):
     sync()
     assert torch.equal(y[:, :N], again[:, :N]) and bool(torch.isnan(y[:, N:]).all()) and not bool(torch.isnan(y[:, :N]).any())
     got = y.cpu().numpy()
-    for r0 in (max(0, first - 48), N - 96):
-        C = oracle.gemm(fmt, W, K, q8, n0=r0, n1=r0 + 96)
+    for r0 in (max(0, seams[list(FMTS.values()).index(fmt)] - 48), N - 96):
+        C, sums = oracle.gemm(fmt, W, K, q8, n0=r0, n1=r0 + 96, want_sums=True)
         assert rel_err(got[:, r0:r0 + 96], C) <= TOL[fmt] * 1e-2
         assert np.abs(got[:, r0:r0 + 96] - C).max() <= 1e-4 * np.abs(C).max()
+        s = capi.gemm_block_sums(fmt, wd, qd, M, N, K, r0, 96)
+        sync()
+        assert np.array_equal(s.cpu().numpy(), sums)
 
 
 @pytest.mark.parametrize("fmt", list(FMTS.values()), ids=list(FMTS))
@@ -204,7 +224,8 @@ def test_dealt_walks_round_no_coarser_than_four_sums(capi, dev, oracle, fmt, M, 
 
 
 @pytest.mark.parametrize("fmt", list(FMTS.values()), ids=list(FMTS))
-@pytest.mark.parametrize("M,N,K", [(40, 1000, 2304), (129, 4999, 1536), (97, 9799, 1536), (255, 24997, 512)])
+@pytest.mark.parametrize("M,N,K", [(40, 1000, 2304), (129, 4999, 1536), (97, 9799, 1536), (255, 24997, 512), (66, 4259, 768), (20, 12001, 1280),
+                                   (35, 4155, 768), (33, 24997, 1280), (67, 8573, 1280), (129, 11253, 768), (324, 5397, 1792)])
 def test_dealt_walks_at_the_ends_of_the_scales(capi, dev, oracle, fmt, M, N, K):
     """Scales that are not finite, and scales that are fp16's smallest: an infinite or undefined scale of one Q8_1 block makes
     exactly that token's outputs what the sums as such are (infinite, or not a number), weights' scales below fp16's normal
@@ -241,7 +262,7 @@ def test_dealt_walks_at_the_ends_of_the_scales(capi, dev, oracle, fmt, M, N, K):
 
 @pytest.mark.parametrize("fmt", list(FMTS.values()), ids=list(FMTS))
 @pytest.mark.parametrize("M,N,K", [(31, 4095, 2304), (20, 12001, 4864), (40, 1000, 2304), (129, 4999, 1536), (33, 24997, 1280),
-                                   (199, 5120, 1536), (255, 24997, 1280), (256, 8192, 2048)])
+                                   (199, 5120, 1536), (255, 24997, 1280), (256, 8192, 2048), (66, 4259, 768), (35, 4155, 768), (324, 5397, 1792)])
 def test_an_infinite_scale_leaves_other_tokens_and_rows_alone(capi, dev, oracle, fmt, M, N, K):
     """An infinity in one token and one in one row of W: every other element has the bits that it has without them."""
     import torch

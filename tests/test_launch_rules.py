@@ -4,12 +4,15 @@ import math
 import re
 from pathlib import Path
 
+import numpy as np
 import pytest
 
-from tests import test_gpu_experts_small, test_gpu_gemm, test_gpu_linear_tiled
+from oracle.binding import FMT_IQ3_S, FMT_Q4_K, FMT_Q6_K
+from tests import fake_hip, test_gpu_experts_small, test_gpu_gemm, test_gpu_linear_tiled
 
 CSRC = Path(__file__).resolve().parent.parent / "llaminar_amd" / "csrc"
 CUS = 256
+FORMATS = [FMT_Q4_K, FMT_Q6_K, FMT_IQ3_S]
 
 
 def over(a, b):
@@ -62,75 +65,142 @@ def test_every_tile_of_grouped_layers_has_sizes(kind):
     assert chosen == set(range(len(TILES[kind])))
 
 
-# ---- prompt GEMM (gemm.hip: gemm_split_choice) -----------------------------------------------------------
+# ---- prompt GEMM (gemm.hip: gemm_plan): what the library launches --------------------------------------------
 
 GEMM = (CSRC / "gemm.hip").read_text()
+TILES_OF_WALKS = [tuple(map(int, t)) for t in re.findall(r"\{(\d), (\d), (\d), \{", re.search(r"SPLIT\[\] = \{(.*?)\}\}; //", GEMM, re.S).group(1))]
+WHOLE = -1   # gemm_kernel, as the tables beside the rule have it
+LAUNCHES = """
+lib = ctypes.CDLL({library!r})
+p, i = ctypes.c_void_p(1 << 20), ctypes.c_int
+def launches(ok):
+    assert ok
+    return [l[1:] for l in log() if l[0] == "launch"]
+answer([[launches(lib.llam_ql_gemm(ctypes.c_uint8(fmt), p, p, p, i(M), i(N), i(K), i(N), i(0), None)),
+         launches(lib.llam_ql_gemm_block_sums(ctypes.c_uint8(fmt), p, p, p, i(M), i(N), i(K), i(row0), i(rows or N), i(0), None))]
+        for fmt, M, N, K, row0, rows in {calls}])
+"""
 
 
-def triples(text):
-    return [tuple(map(float, t)) for t in re.findall(r"\{([\d.]+), ([\d.]+), ([\d.]+)\}", text)]
+def gemm_launches(tmp_path, calls):
+    """(format, M, N, K, first row, rows of the sums; 0: all) -> the launches of the product and of its block sums, each
+    (tile or tokens, grid), as the library makes them."""
+    def read(kernel, *numbers):
+        if tile := re.search(r"gemm_split_kernel\w+TraitsELi(\d)ELi(\d)ELi(\d)ELb[01]ELb([01])E", kernel):
+            return tuple(map(int, tile.groups())), tuple(map(int, numbers[:2]))
+        return int(re.search(r"gemm_kernel\w+TraitsELb[01]ELi(\d+)E", kernel).group(1)), tuple(map(int, numbers[:2]))
+    answer = fake_hip.run(tmp_path, LAUNCHES.format(library=str(CSRC.parent / "lib" / "libllaminar_ql.so"), calls=calls))
+    return [tuple([read(*launch) for launch in side] for side in call) for call in answer]
 
 
-TABLE = re.search(r"SPLIT\[\] = \{(.*?)\}\};", GEMM, re.S).group(1) + "}"
-SPLIT = list(zip([tuple(map(int, t)) for t in re.findall(r"\{(\d), (\d), (\d), \{", TABLE)], triples(TABLE)))
-START, WHOLE_START = map(float, re.search(r"SPLIT_START = ([\d.]+), WHOLE_START = ([\d.]+)", GEMM).groups())
-WHOLE = triples(re.search(r"WHOLE\[\] = \{(.*?)\}\}\};", GEMM, re.S).group(1) + "}")
+def test_block_sums_run_on_the_launches_of_the_product(tmp_path):
+    shapes = [(324, 5397, 1792), (196, 16697, 2304), (77, 17381, 4864), (338, 14686, 2560), (40, 8192, 5120), (130, 257, 256), (9, 70, 768)]
+    calls = [(fmt, *s, 0, 0) for fmt in FORMATS for s in shapes]
+    cut = 0
+    for call, (product, sums) in zip(calls, gemm_launches(tmp_path, calls)):
+        assert product == sums, call
+        cut += len(product) == 2
+    assert cut >= 9
+    # a window on both sides of the seam at row 16384, and one on either: the workgroups that meet it
+    calls = [(FORMATS[0], 196, 16697, 2304, *w) for w in ((16300, 100), (16000, 384), (16384, 64))]
+    (_, both), (_, below), (_, above) = gemm_launches(tmp_path, calls)
+    assert [t[:3] for t, _ in both] == [(4, 4, 1), (1, 1, 4)] and [g for _, g in both] == [(1, 2), (1, 7)]
+    assert [t[:3] for t, _ in below] == [(4, 4, 1)] and below[0][1] == (3, 2)
+    assert [t[:3] for t, _ in above] == [(1, 1, 4)] and above[0][1] == (2, 7)
 
 
-def gemm_choice(fmt, M, N, K):
-    """fmt: 0, 1, 2 for Q4_K, Q6_K, IQ3_S."""
-    SB, kind = K // 256, 0 if M <= 32 else 1 if M <= 64 else 2
-    full, last, alone = (t[fmt] for t in WHOLE[3 * kind:3 * kind + 3])
-    tiles = over(N, 64) * over(M, (32, 64, 128)[kind])
-    before = (tiles - 1) // (2 * CUS)
-    rest = tiles - before * 2 * CUS
-    light = rest == 2 * CUS and (M <= 32 or (M > 64 and SB <= 4))
-    end = alone if rest <= CUS else full if light else last
-    best, choice = 0.97 * (WHOLE_START + SB * (before * full + end)), -1
-    for i, ((mt, rn, ks), step) in enumerate(SPLIT):
-        groups = over(N, 32 * rn) * over(M, 32 * mt)
-        left = groups % CUS
-        rounds = 1.0 if groups <= CUS else groups // CUS + (0.6 + 0.4 * left / CUS if left else 0.0)
-        us = rounds * (over(SB, ks) * step[fmt] + START)
-        if us < best:
-            best, choice = us, i
-    return choice
+def gemm_parts(tmp_path, calls):
+    """(format, M, N, K) -> [(entry of SPLIT or WHOLE, launched tile or tokens, rows of W before it, its rows)], first launch first."""
+    out = []
+    for (_, M, N, K), (product, _) in zip(calls, gemm_launches(tmp_path, [(*c, 0, 1) for c in calls])):
+        entries = [TILES_OF_WALKS.index(t[:3]) if isinstance(t, tuple) else WHOLE for t, _ in product]
+        heights = [32 * t[0] if isinstance(t, tuple) else t for t, _ in product]
+        widths = [32 * t[1] if isinstance(t, tuple) else 64 for t, _ in product]
+        assert [g[1] for _, g in product] == [over(M, h) for h in heights]
+        if len(product) == 1:
+            assert product[0][1][0] == over(N, widths[0])
+            out.append([(entries[0], product[0][0], 0, N)])
+        else:
+            # (the first launch's rows are a multiple of 64: those that leave the second its tiles)
+            first = [f for f in range(64, N, 64) if over(f, widths[0]) == product[0][1][0] and over(N - f, widths[1]) == product[1][1][0]]
+            assert first
+            out.append([(entries[0], product[0][0], 0, first[0]), (entries[1], product[1][0], first[0], N - first[0])])
+    return out
 
 
-def test_the_prompt_gemm_takes_the_fastest_kernel_of_each_measured_size():
+def test_the_prompt_gemm_takes_the_fastest_kernel_of_each_measured_size(tmp_path):
     """The tables of measured times beside the rule: within 3 % of the fastest (two sizes of a table are that close)."""
     names = ["Q4_K", "Q6_K", "IQ3_S"]
     rows = re.findall(r"//   (\d+) x (\d+) x (\d+), (\w+) +([\d. ]+)\n", GEMM)
     assert len(rows) == 16
-    for M, N, K, fmt, times in rows:
+    plans = gemm_parts(tmp_path, [(FORMATS[names.index(fmt)], int(M), int(N), int(K)) for M, N, K, fmt, _ in rows])
+    for (M, N, K, fmt, times), parts in zip(rows, plans):
         times = [float(t) for t in times.split()]
-        assert len(times) == 8
-        assert times[1 + gemm_choice(names.index(fmt), int(M), int(N), int(K))] <= 1.03 * min(times), (M, N, K, fmt)
+        assert len(times) == 1 + len(TILES_OF_WALKS) - 1
+        if len(parts) == 1 and parts[0][0] < len(times) - 1:
+            assert times[1 + parts[0][0]] <= 1.03 * min(times), (M, N, K, fmt)
     number = r"([\d.]+), ([\d.]+), ([\d.]+)"
     full = re.findall(rf"(\d+) x (\d+) x (\d+) +{number} (->|:) {number} \((\d)\)", GEMM)
     assert len(full) == 8
+    plans = iter(gemm_parts(tmp_path, [(fmt, int(M), int(N), int(K)) for M, N, K, *_ in full for fmt in FORMATS]))
     for M, N, K, *rest in full:
         M, N, K, entry = int(M), int(N), int(K), int(rest[7])
         assert over(N, 64) * over(M, 32 if M <= 32 else 64 if M <= 64 else 128) % (2 * CUS) == 0
         whole, other = [float(t) for t in rest[:3]], [float(t) for t in rest[4:7]]
         for fmt in range(3):
-            assert gemm_choice(fmt, M, N, K) == (entry if rest[3] == "->" else -1)
+            assert [p[0] for p in next(plans)] == [entry if rest[3] == "->" else WHOLE]
             assert (other if rest[3] == "->" else whole)[fmt] <= 1.01 * (whole if rest[3] == "->" else other)[fmt]
 
 
-def test_every_kernel_of_the_prompt_gemm_has_sizes():
-    assert len(SPLIT) == GEMM.count("case") - GEMM.count("case LLAM") == 7 and len(WHOLE) == 9
+def entries_of(tmp_path, fmt, shapes):
+    return {p[0] for parts in gemm_parts(tmp_path, [(fmt, *s) for s in shapes]) for p in parts}
+
+
+@pytest.mark.parametrize("fmt", FORMATS)
+def test_every_kernel_of_the_prompt_gemm_has_sizes(fmt, tmp_path):
+    assert len(TILES_OF_WALKS) == GEMM.count("case") - GEMM.count("case LLAM") == 8
+    walks = set(range(len(TILES_OF_WALKS)))
     dealt = sizes(test_gpu_gemm.test_a_walk_dealt_to_wavefronts) + sizes(test_gpu_gemm.test_tiles_of_dealt_walks)
     products = sizes(test_gpu_gemm.test_random_shapes) + dealt
     sums = [s[:3] for s in sizes(test_gpu_gemm.test_block_sums_of_the_gemm_kernel)] + dealt
-    for fmt in range(3):
-        for shapes in (products, sums):
-            chosen = {s: gemm_choice(fmt, *s) for s in shapes}
-            assert set(chosen.values()) == set(range(-1, len(SPLIT)))
-            for i, ((mt, rn, ks), _) in enumerate(SPLIT):
-                own = [s for s in shapes if chosen[s] == i]
-                assert any(M % (32 * mt) for M, N, K in own) and any(N % (32 * rn) for M, N, K in own), (fmt, SPLIT[i])
-                assert ks == 1 or any(K // 256 % ks for M, N, K in own), (fmt, SPLIT[i])
-            undivided = [M for M, N, K in shapes if chosen[M, N, K] == -1]
-            assert {0 if M <= 32 else 1 if M <= 64 else 2 for M in undivided} == {0, 1, 2}, "a tile of 32, 64 or 128 tokens"
-            assert any(M % 64 for M in undivided if 32 < M <= 64)
+    for shapes in (products, sums):
+        plans = dict(zip(shapes, gemm_parts(tmp_path, [(fmt, *s) for s in shapes])))
+        alone = {s: parts[0] for s, parts in plans.items() if len(parts) == 1}
+        assert {p[0] for p in alone.values()} == walks | {WHOLE}
+        for i, (mt, rn, ks) in enumerate(TILES_OF_WALKS):
+            own = [s for s, p in alone.items() if p[0] == i]
+            assert any(M % (32 * mt) for M, N, K in own) and any(N % (32 * rn) for M, N, K in own), TILES_OF_WALKS[i]
+            assert ks == 1 or any(K // 256 % ks for M, N, K in own), TILES_OF_WALKS[i]
+        undivided = [M for (M, N, K), p in alone.items() if p[0] == WHOLE]
+        assert {alone[s][1] for s in alone if alone[s][0] == WHOLE} == {32, 64, 128}
+        assert any(M % 64 for M in undivided if 32 < M <= 64)
+        # (Q4_K walks of 32 x 64: weights by way of LDS for one token tile, straight into registers for several)
+        ways = {p[1][3] for p in alone.values() if p[0] == 1}
+        assert ways == ({0, 1} if fmt == FMT_Q4_K else {1})
+    # scales that are not finite: every walk has a second one
+    for test in (test_gpu_gemm.test_dealt_walks_at_the_ends_of_the_scales, test_gpu_gemm.test_an_infinite_scale_leaves_other_tokens_and_rows_alone):
+        assert entries_of(tmp_path, fmt, sizes(test)) >= walks
+
+
+@pytest.mark.parametrize("fmt", FORMATS)
+def test_launches_in_two_have_sizes(fmt, tmp_path):
+    """The seam of every size is where the GPU test looks, and each format has first and second launches of the tiles that it uses."""
+    cut = sizes(test_gpu_gemm.test_rows_in_two_launches)
+    firsts, rests = set(), set()
+    for (M, N, K, seams), parts in zip(cut, gemm_parts(tmp_path, [(fmt, *s[:3]) for s in cut])):
+        assert seams[FORMATS.index(fmt)] == (parts[1][2] if len(parts) == 2 else 0), (M, N, K)
+        if len(parts) == 2:
+            firsts.add(parts[0][0])
+            rests.add(parts[1][0])
+    random, calls = np.random.default_rng(1), []
+    while len(calls) < 1500:
+        N, K = int(np.exp(random.uniform(np.log(1000), np.log(25600)))), 256 * int(np.exp(random.uniform(np.log(4), np.log(100))))
+        M = int(np.exp(random.uniform(np.log(9), np.log(max(10, min(2048, 512 * 25600 * 5120 // (N * K)))))))
+        calls.append((fmt, M, N, K))
+    count = {}
+    for parts in gemm_parts(tmp_path, calls):
+        if len(parts) == 2:
+            for key in (("first", parts[0][0]), ("rest", parts[1][0])):
+                count[key] = count.get(key, 0) + 1
+    used = {key for key, n in count.items() if n >= 3}
+    assert len(used) >= 5 and used <= {("first", f) for f in firsts} | {("rest", r) for r in rests}
