@@ -964,51 +964,56 @@ namespace llamql
     // Which kernel a shape takes: -1 for gemm_kernel, or an entry of SPLIT.  gemm_kernel's workgroup walks the whole of K
     // alone, two of them on a compute unit; gemm_split_kernel has one there and gives the walk to 2, 4 or 8 wavefronts.
     // The expected times in microseconds are fitted to measurements, weights from memory (us, gemm_kernel and the entries):
-    //   tokens x rows x K             gemm_kernel  0: 1,1,4  1: 1,2,2  2: 2,1,4  3: 2,2,2  4: 2,4,1  5: 3,2,2  6: 4,4,1
-    //   10 x 4096 x 4096, Q4_K            17.0      8.8     12.9     12.3     17.6     28.7     23.2     48.3
-    //   64 x 4096 x 4096, IQ3_S           31.7     11.1     16.2     14.5     19.9     34.1     24.3     48.3
-    //   20 x 12000 x 4096, IQ3_S          25.7     20.0     17.3     27.9     21.0     34.7     25.9     49.0
-    //   40 x 8192 x 5120, IQ3_S           42.0     24.3     20.8     18.2     24.4     42.8     30.6     60.3
-    //   63 x 5034 x 18944, Q6_K            158     78.2     69.9     62.4     87.3      150      104      207
-    //   130 x 5000 x 5120, Q4_K           53.2     39.7     34.6     29.8     23.5     36.2     29.5     61.1
-    //   64 x 25600 x 5120, Q4_K           56.8     73.9     69.6     63.3     46.8     41.7     59.5     65.0
-    //   80 x 9762 x 3072, Q6_K            42.1     35.1     28.0     36.8     32.0     30.4     23.1     40.6
-    //   199 x 5120 x 25600, Q6_K           303      236      241      223      200      204      144      285
-    //   256 x 8192 x 8192, Q4_K           91.9      124      102     93.0     67.2     62.2     87.4     97.3
-    //   1000 x 4096 x 4096, Q4_K          69.3      131      107     97.5     71.0     62.3     72.9     57.6
-    //   256 x 25600 x 5120, Q4_K           156      252      222      194      156      149      157      137
-    //   16 x 25600 x 5120, Q6_K           50.1     51.3     45.4     72.0     54.1     50.0     63.8     66.3
-    //   384 x 25600 x 5120, Q4_K           203      380      322      282      220      195      218      198
-    //   512 x 25600 x 5120, Q4_K           271      500      423      370      286      261      306      264
-    //   2048 x 6400 x 5120, IQ3_S          264      515      465      367      296      291      275      257
+    //   tokens x rows x K             gemm_kernel  0: 1,1,4  1: 1,2,2  2: 2,1,4  3: 2,2,2  4: 2,4,1  5: 3,2,2  6: 4,4,1  7: 4,2,2
+    //   10 x 4096 x 4096, Q4_K           19.0      8.8     12.8     12.5     17.9     30.1     24.0     50.2     28.5
+    //   64 x 4096 x 4096, IQ3_S          33.1     11.3     16.5     15.5     20.1     34.4     25.1     50.0     31.5
+    //   20 x 12000 x 4096, IQ3_S         24.9     19.5     16.8     27.2     20.4     34.3     25.6     49.4     31.9
+    //   40 x 8192 x 5120, IQ3_S          41.1     23.8     20.8     18.0     24.2     42.2     30.8     61.7     39.2
+    //   63 x 5034 x 18944, Q6_K           165     77.8     74.9     67.0     92.2      155      109      219      146
+    //   130 x 5000 x 5120, Q4_K          52.0     38.9     32.4     30.0     23.6     37.3     29.8     61.7     35.6
+    //   64 x 25600 x 5120, Q4_K          53.7     72.0     64.1     61.6     45.7     40.4     59.6     64.4     73.0
+    //   80 x 9762 x 3072, Q6_K           39.9     34.3     28.9     36.6     31.9     30.2     22.9     41.5     30.0
+    //   199 x 5120 x 25600, Q6_K          295      238      249      229      204      209      139      296      194
+    //   256 x 8192 x 8192, Q4_K          87.0      122     96.7     94.9     67.9     62.9     89.9     96.7     62.9
+    //   1000 x 4096 x 4096, Q4_K         66.5      129     99.5     97.6     71.7     64.4     74.3     58.8     64.2
+    //   256 x 25600 x 5120, Q4_K          152      246      203      193      152      153      149      136      146
+    //   16 x 25600 x 5120, Q6_K          49.9     51.2     46.5     73.5     55.1     51.9     66.2     69.4     86.0
+    //   384 x 25600 x 5120, Q4_K          198      374      296      279      216      191      213      200      184
+    //   512 x 25600 x 5120, Q4_K          264      491      389      368      282      267      295      268      254
+    //   2048 x 6400 x 5120, IQ3_S         265      508      465      359      296      293      270      263      259
     // Tiles that fill their last round exactly, one round or several (us, gemm_kernel and the entry that is taken; Q4_K, Q6_K, IQ3_S):
-    //   1024 x 4096 x 4096    67.7, 77.2, 68.1 -> 57.4, 58.3, 56.5 (6)     512 x 16384 x 4096    131, 157, 135 -> 116, 115, 111 (6)
-    //   512 x 8192 x 12800    207, 241, 213 -> 162, 169, 157 (6)           40 x 32768 x 1024     15.3, 19.3, 17.3 -> 13.6, 16.2, 14.3 (4)
-    //   2048 x 4096 x 2048    69.2, 78.3, 71.6 -> 64.1, 64.4, 63.8 (6)     1024 x 8192 x 2048    70.2, 79.5, 70.9 -> 64.4, 64.7, 61.8 (6)
-    //   64 x 32768 x 2048     26.3, 32.8, 29.4 -> 21.1, 26.4, 23.4 (4)
+    //   1024 x 4096 x 4096     66.8, 75.9, 66.8 -> 58.8, 58.9, 57.0 (6)
+    //   512 x 16384 x 4096     128.2, 147.5, 130.3 -> 114.3, 115.4, 112.0 (6)
+    //   512 x 8192 x 12800     197.4, 229.9, 199.7 -> 166.2, 167.5, 161.7 (6)
+    //   40 x 32768 x 1024      14.8, 18.1, 16.0 -> 13.1, 15.5, 13.9 (4)
+    //   2048 x 4096 x 2048     67.5, 75.0, 67.5 -> 63.6, 62.7, 62.1 (6)
+    //   1024 x 8192 x 2048     66.4, 75.2, 66.9 -> 63.2, 63.4, 61.6 (6)
+    //   64 x 32768 x 2048      26.0, 32.5, 28.1 -> 21.2, 26.3, 23.3 (4)
     // and gemm_kernel's (us, gemm_kernel and the entry that would come next):
-    //   1000 x 4096 x 512     13.6, 14.3, 13.6 : 14.5, 14.2, 14.3 (6)
+    //   1000 x 4096 x 512      12.6, 13.4, 12.5 : 14.2, 13.9, 14.0 (6)
     struct SplitTile
     {
         int mt, rn, ks;
         double step[3]; // microseconds: a step (KS super-blocks) of Q4_K, Q6_K and IQ3_S
     };
     constexpr SplitTile SPLIT[] = {
-        {1, 1, 4, {1.7, 1.85, 1.65}}, {1, 2, 2, {1.45, 1.8, 1.65}}, {2, 1, 4, {2.25, 2.9, 2.7}}, {2, 2, 2, {1.85, 2.2, 1.9}},
-        {2, 4, 1, {1.65, 2.15, 2.0}}, {3, 2, 2, {2.5, 2.6, 2.5}}, {4, 4, 1, {3.2, 3.3, 2.9}},
-        {4, 2, 2, {3.75, 4.15, 3.85}}}; // (the last one's activations leave the weights no room in LDS)
+        {1, 1, 4, {1.7, 1.85, 1.75}}, {1, 2, 2, {1.45, 1.8, 1.68}}, {2, 1, 4, {2.25, 2.9, 2.9}}, {2, 2, 2, {1.85, 2.2, 2.07}},
+        {2, 4, 1, {1.65, 2.15, 1.95}}, {3, 2, 2, {2.5, 2.6, 2.7}}, {4, 4, 1, {3.2, 3.3, 2.9}},
+        {4, 2, 2, {3.75, 4.15, 3.6}}}; // (the last one's activations leave the weights no room in LDS)
     constexpr int SPLITS = (int)(sizeof(SPLIT) / sizeof(SPLIT[0]));
     constexpr double SPLIT_START = 3.5, WHOLE_START = 2.0; // a workgroup's start and end
     inline double split_expected(const SplitTile &t, int format, int M, int N, int K, int cus)
     {
         const auto over = [](long a, long b) { return (a + b - 1) / b; };
-        // (a last round of few workgroups is faster: they have the memory and the clock to themselves; not one of at most eight steps,
-        // which is over before that shows: us, 1757 x 3121 x 1792 IQ3_S 49.7 by gemm_kernel and 54.3 by
-        // entry 6, 876 x 2630 x 1280 Q4_K 22.0 by entry 6 and 25.2 by 4)
-        const long groups = over(N, 32 * t.rn) * over(M, 32 * t.mt), left = groups % cus, steps = over(K / 256, t.ks);
-        const double last = left == 0 ? 0.0 : steps <= 8 ? 1.0 : 0.6 + 0.4 * (double)left / cus;
-        const double rounds = groups <= cus ? 1.0 : (double)(groups / cus) + last;
-        return rounds * ((double)steps * t.step[format] + SPLIT_START);
+        const long groups = over(N, 32 * t.rn) * over(M, 32 * t.mt), left = groups % cus;
+        const double round = (double)over(K / 256, t.ks) * t.step[format] + SPLIT_START;
+        // A last round of few workgroups is faster, for they have the memory and the clock to themselves: of a tenth of the chip by 8 % in
+        // rounds of up to 10 us, by a quarter from 40 us on.  (Second rounds of 26 and of 128 workgroups, as shares of whole ones: entry 0, Q4_K,
+        // 5 us 0.91 and 0.86, 18 us 0.90, 0.87; entry 1, Q6_K, 8 us 0.90, 0.87, 19 us 0.78, 0.75; entry 3, Q4_K, 12 us 0.93, 0.92, 35 us 0.86,
+        // 0.90; entry 6, Q4_K, 22 us 0.76, 0.76, 60 us 0.78, 0.83; Q6_K, 35 us 0.68, 0.73; entry 7, Q4_K, 14 us 0.87, 0.85, 50 us 0.81, 0.82.)
+        const double lighter = 0.08 + 0.17 * (round < 10 ? 0.0 : round > 40 ? 1.0 : (round - 10) / 30);
+        const double last = left == 0 ? 0.0 : 1.0 - lighter * (1.0 - (double)left / cus);
+        return (groups <= cus ? 1.0 : (double)(groups / cus) + last) * round;
     }
     // gemm_kernel: microseconds a super-block of a tile of 32, 64 or 128 tokens takes in a round of two workgroups a compute unit
     // that others follow, in the last round, and in a last round of one
@@ -1038,7 +1043,7 @@ namespace llamql
         const double undivided = WHOLE_START + SB * ((double)rounds_before * whole.full[format] + last[format]);
         double best = 0.97 * undivided;
         int choice = -1;
-        for (int i = 0; i < SPLITS - 1; ++i)
+        for (int i = 0; i < SPLITS; ++i)
         {
             const SplitTile &t = SPLIT[i];
             if (over(M, 32 * t.mt) > 65535) // (the grid's second extent)
@@ -1052,11 +1057,11 @@ namespace llamql
         return choice;
     }
 
-    // A launch whose last round of tiles is sparse does better as two: the rows whose tiles fill whole rounds by themselves, and
-    // the rest, as tiles that fit it.  The first's rows are a multiple of 64.  The second waits for the first to end and starts anew: GEMM_SECOND microseconds, and only where a twentieth is gained
-    // and the first's walks have more than eight steps (seven: 1757 x 3121 x 1792 Q4_K 52.1 us in one launch, 56.6 in two, with the quantiser).
+    // A launch whose last round of tiles is sparse does better as two: the rows whose tiles fill whole rounds by themselves (a
+    // multiple of 64), and the rest, as tiles that fit it.  The second waits for the first to end and starts anew: GEMM_SECOND
+    // microseconds, and only where a twentieth is gained.
     // Measured, one launch and two: 512 x 25600 x 5120 Q4_K 260 -> 227 us, Q6_K 263 -> 229, 2048 x 6400 x 5120 Q4_K 262 -> 222, 82 x 19449 x 19968
-    // Q4_K 210 -> 164, 384 x 25600 x 5120 IQ3_S 193 -> 169.
+    // Q4_K 210 -> 164, 384 x 25600 x 5120 IQ3_S 193 -> 169, 37 x 17420 x 7680 Q6_K 78.3 -> 60.3, 101 x 17640 x 3328 Q4_K 43.8 -> 36.9.
     constexpr double GEMM_SECOND = 3.0;
     struct GemmPlan
     {
@@ -1070,17 +1075,13 @@ namespace llamql
         GemmPlan plan = {gemm_split_choice(format, M, N, K, cus, &whole), 0, -1};
         if (K > 1 << 24)
             return plan;
-        // (the last entry for launches that it alone fits in one round or fills evenly; us, the best of the others and this one: 256 x
-        // 8192 x 8192 Q6_K and IQ3_S 76, 72 -> 69.8, 64.8)
-        if (const double us = split_expected(SPLIT[SPLITS - 1], format, M, N, K, cus); us < 0.97 * whole && over(M, 128) <= 65535)
-            plan.choice = SPLITS - 1, whole = us;
         double best = 0.95 * whole;
-        for (int i = 0; i < SPLITS - 1; ++i)
+        for (int i = 0; i < SPLITS; ++i)
         {
             const SplitTile &t = SPLIT[i];
             const long across = over(M, 32 * t.mt), rounds = over(N, 32 * t.rn) * across / cus;
             const int first = (int)(rounds * cus / across * 32 * t.rn) & ~63;
-            if (first < 64 || first >= N || across > 65535 || over(SB, t.ks) <= 8)
+            if (first < 64 || first >= N || across > 65535)
                 continue;
             double after;
             const int rest = gemm_split_choice(format, M, N - first, K, cus, &after);

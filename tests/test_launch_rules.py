@@ -121,10 +121,10 @@ def gemm_parts(tmp_path, calls):
             assert product[0][1][0] == over(N, widths[0])
             out.append([(entries[0], product[0][0], 0, N)])
         else:
-            # (the first launch's rows are a multiple of 64: those that leave the second its tiles)
+            # (the first launch has whole tiles, of rows that are a multiple of 64)
             first = [f for f in range(64, N, 64) if over(f, widths[0]) == product[0][1][0] and over(N - f, widths[1]) == product[1][1][0]]
             assert first
-            out.append([(entries[0], product[0][0], 0, first[0]), (entries[1], product[1][0], first[0], N - first[0])])
+            out.append([(entries[0], product[0][0], 0, first[-1]), (entries[1], product[1][0], first[-1], N - first[-1])])
     return out
 
 
@@ -136,8 +136,8 @@ def test_the_prompt_gemm_takes_the_fastest_kernel_of_each_measured_size(tmp_path
     plans = gemm_parts(tmp_path, [(FORMATS[names.index(fmt)], int(M), int(N), int(K)) for M, N, K, fmt, _ in rows])
     for (M, N, K, fmt, times), parts in zip(rows, plans):
         times = [float(t) for t in times.split()]
-        assert len(times) == 1 + len(TILES_OF_WALKS) - 1
-        if len(parts) == 1 and parts[0][0] < len(times) - 1:
+        assert len(times) == 1 + len(TILES_OF_WALKS)
+        if len(parts) == 1:
             assert times[1 + parts[0][0]] <= 1.03 * min(times), (M, N, K, fmt)
     number = r"([\d.]+), ([\d.]+), ([\d.]+)"
     full = re.findall(rf"(\d+) x (\d+) x (\d+) +{number} (->|:) {number} \((\d)\)", GEMM)
