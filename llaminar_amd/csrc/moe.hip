@@ -1008,6 +1008,7 @@ namespace llamql
     constexpr int MOE_GROUP_THREADS = 1024;
     constexpr int MOE_GROUP_MAX_PAIRS = 4096;
     constexpr int MOE_GROUP_MAX_EXPERTS = 2 * MOE_GROUP_THREADS; // two experts per thread
+    constexpr size_t MOE_GROUP_FIXED_LDS = (2 * MOE_GROUP_MAX_EXPERTS + 1 + 3 * (MOE_GROUP_THREADS / WAVE)) * sizeof(int);
     // Tokens of one expert that share a workgroup's pass over its matrix.  Measured on the
     // 256-expert IQ3_S shape: four pay from about 500 pairs on (64 tokens: 217 against 247 us
     // per step); below that the larger register footprint of the four-row body costs more than
@@ -1092,6 +1093,7 @@ namespace llamql
         extern __shared__ uint32_t grp_count[]; // [wavefront][expert / 2]: two 16-bit counts, of its pairs, later of those before its own
         __shared__ int hist[MOE_GROUP_MAX_EXPERTS + 1], chunk0[MOE_GROUP_MAX_EXPERTS];
         __shared__ int wave_sums[WAVES][3];
+        static_assert(sizeof(hist) + sizeof(chunk0) + sizeof(wave_sums) == MOE_GROUP_FIXED_LDS, "beside the counts");
         const MoEGroupView g = moe_group_view(ws, P);
         const int tid = threadIdx.x, lane = tid & (WAVE - 1), wave = tid >> 6, twos = (n_experts + 1) / 2;
         const int stretch = (P + WAVES * WAVE - 1) / (WAVES * WAVE) * WAVE;
@@ -2135,8 +2137,9 @@ extern "C" bool llam_ql_moe_group(const int32_t *d_ids, int n_tokens, int slot_s
         return fail(fn, "n_experts=%d: at most %d experts are grouped", n_experts, MOE_GROUP_MAX_EXPERTS);
     static LdsGrant grant;
     const size_t lds = (size_t)(MOE_GROUP_THREADS / WAVE) * ((n_experts + 1) / 2) * sizeof(uint32_t);
-    if (lds > 48 * 1024 && allow_lds(grant, reinterpret_cast<const void *>(&moe_group_kernel),
-                                     (size_t)(MOE_GROUP_THREADS / WAVE) * MOE_GROUP_MAX_EXPERTS * sizeof(uint16_t)) != hipSuccess)
+    if (lds + MOE_GROUP_FIXED_LDS > 64 * 1024 &&
+        allow_lds(grant, reinterpret_cast<const void *>(&moe_group_kernel),
+                  (size_t)(MOE_GROUP_THREADS / WAVE) * MOE_GROUP_MAX_EXPERTS * sizeof(uint16_t)) != hipSuccess)
         return fail(fn, "cannot reserve %zu bytes of LDS", lds);
     int bits = 0;
     while ((1 << bits) < n_experts)

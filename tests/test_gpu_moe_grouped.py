@@ -69,7 +69,7 @@ def test_grouped_batches_against_slots(capi, dev, name, hidden, inter, routed, T
         assert torch.equal(out_g[7], base[7] if accumulate else torch.zeros_like(base[7]))
 
 
-@pytest.mark.parametrize("T,S,E", [(1, 1, 1), (455, 9, 257), (4096, 1, 2048), (1, 4096, 3), (1024, 1, 2047), (63, 1, 64), (65, 1, 1)])
+@pytest.mark.parametrize("T,S,E", [(1, 1, 1), (455, 9, 257), (4096, 1, 2048), (1, 4096, 3), (1024, 1, 2047), (63, 1, 64), (65, 1, 1), (999, 1, 1531)])
 def test_pairs_sorted_by_expert(capi, dev, T, S, E):
     import torch
 

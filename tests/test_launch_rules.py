@@ -204,3 +204,20 @@ def test_launches_in_two_have_sizes(fmt, tmp_path):
                 count[key] = count.get(key, 0) + 1
     used = {key for key, n in count.items() if n >= 3}
     assert len(used) >= 5 and used <= {("first", f) for f in firsts} | {("rest", r) for r in rests}
+
+
+# ---- grouping of pairs by expert (moe.hip) ----------------------------------------------------------------
+
+@pytest.mark.parametrize("experts", [1, 1528, 1529, 1536, 1537, 2048])
+def test_grouping_asks_for_the_lds_that_it_takes(experts, tmp_path):
+    """Two counts a word and wavefront beside the arrays of 2048 experts: more than 64 KiB has to be asked for before the launch."""
+    fixed = (2 * 2048 + 1 + 3 * 16) * 4
+    calls = fake_hip.run(tmp_path, f"""
+lib, p, i = ctypes.CDLL({str(CSRC.parent / "lib" / "libllaminar_ql.so")!r}), ctypes.c_void_p(1 << 20), ctypes.c_int
+assert lib.llam_ql_moe_group(p, i(999), i(1), i({experts}), p, i(0), None)
+answer(log())
+""")
+    dynamic = int(calls[-1][-1])
+    assert calls[-1][0] == "launch" and "moe_group_kernel" in calls[-1][1] and dynamic == 16 * over(experts, 2) * 4
+    granted = max([int(c[2]) for c in calls if c[0] == "lds"], default=64 * 1024 - fixed)
+    assert dynamic <= granted
