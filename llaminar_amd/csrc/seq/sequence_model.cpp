@@ -57,8 +57,9 @@ namespace
     constexpr int NORM_FUSE_MAX = 8192; // values a linear layer norms by itself
     constexpr int LOGIT_ROWS = 64;      // rows of logits computed at a time
     // Between two graphs the GPU stands still for 8 us (a step of three sequences, width 2048, fp32: 252), so steps are replayed four at a
-    // time, but only where a shape is decoded for long: a graph of four takes 0.15 ms to make there and 0.45 for
-    // eight of Kogilix, width 2048, what 33 and 85 steps gain (16 steps 3.96 -> 3.88 ms, 32 steps 15.43 -> 15.26).
+    // time, but only where a shape is decoded for long, in calls of as many: a graph of four takes 0.15 ms to make there and 0.45 for
+    // eight of Kogilix, width 2048, what 33 and 85 steps gain (calls after 128 steps of the shape: 16 steps 3.96 -> 3.88 ms, 32 steps
+    // 15.43 -> 15.26).
     constexpr int GRAPH_STEPS = 4, GRAPH_LONG = 128;
     constexpr int DECODE_RING = 4096;   // tokens kept on the device between two host reads
 
@@ -92,7 +93,8 @@ namespace
         struct Graph
         {
             hipGraphExec_t exec = nullptr, many = nullptr;
-            int steps = 0; // done, up to GRAPH_LONG
+            int steps = 0;       // done, up to GRAPH_LONG
+            bool single = false; // no graph of several steps could be made
         };
         std::map<std::pair<int, int>, Graph> graphs; // by (sequences, bound on the length)
         hipEvent_t ev[2] = {nullptr, nullptr};
@@ -820,7 +822,11 @@ extern "C" bool llam_seqm_decode(void *model, int n, const int32_t *h_slot, cons
         hipGraph_t graph = nullptr;
         const hipError_t e = hipStreamEndCapture(md->stream, &graph);
         if (!ok || !hip_ok(fn, "hipStreamEndCapture", e))
+        {
+            if (e == hipSuccess && graph)
+                (void)hipGraphDestroy(graph);
             return false;
+        }
         const hipError_t ei = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
         (void)hipGraphDestroy(graph);
         if (ei != hipSuccess)
@@ -836,8 +842,13 @@ extern "C" bool llam_seqm_decode(void *model, int n, const int32_t *h_slot, cons
         if (steps > 1 && !capture(1, g.exec))
             return false;
     }
-    if (!g.many && g.steps >= GRAPH_LONG && !capture(GRAPH_STEPS, g.many))
-        return false;
+    // (only where this call replays it; where it cannot be made, for want of memory say, steps go on one at a time)
+    if (!g.many && !g.single && g.steps >= GRAPH_LONG && steps - done >= GRAPH_STEPS && !capture(GRAPH_STEPS, g.many))
+    {
+        g.single = true;
+        (void)hipGetLastError();
+        g_error[0] = '\0';
+    }
     g.steps = std::min(g.steps + steps, GRAPH_LONG);
     if (!hip_ok(fn, "hipEventRecord", hipEventRecord(md->ev[0], md->stream)))
         return false;

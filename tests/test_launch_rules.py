@@ -221,3 +221,39 @@ answer(log())
     assert calls[-1][0] == "launch" and "moe_group_kernel" in calls[-1][1] and dynamic == 16 * over(experts, 2) * 4
     granted = max([int(c[2]) for c in calls if c[0] == "lds"], default=64 * 1024 - fixed)
     assert dynamic <= granted
+
+
+# ---- graphs of decoding steps (sequence_model.cpp) ----------------------------------------------------------
+
+DECODE = """
+from llaminar_amd import sequence
+from llaminar_amd.models import kogilix
+from tests import sequence_models as sm
+cfg = sm.config(sm.mlstm(mlp=sm.dense()))
+model = sequence.SequenceModel(kogilix.weights(cfg, sm.random_weights(cfg)), 4, 512, 64, "float32")
+log()
+def decode(steps, times=1):
+    for _ in range(times):
+        model.decode([0, 1], [3, 3], [1, 2], steps)
+    calls = log()
+    return [sum(c[0] == what for c in calls) for what in ("instantiate", "replay", "launch")], [int(c[1]) for c in calls if c[0] == "replay"]
+"""
+
+
+def test_a_graph_of_several_steps_is_made_where_it_is_replayed(tmp_path):
+    """128 steps of a shape in calls of one and three: single steps, before and after; then a call of six replays a graph of four."""
+    ones, threes, six = fake_hip.run(tmp_path, DECODE + "answer([decode(1, 130), decode(3, 50), decode(6)])")
+    assert ones[0][:2] == [0, 0] and ones[0][2] % 130 == 0
+    step = ones[0][2] // 130
+    assert threes[0] == [1, 3 * 50 - 1, step] and set(threes[1]) == {step}
+    assert six[0] == [1, 3, 0] and six[1] == [4 * step, step, step]
+
+
+def test_decoding_goes_on_where_a_graph_of_several_steps_cannot_be_made(tmp_path):
+    long, after, error = fake_hip.run(tmp_path, DECODE + """
+first = decode(2)
+fake.fake_hip_largest_graph(2 * first[1][0])
+answer([decode(8, 16), decode(8, 3), model._error()])
+""")
+    assert long[0] == [0, 8 * 16, 0] and after[0] == [0, 8 * 3, 0] and len(set(long[1] + after[1])) == 1
+    assert error == ""
