@@ -262,11 +262,6 @@ size_t llam_seq_experts_scratch_bytes(int max_rows, int experts, int top, int ff
 bool llam_seq_experts(const llam_seq_experts_args *a, int M, void *d_scratch, size_t scratch_bytes, int dtype,
                       int device_id, void *stream);
 
-/* d_out[*d_count * n + b] = d_ids[b], then *d_count += 1: the tokens of replayed decode steps in
- * order; nothing is written once *d_count has reached max_count. */
-bool llam_seq_record(const int32_t *d_ids, int n, int32_t *d_out, int32_t *d_count, int max_count, int device_id,
-                     void *stream);
-
 #ifdef __cplusplus
 }
 #endif

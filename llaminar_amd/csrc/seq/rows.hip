@@ -123,19 +123,6 @@ namespace llamql
             }
     }
 
-    __global__ void __launch_bounds__(64)
-        seq_record_kernel(const int32_t *__restrict__ ids, int n, int32_t *__restrict__ out, int32_t *__restrict__ count,
-                          int max_count)
-    {
-        const int k = *count;
-        if (k >= max_count)
-            return;
-        for (int b = threadIdx.x; b < n; b += 64)
-            out[(size_t)k * n + b] = ids[b];
-        if (threadIdx.x == 0)
-            *count = k + 1;
-    }
-
     // ---- routed experts -------------------------------------------------------------------------
     struct ExpertArgs
     {
@@ -657,16 +644,4 @@ extern "C" bool llam_seq_experts(const llam_seq_experts_args *a, int M, void *d_
     p.h = a->d_h, p.x = a->d_x, p.ldx = a->ldx;
     return dtype == LLAM_SEQ_F32 ? experts_run<float>(fn, p, M, static_cast<char *>(d_scratch), dtype, device_id, as_stream(stream))
                                  : experts_run<bf16>(fn, p, M, static_cast<char *>(d_scratch), dtype, device_id, as_stream(stream));
-}
-
-extern "C" bool llam_seq_record(const int32_t *d_ids, int n, int32_t *d_out, int32_t *d_count, int max_count,
-                                int device_id, void *stream)
-{
-    static const char *fn = "llam_seq_record";
-    if (n < 1 || max_count < 0 || !d_ids || !d_out || !d_count)
-        return fail(fn, "bad arguments");
-    if (!set_device(fn, device_id))
-        return false;
-    hipLaunchKernelGGL(seq_record_kernel, dim3(1), dim3(64), 0, as_stream(stream), d_ids, n, d_out, d_count, max_count);
-    return launched(fn);
 }

@@ -136,7 +136,6 @@ SIGNATURES = {
                                               c_int, c_int, c_void_p]),
     "llam_seq_experts_scratch_bytes": (c_size_t, [c_int, c_int, c_int, c_int, c_int, c_int]),
     "llam_seq_experts": (c_bool, [POINTER(ExpertsArgs), c_int, c_void_p, c_size_t, c_int, c_int, c_void_p]),
-    "llam_seq_record": (c_bool, [c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_void_p]),
     "llam_seqm_create": (c_void_p, [POINTER(Config)]),
     "llam_seqm_destroy": (None, [c_void_p]),
     "llam_seqm_upload": (c_void_p, [c_void_p, c_void_p, c_size_t]),
