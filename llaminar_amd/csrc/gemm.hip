@@ -440,8 +440,9 @@ namespace llamql
     // Against a subtraction, a multiply-add and scales on the 32-bit matrix unit, weights straight into registers: 199 x 5120 x 25600
     // Q6_K 206 -> 143 us (tiles of 96 x 64; of 128 x 64 that walk is 182), 40 x 8192 x 5120 IQ3_S 21.8 -> 18.2, 512 x 25600 x 5120
     // Q4_K 270 -> 227 (gemm_kernel before; two launches now), 256 x 25600 x 5120 Q4_K 140 -> 137, 130 x 5000 x 5120 Q4_K 26.5 -> 23.5, 63 x 5034 x 18944 Q6_K 71 -> 62.
-    // Errors against 64 bits: 0.4 to 1.0 times those before (199 x 5120 x 25600 Q6_K 2.57e-7 -> 1.91e-7, 512 x 25600 x 5120 Q4_K 3.20e-7 ->
-    // 1.55e-7, 40 x 8192 x 5120 IQ3_S 9.9e-8 -> 9.8e-8), at worst 1.03 (326 x 2709 x 24832 IQ3_S 1.86e-7 -> 1.91e-7).
+    // Errors against 64 bits: 0.4 to 1.0 times those before (199 x 5120 x 25600 Q6_K 2.57e-7 -> 2.04e-7, 512 x 25600 x 5120 Q4_K 3.20e-7 ->
+    // 1.55e-7, 40 x 8192 x 5120 IQ3_S 9.9e-8 -> 9.8e-8); 1.05 to 1.09 for the one size in 2000 that eight sums of block after block were
+    // before and 96 x 64 is now (326 x 2709 x 24832 IQ3_S 1.86e-7 -> 2.03e-7, 145 -> 124 us).
     template <int MT, int RN, int KS>
     struct GemmSplit
     {
@@ -638,8 +639,9 @@ namespace llamql
                 // Sums of a job's two blocks that are added up by themselves (see rescale): with those of the job before, of the job after
                 auto with_before = [](int j) { return APART && (FOURS ? j & 1 : j == MT); };
                 auto with_after = [](int j) { return APART && (FOURS ? !(j & 1) : j == MT - 1); };
-                // (of tiles of 96 and 128 tokens as many as keep the walk as exact as block after block in twice as many sums)
-                constexpr int APARTS = FOURS ? JOBS : KW == 2 ? (F::HAS_MIN ? MT + 2 : JOBS) : F::HAS_MIN ? MT + 1 : MT + 2;
+                // (of 128 x 128 as many as keep two sums as exact as four of block after block; of 96 x 64, which has four, those that cost
+                // no addition more: with one more pair 199 x 5120 x 25600 Q6_K is 1.91e-7 instead of 2.04e-7 away, and 2 % slower)
+                constexpr int APARTS = FOURS ? JOBS : KW == 2 ? (F::HAS_MIN ? MT + 2 : JOBS) : MT + 1;
                 auto is_apart = [](int j) { return APART ? j < APARTS : MT == 4 && j >= MT; };
                 auto fence = []() __attribute__((always_inline)) {
                     if (MT > 1) // (two products of a step are not enough for it: the compiler's order is 10 % faster)
@@ -686,7 +688,7 @@ namespace llamql
                 // among them, before they meet the sum of those before: 1 or 2 roundings at the size of the whole sum instead of 4, or 6
                 // with minima.  Two partial sums are then no coarser than four of block after block: 232 x 16587 x 13312 Q6_K
                 // 1.83e-7 from 64 bits (1.88e-7 by four such sums, 2.28e-7 with two blocks of four apart), Q4_K 2.42e-7 (2.58e-7, 3.38e-7),
-                // at an addition to four or eight multiply-adds (1 to 3 % of 128 x 128 and 96 x 64).  Eight partial sums need it not,
+                // at an addition to four or eight multiply-adds (1 to 3 % of 128 x 128).  Eight partial sums need it not,
                 // 128 x 64 has registers for the second pairs only, and one token tile's with minima stay as they were (17 x 8370 x
                 // 18944 Q4_K 51.1 us and 2.95e-7, or 53.7 and 1.26e-7).
                 v16f apart;

@@ -416,16 +416,11 @@ namespace llamql
         }
     }
 
-    // ---- Q4_K ------------------------------------------------------------------------
-    // Super-block = 144 bytes: header piece {d, dmin, scales[12]} and four 32-byte groups;
-    // group l holds blocks 2l (low nibbles) and 2l+1 (high nibbles), element e in byte e
-    // (Q4_KTensor.cpp:768-792).  Effective scale f16(d*sc), min f16(-dmin*m) with the
-    // packer's fp16 rounding (Q4_KTensor.cpp:794-799, FP16Utils.h:75-118).
     // 32 rows of one half of a super-block, raw, by way of LDS: what the quad lanes 2 half and 2 half + 1 of every row decode.
     // A load of 16 bytes a lane reads a row's piece of a plane with neighbouring lanes (four cover 64 bytes), where a lane that
     // loads for itself meets a cache line of its own: 16 or 32 instead of 64 cycles of the address unit.  A piece lies in LDS where
     // eight lanes that read eight neighbouring rows meet no bank twice.
-    // PIECES: 16-byte pieces of a row; AT: the place of the first of them
+    // PIECES: 16-byte pieces of a row
     template <int PIECES>
     struct HalfRows
     {
@@ -465,6 +460,11 @@ namespace llamql
         }
     };
 
+    // ---- Q4_K ------------------------------------------------------------------------
+    // Super-block = 144 bytes: header piece {d, dmin, scales[12]} and four 32-byte groups;
+    // group l holds blocks 2l (low nibbles) and 2l+1 (high nibbles), element e in byte e
+    // (Q4_KTensor.cpp:768-792).  Effective scale f16(d*sc), min f16(-dmin*m) with the
+    // packer's fp16 rounding (Q4_KTensor.cpp:794-799, FP16Utils.h:75-118).
     struct Q4KQuad
     {
         static constexpr int SB_BYTES = 144;
