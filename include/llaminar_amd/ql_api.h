@@ -291,8 +291,8 @@ bool llam_ql_gemv_describe(uint8_t fmt, int M, int N, int K, int has_plane, int 
  * counterpart of launch_native_vnni_gemm
  * (src/v2/kernels/rocm/gemm/ROCmQuantisedGemmKernel_native_VNNI.hip:2580-2632).
  * Two kernels, chosen by their expected times: token tiles of 32 (M <= 32), 64 (M <= 64) or
- * 128 tokens whose walk along K one workgroup keeps, and, where those would leave the chip
- * partly idle, tiles of 32 or 64 tokens whose walk is dealt to 2, 4 or 8 wavefronts.  The
+ * 128 tokens whose walk along K one workgroup keeps, and tiles of 32 to 128 tokens whose walk
+ * is dealt to 2, 4 or 8 wavefronts; a call is one launch, or two that share the weight rows.  The
  * fp32 sum of a row's blocks is formed in an order that depends on the kernel and the tile,
  * so a row's last bits may differ between calls of different M or N (the per-block int32
  * sums never do).  The same call always gives the same bits. */
@@ -301,7 +301,7 @@ bool llam_ql_gemm(uint8_t fmt, const void *d_w, const void *d_q8, float *d_y,
 
 /* Parity hook of the GEMM: the matrix unit's exact per-block int32 sums of weight rows
  * [row0, row0+nrows) for all M activation rows, d_sums[(m*nrows + r)*(K/32) + kb], from
- * the block-sum variant of the kernel that llam_ql_gemm runs for (M, N, K): same tiles, same
+ * the block-sum variants of the launches that llam_ql_gemm makes for (M, N, K): same tiles, same
  * decode, same MFMA.
  * Counterpart of the reference's int32 accumulators in gemm_2row_native_chunk /
  * gemm_2row_int8_chunk (CPUNativeVNNIGemv.h:1046-1376). */

@@ -438,8 +438,10 @@ namespace llamql
     // two).  The older wavefront of the two is served first and waited at the barrier for a third of the step, so decoding goes
     // ahead of rescaling, and the younger's rescaling ahead of the older's.  One workgroup of eight wavefronts fits a compute unit.
     // Against a subtraction, a multiply-add and scales on the 32-bit matrix unit, weights straight into registers: 199 x 5120 x 25600
-    // Q6_K 206 -> 143 us (tiles of 96 x 64; of 128 x 64 that walk is 182), 40 x 8192 x 5120 IQ3_S 21.8 -> 18.2, 512 x 25600 x 5120
-    // Q4_K 270 -> 227 (gemm_kernel before; two launches now), 256 x 25600 x 5120 Q4_K 140 -> 137, 130 x 5000 x 5120 Q4_K 26.5 -> 23.5, 63 x 5034 x 18944 Q6_K 71 -> 62.
+    // Q6_K 206 -> 136 to 146 us by card (tiles of 96 x 64; of 128 x 64 that walk is 194), 40 x 8192 x 5120 IQ3_S 20.0 -> 17.3, 512 x 25600 x 5120
+    // Q4_K 270 -> 229 to 236 (gemm_kernel before; two launches now), 256 x 25600 x 5120 Q4_K 139 -> 132, 130 x 5000 x 5120 Q4_K 24.9 -> 22.5,
+    // 63 x 5034 x 18944 Q6_K 71 -> 62 to 67.  Counters of 512 x 25600 x 5120: 242 cycles of a SIMD unit a product, the vector unit issues in 0.9
+    // of them and the matrix unit works in 0.23.
     // Errors against 64 bits: 0.4 to 1.0 times those before (199 x 5120 x 25600 Q6_K 2.57e-7 -> 2.04e-7, 512 x 25600 x 5120 Q4_K 3.20e-7 ->
     // 1.55e-7, 40 x 8192 x 5120 IQ3_S 9.9e-8 -> 9.8e-8); 1.05 to 1.09 for the one size in 2000 that eight sums of block after block were
     // before and 96 x 64 is now (326 x 2709 x 24832 IQ3_S 1.86e-7 -> 2.03e-7, 145 -> 124 us).
