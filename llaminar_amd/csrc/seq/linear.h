@@ -44,6 +44,17 @@ namespace llamql
     // pieces add up to nothing.  (Looking out for it costs 8 to 10 % of a prompt's layer: 2048 x 51200 x 5120 2480 -> 2670 us.)
     __device__ __forceinline__ bool pieces_fail(float sum) { return !(fabsf(sum) >= 0x1p-80f) && sum != 0.0f; }
 
+    __device__ __forceinline__ f32x4 relu2(f32x4 v)
+    {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+        {
+            const float z = fmaxf(v[r], 0.0f);
+            v[r] = z * z;
+        }
+        return v;
+    }
+
     // LLAM_SEQ_OUT_*: four neighbouring output columns of one row
     template <typename T>
     __device__ __forceinline__ void store4(const LinearArgs &p, char *ybase, int row, int col, f32x4 v)
@@ -68,13 +79,7 @@ namespace llamql
             break;
         }
         case LLAM_SEQ_OUT_RELU2:
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-            {
-                const float z = fmaxf(v[r], 0.0f);
-                v[r] = z * z;
-            }
-            *reinterpret_cast<t4 *>(reinterpret_cast<T *>(ybase) + at) = __builtin_convertvector(v, t4);
+            *reinterpret_cast<t4 *>(reinterpret_cast<T *>(ybase) + at) = __builtin_convertvector(relu2(v), t4);
             break;
         default:
             *reinterpret_cast<t4 *>(reinterpret_cast<T *>(ybase) + at) = __builtin_convertvector(v, t4);

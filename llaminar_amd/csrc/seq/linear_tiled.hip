@@ -2,7 +2,7 @@
 //
 // Both operands go from global memory straight into LDS, some turns of 64 columns ahead, and from there into registers
 // one sixteen-column step ahead of the products, across the one barrier of a turn.  W is the first operand, so a lane
-// ends with four neighbouring output columns of one row.  32-bit rows are multiplied in three bf16 pieces that add up to
+// ends with four neighbouring output columns of one row; results go through LDS so that they leave by whole lines.  32-bit rows are multiplied in three bf16 pieces that add up to
 // them (weights are bf16 anyway): the products stay exact, the sums 32-bit, on a unit that is 16 times as fast.
 //
 // What bounds it, 2048 x 15440 x 5120 in bf16: the matrix unit is busy in 57 % of the cycles, at the 1.9 GHz that the chip
@@ -11,6 +11,8 @@
 // 5120 1200 -> 940 us, 300 x 2048 x 8192 63 -> 28 us; 32-bit rows (v_mfma_f32_16x16x4 before) 2048 x 51200 x 5120 9490 ->
 // 2480 us, 522 x 2048 x 10240 380 -> 126 us.
 #include "linear.h"
+
+#include <type_traits>
 
 namespace llamql
 {
@@ -60,6 +62,33 @@ namespace llamql
 #pragma unroll
         for (int i = 0; i < 3; ++i)
             out[i] = __builtin_bit_cast(bf16x8, p[i]);
+    }
+
+    constexpr int OUT_BYTES = 4096; // 32 x 32 results
+    // 16 bytes of results into a row of y (whole: rows of 16-bit values start at 16 bytes, else at 8)
+    __device__ __forceinline__ void store_piece(const LinearArgs &p, char *y, bool, int row, int col, f32x4 v)
+    {
+        f32x4 *at = reinterpret_cast<f32x4 *>(reinterpret_cast<float *>(y) + (size_t)row * p.ldy + col);
+        if (p.out == LLAM_SEQ_OUT_F32 && p.bias)
+        {
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                v[r] += p.bias[col + r];
+        }
+        if (p.out == LLAM_SEQ_OUT_ADD)
+            v = *at + v;
+        *at = v;
+    }
+    __device__ __forceinline__ void store_piece(const LinearArgs &p, char *y, bool whole, int row, int col, bf16x8 v)
+    {
+        bf16 *at = reinterpret_cast<bf16 *>(y) + (size_t)row * p.ldy + col;
+        if (whole)
+            *reinterpret_cast<bf16x8 *>(at) = v;
+        else
+        {
+            reinterpret_cast<bf16x4 *>(at)[0] = __builtin_shufflevector(v, v, 0, 1, 2, 3);
+            reinterpret_cast<bf16x4 *>(at)[1] = __builtin_shufflevector(v, v, 4, 5, 6, 7);
+        }
     }
 
     template <typename T>
@@ -406,38 +435,63 @@ namespace llamql
             }
         }
 
+        // Results by way of LDS, where a wavefront lays 32 rows of its own columns and takes them up again by whole rows: straight
+        // from the accumulators a store instruction of 64 lanes touches 32 rows, 8 or 16 bytes a lane, and loads of other workgroups
+        // wait behind that (bf16, straight and by way of LDS: 2048 x 16384 x 2048 165 -> 112 us, 2048 x 16384 x 8192 503 -> 426).
         const size_t elem = p.out == LLAM_SEQ_OUT_F32 || p.out == LLAM_SEQ_OUT_ADD ? 4 : sizeof(T);
         char *y = static_cast<char *>(p.y) + (p.group_offset ? 0 : (size_t)z * p.y_stride * elem);
+        if constexpr (KG == 1)
+            arrive<0>(); // all wavefronts are done with the stages (of several groups, the place of the wavefront's own sums)
+        char *own = smem + wave * (KG == 1 ? TN * OUT_BYTES : TN * TM * 4096);
+        auto out = [&](auto gated, auto value) __attribute__((always_inline)) {
+            typedef decltype(value) V;
+            constexpr bool GATED = decltype(gated)::value;
+            constexpr int COLS = GATED ? TN * 16 : TN * 32, PITCH = COLS * sizeof(V);
+            constexpr int EACH = 16 / sizeof(V), PIECES = COLS / EACH; // values of a 16-byte piece, pieces of a row
+            typedef V four_t __attribute__((ext_vector_type(4)));
+            typedef V piece_t __attribute__((ext_vector_type(EACH)));
+            // piece x of row r lies at x ^ spread(r)
+            auto spread = [](int r) __attribute__((always_inline)) { return r / (PIECES < 8 ? 8 / PIECES : 1) & (PIECES - 1); };
+            const int n0 = (nt * BN + wn * TN * 32) / (GATED ? 2 : 1), columns = GATED ? p.N / 2 : p.N;
+            const bool whole = ((p.ldy | p.y_stride) & (EACH - 1)) == 0; // (rows of 16-bit values may start at 8 bytes)
 #pragma unroll
-        for (int i = 0; i < TM; ++i)
-        {
-            const int m = mt * BM + (wm * TM + i) * 32 + c;
-            if (m >= rows)
-                continue;
-#pragma unroll
-            for (int j = 0; j < TN; ++j)
+            for (int i = 0; i < TM; ++i)
             {
-                const int n0 = nt * BN + (wn * TN + j) * 32;
-                auto four = [&](int q) __attribute__((always_inline)) {
-                    return f32x4{acc[j][i][4 * q], acc[j][i][4 * q + 1], acc[j][i][4 * q + 2], acc[j][i][4 * q + 3]};
-                };
-                if (is_gated(p.out))
-                {
-                    // rows 0 .. 15 of the product are gates, 16 .. 31 the same of up
 #pragma unroll
-                    for (int q = 0; q < 2; ++q)
-                        if (n0 < p.N)
-                            store4<T>(p, y, row0 + m, n0 / 2 + 8 * q + 4 * h, gated4(p, four(q), four(q + 2)));
-                }
-                else
-                {
+                for (int j = 0; j < TN; ++j)
 #pragma unroll
-                    for (int q = 0; q < 4; ++q)
-                        if (n0 + 8 * q < p.N)
-                            store4<T>(p, y, row0 + m, n0 + 8 * q + 4 * h, four(q));
+                    for (int q = 0; q < (GATED ? 2 : 4); ++q)
+                    {
+                        auto four = [&](int q) __attribute__((always_inline)) {
+                            return f32x4{acc[j][i][4 * q], acc[j][i][4 * q + 1], acc[j][i][4 * q + 2], acc[j][i][4 * q + 3]};
+                        };
+                        f32x4 v = four(q);
+                        if constexpr (GATED) // rows 0 .. 15 of the product are gates, 16 .. 31 the same of up
+                            v = gated4(p, v, four(q + 2));
+                        else if (sizeof(V) == sizeof(T) && p.out == LLAM_SEQ_OUT_RELU2)
+                            v = relu2(v);
+                        const int col = j * (GATED ? 16 : 32) + 8 * q + 4 * h;
+                        *reinterpret_cast<four_t *>(own + c * PITCH + (col / EACH ^ spread(c)) * 16 + col % EACH * sizeof(V)) = __builtin_convertvector(v, four_t);
+                    }
+                asm volatile("" ::: "memory"); // (a wavefront's LDS instructions run in order)
+#pragma unroll
+                for (int k = 0; k < PIECES / 2; ++k)
+                {
+                    const int r = (k * 64 + lane) / PIECES, x = (k * 64 + lane) % PIECES, col = n0 + x * EACH;
+                    const int m = mt * BM + (wm * TM + i) * 32 + r;
+                    piece_t v = *reinterpret_cast<const piece_t *>(own + r * PITCH + (x ^ spread(r)) * 16);
+                    if (m < rows && col < columns)
+                        store_piece(p, y, whole, row0 + m, col, v);
                 }
+                asm volatile("" ::: "memory");
             }
-        }
+        };
+        if (is_gated(p.out))
+            out(std::true_type(), T());
+        else if (elem == sizeof(T))
+            out(std::false_type(), T());
+        else
+            out(std::false_type(), float());
     }
 
     namespace
@@ -447,6 +501,7 @@ namespace llamql
         {
             static LdsGrant grant;
             constexpr size_t stages = (size_t)STAGES * KG * (BM * sizeof(T) + BN * 2) * TILE_K, sums = (size_t)(KG - 1) * BM * BN * 4;
+            static_assert(KG > 1 || stages >= (size_t)WM * BN * OUT_BYTES / 32, "the results' place");
             constexpr size_t lds = stages > sums ? stages : sums;
             static_assert(lds <= 160 * 1024, "stages must fit the LDS");
             const auto kernel = &linear_wide_kernel<T, BM, BN, WM, WN, KG, STAGES>;

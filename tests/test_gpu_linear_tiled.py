@@ -168,3 +168,20 @@ def test_small_values_of_32_bit_rows(dev, M, N, K):
     # (a sum that the pieces make zero is taken at its word: of each value less than 2^-133 may be missing)
     bound[y == 0.0] = K * 2.0 ** -133 * float(w.abs().max())
     assert ((y.double() - want).abs() <= bound).all() and (y != 0.0).double().mean() > 0.99
+
+
+@pytest.mark.parametrize("out", [sq.OUT_ELEM, sq.OUT_GATED, sq.OUT_RELU2])
+@pytest.mark.parametrize("M,N,K", SHAPES[:6] + [(300, 2080, 128), (2000, 3104, 64), (520, 2080, 2112)])
+def test_rows_that_start_at_eight_bytes(dev, M, N, K, out):
+    """bf16 results whose rows lie 8 bytes off 16: the same values as of aligned rows, and nothing past them."""
+    import torch
+
+    N = max(32, N // 32 * 32) if out == sq.OUT_GATED else N
+    columns = N // 2 if out == sq.OUT_GATED else N
+    torch.manual_seed(M)
+    a, t = torch.randn(M, K, device=dev).bfloat16(), tiles((torch.randn(N, K, device=dev) * K ** -0.5).bfloat16())
+    aligned, y = torch.full((M, columns + 8), 5.0, device=dev).bfloat16(), torch.full((M + 1, columns + 4), 5.0, device=dev).bfloat16()
+    run(torch, a, t, aligned[:, :columns], BF16, out, N, K)
+    run(torch, a, t, y[:M, :columns], BF16, out, N, K)
+    assert torch.equal(y[:M, :columns], aligned[:, :columns])
+    assert (y[M:] == 5.0).all() and (y[:, columns:] == 5.0).all() and (aligned[:, columns:] == 5.0).all()
