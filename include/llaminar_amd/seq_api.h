@@ -65,6 +65,13 @@ typedef struct
 } llam_seq_linear_args;
 bool llam_seq_linear(const llam_seq_linear_args *a, int dtype, int device_id, void *stream);
 
+/* The same with scratch for partial sums: a layer of many rows whose output would leave most of the chip idle is
+ * cut along K as well, as far as d_scratch (16-byte aligned, may be null) reaches.  Sums are associated otherwise than
+ * without it; they are the same on every call.  llam_seq_linear_scratch_bytes: what a layer of up to max_rows rows makes use of. */
+size_t llam_seq_linear_scratch_bytes(int max_rows, int N, int K, int dtype, int device_id);
+bool llam_seq_linear_within(const llam_seq_linear_args *a, void *d_scratch, size_t scratch_bytes, int dtype, int device_id,
+                            void *stream);
+
 /* Two linear layers over the same M rows with the same K and nothing in common otherwise (the two
  * branches of a parallel layer), unbatched: up to 16 rows in one launch.  Both have d_norm or none has. */
 bool llam_seq_linear_pair(const llam_seq_linear_args *a, const llam_seq_linear_args *b, int dtype, int device_id,

@@ -27,6 +27,9 @@ namespace llamql
         const int *row_source;
         int source_div;
         int groups, group_rows; // groups, and rows of all of them
+        // many rows: tiles from `full` on are cut into slices of K, their sums in `parts` (linear_tiled)
+        f32x4 *parts;
+        int full, slices;
     };
 
     constexpr int SMALL_M = 16;         // most rows of the row-at-a-time kernel: one operand of the matrix unit
@@ -34,7 +37,10 @@ namespace llamql
 
     __host__ __device__ inline bool is_gated(int out) { return out == LLAM_SEQ_OUT_GATED || out == LLAM_SEQ_OUT_GATED_CLAMP; }
     bool linear_small(const char *fn, const LinearArgs &a, int batch, int dtype, int device_id, hipStream_t st);
-    bool linear_tiled(const char *fn, const LinearArgs &a, int batch, int dtype, int device_id, hipStream_t st);
+    // scratch: for sums of tiles cut along K, as far as it reaches; what linear_split_bytes says serves layers of up to max_rows rows
+    bool linear_tiled(const char *fn, const LinearArgs &a, int batch, int dtype, int device_id, hipStream_t st, void *scratch = nullptr,
+                      size_t bytes = 0);
+    size_t linear_split_bytes(int max_rows, int N, int K, int dtype, int device_id);
 
     // Whether a sum of products in three bf16 pieces of each 32-bit value may not be that of the whole values, which then
     // are multiplied once more without pieces: the second and third piece of most values are zero, and zero times an infinite

@@ -457,18 +457,32 @@ namespace
     }
 } // namespace
 
-extern "C" bool llam_seq_linear(const llam_seq_linear_args *a, int dtype, int device_id, void *stream)
+extern "C" size_t llam_seq_linear_scratch_bytes(int max_rows, int N, int K, int dtype, int device_id)
+{
+    if (max_rows <= SMALL_M || N < 1 || K < 1 || K % PAD != 0 || (dtype != LLAM_SEQ_BF16 && dtype != LLAM_SEQ_F32))
+        return 0;
+    return linear_split_bytes(max_rows, N, K, dtype, device_id);
+}
+
+extern "C" bool llam_seq_linear_within(const llam_seq_linear_args *a, void *d_scratch, size_t scratch_bytes, int dtype, int device_id, void *stream)
 {
     static const char *fn = "llam_seq_linear";
     LinearArgs p;
     if (!linear_args(fn, a, dtype, p))
         return false;
+    if (d_scratch && !aligned16(d_scratch))
+        return fail(fn, "misaligned scratch");
     if (a->M == 0)
         return true;
     if (!set_device(fn, device_id))
         return false;
     return a->M <= SMALL_M ? linear_small(fn, p, a->batch, dtype, device_id, as_stream(stream))
-                           : linear_tiled(fn, p, a->batch, dtype, device_id, as_stream(stream));
+                           : linear_tiled(fn, p, a->batch, dtype, device_id, as_stream(stream), d_scratch, scratch_bytes);
+}
+
+extern "C" bool llam_seq_linear(const llam_seq_linear_args *a, int dtype, int device_id, void *stream)
+{
+    return llam_seq_linear_within(a, nullptr, 0, dtype, device_id, stream);
 }
 
 extern "C" bool llam_seq_linear_pair(const llam_seq_linear_args *a, const llam_seq_linear_args *b, int dtype, int device_id, void *stream)

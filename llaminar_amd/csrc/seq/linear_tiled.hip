@@ -91,6 +91,62 @@ namespace llamql
         }
     }
 
+    // 32 rows from m0 on of TN x 32 products, a lane's as the matrix unit leaves them, to rows row0 + m of y.  By way of LDS, where the
+    // wavefront lays them (own) and takes them up again by whole rows: straight from the accumulators a store instruction of 64 lanes
+    // touches 32 rows, 8 or 16 bytes a lane, and loads of other workgroups wait behind that (bf16, straight and by way of LDS:
+    // 2048 x 16384 x 2048 165 -> 112 us, 2048 x 16384 x 8192 503 -> 426).
+    template <typename T, int TN>
+    __device__ __forceinline__ void results(const LinearArgs &p, int z, const f32x16 (&strip)[TN], char *own, int lane, int m0, int rows, int row0, int n0)
+    {
+        const int c = lane & 31, h = lane >> 5;
+        const size_t elem = p.out == LLAM_SEQ_OUT_F32 || p.out == LLAM_SEQ_OUT_ADD ? 4 : sizeof(T);
+        char *y = static_cast<char *>(p.y) + (size_t)z * p.y_stride * elem;
+        auto out = [&](auto gated, auto value) __attribute__((always_inline)) {
+            typedef decltype(value) V;
+            constexpr bool GATED = decltype(gated)::value;
+            constexpr int COLS = GATED ? TN * 16 : TN * 32, PITCH = COLS * sizeof(V);
+            constexpr int EACH = 16 / sizeof(V), PIECES = COLS / EACH; // values of a 16-byte piece, pieces of a row
+            typedef V four_t __attribute__((ext_vector_type(4)));
+            typedef V piece_t __attribute__((ext_vector_type(EACH)));
+            // piece x of row r lies at x ^ spread(r)
+            auto spread = [](int r) __attribute__((always_inline)) { return r / (PIECES < 8 ? 8 / PIECES : 1) & (PIECES - 1); };
+            const int first = GATED ? n0 / 2 : n0, columns = GATED ? p.N / 2 : p.N;
+            const bool whole = ((p.ldy | p.y_stride) & (EACH - 1)) == 0; // (rows of 16-bit values may start at 8 bytes)
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int q = 0; q < (GATED ? 2 : 4); ++q)
+                {
+                    auto four = [&](int q) __attribute__((always_inline)) {
+                        return f32x4{strip[j][4 * q], strip[j][4 * q + 1], strip[j][4 * q + 2], strip[j][4 * q + 3]};
+                    };
+                    f32x4 v = four(q);
+                    if constexpr (GATED) // rows 0 .. 15 of the product are gates, 16 .. 31 the same of up
+                        v = gated4(p, v, four(q + 2));
+                    else if (sizeof(V) == sizeof(T) && p.out == LLAM_SEQ_OUT_RELU2)
+                        v = relu2(v);
+                    const int col = j * (GATED ? 16 : 32) + 8 * q + 4 * h;
+                    *reinterpret_cast<four_t *>(own + c * PITCH + (col / EACH ^ spread(c)) * 16 + col % EACH * sizeof(V)) = __builtin_convertvector(v, four_t);
+                }
+            asm volatile("" ::: "memory"); // (a wavefront's LDS instructions run in order)
+#pragma unroll
+            for (int k = 0; k < PIECES / 2; ++k)
+            {
+                const int r = (k * 64 + lane) / PIECES, x = (k * 64 + lane) % PIECES, col = first + x * EACH;
+                const piece_t v = *reinterpret_cast<const piece_t *>(own + r * PITCH + (x ^ spread(r)) * 16);
+                if (m0 + r < rows && col < columns)
+                    store_piece(p, y, whole, row0 + m0 + r, col, v);
+            }
+            asm volatile("" ::: "memory");
+        };
+        if (is_gated(p.out))
+            out(std::true_type(), T());
+        else if (elem == sizeof(T))
+            out(std::false_type(), T());
+        else
+            out(std::false_type(), float());
+    }
+
     template <typename T>
     struct TiledOperand;
     template <>
@@ -108,9 +164,25 @@ namespace llamql
         static __device__ __forceinline__ void pieces(Raw x, bf16x8 (&out)[3]) { three_pieces(x, out); }
     };
 
+    // Neighbouring tiles go to one die (blocks are dealt round robin over the eight dies), eight tiles of rows side
+    // by side, then the next tile of W: what a die works on at a time is about square.
+    __device__ __forceinline__ int die_order(int id, int count)
+    {
+        const int per = count / 8;
+        return id < per * 8 ? (id & 7) * per + (id >> 3) : id;
+    }
+    __device__ __forceinline__ void tile_place(int id, int m_tiles, int n_tiles, int &mt, int &nt)
+    {
+        const int band = id / (8 * n_tiles), in = id - band * 8 * n_tiles;
+        const int high = m_tiles - band * 8 < 8 ? m_tiles - band * 8 : 8;
+        nt = in / high;
+        mt = band * 8 + in - nt * high;
+    }
+
     // Workgroup tile BM rows of A x BN rows of W; KG groups of WM x WN wavefronts, each with every KG-th turn of 64
-    // columns, STAGES turns of LDS.
-    template <typename T, int BM, int BN, int WM, int WN, int KG, int STAGES>
+    // columns, STAGES turns of LDS.  SPLIT: the tiles from p.full on have p.slices workgroups each, every one with a slice of K,
+    // which leave their accumulators in p.parts for linear_join_kernel.
+    template <typename T, int BM, int BN, int WM, int WN, int KG, int STAGES, bool SPLIT>
     __global__ void __launch_bounds__(WM *WN *KG * 64)
         linear_wide_kernel(LinearArgs p, int m_tiles, int n_tiles)
     {
@@ -156,19 +228,16 @@ namespace llamql
             }
             m_tiles = __builtin_amdgcn_readfirstlane(live);
         }
-        // neighbouring tiles go to one die (blocks are dealt round robin over the eight dies), eight tiles of rows side
-        // by side, then the next tile of W: what a die works on at a time is about square
         const int total = m_tiles * n_tiles;
-        int id = blockIdx.x;
-        if (id >= total)
+        if ((int)blockIdx.x >= (SPLIT ? p.full + (total - p.full) * p.slices : total))
             return;
-        const int per = total / 8;
-        if (id < per * 8)
-            id = (id & 7) * per + (id >> 3);
-        const int band = id / (8 * n_tiles), in = id - band * 8 * n_tiles;
-        const int high = m_tiles - band * 8 < 8 ? m_tiles - band * 8 : 8;
-        const int nt = in / high;
-        int mt = band * 8 + in - nt * high;
+        // (split: behind the whole tiles the first slices of the others, then their second ones, ..: what is at work at a time
+        // reads the same columns)
+        const bool whole = !SPLIT || (int)blockIdx.x < p.full;
+        const int slice = whole ? 0 : ((int)blockIdx.x - p.full) / (total - p.full);
+        const int part = whole ? blockIdx.x : blockIdx.x - p.full - slice * (total - p.full); // of the whole tiles or of the others
+        int mt, nt;
+        tile_place(whole ? die_order(part, SPLIT ? p.full : total) : p.full + die_order(part, total - p.full), m_tiles, n_tiles, mt, nt);
         int z = blockIdx.y, row0 = 0, rows = p.M;
         if (p.group_offset)
         {
@@ -200,8 +269,9 @@ namespace llamql
         const T *abase = static_cast<const T *>(p.a) + (size_t)z * p.a_stride;
         const char *wbase = reinterpret_cast<const char *>(static_cast<const bf16 *>(p.w) + (size_t)z * p.w_stride);
         const int ksteps = p.K >> 5, w_tiles = p.N >> 4, turns = p.K / TILE_K;
-        const int rounds = (turns + KG - 1) / KG; // the group's turn k is columns 64 (k KG + kg) .. of K
-        const int first = kg < turns ? kg : turns - 1;
+        const int turn0 = whole ? 0 : slice * turns / p.slices, count = (whole ? turns : (slice + 1) * turns / p.slices) - turn0; // of K
+        const int rounds = (count + KG - 1) / KG; // the group's turn k is columns 64 (turn0 + k KG + kg) .. of K
+        const int first = turn0 + (kg < count ? kg : count - 1);
 
         // Where the wavefront's loads come from: load i of A fills rows AROWS (wave + i NW) .. of the stage, a lane
         // one 16-byte piece.  Pieces of a row are permuted so that one piece of 16 rows lies in 16 different banks:
@@ -231,7 +301,7 @@ namespace llamql
         auto issue = [&](int i, int buf, int t) __attribute__((always_inline)) {
             const uint32_t at = lds0 + (buf * KG + kg) * STAGE + wave * 1024;
             load_to_lds(src[i], at + (i < ALOADS ? i * NW * 1024 : ABYTES + (i - ALOADS) * NW * 1024));
-            if (KG == 1 || (t + 1) * KG + kg < turns)
+            if (KG == 1 || (t + 1) * KG + kg < count)
                 src[i] += KG * (i < ALOADS ? AROW : 2048);
         };
 
@@ -326,7 +396,7 @@ namespace llamql
             });
             buf = next;
         }
-        if (KG == 1 || (rounds - 1) * KG + kg < turns)
+        if (KG == 1 || (rounds - 1) * KG + kg < count)
         {
 #pragma unroll
             for (int s = 0; s < 3; ++s)
@@ -408,7 +478,7 @@ namespace llamql
 #pragma unroll
                         for (int r = 0; r < 16; ++r)
                             whole[j][i][r] = 0.0f;
-                for (int s = 0; s < 2 * ksteps; ++s) // sixteen columns
+                for (int s = 4 * turn0; s < 4 * (turn0 + count); ++s) // sixteen columns
                 {
                     f32x8 x[TM], v[TN];
 #pragma unroll
@@ -435,63 +505,83 @@ namespace llamql
             }
         }
 
-        // Results by way of LDS, where a wavefront lays 32 rows of its own columns and takes them up again by whole rows: straight
-        // from the accumulators a store instruction of 64 lanes touches 32 rows, 8 or 16 bytes a lane, and loads of other workgroups
-        // wait behind that (bf16, straight and by way of LDS: 2048 x 16384 x 2048 165 -> 112 us, 2048 x 16384 x 8192 503 -> 426).
-        const size_t elem = p.out == LLAM_SEQ_OUT_F32 || p.out == LLAM_SEQ_OUT_ADD ? 4 : sizeof(T);
-        char *y = static_cast<char *>(p.y) + (p.group_offset ? 0 : (size_t)z * p.y_stride * elem);
+        if constexpr (SPLIT)
+        {
+            if (!whole)
+            {
+                // as the lanes hold them
+                f32x4 *part_sums = p.parts + ((size_t)slice * (total - p.full) + die_order(part, total - p.full)) * (BM * BN / 4) +
+                                   wave * (TN * TM * 256) + lane;
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+#pragma unroll
+                    for (int j = 0; j < TN; ++j)
+#pragma unroll
+                        for (int q = 0; q < 4; ++q)
+                            part_sums[((i * TN + j) * 4 + q) * 64] =
+                                f32x4{acc[j][i][4 * q], acc[j][i][4 * q + 1], acc[j][i][4 * q + 2], acc[j][i][4 * q + 3]};
+                return;
+            }
+        }
         if constexpr (KG == 1)
             arrive<0>(); // all wavefronts are done with the stages (of several groups, the place of the wavefront's own sums)
-        char *own = smem + wave * (KG == 1 ? TN * OUT_BYTES : TN * TM * 4096);
-        auto out = [&](auto gated, auto value) __attribute__((always_inline)) {
-            typedef decltype(value) V;
-            constexpr bool GATED = decltype(gated)::value;
-            constexpr int COLS = GATED ? TN * 16 : TN * 32, PITCH = COLS * sizeof(V);
-            constexpr int EACH = 16 / sizeof(V), PIECES = COLS / EACH; // values of a 16-byte piece, pieces of a row
-            typedef V four_t __attribute__((ext_vector_type(4)));
-            typedef V piece_t __attribute__((ext_vector_type(EACH)));
-            // piece x of row r lies at x ^ spread(r)
-            auto spread = [](int r) __attribute__((always_inline)) { return r / (PIECES < 8 ? 8 / PIECES : 1) & (PIECES - 1); };
-            const int n0 = (nt * BN + wn * TN * 32) / (GATED ? 2 : 1), columns = GATED ? p.N / 2 : p.N;
-            const bool whole = ((p.ldy | p.y_stride) & (EACH - 1)) == 0; // (rows of 16-bit values may start at 8 bytes)
+        char *own = smem + wave * (KG == 1 ? TN * OUT_BYTES : TN * TM * OUT_BYTES);
 #pragma unroll
-            for (int i = 0; i < TM; ++i)
-            {
+        for (int i = 0; i < TM; ++i)
+        {
+            f32x16 strip[TN];
 #pragma unroll
-                for (int j = 0; j < TN; ++j)
+            for (int j = 0; j < TN; ++j)
+                strip[j] = acc[j][i];
+            results<T>(p, p.group_offset ? 0 : z, strip, own, lane, mt * BM + (wm * TM + i) * 32, rows, row0, nt * BN + wn * TN * 32);
+        }
+    }
+
+    // A wavefront joins the slices of 32 rows of what a wavefront of linear_wide_kernel had, in the order of K.
+    template <typename T, int BM, int BN, int WM, int WN>
+    __global__ void __launch_bounds__(256)
+        linear_join_kernel(LinearArgs p, int m_tiles, int n_tiles)
+    {
+        constexpr int NW = WM * WN, TM = BM / WM / 32, TN = BN / WN / 32;
+        __shared__ __attribute__((aligned(16))) char smem[4 * TN * OUT_BYTES];
+        const int lane = threadIdx.x & 63, here = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+        const int unit = blockIdx.x * 4 + here, split = m_tiles * n_tiles - p.full;
+        static_assert(NW * TM % 4 == 0, "whole workgroups");
+        const int id = unit / (NW * TM), wave = unit / TM % NW, i = unit % TM;
+        int mt, nt;
+        tile_place(p.full + id, m_tiles, n_tiles, mt, nt);
+        const f32x4 *from = p.parts + (size_t)id * (BM * BN / 4) + (wave * TM + i) * (TN * 256) + lane;
+        f32x16 strip[TN];
 #pragma unroll
-                    for (int q = 0; q < (GATED ? 2 : 4); ++q)
-                    {
-                        auto four = [&](int q) __attribute__((always_inline)) {
-                            return f32x4{acc[j][i][4 * q], acc[j][i][4 * q + 1], acc[j][i][4 * q + 2], acc[j][i][4 * q + 3]};
-                        };
-                        f32x4 v = four(q);
-                        if constexpr (GATED) // rows 0 .. 15 of the product are gates, 16 .. 31 the same of up
-                            v = gated4(p, v, four(q + 2));
-                        else if (sizeof(V) == sizeof(T) && p.out == LLAM_SEQ_OUT_RELU2)
-                            v = relu2(v);
-                        const int col = j * (GATED ? 16 : 32) + 8 * q + 4 * h;
-                        *reinterpret_cast<four_t *>(own + c * PITCH + (col / EACH ^ spread(c)) * 16 + col % EACH * sizeof(V)) = __builtin_convertvector(v, four_t);
-                    }
-                asm volatile("" ::: "memory"); // (a wavefront's LDS instructions run in order)
+        for (int j = 0; j < TN; ++j)
 #pragma unroll
-                for (int k = 0; k < PIECES / 2; ++k)
-                {
-                    const int r = (k * 64 + lane) / PIECES, x = (k * 64 + lane) % PIECES, col = n0 + x * EACH;
-                    const int m = mt * BM + (wm * TM + i) * 32 + r;
-                    piece_t v = *reinterpret_cast<const piece_t *>(own + r * PITCH + (x ^ spread(r)) * 16);
-                    if (m < rows && col < columns)
-                        store_piece(p, y, whole, row0 + m, col, v);
-                }
-                asm volatile("" ::: "memory");
-            }
+            for (int r = 0; r < 16; ++r)
+                strip[j][r] = 0.0f;
+        // `count` slices from k on, asked for together
+        auto add = [&](auto count, int k) __attribute__((always_inline)) {
+            f32x4 v[count.value][TN * 4];
+#pragma unroll
+            for (int u = 0; u < count.value; ++u)
+#pragma unroll
+                for (int x = 0; x < TN * 4; ++x)
+                    v[u][x] = from[(size_t)(k + u) * split * (BM * BN / 4) + x * 64];
+#pragma unroll
+            for (int u = 0; u < count.value; ++u)
+#pragma unroll
+                for (int x = 0; x < TN * 4; ++x)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        strip[x / 4][x % 4 * 4 + r] += v[u][x][r];
         };
-        if (is_gated(p.out))
-            out(std::true_type(), T());
-        else if (elem == sizeof(T))
-            out(std::false_type(), T());
-        else
-            out(std::false_type(), float());
+        constexpr int GROUP = TN > 2 ? 2 : 4;
+        int k = 0;
+        for (; k + GROUP <= p.slices; k += GROUP)
+            add(std::integral_constant<int, GROUP>(), k);
+        if (GROUP == 4 && k + 2 <= p.slices)
+            add(std::integral_constant<int, 2>(), k), k += 2;
+        if (k < p.slices)
+            add(std::integral_constant<int, 1>(), k);
+        results<T>(p, 0, strip, smem + here * (TN * OUT_BYTES), lane, mt * BM + (wave % WM * TM + i) * 32, p.M, 0, nt * BN + wave / WM * TN * 32);
     }
 
     namespace
@@ -504,7 +594,7 @@ namespace llamql
             static_assert(KG > 1 || stages >= (size_t)WM * BN * OUT_BYTES / 32, "the results' place");
             constexpr size_t lds = stages > sums ? stages : sums;
             static_assert(lds <= 160 * 1024, "stages must fit the LDS");
-            const auto kernel = &linear_wide_kernel<T, BM, BN, WM, WN, KG, STAGES>;
+            const auto kernel = &linear_wide_kernel<T, BM, BN, WM, WN, KG, STAGES, false>;
             if (lds > 64 * 1024 && allow_lds(grant, reinterpret_cast<const void *>(kernel), lds) != hipSuccess)
                 return fail(fn, "cannot reserve %zu bytes of LDS", lds);
             const int nt = ceil_div(a.N, BN);
@@ -516,6 +606,24 @@ namespace llamql
             return launched(fn);
         }
 
+        // The same with the tiles from a.full on in a.slices slices of K each, which a second launch joins.
+        template <typename T, int BM, int BN, int WM, int WN, int KG, int STAGES>
+        bool split_launch(const char *fn, const LinearArgs &a, hipStream_t st)
+        {
+            static LdsGrant grant;
+            constexpr size_t stages = (size_t)STAGES * KG * (BM * sizeof(T) + BN * 2) * TILE_K, sums = (size_t)(KG - 1) * BM * BN * 4;
+            constexpr size_t lds = stages > sums ? stages : sums;
+            const auto kernel = &linear_wide_kernel<T, BM, BN, WM, WN, KG, STAGES, true>;
+            if (lds > 64 * 1024 && allow_lds(grant, reinterpret_cast<const void *>(kernel), lds) != hipSuccess)
+                return fail(fn, "cannot reserve %zu bytes of LDS", lds);
+            const int nt = ceil_div(a.N, BN), mt = ceil_div(a.M, BM), split = mt * nt - a.full;
+            hipLaunchKernelGGL(kernel, dim3((unsigned)(a.full + split * a.slices)), dim3(WM * WN * KG * 64), lds, st, a, mt, nt);
+            if (!launched(fn))
+                return false;
+            hipLaunchKernelGGL((linear_join_kernel<T, BM, BN, WM, WN>), dim3((unsigned)(split * (BM / 32) * WN / 4)), dim3(256), 0, st, a, mt, nt);
+            return launched(fn);
+        }
+
         // A tile, and what a turn of it takes in microseconds where few compute units are busy and where all are (with
         // `resident` workgroups each), and a workgroup's start and end.
         struct Tile
@@ -523,6 +631,7 @@ namespace llamql
             int rows, columns, groups, resident;
             float alone, full, start;
             bool (*launch)(const char *, const LinearArgs &, int, hipStream_t);
+            bool (*split)(const char *, const LinearArgs &, hipStream_t); // (none where two workgroups share a compute unit)
         };
         // Measured as time over turns for widths of 2048 to 51200, 40 to 2048 rows and K of 2048 to 30720.  Large tiles
         // read the LDS least per product (256 x 256: 1130 TFLOP/s at 2048 x 51200 x 5120, 128 x 128: 1010), small ones
@@ -533,20 +642,20 @@ namespace llamql
         // 187 rows, 6 of 64 experts of 1408 x 2048 and a shared one: bf16 209 -> 190 us against two tiles by the mean
         // rows of a group, fp32 369 -> 267 against tiles as if every group had all rows.
         const Tile TILES_BF16[] = {
-            {256, 256, 1, 1, 1.30f, 1.70f, 4.0f, wide_launch<bf16, 256, 256, 2, 4, 1, 2>},
-            {256, 128, 1, 1, 0.75f, 1.00f, 4.0f, wide_launch<bf16, 256, 128, 4, 2, 1, 3>},
-            {128, 128, 1, 2, 0.65f, 1.05f, 4.0f, wide_launch<bf16, 128, 128, 2, 2, 1, 2>},
-            {128, 128, 1, 1, 0.57f, 0.60f, 3.0f, wide_launch<bf16, 128, 128, 4, 2, 1, 3>},
-            {128, 64, 2, 1, 0.60f, 0.70f, 3.0f, wide_launch<bf16, 128, 64, 2, 2, 2, 3>},
-            {64, 64, 2, 1, 0.40f, 0.50f, 3.0f, wide_launch<bf16, 64, 64, 2, 2, 2, 4>},
-            {64, 64, 1, 2, 0.26f, 0.43f, 3.0f, wide_launch<bf16, 64, 64, 2, 2, 1, 4>},
+            {256, 256, 1, 1, 1.30f, 1.70f, 4.0f, wide_launch<bf16, 256, 256, 2, 4, 1, 2>, split_launch<bf16, 256, 256, 2, 4, 1, 2>},
+            {256, 128, 1, 1, 0.75f, 1.00f, 4.0f, wide_launch<bf16, 256, 128, 4, 2, 1, 3>, split_launch<bf16, 256, 128, 4, 2, 1, 3>},
+            {128, 128, 1, 2, 0.65f, 1.05f, 4.0f, wide_launch<bf16, 128, 128, 2, 2, 1, 2>, nullptr},
+            {128, 128, 1, 1, 0.57f, 0.60f, 3.0f, wide_launch<bf16, 128, 128, 4, 2, 1, 3>, split_launch<bf16, 128, 128, 4, 2, 1, 3>},
+            {128, 64, 2, 1, 0.60f, 0.70f, 3.0f, wide_launch<bf16, 128, 64, 2, 2, 2, 3>, split_launch<bf16, 128, 64, 2, 2, 2, 3>},
+            {64, 64, 2, 1, 0.40f, 0.50f, 3.0f, wide_launch<bf16, 64, 64, 2, 2, 2, 4>, split_launch<bf16, 64, 64, 2, 2, 2, 4>},
+            {64, 64, 1, 2, 0.26f, 0.43f, 3.0f, wide_launch<bf16, 64, 64, 2, 2, 1, 4>, nullptr},
         };
         // (in three pieces: the cutting up of A costs as much as the products where a wavefront has few columns)
         const Tile TILES_F32[] = {
-            {128, 256, 1, 1, 2.00f, 2.60f, 4.0f, wide_launch<float, 128, 256, 4, 2, 1, 2>},
-            {128, 128, 1, 1, 1.34f, 1.65f, 3.0f, wide_launch<float, 128, 128, 4, 2, 1, 3>},
-            {64, 128, 2, 1, 1.45f, 1.75f, 3.0f, wide_launch<float, 64, 128, 2, 2, 2, 2>},
-            {64, 64, 2, 1, 1.15f, 1.30f, 3.0f, wide_launch<float, 64, 64, 2, 2, 2, 3>},
+            {128, 256, 1, 1, 2.00f, 2.60f, 4.0f, wide_launch<float, 128, 256, 4, 2, 1, 2>, split_launch<float, 128, 256, 4, 2, 1, 2>},
+            {128, 128, 1, 1, 1.34f, 1.65f, 3.0f, wide_launch<float, 128, 128, 4, 2, 1, 3>, split_launch<float, 128, 128, 4, 2, 1, 3>},
+            {64, 128, 2, 1, 1.45f, 1.75f, 3.0f, wide_launch<float, 64, 128, 2, 2, 2, 2>, split_launch<float, 64, 128, 2, 2, 2, 2>},
+            {64, 64, 2, 1, 1.15f, 1.30f, 3.0f, wide_launch<float, 64, 64, 2, 2, 2, 3>, split_launch<float, 64, 64, 2, 2, 2, 3>},
         };
 
         float expected(const Tile &t, const LinearArgs &a, int batch, int cus)
@@ -565,14 +674,88 @@ namespace llamql
         }
     } // namespace
 
-    bool linear_tiled(const char *fn, const LinearArgs &a, int batch, int dtype, int device_id, hipStream_t st)
+    namespace
+    {
+        // Tiles that fill no round of workgroups by themselves, cut into slices of K that do: in the time of a slice instead of that of a
+        // tile, for the sums that leave and come back and a launch that joins them.  (us, whole and in slices: bf16, 2048 x 5120 x 30720 682 -> 583,
+        // 500 x 5120 x 30720 247 -> 165, 64 x 2048 x 10240 31 -> 15, 1000 x 51200 x 5120 520 -> 466; fp32, 522 x 2048 x 10240 114 -> 82,
+        // 64 x 2048 x 16384 135 -> 28.)  Over 17 layers of 1280 to 51200 x 1024 to 30720 with 14 numbers of rows in bf16, 12 with 9 in fp32, 105 of 252
+        // and 75 of 108 are cut, to 0.74 and 0.56 times their time in the mean; none is slower, the choice is 1.2 % above the best of all.
+        constexpr int SLICES = 8;                        // at most
+        constexpr size_t SPLIT_BYTES = (size_t)192 << 20; // sums of a launch, at most
+        constexpr float JOIN_START = 4.0f, JOIN_BYTE = 0.45e-6f; // microseconds: a launch; a byte there and back
+
+        struct Split
+        {
+            float us; // expected
+            int full, slices;
+            size_t bytes;
+        };
+        Split best_split(const Tile &t, const LinearArgs &a, size_t bytes, int cus)
+        {
+            Split best = {1e30f, 0, 0, 0};
+            const long tiles = (long)ceil_div(a.M, t.rows) * ceil_div(a.N, t.columns), full = tiles / cus * cus, rest = tiles - full;
+            const int turns = a.K / TILE_K;
+            if (!t.split || rest == 0 || full + rest * SLICES > 0x7fffffff)
+                return best;
+            for (int slices = 2; slices <= SLICES && slices * 2 * t.groups <= turns; ++slices)
+            {
+                const long pieces = rest * slices, rounds = (pieces + cus - 1) / cus;
+                const size_t need = (size_t)pieces * t.rows * t.columns * 4;
+                if (need > bytes)
+                    break;
+                const float turn = t.alone + (t.full - t.alone) * (pieces < cus ? (float)pieces / cus : 1.0f);
+                const float us = (float)(full / cus) * (ceil_div(turns, t.groups) * t.full + t.start) +
+                                 rounds * (ceil_div(ceil_div(turns, slices), t.groups) * turn + t.start) + JOIN_START + JOIN_BYTE * need;
+                if (us < best.us)
+                    best = {us, (int)full, slices, need};
+            }
+            return best;
+        }
+
+        struct Plan
+        {
+            const Tile *tile;
+            Split split; // slices = 0: every tile whole
+        };
+        Plan linear_plan(const LinearArgs &a, int batch, int dtype, size_t bytes, int cus)
+        {
+            const Tile *tiles = dtype == LLAM_SEQ_F32 ? TILES_F32 : TILES_BF16;
+            const size_t n = dtype == LLAM_SEQ_F32 ? sizeof TILES_F32 / sizeof(Tile) : sizeof TILES_BF16 / sizeof(Tile);
+            Plan plan = {tiles, {expected(*tiles, a, batch, cus), 0, 0, 0}};
+            for (size_t i = 1; i < n; ++i)
+                if (const float us = expected(tiles[i], a, batch, cus); us < plan.split.us)
+                    plan = {&tiles[i], {us, 0, 0, 0}};
+            if (batch == 1 && !a.group_offset && bytes)
+                for (size_t i = 0; i < n; ++i)
+                    if (const Split s = best_split(tiles[i], a, bytes < SPLIT_BYTES ? bytes : SPLIT_BYTES, cus); s.us < plan.split.us)
+                        plan = {&tiles[i], s};
+            return plan;
+        }
+    } // namespace
+
+    size_t linear_split_bytes(int max_rows, int N, int K, int dtype, int device_id)
     {
         const int cus = cu_count(device_id);
-        const Tile *tiles = dtype == LLAM_SEQ_F32 ? TILES_F32 : TILES_BF16, *best = tiles;
-        const size_t n = dtype == LLAM_SEQ_F32 ? sizeof TILES_F32 / sizeof(Tile) : sizeof TILES_BF16 / sizeof(Tile);
-        for (size_t i = 1; i < n; ++i)
-            if (expected(tiles[i], a, batch, cus) < expected(*best, a, batch, cus))
-                best = &tiles[i];
-        return best->launch(fn, a, batch, st);
+        size_t most = 0;
+        LinearArgs a{};
+        a.N = N, a.K = K;
+        for (int rows = 64; rows - 64 < max_rows; rows += 64) // (a plan depends on the tiles of rows alone)
+        {
+            a.M = rows < max_rows ? rows : max_rows;
+            const size_t need = a.M > SMALL_M ? linear_plan(a, 1, dtype, SPLIT_BYTES, cus).split.bytes : 0;
+            most = need > most ? need : most;
+        }
+        return most;
+    }
+
+    bool linear_tiled(const char *fn, const LinearArgs &a, int batch, int dtype, int device_id, hipStream_t st, void *scratch, size_t bytes)
+    {
+        const Plan plan = linear_plan(a, batch, dtype, scratch ? bytes : 0, cu_count(device_id));
+        if (plan.split.slices == 0)
+            return plan.tile->launch(fn, a, batch, st);
+        LinearArgs cut = a;
+        cut.parts = static_cast<f32x4 *>(scratch), cut.full = plan.split.full, cut.slices = plan.split.slices;
+        return plan.tile->split(fn, cut, st);
     }
 } // namespace llamql

@@ -200,7 +200,7 @@ namespace
             l.d_a = a, l.lda = lda, l.d_w = w, l.N = N, l.K = K, l.d_y = y, l.ldy = ldy, l.out = out, l.M = M;
             l.d_bias = bias, l.d_norm = norm, l.k_real = k_real, l.eps = c.eps, l.d_h_out = h_out;
             l.batch = batch, l.a_stride = as, l.w_stride = ws, l.y_stride = ys;
-            return forward(fn, llam_seq_linear(&l, c.dtype, c.device_id, st));
+            return forward(fn, llam_seq_linear_within(&l, md.scratch, md.scratch_bytes, c.dtype, c.device_id, st));
         }
 
         static bool fused(int M, int K) { return M <= ROW_MAX && (long)M * K <= NORM_FUSE_MAX; }
@@ -234,7 +234,10 @@ namespace
             a.d_norm = fuse ? w.norm1 : nullptr, f.d_norm = fuse ? w.norm2 : nullptr;
             for (llam_seq_linear_args *l : {&a, &f})
                 l->M = s.M, l->K = K, l->lda = fuse ? md.wp : K, l->k_real = c.width, l->eps = c.eps, l->batch = 1;
-            return forward(fn, llam_seq_linear_pair(&a, &f, c.dtype, c.device_id, st));
+            if (s.M <= ROW_MAX)
+                return forward(fn, llam_seq_linear_pair(&a, &f, c.dtype, c.device_id, st));
+            return forward(fn, llam_seq_linear_within(&a, md.scratch, md.scratch_bytes, c.dtype, c.device_id, st)) &&
+                   forward(fn, llam_seq_linear_within(&f, md.scratch, md.scratch_bytes, c.dtype, c.device_id, st));
         }
 
         // x += W_out of the mixer's heads (and of a parallel layer's feed-forward)
@@ -559,15 +562,23 @@ extern "C" bool llam_seqm_set_globals(void *model, const llam_seqm_globals *g)
     bool parallel = false;
     size_t n_in = 0, q = 0, lat = 0, mix = 0, act = 0, z = 16, h = md->wp, latf = 0, scratch = 0;
     const int portions = std::max(1, std::min(c.slots, c.max_rows / 2)); // (of two tokens at least) in a step
+    // (the linear layers and what else needs scratch take turns)
+    const auto linear = [&](size_t rows, int columns, size_t K) {
+        scratch = std::max(scratch, llam_seq_linear_scratch_bytes((int)rows, columns, (int)K, c.dtype, c.device_id));
+    };
+    const size_t step_rows = std::max(c.max_rows, c.slots);
     for (const llam_seqm_layer &w : md->layers)
     {
         const size_t H = w.heads, dp = P(w.dim), vp = P(w.vdim);
         mix = std::max(mix, (size_t)mix_columns(w));
+        size_t layer_in = 0; // columns of the mixer's projections
         parallel |= w.parallel && w.ffn;
         if (w.mixer == LLAM_MIXER_LATENT_ATTENTION)
         {
             const size_t rp = P(w.kv_rank);
-            n_in = std::max(n_in, (size_t)P(w.q_rank) + rp);
+            layer_in = (size_t)P(w.q_rank) + rp;
+            linear(step_rows, P(w.q_rank) + (w.kv_from < 0 ? (int)rp : 0), md->wp);
+            linear(step_rows, (int)(H * dp), P(w.q_rank));
             h = std::max(h, (size_t)P(w.q_rank));
             q = std::max(q, H * dp);
             lat = std::max(lat, H * rp);
@@ -575,29 +586,40 @@ extern "C" bool llam_seqm_set_globals(void *model, const llam_seqm_globals *g)
         }
         else if (w.mixer == LLAM_MIXER_ATTENTION)
         {
-            n_in = std::max(n_in, H * A(w.dim) + (w.kv_from < 0 ? (size_t)w.kv_heads * (A(w.dim) + A(w.vdim)) : 0));
+            layer_in = H * A(w.dim) + (w.kv_from < 0 ? (size_t)w.kv_heads * (A(w.dim) + A(w.vdim)) : 0);
             q = std::max(q, H * A(w.dim));
             latf = std::max(latf, llam_seq_attention_scratch_floats(A(w.vdim)));
         }
         else if (w.mixer == LLAM_MIXER_DELTA)
         {
-            n_in = std::max(n_in, (size_t)pad((int)(2 * w.kv_heads * dp + 2 * H * vp + 2 * H), 16));
+            layer_in = pad((int)(2 * w.kv_heads * dp + 2 * H * vp + 2 * H), 16);
             scratch = std::max(scratch, llam_seq_delta_portions_scratch_bytes(c.max_rows, portions, w.heads, w.kv_heads, (int)dp, (int)vp));
         }
         else
         {
-            n_in = std::max(n_in, (size_t)pad((int)(2 * H * (dp + vp) + 2 * H), 16));
+            layer_in = pad((int)(2 * H * (dp + vp) + 2 * H), 16);
             scratch = std::max(scratch, llam_seq_memory_portions_scratch_bytes(std::max(c.max_rows, c.slots), portions, w.heads, (int)dp, (int)vp));
         }
+        n_in = std::max(n_in, layer_in);
+        if (w.mixer != LLAM_MIXER_LATENT_ATTENTION)
+            linear(step_rows, (int)layer_in, md->wp);
+        linear(step_rows, md->wp, mix_columns(w));
+        if (gated(w.ffn))
+            linear(step_rows, 2 * P(w.ff), md->wp);
         if (gated(w.ffn) && !w.parallel)
+        {
             act = std::max(act, (size_t)P(w.ff));
+            linear(step_rows, md->wp, P(w.ff));
+        }
         if (w.ffn == LLAM_FFN_EXPERTS)
         {
             z = std::max(z, (size_t)pad(w.experts + 1, 16));
+            linear(step_rows, pad(w.experts + (w.shared_ff ? 1 : 0), 16), md->wp);
             scratch = std::max(scratch, llam_seq_experts_scratch_bytes(c.max_rows, w.experts, w.top, P(w.ff),
                                                                        w.shared_ff ? P(w.shared_ff) : 0, md->wp));
         }
     }
+    linear(std::max(LOGIT_ROWS, c.slots), md->vp, md->wp);
     md->lat_floats = latf;
     md->scratch_bytes = scratch;
     bool ok = (md->x = (float *)md->take(fn, M * md->wp * 4)) && (md->h = md->take(fn, M * h * elem)) && (md->h2 = md->take(fn, parallel ? M * md->wp * elem : 0)) &&

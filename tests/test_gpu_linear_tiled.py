@@ -185,3 +185,86 @@ def test_rows_that_start_at_eight_bytes(dev, M, N, K, out):
     run(torch, a, t, y[:M, :columns], BF16, out, N, K)
     assert torch.equal(y[:M, :columns], aligned[:, :columns])
     assert (y[M:] == 5.0).all() and (y[:, columns:] == 5.0).all() and (aligned[:, columns:] == 5.0).all()
+
+
+# ---- tiles cut along K (llam_seq_linear_within) ------------------------------------------------------------
+
+# every tile that is cut, with and without whole ones beside it, slices of unequal length (test_launch_rules.py)
+SPLIT = [(17, 48, 2112), (33, 80, 1024), (65, 2064, 8256), (257, 2064, 8256), (1000, 16400, 512), (700, 6160, 8256), (2048, 4112, 2112),
+         (65, 2064, 1024), (2048, 272, 4160), (1500, 6160, 512), (200, 4112, 4160)]
+
+
+def run_within(torch, a, w, y, dtype, out=sq.OUT_F32, N=None, K=None, bias=None, short=0):
+    """The layer with the scratch that it asks for, `short` bytes less; what lies behind the scratch stays as it is."""
+    M = y.shape[0]
+    need = sq.load().llam_seq_linear_scratch_bytes(M, N, K, dtype, 0)
+    scratch = torch.full((need + 4096,), 171, dtype=torch.uint8, device=y.device)
+    args = sq.LinearArgs(d_a=a.data_ptr(), d_w=w.data_ptr(), d_y=y.data_ptr(), M=M, N=N, K=K, lda=a.stride(-2), ldy=y.stride(-2), out=out,
+                         batch=1, limit=7.0, d_bias=0 if bias is None else bias.data_ptr())
+    ok = sq.load().llam_seq_linear_within(ctypes.byref(args), scratch.data_ptr(), need - short, dtype, 0, torch.cuda.current_stream().cuda_stream)
+    assert ok, sq.load().llam_ql_last_error()
+    torch.cuda.synchronize()
+    assert (scratch[need - short:] == 171).all(), "written past the scratch"
+    return need
+
+
+@pytest.mark.parametrize("dtype", [BF16, F32])
+@pytest.mark.parametrize("M,N,K", SPLIT)
+def test_slices_of_k(dev, M, N, K, dtype):
+    import torch
+
+    torch.manual_seed(M + N)
+    a = torch.randn(M, K, device=dev)
+    a = a if dtype == F32 else a.bfloat16()
+    w, bias = torch.randn(N, K, device=dev).bfloat16(), torch.randn(N, device=dev)
+    y = torch.full((M + 1, N + 4), 5.0, device=dev)
+    run_within(torch, a, tiles(w), y[:M, :N], dtype, N=N, K=K)
+    close(torch, y[:M, :N], a, w, K)
+    assert (y[M:] == 5.0).all() and (y[:, N:] == 5.0).all(), "written past the output"
+    again = torch.empty(M, N, device=dev)
+    run_within(torch, a, tiles(w), again, dtype, N=N, K=K)
+    assert torch.equal(again, y[:M, :N])
+    run_within(torch, a, tiles(w), again, dtype, N=N, K=K, bias=bias)
+    assert torch.equal(again, y[:M, :N] + bias)
+    run_within(torch, a, tiles(w), again, dtype, N=N, K=K, short=16)   # (fewer slices, or none)
+    close(torch, again, a, w, K)
+
+
+@pytest.mark.parametrize("dtype", [BF16, F32])
+@pytest.mark.parametrize("out", [sq.OUT_ADD, sq.OUT_ELEM, sq.OUT_GATED, sq.OUT_RELU2, sq.OUT_GATED_CLAMP])
+@pytest.mark.parametrize("M,N,K", [(40, 96, 2112), (300, 2080, 4160), (700, 6176, 4160)])
+def test_outputs_of_slices(dev, M, N, K, out, dtype):
+    """The same values as without scratch: sums of unit size differ by their rounding, 2^-23 K, through slopes below 20."""
+    import torch
+
+    torch.manual_seed(out)
+    a, w = torch.randn(M, K, device=dev), tiles((torch.randn(N, K, device=dev) * K ** -0.5).bfloat16())
+    a = a if dtype == F32 else a.bfloat16()
+    kind = torch.float32 if dtype == F32 or out == sq.OUT_ADD else torch.bfloat16
+    y = torch.randn(M, N // 2 if out in (sq.OUT_GATED, sq.OUT_GATED_CLAMP) else N, device=dev).to(kind)
+    want = y.clone()
+    run(torch, a, w, want, dtype, out, N, K)
+    run_within(torch, a, w, y, dtype, out, N, K)
+    off = (y.double() - want.double()).abs()
+    assert (off <= (2.0 ** -8 if kind == torch.bfloat16 else 2.0 ** -20) * want.double().abs() + 20 * K * 2.0 ** -23).all()
+
+
+@pytest.mark.parametrize("M,N,K", [(20, 64, 2048), (65, 2064, 1024), (200, 4112, 4160)])
+def test_infinite_and_small_values_in_slices(dev, M, N, K):
+    """32-bit rows in three pieces: what the pieces do not carry is multiplied once more, slice by slice."""
+    import torch
+
+    torch.manual_seed(M)
+    a, w = torch.randn(M, K, device=dev).bfloat16().float(), torch.randn(N, K, device=dev).bfloat16()
+    w[3, 5], w[N - 1, K - 1], w[N // 2, 0], w[N // 2, K - 9] = float("inf"), float("-inf"), float("inf"), float("-inf")
+    a[2, 5], a[M - 1, 7] = 0.0, float("inf")
+    a[5] = 0.0
+    a[5, 3], a[5, K - 2] = 1.2345678e-33, -2.3e-34
+    y = torch.zeros(M, N, device=dev)
+    assert run_within(torch, a, tiles(w), y, F32, N=N, K=K) > 0
+    want = (a.double() @ w.double().T).float()
+    assert torch.isposinf(want[:, 3]).any() and torch.isnan(want[2, 3])
+    for kind in (torch.isnan, torch.isposinf, torch.isneginf):
+        assert torch.equal(kind(y), kind(want))
+    plain = [n for n in range(N) if n not in (3, N // 2, N - 1)]
+    close(torch, y[:M - 1][:, plain], a[:M - 1], w[plain], K)

@@ -257,3 +257,63 @@ answer([decode(8, 16), decode(8, 3), model._error()])
 """)
     assert long[0] == [0, 8 * 16, 0] and after[0] == [0, 8 * 3, 0] and len(set(long[1] + after[1])) == 1
     assert error == ""
+
+
+# ---- linear layers cut along K (linear_tiled.hip: linear_plan): what the library launches --------------------
+
+SLICED = """
+from llaminar_amd import sequence as sq
+lib = sq.load()
+p = 1 << 20
+def launches(M, N, K, dtype, bytes, scratch=p):
+    a = sq.LinearArgs(d_a=p, d_w=p, d_y=p, M=M, N=N, K=K, lda=K, ldy=N, batch=1)
+    assert lib.llam_seq_linear_within(ctypes.byref(a), scratch, bytes, dtype, 0, None)
+    return [l[1:] for l in log() if l[0] == "launch"]
+def need(M, N, K, dtype):
+    return lib.llam_seq_linear_scratch_bytes(M, N, K, dtype, 0)
+"""
+WIDE = re.compile(r"linear_wide_kernelI(DF16b|f)((?:Li\d+E)+)Lb([01])E")
+
+
+def sliced(launched):
+    """(type and tile, pieces) of a layer's launches, None where nothing is cut."""
+    kind, tile, split = WIDE.search(launched[0][0]).groups()
+    assert (split == "1") == (len(launched) == 2)
+    if split == "0":
+        return None
+    return (kind, tuple(map(int, re.findall(r"\d+", tile)))), int(launched[0][1])
+
+
+def test_every_tile_that_is_cut_has_sizes(tmp_path):
+    chosen = fake_hip.run(tmp_path, SLICED + f"""
+answer([launches(M, N, K, dtype, need(M, N, K, dtype)) for dtype in (0, 1) for M, N, K in {test_gpu_linear_tiled.SPLIT}])""")
+    cuts = [c for c in map(sliced, chosen) if c]
+    for kind, name in (("DF16b", "bf16"), ("f", "float")):
+        every = {tuple(map(int, re.findall(r"\d+", t))) for t in re.findall(r"split_launch<%s, ([\d, ]+)>\}" % name, LINEAR)}
+        assert {t for (k, t), _ in cuts if k == kind} == every and len(every) >= 4
+
+
+def test_a_layer_stays_within_its_scratch(tmp_path):
+    """What is asked for serves every number of rows up to the most, none is written past it, and without any nothing is cut."""
+    rng = np.random.default_rng(5)
+    layers = [(int(rng.integers(17, 2100)), 16 * int(2 ** rng.uniform(0, 11)), 64 * int(2 ** rng.uniform(0, 9)), int(rng.integers(2))) for _ in range(60)]
+    found = fake_hip.run(tmp_path, SLICED + f"""
+rows = lambda most: sorted({{17, 64, 65, 129, 257, most // 2, most - 1, most}} & set(range(17, most + 1)))
+answer([[need(most, N, K, dtype), need(most, N, K, dtype) // 2,
+         [[launches(M, N, K, dtype, size) for M in rows(most)] for size in (need(most, N, K, dtype), 1 << 40, need(most, N, K, dtype) // 2, 0)],
+         [launches(M, N, K, dtype, 1 << 40, None) for M in rows(most)]] for most, N, K, dtype in {layers}])""")
+    cut = 0
+    for (most, N, K, dtype), (need, half, (enough, plenty, little, none), null) in zip(layers, found):
+        assert enough == plenty and none == null and all(sliced(l) is None for l in none) and need <= 192 << 20
+        rows = sorted({17, 64, 65, 129, 257, most // 2, most - 1, most} & set(range(17, most + 1)))
+        for launched, limit in ((enough, need), (little, half)):
+            for M, l in zip(rows, launched):
+                if sliced(l):
+                    cut += 1
+                    (_, (height, width, *_)), pieces = sliced(l)
+                    whole = over(M, height) * over(N, width) // CUS * CUS
+                    rest = over(M, height) * over(N, width) - whole
+                    slices = (pieces - whole) // rest
+                    assert pieces == whole + rest * slices and 2 <= slices <= 8 and slices <= K // 64
+                    assert rest * slices * height * width * 4 <= limit
+    assert cut > 50
