@@ -180,9 +180,9 @@ namespace llamql
     }
 
     // Workgroup tile BM rows of A x BN rows of W; KG groups of WM x WN wavefronts, each with every KG-th turn of 64
-    // columns, STAGES turns of LDS.  SPLIT: the tiles from p.full on have p.slices workgroups each, every one with a slice of K,
+    // columns, STAGES turns of A in LDS and WSTAGES of W.  SPLIT: the tiles from p.full on have p.slices workgroups each, every one with a slice of K,
     // which leave their accumulators in p.parts for linear_join_kernel.
-    template <typename T, int BM, int BN, int WM, int WN, int KG, int STAGES, bool SPLIT>
+    template <typename T, int BM, int BN, int WM, int WN, int KG, int STAGES, int WSTAGES, bool SPLIT>
     __global__ void __launch_bounds__(WM *WN *KG * 64)
         linear_wide_kernel(LinearArgs p, int m_tiles, int n_tiles)
     {
@@ -191,9 +191,9 @@ namespace llamql
         constexpr int TM = BM / WM / 32, TN = BN / WN / 32; // 32x32 products of a wavefront
         constexpr int AROW = TILE_K * sizeof(T), AROWS = 1024 / AROW, APIECES = AROW / 16; // bytes; rows of a load; 16-byte pieces
         constexpr int ALOADS = BM / AROWS / NW, WLOADS = BN / 8 / NW, LOADS = ALOADS + WLOADS; // of a turn, per wavefront
-        constexpr int ABYTES = BM * AROW, STAGE = ABYTES + BN * TILE_K * 2;
+        constexpr int ABYTES = BM * AROW, WBYTES = BN * TILE_K * 2, WBASE = STAGES * KG * ABYTES; // a turn's, where W's turns begin
         static_assert(BM % (AROWS * NW) == 0 && BN % (8 * NW) == 0 && TM >= 1 && TN >= 1, "whole loads and products");
-        static_assert(STAGES >= 2 && (STAGES - 1) * LOADS < 64, "counted by six bits");
+        static_assert(STAGES >= 2 && (WSTAGES == STAGES || WSTAGES == STAGES + 1) && (WSTAGES - 1) * LOADS < 64, "counted by six bits");
         extern __shared__ __attribute__((aligned(16))) char smem[];
         const int lane = threadIdx.x & 63, all = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
         const int kg = KG == 1 ? 0 : all / NW, wave = KG == 1 ? all : all % NW;
@@ -299,8 +299,7 @@ namespace llamql
         const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)smem;
         // load i of turn t into its buffer; a group without a turn t reads its last one again, which nothing uses
         auto issue = [&](int i, int buf, int t) __attribute__((always_inline)) {
-            const uint32_t at = lds0 + (buf * KG + kg) * STAGE + wave * 1024;
-            load_to_lds(src[i], at + (i < ALOADS ? i * NW * 1024 : ABYTES + (i - ALOADS) * NW * 1024));
+            load_to_lds(src[i], lds0 + wave * 1024 + (i < ALOADS ? (buf * KG + kg) * ABYTES + i * NW * 1024 : WBASE + (buf * KG + kg) * WBYTES + (i - ALOADS) * NW * 1024));
             if (KG == 1 || (t + 1) * KG + kg < count)
                 src[i] += KG * (i < ALOADS ? AROW : 2048);
         };
@@ -315,25 +314,24 @@ namespace llamql
                     acc[j][i][r] = 0.0f;
 
 #pragma unroll
-        for (int t = 0; t < STAGES; ++t)
+        for (int t = 0; t < WSTAGES; ++t)
             if (t < rounds)
             {
 #pragma unroll
-                for (int i = 0; i < LOADS; ++i)
+                for (int i = t < STAGES ? 0 : ALOADS; i < LOADS; ++i)
                     issue(i, t, t);
             }
-        const int arow = (wm * TM * 32 + c) * AROW, wrow = ABYTES + (wn * TN * 2 + (c >> 4)) * 2048 + (h * 16 + (c & 15)) * 16;
+        const int arow = (wm * 32 + c) * AROW, wrow = WBASE + (wn * TN * 2 + (c >> 4)) * 2048 + (h * 16 + (c & 15)) * 16;
         typename O::Raw a[2][TM];
         bf16x8 w[2][TN];
         // operand n of the 16 columns s of a stage (k-step s / 2 of W, its pieces 2 (s & 1) + h): A's first, W's, A's others
-        auto read = [&](int buf, int s, int b, int n) __attribute__((always_inline)) {
-            const char *at = smem + (buf * KG + kg) * STAGE;
+        auto read = [&](int buf, int wbuf, int s, int b, int n) __attribute__((always_inline)) {
             if (n >= 1 && n <= TN)
-                w[b][n - 1] = *reinterpret_cast<const bf16x8 *>(at + wrow + (n - 1) * 4096 + (s >> 1) * 1024 + (s & 1) * 512);
+                w[b][n - 1] = *reinterpret_cast<const bf16x8 *>(smem + (wbuf * KG + kg) * WBYTES + wrow + (n - 1) * 4096 + (s >> 1) * 1024 + (s & 1) * 512);
             else
             {
                 const int i = n == 0 ? 0 : n - TN;
-                const char *row = at + arow + i * 32 * AROW;
+                const char *row = smem + (buf * KG + kg) * ABYTES + arow + i * WM * 32 * AROW;
                 if constexpr (sizeof(T) == 2)
                     a[b][i] = *reinterpret_cast<const bf16x8 *>(row + ((2 * s + h) ^ swizzle(c)) * 16);
                 else
@@ -341,68 +339,85 @@ namespace llamql
                                                       *reinterpret_cast<const f32x4 *>(row + ((4 * s + 2 * h + 1) ^ swizzle(c)) * 16), 0, 1, 2, 3, 4, 5, 6, 7);
             }
         };
-        // the products of the operands b, in this order, with what `between` asks for after each: left to itself the
-        // compiler asks for operands just before it needs them
-        auto multiply = [&](int b, auto between) __attribute__((always_inline)) {
+        // all turns, with the first `strips` of the wavefront's TM strips of 32 rows
+        auto walk = [&](auto strips) __attribute__((always_inline)) {
+            constexpr int L = decltype(strips)::value;
+            // the products of the operands b, in this order, with what `between` asks for after each: left to itself the
+            // compiler asks for operands just before it needs them
+            auto multiply = [&](int b, auto between) __attribute__((always_inline)) {
 #pragma unroll
-            for (int i = 0; i < TM; ++i)
-            {
-                bf16x8 piece[O::PIECES];
-                O::pieces(a[b][i], piece);
-#pragma unroll
-                for (int j = 0; j < TN; ++j)
+                for (int i = 0; i < L; ++i)
                 {
+                    bf16x8 piece[O::PIECES];
+                    O::pieces(a[b][i], piece);
 #pragma unroll
-                    for (int k = O::PIECES - 1; k >= 0; --k)
-                        acc[j][i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[b][j], piece[k], acc[j][i], 0, 0, 0);
-                    __builtin_amdgcn_sched_barrier(0);
-                    between(i * TN + j);
-                    __builtin_amdgcn_sched_barrier(0);
+                    for (int j = 0; j < TN; ++j)
+                    {
+#pragma unroll
+                        for (int k = O::PIECES - 1; k >= 0; --k)
+                            acc[j][i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[b][j], piece[k], acc[j][i], 0, 0, 0);
+                        __builtin_amdgcn_sched_barrier(0);
+                        between(i * TN + j);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
                 }
-            }
-        };
-        // f(0) .. f(count - 1), dealt to the products
-        auto deal = [&](int n, auto f, int count) __attribute__((always_inline)) {
-            const int each = (count + TN * TM - 1) / (TN * TM);
+            };
+            // f(0) .. f(count - 1), dealt to the products
+            auto deal = [&](int n, auto f, int count) __attribute__((always_inline)) {
+                const int each = (count + TN * L - 1) / (TN * L);
 #pragma unroll
-            for (int k = 0; k < 16; ++k)
-                if (k < each && n * each + k < count)
-                    f(n * each + k);
-        };
-        if (rounds >= STAGES)
-            arrive<(STAGES - 1) * LOADS>();
-        else
-            arrive<0>();
-#pragma unroll
-        for (int n = 0; n < TM + TN; ++n)
-            read(0, 0, 0, n);
-        int buf = 0;
-        for (int t = 0; t < rounds - 1; ++t)
-        {
-            const int next = buf + 1 < STAGES ? buf + 1 : 0;
-#pragma unroll
-            for (int s = 0; s < 3; ++s)
-                multiply(s & 1, [&](int n) { deal(n, [&](int k) { read(buf, s + 1, (s + 1) & 1, k); }, TM + TN); });
-            // this stage is in registers; the next one has arrived, later ones may be on their way
-            if (t + STAGES <= rounds)
-                arrive<(STAGES - 2) * LOADS>();
+                for (int k = 0; k < 16; ++k)
+                    if (k < each && n * each + k < count)
+                        f(n * each + k);
+            };
+            if (rounds >= WSTAGES)
+                arrive<(STAGES - 1) * LOADS + (WSTAGES - STAGES) * WLOADS>();
             else
                 arrive<0>();
-            const bool more = t + STAGES < rounds;
-            multiply(1, [&](int n) {
-                deal(n, [&](int k) { read(next, 0, 0, k); }, TM + TN);
-                if (more)
-                    deal(n, [&](int k) { issue(k, buf, t + STAGES); }, LOADS);
-            });
-            buf = next;
-        }
-        if (KG == 1 || (rounds - 1) * KG + kg < count)
-        {
 #pragma unroll
-            for (int s = 0; s < 3; ++s)
-                multiply(s & 1, [&](int n) { deal(n, [&](int k) { read(buf, s + 1, (s + 1) & 1, k); }, TM + TN); });
-            multiply(1, [](int) {});
-        }
+            for (int n = 0; n < L + TN; ++n)
+                read(0, 0, 0, 0, n);
+            int buf = 0, wbuf = 0;
+            for (int t = 0; t < rounds - 1; ++t)
+            {
+                const int next = buf + 1 < STAGES ? buf + 1 : 0, wnext = wbuf + 1 < WSTAGES ? wbuf + 1 : 0;
+#pragma unroll
+                for (int s = 0; s < 3; ++s)
+                    multiply(s & 1, [&](int n) { deal(n, [&](int k) { read(buf, wbuf, s + 1, (s + 1) & 1, k); }, L + TN); });
+                // this stage is in registers; the next one has arrived, later ones may be on their way
+                if (t + WSTAGES <= rounds)
+                    arrive<(STAGES - 2) * LOADS + (WSTAGES - STAGES) * WLOADS>();
+                else
+                    arrive<0>();
+                const bool more = t + STAGES < rounds, wmore = t + WSTAGES < rounds;
+                multiply(1, [&](int n) {
+                    deal(n, [&](int k) { read(next, wnext, 0, 0, k); }, L + TN);
+                    deal(n, [&](int k) {
+                        if (k < ALOADS ? more : wmore)
+                            issue(k, k < ALOADS ? buf : wbuf, t + (k < ALOADS ? STAGES : WSTAGES));
+                    }, LOADS);
+                });
+                buf = next, wbuf = wnext;
+            }
+            if (KG == 1 || (rounds - 1) * KG + kg < count)
+            {
+#pragma unroll
+                for (int s = 0; s < 3; ++s)
+                    multiply(s & 1, [&](int n) { deal(n, [&](int k) { read(buf, wbuf, s + 1, (s + 1) & 1, k); }, L + TN); });
+                multiply(1, [](int) {});
+            }
+        };
+        // strips past the last row are left out: a wavefront's strips lie WM apart, so all wavefronts have about as many.  (64 experts
+        // of 52 to 87 rows, tiles of 256 x 128: 1408 x 2048 103 -> 83 us; the matrix unit is also what the clock goes down for.)
+        const int strips = __builtin_amdgcn_readfirstlane((rows - mt * BM + (WM - 1 - wm) * 32 + 31) / (WM * 32));
+        if (TM > 3 && strips == 3)
+            walk(std::integral_constant<int, (TM > 3 ? 3 : TM)>());
+        else if (TM > 2 && strips == 2)
+            walk(std::integral_constant<int, (TM > 2 ? 2 : TM)>());
+        else if (TM > 1 && strips < 2)
+            walk(std::integral_constant<int, 1>());
+        else
+            walk(std::integral_constant<int, TM>());
 
         if constexpr (KG > 1)
         {
@@ -457,7 +472,7 @@ namespace llamql
 #pragma unroll
                 for (int i = 0; i < TM; ++i)
                 {
-                    int m = mt * BM + (wm * TM + i) * 32 + c;
+                    int m = mt * BM + (wm + i * WM) * 32 + c;
                     m = row0 + (m < rows ? m : rows - 1);
                     if (p.row_source)
                         m = p.row_source[m] / p.source_div;
@@ -533,7 +548,7 @@ namespace llamql
 #pragma unroll
             for (int j = 0; j < TN; ++j)
                 strip[j] = acc[j][i];
-            results<T>(p, p.group_offset ? 0 : z, strip, own, lane, mt * BM + (wm * TM + i) * 32, rows, row0, nt * BN + wn * TN * 32);
+            results<T>(p, p.group_offset ? 0 : z, strip, own, lane, mt * BM + (wm + i * WM) * 32, rows, row0, nt * BN + wn * TN * 32);
         }
     }
 
@@ -581,20 +596,20 @@ namespace llamql
             add(std::integral_constant<int, 2>(), k), k += 2;
         if (k < p.slices)
             add(std::integral_constant<int, 1>(), k);
-        results<T>(p, 0, strip, smem + here * (TN * OUT_BYTES), lane, mt * BM + (wave % WM * TM + i) * 32, p.M, 0, nt * BN + wave / WM * TN * 32);
+        results<T>(p, 0, strip, smem + here * (TN * OUT_BYTES), lane, mt * BM + (wave % WM + i * WM) * 32, p.M, 0, nt * BN + wave / WM * TN * 32);
     }
 
     namespace
     {
-        template <typename T, int BM, int BN, int WM, int WN, int KG, int STAGES>
+        template <typename T, int BM, int BN, int WM, int WN, int KG, int STAGES, int WSTAGES = STAGES>
         bool wide_launch(const char *fn, const LinearArgs &a, int batch, hipStream_t st)
         {
             static LdsGrant grant;
-            constexpr size_t stages = (size_t)STAGES * KG * (BM * sizeof(T) + BN * 2) * TILE_K, sums = (size_t)(KG - 1) * BM * BN * 4;
+            constexpr size_t stages = (size_t)KG * (STAGES * BM * sizeof(T) + WSTAGES * BN * 2) * TILE_K, sums = (size_t)(KG - 1) * BM * BN * 4;
             static_assert(KG > 1 || stages >= (size_t)WM * BN * OUT_BYTES / 32, "the results' place");
             constexpr size_t lds = stages > sums ? stages : sums;
             static_assert(lds <= 160 * 1024, "stages must fit the LDS");
-            const auto kernel = &linear_wide_kernel<T, BM, BN, WM, WN, KG, STAGES, false>;
+            const auto kernel = &linear_wide_kernel<T, BM, BN, WM, WN, KG, STAGES, WSTAGES, false>;
             if (lds > 64 * 1024 && allow_lds(grant, reinterpret_cast<const void *>(kernel), lds) != hipSuccess)
                 return fail(fn, "cannot reserve %zu bytes of LDS", lds);
             const int nt = ceil_div(a.N, BN);
@@ -607,13 +622,13 @@ namespace llamql
         }
 
         // The same with the tiles from a.full on in a.slices slices of K each, which a second launch joins.
-        template <typename T, int BM, int BN, int WM, int WN, int KG, int STAGES>
+        template <typename T, int BM, int BN, int WM, int WN, int KG, int STAGES, int WSTAGES = STAGES>
         bool split_launch(const char *fn, const LinearArgs &a, hipStream_t st)
         {
             static LdsGrant grant;
-            constexpr size_t stages = (size_t)STAGES * KG * (BM * sizeof(T) + BN * 2) * TILE_K, sums = (size_t)(KG - 1) * BM * BN * 4;
+            constexpr size_t stages = (size_t)KG * (STAGES * BM * sizeof(T) + WSTAGES * BN * 2) * TILE_K, sums = (size_t)(KG - 1) * BM * BN * 4;
             constexpr size_t lds = stages > sums ? stages : sums;
-            const auto kernel = &linear_wide_kernel<T, BM, BN, WM, WN, KG, STAGES, true>;
+            const auto kernel = &linear_wide_kernel<T, BM, BN, WM, WN, KG, STAGES, WSTAGES, true>;
             if (lds > 64 * 1024 && allow_lds(grant, reinterpret_cast<const void *>(kernel), lds) != hipSuccess)
                 return fail(fn, "cannot reserve %zu bytes of LDS", lds);
             const int nt = ceil_div(a.N, BN), mt = ceil_div(a.M, BM), split = mt * nt - a.full;
@@ -641,8 +656,11 @@ namespace llamql
         // the best in the mean, 15 % at most (1000 rows, 2 of 16 experts of 1536 x 5120, up: 210 and 182 us); fp32 0.6 %, 15 %.
         // 187 rows, 6 of 64 experts of 1408 x 2048 and a shared one: bf16 209 -> 190 us against two tiles by the mean
         // rows of a group, fp32 369 -> 267 against tiles as if every group had all rows.
+        // 256 x 256 has a third turn of W in its LDS, for that is what comes from memory, where A mostly comes from the cache: 64 experts of 155 to
+        // 217 rows, 2048 x 1408 108 -> 105 us, 1536 x 5120 287 -> 263, 2048 x 5120 x 30720 662 -> 645; the tile that such experts had, 128 x 128
+        // by four wavefronts, takes 129 and 297.  (A third turn of W for the others, of 256 x 128 a fourth: no faster.)
         const Tile TILES_BF16[] = {
-            {256, 256, 1, 1, 1.30f, 1.70f, 4.0f, wide_launch<bf16, 256, 256, 2, 4, 1, 2>, split_launch<bf16, 256, 256, 2, 4, 1, 2>},
+            {256, 256, 1, 1, 1.15f, 1.45f, 4.0f, wide_launch<bf16, 256, 256, 2, 4, 1, 2, 3>, split_launch<bf16, 256, 256, 2, 4, 1, 2, 3>},
             {256, 128, 1, 1, 0.75f, 1.00f, 4.0f, wide_launch<bf16, 256, 128, 4, 2, 1, 3>, split_launch<bf16, 256, 128, 4, 2, 1, 3>},
             {128, 128, 1, 2, 0.65f, 1.05f, 4.0f, wide_launch<bf16, 128, 128, 2, 2, 1, 2>, nullptr},
             {128, 128, 1, 1, 0.57f, 0.60f, 3.0f, wide_launch<bf16, 128, 128, 4, 2, 1, 3>, split_launch<bf16, 128, 128, 4, 2, 1, 3>},

@@ -191,7 +191,7 @@ def test_rows_that_start_at_eight_bytes(dev, M, N, K, out):
 
 # every tile that is cut, with and without whole ones beside it, slices of unequal length (test_launch_rules.py)
 SPLIT = [(17, 48, 2112), (33, 80, 1024), (65, 2064, 8256), (257, 2064, 8256), (1000, 16400, 512), (700, 6160, 8256), (2048, 4112, 2112),
-         (65, 2064, 1024), (2048, 272, 4160), (1500, 6160, 512), (200, 4112, 4160)]
+         (65, 2064, 1024), (2048, 272, 4160), (2048, 1280, 8256), (1500, 6160, 512), (200, 4112, 4160)]
 
 
 def run_within(torch, a, w, y, dtype, out=sq.OUT_F32, N=None, K=None, bias=None, short=0):
