@@ -541,6 +541,49 @@ namespace llamql
         }
     }
 
+    // The same of up to MOST stretches: DV / 4 threads a row, a row's stretches asked for together (2048 tokens of 16 heads of 128, two
+    // stretches: 62 -> 10 us)
+    template <typename T, int DV, int MOST>
+    __global__ void __launch_bounds__(ATT_THREADS)
+        attention_merge_few_kernel(AttentionArgs p)
+    {
+        typedef T t4 __attribute__((ext_vector_type(4)));
+        constexpr int LANES = DV / 4, ROWS = ATT_THREADS / LANES;
+        const int ei = blockIdx.y / p.groups, kv = blockIdx.y - ei * p.groups, e = p.first + ei;
+        const int row = blockIdx.x * ROWS + threadIdx.x / LANES, d = threadIdx.x % LANES * 4;
+        const int per = p.heads / p.groups;
+        const AttentionCut cut = attention_cut(p, ei);
+        if (row >= p.ntok[e] * per || cut.nsplit == 1)
+            return;
+        const int tok = row / per, pos0 = p.pos[e];
+        const int low = att_low(pos0 + row / p.block_rows * p.block_rows / per, p.chunk); // of the row's block
+        int used = (pos0 + tok - low) / cut.stretch + 1;
+        used = used < cut.nsplit ? used : cut.nsplit;
+        const size_t at = cut.first + (size_t)kv * cut.nsplit * cut.rows + row;
+        float m[MOST], l[MOST], M = -INFINITY, L = 0.0f;
+        f32x4 o[MOST], y = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int s = 0; s < MOST; ++s)
+        {
+            const size_t k = at + (size_t)(s < used ? s : 0) * cut.rows;
+            m[s] = s < used ? p.part_ml[k * 2] : -INFINITY, l[s] = p.part_ml[k * 2 + 1];
+            o[s] = *reinterpret_cast<const f32x4 *>(p.part_o + k * DV + d);
+            M = fmaxf(M, m[s]);
+        }
+        const float base = M == -INFINITY ? 0.0f : M;
+#pragma unroll
+        for (int s = 0; s < MOST; ++s)
+        {
+            const float f = s < used ? expf(m[s] - base) : 0.0f;
+            L += s < used ? f * l[s] : 0.0f;
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                y[j] += s < used ? o[s][j] * f : 0.0f;
+        }
+        T *out = static_cast<T *>(p.o) + (size_t)(p.row0[e] + tok) * p.ldo + (size_t)(kv * per + row - tok * per) * DV;
+        *reinterpret_cast<t4 *>(out + d) = __builtin_convertvector(y * (1.0f / L), t4);
+    }
+
     // ---- rotary positions, cache rows ---------------------------------------------------------------
     struct RotaryArgs
     {
@@ -667,7 +710,16 @@ namespace llamql
                 ok = attention_launch<T, DK, DV, 4, RG>(fn, p, row_blocks, z, st);
             if (!ok || p.nsplit == 1)
                 return ok;
-            hipLaunchKernelGGL((attention_merge_kernel<T, DV>), dim3(p.rcap, z), dim3(ATT_THREADS), 0, st, p);
+            // (a workgroup for every row pays where a row has many stretches)
+            const dim3 rows(ceil_div(p.rcap, ATT_THREADS / (DV / 4)), z);
+            if (p.nsplit <= 2)
+                hipLaunchKernelGGL((attention_merge_few_kernel<T, DV, 2>), rows, dim3(ATT_THREADS), 0, st, p);
+            else if (p.nsplit <= 4)
+                hipLaunchKernelGGL((attention_merge_few_kernel<T, DV, 4>), rows, dim3(ATT_THREADS), 0, st, p);
+            else if (p.nsplit <= 8)
+                hipLaunchKernelGGL((attention_merge_few_kernel<T, DV, 8>), rows, dim3(ATT_THREADS), 0, st, p);
+            else
+                hipLaunchKernelGGL((attention_merge_kernel<T, DV>), dim3(p.rcap, z), dim3(ATT_THREADS), 0, st, p);
             return launched(fn);
         }
         template <typename T, int DK, int DV>

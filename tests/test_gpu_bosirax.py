@@ -101,6 +101,15 @@ def test_attention_of_many_entries(dev, dtype):
     attend(dev, dtype, 4, 2, 64, 128, 9, 0, 120, None, 5)
 
 
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("vdim", [64, 128, 256])
+@pytest.mark.parametrize("length", [120, 128, 129, 200, 260, 500, 512, 513, 577, 700])
+def test_attention_in_few_stretches(dev, length, vdim, dtype):
+    """Two to nine stretches and more, which are merged otherwise: rows that see all of them and rows that see the first alone."""
+    attend(dev, dtype, 6, 2, 64, vdim, 70, 0, length - 70)
+    attend(dev, dtype, 2, 2, 64, vdim, 41, 300, length - 41)
+
+
 def test_attention_refuses_what_the_cache_does_not_hold():
     L = sequence.load()
     a = sequence.AttentionArgs(4, 2, 64, 64, 128, 100, 1.0, 1 << 20, 1 << 20)
