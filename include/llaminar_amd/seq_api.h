@@ -72,6 +72,9 @@ size_t llam_seq_linear_scratch_bytes(int max_rows, int N, int K, int dtype, int 
 bool llam_seq_linear_within(const llam_seq_linear_args *a, void *d_scratch, size_t scratch_bytes, int dtype, int device_id,
                             void *stream);
 
+/* `batch` tiled matrices of N rows and K columns, one behind the other, as those of K rows and N columns; N and K multiples of 32. */
+bool llam_seq_transpose_tiles(const void *d_w, void *d_out, int N, int K, int batch, int device_id, void *stream);
+
 /* Two linear layers over the same M rows with the same K and nothing in common otherwise (the two
  * branches of a parallel layer), unbatched: up to 16 rows in one launch.  Both have d_norm or none has. */
 bool llam_seq_linear_pair(const llam_seq_linear_args *a, const llam_seq_linear_args *b, int dtype, int device_id,

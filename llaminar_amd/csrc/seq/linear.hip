@@ -502,3 +502,37 @@ extern "C" bool llam_seq_linear_pair(const llam_seq_linear_args *a, const llam_s
         return dtype == LLAM_SEQ_F32 ? small_pair_dispatch<float>(fn, p, q, st) : small_pair_dispatch<bf16>(fn, p, q, st);
     return linear_tiled(fn, p, 1, dtype, device_id, st) && linear_tiled(fn, q, 1, dtype, device_id, st);
 }
+
+namespace
+{
+    // Eight values of an inner row of the turned matrix a thread
+    __global__ void __launch_bounds__(256)
+        transpose_tiles_kernel(const bf16 *__restrict__ w, bf16 *__restrict__ out, int N, int K)
+    {
+        const int piece = blockIdx.x * 256 + threadIdx.x;
+        if (piece >= N * K / 8)
+            return;
+        const int lane = piece & 63, tile = piece >> 6, steps = N >> 5; // of the turned matrix, [K/16][N/32][64]
+        const int k = tile / steps * 16 + (lane & 15), n0 = tile % steps * 32 + 8 * (lane >> 4);
+        const bf16 *from = w + (size_t)blockIdx.y * N * K + ((size_t)(n0 >> 4) * (K >> 5) + (k >> 5)) * 512 + ((k & 31) >> 3) * 128 + (n0 & 15) * 8 + (k & 7);
+        bf16x8 v;
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+            v[e] = from[e * 8];
+        *reinterpret_cast<bf16x8 *>(out + (size_t)blockIdx.y * N * K + (size_t)piece * 8) = v;
+    }
+} // namespace
+
+extern "C" bool llam_seq_transpose_tiles(const void *d_w, void *d_out, int N, int K, int batch, int device_id, void *stream)
+{
+    static const char *fn = "llam_seq_transpose_tiles";
+    if (N < 1 || K < 1 || N % 32 != 0 || K % 32 != 0 || batch < 1 || batch > 65535 || (long)N * K > 0x7fffffff)
+        return fail(fn, "bad size (N=%d K=%d batch=%d)", N, K, batch);
+    if (!d_w || !d_out || !aligned16(d_w) || !aligned16(d_out))
+        return fail(fn, "null or misaligned pointer");
+    if (!set_device(fn, device_id))
+        return false;
+    hipLaunchKernelGGL(transpose_tiles_kernel, dim3(ceil_div(N * (K / 8), 256), batch), dim3(256), 0, as_stream(stream), static_cast<const bf16 *>(d_w),
+                       static_cast<bf16 *>(d_out), N, K);
+    return launched(fn);
+}

@@ -85,6 +85,7 @@ namespace
         float *x = nullptr, *in = nullptr, *z = nullptr, *logits = nullptr, *lat_scratch = nullptr;
         void *h = nullptr, *h2 = nullptr, *q = nullptr, *qlat = nullptr, *olat = nullptr, *mix = nullptr, *act = nullptr;
         void *scratch = nullptr, *arg_scratch = nullptr;
+        int32_t *none = nullptr; // a zero for each slot
         size_t lat_floats = 0, scratch_bytes = 0;
         // integers of a step: ids, slot and position per row; first row, tokens, slot, position per entry; wanted rows
         int32_t *meta = nullptr, *h_meta = nullptr, *best = nullptr, *ring = nullptr, *count = nullptr;
@@ -143,12 +144,58 @@ namespace
         llam_seq_entries entries() const { return {entry(0), entry(1), entry(2), entry(3)}; }
     };
 
+    // Where keys and values made from latent rows lie in the scratch, behind the turned W_uk
+    struct LatentExpansion
+    {
+        size_t keys, values, bytes;
+    };
+    LatentExpansion latent_expansion(const llam_seqm_layer &w, int len, int elem)
+    {
+        const size_t H = w.heads, ring = pad(len, 128);
+        LatentExpansion at;
+        at.keys = H * P(w.dim) * P(w.kv_rank) * 2;
+        at.values = at.keys + H * ring * P(w.dim) * elem;
+        at.bytes = at.values + H * ring * P(w.vdim) * elem;
+        return at;
+    }
+    // Attending in latent space takes sums of kv_rank for every score and every output column, twice for outputs of two pieces, where
+    // keys and values of every head take sums of the head's width, but have to be made from every latent row first.  Worth it from
+    // so many multiplications on (one portion, us a layer with its projections, in latent space and expanded):
+    //   16 heads of 128, rank 512, bf16, width 2048: 251 tokens 76, 74; 512 94, 84; 1024 157, 122; 2048 277, 202; 512 at 1536 138, 112; 512 at
+    //   7680 313, 197; 128 at 1920 85, 89; 128 at 8064 127, 139; 64 at 8128 102, 134
+    //   64 heads, width 5120: 100 tokens 112, 106; 251 167, 143; 512 221, 196; 1024 437, 309; 2048 1052, 677; 128 at 1920 178, 185; 64 at 8128 222, 374
+    //   16 heads, fp32: 100 tokens 110, 96; 200 139, 106; 512 275, 137; 2048 1606, 556; 128 at 1920 247, 138
+    // (Portions in latent space share launches, expanded ones do not: the line lies where a portion gains some 10 us alone.)  A portion's own sizes
+    // decide, so that its outputs do not depend on those beside it.
+    bool latent_gains(const llam_seqm_layer &w, int ntok, int len, int dtype)
+    {
+        const double dp = P(w.dim), vp = P(w.vdim), rp = P(w.kv_rank), pieces = dtype == LLAM_SEQ_F32 ? 1 : 2;
+        const double saved = ntok * (len - 0.5 * ntok) * (rp - dp + pieces * (rp - vp)) - (double)(len - ntok) * (dp + vp) * rp;
+        return ntok > ROW_MAX && saved * w.heads > (dtype == LLAM_SEQ_F32 ? 0.2e9 : 3.0e9);
+    }
+    constexpr size_t EXPANSION_BYTES = (size_t)320 << 20; // at most
+    bool latent_expands(const llam_seqm_layer &w, int ntok, int len, int dtype, size_t scratch_bytes)
+    {
+        const int dp = P(w.dim), vp = P(w.vdim);
+        const auto head_size = [](int n) { return n == 64 || n == 128 || n == 256; }; // of the attention kernels
+        const size_t need = latent_expansion(w, len, dtype == LLAM_SEQ_F32 ? 4 : 2).bytes;
+        return head_size(dp) && head_size(vp) && need <= EXPANSION_BYTES && need <= scratch_bytes && latent_gains(w, ntok, len, dtype);
+    }
+    // what the portions of up to max_rows tokens of sequences of up to cap make use of
+    size_t latent_expansion_bytes(const llam_seqm_layer &w, int max_rows, int cap, int dtype)
+    {
+        for (int len = cap; len > 0; len -= 128)
+            if (latent_expands(w, std::min(max_rows, len), len, dtype, EXPANSION_BYTES))
+                return latent_expansion(w, len, dtype == LLAM_SEQ_F32 ? 4 : 2).bytes;
+        return 0;
+    }
+
     // what a step looks like to the layers: `single` one-token entries first, then the portions, in runs
     struct Step
     {
         int M = 0, single = 0;
         int max_len = 1; // bound on the length of the one-token entries' sequences
-        std::vector<int> ntok, len; // the portions' tokens, and their sequences' lengths afterwards
+        std::vector<int> ntok, len, slot; // the portions' tokens, their sequences' lengths afterwards, and slots
         // runs of portions that the recurrent mixers launch together: entries first .. first + n - 1, the most tokens
         struct Run
         {
@@ -162,9 +209,9 @@ namespace
         // as well: Kogilix 5.1 -> 4.3 ms, Bosirax 3.6 -> 2.7); a grid is made for the longest, so a portion that would leave two
         // thirds of it empty starts a run of its own.  What a portion's outputs are does not depend on its run: every mixer cuts
         // a portion up by its own length.
-        void add(int entry, int tokens, int length)
+        void add(int entry, int tokens, int length, int in)
         {
-            ntok.push_back(tokens), len.push_back(length);
+            ntok.push_back(tokens), len.push_back(length), slot.push_back(in);
             if (!runs.empty())
             {
                 Run &r = runs.back();
@@ -304,20 +351,57 @@ namespace
             if (own && !forward(fn, llam_seq_latent_append(md.in + qp, n_in, w.kv_norm, c.eps, w.kv_rank, s.row_slot, s.row_pos,
                                                            cache, s.M, rp, c.cap, c.dtype, c.device_id, st)))
                 return false;
-            if (!norm_linear(md.in, n_in, w.q_norm, w.q_rank, w.w_uq, H * dp, md.q, H * dp, LLAM_SEQ_OUT_ELEM, s.M) ||
-                !linear(md.q, H * dp, w.w_uk_t, rp, dp, md.qlat, H * rp, LLAM_SEQ_OUT_ELEM, s.M, nullptr, nullptr, 0, nullptr, H,
-                        dp, (long)rp * dp, rp))
+            if (!norm_linear(md.in, n_in, w.q_norm, w.q_rank, w.w_uq, H * dp, md.q, H * dp, LLAM_SEQ_OUT_ELEM, s.M))
                 return false;
             const llam_seq_entries e = md.entries();
-            if (s.single && !forward(fn, llam_seq_latent_attention(md.qlat, cache, &e, 0, s.single, 1, s.max_len, H, rp, c.cap, w.scale,
-                                                                   md.olat, md.lat_scratch, md.lat_floats, c.dtype, c.device_id, st)))
-                return false;
-            if (s.portions() && !forward(fn, llam_seq_latent_portions(md.qlat, cache, &e, s.single, s.portions(), s.ntok.data(), s.len.data(), H, rp, c.cap,
-                                                                      w.scale, md.olat, md.lat_scratch, md.lat_floats, c.dtype, c.device_id, st)))
-                return false;
-            return linear(md.olat, H * rp, w.w_uv, vp, rp, md.mix, mix_columns(w), LLAM_SEQ_OUT_ELEM, s.M, nullptr, nullptr, 0, nullptr, H,
-                          rp, (long)vp * rp, vp) &&
-                   add_output(w, s);
+            std::vector<bool> expanded(s.portions());
+            int left = s.single; // entries that attend in latent space
+            for (int i = 0; i < s.portions(); ++i)
+                left += !(expanded[i] = latent_expands(w, s.ntok[i], s.len[i], c.dtype, md.scratch_bytes));
+            if (left)
+            {
+                if (!linear(md.q, H * dp, w.w_uk_t, rp, dp, md.qlat, H * rp, LLAM_SEQ_OUT_ELEM, s.M, nullptr, nullptr, 0, nullptr, H, dp,
+                            (long)rp * dp, rp))
+                    return false;
+                if (s.single && !forward(fn, llam_seq_latent_attention(md.qlat, cache, &e, 0, s.single, 1, s.max_len, H, rp, c.cap, w.scale,
+                                                                       md.olat, md.lat_scratch, md.lat_floats, c.dtype, c.device_id, st)))
+                    return false;
+                for (int i = 0, n; i < s.portions(); i += n)
+                {
+                    for (n = 1; i + n < s.portions() && expanded[i + n] == expanded[i]; ++n)
+                        ;
+                    if (!expanded[i] && !forward(fn, llam_seq_latent_portions(md.qlat, cache, &e, s.single + i, n, s.ntok.data() + i, s.len.data() + i, H,
+                                                                              rp, c.cap, w.scale, md.olat, md.lat_scratch, md.lat_floats, c.dtype,
+                                                                              c.device_id, st)))
+                        return false;
+                }
+                // (rows of expanded portions hold what lay there: they are written below)
+                if (!linear(md.olat, H * rp, w.w_uv, vp, rp, md.mix, mix_columns(w), LLAM_SEQ_OUT_ELEM, s.M, nullptr, nullptr, 0, nullptr, H,
+                            rp, (long)vp * rp, vp))
+                    return false;
+            }
+            for (int i = 0; i < s.portions(); ++i)
+                if (expanded[i] && !latent_expanded(w, cache, s.single + i, s.ntok[i], s.len[i], s.slot[i]))
+                    return false;
+            return add_output(w, s);
+        }
+
+        // A portion whose keys and values are made from the latent rows for every head
+        bool latent_expanded(const llam_seqm_layer &w, void *cache, int entry, int ntok, int len, int slot)
+        {
+            const int H = w.heads, dp = P(w.dim), vp = P(w.vdim), rp = P(w.kv_rank), ring = pad(len, 128);
+            const LatentExpansion at = latent_expansion(w, len, md.elem);
+            char *uk = static_cast<char *>(md.scratch), *k = uk + at.keys, *v = uk + at.values;
+            const char *rows = static_cast<const char *>(cache) + (size_t)slot * c.cap * rp * md.elem;
+            llam_seq_attention_args a{};
+            a.heads = a.kv_heads = H, a.dim = dp, a.vdim = vp, a.ring = ring, a.scale = w.scale, a.d_k = k, a.d_v = v;
+            llam_seq_entries e = md.entries();
+            e.d_slot = md.none; // (keys and values of this portion alone)
+            return forward(fn, llam_seq_transpose_tiles(w.w_uk_t, uk, rp, dp, H, c.device_id, st)) &&
+                   linear(rows, rp, uk, dp, rp, k, dp, LLAM_SEQ_OUT_ELEM, len, nullptr, nullptr, 0, nullptr, H, 0, (long)dp * rp, (long)ring * dp) &&
+                   linear(rows, rp, w.w_uv, vp, rp, v, vp, LLAM_SEQ_OUT_ELEM, len, nullptr, nullptr, 0, nullptr, H, 0, (long)vp * rp, (long)ring * vp) &&
+                   forward(fn, llam_seq_attention_portions(&a, md.q, &e, entry, 1, &ntok, &len, md.mix, mix_columns(w), md.lat_scratch, md.lat_floats,
+                                                           c.dtype, c.device_id, st));
         }
 
         bool memory(const llam_seqm_layer &w, int index, const Step &s)
@@ -583,6 +667,8 @@ extern "C" bool llam_seqm_set_globals(void *model, const llam_seqm_globals *g)
             q = std::max(q, H * dp);
             lat = std::max(lat, H * rp);
             latf = std::max(latf, llam_seq_latent_scratch_floats(c.max_rows, c.slots, w.heads, (int)rp, c.cap));
+            latf = std::max(latf, llam_seq_attention_scratch_floats((int)vp));
+            scratch = std::max(scratch, latent_expansion_bytes(w, c.max_rows, c.cap, c.dtype));
         }
         else if (w.mixer == LLAM_MIXER_ATTENTION)
         {
@@ -629,6 +715,7 @@ extern "C" bool llam_seqm_set_globals(void *model, const llam_seqm_globals *g)
               (md->z = (float *)md->take(fn, M * z * 4)) && (md->scratch = md->take(fn, scratch)) &&
               (md->lat_scratch = (float *)md->take(fn, latf * 4)) &&
               (md->logits = (float *)md->take(fn, (size_t)std::max(LOGIT_ROWS, c.slots) * md->vp * 4)) &&
+              (md->none = (int32_t *)md->take(fn, (size_t)c.slots * 4)) &&
               (md->arg_scratch = md->take(fn, llam_dec_argmax_scratch_bytes(std::max(LOGIT_ROWS, c.slots), c.vocab))) &&
               (md->meta = (int32_t *)md->take(fn, md->meta_ints() * 4)) &&
               (md->best = (int32_t *)md->take(fn, (size_t)LOGIT_ROWS * 4)) &&
@@ -694,6 +781,9 @@ extern "C" bool llam_seqm_set_globals(void *model, const llam_seqm_globals *g)
             md->slot_bytes += (per + w.heads) * 4;
         }
     }
+    const std::vector<int32_t> zeros(c.slots, 0);
+    if (!hip_ok(fn, "hipMemcpy", hipMemcpy(md->none, zeros.data(), zeros.size() * 4, hipMemcpyHostToDevice)))
+        return false;
     if (!hip_ok(fn, "hipDeviceSynchronize", hipDeviceSynchronize()))
         return false;
     md->ready = true;
@@ -762,7 +852,7 @@ extern "C" bool llam_seqm_forward(void *model, int n, const int32_t *h_slot, con
     for (int e = 0; e < n; ++e)
         if (h_ntok[e] > 1)
         {
-            s.add(placed, h_ntok[e], h_pos[e] + h_ntok[e]);
+            s.add(placed, h_ntok[e], h_pos[e] + h_ntok[e], h_slot[e]);
             place(e);
         }
     s.row_slot = md->row_slot();

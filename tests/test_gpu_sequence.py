@@ -438,3 +438,61 @@ def test_decoding_for_long_replays_several_steps_at_once(whole, dtype):
         runs.append(np.concatenate(out))
     assert np.array_equal(runs[0], runs[1]) and np.array_equal(runs[0], runs[2])
     model.close()
+
+
+# Latent layers whose longer portions make keys and values of every head (sequence_model.cpp: latent_gains): from some 130 tokens on in
+# fp32, 400 in bf16.  The last one's heads are no size that the attention kernels have: it stays in latent space.
+EXPANDED = {
+    "heads of 64": sm.latent(heads=40, dim=24, vdim=40, q_rank=64, kv_rank=330),
+    "heads of 128 and 256": sm.latent(heads=20, dim=100, vdim=200, q_rank=64, kv_rank=600, scale=0.1),
+    "heads of 192": sm.latent(heads=40, dim=130, vdim=40, q_rank=64, kv_rank=330, scale=0.1),
+}
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("name", EXPANDED)
+def test_keys_and_values_of_every_head(name, dtype):
+    """Whole prompts and portions onto earlier ones, latent and expanded in turn, odd sizes, tokens that follow; a second layer on the
+    first one's cache."""
+    shared = sm.latent(kv_from=0, heads=30, dim=50, vdim=64, q_rank=90, scale=0.2)
+    shared["mixer"]["kv_rank"] = EXPANDED[name]["mixer"]["kv_rank"]
+    cfg = sm.config(EXPANDED[name], shared, width=64)
+    t = sm.random_weights(cfg, 5)
+    tokens = tokens_of(cfg, 767)
+    want = so.kogilix(cfg, t.plain(), tokens)
+    model = load(cfg, t, dtype, cap=800, max_rows=767)
+    for cuts in ([767], [450, 1, 316], [3, 129, 635], [20, 500, 17, 229, 1]):
+        check(run(model, 1, tokens, cuts), want, dtype, note=f"{name} {cuts}")
+    model.close()
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_expanded_portions_beside_others(dtype):
+    """A step of portions of both kinds and single tokens: each sequence against itself alone, and the same bits whatever lies beside."""
+    cfg = sm.config(EXPANDED["heads of 64"], width=64)
+    t = sm.random_weights(cfg, 6)
+    model = load(cfg, t, dtype, slots=8, cap=700, max_rows=1600)
+    lengths = [(30, 500), (7, 1), (200, 450), (1, 20), (90, 2), (3, 1), (500, 180)]
+    seqs, plain = [tokens_of(cfg, sum(n), seed=b) for b, n in enumerate(lengths)], t.plain()
+    for k in range(2):
+        logits, row = model.forward([(b, sum(n[:k]), seqs[b][sum(n[:k]):sum(n[:k + 1])]) for b, n in enumerate(lengths)],
+                                    range(sum(n[k] for n in lengths))), 0
+        for b, n in enumerate(lengths):
+            check(logits[row:row + n[k]], so.kogilix(cfg, plain, seqs[b])[sum(n[:k]):sum(n[:k + 1])], dtype, note=f"sequence {b}")
+            row += n[k]
+    got = sm.beside(model, cfg, 100, 500, [[600], [500, 100], [20] * 5 + [500], [300, 300]])
+    for g in got:
+        assert np.array_equal(g[:500], got[0][:500])
+    model.close()
+
+
+@pytest.mark.parametrize("N,K,batch", [(64, 64, 1), (96, 32, 3), (512, 128, 16), (320, 192, 5)])
+def test_tiles_of_the_transposed_matrix(dev, N, K, batch):
+    import torch
+
+    w = torch.randn(batch, N, K, device=dev).bfloat16()
+    tiled = lambda m: m.reshape(batch, m.shape[1] // 16, 16, m.shape[2] // 32, 4, 8).permute(0, 1, 3, 4, 2, 5).contiguous()  # noqa: E731
+    out = torch.zeros(batch * N * K + 8, device=dev).bfloat16()
+    assert sequence.load().llam_seq_transpose_tiles(tiled(w).data_ptr(), out.data_ptr(), N, K, batch, 0, torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    assert torch.equal(out[:-8], tiled(w.transpose(1, 2)).reshape(-1)) and (out[-8:] == 0).all()

@@ -317,3 +317,40 @@ answer([[need(most, N, K, dtype), need(most, N, K, dtype) // 2,
                     assert pieces == whole + rest * slices and 2 <= slices <= 8 and slices <= K // 64
                     assert rest * slices * height * width * 4 <= limit
     assert cut > 50
+
+
+# ---- latent portions with keys and values of every head (sequence_model.cpp: latent_expands) -----------------
+
+LATENT = """
+from llaminar_amd import sequence
+from llaminar_amd.models import kogilix
+from tests import sequence_models as sm, test_gpu_sequence as tg
+def steps(layer, dtype, cap, rows, *portions):
+    cfg = sm.config(layer, width=64)
+    model = sequence.SequenceModel(kogilix.weights(cfg, sm.random_weights(cfg)), 6, cap, rows, dtype)
+    bytes, got = model.device_bytes(), []
+    for p in portions:
+        log()
+        model.forward([(b, at, [1] * n) for b, (at, n) in enumerate(p)], [])
+        got.append([next((k for k in ("transpose_tiles", "latent_attention", "16attention") if k in l[1]), "") for l in log() if l[0] == "launch"])
+    model.close()
+    return bytes, got
+layer = lambda name: tg.EXPANDED[name]
+"""
+
+
+def test_latent_portions_are_expanded_where_it_gains(tmp_path):
+    """By a portion's own size, whatever lies beside it; never where the heads are no size of the attention kernels, or for few tokens."""
+    single, bf16, wide, far, small = fake_hip.run(tmp_path, LATENT + """
+answer([steps(layer("heads of 64"), "float32", 1024, 1024, [(0, 60)], [(0, 400)], [(0, 60), (0, 400), (0, 1), (0, 300), (0, 30)], [(1000, 1)], [(900, 20)]),
+        steps(layer("heads of 64"), "bfloat16", 1024, 1024, [(0, 300)], [(0, 700)], [(300, 500)]),
+        steps(layer("heads of 192"), "bfloat16", 1024, 1024, [(0, 700)]),
+        steps(layer("heads of 64"), "float32", 40000, 1024, [(0, 900)], [(39000, 900)]),
+        steps(layer("heads of 64"), "float32", 1024, 64, [(0, 64)])])""")
+    count = lambda launches: [launches.count(k) for k in ("transpose_tiles", "latent_attention", "16attention")]  # noqa: E731
+    assert [count(l) for l in single[1]] == [[0, 1, 0], [1, 0, 1], [2, 3, 2], [0, 1, 0], [0, 1, 0]]
+    assert [count(l)[0] for l in bf16[1]] == [0, 1, 1]
+    assert [count(l)[0] for l in wide[1]] == [0]
+    # (the keys and values of 40,000 positions would be more than the scratch that is kept for them at most)
+    assert [count(l)[0] for l in far[1]] == [1, 0] and far[0] - single[0] < (320 << 20) + 6 * 39000 * 400 * 4
+    assert [count(l)[0] for l in small[1]] == [0] and small[0] < single[0]
