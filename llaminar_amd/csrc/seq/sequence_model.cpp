@@ -397,9 +397,14 @@ namespace
             a.heads = a.kv_heads = H, a.dim = dp, a.vdim = vp, a.ring = ring, a.scale = w.scale, a.d_k = k, a.d_v = v;
             llam_seq_entries e = md.entries();
             e.d_slot = md.none; // (keys and values of this portion alone)
-            return forward(fn, llam_seq_transpose_tiles(w.w_uk_t, uk, rp, dp, H, c.device_id, st)) &&
-                   linear(rows, rp, uk, dp, rp, k, dp, LLAM_SEQ_OUT_ELEM, len, nullptr, nullptr, 0, nullptr, H, 0, (long)dp * rp, (long)ring * dp) &&
-                   linear(rows, rp, w.w_uv, vp, rp, v, vp, LLAM_SEQ_OUT_ELEM, len, nullptr, nullptr, 0, nullptr, H, 0, (long)vp * rp, (long)ring * vp) &&
+            // of every latent row, without scratch: these layers' matrix and results lie in it
+            const auto of_rows = [&](const void *matrix, int n, void *y) {
+                llam_seq_linear_args l{};
+                l.d_a = rows, l.lda = rp, l.d_w = matrix, l.N = n, l.K = rp, l.d_y = y, l.ldy = n, l.out = LLAM_SEQ_OUT_ELEM, l.M = len;
+                l.batch = H, l.w_stride = (long)n * rp, l.y_stride = (long)ring * n;
+                return forward(fn, llam_seq_linear(&l, c.dtype, c.device_id, st));
+            };
+            return forward(fn, llam_seq_transpose_tiles(w.w_uk_t, uk, rp, dp, H, c.device_id, st)) && of_rows(uk, dp, k) && of_rows(w.w_uv, vp, v) &&
                    forward(fn, llam_seq_attention_portions(&a, md.q, &e, entry, 1, &ntok, &len, md.mix, mix_columns(w), md.lat_scratch, md.lat_floats,
                                                            c.dtype, c.device_id, st));
         }

@@ -445,6 +445,8 @@ def test_decoding_for_long_replays_several_steps_at_once(whole, dtype):
 EXPANDED = {
     "heads of 64": sm.latent(heads=40, dim=24, vdim=40, q_rank=64, kv_rank=330),
     "heads of 128 and 256": sm.latent(heads=20, dim=100, vdim=200, q_rank=64, kv_rank=600, scale=0.1),
+    # (a layer of one head is a plain product, that another caller would have cut along K)
+    "one head": sm.latent(heads=1, dim=50, vdim=60, q_rank=64, kv_rank=900, scale=0.2),
     "heads of 192": sm.latent(heads=40, dim=130, vdim=40, q_rank=64, kv_rank=330, scale=0.1),
 }
 
