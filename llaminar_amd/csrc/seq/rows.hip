@@ -1,6 +1,7 @@
 // Row operators of sequence models: token embedding, RMS norm, and the routed expert
 // feed-forward (choice of experts, grouping of tokens by expert, weighted sum).
 #include "linear.h"
+#include <algorithm>
 #include <climits>
 
 namespace llamql
@@ -138,7 +139,31 @@ namespace llamql
         float *weights; // [M][top + 1]: of the chosen experts, then of the shared one
         bool routed;    // few rows: ids and weights are there already
         void *act;      // T: few rows [M][top * ff + shared_ff], many rows [M * top][ff] then [M][shared_ff]
+        int *lists;     // few rows (see ExpertUse)
     };
+
+    // Few rows: what their choices come to.  A list for every EXPERT_ROWS rows or half as many: the count of the experts that any of them
+    // chose, in a piece of 16 bytes, [most][rows] uses of an expert by a row, in the order of the experts' numbers, and the numbers.
+    constexpr int EXPERT_ROWS = 16;
+    struct ExpertUse
+    {
+        float weight;
+        int act; // where the row's activations begin, and the top bit; without that the row did not choose the expert (and they are another row's)
+    };
+    struct ExpertLists
+    {
+        int rows, most; // rows of a list, experts at most
+        __host__ __device__ size_t ints() const { return 4 + (size_t)most * (rows * 2 + 1) + 3 & ~(size_t)3; }
+        __device__ __forceinline__ int *at(int *lists, int i) const { return lists + i * ints(); }
+        __device__ __forceinline__ ExpertUse *uses(int *list) const { return reinterpret_cast<ExpertUse *>(list + 4); }
+        __device__ __forceinline__ int *numbers(int *list) const { return list + 4 + most * rows * 2; }
+    };
+    ExpertLists expert_lists(int M, int rows, int experts, int top)
+    {
+        const int of = M < rows ? M : rows;
+        return {rows, of * top < experts ? of * top : experts};
+    }
+    __device__ __forceinline__ ExpertUse expert_use(float weight, int act, bool chosen) { return {weight, chosen ? act | (int)0x80000000 : act}; }
 
     // A wavefront per token chooses its experts.
     __global__ void __launch_bounds__(ROW_THREADS)
@@ -160,6 +185,102 @@ namespace llamql
             p.weights[m * (p.top + 1) + p.top] = sigmoidf(z[p.experts]);
     }
 
+    constexpr int EXPERT_WAVES = 8;
+    // The lists of few rows, by one workgroup beside those of the up projections, which need none (by the launch that chooses: 1.8 us more).
+    __device__ __forceinline__ void expert_list(const ExpertArgs &p, int M, ExpertLists lists)
+    {
+        constexpr int THREADS = EXPERT_WAVES * 64, BLOCKS = 64 * ROUTE_MAX / 64; // of experts, 64 in each
+        struct Choice
+        {
+            int id;
+            float weight;
+        };
+        __shared__ Choice s_choice[EXPERT_ROWS * 64];
+        __shared__ int s_count[BLOCKS], s_number[64 * ROUTE_MAX];
+        __shared__ uint8_t s_used[64 * ROUTE_MAX];
+        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+        for (int i = threadIdx.x; i < M * p.top; i += THREADS)
+            s_choice[i] = {p.ids[i], p.weights[i + i / p.top]};
+        for (int first = 0; first < M; first += lists.rows)
+        {
+            int *list = lists.at(p.lists, first / lists.rows);
+            for (int i = threadIdx.x; i < 64 * ROUTE_MAX; i += THREADS)
+                s_used[i] = 0;
+            __syncthreads();
+            const int rows = lists.rows < M - first ? lists.rows : M - first;
+            for (int i = threadIdx.x; i < rows * p.top; i += THREADS)
+                s_used[s_choice[first * p.top + i].id] = 1;
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < BLOCKS / EXPERT_WAVES; ++i)
+            {
+                const unsigned long long used = __ballot(s_used[(i * EXPERT_WAVES + wave) * 64 + lane]);
+                if (lane == 0)
+                    s_count[i * EXPERT_WAVES + wave] = __builtin_popcountll(used);
+            }
+            __syncthreads();
+            int count = 0;
+            for (int i = 0; i < BLOCKS; ++i)
+            {
+                if (i % EXPERT_WAVES == wave)
+                {
+                    const bool is = s_used[i * 64 + lane];
+                    const int place = count + __builtin_popcountll(__ballot(is) & ((1ull << lane) - 1));
+                    if (is)
+                        s_number[place] = lists.numbers(list)[place] = i * 64 + lane;
+                }
+                count += s_count[i];
+            }
+            if (threadIdx.x == 0)
+                list[0] = count;
+            __syncthreads();
+            // a thread for every expert of the list and row, sixteen lanes for one
+            const int n = threadIdx.x & (EXPERT_ROWS - 1), pitch = p.top * p.ff + p.shared_ff;
+            for (int i = threadIdx.x / EXPERT_ROWS; i < ((count + 3) & ~3); i += THREADS / EXPERT_ROWS)
+            {
+                const int id = s_number[i < count ? i : 0];
+                float weight = 0.0f;
+                int at = -1;
+                for (int j = 0; j < p.top; ++j)
+                {
+                    const Choice c = s_choice[(n < rows ? first + n : 0) * p.top + j];
+                    const bool is = n < rows && c.id == id;
+                    weight += is ? c.weight : 0.0f; // (several: logits that are not numbers)
+                    at = is && at < 0 ? j : at;
+                }
+                const unsigned chosen = (unsigned)(__ballot(at >= 0) >> (lane & 48)) & 0xffff;
+                const int lead = (lane & 48) | (__builtin_ctz(chosen | 0x10000) & 15);
+                const int act = (first + n) * pitch + at * p.ff, others = __shfl(act, lead, 64);
+                if (i < count && n < lists.rows)
+                    lists.uses(list)[i * lists.rows + n] = expert_use(weight, at >= 0 ? act : others, at >= 0);
+            }
+            __syncthreads();
+        }
+    }
+    // the list of a single row, by the wavefront that has chosen
+    __device__ __forceinline__ void expert_list_one(const ExpertArgs &p, ExpertLists lists, int lane, int id, float weight)
+    {
+        int place = 0, first = lane;
+        float sum = 0.0f;
+        for (int j = p.top - 1; j >= 0; --j)
+            first = __builtin_amdgcn_readlane(id, j) == id ? j : first;
+        const unsigned long long leads = __ballot(lane < p.top && first == lane);
+        for (int j = 0; j < p.top; ++j)
+        {
+            const int other = __builtin_amdgcn_readlane(id, j);
+            sum += other == id ? __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, weight), j)) : 0.0f;
+            place += (leads >> j & 1) != 0 && other < id ? 1 : 0;
+        }
+        if ((leads >> lane & 1) != 0)
+        {
+            for (int n = 0; n < lists.rows; ++n)
+                lists.uses(p.lists)[place * lists.rows + n] = expert_use(sum, lane * p.ff, n == 0);
+            lists.numbers(p.lists)[place] = id;
+        }
+        if (lane == 0)
+            p.lists[0] = __builtin_popcountll(leads);
+    }
+
     // Few rows.  Workgroup = 16 outputs of one expert, for every token that chose it: the tokens are the columns of the
     // matrix unit's second operand, so an expert's weights are read once however many chose it (the shared one: all).  Of
     // the workgroups of a (token, choice) pair those of the first token to choose the expert work, the others end.
@@ -167,10 +288,9 @@ namespace llamql
     // the choice for the down projections; with more, a launch before has chosen.
     // Bound by the weights: 8 tokens, 6 of 64 experts of 1408 x 2048 each and a shared one of 2816, 56 us when each token
     // read its own and 44 now (about 200 MB of distinct weights).  The bits are the same: columns do not meet.
-    constexpr int EXPERT_WAVES = 8;
     template <typename T>
     __global__ void __launch_bounds__(EXPERT_WAVES * 64)
-        expert_up_small_kernel(ExpertArgs p, int M)
+        expert_up_small_kernel(ExpertArgs p, int M, ExpertLists lists)
     {
         using O = Operand<T>;
         typedef T t4 __attribute__((ext_vector_type(4)));
@@ -184,6 +304,8 @@ namespace llamql
         unsigned long long mine = n < M ? 1 : 0; // which of token n's choices the expert is (several: logits that are not numbers)
         if (shared)
         {
+            if (m == 1 && tile == 0)
+                expert_list(p, M, lists);
             if (m > 0 || tile * 16 >= p.shared_ff)
                 return;
         }
@@ -208,11 +330,7 @@ namespace llamql
             route_wave(z, p.experts, p.top, lane, id, weight);
             if (tile == 0 && job == 0 && wave == 0)
             {
-                if (lane < p.top)
-                {
-                    p.ids[m * p.top + lane] = id;
-                    p.weights[m * (p.top + 1) + lane] = weight;
-                }
+                expert_list_one(p, lists, lane, id, weight);
                 if (lane == 0 && p.shared_ff)
                     p.weights[m * (p.top + 1) + p.top] = sigmoidf(z[p.experts]);
             }
@@ -265,68 +383,135 @@ namespace llamql
         }
     }
 
-    // Workgroup = 16 columns of one token's output over all its experts: the k-steps of all of them
-    // in one list, dealt to the wavefronts.
-    template <typename T>
-    __global__ void __launch_bounds__(EXPERT_WAVES * 64)
-        expert_down_small_kernel(ExpertArgs p)
+    // Few rows.  Workgroup = 8 columns of the output, or 16, of up to as many rows and over all experts that any of these chose: the shared
+    // one, then those of the list, so that an expert's weights are read once however many rows chose it.  The k-steps of an expert
+    // are taken in twos and dealt to the wavefronts, beginning with another one for every expert; a row's sums are of its own
+    // experts, in the order of their numbers, so its bits are the same whatever other rows there are, also none.
+    // HALF: rows 8 .. of the matrix unit's first operand are the same columns' second k-step of the two, and columns 8 .. of the
+    // second operand the rows' (see linear_small_tile): twice the workgroups, and one product where there were two.
+    // Bound by the weights, and for one or two rows by the chain of list, first weights and sums.  A layer of 6 of 64 experts of 1408 x 2048 and a
+    // shared one of 2816, us, against a workgroup for every row that read its own experts: 8 rows that choose alike (12 experts in all) bf16
+    // 63.8 -> 45.2, fp32 108 -> 61; that choose evenly (35) 95.7 -> 86.8, 142 -> 126; 16 rows 156 -> 135; 1 row 25.7 -> 24.0, fp32 41.1 -> 33.2.
+    // 16 rows at 1536 x 5120: 423 -> 332.  Slower only where small experts are hardly shared: 4 rows, 8 of 128 of 768 x 2048 45.7 -> 48.9, fp32 58 -> 65.
+    template <typename T, bool HALF>
+    __global__ void __launch_bounds__(EXPERT_WAVES * 64, 4)
+        expert_down_small_kernel(ExpertArgs p, int M, ExpertLists lists)
     {
         using O = Operand<T>;
         using V = typename O::V;
-        __shared__ __attribute__((aligned(16))) float s_red[EXPERT_WAVES][64][4];
-        const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4;
-        const int tile = blockIdx.x, m = blockIdx.y;
-        const int esteps = p.ff >> 5, ssteps = p.shared_ff >> 5;
-        const int total = p.top * esteps + ssteps;
-        // lane j: the expert of choice j and its weight
-        const int own_id = lane < p.top ? p.ids[m * p.top + lane] : 0;
-        const float own_weight = lane < p.top ? p.weights[m * (p.top + 1) + lane] : 0.0f, shared_weight = p.weights[m * (p.top + 1) + p.top];
-        const T *act = static_cast<const T *>(p.act) + (size_t)m * (p.top * p.ff + p.shared_ff) + 8 * g;
-        f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-        constexpr int U = 8;
-        // the wavefront's place in the list: step s is step `in` of expert `job` (scalars: as vector code, with the experts in LDS,
-        // eighty instructions and a wait stood between two loads; a layer of 8 fp32 rows, 6 of 64 experts: 149 -> 141 us)
-        int job = 0, in = wave;
-        for (int s0 = wave; s0 < total; s0 += EXPERT_WAVES * U)
-        {
-            u32x4 raw[U];
-            V b[U];
-            float scale[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u)
-            {
-                const int s = s0 + u * EXPERT_WAVES;
-                while (job < p.top && in >= esteps)
-                {
-                    in -= esteps;
-                    ++job;
-                }
-                const bool live = s < total;
-                const int id = __builtin_amdgcn_readlane(own_id, job < p.top ? job : 0);
-                // (past the end: any step of the first expert, with weight zero)
-                const u32x4 *w = job < p.top || !live ? weight_tile(p.down + (size_t)id * p.down_stride, tile, esteps, lane)
-                                             : weight_tile(p.shared_down, tile, ssteps, lane);
-                raw[u] = w[(size_t)(live ? in : 0) * 64];
-                b[u] = O::load(act + (size_t)(live ? s : 0) * 32);
-                scale[u] = !live ? 0.0f : job < p.top ? __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, own_weight), job)) : shared_weight;
-                in += EXPERT_WAVES;
-            }
-#pragma unroll
-            for (int u = 0; u < U; ++u)
-            {
-                const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
-                acc = acc + O::mma(O::from_weights(raw[u]), b[u], zero) * scale[u];
-            }
-        }
-        *reinterpret_cast<f32x4 *>(s_red[wave][lane]) = acc;
+        constexpr int P = HALF ? 1 : 2;                    // products of a step
+        constexpr int U = sizeof(T) == 2 ? 4 / P : 3 / P;  // steps in flight
+        __shared__ __attribute__((aligned(16))) float s_red[EXPERT_WAVES][P][64][4];
+        extern __shared__ __attribute__((aligned(16))) char smem[]; // the list's uses and numbers
+        const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), n = lane & 15, g = lane >> 4;
+        const int tile = HALF ? blockIdx.x >> 1 : blockIdx.x;
+        const int second = HALF ? n >> 3 : 0, row = HALF ? n & 7 : n, first = blockIdx.y * lists.rows;
+        const int rows = lists.rows < M - first ? lists.rows : M - first, mine = row < rows ? row : 0;
+        const int piece = (HALF ? g * 16 + (blockIdx.x & 1) * 8 + (n & 7) : lane) + second * 64;
+        const int pitch = p.top * p.ff + p.shared_ff;
+        // (the shared expert is the first of the list here, of a number that turns nothing)
+        const int own = p.shared_ff ? 1 : 0;
+        int *list = lists.at(p.lists, blockIdx.y);
+        ExpertUse *uses = reinterpret_cast<ExpertUse *>(smem);
+        int *numbers = reinterpret_cast<int *>(uses + (lists.most + own) * lists.rows);
+        for (int i = threadIdx.x; i < lists.most * lists.rows; i += EXPERT_WAVES * 64)
+            uses[own * lists.rows + i] = lists.uses(list)[i];
+        for (int i = threadIdx.x; i < lists.most; i += EXPERT_WAVES * 64)
+            numbers[own + i] = lists.numbers(list)[i];
+        if (own && (int)threadIdx.x < rows)
+            uses[threadIdx.x] = expert_use(p.weights[(first + threadIdx.x) * (p.top + 1) + p.top], (first + threadIdx.x) * pitch + p.top * p.ff, true);
+        if (own && threadIdx.x == 0)
+            numbers[0] = -EXPERT_WAVES;
+        const int count = own + __builtin_amdgcn_readfirstlane(list[0]);
         __syncthreads();
-        if (threadIdx.x < 64 && (lane & 15) == 0)
+
+        // the wavefront's place: steps that are left of the `job`-th of the list (none: it has none of that expert's), the next one's
+        // weights and this lane's activations; past the end those of the last expert's step 0, which every expert has
+        int job = 0, left = 0;
+        const u32x4 *w = nullptr;
+        const T *b = nullptr;
+        ExpertUse use = {};
+        const auto enter = [&]() __attribute__((always_inline)) {
+            const int id = __builtin_amdgcn_readfirstlane(numbers[job]), start = (wave + id) & (EXPERT_WAVES - 1);
+            const int steps = (id < 0 ? p.shared_ff : p.ff) >> 6;
+            const bf16 *matrix = id < 0 ? p.shared_down : p.down + (size_t)id * p.down_stride;
+            use = uses[job * lists.rows + mine];
+            left = start < steps ? (steps - start + EXPERT_WAVES - 1) / EXPERT_WAVES : 0;
+            const int at = left > 0 ? start : 0;
+            w = reinterpret_cast<const u32x4 *>(matrix) + ((size_t)tile * steps + at) * 128;
+            b = static_cast<const T *>(p.act) + (size_t)(use.act & 0x7fffffff) + at * 64 + 8 * g + second * 32;
+        };
+        const auto advance = [&]() __attribute__((always_inline)) {
+            while (left == 0 && ++job < count)
+                enter();
+        };
+        struct Held
         {
-            f32x4 *x = reinterpret_cast<f32x4 *>(p.x + (size_t)m * p.ldx + tile * 16 + 4 * g);
+            u32x4 raw[U][P];
+            V b[U][P];
+            float scale[U];
+            bool chosen[U];
+        };
+        Held next;
+        const auto fetch = [&]() __attribute__((always_inline)) {
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+            {
+                const bool live = job < count;
+#pragma unroll
+                for (int i = 0; i < P; ++i)
+                {
+                    next.raw[u][i] = w[i * 64 + piece];
+                    next.b[u][i] = O::load(b + i * 32);
+                }
+                next.scale[u] = use.weight;
+                next.chosen[u] = live && use.act < 0;
+                if (live)
+                {
+                    // (the last one of an expert stays where it is, within it)
+                    if (--left > 0)
+                        w += EXPERT_WAVES * 128, b += EXPERT_WAVES * 64;
+                    else
+                        advance();
+                }
+            }
+        };
+        f32x4 acc[P];
+#pragma unroll
+        for (int i = 0; i < P; ++i)
+            acc[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        enter();
+        advance();
+        fetch();
+        for (bool more = true; more;)
+        {
+            const Held cur = next;
+            more = job < count;
+            if (more)
+                fetch();
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+#pragma unroll
+                for (int i = 0; i < P; ++i)
+                {
+                    const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+                    const f32x4 sum = acc[i] + O::mma(O::from_weights(cur.raw[u][i]), cur.b[u][i], zero) * cur.scale[u];
+                    acc[i] = cur.chosen[u] ? sum : acc[i];
+                }
+        }
+#pragma unroll
+        for (int i = 0; i < P; ++i)
+            *reinterpret_cast<f32x4 *>(s_red[wave][i][lane]) = acc[i];
+        __syncthreads();
+        if (threadIdx.x < 64 && n < rows && (!HALF || g < 2))
+        {
+            f32x4 *x = reinterpret_cast<f32x4 *>(p.x + (size_t)(first + n) * p.ldx + blockIdx.x * (HALF ? 8 : 16) + 4 * g);
             f32x4 v = *x;
 #pragma unroll
-            for (int i = 0; i < EXPERT_WAVES; ++i)
-                v = v + *reinterpret_cast<const f32x4 *>(s_red[i][lane]);
+            for (int half = 0; half < 2; ++half)
+#pragma unroll
+                for (int i = 0; i < EXPERT_WAVES; ++i)
+                    v = v + *reinterpret_cast<const f32x4 *>(s_red[i][HALF ? 0 : half][HALF ? lane + half * 40 : lane]);
             *x = v;
         }
     }
@@ -447,7 +632,7 @@ namespace llamql
         // scratch of the experts, from one buffer
         struct ExpertScratch
         {
-            size_t ids, weights, act, offset, order, place, pair_out, shared_out, total;
+            size_t ids, weights, act, lists, offset, order, place, pair_out, shared_out, total;
         };
         ExpertScratch expert_scratch(int M, int experts, int top, int ff, int shared_ff, int N)
         {
@@ -462,6 +647,10 @@ namespace llamql
             s.ids = take(pairs * 4);
             s.weights = take((size_t)M * (top + 1) * 4);
             s.act = take((pairs * ff + (size_t)M * shared_ff) * 4);
+            size_t lists = 0;
+            for (int rows : {EXPERT_ROWS / 2, EXPERT_ROWS})
+                lists = std::max(lists, ceil_div(std::min(M, EXPERT_ROWS), rows) * expert_lists(M, rows, experts, top).ints());
+            s.lists = take(lists * 4);
             s.offset = take((size_t)(experts + 1) * 4);
             s.order = take(pairs * 4);
             s.place = take(pairs * 4);
@@ -469,6 +658,18 @@ namespace llamql
             s.shared_out = take(shared_ff ? (size_t)M * N * 4 : 0);
             s.total = at;
             return s;
+        }
+
+        template <typename T, bool HALF>
+        bool expert_down_launch(const char *fn, const ExpertArgs &p, int M, ExpertLists lists, hipStream_t st)
+        {
+            auto *kernel = expert_down_small_kernel<T, HALF>;
+            static LdsGrant grant;
+            const size_t use = lists.rows * sizeof(ExpertUse) + 4, lds = (lists.most + (p.shared_ff ? 1 : 0)) * use;
+            if (lds > 48 * 1024 && allow_lds(grant, reinterpret_cast<const void *>(kernel), (64 * ROUTE_MAX + 1) * (EXPERT_ROWS / (HALF ? 2 : 1) * sizeof(ExpertUse) + 4)) != hipSuccess)
+                return fail(fn, "cannot reserve %zu bytes of LDS", lds);
+            hipLaunchKernelGGL(kernel, dim3(p.N / (HALF ? 8 : 16), ceil_div(M, lists.rows)), dim3(EXPERT_WAVES * 64), lds, st, p, M, lists);
+            return launched(fn);
         }
 
         template <typename T>
@@ -487,13 +688,19 @@ namespace llamql
             }
             if (M <= SMALL_M)
             {
+                static_assert(SMALL_M == EXPERT_ROWS, "a list has a column for each of few rows");
+                // Halves of tiles, for eight rows at a time, but for more rows whole ones where these alone occupy the chip (bf16, us, halves
+                // and whole tiles: 16 rows, 64 experts of 1536 x 5120 351, 332; 16 of 4096 x 4096 207, 170; 64 of 1408 x 2048 135, 141;
+                // 8 rows, 1536 x 5120 226, 238).
+                const bool half = M <= EXPERT_ROWS / 2 || p.N / 16 < cu_count(device_id);
+                const ExpertLists lists = expert_lists(M, half ? EXPERT_ROWS / 2 : EXPERT_ROWS, p.experts, p.top);
+                p.lists = reinterpret_cast<int *>(scratch + at.lists);
                 const int widest = p.shared_ff > p.ff ? p.shared_ff : p.ff;
-                hipLaunchKernelGGL(expert_up_small_kernel<T>, dim3(widest / 16, p.top + (p.shared_ff ? 1 : 0), M),
-                                   dim3(EXPERT_WAVES * 64), 0, st, p, M);
+                hipLaunchKernelGGL(expert_up_small_kernel<T>, dim3(widest / 16, p.top + (p.shared_ff || M > 1 ? 1 : 0), M),
+                                   dim3(EXPERT_WAVES * 64), 0, st, p, M, lists);
                 if (!launched(fn))
                     return false;
-                hipLaunchKernelGGL(expert_down_small_kernel<T>, dim3(p.N / 16, M), dim3(EXPERT_WAVES * 64), 0, st, p);
-                return launched(fn);
+                return half ? expert_down_launch<T, true>(fn, p, M, lists, st) : expert_down_launch<T, false>(fn, p, M, lists, st);
             }
             int *offset = reinterpret_cast<int *>(scratch + at.offset), *order = reinterpret_cast<int *>(scratch + at.order);
             int *place = reinterpret_cast<int *>(scratch + at.place);

@@ -43,6 +43,47 @@ def test_rows_together_are_rows_alone(dev, M, experts, top, ff, shared, dtype):
     assert torch.equal(together, alone)
 
 
+# rows, experts, of a row, widths of an expert, the shared one and the model: one list and two, halves of tiles and (more than 8 rows
+# of a wide model) whole ones; fewer k-steps than wavefronts, a remainder of them, more
+@pytest.mark.parametrize("dtype", [sq.BF16, sq.F32])
+@pytest.mark.parametrize("M,experts,top,ff,shared,K", [(1, 6, 4, 64, 64, 128), (8, 40, 3, 576, 0, 192), (9, 5, 5, 64, 1216, 128), (9, 30, 2, 640, 64, 4160),
+                                                       (16, 1024, 4, 64, 0, 4096), (16, 300, 64, 64, 64, 192), (13, 2, 1, 192, 0, 4160)])
+def test_few_rows_against_64_bits(dev, M, experts, top, ff, shared, K, dtype):
+    import torch
+
+    T = torch.float32 if dtype == sq.F32 else torch.bfloat16
+    torch.manual_seed(M + experts)
+    tiled = lambda w: w.reshape(w.shape[0], w.shape[1] // 16, 16, w.shape[2] // 32, 4, 8).permute(0, 1, 3, 4, 2, 5).contiguous()  # noqa: E731
+    matrix = lambda n, rows, k: (torch.randn(n, rows, k, device=dev) * k ** -0.5).bfloat16()  # noqa: E731
+    up, down = matrix(experts, ff, K), matrix(experts, K, ff)
+    both = [matrix(1, max(shared, 64), K), matrix(1, K, max(shared, 64))]
+    logits, h, x = torch.randn(M, experts + 16, device=dev), torch.randn(M, K, device=dev).to(T), torch.randn(M, K, device=dev)
+    want = x.double()
+    weights, ids = logits[:, :experts].double().topk(top, 1)
+    weights = torch.softmax(weights, 1)
+
+    def part(m, u, d):
+        return d.double() @ torch.relu(u.double() @ h[m].double()).square().to(T).double()
+
+    for m in range(M):
+        for j in range(top):
+            want[m] += weights[m, j] * part(m, up[ids[m, j]], down[ids[m, j]])
+        if shared:
+            want[m] += torch.sigmoid(logits[m, experts].double()) * part(m, both[0][0], both[1][0])
+    lib, laid = sq.load(), [tiled(w) for w in (up, down, *both)]
+    size = lib.llam_seq_experts_scratch_bytes(M, experts, top, ff, shared, K)
+    scratch = torch.full((size + 64,), 255, dtype=torch.uint8, device=dev)
+    a = sq.ExpertsArgs(d_logits=logits.data_ptr(), ldz=experts + 16, d_up=laid[0].data_ptr(), d_down=laid[1].data_ptr(), up_stride=ff * K,
+                       down_stride=ff * K, experts=experts, top=top, ff=ff, shared_ff=shared, K=K, N=K, d_h=h.data_ptr(), d_x=x.data_ptr(), ldx=K)
+    if shared:
+        a.d_shared_up, a.d_shared_down = laid[2].data_ptr(), laid[3].data_ptr()
+    assert lib.llam_seq_experts(ctypes.byref(a), M, scratch.data_ptr(), size, dtype, 0, torch.cuda.current_stream().cuda_stream), lib.llam_ql_last_error()
+    torch.cuda.synchronize()
+    assert (scratch[size:] == 255).all()
+    # fp32: sums of up to K products, 2^-24 each.  bf16: the square of a sum whose rounding may fall to the other side, 2^-8 of few of the ff values
+    assert (x.double() - want).norm() / (want.norm()) < (2e-6 if dtype == sq.F32 else 2e-3)
+
+
 # rows, experts, of a row, width of an expert, of the model, slope of the logits: few rows; more than 64 experts, evenly and
 # mostly the first ones chosen, many without a row; groups of several tiles with a last one of few rows, of all rows; each tile
 # (test_launch_rules.py)
