@@ -498,3 +498,17 @@ def test_tiles_of_the_transposed_matrix(dev, N, K, batch):
     assert sequence.load().llam_seq_transpose_tiles(tiled(w).data_ptr(), out.data_ptr(), N, K, batch, 0, torch.cuda.current_stream().cuda_stream)
     torch.cuda.synchronize()
     assert torch.equal(out[:-8], tiled(w.transpose(1, 2)).reshape(-1)) and (out[-8:] == 0).all()
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("dim,n", [(40, 33), (256, 65), (300, 97), (512, 150)])
+def test_products_of_a_chunk_in_blocks_of_columns(dim, n, dtype):
+    """One block of the columns of q and k, a whole one and a rest of the next, two; a last chunk of few tokens; a portion behind another."""
+    cfg = sm.config(sm.mlstm(heads=2, dim=dim, vdim=40), width=64)
+    t = sm.random_weights(cfg, dim)
+    tokens = tokens_of(cfg, n)
+    want = so.kogilix(cfg, t.plain(), tokens)
+    model = load(cfg, t, dtype, cap=200, max_rows=200)
+    for cuts in ([n], [n - 30, 30]):
+        check(run(model, 1, tokens, cuts), want, dtype, note=f"dim {dim} {cuts}")
+    model.close()
