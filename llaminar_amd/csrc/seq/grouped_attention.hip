@@ -64,6 +64,7 @@ namespace llamql
         const int32_t *row0, *ntok, *slot, *pos;
         int first, heads, groups, ring, chunk; // chunk: INT_MAX without a mask
         int stretch, nsplit, rcap, block_rows;
+        int cus, round; // compute units; workgroups of a round, 0: in the order of the grid (att_place)
         float scale;
         void *o;
         int ldo;
@@ -107,6 +108,25 @@ namespace llamql
     // first position that position i sees
     __device__ __forceinline__ int att_low(int i, int chunk) { return i / chunk * chunk; }
 
+    // Which row block, stretch and key/value head a workgroup of many rows takes.  The longest walks go first, a row block of all heads after
+    // the other (a die's workgroups have few heads, whose keys and values stay in its cache), and every second round of
+    // workgroups backwards, so that a compute unit which has a long walk gets a short one beside it.  Head after head two long ones met:
+    // bf16, 2048 tokens, 16 heads of 128 in two stretches 71.6 -> 60.5 us (without turning back 71.8, with rounds of half or twice as many
+    // workgroups 70.9, 70.6), 40 heads in 8 groups 146 -> 118 (a walk of 2048 positions takes 115 by itself).
+    // Short walks of bf16 gain nothing and pay for the order, and keep that of the grid: 16 heads in 4 groups, 500 tokens 21.5 and 22.4 us,
+    // 512 at position 1536 33.6 and 35.4; fp32, 500 tokens 33.4 and 28.2.
+    constexpr int ATT_LONG = 512; // positions of a stretch from which on they do
+    __device__ __forceinline__ void att_place(unsigned round, int &x, int &y, int &z)
+    {
+        x = gridDim.x - 1 - blockIdx.x, y = blockIdx.y, z = blockIdx.z;
+        if (round == 0)
+            return;
+        const unsigned X = gridDim.x, Z = gridDim.z, total = X * gridDim.y * Z, id = blockIdx.x + X * (blockIdx.y + gridDim.y * blockIdx.z);
+        const unsigned base = id / round * round, end = base + round < total ? base + round : total;
+        const unsigned at = (id / round & 1) != 0 ? base + (end - 1 - id) : id, t = at / Z;
+        z = at - t * Z, y = t / X, x = X - 1 - (t - y * X);
+    }
+
     template <typename T, int DK, int DV, int WR, int RG>
     __global__ void __launch_bounds__(ATT_THREADS, sizeof(T) == 2 && WR == 4 && DK + DV <= 256 ? 2 : 1)
         attention_kernel(AttentionArgs p)
@@ -130,11 +150,14 @@ namespace llamql
         const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
         const int c = lane & 15, g = lane >> 4;
         const int wr = WR == 1 ? 0 : wave, wp = WR == 1 ? wave : 0;
-        const int ei = blockIdx.z / p.groups, kv = blockIdx.z - ei * p.groups;
-        const int e = p.first + ei, split = blockIdx.y;
+        int block = blockIdx.x, split = blockIdx.y, z = blockIdx.z;
+        if (WR > 1)
+            att_place(p.round, block, split, z);
+        const int ei = z / p.groups, kv = z - ei * p.groups;
+        const int e = p.first + ei;
         const int per = p.heads / p.groups;
         const int R = p.ntok[e] * per, pos0 = p.pos[e], row0 = p.row0[e];
-        const int rb = (gridDim.x - 1 - blockIdx.x) * 16 * RG * WR; // the longest walks first
+        const int rb = block * 16 * RG * WR;
         if (rb >= R)
             return;
         const int last_row = rb + 16 * RG * WR - 1 < R ? rb + 16 * RG * WR - 1 : R - 1;
@@ -702,6 +725,7 @@ namespace llamql
             constexpr int RG = sizeof(T) == 2 && DK + DV <= 384 ? 2 : 1;
             const int z = n * p.groups;
             p.block_rows = pl.block_rows;
+            p.round = sizeof(T) == 4 || pl.stretch >= ATT_LONG ? p.cus : 0;
             p.part_ml = p.part_o + parts * DV;
             bool ok;
             if constexpr (NARROW)
@@ -865,6 +889,7 @@ extern "C" bool llam_seq_attention(const llam_seq_attention_args *a, const void 
     if (!attention_args(fn, a, d_q, e, first, d_o, ldo, d_scratch, p) || !set_device(fn, device_id))
         return false;
     hipStream_t st = as_stream(stream);
+    p.cus = cu_count(device_id);
     if (dtype == LLAM_SEQ_F32)
         return attention_keys<float>(a->dim, a->vdim, fn, p, n, max_ntok, max_len, scratch_floats, st);
     return attention_keys<bf16>(a->dim, a->vdim, fn, p, n, max_ntok, max_len, scratch_floats, st);
@@ -899,6 +924,7 @@ extern "C" bool llam_seq_attention_decode(const llam_seq_attention_args *a, cons
         return false;
     p.proj = d_proj, p.ldp = ldp, p.turns = d_turns, p.half = rot_dims / 2, p.append = append;
     hipStream_t st = as_stream(stream);
+    p.cus = cu_count(device_id);
     if (dtype == LLAM_SEQ_F32)
         return attention_keys<float>(a->dim, a->vdim, fn, p, n, 1, max_len, scratch_floats, st);
     return attention_keys<bf16>(a->dim, a->vdim, fn, p, n, 1, max_len, scratch_floats, st);
@@ -926,6 +952,7 @@ extern "C" bool llam_seq_attention_portions(const llam_seq_attention_args *a, co
     if (!attention_args(fn, a, d_q, e, first, d_o, ldo, d_scratch, p) || !set_device(fn, device_id))
         return false;
     hipStream_t st = as_stream(stream);
+    p.cus = cu_count(device_id);
     if (dtype == LLAM_SEQ_F32)
         return attention_keys<float>(a->dim, a->vdim, fn, p, n, ntok, len, scratch_floats, st);
     return attention_keys<bf16>(a->dim, a->vdim, fn, p, n, ntok, len, scratch_floats, st);

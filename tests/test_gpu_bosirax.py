@@ -102,6 +102,13 @@ def test_attention_of_many_entries(dev, dtype):
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("heads,groups,ntok,chunk,pos,n", [(10, 10, 650, 0, 0, 1), (8, 8, 129, 0, 500, 5), (36, 12, 333, 90, 20, 1), (3, 1, 5700, 64, 0, 2)])
+def test_attention_of_several_rounds_of_workgroups(dev, heads, groups, ntok, chunk, pos, n, dtype):
+    """More workgroups than compute units, whose second and fourth round are dealt backwards: a last round that is odd, even, not full."""
+    attend(dev, dtype, heads, groups, 64, 64, ntok, chunk, pos, None, n)
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("vdim", [64, 128, 256])
 @pytest.mark.parametrize("length", [120, 128, 129, 200, 260, 500, 512, 513, 577, 700])
 def test_attention_in_few_stretches(dev, length, vdim, dtype):
