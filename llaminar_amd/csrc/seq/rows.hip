@@ -391,7 +391,7 @@ namespace llamql
     // second operand the rows' (see linear_small_tile): twice the workgroups, and one product where there were two.
     // Bound by the weights, and for one or two rows by the chain of list, first weights and sums.  A layer of 6 of 64 experts of 1408 x 2048 and a
     // shared one of 2816, us, against a workgroup for every row that read its own experts: 8 rows that choose alike (12 experts in all) bf16
-    // 63.8 -> 45.2, fp32 108 -> 61; that choose evenly (35) 95.7 -> 86.8, 142 -> 126; 16 rows 156 -> 135; 1 row 25.7 -> 24.0, fp32 41.1 -> 33.2.
+    // 63.8 -> 45.9, fp32 108 -> 62.8; that choose evenly (35) 95.7 -> 86.8, 142 -> 126; 16 rows 156 -> 135; 1 row 25.7 -> 24.0, fp32 41.1 -> 33.2.
     // 16 rows at 1536 x 5120: 423 -> 332.  Slower only where small experts are hardly shared: 4 rows, 8 of 128 of 768 x 2048 45.7 -> 48.9, fp32 58 -> 65.
     template <typename T, bool HALF>
     __global__ void __launch_bounds__(EXPERT_WAVES * 64, 4)
