@@ -40,6 +40,8 @@ namespace llamql
     // scratch: for sums of tiles cut along K, as far as it reaches; what linear_split_bytes says serves layers of up to max_rows rows
     bool linear_tiled(const char *fn, const LinearArgs &a, int batch, int dtype, int device_id, hipStream_t st, void *scratch = nullptr,
                       size_t bytes = 0);
+    // The same for rows of a layer of M in all, with the bits that they have among these
+    bool linear_tiled_rows(const char *fn, const LinearArgs &a, int M, int batch, int dtype, int device_id, hipStream_t st);
     size_t linear_split_bytes(int max_rows, int N, int K, int dtype, int device_id);
 
     // Whether a sum of products in three bf16 pieces of each 32-bit value may not be that of the whole values, which then

@@ -485,6 +485,25 @@ extern "C" bool llam_seq_linear(const llam_seq_linear_args *a, int dtype, int de
     return llam_seq_linear_within(a, nullptr, 0, dtype, device_id, stream);
 }
 
+extern "C" bool llam_seq_linear_rows(const llam_seq_linear_args *a, int first, int n, int dtype, int device_id, void *stream)
+{
+    static const char *fn = "llam_seq_linear_rows";
+    LinearArgs p;
+    if (!linear_args(fn, a, dtype, p))
+        return false;
+    if (a->M <= SMALL_M || first < 0 || n < 0 || first > a->M - n)
+        return fail(fn, "rows %d .. of %d, %d of them (of more than %d)", first, a->M, n, SMALL_M);
+    if (n == 0)
+        return true;
+    if (!set_device(fn, device_id))
+        return false;
+    const size_t elem = dtype == LLAM_SEQ_F32 ? 4 : 2, out = a->out == LLAM_SEQ_OUT_F32 || a->out == LLAM_SEQ_OUT_ADD ? 4 : elem;
+    p.a = static_cast<const char *>(p.a) + (size_t)first * a->lda * elem;
+    p.y = static_cast<char *>(p.y) + (size_t)first * a->ldy * out;
+    p.M = n;
+    return linear_tiled_rows(fn, p, a->M, a->batch, dtype, device_id, as_stream(stream));
+}
+
 extern "C" bool llam_seq_linear_pair(const llam_seq_linear_args *a, const llam_seq_linear_args *b, int dtype, int device_id, void *stream)
 {
     static const char *fn = "llam_seq_linear_pair";

@@ -736,10 +736,18 @@ namespace llamql
             const Tile *tile;
             Split split; // slices = 0: every tile whole
         };
+        struct Tiles
+        {
+            const Tile *tiles;
+            size_t n;
+        };
+        Tiles tiles_of(int dtype)
+        {
+            return dtype == LLAM_SEQ_F32 ? Tiles{TILES_F32, sizeof TILES_F32 / sizeof(Tile)} : Tiles{TILES_BF16, sizeof TILES_BF16 / sizeof(Tile)};
+        }
         Plan linear_plan(const LinearArgs &a, int batch, int dtype, size_t bytes, int cus)
         {
-            const Tile *tiles = dtype == LLAM_SEQ_F32 ? TILES_F32 : TILES_BF16;
-            const size_t n = dtype == LLAM_SEQ_F32 ? sizeof TILES_F32 / sizeof(Tile) : sizeof TILES_BF16 / sizeof(Tile);
+            const auto [tiles, n] = tiles_of(dtype);
             Plan plan = {tiles, {expected(*tiles, a, batch, cus), 0, 0, 0}};
             for (size_t i = 1; i < n; ++i)
                 if (const float us = expected(tiles[i], a, batch, cus); us < plan.split.us)
@@ -765,6 +773,21 @@ namespace llamql
             most = need > most ? need : most;
         }
         return most;
+    }
+
+    // A sum is of the turns of its group of wavefronts, one after the other, so tiles of as many groups have the same bits
+    // (all with one are rows of 32x32 products of 16 columns each).  Among these, the best for the rows that there are.
+    bool linear_tiled_rows(const char *fn, const LinearArgs &a, int M, int batch, int dtype, int device_id, hipStream_t st)
+    {
+        const int cus = cu_count(device_id);
+        LinearArgs all = a;
+        all.M = M;
+        const Tile *tile = linear_plan(all, batch, dtype, 0, cus).tile;
+        const auto [tiles, n] = tiles_of(dtype);
+        for (size_t i = 0; i < n; ++i)
+            if (tiles[i].groups == tile->groups && expected(tiles[i], a, batch, cus) < expected(*tile, a, batch, cus))
+                tile = &tiles[i];
+        return tile->launch(fn, a, batch, st);
     }
 
     bool linear_tiled(const char *fn, const LinearArgs &a, int batch, int dtype, int device_id, hipStream_t st, void *scratch, size_t bytes)

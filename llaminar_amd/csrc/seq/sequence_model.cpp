@@ -5,6 +5,7 @@
 #include <hip/hip_runtime_api.h>
 
 #include <algorithm>
+#include <array>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
@@ -195,7 +196,7 @@ namespace
     {
         int M = 0, single = 0;
         int max_len = 1; // bound on the length of the one-token entries' sequences
-        std::vector<int> ntok, len, slot; // the portions' tokens, their sequences' lengths afterwards, and slots
+        std::vector<int> ntok, len, slot, row; // the portions' tokens, their sequences' lengths afterwards, slots, and first rows
         // runs of portions that the recurrent mixers launch together: entries first .. first + n - 1, the most tokens
         struct Run
         {
@@ -209,9 +210,9 @@ namespace
         // as well: Kogilix 5.1 -> 4.3 ms, Bosirax 3.6 -> 2.7); a grid is made for the longest, so a portion that would leave two
         // thirds of it empty starts a run of its own.  What a portion's outputs are does not depend on its run: every mixer cuts
         // a portion up by its own length.
-        void add(int entry, int tokens, int length, int in)
+        void add(int entry, int tokens, int length, int in, int at)
         {
-            ntok.push_back(tokens), len.push_back(length), slot.push_back(in);
+            ntok.push_back(tokens), len.push_back(length), slot.push_back(in), row.push_back(at);
             if (!runs.empty())
             {
                 Run &r = runs.back();
@@ -355,13 +356,34 @@ namespace
                 return false;
             const llam_seq_entries e = md.entries();
             std::vector<bool> expanded(s.portions());
-            int left = s.single; // entries that attend in latent space
+            // rows that attend in latent space, first and number: of all rows the products cost as much as without expanded portions, on top
+            // of these (16 heads of 128, rank 512, one token beside 1024 of bf16: 162 -> 143 us a layer, fp32 280 -> 258)
+            std::vector<std::array<int, 2>> rows;
+            int at = 0;
             for (int i = 0; i < s.portions(); ++i)
-                left += !(expanded[i] = latent_expands(w, s.ntok[i], s.len[i], c.dtype, md.scratch_bytes));
-            if (left)
+                if ((expanded[i] = latent_expands(w, s.ntok[i], s.len[i], c.dtype, md.scratch_bytes)))
+                {
+                    if (at < s.row[i])
+                        rows.push_back({at, s.row[i] - at});
+                    at = s.row[i] + s.ntok[i];
+                }
+            if (at < s.M)
+                rows.push_back({at, s.M - at});
+            if (!rows.empty())
             {
-                if (!linear(md.q, H * dp, w.w_uk_t, rp, dp, md.qlat, H * rp, LLAM_SEQ_OUT_ELEM, s.M, nullptr, nullptr, 0, nullptr, H, dp,
-                            (long)rp * dp, rp))
+                // (never in slices of K, which a layer of one head would get by its number of rows)
+                const auto of_heads = [&](const void *a, int K, const void *matrix, int N, void *y, int ldy) {
+                    llam_seq_linear_args l{};
+                    l.d_a = a, l.lda = H * K, l.d_w = matrix, l.N = N, l.K = K, l.d_y = y, l.ldy = ldy, l.out = LLAM_SEQ_OUT_ELEM, l.M = s.M;
+                    l.batch = H, l.a_stride = K, l.w_stride = (long)N * K, l.y_stride = N;
+                    if (s.M <= ROW_MAX)
+                        return forward(fn, llam_seq_linear(&l, c.dtype, c.device_id, st));
+                    for (const auto &[first, n] : rows)
+                        if (!forward(fn, llam_seq_linear_rows(&l, first, n, c.dtype, c.device_id, st)))
+                            return false;
+                    return true;
+                };
+                if (!of_heads(md.q, dp, w.w_uk_t, rp, md.qlat, H * rp))
                     return false;
                 if (s.single && !forward(fn, llam_seq_latent_attention(md.qlat, cache, &e, 0, s.single, 1, s.max_len, H, rp, c.cap, w.scale,
                                                                        md.olat, md.lat_scratch, md.lat_floats, c.dtype, c.device_id, st)))
@@ -375,9 +397,7 @@ namespace
                                                                               c.device_id, st)))
                         return false;
                 }
-                // (rows of expanded portions hold what lay there: they are written below)
-                if (!linear(md.olat, H * rp, w.w_uv, vp, rp, md.mix, mix_columns(w), LLAM_SEQ_OUT_ELEM, s.M, nullptr, nullptr, 0, nullptr, H,
-                            rp, (long)vp * rp, vp))
+                if (!of_heads(md.olat, rp, w.w_uv, vp, md.mix, mix_columns(w)))
                     return false;
             }
             for (int i = 0; i < s.portions(); ++i)
@@ -857,7 +877,7 @@ extern "C" bool llam_seqm_forward(void *model, int n, const int32_t *h_slot, con
     for (int e = 0; e < n; ++e)
         if (h_ntok[e] > 1)
         {
-            s.add(placed, h_ntok[e], h_pos[e] + h_ntok[e], h_slot[e]);
+            s.add(placed, h_ntok[e], h_pos[e] + h_ntok[e], h_slot[e], row0[e]);
             place(e);
         }
     s.row_slot = md->row_slot();

@@ -187,6 +187,32 @@ def test_rows_that_start_at_eight_bytes(dev, M, N, K, out):
     assert (y[M:] == 5.0).all() and (y[:, columns:] == 5.0).all() and (aligned[:, columns:] == 5.0).all()
 
 
+@pytest.mark.parametrize("dtype", [BF16, F32])
+@pytest.mark.parametrize("M,N,K,batch", [(*s, 1) for s in SHAPES] + [(70, 48, 128, 5), (601, 512, 128, 16), (2049, 128, 512, 16)])
+def test_some_rows_of_a_layer(dev, M, N, K, batch, dtype):
+    """The bits that the rows have among all, whatever tile they get by themselves; the others are neither read nor written."""
+    import torch
+
+    torch.manual_seed(M + N)
+    kind, out = (torch.float32, sq.OUT_F32) if dtype == F32 or batch == 1 else (torch.bfloat16, sq.OUT_ELEM)
+    a = torch.randn(M, batch * K, device=dev).to(torch.float32 if dtype == F32 else torch.bfloat16)
+    t = torch.stack([tiles((torch.randn(N, K, device=dev) * K ** -0.5).bfloat16()) for _ in range(batch)])
+    all_rows, y = torch.zeros(M, batch * N + 4, device=dev, dtype=kind), torch.empty(M, batch * N + 4, device=dev, dtype=kind)
+    args = sq.LinearArgs(d_w=t.data_ptr(), M=M, N=N, K=K, lda=batch * K, ldy=batch * N + 4, out=out, batch=batch, a_stride=K, w_stride=N * K,
+                         y_stride=N)
+    args.d_a, args.d_y = a.data_ptr(), all_rows.data_ptr()
+    lib, stream = sq.load(), torch.cuda.current_stream().cuda_stream
+    assert lib.llam_seq_linear(ctypes.byref(args), dtype, 0, stream), lib.llam_ql_last_error()
+    for first, n in [(0, 1), (M - 1, 1), (M // 3, 7), (1, M - 1), (0, M // 2), (M - 17, 17), (0, M), (5, 0)]:
+        only = torch.full_like(a, float("nan"))
+        only[first:first + n] = a[first:first + n]
+        args.d_a, args.d_y = only.data_ptr(), y.fill_(5.0).data_ptr()
+        assert lib.llam_seq_linear_rows(ctypes.byref(args), first, n, dtype, 0, stream), lib.llam_ql_last_error()
+        torch.cuda.synchronize()
+        assert torch.equal(y[first:first + n, :batch * N], all_rows[first:first + n, :batch * N]), (first, n)
+        assert (y[:first] == 5.0).all() and (y[first + n:] == 5.0).all() and (y[:, batch * N:] == 5.0).all()
+
+
 # ---- tiles cut along K (llam_seq_linear_within) ------------------------------------------------------------
 
 # every tile that is cut, with and without whole ones beside it, slices of unequal length (test_launch_rules.py)
