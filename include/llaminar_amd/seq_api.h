@@ -72,9 +72,9 @@ size_t llam_seq_linear_scratch_bytes(int max_rows, int N, int K, int dtype, int 
 bool llam_seq_linear_within(const llam_seq_linear_args *a, void *d_scratch, size_t scratch_bytes, int dtype, int device_id,
                             void *stream);
 
-/* Rows first .. first + n - 1 of llam_seq_linear's M, of more than 16: the same bits as with all of them.  The other rows of A are not read,
- * those of Y stay as they are. */
-bool llam_seq_linear_rows(const llam_seq_linear_args *a, int first, int n, int dtype, int device_id, void *stream);
+/* Some of llam_seq_linear's M rows, of more than 16, with the bits that they have among all: `n` stretches of `rows` rows from row
+ * `first` on (on the host, one behind the other).  The other rows of A are not read, those of Y stay as they are. */
+bool llam_seq_linear_rows(const llam_seq_linear_args *a, int n, const int *first, const int *rows, int dtype, int device_id, void *stream);
 
 /* `batch` tiled matrices of N rows and K columns, one behind the other, as those of K rows and N columns; N and K multiples of 32. */
 bool llam_seq_transpose_tiles(const void *d_w, void *d_out, int N, int K, int batch, int device_id, void *stream);

@@ -485,23 +485,28 @@ extern "C" bool llam_seq_linear(const llam_seq_linear_args *a, int dtype, int de
     return llam_seq_linear_within(a, nullptr, 0, dtype, device_id, stream);
 }
 
-extern "C" bool llam_seq_linear_rows(const llam_seq_linear_args *a, int first, int n, int dtype, int device_id, void *stream)
+extern "C" bool llam_seq_linear_rows(const llam_seq_linear_args *a, int n, const int *first, const int *rows, int dtype, int device_id, void *stream)
 {
     static const char *fn = "llam_seq_linear_rows";
     LinearArgs p;
     if (!linear_args(fn, a, dtype, p))
         return false;
-    if (a->M <= SMALL_M || first < 0 || n < 0 || first > a->M - n)
-        return fail(fn, "rows %d .. of %d, %d of them (of more than %d)", first, a->M, n, SMALL_M);
-    if (n == 0)
-        return true;
-    if (!set_device(fn, device_id))
+    if (a->M <= SMALL_M || n < 0 || (n > 0 && (!first || !rows)))
+        return fail(fn, "bad size (M=%d, of more than %d; n=%d)", a->M, SMALL_M, n);
+    for (int i = 0, at = 0; i < n; at = first[i] + rows[i], ++i)
+        if (rows[i] < 1 || first[i] < at || first[i] > a->M - rows[i])
+            return fail(fn, "stretch %d: %d rows from row %d of %d", i, rows[i], first[i], a->M);
+    if (n > 0 && !set_device(fn, device_id))
         return false;
-    const size_t elem = dtype == LLAM_SEQ_F32 ? 4 : 2, out = a->out == LLAM_SEQ_OUT_F32 || a->out == LLAM_SEQ_OUT_ADD ? 4 : elem;
-    p.a = static_cast<const char *>(p.a) + (size_t)first * a->lda * elem;
-    p.y = static_cast<char *>(p.y) + (size_t)first * a->ldy * out;
-    p.M = n;
-    return linear_tiled_rows(fn, p, a->M, a->batch, dtype, device_id, as_stream(stream));
+    for (int i = 0; i < n; i += p.stretches)
+    {
+        p.stretches = n - i < LINEAR_STRETCHES ? n - i : LINEAR_STRETCHES;
+        for (int k = 0; k < p.stretches; ++k)
+            p.stretch_first[k] = first[i + k], p.stretch_rows[k] = rows[i + k];
+        if (!linear_tiled_rows(fn, p, a->batch, dtype, device_id, as_stream(stream)))
+            return false;
+    }
+    return true;
 }
 
 extern "C" bool llam_seq_linear_pair(const llam_seq_linear_args *a, const llam_seq_linear_args *b, int dtype, int device_id, void *stream)

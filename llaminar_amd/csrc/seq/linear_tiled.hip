@@ -228,6 +228,12 @@ namespace llamql
             }
             m_tiles = __builtin_amdgcn_readfirstlane(live);
         }
+        int row0 = 0, rows = p.M;
+        if (p.stretches)
+        {
+            row0 = p.stretch_first[blockIdx.z], rows = p.stretch_rows[blockIdx.z];
+            m_tiles = (rows + BM - 1) / BM;
+        }
         const int total = m_tiles * n_tiles;
         if ((int)blockIdx.x >= (SPLIT ? p.full + (total - p.full) * p.slices : total))
             return;
@@ -238,7 +244,7 @@ namespace llamql
         const int part = whole ? blockIdx.x : blockIdx.x - p.full - slice * (total - p.full); // of the whole tiles or of the others
         int mt, nt;
         tile_place(whole ? die_order(part, SPLIT ? p.full : total) : p.full + die_order(part, total - p.full), m_tiles, n_tiles, mt, nt);
-        int z = blockIdx.y, row0 = 0, rows = p.M;
+        int z = blockIdx.y;
         if (p.group_offset)
         {
             // the mt-th tile of rows among those of all groups
@@ -617,7 +623,7 @@ namespace llamql
             const long mt = a.group_offset ? a.group_rows / BM + (batch < a.group_rows ? batch : a.group_rows) : ceil_div(a.M, BM);
             if (mt * nt > 0x7fffffff)
                 return fail(fn, "M=%d rows of N=%d columns are too many", a.M, a.N);
-            hipLaunchKernelGGL(kernel, dim3((unsigned)(mt * nt), a.group_offset ? 1 : batch), dim3(WM * WN * KG * 64), lds, st, a, (int)mt, nt);
+            hipLaunchKernelGGL(kernel, dim3((unsigned)(mt * nt), a.group_offset ? 1 : batch, a.stretches ? a.stretches : 1), dim3(WM * WN * KG * 64), lds, st, a, (int)mt, nt);
             return launched(fn);
         }
 
@@ -777,17 +783,19 @@ namespace llamql
 
     // A sum is of the turns of its group of wavefronts, one after the other, so tiles of as many groups have the same bits
     // (all with one are rows of 32x32 products of 16 columns each).  Among these, the best for the rows that there are.
-    bool linear_tiled_rows(const char *fn, const LinearArgs &a, int M, int batch, int dtype, int device_id, hipStream_t st)
+    bool linear_tiled_rows(const char *fn, const LinearArgs &a, int batch, int dtype, int device_id, hipStream_t st)
     {
         const int cus = cu_count(device_id);
-        LinearArgs all = a;
-        all.M = M;
-        const Tile *tile = linear_plan(all, batch, dtype, 0, cus).tile;
+        const Tile *all = linear_plan(a, batch, dtype, 0, cus).tile, *tile = all;
+        LinearArgs some = a;
+        some.M = 0;
+        for (int k = 0; k < a.stretches; ++k)
+            some.M = some.M > a.stretch_rows[k] ? some.M : a.stretch_rows[k]; // (the grid is of the longest)
         const auto [tiles, n] = tiles_of(dtype);
         for (size_t i = 0; i < n; ++i)
-            if (tiles[i].groups == tile->groups && expected(tiles[i], a, batch, cus) < expected(*tile, a, batch, cus))
+            if (tiles[i].groups == all->groups && expected(tiles[i], some, batch * a.stretches, cus) < expected(*tile, some, batch * a.stretches, cus))
                 tile = &tiles[i];
-        return tile->launch(fn, a, batch, st);
+        return tile->launch(fn, some, batch, st);
     }
 
     bool linear_tiled(const char *fn, const LinearArgs &a, int batch, int dtype, int device_id, hipStream_t st, void *scratch, size_t bytes)

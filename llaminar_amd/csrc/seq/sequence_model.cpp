@@ -5,7 +5,6 @@
 #include <hip/hip_runtime_api.h>
 
 #include <algorithm>
-#include <array>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
@@ -356,19 +355,19 @@ namespace
                 return false;
             const llam_seq_entries e = md.entries();
             std::vector<bool> expanded(s.portions());
-            // rows that attend in latent space, first and number: of all rows the products cost as much as without expanded portions, on top
+            // rows that attend in latent space, in stretches: of all rows the products cost as much as without expanded portions, on top
             // of these (16 heads of 128, rank 512, one token beside 1024 of bf16: 162 -> 143 us a layer, fp32 280 -> 258)
-            std::vector<std::array<int, 2>> rows;
+            std::vector<int> first, rows;
             int at = 0;
             for (int i = 0; i < s.portions(); ++i)
                 if ((expanded[i] = latent_expands(w, s.ntok[i], s.len[i], c.dtype, md.scratch_bytes)))
                 {
                     if (at < s.row[i])
-                        rows.push_back({at, s.row[i] - at});
+                        first.push_back(at), rows.push_back(s.row[i] - at);
                     at = s.row[i] + s.ntok[i];
                 }
             if (at < s.M)
-                rows.push_back({at, s.M - at});
+                first.push_back(at), rows.push_back(s.M - at);
             if (!rows.empty())
             {
                 // (never in slices of K, which a layer of one head would get by its number of rows)
@@ -378,10 +377,7 @@ namespace
                     l.batch = H, l.a_stride = K, l.w_stride = (long)N * K, l.y_stride = N;
                     if (s.M <= ROW_MAX)
                         return forward(fn, llam_seq_linear(&l, c.dtype, c.device_id, st));
-                    for (const auto &[first, n] : rows)
-                        if (!forward(fn, llam_seq_linear_rows(&l, first, n, c.dtype, c.device_id, st)))
-                            return false;
-                    return true;
+                    return forward(fn, llam_seq_linear_rows(&l, (int)rows.size(), first.data(), rows.data(), c.dtype, c.device_id, st));
                 };
                 if (!of_heads(md.q, dp, w.w_uk_t, rp, md.qlat, H * rp))
                     return false;

@@ -99,7 +99,7 @@ SIGNATURES = {
     "llam_seq_linear": (c_bool, [POINTER(LinearArgs), c_int, c_int, c_void_p]),
     "llam_seq_linear_scratch_bytes": (c_size_t, [c_int, c_int, c_int, c_int, c_int]),
     "llam_seq_linear_within": (c_bool, [POINTER(LinearArgs), c_void_p, c_size_t, c_int, c_int, c_void_p]),
-    "llam_seq_linear_rows": (c_bool, [POINTER(LinearArgs), c_int, c_int, c_int, c_int, c_void_p]),
+    "llam_seq_linear_rows": (c_bool, [POINTER(LinearArgs), c_int, _I32P, _I32P, c_int, c_int, c_void_p]),
     "llam_seq_transpose_tiles": (c_bool, [c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p]),
     "llam_seq_linear_pair": (c_bool, [POINTER(LinearArgs), POINTER(LinearArgs), c_int, c_int, c_void_p]),
     "llam_seq_embed": (c_bool, [POINTER(EmbedArgs), c_void_p, c_void_p, c_int, c_int, c_int, c_void_p]),

@@ -203,14 +203,18 @@ def test_some_rows_of_a_layer(dev, M, N, K, batch, dtype):
     args.d_a, args.d_y = a.data_ptr(), all_rows.data_ptr()
     lib, stream = sq.load(), torch.cuda.current_stream().cuda_stream
     assert lib.llam_seq_linear(ctypes.byref(args), dtype, 0, stream), lib.llam_ql_last_error()
-    for first, n in [(0, 1), (M - 1, 1), (M // 3, 7), (1, M - 1), (0, M // 2), (M - 17, 17), (0, M), (5, 0)]:
-        only = torch.full_like(a, float("nan"))
-        only[first:first + n] = a[first:first + n]
+    for stretches in [[(0, 1)], [(M - 1, 1)], [(1, M - 1)], [(0, M // 2), (M - 7, 7)], [(0, M)], [], [(i, 1) for i in range(0, 17, 2)],
+                      [(0, 3), (3, M // 3), (M // 2, M // 4), (M - 1, 1)]]:
+        only, others = torch.full_like(a, float("nan")), torch.ones(M, dtype=torch.bool, device=dev)
+        for first, n in stretches:
+            only[first:first + n] = a[first:first + n]
+            others[first:first + n] = False
         args.d_a, args.d_y = only.data_ptr(), y.fill_(5.0).data_ptr()
-        assert lib.llam_seq_linear_rows(ctypes.byref(args), first, n, dtype, 0, stream), lib.llam_ql_last_error()
+        first, n = ((ctypes.c_int32 * len(stretches))(*(s[i] for s in stretches)) for i in (0, 1))
+        assert lib.llam_seq_linear_rows(ctypes.byref(args), len(stretches), first, n, dtype, 0, stream), lib.llam_ql_last_error()
         torch.cuda.synchronize()
-        assert torch.equal(y[first:first + n, :batch * N], all_rows[first:first + n, :batch * N]), (first, n)
-        assert (y[:first] == 5.0).all() and (y[first + n:] == 5.0).all() and (y[:, batch * N:] == 5.0).all()
+        assert torch.equal(y[~others, :batch * N], all_rows[~others, :batch * N]), stretches
+        assert (y[others] == 5.0).all() and (y[:, batch * N:] == 5.0).all()
 
 
 # ---- tiles cut along K (llam_seq_linear_within) ------------------------------------------------------------

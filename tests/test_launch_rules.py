@@ -325,20 +325,23 @@ def test_some_rows_get_a_tile_of_as_many_groups(tmp_path):
     layers = [(M, N, K, batch, dtype) for dtype in (0, 1) for M, N, K, batch in
               [(*s, 1) for s in test_gpu_linear_tiled.SHAPES] + [(601, 512, 128, 16), (2049, 128, 512, 16), (1025, 512, 128, 64)]]
     found = fake_hip.run(tmp_path, SLICED + f"""
-def rows(M, N, K, batch, dtype, first, n):
+def rows(M, N, K, batch, dtype, *stretches):
     a = sq.LinearArgs(d_a=p, d_w=p, d_y=p, M=M, N=N, K=K, lda=K * batch, ldy=N * batch, batch=batch, a_stride=K, w_stride=N * K, y_stride=N)
-    ok = lib.llam_seq_linear_rows(ctypes.byref(a), first, n, dtype, 0, None)
+    first, n = ((ctypes.c_int32 * len(stretches))(*(s[i] for s in stretches)) for i in (0, 1))
+    ok = lib.llam_seq_linear_rows(ctypes.byref(a), len(stretches), first, n, dtype, 0, None)
     return [ok] + [l[1:] for l in log() if l[0] == "launch"]
-answer([[[rows(*l, first, n) for first, n in ((0, l[0]), (l[0] // 2, 1), (0, 17), (3, 0))] for l in {layers}],
-        [rows(40, 64, 128, 1, 0, first, n)[0] for first, n in ((-1, 5), (0, 41), (40, 1), (2, -1), (40, 0))], rows(16, 64, 128, 1, 0, 0, 16)[0]])""")
+answer([[[rows(*l, *s) for s in ([(0, l[0])], [(l[0] // 2, 1)], [(0, 2), (5, 7), (13, 4)], [])] for l in {layers}],
+        [rows(40, 64, 128, 1, 0, *s)[0] for s in ([(-1, 5)], [(0, 41)], [(40, 1)], [(2, 0)], [(3, 2), (4, 1)], [(3, 2), (0, 1)], [(3, 2), (5, 35)])],
+        rows(40, 64, 128, 1, 0, *[(i, 1) for i in range(0, 40, 2)]), rows(16, 64, 128, 1, 0, (0, 16))[0]])""")
     for (M, N, K, batch, dtype), (whole, *some, none) in zip(layers, found[0]):
         assert none == [True]
         (height, width, _, _, groups, *_), = [tuple(map(int, re.findall(r"\d+", WIDE.search(whole[1][0]).group(2))))]
-        assert [int(v) for v in whole[1][1:3]] == [over(M, height) * over(N, width), batch]
-        for ok, launch in some:
+        assert [int(v) for v in whole[1][1:4]] == [over(M, height) * over(N, width), batch, 1]
+        for (ok, launch), stretches in zip(some, (1, 3)):
             tile = tuple(map(int, re.findall(r"\d+", WIDE.search(launch[0]).group(2))))
-            assert ok and tile[4] == groups and tile[0] <= height and int(launch[1]) == over(N, tile[1])
-    assert found[1] == [False] * 4 + [True] and found[2] is False
+            assert ok and tile[4] == groups and tile[0] <= height and [int(v) for v in launch[1:4]] == [over(N, tile[1]), batch, stretches]
+    assert found[1] == [False] * 6 + [True] and found[3] is False
+    assert [int(l[3]) for l in found[2][1:]] == [8, 8, 4]
 
 
 # ---- latent portions with keys and values of every head (sequence_model.cpp: latent_expands) -----------------
@@ -379,12 +382,12 @@ answer([steps(layer("heads of 64"), "float32", 1024, 1024, [(0, 60)], [(0, 400)]
 
 
 def test_latent_products_are_of_the_rows_that_stay(tmp_path):
-    """Beside portions that are expanded, W_uk and W_uv meet the others' rows alone, those that lie together at once."""
-    found = fake_hip.run(tmp_path, LATENT.replace("[next((", "[l[1:4] if l[3] == '40' and 'linear_' in l[1] else next((") + """
+    """Beside portions that are expanded, W_uk and W_uv meet the others' rows alone, in one launch."""
+    found = fake_hip.run(tmp_path, LATENT.replace("[next((", "[l[1:5] if l[3] == '40' and 'linear_' in l[1] else next((") + """
 answer(steps(layer("heads of 64"), "float32", 1024, 1600, [(0, 400)], [(0, 400), (500, 1)], [(0, 60), (0, 400), (500, 1), (0, 450), (0, 30), (7, 1)])[1])""")
     for launches, rows, expanded in zip(found, ([], [1], [60, 1, 31]), (1, 1, 2)):
         products = [l for l in launches if isinstance(l, list)]
-        assert len(products) == 2 * (len(rows) + expanded)
-        for (name, x, _), n, N in zip(products, rows * 2, [384] * len(rows) + [64] * len(rows)):
+        assert len(products) == 2 * (len(rows) > 0) + 2 * expanded
+        for (name, x, _, z), N in zip(products, [384, 64] * (len(rows) > 0)):
             height, width = map(int, re.findall(r"\d+", WIDE.search(name).group(2))[:2])
-            assert int(x) == over(n, height) * over(N, width) and height <= 128
+            assert int(x) == over(max(rows), height) * over(N, width) and height <= 128 and int(z) == len(rows)
