@@ -9,6 +9,7 @@
 #include <cstdio>
 #include <cstring>
 #include <map>
+#include <numeric>
 #include <utility>
 #include <vector>
 
@@ -195,6 +196,7 @@ namespace
     {
         int M = 0, single = 0;
         int max_len = 1; // bound on the length of the one-token entries' sequences
+        std::vector<int> from;                 // the caller's row of each row (empty: the same)
         std::vector<int> ntok, len, slot, row; // the portions' tokens, their sequences' lengths afterwards, slots, and first rows
         // runs of portions that the recurrent mixers launch together: entries first .. first + n - 1, the most tokens
         struct Run
@@ -481,10 +483,16 @@ namespace
                     return false;
                 if (w.ffn != LLAM_FFN_NONE && !w.parallel && !ffn(w, s))
                     return false;
-                if (md.trace && !hip_ok(fn, "hipMemcpy2DAsync", hipMemcpy2DAsync(md.trace + (size_t)l * s.M * c.width, (size_t)c.width * 4, md.x,
-                                                                                 (size_t)md.wp * 4, (size_t)c.width * 4, s.M,
-                                                                                 hipMemcpyDeviceToHost, md.stream)))
-                    return false;
+                for (int r = 0, n; md.trace && r < s.M; r += n)
+                {
+                    const int to = s.from.empty() ? r : s.from[r];
+                    for (n = 1; r + n < s.M && (s.from.empty() || s.from[r + n] == to + n); ++n)
+                        ;
+                    if (!hip_ok(fn, "hipMemcpy2DAsync", hipMemcpy2DAsync(md.trace + ((size_t)l * s.M + to) * c.width, (size_t)c.width * 4,
+                                                                         md.x + (size_t)r * md.wp, (size_t)md.wp * 4, (size_t)c.width * 4, n,
+                                                                         hipMemcpyDeviceToHost, md.stream)))
+                        return false;
+                }
             }
             return true;
         }
@@ -521,6 +529,31 @@ namespace
         if (pos < 0 || ntok < 1 || pos > md.cfg.cap - ntok)
             return fail(fn, "%d tokens at position %d do not fit the %d positions of a slot", ntok, pos, md.cfg.cap);
         return true;
+    }
+
+    // The order of a step's entries in its rows: as given, or first the single tokens, then the portions that attend in latent space, then
+    // the expanded ones, where the second kind would lie in three or more stretches.  Portions side by side share launches: us a layer, 16
+    // heads, in turn and one kind after the other, fp32 200 and 100 tokens, four of each 443, 360, bf16 600 and 100, three of each 304, 269;
+    // two of each gain nothing (bf16 800 and 200 244, 239, 64 heads of 300 and 100 361, 369).
+    constexpr int LATENT_STRETCHES = 3;
+    std::vector<int> row_order(const Model &md, int n, const int32_t *pos, const int32_t *ntok)
+    {
+        std::vector<int> order(n), kind(n, 0);
+        std::iota(order.begin(), order.end(), 0);
+        const auto latent = std::find_if(md.layers.begin(), md.layers.end(), [](const llam_seqm_layer &w) { return w.mixer == LLAM_MIXER_LATENT_ATTENTION; });
+        if (latent == md.layers.end())
+            return order;
+        int stretches = 0, before = 2; // kind of the portion before
+        for (int e = 0; e < n; ++e)
+            if (ntok[e] > 1)
+            {
+                kind[e] = latent_expands(*latent, ntok[e], pos[e] + ntok[e], md.cfg.dtype, md.scratch_bytes) ? 2 : 1;
+                stretches += kind[e] == 1 && before == 2;
+                before = kind[e];
+            }
+        if (stretches >= LATENT_STRETCHES)
+            std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return kind[a] < kind[b]; });
+        return order;
     }
 } // namespace
 
@@ -843,18 +876,28 @@ extern "C" bool llam_seqm_forward(void *model, int n, const int32_t *h_slot, con
             return fail(fn, "wanted row %d outside the step", h_want[k]);
     int32_t *hm = md->h_meta;
     const int R = c.max_rows;
-    memcpy(hm, h_ids, sizeof(int32_t) * s.M);
+    const std::vector<int> order = row_order(*md, n, h_pos, h_ntok); // of the entries' rows, and of the portions
     int at = 0, placed = 0;
-    std::vector<int> row0(n);
-    for (int e = 0; e < n; ++e)
+    std::vector<int> row0(n), first(n), row_of(s.M); // first: of the caller's rows
+    for (int e = 1; e < n; ++e)
+        first[e] = first[e - 1] + h_ntok[e - 1];
+    const bool turned = !std::is_sorted(order.begin(), order.end());
+    for (int e : order)
     {
         row0[e] = at;
         for (int t = 0; t < h_ntok[e]; ++t, ++at)
         {
+            hm[at] = h_ids[first[e] + t];
             hm[R + at] = h_slot[e];
             hm[2 * R + at] = h_pos[e] + t;
+            row_of[first[e] + t] = at;
+            if (turned)
+                s.from.push_back(first[e] + t);
         }
     }
+    std::vector<int32_t> want(n_want);
+    for (int k = 0; k < n_want; ++k)
+        want[k] = row_of[h_want[k]];
     auto place = [&](int e) {
         int32_t *q = hm + 4 * R;
         q[placed] = row0[e];
@@ -870,7 +913,7 @@ extern "C" bool llam_seqm_forward(void *model, int n, const int32_t *h_slot, con
             s.max_len = std::max(s.max_len, h_pos[e] + 1);
         }
     s.single = placed;
-    for (int e = 0; e < n; ++e)
+    for (int e : order)
         if (h_ntok[e] > 1)
         {
             s.add(placed, h_ntok[e], h_pos[e] + h_ntok[e], h_slot[e], row0[e]);
@@ -886,7 +929,7 @@ extern "C" bool llam_seqm_forward(void *model, int n, const int32_t *h_slot, con
     for (int w0 = 0; w0 < n_want; w0 += LOGIT_ROWS)
     {
         const int k = std::min(LOGIT_ROWS, n_want - w0);
-        if (!hip_ok(fn, "hipMemcpyAsync", hipMemcpyAsync(md->want(), h_want + w0, (size_t)k * 4, hipMemcpyHostToDevice, md->stream)) ||
+        if (!hip_ok(fn, "hipMemcpyAsync", hipMemcpyAsync(md->want(), want.data() + w0, (size_t)k * 4, hipMemcpyHostToDevice, md->stream)) ||
             !run.logits(md->want(), k))
             return false;
         if (h_logits && !hip_ok(fn, "hipMemcpy2DAsync", hipMemcpy2DAsync(h_logits + (size_t)w0 * c.vocab, (size_t)c.vocab * 4, md->logits,

@@ -488,6 +488,27 @@ def test_expanded_portions_beside_others(dtype):
     model.close()
 
 
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_portions_of_both_kinds_in_turn(dtype):
+    """Rows are taken in another order where latent and expanded portions take turns: the same bits as one kind after the other, what is asked
+    for in the caller's order."""
+    latent, shared = EXPANDED["heads of 64"], sm.latent(kv_from=0, heads=30, dim=50, vdim=64, q_rank=90, scale=0.2)
+    shared["mixer"]["kv_rank"] = latent["mixer"]["kv_rank"]
+    cfg = sm.config(latent, sm.mlstm(mlp=sm.moe()), shared, width=64)
+    model = load(cfg, sm.random_weights(cfg, 7), dtype, slots=9, cap=520, max_rows=1700)
+    tokens = [tokens_of(cfg, n, seed=b) for b, n in enumerate([30, 500, 17, 450, 3, 2, 420, 8])]
+    wanted, got, traces = [0, 29, 400, 529, 530, 700, 1000, 1001, 1003, 1200, 1429], [], []
+    for order in (range(8), (0, 2, 4, 5, 7, 1, 3, 6)):
+        start = np.cumsum([0] + [len(tokens[b]) for b in order])
+        row = {(b, t): start[i] + t for i, b in enumerate(order) for t in range(len(tokens[b]))}
+        plain = [(b, t) for b in range(8) for t in range(len(tokens[b]))]
+        entries = [(b, 0, tokens[b]) for b in order] + [(8, 0, tokens[4][:1])]
+        got.append(model.forward(entries, [int(row[plain[w]]) for w in wanted] + [1430]))
+        traces.append(model.trace_layers(entries)[:, [row[p] for p in plain] + [1430]])
+    assert np.array_equal(got[0], got[1]) and np.array_equal(traces[0], traces[1])
+    model.close()
+
+
 @pytest.mark.parametrize("N,K,batch", [(64, 64, 1), (96, 32, 3), (512, 128, 16), (320, 192, 5)])
 def test_tiles_of_the_transposed_matrix(dev, N, K, batch):
     import torch

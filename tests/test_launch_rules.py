@@ -382,10 +382,13 @@ answer([steps(layer("heads of 64"), "float32", 1024, 1024, [(0, 60)], [(0, 400)]
 
 
 def test_latent_products_are_of_the_rows_that_stay(tmp_path):
-    """Beside portions that are expanded, W_uk and W_uv meet the others' rows alone, in one launch."""
+    """Beside portions that are expanded, W_uk and W_uv meet the others' rows alone, in one launch;
+    where portions of both kinds take turns, those that stay go first."""
     found = fake_hip.run(tmp_path, LATENT.replace("[next((", "[l[1:5] if l[3] == '40' and 'linear_' in l[1] else next((") + """
-answer(steps(layer("heads of 64"), "float32", 1024, 1600, [(0, 400)], [(0, 400), (500, 1)], [(0, 60), (0, 400), (500, 1), (0, 450), (0, 30), (7, 1)])[1])""")
-    for launches, rows, expanded in zip(found, ([], [1], [60, 1, 31]), (1, 1, 2)):
+answer(steps(layer("heads of 64"), "float32", 1024, 1600, [(0, 400)], [(0, 400), (500, 1)], [(0, 60), (0, 400), (500, 1), (0, 450), (0, 30), (7, 1)],
+             [(0, 60), (0, 400), (0, 30), (0, 450), (7, 1), (0, 350)], [(0, 60), (0, 400), (0, 30), (0, 450), (7, 1), (0, 20)])[1])""")
+    assert found[4].index("transpose_tiles") > max(i for i, l in enumerate(found[4]) if l == "latent_attention")
+    for launches, rows, expanded in zip(found, ([], [1], [60, 1, 31], [60, 30, 1], [111]), (1, 1, 2, 3, 2)):
         products = [l for l in launches if isinstance(l, list)]
         assert len(products) == 2 * (len(rows) > 0) + 2 * expanded
         for (name, x, _, z), N in zip(products, [384, 64] * (len(rows) > 0)):
