@@ -160,19 +160,24 @@ namespace
         return at;
     }
     // Attending in latent space takes sums of kv_rank for every score and every output column, twice for outputs of two pieces, where
-    // keys and values of every head take sums of the head's width, but have to be made from every latent row first.  Worth it from
-    // so many multiplications on (one portion, us a layer with its projections, in latent space and expanded):
-    //   16 heads of 128, rank 512, bf16, width 2048: 251 tokens 76, 74; 512 94, 84; 1024 157, 122; 2048 277, 202; 512 at 1536 138, 112; 512 at
-    //   7680 313, 197; 128 at 1920 85, 89; 128 at 8064 127, 139; 64 at 8128 102, 134
-    //   64 heads, width 5120: 100 tokens 112, 106; 251 167, 143; 512 221, 196; 1024 437, 309; 2048 1052, 677; 128 at 1920 178, 185; 64 at 8128 222, 374
-    //   16 heads, fp32: 100 tokens 110, 96; 200 139, 106; 512 275, 137; 2048 1606, 556; 128 at 1920 247, 138
-    // (Portions in latent space share launches, expanded ones do not: the line lies where a portion gains some 10 us alone.)  A portion's own sizes
-    // decide, so that its outputs do not depend on those beside it.
+    // keys and values of every head take sums of the head's width, but have to be made from every latent row first.  (32-bit attention
+    // multiplies 32-bit values, at less than a fifth of the rate at which these are made in pieces.)  Worth it from so many multiplications
+    // on, in bf16 also those in whose time W_uk is turned, some 280 a value.  One portion, us a layer with its projections, in latent space and
+    // expanded, and with one token beside it that stays (tests/test_launch_rules.py holds the sides of the line):
+    //   16 heads of 128, rank 512, bf16, width 2048: 512 tokens 95 81, 127 113; 600 114 97, 131 122; 1024 142 115, 159 143; 128 at 1920
+    //   88 86, 104 110; 400 at 1920 154 113, 169 138; 128 at 7680 128 144, 145 168; 256 at 7680 186 164, 202 186
+    //   64 heads, width 5120: 300 tokens 172 163, 190 194; 400 192 181, 213 212; 600 253 247, 279 276; 128 at 1920 180 184, 204 212
+    //   16 heads, fp32: 100 tokens 108 95, 129 128; 200 136 103, 160 136; 48 at 512 104 95, 126 130; 64 at 512 122 96, 149 135; 128 at 1920 245 133, 273 167;
+    //   32 at 7680 244 240, 266 280; 64 at 7680 392 245, 420 285
+    // Portions in latent space share launches, expanded ones do not: the line lies above where a portion gains by itself (us a layer of all, fp32:
+    // 187, 174 and 161 tokens 197 207; eight of 200 421 434, of 251 622 466; bf16, 64 heads, eight of 300 724 790).  A portion's own sizes decide,
+    // so that its outputs do not depend on those beside it.
     bool latent_gains(const llam_seqm_layer &w, int ntok, int len, int dtype)
     {
-        const double dp = P(w.dim), vp = P(w.vdim), rp = P(w.kv_rank), pieces = dtype == LLAM_SEQ_F32 ? 1 : 2;
-        const double saved = ntok * (len - 0.5 * ntok) * (rp - dp + pieces * (rp - vp)) - (double)(len - ntok) * (dp + vp) * rp;
-        return ntok > ROW_MAX && saved * w.heads > (dtype == LLAM_SEQ_F32 ? 0.2e9 : 3.0e9);
+        const bool f32 = dtype == LLAM_SEQ_F32;
+        const double dp = P(w.dim), vp = P(w.vdim), rp = P(w.kv_rank), pieces = f32 ? 1.0 : 2.0, made = f32 ? 0.18 : 1.0;
+        const double saved = ntok * (len - 0.5 * ntok) * (rp - dp + pieces * (rp - vp)) - made * (len - ntok) * (dp + vp) * rp;
+        return ntok > ROW_MAX && saved * w.heads > (f32 ? 0.23e9 : 2.8e9 + 280.0 * w.heads * dp * rp);
     }
     constexpr size_t EXPANSION_BYTES = (size_t)320 << 20; // at most
     bool latent_expands(const llam_seqm_layer &w, int ntok, int len, int dtype, size_t scratch_bytes)

@@ -381,6 +381,19 @@ answer([steps(layer("heads of 64"), "float32", 1024, 1024, [(0, 60)], [(0, 400)]
     assert [count(l)[0] for l in small[1]] == [0] and small[0] < single[0]
 
 
+def test_the_line_of_expanded_portions(tmp_path):
+    """Portions that were measured on both sides (sequence_model.cpp: latent_gains), by heads and type: tokens and positions before them."""
+    sides = [(16, "bfloat16", [(600, 0), (1024, 0), (400, 1920), (256, 7680)], [(512, 0), (128, 1920), (128, 7680)]),
+             (64, "bfloat16", [(400, 0), (600, 0)], [(300, 0), (128, 1920)]),
+             (16, "float32", [(200, 0), (251, 0), (64, 512), (48, 1920), (128, 1920), (64, 7680)], [(100, 0), (187, 0), (48, 512), (17, 1920), (32, 7680)]),
+             (40, "float32", [(130, 0), (64, 512), (64, 1920)], [(100, 0), (17, 512), (32, 1920)])]
+    found = fake_hip.run(tmp_path, LATENT + f"""
+answer([[["transpose_tiles" in got for got in steps(sm.latent(heads=heads, dim=128, vdim=128, q_rank=64, kv_rank=512), dtype, 8000, 1100,
+                                                    *[[(at, n)] for n, at in side])[1]] for side in (gains, stays)] for heads, dtype, gains, stays in {sides}])""")
+    for (gains, stays), (_, _, a, b) in zip(found, sides):
+        assert gains == [True] * len(a) and stays == [False] * len(b)
+
+
 def test_latent_products_are_of_the_rows_that_stay(tmp_path):
     """Beside portions that are expanded, W_uk and W_uv meet the others' rows alone, in one launch;
     where portions of both kinds take turns, those that stay go first."""
