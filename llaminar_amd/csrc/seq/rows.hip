@@ -3,6 +3,7 @@
 #include "linear.h"
 #include <algorithm>
 #include <climits>
+#include <type_traits>
 
 namespace llamql
 {
@@ -187,7 +188,7 @@ namespace llamql
 
     constexpr int EXPERT_WAVES = 8;
     // The lists of few rows, by one workgroup beside those of the up projections, which need none (by the launch that chooses: 1.8 us more).
-    __device__ __forceinline__ void expert_list(const ExpertArgs &p, int M, ExpertLists lists)
+    __device__ __forceinline__ void expert_list(const ExpertArgs &p, int M, ExpertLists lists, int from, int step)
     {
         constexpr int THREADS = EXPERT_WAVES * 64, BLOCKS = 64 * ROUTE_MAX / 64; // of experts, 64 in each
         struct Choice
@@ -201,7 +202,7 @@ namespace llamql
         const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
         for (int i = threadIdx.x; i < M * p.top; i += THREADS)
             s_choice[i] = {p.ids[i], p.weights[i + i / p.top]};
-        for (int first = 0; first < M; first += lists.rows)
+        for (int first = from * lists.rows; first < M; first += step * lists.rows)
         {
             int *list = lists.at(p.lists, first / lists.rows);
             for (int i = threadIdx.x; i < 64 * ROUTE_MAX; i += THREADS)
@@ -304,8 +305,8 @@ namespace llamql
         unsigned long long mine = n < M ? 1 : 0; // which of token n's choices the expert is (several: logits that are not numbers)
         if (shared)
         {
-            if (m == 1 && tile == 0)
-                expert_list(p, M, lists);
+            if (m >= 1 && tile == 0)
+                expert_list(p, M, lists, m - 1, M - 1);
             if (m > 0 || tile * 16 >= p.shared_ff)
                 return;
         }
@@ -389,115 +390,145 @@ namespace llamql
     // experts, in the order of their numbers, so its bits are the same whatever other rows there are, also none.
     // HALF: rows 8 .. of the matrix unit's first operand are the same columns' second k-step of the two, and columns 8 .. of the
     // second operand the rows' (see linear_small_tile): twice the workgroups, and one product where there were two.
-    // Bound by the weights, and for one or two rows by the chain of list, first weights and sums.  A layer of 6 of 64 experts of 1408 x 2048 and a
-    // shared one of 2816, us, against a workgroup for every row that read its own experts: 8 rows that choose alike (12 experts in all) bf16
-    // 63.8 -> 45.9, fp32 108 -> 62.8; that choose evenly (35) 95.7 -> 86.8, 142 -> 126; 16 rows 156 -> 135; 1 row 25.7 -> 24.0, fp32 41.1 -> 33.2.
-    // 16 rows at 1536 x 5120: 423 -> 332.  Slower only where small experts are hardly shared: 4 rows, 8 of 128 of 768 x 2048 45.7 -> 48.9, fp32 58 -> 65.
-    template <typename T, bool HALF>
+    // U: steps asked for at once, two turns of them on their way.
+    // Bound by the weights, and for one or two rows by the chain of list, first weights and sums.  The weights were waited for where they were asked
+    // for (the turn that is used was a copy of the one that came), and with small experts the walk from one to the next, by what LDS says, took as
+    // long as they did.  us of this launch, 6 of 64 experts of 1408 x 2048 and a shared one of 2816 (in brackets: a workgroup for every row that
+    // reads its own experts): 8 rows bf16 (47) 37.7 -> 37.8, fp32 (76) 57 -> 53; 16 rows 63.4 -> 57, 94 -> 88; 1 row (12) 10.7 -> 10.3,
+    // (24) 15.9 -> 15.2.  8 of 128 of 768 x 2048, evenly chosen, 4 rows (17.2) 19.7 -> 17.7, fp32 (23) 29.5 -> 25.6; 8 rows (30.4) 32 -> 29, (43) 50 -> 42.
+    // 4 of 128 of 256 x 1024, 8 rows (5.8) 12 -> 7.7.  16 rows at 1536 x 5120 177 -> 174, fp32 238 -> 223.
+    // Slower than a workgroup for every row only where experts are hardly shared: a layer of 4 rows, 8 of 128 of 768 x 2048 45.6 and 47.0, fp32
+    // 58.1 and 61.1, and by the list's 1 to 2 us at widths of 1024 and less.
+    // Halves with U = 3 or 4: 8 rows 40.8, 41.2; U = 1, bf16, 8 rows 41, 9 rows 45.7 against 42.8, 12 rows 53.2 and 53.6, 16 rows 57 and 65.5.
+    constexpr int DOWN_MANY = 10; // rows from beyond which on a step at a time is better
+    template <typename T, bool HALF, int U>
     __global__ void __launch_bounds__(EXPERT_WAVES * 64, 4)
         expert_down_small_kernel(ExpertArgs p, int M, ExpertLists lists)
     {
         using O = Operand<T>;
         using V = typename O::V;
-        constexpr int P = HALF ? 1 : 2;                    // products of a step
-        constexpr int U = sizeof(T) == 2 ? 4 / P : 3 / P;  // steps in flight
+        constexpr int P = HALF ? 1 : 2; // products of a step
         __shared__ __attribute__((aligned(16))) float s_red[EXPERT_WAVES][P][64][4];
-        extern __shared__ __attribute__((aligned(16))) char smem[]; // the list's uses and numbers
+        extern __shared__ __attribute__((aligned(16))) char smem[]; // the list's uses
         const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), n = lane & 15, g = lane >> 4;
         const int tile = HALF ? blockIdx.x >> 1 : blockIdx.x;
         const int second = HALF ? n >> 3 : 0, row = HALF ? n & 7 : n, first = blockIdx.y * lists.rows;
         const int rows = lists.rows < M - first ? lists.rows : M - first, mine = row < rows ? row : 0;
         const int piece = (HALF ? g * 16 + (blockIdx.x & 1) * 8 + (n & 7) : lane) + second * 64;
-        const int pitch = p.top * p.ff + p.shared_ff;
+        const int pitch = p.top * p.ff + p.shared_ff, esteps = p.ff >> 6, ssteps = p.shared_ff >> 6;
         // (the shared expert is the first of the list here, of a number that turns nothing)
         const int own = p.shared_ff ? 1 : 0;
         int *list = lists.at(p.lists, blockIdx.y);
+        const auto number = [&](int job) __attribute__((always_inline)) {
+            const int at = job - own < lists.most ? job - own : lists.most - 1;
+            return at < 0 ? -EXPERT_WAVES : lists.numbers(list)[at];
+        };
+        int coming = number(lane);
+        const int count = own + __builtin_amdgcn_readfirstlane(list[0]);
         ExpertUse *uses = reinterpret_cast<ExpertUse *>(smem);
-        int *numbers = reinterpret_cast<int *>(uses + (lists.most + own) * lists.rows);
         for (int i = threadIdx.x; i < lists.most * lists.rows; i += EXPERT_WAVES * 64)
             uses[own * lists.rows + i] = lists.uses(list)[i];
-        for (int i = threadIdx.x; i < lists.most; i += EXPERT_WAVES * 64)
-            numbers[own + i] = lists.numbers(list)[i];
         if (own && (int)threadIdx.x < rows)
             uses[threadIdx.x] = expert_use(p.weights[(first + threadIdx.x) * (p.top + 1) + p.top], (first + threadIdx.x) * pitch + p.top * p.ff, true);
-        if (own && threadIdx.x == 0)
-            numbers[0] = -EXPERT_WAVES;
-        const int count = own + __builtin_amdgcn_readfirstlane(list[0]);
-        __syncthreads();
 
-        // the wavefront's place: steps that are left of the `job`-th of the list (none: it has none of that expert's), the next one's
-        // weights and this lane's activations; past the end those of the last expert's step 0, which every expert has
-        int job = 0, left = 0;
-        const u32x4 *w = nullptr;
-        const T *b = nullptr;
-        ExpertUse use = {};
-        const auto enter = [&]() __attribute__((always_inline)) {
-            const int id = __builtin_amdgcn_readfirstlane(numbers[job]), start = (wave + id) & (EXPERT_WAVES - 1);
-            const int steps = (id < 0 ? p.shared_ff : p.ff) >> 6;
-            const bf16 *matrix = id < 0 ? p.shared_down : p.down + (size_t)id * p.down_stride;
-            use = uses[job * lists.rows + mine];
-            left = start < steps ? (steps - start + EXPERT_WAVES - 1) / EXPERT_WAVES : 0;
-            const int at = left > 0 ? start : 0;
-            w = reinterpret_cast<const u32x4 *>(matrix) + ((size_t)tile * steps + at) * 128;
-            b = static_cast<const T *>(p.act) + (size_t)(use.act & 0x7fffffff) + at * 64 + 8 * g + second * 32;
-        };
-        const auto advance = [&]() __attribute__((always_inline)) {
-            while (left == 0 && ++job < count)
-                enter();
-        };
-        struct Held
-        {
-            u32x4 raw[U][P];
-            V b[U][P];
-            float scale[U];
-            bool chosen[U];
-        };
-        Held next;
-        const auto fetch = [&]() __attribute__((always_inline)) {
-#pragma unroll
-            for (int u = 0; u < U; ++u)
-            {
-                const bool live = job < count;
-#pragma unroll
-                for (int i = 0; i < P; ++i)
-                {
-                    next.raw[u][i] = w[i * 64 + piece];
-                    next.b[u][i] = O::load(b + i * 32);
-                }
-                next.scale[u] = use.weight;
-                next.chosen[u] = live && use.act < 0;
-                if (live)
-                {
-                    // (the last one of an expert stays where it is, within it)
-                    if (--left > 0)
-                        w += EXPERT_WAVES * 128, b += EXPERT_WAVES * 64;
-                    else
-                        advance();
-                }
-            }
-        };
         f32x4 acc[P];
 #pragma unroll
         for (int i = 0; i < P; ++i)
             acc[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-        enter();
-        advance();
-        fetch();
-        for (bool more = true; more;)
+        for (int w0 = 0; w0 < count; w0 += 64)
         {
-            const Held cur = next;
-            more = job < count;
-            if (more)
-                fetch();
+            // Lane j: the (w0 + j)-th of the list, the first of its steps among the wavefront's and their end.  An expert has as many as the
+            // others or one more, so they are counted by one ballot and a step is found by another.
+            const int job = w0 + lane, id = job < count ? coming : 0, start = (wave + id) & (EXPERT_WAVES - 1);
+            coming = number(job + 64);
+            const bool shared = own && job == 0;
+            const int each = esteps / EXPERT_WAVES, some = (shared ? ssteps : esteps) & (EXPERT_WAVES - 1);
+            const unsigned long long more = __ballot(job >= own && job < count && start < some);
+            const int before = w0 > 0 || own == 0 || lane == 0 ? lane * each
+                               : (lane - 1) * each + ssteps / EXPERT_WAVES + (wave < (ssteps & (EXPERT_WAVES - 1)) ? 1 : 0);
+            const int from = before + __builtin_popcountll(more & ((1ull << lane) - 1));
+            const int end = job < count ? from + (shared ? ssteps : esteps) / EXPERT_WAVES + (start < some ? 1 : 0) : INT_MAX;
+            const int total = __builtin_amdgcn_readlane(end, (count - w0 < 64 ? count - w0 : 64) - 1);
+            // the wavefront's steps s0 .. : their weights, their place in the expert, its uses (past the end the last step again, for no row)
+            const u32x4 *w[U];
+            int at[U], use_at[U];
+            ExpertUse use[U];
+            const auto find = [&](int s0) __attribute__((always_inline)) {
 #pragma unroll
-            for (int u = 0; u < U; ++u)
-#pragma unroll
-                for (int i = 0; i < P; ++i)
+                for (int u = 0; u < U; ++u)
                 {
-                    const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
-                    const f32x4 sum = acc[i] + O::mma(O::from_weights(cur.raw[u][i]), cur.b[u][i], zero) * cur.scale[u];
-                    acc[i] = cur.chosen[u] ? sum : acc[i];
+                    const int s = s0 + u < total ? s0 + u : total - 1;
+                    const int j = __builtin_popcountll(__ballot(end <= s));
+                    const int e = __builtin_amdgcn_readlane(id, j), steps = e < 0 ? ssteps : esteps;
+                    at[u] = ((wave + e) & (EXPERT_WAVES - 1)) + (s - __builtin_amdgcn_readlane(from, j)) * EXPERT_WAVES;
+                    w[u] = reinterpret_cast<const u32x4 *>(e < 0 ? p.shared_down : p.down + (size_t)e * p.down_stride) + ((size_t)tile * steps + at[u]) * 128;
+                    use_at[u] = (w0 + j) * lists.rows + mine;
                 }
+            };
+            const auto look = [&]() __attribute__((always_inline)) {
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+                    use[u] = uses[use_at[u]];
+            };
+            // Two turns of steps, one after the other: handed over (cur = next), the weights were waited for where they were asked for.
+            u32x4 raw[2][U][P];
+            V b[2][U][P];
+            float scale[2][U];
+            int act[2][U];
+            const auto ask = [&](auto half) __attribute__((always_inline)) {
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+#pragma unroll
+                    for (int i = 0; i < P; ++i)
+                        raw[half.value][u][i] = w[u][i * 64 + piece];
+            };
+            const auto meet = [&](auto half, int s0) __attribute__((always_inline)) {
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+                {
+                    const T *from = static_cast<const T *>(p.act) + (size_t)(use[u].act & 0x7fffffff) + at[u] * 64 + 8 * g + second * 32;
+#pragma unroll
+                    for (int i = 0; i < P; ++i)
+                        b[half.value][u][i] = O::load(from + i * 32);
+                    scale[half.value][u] = use[u].weight;
+                    act[half.value][u] = s0 + u < total ? use[u].act : 0;
+                }
+                find(s0 + U); // (a turn ahead of the weights)
+                look();
+            };
+            const auto add = [&](auto half) __attribute__((always_inline)) {
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+#pragma unroll
+                    for (int i = 0; i < P; ++i)
+                    {
+                        const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+                        const f32x4 sum = acc[i] + O::mma(O::from_weights(raw[half.value][u][i]), b[half.value][u][i], zero) * scale[half.value][u];
+                        acc[i] = act[half.value][u] < 0 ? sum : acc[i];
+                    }
+            };
+            const std::integral_constant<int, 0> one;
+            const std::integral_constant<int, 1> two;
+            if (total > 0)
+            {
+                find(0);
+                ask(one);
+            }
+            if (w0 == 0)
+                __syncthreads(); // the uses are in LDS
+            if (total == 0)
+                continue;
+            look();
+            meet(one, 0);
+            for (int s = 0; s < total; s += 2 * U)
+            {
+                ask(two);
+                meet(two, s + U);
+                add(one);
+                ask(one);
+                meet(one, s + 2 * U);
+                add(two);
+            }
         }
 #pragma unroll
         for (int i = 0; i < P; ++i)
@@ -648,7 +679,7 @@ namespace llamql
             s.weights = take((size_t)M * (top + 1) * 4);
             s.act = take((pairs * ff + (size_t)M * shared_ff) * 4);
             size_t lists = 0;
-            for (int rows : {EXPERT_ROWS / 2, EXPERT_ROWS})
+            for (int rows = EXPERT_ROWS; rows > 0; rows /= 2)
                 lists = std::max(lists, ceil_div(std::min(M, EXPERT_ROWS), rows) * expert_lists(M, rows, experts, top).ints());
             s.lists = take(lists * 4);
             s.offset = take((size_t)(experts + 1) * 4);
@@ -660,13 +691,13 @@ namespace llamql
             return s;
         }
 
-        template <typename T, bool HALF>
+        template <typename T, bool HALF, int U>
         bool expert_down_launch(const char *fn, const ExpertArgs &p, int M, ExpertLists lists, hipStream_t st)
         {
-            auto *kernel = expert_down_small_kernel<T, HALF>;
+            auto *kernel = expert_down_small_kernel<T, HALF, U>;
             static LdsGrant grant;
-            const size_t use = lists.rows * sizeof(ExpertUse) + 4, lds = (lists.most + (p.shared_ff ? 1 : 0)) * use;
-            if (lds > 48 * 1024 && allow_lds(grant, reinterpret_cast<const void *>(kernel), (64 * ROUTE_MAX + 1) * (EXPERT_ROWS / (HALF ? 2 : 1) * sizeof(ExpertUse) + 4)) != hipSuccess)
+            const size_t use = lists.rows * sizeof(ExpertUse), lds = (lists.most + (p.shared_ff ? 1 : 0)) * use;
+            if (lds > 48 * 1024 && allow_lds(grant, reinterpret_cast<const void *>(kernel), (64 * ROUTE_MAX + 1) * EXPERT_ROWS / (HALF ? 2 : 1) * sizeof(ExpertUse)) != hipSuccess)
                 return fail(fn, "cannot reserve %zu bytes of LDS", lds);
             hipLaunchKernelGGL(kernel, dim3(p.N / (HALF ? 8 : 16), ceil_div(M, lists.rows)), dim3(EXPERT_WAVES * 64), lds, st, p, M, lists);
             return launched(fn);
@@ -691,16 +722,23 @@ namespace llamql
                 static_assert(SMALL_M == EXPERT_ROWS, "a list has a column for each of few rows");
                 // Halves of tiles, for eight rows at a time, but for more rows whole ones where these alone occupy the chip (bf16, us, halves
                 // and whole tiles: 16 rows, 64 experts of 1536 x 5120 351, 332; 16 of 4096 x 4096 207, 170; 64 of 1408 x 2048 135, 141;
-                // 8 rows, 1536 x 5120 226, 238).
+                // 8 rows, 1536 x 5120 226, 238; the down projections alone, 12 rows of 1408 x 2048 54, 62).
                 const bool half = M <= EXPERT_ROWS / 2 || p.N / 16 < cu_count(device_id);
-                const ExpertLists lists = expert_lists(M, half ? EXPERT_ROWS / 2 : EXPERT_ROWS, p.experts, p.top);
+                // Fewer rows at a time where these would leave compute units without a workgroup (us, 8 rows, 4 of 128 of 256 x 1024, lists
+                // of 8 and 4 rows 19.1, 17.9, fp32 25.3, 22.5).
+                int rows = half ? EXPERT_ROWS / 2 : EXPERT_ROWS;
+                while (half && rows > 1 && p.N / 8 * ceil_div(M, rows) < cu_count(device_id))
+                    rows /= 2;
+                const ExpertLists lists = expert_lists(M, rows, p.experts, p.top);
                 p.lists = reinterpret_cast<int *>(scratch + at.lists);
                 const int widest = p.shared_ff > p.ff ? p.shared_ff : p.ff;
                 hipLaunchKernelGGL(expert_up_small_kernel<T>, dim3(widest / 16, p.top + (p.shared_ff || M > 1 ? 1 : 0), M),
                                    dim3(EXPERT_WAVES * 64), 0, st, p, M, lists);
                 if (!launched(fn))
                     return false;
-                return half ? expert_down_launch<T, true>(fn, p, M, lists, st) : expert_down_launch<T, false>(fn, p, M, lists, st);
+                if (!half)
+                    return expert_down_launch<T, false, sizeof(T) == 2 ? 2 : 1>(fn, p, M, lists, st);
+                return M > DOWN_MANY ? expert_down_launch<T, true, 1>(fn, p, M, lists, st) : expert_down_launch<T, true, 2>(fn, p, M, lists, st);
             }
             int *offset = reinterpret_cast<int *>(scratch + at.offset), *order = reinterpret_cast<int *>(scratch + at.order);
             int *place = reinterpret_cast<int *>(scratch + at.place);

@@ -49,6 +49,50 @@ def test_rows_together_are_rows_alone(dev, M, experts, top, ff, shared, dtype):
 @pytest.mark.parametrize("M,experts,top,ff,shared,K", [(1, 6, 4, 64, 64, 128), (8, 40, 3, 576, 0, 192), (9, 5, 5, 64, 1216, 128), (9, 30, 2, 640, 64, 4160),
                                                        (16, 1024, 4, 64, 0, 4096), (16, 300, 64, 64, 64, 192), (13, 2, 1, 192, 0, 4160)])
 def test_few_rows_against_64_bits(dev, M, experts, top, ff, shared, K, dtype):
+    few_rows_against_64_bits(dev, M, experts, top, ff, shared, K, dtype)
+
+
+# lists of some hundred experts, whose uses are more than the 48 KB of LDS that a launch has without asking, up to the most there can be; several
+# windows of 64 experts, with the shared one first; lists of one row, two and four, of eight rows each of experts of one step, of nine
+@pytest.mark.parametrize("dtype", [sq.BF16, sq.F32])
+@pytest.mark.parametrize("M,experts,top,ff,shared,K", [(16, 448, 28, 64, 0, 4096), (16, 1024, 64, 64, 64, 4096), (8, 600, 64, 64, 128, 4096), (16, 600, 64, 64, 704, 2048),
+                                                       (3, 9, 2, 128, 64, 1024), (5, 9, 3, 576, 0, 1024), (11, 40, 7, 64, 0, 512), (16, 70, 5, 576, 576, 256)])
+def test_long_lists_and_short_ones(dev, M, experts, top, ff, shared, K, dtype):
+    few_rows_against_64_bits(dev, M, experts, top, ff, shared, K, dtype)
+
+
+@pytest.mark.parametrize("dtype", [sq.BF16, sq.F32])
+@pytest.mark.parametrize("M,K", [(4, 192), (8, 2048), (9, 4160), (16, 2048)])
+def test_rows_beside_rows_that_are_not_finite(dev, M, K, dtype):
+    """Rows of infinities and of no numbers that chose the same experts: every other row has the bits that it has beside finite ones."""
+    import torch
+
+    lib, experts, top, ff, shared = sq.load(), 5, 3, 192, 64
+    T = torch.float32 if dtype == sq.F32 else torch.bfloat16
+    torch.manual_seed(M)
+    laid = [(torch.randn(n, device=dev) * k ** -0.5).bfloat16() for n, k in ((experts * ff * K, K), (experts * K * ff, ff), (shared * K, K), (K * shared, shared))]
+    logits, h, x = torch.randn(M, 16, device=dev), torch.randn(M, K, device=dev).to(T), torch.randn(M, K, device=dev)
+    logits[:, 1] = 9.0
+    size = lib.llam_seq_experts_scratch_bytes(M, experts, top, ff, shared, K)
+    bad, got = [1, M - 1], []
+    for value in (None, float("inf"), float("nan")):
+        rows, y = h.clone(), x.clone()
+        if value is not None:
+            rows[bad[0], 0], rows[bad[1], 3] = value, -value
+        scratch = torch.full((size,), 255, dtype=torch.uint8, device=dev)
+        a = sq.ExpertsArgs(d_logits=logits.data_ptr(), ldz=16, d_up=laid[0].data_ptr(), d_down=laid[1].data_ptr(), up_stride=ff * K, down_stride=ff * K,
+                           experts=experts, top=top, ff=ff, shared_ff=shared, K=K, N=K, d_h=rows.data_ptr(), d_x=y.data_ptr(), ldx=K,
+                           d_shared_up=laid[2].data_ptr(), d_shared_down=laid[3].data_ptr())
+        assert lib.llam_seq_experts(ctypes.byref(a), M, scratch.data_ptr(), size, dtype, 0, torch.cuda.current_stream().cuda_stream), lib.llam_ql_last_error()
+        torch.cuda.synchronize()
+        got.append(y)
+    good = [m for m in range(M) if m not in bad]
+    for y in got[1:]:
+        assert torch.equal(y[good], got[0][good]) and torch.isfinite(y[good]).all()
+    assert not torch.isfinite(got[1][bad]).any()  # (of sums that are no numbers max(z, 0) is 0)
+
+
+def few_rows_against_64_bits(dev, M, experts, top, ff, shared, K, dtype):
     import torch
 
     T = torch.float32 if dtype == sq.F32 else torch.bfloat16
