@@ -104,8 +104,20 @@ def test_attention_of_many_entries(dev, dtype):
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("heads,groups,ntok,chunk,pos,n", [(10, 10, 650, 0, 0, 1), (8, 8, 129, 0, 500, 5), (36, 12, 333, 90, 20, 1), (3, 1, 5700, 64, 0, 2)])
 def test_attention_of_several_rounds_of_workgroups(dev, heads, groups, ntok, chunk, pos, n, dtype):
-    """More workgroups than compute units, whose second and fourth round are dealt backwards: a last round that is odd, even, not full."""
+    """More workgroups than compute units, whose second and fourth round are dealt backwards: a last round that is odd, even, not full.
+    (So in fp32: in bf16 walks as short as these keep the order of the grid.)"""
     attend(dev, dtype, heads, groups, 64, 64, ntok, chunk, pos, None, n)
+
+
+# heads, key/value heads, head size, tokens, position, entries: walks long enough for that order in bf16 too (test_launch_rules.py holds them to it), in
+# two stretches and in one, two whole rounds, a last one of half as many workgroups, of a few
+LONG_WALKS = [(16, 4, 128, 2048, 0, 1), (40, 8, 64, 2048, 0, 1), (12, 4, 64, 1500, 37, 2), (6, 2, 64, 900, 200, 9)]
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("heads,groups,dim,ntok,pos,n", LONG_WALKS)
+def test_attention_of_long_walks_in_rounds(dev, heads, groups, dim, ntok, pos, n, dtype):
+    attend(dev, dtype, heads, groups, dim, dim, ntok, 0, pos, None, n)
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])

@@ -469,6 +469,20 @@ def test_keys_and_values_of_every_head(name, dtype):
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_keys_and_values_of_one_head(dtype):
+    """As many tokens as that layer expands in either type (test_launch_rules.py): its products are plain ones, over scratch that holds its matrix
+    and results."""
+    cfg = sm.config(EXPANDED["one head"], width=64)
+    t = sm.random_weights(cfg, 8)
+    tokens = tokens_of(cfg, 1600)
+    want = so.kogilix(cfg, t.plain(), tokens)
+    model = load(cfg, t, dtype, cap=1600, max_rows=1600)
+    for cuts in ([1600], [90, 1510]):
+        check(run(model, 1, tokens, cuts), want, dtype, note=f"{cuts}")
+    model.close()
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 def test_expanded_portions_beside_others(dtype):
     """A step of portions of both kinds and single tokens: each sequence against itself alone, and the same bits whatever lies beside."""
     cfg = sm.config(EXPANDED["heads of 64"], width=64)

@@ -8,7 +8,7 @@ import numpy as np
 import pytest
 
 from oracle.binding import FMT_IQ3_S, FMT_Q4_K, FMT_Q6_K
-from tests import fake_hip, test_gpu_experts_small, test_gpu_gemm, test_gpu_linear_tiled
+from tests import fake_hip, test_gpu_bosirax, test_gpu_experts_small, test_gpu_gemm, test_gpu_linear_tiled
 
 CSRC = Path(__file__).resolve().parent.parent / "llaminar_amd" / "csrc"
 CUS = 256
@@ -344,6 +344,27 @@ answer([[[rows(*l, *s) for s in ([(0, l[0])], [(l[0] // 2, 1)], [(0, 2), (5, 7),
     assert [int(l[3]) for l in found[2][1:]] == [8, 8, 4]
 
 
+# ---- order of the workgroups of attention (grouped_attention.hip: attention_run) -------------------------------
+
+def test_long_walks_are_dealt_in_rounds(tmp_path):
+    """The shapes of the GPU test have more workgroups than compute units, whose walks are long enough for the order of rounds."""
+    found = fake_hip.run(tmp_path, f"""
+from llaminar_amd import sequence as sq
+lib, p = sq.load(), 1 << 20
+def launches(heads, groups, dim, ntok, pos, n, dtype):
+    a = sq.AttentionArgs(heads, groups, dim, dim, -(-(pos + ntok) // 128) * 128, 0, 1.0, p, p)
+    e = sq.Entries(p, p, p, p)
+    assert lib.llam_seq_attention(ctypes.byref(a), p, ctypes.byref(e), 0, n, ntok, pos + ntok, p, heads * dim, p, 1 << 40, dtype, 0, None), lib.llam_ql_last_error()
+    return [int(v) for v in next(l for l in log() if l[0] == "launch" and "16attention_kernel" in l[1])[2:5]]
+answer([[launches(*case, dtype) for dtype in (0, 1)] for case in {test_gpu_bosirax.LONG_WALKS}])""")
+    long = int(re.search(r"ATT_LONG = (\d+);", (CSRC / "seq" / "grouped_attention.hip").read_text()).group(1))
+    rests = set()
+    for (_, _, _, ntok, pos, _), (bf16, f32) in zip(test_gpu_bosirax.LONG_WALKS, found):
+        assert (pos + ntok) / bf16[1] >= long and math.prod(bf16) > CUS and math.prod(f32) > CUS
+        rests.add(math.prod(bf16) % CUS)
+    assert 0 in rests and len(rests) > 2
+
+
 # ---- latent portions with keys and values of every head (sequence_model.cpp: latent_expands) -----------------
 
 LATENT = """
@@ -379,6 +400,17 @@ answer([steps(layer("heads of 64"), "float32", 1024, 1024, [(0, 60)], [(0, 400)]
     # (the keys and values of 40,000 positions would be more than the scratch that is kept for them at most)
     assert [count(l)[0] for l in far[1]] == [1, 0] and far[0] - single[0] < (320 << 20) + 6 * 39000 * 400 * 4
     assert [count(l)[0] for l in small[1]] == [0] and small[0] < single[0]
+
+
+def test_one_head_is_expanded_without_slices(tmp_path):
+    """The keys and values of a layer of one head are plain products, which must not be cut along K: what is left there would overwrite them."""
+    found = fake_hip.run(tmp_path, LATENT.replace("got.append(", "got.append([l[1] for l in log(False) if l[0] == 'launch']); (lambda _: None)(") + """
+answer([steps(layer("one head"), dtype, 1600, 1600, [(0, 1600)], [(90, 1510)])[1] for dtype in ("float32", "bfloat16")])""")
+    for launched in sum(found, []):
+        first, = [i for i, name in enumerate(launched) if "transpose_tiles" in name]
+        last = next(i for i, name in enumerate(launched) if "16attention" in name)
+        products = launched[first + 1:last]
+        assert len(products) == 2 and all(WIDE.search(name).group(3) == "0" for name in products), products
 
 
 def test_the_line_of_expanded_portions(tmp_path):
