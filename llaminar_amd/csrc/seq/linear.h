@@ -6,7 +6,6 @@
 
 namespace llamql
 {
-    constexpr int LINEAR_STRETCHES = 8; // of rows in a launch, at most
     struct LinearArgs
     {
         const void *a; // T [M][lda], or fp32 [M][lda] when norm is set
@@ -31,9 +30,14 @@ namespace llamql
         // many rows: tiles from `full` on are cut into slices of K, their sums in `parts` (linear_tiled)
         f32x4 *parts;
         int full, slices;
-        // many rows: `stretches` of them alone (0: all), one a layer of the grid
+    };
+    // Some of many rows: one stretch a layer of the grid.  (A type and a kernel of its own: read as part of the others' arguments it cost each of
+    // their launches 0.5 to 1 us, bf16 24 x 15440 x 5120 28.9 -> 29.9.)
+    constexpr int LINEAR_STRETCHES = 8; // in a launch, at most
+    struct LinearSomeArgs : LinearArgs
+    {
         int stretches;
-        int stretch_first[LINEAR_STRETCHES], stretch_rows[LINEAR_STRETCHES];
+        int first[LINEAR_STRETCHES], rows[LINEAR_STRETCHES];
     };
 
     constexpr int SMALL_M = 16;         // most rows of the row-at-a-time kernel: one operand of the matrix unit
@@ -44,8 +48,8 @@ namespace llamql
     // scratch: for sums of tiles cut along K, as far as it reaches; what linear_split_bytes says serves layers of up to max_rows rows
     bool linear_tiled(const char *fn, const LinearArgs &a, int batch, int dtype, int device_id, hipStream_t st, void *scratch = nullptr,
                       size_t bytes = 0);
-    // The same for a.stretches of its rows, with the bits that they have among all
-    bool linear_tiled_rows(const char *fn, const LinearArgs &a, int batch, int dtype, int device_id, hipStream_t st);
+    // The same for some of its rows, with the bits that they have among all
+    bool linear_tiled_rows(const char *fn, const LinearSomeArgs &a, int batch, int dtype, int device_id, hipStream_t st);
     size_t linear_split_bytes(int max_rows, int N, int K, int dtype, int device_id);
 
     // Whether a sum of products in three bf16 pieces of each 32-bit value may not be that of the whole values, which then

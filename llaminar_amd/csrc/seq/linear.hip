@@ -488,7 +488,7 @@ extern "C" bool llam_seq_linear(const llam_seq_linear_args *a, int dtype, int de
 extern "C" bool llam_seq_linear_rows(const llam_seq_linear_args *a, int n, const int *first, const int *rows, int dtype, int device_id, void *stream)
 {
     static const char *fn = "llam_seq_linear_rows";
-    LinearArgs p;
+    LinearSomeArgs p{};
     if (!linear_args(fn, a, dtype, p))
         return false;
     if (a->M <= SMALL_M || n < 0 || (n > 0 && (!first || !rows)))
@@ -502,7 +502,7 @@ extern "C" bool llam_seq_linear_rows(const llam_seq_linear_args *a, int n, const
     {
         p.stretches = n - i < LINEAR_STRETCHES ? n - i : LINEAR_STRETCHES;
         for (int k = 0; k < p.stretches; ++k)
-            p.stretch_first[k] = first[i + k], p.stretch_rows[k] = rows[i + k];
+            p.first[k] = first[i + k], p.rows[k] = rows[i + k];
         if (!linear_tiled_rows(fn, p, a->batch, dtype, device_id, as_stream(stream)))
             return false;
     }

@@ -181,10 +181,10 @@ namespace llamql
 
     // Workgroup tile BM rows of A x BN rows of W; KG groups of WM x WN wavefronts, each with every KG-th turn of 64
     // columns, STAGES turns of A in LDS and WSTAGES of W.  SPLIT: the tiles from p.full on have p.slices workgroups each, every one with a slice of K,
-    // which leave their accumulators in p.parts for linear_join_kernel.
-    template <typename T, int BM, int BN, int WM, int WN, int KG, int STAGES, int WSTAGES, bool SPLIT>
+    // which leave their accumulators in p.parts for linear_join_kernel.  Args: LinearSomeArgs for some of the rows alone.
+    template <typename T, int BM, int BN, int WM, int WN, int KG, int STAGES, int WSTAGES, bool SPLIT, typename Args = LinearArgs>
     __global__ void __launch_bounds__(WM *WN *KG * 64)
-        linear_wide_kernel(LinearArgs p, int m_tiles, int n_tiles)
+        linear_wide_kernel(Args p, int m_tiles, int n_tiles)
     {
         using O = TiledOperand<T>;
         constexpr int NW = WM * WN;                         // wavefronts of a group
@@ -229,9 +229,9 @@ namespace llamql
             m_tiles = __builtin_amdgcn_readfirstlane(live);
         }
         int row0 = 0, rows = p.M;
-        if (p.stretches)
+        if constexpr (std::is_same_v<Args, LinearSomeArgs>)
         {
-            row0 = p.stretch_first[blockIdx.z], rows = p.stretch_rows[blockIdx.z];
+            row0 = p.first[blockIdx.z], rows = p.rows[blockIdx.z];
             m_tiles = (rows + BM - 1) / BM;
         }
         const int total = m_tiles * n_tiles;
@@ -611,9 +611,9 @@ namespace llamql
     namespace
     {
         template <typename T, int BM, int BN, int WM, int WN, int KG, int STAGES, int WSTAGES = STAGES>
-        bool wide_launch(const char *fn, const LinearArgs &a, int batch, hipStream_t st)
+        bool wide_launch(const char *fn, const LinearArgs &a, int batch, hipStream_t st, const LinearSomeArgs *some)
         {
-            static LdsGrant grant;
+            static LdsGrant grant, grant_some;
             constexpr size_t stages = (size_t)KG * (STAGES * BM * sizeof(T) + WSTAGES * BN * 2) * TILE_K, sums = (size_t)(KG - 1) * BM * BN * 4;
             static_assert(KG > 1 || stages >= (size_t)WM * BN * OUT_BYTES / 32, "the results' place");
             constexpr size_t lds = stages > sums ? stages : sums;
@@ -626,7 +626,15 @@ namespace llamql
             const long mt = a.group_offset ? a.group_rows / BM + (batch < a.group_rows ? batch : a.group_rows) : ceil_div(a.M, BM);
             if (mt * nt > 0x7fffffff)
                 return fail(fn, "M=%d rows of N=%d columns are too many", a.M, a.N);
-            hipLaunchKernelGGL(kernel, dim3((unsigned)(mt * nt), a.group_offset ? 1 : batch, a.stretches ? a.stretches : 1), dim3(WM * WN * KG * 64), lds, st, a, (int)mt, nt);
+            if (some)
+            {
+                const auto rows = &linear_wide_kernel<T, BM, BN, WM, WN, KG, STAGES, WSTAGES, false, LinearSomeArgs>;
+                if (lds > 64 * 1024 && allow_lds(grant_some, reinterpret_cast<const void *>(rows), lds) != hipSuccess)
+                    return fail(fn, "cannot reserve %zu bytes of LDS", lds);
+                hipLaunchKernelGGL(rows, dim3((unsigned)(mt * nt), batch, some->stretches), dim3(WM * WN * KG * 64), lds, st, *some, 0, nt);
+                return launched(fn);
+            }
+            hipLaunchKernelGGL(kernel, dim3((unsigned)(mt * nt), a.group_offset ? 1 : batch), dim3(WM * WN * KG * 64), lds, st, a, (int)mt, nt);
             return launched(fn);
         }
 
@@ -654,7 +662,7 @@ namespace llamql
         {
             int rows, columns, groups, resident;
             float alone, full, start;
-            bool (*launch)(const char *, const LinearArgs &, int, hipStream_t);
+            bool (*launch)(const char *, const LinearArgs &, int, hipStream_t, const LinearSomeArgs *);
             bool (*split)(const char *, const LinearArgs &, hipStream_t); // (none where two workgroups share a compute unit)
         };
         // Measured as time over turns for widths of 2048 to 51200, 40 to 2048 rows and K of 2048 to 30720.  Large tiles
@@ -786,26 +794,26 @@ namespace llamql
 
     // A sum is of the turns of its group of wavefronts, one after the other, so tiles of as many groups have the same bits
     // (all with one are rows of 32x32 products of 16 columns each).  Among these, the best for the rows that there are.
-    bool linear_tiled_rows(const char *fn, const LinearArgs &a, int batch, int dtype, int device_id, hipStream_t st)
+    bool linear_tiled_rows(const char *fn, const LinearSomeArgs &a, int batch, int dtype, int device_id, hipStream_t st)
     {
         const int cus = cu_count(device_id);
         const Tile *all = linear_plan(a, batch, dtype, 0, cus).tile, *tile = all;
-        LinearArgs some = a;
+        LinearSomeArgs some = a;
         some.M = 0;
         for (int k = 0; k < a.stretches; ++k)
-            some.M = some.M > a.stretch_rows[k] ? some.M : a.stretch_rows[k]; // (the grid is of the longest)
+            some.M = some.M > a.rows[k] ? some.M : a.rows[k]; // (the grid is of the longest)
         const auto [tiles, n] = tiles_of(dtype);
         for (size_t i = 0; i < n; ++i)
             if (tiles[i].groups == all->groups && expected(tiles[i], some, batch * a.stretches, cus) < expected(*tile, some, batch * a.stretches, cus))
                 tile = &tiles[i];
-        return tile->launch(fn, some, batch, st);
+        return tile->launch(fn, some, batch, st, &some);
     }
 
     bool linear_tiled(const char *fn, const LinearArgs &a, int batch, int dtype, int device_id, hipStream_t st, void *scratch, size_t bytes)
     {
         const Plan plan = linear_plan(a, batch, dtype, scratch ? bytes : 0, cu_count(device_id));
         if (plan.split.slices == 0)
-            return plan.tile->launch(fn, a, batch, st);
+            return plan.tile->launch(fn, a, batch, st, nullptr);
         LinearArgs cut = a;
         cut.parts = static_cast<f32x4 *>(scratch), cut.full = plan.split.full, cut.slices = plan.split.slices;
         return plan.tile->split(fn, cut, st);

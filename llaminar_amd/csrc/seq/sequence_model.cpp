@@ -382,7 +382,7 @@ namespace
                     llam_seq_linear_args l{};
                     l.d_a = a, l.lda = H * K, l.d_w = matrix, l.N = N, l.K = K, l.d_y = y, l.ldy = ldy, l.out = LLAM_SEQ_OUT_ELEM, l.M = s.M;
                     l.batch = H, l.a_stride = K, l.w_stride = (long)N * K, l.y_stride = N;
-                    if (s.M <= ROW_MAX)
+                    if (rows[0] == s.M)
                         return forward(fn, llam_seq_linear(&l, c.dtype, c.device_id, st));
                     return forward(fn, llam_seq_linear_rows(&l, (int)rows.size(), first.data(), rows.data(), c.dtype, c.device_id, st));
                 };
