@@ -111,8 +111,9 @@ namespace llamql
     // Which row block, stretch and key/value head a workgroup of many rows takes.  The longest walks go first, a row block of all heads after
     // the other (a die's workgroups have few heads, whose keys and values stay in its cache), and every second round of
     // workgroups backwards, so that a compute unit which has a long walk gets a short one beside it.  Head after head two long ones met:
-    // bf16, 2048 tokens, 16 heads of 128 in two stretches 71.6 -> 60.5 us (without turning back 71.8, with rounds of half or twice as many
-    // workgroups 70.9, 70.6), 40 heads in 8 groups 146 -> 118 (a walk of 2048 positions takes 115 by itself).
+    // bf16, one call behind the other, with the merge where there is one: 2048 tokens, 16 heads of 128 in two stretches 78.4 -> 67.6 us,
+    // 40 heads in 8 groups 135 -> 104; 1024 tokens of 64 heads 71 -> 53; 4096 tokens of 16 heads in 4 groups 224 -> 173.  The turning
+    // back is what gives it: without, or with rounds of half or twice as many workgroups, the first of these stayed within 2 % of the grid's order.
     // Short walks of bf16 gain nothing and pay for the order, and keep that of the grid: 16 heads in 4 groups, 500 tokens 21.5 and 22.4 us,
     // 512 at position 1536 33.6 and 35.4; fp32, 500 tokens 33.4 and 28.2.
     constexpr int ATT_LONG = 512; // positions of a stretch from which on they do

@@ -5,11 +5,11 @@
 // ends with four neighbouring output columns of one row; results go through LDS so that they leave by whole lines.  32-bit rows are multiplied in three bf16 pieces that add up to
 // them (weights are bf16 anyway): the products stay exact, the sums 32-bit, on a unit that is 16 times as fast.
 //
-// What bounds it, 2048 x 15440 x 5120 in bf16: the matrix unit is busy in 57 % of the cycles, at the 1.9 GHz that the chip
-// holds under this load; without any loads of A and W the same loop takes 260 instead of 285 us, LDS conflicts are none.
-// Time before (128 x 128 tiles staged through registers) and now: 390 -> 285 us (830 -> 1140 TFLOP/s), 2048 x 51200 x
-// 5120 1200 -> 940 us, 300 x 2048 x 8192 63 -> 28 us; 32-bit rows (v_mfma_f32_16x16x4 before) 2048 x 51200 x 5120 9490 ->
-// 2480 us, 522 x 2048 x 10240 380 -> 126 us.
+// What bounds it, 2048 x 15440 x 5120 in bf16: the matrix unit is busy in 63 % of the cycles (2048 x 51200 x 5120 68 %, 32-bit rows, 522 x 51200 x
+// 5120, 65 %), the LDS with reads in 25 %, and the two wavefronts of a SIMD unit meet at the barrier of every turn; where such products
+// follow each other the clock falls, from 1.85 to 1.3 GHz (266 to 380 us).
+// Time before (128 x 128 tiles staged through registers) and now, with the clock up: 390 -> 266 us (830 -> 1220 TFLOP/s), 2048 x 51200 x
+// 5120 1200 -> 875 us, 333 x 2048 x 8192 63 -> 28 us; 32-bit rows (v_mfma_f32_16x16x4 before) 522 x 2048 x 10240 380 -> 82 us (in slices).
 #include "linear.h"
 
 #include <type_traits>
@@ -666,11 +666,13 @@ namespace llamql
             bool (*split)(const char *, const LinearArgs &, hipStream_t); // (none where two workgroups share a compute unit)
         };
         // Measured as time over turns for widths of 2048 to 51200, 40 to 2048 rows and K of 2048 to 30720.  Large tiles
-        // read the LDS least per product (256 x 256: 1130 TFLOP/s at 2048 x 51200 x 5120, 128 x 128: 1010), small ones
+        // read the LDS least per product (256 x 256: 1220 TFLOP/s at 2048 x 51200 x 5120, 128 x 128: 1010), small ones
         // and groups of wavefronts that share K fill the chip where there are few tiles (522 x 2048 x 10240: 50 us with
-        // 128 x 64 and two groups, 120 with 256 x 128).  The same figures hold for the rows of routed experts: over 7 models' experts
-        // (8 to 256 of 64 to 1536, both ways) and 17 to 2000 rows, evenly chosen and not, the tile chosen is 0.9 % slower than
-        // the best in the mean, 15 % at most (1000 rows, 2 of 16 experts of 1536 x 5120, up: 210 and 182 us); fp32 0.6 %, 15 %.
+        // 128 x 64 and two groups, 120 with 256 x 128).  Over 16 layers of 1280 to 51200 x 1024 to 30720 with 12 numbers of rows in bf16 the tile
+        // chosen is 1.1 % above the best in the mean, 27 % at most (1000 rows of 5120 columns, 256 x 128 would be better: x 25600 399 and 315 us); of
+        // 10 with 8 in fp32 it is the best.  The same figures hold for the rows of routed experts: over 7 models' experts
+        // (8 to 256 of 512 to 4096, both ways) and 17 to 2000 rows, evenly chosen and not, a layer is 4.5 % above that of the best two tiles,
+        // 26 % at most (512 rows, 4 of 32 experts of 1024 x 2048, unevenly: 102 and 81 us); fp32 3.1 %, 30 %.
         // 187 rows, 6 of 64 experts of 1408 x 2048 and a shared one: bf16 209 -> 190 us against two tiles by the mean
         // rows of a group, fp32 369 -> 267 against tiles as if every group had all rows.
         // 256 x 256 has a third turn of W in its LDS, for that is what comes from memory, where A mostly comes from the cache: 64 experts of 155 to
@@ -712,10 +714,11 @@ namespace llamql
     namespace
     {
         // Tiles that fill no round of workgroups by themselves, cut into slices of K that do: in the time of a slice instead of that of a
-        // tile, for the sums that leave and come back and a launch that joins them.  (us, whole and in slices: bf16, 2048 x 5120 x 30720 682 -> 583,
-        // 500 x 5120 x 30720 247 -> 165, 64 x 2048 x 10240 31 -> 15, 1000 x 51200 x 5120 520 -> 466; fp32, 522 x 2048 x 10240 114 -> 82,
-        // 64 x 2048 x 16384 135 -> 28.)  Over 17 layers of 1280 to 51200 x 1024 to 30720 with 14 numbers of rows in bf16, 12 with 9 in fp32, 105 of 252
-        // and 75 of 108 are cut, to 0.74 and 0.56 times their time in the mean; none is slower, the choice is 1.2 % above the best of all.
+        // tile, for the sums that leave and come back and a launch that joins them.  (us, whole and in slices: bf16, 2048 x 5120 x 30720 637 -> 558,
+        // 512 x 5120 x 30720 251 -> 158, 64 x 2048 x 10240 32 -> 17, 1000 x 51200 x 5120 487 -> 449; fp32, 522 x 2048 x 10240 106 -> 80,
+        // 64 x 2048 x 16384 130 -> 30.)  Over 16 layers of 1280 to 51200 x 1024 to 30720 with 12 numbers of rows in bf16, 10 with 8 in fp32, 71 of 192
+        // and 57 of 80 are cut, to 0.76 and 0.69 times their time in the mean; none is slower by more than 3 % (0.3 us); the choice is 1.9 and 1.6 % above
+        // the best of all, 25 and 30 % at most (187 x 5120 x 10240 48 and 38 us; 20 x 2816 x 2048 16.7 and 12.9).
         constexpr int SLICES = 8;                        // at most
         constexpr size_t SPLIT_BYTES = (size_t)192 << 20; // sums of a launch, at most
         constexpr float JOIN_START = 4.0f, JOIN_BYTE = 0.45e-6f; // microseconds: a launch; a byte there and back
